@@ -85,6 +85,32 @@ def test_device_sampler_strided_rows_and_degenerate_input(trained, corc):
     assert err.value.status == ffi.E_SHAPE
 
 
+@pytest.mark.parametrize("V", [1, 63, 64, 65, 257, 1024, 1025])
+def test_device_sampler_at_the_edges_of_its_forms(trained, corc, V):
+    """One wavefront up to 256 and up to 1024 values, a workgroup beyond: the drawn index is the oracle's wherever the
+    variate lies more than 1e-5 (some tens of roundings of expf and of the running sums) from a boundary."""
+    from burn_dragon_amd.generation import sample_from_logits
+
+    model = trained[0]
+    rng = np.random.default_rng(100 + V)
+    B = 24
+    logits = (2.5 * rng.standard_normal((B, V))).astype(np.float32)
+    logits[2] = -np.inf  # no finite value at all: the uniform distribution
+    us = rng.random(B).astype(np.float32)
+    checked = 0
+    for temperature, top_k in [(0.8, 40), (1.0, None), (1.0, 1), (1.1, max(V - 1, 1))]:
+        got = sample_from_logits(model, torch.from_numpy(logits).to(DEV), temperature, top_k,
+                                 torch.from_numpy(us).to(DEV)).cpu().numpy()
+        for b in range(B):
+            want, p = corc.sample_from_logits(logits[b], temperature, top_k, float(us[b]))
+            cdf = np.cumsum(p.astype(np.float64))
+            if np.abs(cdf - np.float64(us[b]) * cdf[-1]).min() < 1e-5:
+                continue
+            assert got[b] == want, (temperature, top_k, b)
+            checked += 1
+    assert checked > 2 * B
+
+
 def test_trained_checkpoint_matches_oracle_and_predicts_the_text(trained, corc):
     model, tok, _, shape, w = trained
     ids = np.array([tok.encode(TEXT)])
