@@ -5,14 +5,15 @@
 // This is the reference's training-path form; it is kept in f32 and follows the reference's
 // block semantics exactly (including the ALiBi term being added to every entry of an active
 // block).  Small problems take a row-per-workgroup kernel; from T = 128 on the two products run
-// on the f32 matrix cores (v_mfma_f32_32x32x2_f32): S = mask(Q Q^T) + bias is materialised per
-// slice, a row pass sums |S|, and out = (S V) / (norm + eps).  The bf16 form for inference is in
-// prefill.hip.
+// on the matrix cores (gemm_f32.hip): S = mask(Q Q^T) + bias is materialised per slice, and
+// out = (S V) / (norm + eps) sums |S| on the way.  The bf16 form for inference is in prefill.hip.
+// The many-token form of the state step, the encoder E over many rows and relu_lowrank over many
+// rows are here as well.
 #include <algorithm>
 #include <cstring>
 #include <vector>
 
-#include "bdh_internal.h"
+#include "gemm_f32.h"
 
 namespace {
 
@@ -23,6 +24,7 @@ struct FsaSlopes {
 
 constexpr float kTwoPi = 6.28318530717958647692f;
 constexpr float kRowNormEps = 1e-6f;  // src/kernel/linear_attention.rs:9
+constexpr float kLnEps = 1e-5f;       // src/model/bdh.rs:17
 
 // q_rot [S,T,Nq] from query [S,T,N], positions 0..T (src/kernel/linear_attention.rs:23-40)
 __global__ __launch_bounds__(256) void k_rotate_f32(const float *__restrict__ x, const float *__restrict__ freqs,
@@ -34,10 +36,6 @@ __global__ __launch_bounds__(256) void k_rotate_f32(const float *__restrict__ x,
   const int Nq = rotary == BDH_POPE ? 2 * N : N;
   float *qr = q + row * Nq;
   for (int n = threadIdx.x; n < N; n += 256) {
-    if (rotary == BDH_ALIBI) {
-      qr[n] = xr[n];
-      continue;
-    }
     const float raw = pos * freqs[n];
     const float ph = (raw - floorf(raw)) * kTwoPi;
     float s, c;
@@ -186,145 +184,235 @@ __global__ __launch_bounds__(256) void k_fsa_row(const float *__restrict__ q, co
   }
 }
 
+// The sums of a scores product whose K was cut into parts: S[row][col] = sum of the parts in order, then the mask, the
+// decay and the ALiBi term of the GEMM_SCORES epilogue.  One workgroup per row; columns up to the end of the last time
+// block of the row's 128-row group (nothing reads beyond it), all of them with a sparse pattern.
+__global__ __launch_bounds__(256) void k_scores_reduce(const float *__restrict__ parts, long c_split, GemmF32 g) {
+  const long r = blockIdx.x;
+  const int slice = (int)(r / g.M), row = (int)(r - (long)slice * g.M);
+  const int bs = g.block_size;
+  const int end = g.active ? g.N : min(g.N, ((min((row | 127) + 1, g.M) - 1) / bs + 1) * bs);
+  const float *p = parts + ((long)slice * g.M + row) * g.N;
+  float *C = g.C + (long)(slice / g.mod) * g.c_s1 + (long)(slice % g.mod) * g.c_s2 + (long)row * g.ldc;
+  const int rb = row / bs;
+  const float ld = g.log_decay[slice % g.heads], slope = g.slopes[slice % g.heads];
+  for (int col = threadIdx.x; col < end; col += 256) {
+    const int cb = col / bs;
+    const bool act = g.active ? g.active[(long)rb * g.tb + cb] != 0 : cb <= rb;
+    float v = 0.0f;
+    if (act) {
+      if (!(rb == cb && col >= row))
+        for (int k = 0; k < g.ks; ++k) v += p[k * c_split + col];
+      if (g.decay_scores && col < row) v = v * expf((float)(row - col) * ld);
+      if (g.use_alibi) {
+        const float al = slope * ((float)col - (float)row);
+        v = v + al;
+      }
+    }
+    C[col] = v;
+  }
+}
+
+// out[slice][t0 + t][:] = the sum of the parts [part][slice][tc][d], in order, and, when out_ln is given, its LayerNorm
+// (src/model/bdh.rs:359).  One wavefront per row, d <= 1024.
+__global__ __launch_bounds__(256) void k_rows_reduce(const float *__restrict__ parts, int ks, long c_split, int tc, int d,
+                                                     long rows, float *__restrict__ out, float *__restrict__ out_ln,
+                                                     long slice_stride) {
+  const int lane = threadIdx.x & 63;
+  const long r = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (r >= rows) return;
+  const long o = r / tc * slice_stride + r % tc * d;
+  float v[16], s = 0.0f;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    const int c = j * 64 + lane;
+    v[j] = 0.0f;
+    if (c < d) {
+      for (int k = 0; k < ks; ++k) v[j] += parts[k * c_split + r * d + c];
+      out[o + c] = v[j];
+      s += v[j];
+    }
+  }
+  if (!out_ln) return;
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+  const float mean = s / (float)d;
+  float q = 0.0f;
+#pragma unroll
+  for (int j = 0; j < 16; ++j)
+    if (j * 64 + lane < d) q += (v[j] - mean) * (v[j] - mean);
+  for (int off = 32; off > 0; off >>= 1) q += __shfl_xor(q, off);
+  const float den = sqrtf(q / (float)d + kLnEps);
+#pragma unroll
+  for (int j = 0; j < 16; ++j)
+    if (j * 64 + lane < d) out_ln[o + j * 64 + lane] = (v[j] - mean) / den;
+}
+
 // ------------------------------------------------------------------------------------
-// f32 matrix-core path
+// relu_lowrank over many rows on the f32 matrix cores: [M, d] x [d, N] per head.
+// The eight matrix instructions of a 16-wide k stage take k = 0,1 | 2,3 | ...; v_mfma_f32_32x32x2_f32 adds its two k-steps
+// one after the other as fused multiply-adds, so every output is ONE k-sequential fmaf chain -- the bits of k_relu_lowrank.
+// The rows of all sequences of the call form one list (row m = token m % T of sequence m / T): a ragged T costs at most
+// one partly filled tile per head and not one per sequence.
 // ------------------------------------------------------------------------------------
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-
-// Eight floats as three bf16x8 operands h + m + l that add up to the floats exactly: each term is the remainder so far
-// rounded to bf16 (v_cvt_pk_bf16_f32, round to nearest even); a remainder is a difference of neighbours and therefore
-// exact, and the third one has at most eight significant bits.  A product of two such sums is taken as the six matrix
-// instructions l h, h l, m m, m h, h m, h h (smallest terms first); what is left out (m l, l m, l l) is below 2^-23 of
-// |a b|, the size of one f32 rounding.  An infinite input, or a finite one that rounds to an infinite bf16 (above
-// 3.389e38), gives NaN (inf - inf in the remainder).
-__device__ __forceinline__ void fsa_split3(const float (&a)[8], bf16x8 &h, bf16x8 &m, bf16x8 &l) {
-  typedef float f32x2 __attribute__((ext_vector_type(2)));
-  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-  u32x4 ph, pm, pl;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {  // element 2q in the low half of a dword, 2q + 1 in the high half
-    const f32x2 a2 = {a[2 * q], a[2 * q + 1]};
-    ph[q] = __builtin_bit_cast(unsigned int, __builtin_convertvector(a2, bf16x2));
-    const f32x2 r1 = {a2[0] - __uint_as_float(ph[q] << 16), a2[1] - __uint_as_float(ph[q] & 0xffff0000u)};
-    pm[q] = __builtin_bit_cast(unsigned int, __builtin_convertvector(r1, bf16x2));
-    const f32x2 r2 = {r1[0] - __uint_as_float(pm[q] << 16), r1[1] - __uint_as_float(pm[q] & 0xffff0000u)};
-    pl[q] = __builtin_bit_cast(unsigned int, __builtin_convertvector(r2, bf16x2));
-  }
-  h = __builtin_bit_cast(bf16x8, ph);
-  m = __builtin_bit_cast(bf16x8, pm);
-  l = __builtin_bit_cast(bf16x8, pl);
-}
 constexpr int FK = 16;    // k per LDS stage
-constexpr int FLD = 20;   // LDS row stride in floats (80 bytes: 16-byte aligned, spreads the banks)
+constexpr int FLD = 20;   // LDS row stride of A in floats (80 bytes: 16-byte aligned, spreads the banks)
 
-struct FsaArgs {
-  const float *A;   // A_KMAJOR ? [slices][K][lda] (m contiguous) : [slices][M][lda] (k contiguous)
-  const float *Bm;  // B_KMAJOR ? [b][K][ldb] (n contiguous) : [slices][N][ldb] (k contiguous)
-  float *C;         // [slices][M][ldc]
-  long a_batch, b_batch, c_batch;
-  int lda, ldb, ldc, M, N, K;
-  int b_div;        // B slice = slice / b_div
-  int n_slices;
-  int mt, nt;       // tile grid (rows, columns) of one slice
-  // scores epilogue
-  int block_size, tb, h, use_alibi, dense;
-  const unsigned char *active;  // [tb*tb] when !dense
-  float slopes[64];             // per head, by value (no device copy, no host synchronisation)
-  // output epilogue
-  const float *norm;            // [slices][M] or null
-  int beta;                     // EPI 2: C += acc instead of C = acc
-  // mod > 0: slice = s1 * mod + s2 and operand X starts at s1 * x_batch + s2 * x_mod_stride
-  int mod;
-  long a_mod_stride, b_mod_stride, c_mod_stride;
-  // ALiBi state decay (src/model/bdh.rs:299-301) in the many-token form, g = exp(log_decay[slice % h]):
-  //   FSA_DECAY_SCORES  EPI 0: S[t,s] *= g^(t-s)
-  //   FSA_DECAY_ROWS    EPI 2: acc[t,:] *= g^t
-  //   FSA_DECAY_STATE   EPI 2, A k-major: A[k,:] *= g^(K-k) on load and C = g^K * C + acc
-  int decay_mode;
-  float log_decay[64];
-  // EPI 3, relu_lowrank (src/kernel/relu_lowrank.rs:7-37): C = gate * mask * relu(acc + bias - thr), head = slice % mod
-  const float *rl_bias;            // [h][N] or null
-  float rl_thr;
-  const unsigned char *rl_mask;    // one byte per latent block (device) or null
-  int rl_block, rl_nblocks;
-  const float *rl_gate;            // laid out like C, or null
+struct RlArgs {
+  const float *A, *W;
+  float *C;
+  long a_outer, a_head;     // row m of head hh: A + (m / T) * a_outer + hh * a_head + (m % T) * d
+  int T, M, N, d, h;
+  int mt, nt;               // tile grid of one head
+  const float *bias;        // [h][N] or null
+  float thr;
+  const unsigned char *mask;  // one byte per latent block (device) or null
+  int block, n_blocks;
+  const float *gate;        // laid out like C, or null
 };
-constexpr int FSA_DECAY_SCORES = 1, FSA_DECAY_ROWS = 2, FSA_DECAY_STATE = 4;
 
-__device__ __forceinline__ float4 fsa_ld4(const float *p, int n_valid, bool vec_ok) {
-  if (n_valid >= 4 && vec_ok) return *reinterpret_cast<const float4 *>(p);
-  float4 r = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (n_valid > 0) r.x = p[0];
-  if (n_valid > 1) r.y = p[1];
-  if (n_valid > 2) r.z = p[2];
-  if (n_valid > 3) r.w = p[3];
-  return r;
+// What the two kernels below share: which tile, and what becomes of the sums.
+template <int BM, int BN, int NWM, int NWN>
+struct RlTile {
+  static constexpr int MI = BM / NWM / 32, NJ = BN / NWN / 32;
+  int hh, m0, n0, lane, wm, wn;
+  // false: a workgroup of the rounding-up.  Each XCD takes one contiguous eighth of the (head, tile) list (workgroup ids are
+  // dealt round-robin to the XCDs), tiles column by column: neighbours share a block of weight columns in one L2.
+  __device__ __forceinline__ bool init(const RlArgs &g) {
+    const int tiles = g.mt * g.nt;
+    const long total = (long)g.h * tiles;
+    const int xcd = blockIdx.x & 7;
+    const long at = total * xcd / 8 + (blockIdx.x >> 3);
+    if (at >= total * (xcd + 1) / 8) return false;
+    hh = (int)(at / tiles);
+    const int tile = (int)(at % tiles);
+    m0 = (tile % g.mt) * BM;
+    n0 = (tile / g.mt) * BN;
+    lane = threadIdx.x & 63;
+    wm = (threadIdx.x >> 6) / NWN;
+    wn = (threadIdx.x >> 6) % NWN;
+    return true;
+  }
+  // row m of A, clamped to the last one (the sums of the repeats are not stored)
+  __device__ __forceinline__ const float *a_row(const RlArgs &g, int m) const {
+    m = min(m, g.M - 1);
+    return g.A + (long)(m / g.T) * g.a_outer + (long)hh * g.a_head + (long)(m % g.T) * g.d;
+  }
+  // C = gate * mask * relu(acc + bias - thr) (src/kernel/relu_lowrank.rs:7-37); accumulator element e of lane l in a
+  // 32x32 tile: row = (e/4)*8 + (l/32)*4 + (e%4), col = l%32.  The place of a row is worked out once per four adjacent
+  // rows, and the gate values of a 32x32 tile are all asked for, under no branch, before the first of them is used.
+  __device__ __forceinline__ void finish(const RlArgs &g, const f32x16 (&acc)[MI][NJ]) const {
+    const bool whole = m0 + BM <= g.M && n0 + BN <= g.N;
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      long at_row[16];
+      int rows[16];
+#pragma unroll
+      for (int e4 = 0; e4 < 4; ++e4) {
+        const int row = m0 + wm * (BM / NWM) + i * 32 + e4 * 8 + (lane >> 5) * 4;
+        int b = row / g.T, t = row - b * g.T;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          rows[e4 * 4 + e] = row + e;
+          at_row[e4 * 4 + e] = (((long)b * g.h + hh) * g.T + t) * g.N;
+          if (++t == g.T) { t = 0; ++b; }
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const int col = n0 + wn * (BN / NWN) + j * 32 + (lane & 31);
+        const int cc = min(col, g.N - 1);
+        const float bv = g.bias ? g.bias[(long)hh * g.N + cc] : 0.0f;
+        float mk = 1.0f;
+        if (g.mask) {
+          const int blk = cc / g.block;
+          mk = (blk < g.n_blocks && g.mask[blk]) ? 1.0f : 0.0f;
+        }
+        // the gate and the output are touched once per call: streaming accesses leave the L2 to the operand tiles
+        float gv[16];
+        if (g.gate) {
+          const long last = (((long)(g.M / g.T - 1) * g.h + hh) * g.T + g.T - 1) * g.N;
+#pragma unroll
+          for (int e = 0; e < 16; ++e) gv[e] = __builtin_nontemporal_load(g.gate + min(at_row[e], last) + cc);
+        }
+        float y[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          float pv = acc[i][j][e];
+          if (g.bias) pv = pv + bv;
+          if (g.thr != 0.0f) pv = pv - g.thr;
+          y[e] = pv > 0.0f ? pv : 0.0f;
+          if (g.mask) y[e] = y[e] * mk;
+          if (g.gate) y[e] = gv[e] * y[e];
+        }
+        if (whole) {
+#pragma unroll
+          for (int e = 0; e < 16; ++e) __builtin_nontemporal_store(y[e], g.C + at_row[e] + col);
+        } else if (col < g.N) {
+#pragma unroll
+          for (int e = 0; e < 16; ++e)
+            if (rows[e] < g.M) __builtin_nontemporal_store(y[e], g.C + at_row[e] + col);
+        }
+      }
+    }
+  }
+};
+
+// d a multiple of 32, N of 4, 16-byte aligned operands: both tiles go from memory straight into LDS (no registers, no
+// address arithmetic to wait for), 32 k at a time into two buffers in turn, one barrier per stage.  The 16-byte pieces of
+// a row of A (128 bytes), and those of an odd k row of W, are rotated against each other so that the 16-byte reads of 16
+// consecutive rows of A, and the 4-byte reads of two k rows of W, cover the 64 banks once.  What bounds it: the f32 matrix
+// instruction (64 cycles for 32 x 32 x 2: 157 TFLOP/s); [1500 x 256] x [256 x 32768] 412 -> 273 us (92 TFLOP/s, of which
+// about 60 us the 200 MB of output), [8192 x 512] x [512 x 131072] 9.8 -> 9.1 ms (120), [128 x 256] x [256 x 1024] 17 -> 10 us
+// against the same products staged through registers, whose loads were waited for where they were issued.
+//
+// Copies 16 bytes per lane from *src to LDS, the 64 lanes' pieces one after the other from dst (uniform over the
+// wavefront).  Written out because the compiler waits for every copy that it knows of before any LDS read that might see
+// it; here the barrier at the end of a stage, behind s_waitcnt, is what orders the two.
+typedef __attribute__((address_space(3))) void *lptr_t;
+__device__ __forceinline__ void copy_to_lds(const float *src, float *dst) {
+  const unsigned int at = __builtin_amdgcn_readfirstlane((unsigned int)(uintptr_t)(lptr_t)dst);
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(at), "v"(src) : "memory");
 }
 
-// EPI 0: scores (mask, ALiBi term, zero outside the pattern); EPI 1: out = acc / (norm + eps);
-// EPI 2: C = acc or C += acc; EPI 3: the relu_lowrank epilogue.
-// SEQK: the eight matrix instructions of a 16-wide k stage take k = 0,1 | 2,3 | ... instead of 0,8 | 1,9 | ...; an
-// instruction adds its two k-steps one after the other as fused multiply-adds, so every output is then ONE
-// k-sequential fmaf chain -- the same bits as a scalar loop over k (A rows k-contiguous, B k-major only).
-// A k-major operand (its reduction index is the slow one in memory) is staged as it lies, [k][m] with a
-// row stride of tile + 4 floats: float4 stores, and fragment reads of one float per lane in which the
-// 32 lanes of a half-wave take consecutive addresses and the two halves (k and k + 8) fall on the two
-// halves of the 64 banks.
-// SPLIT3: the products run on the bf16 matrix instructions (16 times the f32 rate) with every f32 operand split into
-// three bf16 terms in registers, six instructions per f32 one: f32-level accuracy (the result differs from the f32
-// instruction's by about one rounding of a product), not the bits of any particular summation order.  The fragment a
-// lane holds for eight f32 steps (k = half*8 .. +7 of its row) is the fragment of one 32 x 32 x 16 instruction.
-// Tile BM x BN, NWM x NWN waves, each wave (BM/NWM) x (BN/NWN).  The 128 x 128 tile needs 8 bytes per
-// clock and workgroup from the L2, which three resident workgroups per CU do not get; the
-// 256 x 256 tile halves that per FLOP and is the one that keeps the matrix cores busy.
-template <int EPI, bool A_KMAJOR, bool B_KMAJOR, int BM, int BN, int NWM, int NWN, bool SEQK = false, bool SPLIT3 = false>
-__global__ __launch_bounds__(NWM * NWN * 64) void k_fsa_gemm_f32(FsaArgs g) {
-  static_assert(!(SEQK && SPLIT3), "the split product does not keep the bits of a scalar loop");
-  static_assert(!SEQK || (!A_KMAJOR && B_KMAJOR), "sequential k order is built for row-major A and k-major B");
-  constexpr int NT = NWM * NWN * 64;
-  constexpr int KLA = BM + 4, KLB = BN + 4;  // row strides of the k-major LDS layouts
-  static_assert(FK * KLA <= BM * FLD && FK * KLB <= BN * FLD, "k-major tile must fit");
-  constexpr int MI = BM / NWM / 32, NJ = BN / NWN / 32;
-  constexpr int CA = BM * 4 / NT, CB = BN * 4 / NT;  // float4 chunks per thread and stage
-  static_assert(CA >= 1 && CB >= 1 && CA * NT == BM * 4 && CB * NT == BN * 4, "tile does not divide over the threads");
-  __shared__ __attribute__((aligned(16))) float s_a[BM * FLD];
-  __shared__ __attribute__((aligned(16))) float s_b[BN * FLD];
-  // XCD-aware mapping: workgroup ids are dealt round-robin to the 8 XCDs, so ids with the same
-  // (id % 8) share an L2; all tiles of one slice go to one XCD and reuse its operand rows there.
-  const int xcd = blockIdx.x & 7;
-  const int rr = blockIdx.x >> 3;
-  const int tiles = g.mt * g.nt;
-  const int slice = xcd + 8 * (rr / tiles);
-  if (slice >= g.n_slices) return;
-  const int tile = rr % tiles;
-  const int m0 = (tile / g.nt) * BM, n0 = (tile % g.nt) * BN;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave / NWN, wn = wave % NWN;
-  const float *A = g.A + (long)slice * g.a_batch;
-  const float *Bm = g.Bm + (long)(slice / g.b_div) * g.b_batch;
-  float *C = g.C + (long)slice * g.c_batch;
-  if (g.mod > 0) {
-    const long s1 = slice / g.mod, s2 = slice % g.mod;
-    A = g.A + s1 * g.a_batch + s2 * g.a_mod_stride;
-    Bm = g.Bm + s1 * g.b_batch + s2 * g.b_mod_stride;
-    C = g.C + s1 * g.c_batch + s2 * g.c_mod_stride;
+template <int BM, int BN>
+__global__ __launch_bounds__(256) void k_relu_lowrank_direct(RlArgs g) {
+  using Tl = RlTile<BM, BN, 2, 2>;
+  constexpr int MI = Tl::MI, NJ = Tl::NJ, SK = 32;
+  constexpr int AP = SK / 4;  // pieces of a row of A
+  auto a_turn = [](int row) { return (row >> 1) & 7; };
+  constexpr int CA = BM * SK / 4 / 256, CB = BN * SK / 4 / 256;  // 16-byte pieces per thread and stage
+  extern __shared__ __attribute__((aligned(1024))) float s_tiles[];  // two stages of A [BM][32], W [32][BN]
+  constexpr int STAGE = (BM + BN) * SK;
+  Tl t;
+  if (!t.init(g)) return;
+  const int tid = threadIdx.x, lane = t.lane, wave = tid >> 6;
+  const float *W = g.W + (long)t.hh * g.d * g.N;
+  const float *pa[CA], *pb[CB];
+#pragma unroll
+  for (int c = 0; c < CA; ++c) {
+    const int piece = c * 256 + tid, row = piece / AP;
+    pa[c] = t.a_row(g, t.m0 + row) + ((piece % AP) ^ a_turn(row)) * 4;
   }
-  const int bs = g.block_size;
-
-  int K = g.K;
-  bool tile_active = true;
-  if (EPI == 0) {
-    // dense pattern: block (rb, cb) is active iff cb <= rb; a tile all of whose blocks lie above
-    // the diagonal only writes zeros
-    if (g.dense && n0 / bs > (min(m0 + BM, g.M) - 1) / bs) tile_active = false;
-  } else if (g.dense) {
-    K = min(K, ((min(m0 + BM, g.M) - 1) / bs + 1) * bs);  // S is zero beyond the row tile's last block
+#pragma unroll
+  for (int c = 0; c < CB; ++c) {
+    const int piece = c * 256 + tid, k = piece / (BN / 4);
+    const int nc = ((piece % (BN / 4)) ^ ((k & 1) << 3)) * 4;
+    pb[c] = W + (long)k * g.N + min(t.n0 + nc, g.N - 4);  // four columns are all in or all out
   }
-  if (K <= 0) tile_active = false;
-  const float ld = g.decay_mode ? g.log_decay[slice % g.h] : 0.0f;
-
+  const long b_step = (long)SK * g.N;
+  auto issue = [&](int buf) {
+#pragma unroll
+    for (int c = 0; c < CA; ++c) {
+      copy_to_lds(pa[c], s_tiles + buf * STAGE + (c * 256 + wave * 64) * 4);
+      pa[c] += SK;
+    }
+#pragma unroll
+    for (int c = 0; c < CB; ++c) {
+      copy_to_lds(pb[c], s_tiles + buf * STAGE + BM * SK + (c * 256 + wave * 64) * 4);
+      pb[c] += b_step;
+    }
+  };
   f32x16 acc[MI][NJ];
 #pragma unroll
   for (int i = 0; i < MI; ++i)
@@ -332,258 +420,225 @@ __global__ __launch_bounds__(NWM * NWN * 64) void k_fsa_gemm_f32(FsaArgs g) {
     for (int j = 0; j < NJ; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-
-  if (tile_active) {
-    const bool a_vec = (g.lda % 4 == 0) && (reinterpret_cast<uintptr_t>(A) % 16 == 0);
-    const bool b_vec = (g.ldb % 4 == 0) && (reinterpret_cast<uintptr_t>(Bm) % 16 == 0);
-    float4 ra[1][CA], rb[1][CB];
-    // a tile that lies inside both operands, 16-byte aligned: its loads need no checks, and loads that sit
-    // under no branch are issued back to back
-    const bool tile_full = a_vec && b_vec && m0 + BM <= g.M && n0 + BN <= g.N;
-    auto load = [&](float4 *pa, float4 *pb, int k0) {
-      if (tile_full && k0 + FK <= K) {
-#pragma unroll
-        for (int c = 0; c < CA; ++c) {
-          const int chunk = c * NT + tid;
-          if (!A_KMAJOR) {
-            const int row = chunk >> 2, kc = (chunk & 3) * 4;
-            pa[c] = *reinterpret_cast<const float4 *>(A + (long)(m0 + row) * g.lda + k0 + kc);
-          } else {
-            const int kr = chunk / (BM / 4), mc = (chunk % (BM / 4)) * 4;
-            pa[c] = *reinterpret_cast<const float4 *>(A + (long)(k0 + kr) * g.lda + m0 + mc);
-          }
-        }
-#pragma unroll
-        for (int c = 0; c < CB; ++c) {
-          const int chunk = c * NT + tid;
-          if (!B_KMAJOR) {
-            const int row = chunk >> 2, kc = (chunk & 3) * 4;
-            pb[c] = *reinterpret_cast<const float4 *>(Bm + (long)(n0 + row) * g.ldb + k0 + kc);
-          } else {
-            const int kr = chunk / (BN / 4), nc = (chunk % (BN / 4)) * 4;
-            pb[c] = *reinterpret_cast<const float4 *>(Bm + (long)(k0 + kr) * g.ldb + n0 + nc);
-          }
-        }
-        if (A_KMAJOR && EPI == 2 && (g.decay_mode & FSA_DECAY_STATE)) {
-#pragma unroll
-          for (int c = 0; c < CA; ++c) {
-            const int kr = (c * NT + tid) / (BM / 4);
-            const float f = expf((float)(K - (k0 + kr)) * ld);
-            pa[c].x *= f; pa[c].y *= f; pa[c].z *= f; pa[c].w *= f;
-          }
-        }
-        return;
-      }
-#pragma unroll
-      for (int c = 0; c < CA; ++c) {
-        const int chunk = c * NT + tid;
-        if (!A_KMAJOR) {
-          const int row = chunk >> 2, kc = (chunk & 3) * 4;
-          pa[c] = (m0 + row < g.M && k0 < K) ? fsa_ld4(A + (long)(m0 + row) * g.lda + k0 + kc, K - (k0 + kc), a_vec)
-                                             : make_float4(0.f, 0.f, 0.f, 0.f);
-        } else {
-          const int kr = chunk / (BM / 4), mc = (chunk % (BM / 4)) * 4;  // BM/4 chunks of 4 rows per k row
-          pa[c] = (k0 + kr < K) ? fsa_ld4(A + (long)(k0 + kr) * g.lda + m0 + mc, g.M - (m0 + mc), a_vec)
-                                : make_float4(0.f, 0.f, 0.f, 0.f);
-          if (EPI == 2 && (g.decay_mode & FSA_DECAY_STATE)) {  // token k of K is decayed K - k times by the end
-            const float f = expf((float)(K - (k0 + kr)) * ld);
-            pa[c].x *= f; pa[c].y *= f; pa[c].z *= f; pa[c].w *= f;
-          }
-        }
-      }
-#pragma unroll
-      for (int c = 0; c < CB; ++c) {
-        const int chunk = c * NT + tid;
-        if (!B_KMAJOR) {
-          const int row = chunk >> 2, kc = (chunk & 3) * 4;
-          pb[c] = (n0 + row < g.N && k0 < K) ? fsa_ld4(Bm + (long)(n0 + row) * g.ldb + k0 + kc, K - (k0 + kc), b_vec)
-                                             : make_float4(0.f, 0.f, 0.f, 0.f);
-        } else {
-          const int kr = chunk / (BN / 4), nc = (chunk % (BN / 4)) * 4;  // BN/4 chunks of 4 columns per k row
-          pb[c] = (k0 + kr < K) ? fsa_ld4(Bm + (long)(k0 + kr) * g.ldb + n0 + nc, g.N - (n0 + nc), b_vec)
-                                : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-      }
-    };
-    auto store = [&](const float4 *pa, const float4 *pb) {
-#pragma unroll
-      for (int c = 0; c < CA; ++c) {
-        const int chunk = c * NT + tid;
-        if (!A_KMAJOR) {
-          const int row = chunk >> 2, kc = (chunk & 3) * 4;
-          if (SEQK) {  // k = kc, kc + 2 to places kc / 2, kc / 2 + 1; k = kc + 1, kc + 3 to places 8 + kc / 2, ...
-            *reinterpret_cast<float2 *>(s_a + row * FLD + (kc >> 1)) = make_float2(pa[c].x, pa[c].z);
-            *reinterpret_cast<float2 *>(s_a + row * FLD + 8 + (kc >> 1)) = make_float2(pa[c].y, pa[c].w);
-          } else {
-            *reinterpret_cast<float4 *>(s_a + row * FLD + kc) = pa[c];
-          }
-        } else {
-          const int kr = chunk / (BM / 4), mc = (chunk % (BM / 4)) * 4;
-          *reinterpret_cast<float4 *>(s_a + kr * KLA + mc) = pa[c];
-        }
-      }
-#pragma unroll
-      for (int c = 0; c < CB; ++c) {
-        const int chunk = c * NT + tid;
-        if (!B_KMAJOR) {
-          const int row = chunk >> 2, kc = (chunk & 3) * 4;
-          *reinterpret_cast<float4 *>(s_b + row * FLD + kc) = pb[c];
-        } else {
-          const int kr = chunk / (BN / 4), nc = (chunk % (BN / 4)) * 4;
-          *reinterpret_cast<float4 *>(s_b + kr * KLB + nc) = pb[c];
-        }
-      }
-    };
-    auto multiply = [&]() {
-      // lane (r = lane % 32, half = lane / 32) feeds k = half*8 + q to the q-th of eight 32x32x2 steps
-      const int r = lane & 31, kb = (lane >> 5) * 8;
-      float fa[MI][8], fb[NJ][8];
+  const int r = lane & 31, half = lane >> 5;
+  issue(0);
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  int cur = 0;
+  for (int k0 = 0; k0 < g.d; k0 += SK) {
+    if (k0 + SK < g.d) issue(cur ^ 1);  // lands while the matrix cores work on this stage
+    const float *sa = s_tiles + cur * STAGE, *sb = sa + BM * SK;
+    // four k at a time: instruction 0 takes k = 4c, 4c + 1, instruction 1 takes 4c + 2, 4c + 3.  The operands of the next
+    // four are on their way while these are multiplied.
+    float4 va[2][MI];
+    float vb[2][2][NJ];
+    auto fragments = [&](int c) {
 #pragma unroll
       for (int i = 0; i < MI; ++i) {
-        if (A_KMAJOR) {
-          const float *p = s_a + kb * KLA + wm * (BM / NWM) + i * 32 + r;
-#pragma unroll
-          for (int q = 0; q < 8; ++q) fa[i][q] = p[q * KLA];
-          continue;
-        }
-        // (SEQK: the stage was stored with its even k in the first eight places of a row and its odd k in the
-        // last eight, so the same two reads give this half-wave k = 2 q + half)
-        const float *p = s_a + (wm * (BM / NWM) + i * 32 + r) * FLD + kb;
-        const float4 lo = *reinterpret_cast<const float4 *>(p), hi = *reinterpret_cast<const float4 *>(p + 4);
-        fa[i][0] = lo.x; fa[i][1] = lo.y; fa[i][2] = lo.z; fa[i][3] = lo.w;
-        fa[i][4] = hi.x; fa[i][5] = hi.y; fa[i][6] = hi.z; fa[i][7] = hi.w;
+        const int row = t.wm * (BM / 2) + i * 32 + r;
+        va[c & 1][i] = *reinterpret_cast<const float4 *>(sa + row * SK + (c ^ a_turn(row)) * 4);
       }
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
-        if (B_KMAJOR) {
-          const float *p = s_b + (SEQK ? (lane >> 5) : kb) * KLB + wn * (BN / NWN) + j * 32 + r;
-#pragma unroll
-          for (int q = 0; q < 8; ++q) fb[j][q] = p[(SEQK ? 2 * q : q) * KLB];
-          continue;
-        }
-        const float *p = s_b + (wn * (BN / NWN) + j * 32 + r) * FLD + kb;
-        const float4 lo = *reinterpret_cast<const float4 *>(p), hi = *reinterpret_cast<const float4 *>(p + 4);
-        fb[j][0] = lo.x; fb[j][1] = lo.y; fb[j][2] = lo.z; fb[j][3] = lo.w;
-        fb[j][4] = hi.x; fb[j][5] = hi.y; fb[j][6] = hi.z; fb[j][7] = hi.w;
+        const int col = (t.wn * (BN / 2) + j * 32 + r) ^ (half << 5);
+        vb[c & 1][0][j] = sb[(4 * c + half) * BN + col];
+        vb[c & 1][1][j] = sb[(4 * c + 2 + half) * BN + col];
       }
-      if (SPLIT3) {
-        bf16x8 ah[MI], am[MI], al[MI], bh[NJ], bm[NJ], bl[NJ];
+    };
+    fragments(0);
 #pragma unroll
-        for (int i = 0; i < MI; ++i) fsa_split3(fa[i], ah[i], am[i], al[i]);
+    for (int c = 0; c < AP; ++c) {
+      if (c + 1 < AP) fragments(c + 1);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) fsa_split3(fb[j], bh[j], bm[j], bl[j]);
+      for (int q = 0; q < 2; ++q)
 #pragma unroll
-        for (int i = 0; i < MI; ++i)
-#pragma unroll
-          for (int j = 0; j < NJ; ++j) {
-            f32x16 c = acc[i][j];
-            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[i], bh[j], c, 0, 0, 0);
-            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i], bl[j], c, 0, 0, 0);
-            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(am[i], bm[j], c, 0, 0, 0);
-            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(am[i], bh[j], c, 0, 0, 0);
-            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i], bm[j], c, 0, 0, 0);
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i], bh[j], c, 0, 0, 0);
-          }
-        return;
-      }
-#pragma unroll
-      for (int q = 0; q < 8; ++q)
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
+        for (int i = 0; i < MI; ++i) {
+          const float4 v = va[c & 1][i];
+          const float a = q == 0 ? (half ? v.y : v.x) : (half ? v.w : v.z);
 #pragma unroll
           for (int j = 0; j < NJ; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i][q], fb[j][q], acc[i][j], 0, 0, 0);
-    };
-    // one register stage: a second one (loads two k-steps ahead) measured no faster
-    load(ra[0], rb[0], 0);
-    for (int k0 = 0; k0 < K; k0 += FK) {
-      __syncthreads();  // the previous step's fragment reads are done
-      store(ra[0], rb[0]);
-      __syncthreads();
-      load(ra[0], rb[0], k0 + FK);  // an out-of-range stage loads nothing
-      multiply();
-    }
-  }
-
-  // accumulator element e of lane l in a 32x32 tile: row = (e/4)*8 + (l/32)*4 + (e%4), col = l%32
-  const float slope = (EPI == 0 && g.use_alibi) ? g.slopes[slice % g.h] : 0.0f;
-#pragma unroll
-  for (int i = 0; i < MI; ++i)
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const int col = n0 + wn * (BN / NWN) + j * 32 + (lane & 31);
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int row = m0 + wm * (BM / NWM) + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
-        if (row >= g.M) continue;
-        if (EPI == 0) {
-          if (col >= g.ldc) continue;
-          float v = 0.0f;
-          if (col < g.N) {
-            const int rbk = row / bs, cbk = col / bs;
-            const bool act = g.dense ? (cbk <= rbk) : (g.active[(long)rbk * g.tb + cbk] != 0);
-            if (act) {
-              v = (rbk == cbk && col >= row) ? 0.0f : acc[i][j][e];  // tril(-1) on diagonal blocks (:88-90)
-              if ((g.decay_mode & FSA_DECAY_SCORES) && col < row) v = v * expf((float)(row - col) * ld);
-              if (g.use_alibi) {  // added to every entry of an active block (:97-100)
-                const float al = slope * ((float)col - (float)row);
-                v = v + al;
-              }
-            }
-          }
-          C[(long)row * g.ldc + col] = v;
-        } else if (EPI == 1) {
-          if (col >= g.N) continue;
-          float v = acc[i][j][e];
-          if (g.norm) v = v / (g.norm[(long)slice * g.M + row] + kRowNormEps);
-          C[(long)row * g.ldc + col] = v;
-        } else if (EPI == 3) {
-          if (col >= g.N) continue;
-          const int hh = g.mod > 0 ? slice % g.mod : 0;
-          float pv = acc[i][j][e];
-          if (g.rl_bias) pv = pv + g.rl_bias[(long)hh * g.N + col];
-          if (g.rl_thr != 0.0f) pv = pv - g.rl_thr;
-          float y = pv > 0.0f ? pv : 0.0f;
-          if (g.rl_mask) {
-            const int blk = col / g.rl_block;
-            y = y * ((blk < g.rl_nblocks && g.rl_mask[blk]) ? 1.0f : 0.0f);
-          }
-          const long o = (long)row * g.ldc + col;
-          // the gate and the output are touched once per call: streaming accesses leave the L2 to the operand tiles
-          // ([8192 x 512] x [512 x 131072]: 9.98 -> 9.69 ms)
-          if (g.rl_gate) y = __builtin_nontemporal_load(g.rl_gate + (C - g.C) + o) * y;
-          __builtin_nontemporal_store(y, C + o);
-        } else {
-          if (col >= g.N) continue;
-          float *p = C + (long)row * g.ldc + col;
-          float v = acc[i][j][e];
-          if (g.decay_mode & FSA_DECAY_ROWS) v = v * expf((float)row * ld);
-          if (g.decay_mode & FSA_DECAY_STATE)
-            *p = *p * expf((float)g.K * ld) + v;
-          else if (g.beta)
-            // C += acc as one no-return add per element, done by the L2: the wavefront does not wait for C to arrive,
-            // so a short-K tile's epilogue overlaps the next workgroup's products (rho += Q^T V at B=32, h=8,
-            // N=16384, d=512, K=256: 12.1 -> 10.1 ms).  One add per element and call: the same rounding as
-            // *p + v and no race; the L2's adder flushes results below the smallest normal float to zero.
-            unsafeAtomicAdd(p, v);
-          else
-            *p = v;
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, vb[c & 1][q][j], acc[i][j], 0, 0, 0);
         }
-      }
     }
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    cur ^= 1;
+  }
+  t.finish(g, acc);
 }
 
-// norm[row] = sum_s |S[row, s]|: one wave per row
-__global__ __launch_bounds__(256) void k_fsa_row_abs_sum(const float *__restrict__ S, long rows, int T, int ld,
-                                                         float *__restrict__ norm) {
-  const long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (row >= rows) return;
-  const int lane = threadIdx.x & 63;
-  const float *p = S + row * ld;
-  float a = 0.0f;
-  for (int c = lane; c < T; c += 64) a += fabsf(p[c]);
-  for (int o = 32; o > 0; o >>= 1) a += __shfl_xor(a, o);
-  if (lane == 0) norm[row] = a;
+// Few rows, or few tiles: 16 * RT rows x 64 columns per workgroup on v_mfma_f32_16x16x4_f32, whose four k-steps are also
+// added one after the other (the bits of the scalar chain again).  A wavefront owns 16 columns, so a chain of d steps takes
+// 8 cycles a step and row tile where the 32 x 32 instruction takes 32, and a few rows give four times the wavefronts: what
+// bounds it is the stream of the weights, every one of them copied to LDS once per 16 * RT rows.
+// Two stages in LDS: a third or fourth changed nothing.  us per call, the VALU and matrix-core kernels it took over from |
+// this: h*N = 1024, d = 256, 63 rows 7.6 | 6.1; 8192, 512, 48 rows 52.5 | 11.5; 32768, 256, 16 rows 29.7 | 8.4;
+// 131072, 512 (268 MB of weights), 16 rows 57.9 | 47.8, 32 rows 65.5 | 58.6.
+template <int RT>
+__global__ __launch_bounds__(256) void k_relu_lowrank_rows(RlArgs g) {
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  constexpr int BM = 16 * RT, BN = 64, SK = 32;
+  constexpr int STAGE = (BM + BN) * SK;
+  extern __shared__ __attribute__((aligned(1024))) float s_tiles[];  // two stages of A [BM][32], W [32][64]
+  const int tiles = g.mt * g.nt;
+  const long total = (long)g.h * tiles;
+  const int xcd = blockIdx.x & 7;
+  const long at = total * xcd / 8 + (blockIdx.x >> 3);
+  if (at >= total * (xcd + 1) / 8) return;
+  const int hh = (int)(at / tiles), tile = (int)(at % tiles);
+  const int m0 = (tile % g.mt) * BM, n0 = (tile / g.mt) * BN;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const float *W = g.W + (long)hh * g.d * g.N;
+  // A: BM * 8 pieces of 16 bytes, W: 512; a piece of row r of A sits at place (piece ^ r / 2), one of k row k of W at place
+  // (piece ^ 4 (k % 4)): the 4-byte reads below then cover the 64 banks once
+  constexpr int CA = (BM * 8 + 255) / 256;
+  const float *pa[CA], *pb[2];
+#pragma unroll
+  for (int c = 0; c < CA; ++c) {
+    const int piece = c * 256 + tid, row = piece >> 3, m = min(m0 + row, g.M - 1);
+    pa[c] = g.A + (long)(m / g.T) * g.a_outer + (long)hh * g.a_head + (long)(m % g.T) * g.d + ((piece & 7) ^ ((row >> 1) & 7)) * 4;
+  }
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const int piece = c * 256 + tid, k = piece >> 4;
+    pb[c] = W + (long)k * g.N + min(n0 + ((piece & 15) ^ ((k & 3) << 2)) * 4, g.N - 4);
+  }
+  const long b_step = (long)SK * g.N;
+  auto issue = [&](int buf) {
+    float *s = s_tiles + buf * STAGE;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      copy_to_lds(pb[c], s + BM * SK + (c * 256 + wave * 64) * 4);
+      pb[c] += b_step;
+    }
+#pragma unroll
+    for (int c = 0; c < CA; ++c) {
+      if (BM * 8 >= 256 || wave * 64 < BM * 8) copy_to_lds(pa[c], s + (c * 256 + wave * 64) * 4);
+      pa[c] += SK;
+    }
+  };
+  f32x4 acc[RT];
+#pragma unroll
+  for (int i = 0; i < RT; ++i) acc[i] = (f32x4)(0.0f);
+  const int r = lane & 15, q = lane >> 4;
+  issue(0);
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  int cur = 0;
+  for (int k0 = 0; k0 < g.d; k0 += SK) {
+    if (k0 + SK < g.d) issue(cur ^ 1);  // lands while the matrix cores work on this stage
+    const float *sa = s_tiles + cur * STAGE, *sb = sa + BM * SK;
+    float fa[SK / 4][RT], fb[SK / 4];
+#pragma unroll
+    for (int c = 0; c < SK / 4; ++c) {
+      fb[c] = sb[(4 * c + q) * BN + ((wave * 16 + r) ^ (q << 4))];
+#pragma unroll
+      for (int i = 0; i < RT; ++i) {
+        const int row = i * 16 + r;
+        fa[c][i] = sa[row * SK + (c ^ ((row >> 1) & 7)) * 4 + q];
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < SK / 4; ++c)
+#pragma unroll
+      for (int i = 0; i < RT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[c][i], fb[c], acc[i], 0, 0, 0);
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    cur ^= 1;
+  }
+  // element e of lane l: row = (l/16)*4 + e, column = l%16
+  const int col = n0 + wave * 16 + r;
+  if (col >= g.N) return;
+  const float bv = g.bias ? g.bias[(long)hh * g.N + col] : 0.0f;
+  float mk = 1.0f;
+  if (g.mask) {
+    const int blk = col / g.block;
+    mk = (blk < g.n_blocks && g.mask[blk]) ? 1.0f : 0.0f;
+  }
+#pragma unroll
+  for (int i = 0; i < RT; ++i) {
+    const int row = m0 + i * 16 + q * 4;
+    int b = row / g.T, t = row - b * g.T;
+    long o[4];
+    float gv[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      o[e] = row + e < g.M ? (((long)b * g.h + hh) * g.T + t) * g.N + col : -1;
+      if (++t == g.T) { t = 0; ++b; }
+    }
+    if (g.gate) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) gv[e] = g.gate[o[e] >= 0 ? o[e] : 0];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float pv = acc[i][e];
+      if (g.bias) pv = pv + bv;
+      if (g.thr != 0.0f) pv = pv - g.thr;
+      float y = pv > 0.0f ? pv : 0.0f;
+      if (g.mask) y = y * mk;
+      if (g.gate) y = gv[e] * y;
+      if (o[e] >= 0) g.C[o[e]] = y;
+    }
+  }
+}
+
+// any d and N: 64 x 64 tiles staged through registers, with checks
+__global__ __launch_bounds__(256) void k_relu_lowrank_gemm(RlArgs g) {
+  constexpr int BM = 64, BN = 64;
+  using Tl = RlTile<BM, BN, 2, 2>;
+  __shared__ __attribute__((aligned(16))) float s_a[BM * FLD];
+  __shared__ __attribute__((aligned(16))) float s_b[FK * (BN + 32)];
+  Tl t;
+  if (!t.init(g)) return;
+  const int tid = threadIdx.x, lane = t.lane;
+  const float *W = g.W + (long)t.hh * g.d * g.N;
+  const int K = g.d;
+  const float *pa = t.a_row(g, t.m0 + (tid >> 2));
+  const int kb = tid >> 4, nc = (tid & 15) * 4;
+  f32x16 acc[1][1];
+#pragma unroll
+  for (int e = 0; e < 16; ++e) acc[0][0][e] = 0.0f;
+  float ra[4], rb[4];
+  auto load = [&](int k0) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int k = k0 + (tid & 3) * 4 + u;
+      ra[u] = k < K ? pa[k] : 0.0f;
+      rb[u] = k0 + kb < K ? W[(long)(k0 + kb) * g.N + min(t.n0 + nc + u, g.N - 1)] : 0.0f;
+    }
+  };
+  load(0);
+  for (int k0 = 0; k0 < K; k0 += FK) {
+    __syncthreads();  // the previous step's fragment reads are done
+    // k = kc, kc + 2 to places kc / 2, kc / 2 + 1 of a row; k = kc + 1, kc + 3 to places 8 + kc / 2, ...: the two
+    // 16-byte reads below then give a half-wave k = 2 q + half
+    float *sa = s_a + (tid >> 2) * FLD + (tid & 3) * 2;
+    sa[0] = ra[0]; sa[1] = ra[2]; sa[8] = ra[1]; sa[9] = ra[3];
+    *reinterpret_cast<float4 *>(s_b + kb * (BN + 32) + nc) = make_float4(rb[0], rb[1], rb[2], rb[3]);
+    __syncthreads();
+    if (k0 + FK < K) load(k0 + FK);
+    const int r = lane & 31, half = lane >> 5;
+    const float *p = s_a + (t.wm * 32 + r) * FLD + half * 8;
+    const float *q = s_b + half * (BN + 32) + t.wn * 32 + r;
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(p[u], q[2 * u * (BN + 32)], acc[0][0], 0, 0, 0);
+  }
+  t.finish(g, acc);
+}
+
+// the scores product and, when its K is cut into parts, their reduction
+int launch_scores(bdh_ctx *ctx, const GemmF32 &g, const GemmPlan &plan, float *parts) {
+  const int rc = bdh_launch_gemm_f32(ctx, g, false, false, plan, parts);
+  if (rc != BDH_OK || plan.ks == 1) return rc;
+  GemmF32 r = g;
+  r.ks = plan.ks;
+  hipLaunchKernelGGL(k_scores_reduce, dim3((unsigned)((long)g.n_slices * g.M)), dim3(256), 0, ctx->stream, parts,
+                     (long)g.n_slices * g.M * g.N, r);
+  BDH_LAUNCH_CHECK(ctx, "k_scores_reduce");
+  return BDH_OK;
 }
 
 }  // namespace
@@ -617,16 +672,38 @@ extern "C" int bdh_fused_state_aligned(bdh_ctx *ctx, int B, int h, int T, int N,
   if (S * T > 0x7fffffffL || (S + 7) / 8 * 8 * (long)(((T + 127) / 128) * ((T + 127) / 128)) > 0x7fffffffL) return bdh_fail(ctx, BDH_E_SHAPE, "B*h*T too large");
 
   const int Tp = (T + 3) & ~3;  // row stride of the score matrix
-  const size_t q_bytes = bdh_align_up(sizeof(float) * (size_t)S * T * Nq, 256);
-  const size_t act_bytes = sparse ? bdh_align_up((size_t)tb * tb, 256) : 0;
+  FsaSlopes slopes_dev{};
+  if (alibi_slopes_host) memcpy(slopes_dev.v, alibi_slopes_host, sizeof(float) * h);
+  // the two products of the matrix-core path: S = mask(Q Q^T) + bias, then (S V) / (sum |S| + eps)
+  GemmF32 g, o;
+  GemmPlan plan_g, plan_o;
+  size_t part_bytes = 0;
+  if (path == 1) {
+    g.epilogue = GEMM_SCORES;
+    g.a_s1 = g.b_s1 = (long)T * Nq; g.c_s1 = (long)T * Tp;
+    g.lda = g.ldb = Nq; g.ldc = Tp; g.M = g.N = T; g.K = Nq; g.n_slices = (int)S; g.heads = h;
+    g.block_size = block_size; g.tb = tb; g.use_alibi = alibi_slopes_host != nullptr;
+    memcpy(g.slopes, slopes_dev.v, sizeof(g.slopes));
+    g.sparse_pattern = sparse;
+    o.epilogue = row_normalize ? GEMM_NORM : GEMM_STORE;
+    o.mod = h;
+    o.a_s1 = (long)h * T * Tp; o.a_s2 = (long)T * Tp; o.b_s1 = (long)T * dv; o.c_s1 = (long)h * T * dv; o.c_s2 = (long)T * dv;
+    o.lda = Tp; o.ldb = dv; o.ldc = dv; o.M = T; o.N = dv; o.K = T; o.n_slices = (int)S; o.heads = h;
+    o.block_size = block_size; o.causal_k = !sparse;
+    plan_o = bdh_gemm_f32_plan(ctx, o, 1);
+    g.reader_rows = bdh_gemm_f32_rows(plan_o);
+    const size_t one = sizeof(float) * (size_t)S * T * T;
+    plan_g = bdh_gemm_f32_plan(ctx, g, (int)std::min<size_t>(16, (size_t(256) << 20) / one));
+    if (plan_g.ks > 1) part_bytes = bdh_align_up(one * plan_g.ks, 256);
+  }
+  const size_t q_bytes = rotary == BDH_ALIBI ? 0 : bdh_align_up(sizeof(float) * (size_t)S * T * Nq, 256);
   const size_t sc_bytes = path == 1 ? bdh_align_up(sizeof(float) * (size_t)S * T * Tp, 256) : 0;
-  const size_t nm_bytes = path == 1 ? bdh_align_up(sizeof(float) * (size_t)S * T, 256) : 0;
-  int rc = bdh_ws_reserve(ctx, q_bytes + sc_bytes + nm_bytes);
+  int rc = bdh_ws_reserve(ctx, q_bytes + sc_bytes + part_bytes);
   if (rc != BDH_OK) return rc;
   char *ws = static_cast<char *>(ctx->ws);
-  float *q = reinterpret_cast<float *>(ws);
+  float *rotated = reinterpret_cast<float *>(ws);
   float *scores = reinterpret_cast<float *>(ws + q_bytes);
-  float *norm = reinterpret_cast<float *>(ws + q_bytes + sc_bytes);
+  float *parts = reinterpret_cast<float *>(ws + q_bytes + sc_bytes);
   // The time-block mask of a sparse pattern lives in memory the context owns and is uploaded only when the
   // pattern differs from the one already there (a model calls with the same pattern every time): no copy and
   // no host synchronisation on the usual call.  The ALiBi slopes travel as a kernel argument.
@@ -659,48 +736,18 @@ extern "C" int bdh_fused_state_aligned(bdh_ctx *ctx, int B, int h, int T, int N,
     }
     active = static_cast<unsigned char *>(ctx->fsa_mask);
   }
-  FsaSlopes slopes_dev{};
-  if (alibi_slopes_host) memcpy(slopes_dev.v, alibi_slopes_host, sizeof(float) * h);
-  hipLaunchKernelGGL(k_rotate_f32, dim3((unsigned)(S * T)), dim3(256), 0, ctx->stream, query, freqs, q, T, N, rotary);
-  BDH_LAUNCH_CHECK(ctx, "k_rotate_f32");
+  const float *q = query;  // ALiBi does not rotate
+  if (rotary != BDH_ALIBI) {
+    hipLaunchKernelGGL(k_rotate_f32, dim3((unsigned)(S * T)), dim3(256), 0, ctx->stream, query, freqs, rotated, T, N, rotary);
+    BDH_LAUNCH_CHECK(ctx, "k_rotate_f32");
+    q = rotated;
+  }
   if (path == 1) {
-    FsaArgs g{};
-    g.A = q; g.Bm = q; g.C = scores;
-    g.a_batch = g.b_batch = (long)T * Nq; g.c_batch = (long)T * Tp;
-    g.lda = g.ldb = Nq; g.ldc = Tp; g.M = g.N = T; g.K = Nq; g.b_div = 1; g.n_slices = (int)S;
-    g.block_size = block_size; g.tb = tb; g.h = h; g.use_alibi = alibi_slopes_host ? 1 : 0; g.dense = sparse ? 0 : 1;
-    g.active = active; g.norm = nullptr;
-    memcpy(g.slopes, slopes_dev.v, sizeof(g.slopes));
-    // big tiles once there are enough of them to cover the chip; small ones for short sequences
-    const bool big = (long)S * ((T + 255) / 256) * ((T + 255) / 256) >= 256;
-    const unsigned groups = (unsigned)((S + 7) / 8);
-    if (big) {
-      g.mt = g.nt = (T + 255) / 256;
-      hipLaunchKernelGGL((k_fsa_gemm_f32<0, false, false, 256, 256, 2, 4, false, true>), dim3(8 * groups * g.mt * g.nt), dim3(512), 0,
-                         ctx->stream, g);
-    } else {
-      g.mt = g.nt = (T + 127) / 128;
-      hipLaunchKernelGGL((k_fsa_gemm_f32<0, false, false, 128, 128, 2, 2, false, true>), dim3(8 * groups * g.mt * g.nt), dim3(256), 0,
-                         ctx->stream, g);
-    }
-    BDH_LAUNCH_CHECK(ctx, "k_fsa_gemm_f32<scores>");
-    if (row_normalize) {
-      hipLaunchKernelGGL(k_fsa_row_abs_sum, dim3((unsigned)((S * T + 3) / 4)), dim3(256), 0, ctx->stream, scores,
-                         S * T, T, Tp, norm);
-      BDH_LAUNCH_CHECK(ctx, "k_fsa_row_abs_sum");
-    }
-    FsaArgs o{};
-    o.A = scores; o.Bm = value; o.C = out;
-    o.a_batch = (long)T * Tp; o.b_batch = (long)T * dv; o.c_batch = (long)T * dv;
-    o.lda = Tp; o.ldb = dv; o.ldc = dv; o.M = T; o.N = dv; o.K = T; o.b_div = h; o.n_slices = (int)S;
-    o.block_size = block_size; o.tb = tb; o.h = h; o.dense = sparse ? 0 : 1;
-    o.norm = row_normalize ? norm : nullptr;
-    o.mt = (T + 127) / 128;
-    o.nt = (dv + 127) / 128;
-    hipLaunchKernelGGL((k_fsa_gemm_f32<1, false, true, 128, 128, 2, 2, false, true>), dim3(8 * groups * o.mt * o.nt), dim3(256), 0,
-                       ctx->stream, o);
-    BDH_LAUNCH_CHECK(ctx, "k_fsa_gemm_f32<out>");
-    return BDH_OK;
+    g.A = g.B = q; g.C = scores; g.active = active;
+    rc = launch_scores(ctx, g, plan_g, parts);
+    if (rc != BDH_OK) return rc;
+    o.A = scores; o.B = value; o.C = out;
+    return bdh_launch_gemm_f32(ctx, o, false, true, plan_o, nullptr);
   }
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_fsa_row),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -743,33 +790,80 @@ int bdh_launch_state_chunks_f32(bdh_ctx *ctx, const StateStepParams &p, float *o
   Tc = std::min<long>(512, std::max<long>(128, Tc));
   Tc = std::min<long>(Tc, T);
   const int Tcp = ((int)Tc + 3) & ~3;
+  if (S * Tc > 0x7fffffffL) return bdh_fail(ctx, BDH_E_SHAPE, "B*h*T too large");
+  // the products of a chunk of tc tokens; what differs from chunk to chunk is filled in below
+  auto with_decay = [&](GemmF32 &g) {
+    g.heads = h;
+    if (alibi) memcpy(g.log_decay, log_decay, sizeof(g.log_decay));
+  };
+  struct Chunk {
+    GemmF32 scores, out, state;
+    GemmPlan p_scores, p_out, p_state;
+    size_t parts_bytes = 0;
+  };
+  auto chunk_of = [&](int tc, long q_batch) {
+    Chunk c;
+    GemmF32 &g = c.scores;  // S = tril(-1)(Q Q^T)   (ALiBi: S[t,s] *= decay^(t-s))
+    g.epilogue = GEMM_SCORES;
+    g.a_s1 = g.b_s1 = q_batch; g.c_s1 = (long)Tc * Tcp;
+    g.lda = g.ldb = Nq; g.ldc = Tcp; g.M = g.N = tc; g.K = Nq; g.n_slices = (int)S;
+    with_decay(g);
+    g.decay_scores = alibi;
+    // out = Q rho + S V   (the state before this chunk; S limited to the causal prefix of each row tile; ALiBi: the
+    // first term's row t *= decay^t)
+    GemmF32 &o = c.out;
+    o.mod = h;
+    o.a_s1 = h * q_batch; o.a_s2 = q_batch; o.b_s1 = (long)h * Nq * d; o.b_s2 = (long)Nq * d;
+    o.c_s1 = (long)h * T * d; o.c_s2 = (long)T * d;
+    o.lda = Nq; o.ldb = d; o.ldc = d; o.M = tc; o.N = d; o.K = Nq; o.n_slices = (int)S;
+    o.a2_s1 = (long)h * Tc * Tcp; o.a2_s2 = (long)Tc * Tcp; o.b2_s1 = (long)T * d; o.lda2 = Tcp; o.ldb2 = d; o.K2 = tc;
+    o.causal_k = true;
+    with_decay(o);
+    o.decay_rows = alibi;
+    // rho += Q^T V   (both operands k-major: the reduction runs over the tokens; ALiBi: rho = decay^tc rho +
+    // sum_s decay^(tc-s) q_s (x) v_s)
+    GemmF32 &r = c.state;
+    r.mod = h;
+    r.a_s1 = h * q_batch; r.a_s2 = q_batch; r.b_s1 = (long)T * d; r.c_s1 = (long)h * Nq * d; r.c_s2 = (long)Nq * d;
+    r.lda = Nq; r.ldb = d; r.ldc = d; r.M = Nq; r.N = d; r.K = tc; r.n_slices = (int)S;
+    r.accumulate = true;
+    with_decay(r);
+    r.decay_state = alibi;
+    const size_t most = size_t(256) << 20;
+    const size_t one_s = sizeof(float) * (size_t)S * tc * tc, one_o = sizeof(float) * (size_t)S * tc * d;
+    o.A2 = reinterpret_cast<const float *>(1);  // counts K2 in the plan; set below
+    c.p_out = bdh_gemm_f32_plan(ctx, o, (int)std::min<size_t>(32, std::max<size_t>(1, most / one_o)));
+    g.reader_rows = bdh_gemm_f32_rows(c.p_out);
+    c.p_scores = bdh_gemm_f32_plan(ctx, g, (int)std::min<size_t>(32, std::max<size_t>(1, most / one_s)));
+    c.p_state = bdh_gemm_f32_plan(ctx, r, 1);
+    // the parts of the scores are used up before those of the readout are written
+    c.parts_bytes = std::max(c.p_scores.ks > 1 ? one_s * c.p_scores.ks : 0, c.p_out.ks > 1 ? one_o * c.p_out.ks : 0);
+    return c;
+  };
+  const int tc_last = T % Tc ? T % (int)Tc : (int)Tc;
+  const size_t parts_bytes = bdh_align_up(std::max(chunk_of((int)Tc, 0).parts_bytes, chunk_of(tc_last, 0).parts_bytes), 256);
   const size_t q_bytes = alibi ? 0 : bdh_align_up(per_token * (size_t)Tc, 256);  // ALiBi does not rotate: q = x
   const size_t sc_bytes = bdh_align_up(sizeof(float) * (size_t)S * Tc * Tcp, 256);
   // a bf16 state is widened to f32 for the call and rounded back once at its end (the token loop rounds
   // after every token)
   const size_t n_state = (size_t)S * Nq * d;
   const size_t wide_bytes = bf16_state ? bdh_align_up(sizeof(float) * n_state, 256) : 0;
-  int rc = bdh_ws_reserve(ctx, q_bytes + sc_bytes + wide_bytes);
+  int rc = bdh_ws_reserve(ctx, q_bytes + sc_bytes + parts_bytes + wide_bytes);
   if (rc != BDH_OK) return rc;
-  float *q = static_cast<float *>(ctx->ws);
-  float *scores = reinterpret_cast<float *>(static_cast<char *>(ctx->ws) + q_bytes);
+  char *ws = static_cast<char *>(ctx->ws);
+  float *q = reinterpret_cast<float *>(ws);
+  float *scores = reinterpret_cast<float *>(ws + q_bytes);
+  float *parts = reinterpret_cast<float *>(ws + q_bytes + sc_bytes);
   float *rho = static_cast<float *>(p.rho);
   if (bf16_state) {
-    rho = reinterpret_cast<float *>(static_cast<char *>(ctx->ws) + q_bytes + sc_bytes);
+    rho = reinterpret_cast<float *>(ws + q_bytes + sc_bytes + parts_bytes);
     hipLaunchKernelGGL(k_widen_bf16, dim3((unsigned)std::min<size_t>((n_state + 255) / 256, 1u << 20)), dim3(256), 0,
                        ctx->stream, static_cast<const unsigned short *>(p.rho), rho, n_state);
     BDH_LAUNCH_CHECK(ctx, "k_widen_bf16");
   }
-  const unsigned groups = (unsigned)((S + 7) / 8);
-  const int nt_d = (d + 127) / 128;
-  if ((long)groups * 8 * ((Nq + 127) / 128) * nt_d > 0x7fffffffL) return bdh_fail(ctx, BDH_E_SHAPE, "too many tiles");
-
-  const int n_cu = ctx->n_cu > 0 ? ctx->n_cu : 256;
+  bool normed = false;
   for (int t0 = 0; t0 < T; t0 += (int)Tc) {
     const int tc = (int)std::min<long>(Tc, T - t0);
-    // a small model or a short call: with 128 x 128 tiles the products would run on a few CUs, each a chain of
-    // load latencies; 32 x 64 tiles give sixteen times the workgroups
-    const bool small_tiles = (long)8 * groups * ((tc + 127) / 128) * nt_d < n_cu;
     const float *qc = q;           // this chunk's rotated activations [S][tc][Nq]
     long q_batch = (long)tc * Nq;
     if (alibi) {
@@ -780,88 +874,23 @@ int bdh_launch_state_chunks_f32(bdh_ctx *ctx, const StateStepParams &p, float *o
                          (long)T * N, p.freqs, q, tc, N, p.rotary, (long)(p.position + t0), p.positions_dev, t0, h);
       BDH_LAUNCH_CHECK(ctx, "k_rotate_chunk_f32");
     }
-    auto with_decay = [&](FsaArgs &g, int mode) {
-      if (!alibi) return;
-      g.decay_mode = mode;
-      memcpy(g.log_decay, log_decay, sizeof(log_decay));
-    };
-    {  // S = tril(-1)(Q Q^T)   (ALiBi: S[t,s] *= decay^(t-s))
-      FsaArgs g{};
-      g.A = qc; g.Bm = qc; g.C = scores;
-      g.a_batch = g.b_batch = q_batch; g.c_batch = (long)Tc * Tcp;
-      g.lda = g.ldb = Nq; g.ldc = Tcp; g.M = g.N = tc; g.K = Nq; g.b_div = 1; g.n_slices = (int)S;
-      g.block_size = 1; g.tb = tc; g.h = h; g.use_alibi = 0; g.dense = 1;
-      with_decay(g, FSA_DECAY_SCORES);
-      const bool big = S * ((tc + 255) / 256) * ((tc + 255) / 256) >= 256;
-      if (small_tiles) {
-        g.mt = (tc + 31) / 32; g.nt = (tc + 63) / 64;
-        hipLaunchKernelGGL((k_fsa_gemm_f32<0, false, false, 32, 64, 1, 2>), dim3(8 * groups * g.mt * g.nt), dim3(128),
-                           0, ctx->stream, g);
-      } else if (big) {
-        g.mt = g.nt = (tc + 255) / 256;
-        hipLaunchKernelGGL((k_fsa_gemm_f32<0, false, false, 256, 256, 2, 4, false, true>), dim3(8 * groups * g.mt * g.nt), dim3(512),
-                           0, ctx->stream, g);
-      } else {
-        g.mt = g.nt = (tc + 127) / 128;
-        hipLaunchKernelGGL((k_fsa_gemm_f32<0, false, false, 128, 128, 2, 2, false, true>), dim3(8 * groups * g.mt * g.nt), dim3(256),
-                           0, ctx->stream, g);
-      }
-      BDH_LAUNCH_CHECK(ctx, "k_fsa_gemm_f32<chunk scores>");
+    Chunk c = chunk_of(tc, q_batch);
+    c.scores.A = c.scores.B = qc; c.scores.C = scores;
+    rc = launch_scores(ctx, c.scores, c.p_scores, parts);
+    if (rc != BDH_OK) return rc;
+    c.out.A = qc; c.out.B = rho; c.out.A2 = scores; c.out.B2 = p.v + (long)t0 * d; c.out.C = p.out + (long)t0 * d;
+    rc = bdh_launch_gemm_f32(ctx, c.out, false, true, c.p_out, parts);
+    if (rc != BDH_OK) return rc;
+    if (c.p_out.ks > 1) {
+      const long rows = S * tc;
+      hipLaunchKernelGGL(k_rows_reduce, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, ctx->stream, parts, c.p_out.ks,
+                         rows * d, tc, d, rows, p.out + (long)t0 * d, out_ln ? out_ln + (long)t0 * d : nullptr, (long)T * d);
+      BDH_LAUNCH_CHECK(ctx, "k_rows_reduce");
+      normed = tc == T;
     }
-    {  // out = Q rho   (the state before this chunk; B = rho [Nq,d] is k-major; ALiBi: row t *= decay^t)
-      FsaArgs g{};
-      g.A = qc; g.Bm = rho; g.C = p.out + (long)t0 * d;
-      g.a_batch = q_batch; g.b_batch = (long)Nq * d; g.c_batch = (long)T * d;
-      g.lda = Nq; g.ldb = d; g.ldc = d; g.M = tc; g.N = d; g.K = Nq; g.b_div = 1; g.n_slices = (int)S;
-      g.block_size = 1; g.h = h; g.dense = 0; g.beta = 0;
-      with_decay(g, FSA_DECAY_ROWS);
-      if (small_tiles) {
-        g.mt = (tc + 31) / 32; g.nt = (d + 63) / 64;
-        hipLaunchKernelGGL((k_fsa_gemm_f32<2, false, true, 32, 64, 1, 2>), dim3(8 * groups * g.mt * g.nt), dim3(128), 0,
-                           ctx->stream, g);
-      } else {
-        g.mt = (tc + 127) / 128; g.nt = nt_d;
-        hipLaunchKernelGGL((k_fsa_gemm_f32<2, false, true, 128, 128, 2, 2, false, true>), dim3(8 * groups * g.mt * g.nt), dim3(256), 0,
-                           ctx->stream, g);
-      }
-      BDH_LAUNCH_CHECK(ctx, "k_fsa_gemm_f32<Q rho>");
-    }
-    {  // out += S V   (K limited to the causal prefix of each row tile)
-      FsaArgs g{};
-      g.A = scores; g.Bm = p.v + (long)t0 * d; g.C = p.out + (long)t0 * d;
-      g.a_batch = (long)Tc * Tcp; g.b_batch = (long)T * d; g.c_batch = (long)T * d;
-      g.lda = Tcp; g.ldb = d; g.ldc = d; g.M = tc; g.N = d; g.K = tc; g.b_div = h; g.n_slices = (int)S;
-      g.block_size = 1; g.h = h; g.dense = 1; g.beta = 1;
-      if (small_tiles) {
-        g.mt = (tc + 31) / 32; g.nt = (d + 63) / 64;
-        hipLaunchKernelGGL((k_fsa_gemm_f32<2, false, true, 32, 64, 1, 2>), dim3(8 * groups * g.mt * g.nt), dim3(128), 0,
-                           ctx->stream, g);
-      } else {
-        g.mt = (tc + 127) / 128; g.nt = nt_d;
-        hipLaunchKernelGGL((k_fsa_gemm_f32<2, false, true, 128, 128, 2, 2, false, true>), dim3(8 * groups * g.mt * g.nt), dim3(256), 0,
-                           ctx->stream, g);
-      }
-      BDH_LAUNCH_CHECK(ctx, "k_fsa_gemm_f32<S V>");
-    }
-    {  // rho += Q^T V   (both operands k-major: the reduction runs over the tokens)
-       // ALiBi: rho = decay^tc * rho + sum_s decay^(tc-s) q_s (x) v_s
-      FsaArgs g{};
-      g.A = qc; g.Bm = p.v + (long)t0 * d; g.C = rho;
-      g.a_batch = q_batch; g.b_batch = (long)T * d; g.c_batch = (long)Nq * d;
-      g.lda = Nq; g.ldb = d; g.ldc = d; g.M = Nq; g.N = d; g.K = tc; g.b_div = h; g.n_slices = (int)S;
-      g.block_size = 1; g.h = h; g.dense = 0; g.beta = 1;
-      with_decay(g, FSA_DECAY_STATE);
-      if (small_tiles) {
-        g.mt = (Nq + 31) / 32; g.nt = (d + 63) / 64;
-        hipLaunchKernelGGL((k_fsa_gemm_f32<2, true, true, 32, 64, 1, 2>), dim3(8 * groups * g.mt * g.nt), dim3(128), 0,
-                           ctx->stream, g);
-      } else {
-        g.mt = (Nq + 127) / 128; g.nt = nt_d;
-        hipLaunchKernelGGL((k_fsa_gemm_f32<2, true, true, 128, 128, 2, 2, false, true>), dim3(8 * groups * g.mt * g.nt), dim3(256), 0,
-                           ctx->stream, g);
-      }
-      BDH_LAUNCH_CHECK(ctx, "k_fsa_gemm_f32<Q^T V>");
-    }
+    c.state.A = qc; c.state.B = p.v + (long)t0 * d; c.state.C = rho;
+    rc = bdh_launch_gemm_f32(ctx, c.state, true, true, c.p_state, nullptr);
+    if (rc != BDH_OK) return rc;
   }
   if (bf16_state) {
     hipLaunchKernelGGL(k_narrow_bf16, dim3((unsigned)std::min<size_t>((n_state + 255) / 256, 1u << 20)), dim3(256), 0,
@@ -874,31 +903,33 @@ int bdh_launch_state_chunks_f32(bdh_ctx *ctx, const StateStepParams &p, float *o
                        (long)h * N, (long)(p.position + T), p.positions_dev, T);
     BDH_LAUNCH_CHECK(ctx, "k_set_stamps");
   }
-  if (out_ln) return bdh_launch_layer_norm_rows(ctx, (int64_t)S * T, d, p.out, out_ln);
+  if (out_ln && !normed) return bdh_launch_layer_norm_rows(ctx, (int64_t)S * T, d, p.out, out_ln);
   return BDH_OK;
 }
 
-// The encoder E over many rows (src/model/bdh.rs:383,436-438): mixed [B*T, h*N] . decoder [h*N, d], as one
-// product per (sequence, head) on the f32 matrix cores.  partial [h][B*T][d] receives the h per-head terms
-// of every output row; the caller sums them in head order.
-int bdh_launch_decoder_partials_f32(bdh_ctx *ctx, int B, int T, int h, int N, int d, const float *xy,
-                                    const float *decoder, float *partial) {
-  const long S = (long)B * h;
-  const unsigned groups = (unsigned)((S + 7) / 8);
-  FsaArgs g{};
-  g.A = xy; g.Bm = decoder; g.C = partial;
-  g.mod = h;
-  g.a_batch = (long)h * T * N; g.a_mod_stride = (long)T * N;  // xy [B,h,T,N]
-  g.b_batch = 0; g.b_mod_stride = (long)N * d;                // decoder rows hh*N .. hh*N+N-1
-  g.c_batch = (long)T * d; g.c_mod_stride = (long)B * T * d;
-  g.lda = N; g.ldb = d; g.ldc = d; g.M = T; g.N = d; g.K = N; g.b_div = 1; g.n_slices = (int)S;
-  g.block_size = 1; g.h = h; g.dense = 0; g.beta = 0;
-  g.mt = (T + 127) / 128; g.nt = (d + 127) / 128;
-  if ((long)groups * 8 * g.mt * g.nt > 0x7fffffffL) return bdh_fail(ctx, BDH_E_SHAPE, "too many tiles");
-  hipLaunchKernelGGL((k_fsa_gemm_f32<2, false, true, 128, 128, 2, 2, false, true>), dim3(8 * groups * g.mt * g.nt), dim3(256), 0,
-                     ctx->stream, g);
-  BDH_LAUNCH_CHECK(ctx, "k_fsa_gemm_f32<decoder>");
-  return BDH_OK;
+// The encoder E over many rows (src/model/bdh.rs:383,436-438): mixed [B*T, h*N] . decoder [h*N, d] as one product per head
+// (T = 1: mixed is contiguous per sequence, one product), K cut into as many parts as the chip wants.
+// partial [*rows_out][B*T][d] receives the terms of every output row; the caller sums them in order.
+int bdh_launch_decoder_partials_f32(bdh_ctx *ctx, int B, int T, int h, int N, int d, const float *xy, const float *decoder,
+                                    int *rows_out) {
+  GemmF32 g;
+  g.A = xy; g.B = decoder;
+  g.lda = N; g.ldb = d; g.ldc = d; g.M = B * T; g.N = d;
+  if (T == 1) {
+    g.lda = g.K = h * N;
+  } else {
+    g.K = N; g.n_slices = h; g.mod = h;
+    g.a_s2 = (long)T * N; g.b_s2 = (long)N * d; g.c_s2 = (long)B * T * d;
+    g.rows_per = T; g.a_outer = (long)h * T * N;
+    g.c_outer = (long)T * d;
+  }
+  const size_t one = sizeof(float) * (size_t)g.n_slices * g.M * d;
+  const GemmPlan plan = bdh_gemm_f32_plan(ctx, g, (int)std::min<size_t>(64, std::max<size_t>(1, (size_t(256) << 20) / one)));
+  int rc = bdh_ws_reserve(ctx, one * plan.ks);
+  if (rc != BDH_OK) return rc;
+  g.C = static_cast<float *>(ctx->ws);
+  *rows_out = g.n_slices * plan.ks;
+  return bdh_launch_gemm_f32(ctx, g, false, true, plan, g.C);
 }
 
 extern "C" int bdh_rotate(bdh_ctx *ctx, int B, int h, int T, int N, int rotary, const float *x, const float *freqs,
@@ -926,73 +957,53 @@ extern "C" int bdh_rotate(bdh_ctx *ctx, int B, int h, int T, int N, int rotary, 
   return BDH_OK;
 }
 
-// The encoder E of a decode step for a batch of sequences (T = 1, src/model/bdh.rs:383,436-438): mixed [B, h*N] is
-// contiguous per sequence, so the product is one [B x K] . [K x d] GEMM split over K: slice s takes k in
-// [s*KB, (s+1)*KB) and writes partial[s][B][d].  With 8 or more sequences nearly every row of E is needed by some
-// sequence, so the weights are streamed once through the matrix cores instead of skipping inactive rows.
-int bdh_launch_decoder_splitk_f32(bdh_ctx *ctx, int M, long K, int d, int KB, const float *xy, const float *decoder,
-                                  float *partial) {
-  const long KBN = (K + KB - 1) / KB;
-  const unsigned groups = (unsigned)((KBN + 7) / 8);
-  FsaArgs g{};
-  g.A = xy; g.Bm = decoder; g.C = partial;
-  g.a_batch = KB; g.b_batch = (long)KB * d; g.c_batch = (long)M * d;
-  g.lda = (int)K; g.ldb = d; g.ldc = d; g.M = M; g.N = d; g.K = KB; g.b_div = 1; g.n_slices = (int)KBN;
-  g.block_size = 1; g.h = 1; g.dense = 0; g.beta = 0;
-  g.mt = (M + 31) / 32; g.nt = (d + 63) / 64;
-  if (K % KB != 0) return bdh_fail(ctx, BDH_E_SHAPE, "split-K block %d does not divide K=%ld", KB, K);
-  if ((long)groups * 8 * g.mt * g.nt > 0x7fffffffL) return bdh_fail(ctx, BDH_E_SHAPE, "too many tiles");
-  hipLaunchKernelGGL((k_fsa_gemm_f32<2, false, true, 32, 64, 1, 2>), dim3(8 * groups * g.mt * g.nt), dim3(128), 0,
-                     ctx->stream, g);
-  BDH_LAUNCH_CHECK(ctx, "k_fsa_gemm_f32<decoder split-K>");
-  return BDH_OK;
-}
-
-// relu_lowrank for many rows per (sequence, head) on the f32 matrix cores: one product [T, d] x [d, N] per slice with
-// the k order of a scalar loop (SEQK), so the outputs are the bits of k_relu_lowrank.  mask_dev: one byte per latent
-// block in device memory, or null.
+// relu_lowrank for many rows on the f32 matrix cores with the k order of a scalar loop, so the outputs are the bits of
+// k_relu_lowrank.  mask_dev: one byte per latent block in device memory, or null.
 int bdh_launch_relu_lowrank_gemm(bdh_ctx *ctx, const ReluLowrankParams &p, const unsigned char *mask_dev) {
-  FsaArgs g{};
+  RlArgs g{};
   g.A = p.in;
-  g.Bm = p.weight;
+  g.W = p.weight;
   g.C = p.out;
-  g.mod = p.h;                                   // slice = b * h + head
-  g.a_batch = (long)p.h_in * p.T * p.d;
-  g.a_mod_stride = p.h_in == 1 ? 0 : (long)p.T * p.d;
-  g.b_batch = 0;
-  g.b_mod_stride = (long)p.d * p.N;
-  g.c_batch = (long)p.h * p.T * p.N;
-  g.c_mod_stride = (long)p.T * p.N;
-  g.lda = p.d;
-  g.ldb = p.N;
-  g.ldc = p.N;
-  g.M = p.T;
+  g.T = p.T;
+  g.a_outer = (long)p.h_in * p.T * p.d;
+  g.a_head = p.h_in == 1 ? 0 : (long)p.T * p.d;
+  g.M = p.B * p.T;
   g.N = p.N;
-  g.K = p.d;
-  g.b_div = 1;
-  g.n_slices = p.B * p.h;
-  g.block_size = 1;
+  g.d = p.d;
   g.h = p.h;
-  g.rl_bias = p.bias;
-  g.rl_thr = p.threshold;
-  g.rl_mask = mask_dev;
-  g.rl_block = p.block_size > 0 ? p.block_size : 1;
-  g.rl_nblocks = p.n_blocks;
-  g.rl_gate = p.gate;
-  const int groups = (g.n_slices + 7) / 8;
-  // 128 x 128 tiles: K = d is short (a 256 x 256 tile spends as long in its prologue and 256 KiB epilogue as in its
-  // 32 k stages: 12.1 against 10.8 ms for [8192 x 512] x [512 x 131072])
-  // 128 x 256 tiles for wide matrices: 10.8 -> 10.1 ms for [8192 x 512] x [512 x 131072]
-  g.mt = (p.T + 127) / 128;
-  const bool wide = p.N % 256 == 0 && (long)p.B * p.h * g.mt * (p.N / 256) >= 2L * (ctx->n_cu > 0 ? ctx->n_cu : 256);
-  g.nt = wide ? p.N / 256 : (p.N + 127) / 128;
-  if ((long)8 * groups * g.mt * g.nt > 0x7fffffffL) return bdh_fail(ctx, BDH_E_SHAPE, "too many tiles");
-  if (wide)
-    hipLaunchKernelGGL((k_fsa_gemm_f32<3, false, true, 128, 256, 2, 4, true>), dim3(8 * groups * g.mt * g.nt), dim3(512), 0,
-                       ctx->stream, g);
-  else
-    hipLaunchKernelGGL((k_fsa_gemm_f32<3, false, true, 128, 128, 2, 2, true>), dim3(8 * groups * g.mt * g.nt), dim3(256), 0,
-                       ctx->stream, g);
-  BDH_LAUNCH_CHECK(ctx, "k_fsa_gemm_f32<relu_lowrank>");
+  g.bias = p.bias;
+  g.thr = p.threshold;
+  g.mask = mask_dev;
+  g.block = p.block_size > 0 ? p.block_size : 1;
+  g.n_blocks = p.n_blocks;
+  g.gate = p.gate;
+  const long n_cu = ctx->n_cu > 0 ? ctx->n_cu : 256;
+  auto tiles = [&](int bm, int bn) {
+    g.mt = (g.M + bm - 1) / bm;
+    g.nt = (g.N + bn - 1) / bn;
+    return (long)g.h * g.mt * g.nt;
+  };
+  // Narrow tiles (16 rows) while there are no more than four for every CU: the latency of one tile is what counts.  Beyond
+  // that up to 32 and 64 rows in one tile, so that the weights pass once; more rows 64 x 64, and 128 x 128 once there are
+  // four of those for every CU (us, 16-row | 32-row | 64-row | 64 x 64 tiles: [128 x 256] x [256 x 4096] 7.7 | 8.4 | 12.2 |
+  // 10.2, [256 x ..] 11.3 | 10.9 | 12.8 | 11.0, [512 x ..] 18.1 | 17.0 | 17.3 | 16.2; [32 x 512] x [512 x 131072] 67 | 59 | 85 |
+  // 153, [63 x ..] 118 | 100 | 94 | 157; 128 x 128 | 64 x 64: [1536 x 256] x [256 x 32768] 253 | 273, [512 x 512] x
+  // [512 x 20480] 111 | 104)
+  const bool direct = p.d % 32 == 0 && p.N % 4 == 0 && bdh_aligned(p.in, 16) && bdh_aligned(p.weight, 16);
+  const bool big = direct && tiles(128, 128) >= 4 * n_cu;
+  const int rt = !direct ? 0 : g.M <= 16 || tiles(16, 64) <= 4 * n_cu ? 1 : g.M <= 32 ? 2 : g.M <= 64 ? 4 : 0;
+  const long total = rt ? tiles(16 * rt, 64) : big ? tiles(128, 128) : tiles(64, 64);
+  if (total + 8 > 0x7fffffffL) return bdh_fail(ctx, BDH_E_SHAPE, "too many tiles");
+  const dim3 grid((unsigned)(8 * ((total + 7) / 8)));
+#define BDH_RLD(KERNEL_, ROWS_, COLS_) \
+  hipLaunchKernelGGL((KERNEL_), grid, dim3(256), 2 * (ROWS_ + COLS_) * 32 * sizeof(float), ctx->stream, g)
+  if (rt == 1) BDH_RLD(k_relu_lowrank_rows<1>, 16, 64);
+  else if (rt == 2) BDH_RLD(k_relu_lowrank_rows<2>, 32, 64);
+  else if (rt == 4) BDH_RLD(k_relu_lowrank_rows<4>, 64, 64);
+  else if (big) BDH_RLD((k_relu_lowrank_direct<128, 128>), 128, 128);
+  else if (direct) BDH_RLD((k_relu_lowrank_direct<64, 64>), 64, 64);
+  else hipLaunchKernelGGL(k_relu_lowrank_gemm, grid, dim3(256), 0, ctx->stream, g);
+#undef BDH_RLD
+  BDH_LAUNCH_CHECK(ctx, "k_relu_lowrank_gemm");
   return BDH_OK;
 }

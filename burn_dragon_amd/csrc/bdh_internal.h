@@ -23,14 +23,12 @@ struct bdh_ctx {
   int n_cu = 0;
   int opt_step_split = -1;  // -1 choose by grid size, 0 / 1 force the 256- / 64-pair workgroup
   int opt_step_dense = -1;  // many-token state step as dense f32 products: -1 from T = 128, 0 never, 1 always
-  int opt_lowrank_tile = 1;  // 0: relu_lowrank never takes the 64-row tile kernel
   int opt_decoder_mfma = 1;  // 0: the encoder E never takes the f32 matrix-core form
   int opt_model_one_launch = 1;  // small model's decode step in one launch: 1 when it pays, 2 whenever it fits, 0 never
   int opt_lowrank_row = 1;     // 0: relu_lowrank with one input row and a small matrix uses the column-per-thread kernel
   int opt_model_phase_batch = 1 << 30;  // two launches per layer for a decode step of at most this many sequences (0: never)
-  int opt_lowrank_gemm_rows = 64;  // relu_lowrank with this many tokens per sequence or more runs as a matrix-core product (0: never)
-  int opt_lowrank_mfma_rows = 8;  // relu_lowrank takes the f32 matrix cores from this many rows on (0: never)
-  int opt_lowrank_scalar = 1;  // 0: relu_lowrank with 8 to 63 rows stages its inputs in LDS instead of scalar loads
+  int opt_lowrank_gemm_rows = 64;  // relu_lowrank of 64 rows and more takes the f32 matrix cores from this many on (0: never)
+  int opt_lowrank_mfma_rows = 2;  // relu_lowrank of fewer than 64 rows takes the f32 matrix cores from this many on (0: never)
   int opt_step_dense_kernel = 1;  // 0: PoPE / eager ALiBi at d in {256,512} take the generic kernel
   int opt_decoder_splitk_rows = 24;  // decode-step encoder on the matrix cores from this many sequences on
   int opt_fsa_path = -1;    // fused_state_aligned: -1 choose by T, 0 row kernel, 1 f32 matrix cores
@@ -218,12 +216,10 @@ int bdh_launch_decoder_residual(bdh_ctx *ctx, int B, int T, int h, int N, int d,
                                 const float *xy, const float *decoder, float *cur,
                                 const DecoderHead *head = nullptr);
 // logits = cur . lm_head (+ argmax of the last token per sequence) (src/model/bdh.rs:446-449)
-// attention_parallel.hip: partial[hh][b*T+t][:] = xy[b,hh,t,:] . decoder[hh*N.., :] on the f32 matrix cores
-int bdh_launch_decoder_partials_f32(bdh_ctx *ctx, int B, int T, int h, int N, int d, const float *xy,
-                                    const float *decoder, float *partial);
-// attention_parallel.hip: decode-step encoder for a batch (T = 1): partial[s][m][:] = xy[m, s*KB..] . decoder[s*KB.., :]
-int bdh_launch_decoder_splitk_f32(bdh_ctx *ctx, int M, long K, int d, int KB, const float *xy, const float *decoder,
-                                  float *partial);
+// attention_parallel.hip: the encoder's terms [*rows_out][B*T][d] in the context's workspace, from products on the matrix
+// cores (all of E is streamed, whatever is active)
+int bdh_launch_decoder_partials_f32(bdh_ctx *ctx, int B, int T, int h, int N, int d, const float *xy, const float *decoder,
+                                    int *rows_out);
 int bdh_launch_lm_head(bdh_ctx *ctx, int B, int T, int d, int V, const float *cur,
                        const float *lm_head, float *logits, int64_t *next_tokens);
 // positions[b] = min(positions[b] + delta, INT32_MAX): the device-side form of state.position += T

@@ -1,0 +1,467 @@
+// Dense f32 products on the bf16 matrix cores (see gemm_f32.h).
+//
+// Every f32 operand is taken as a sum of three bf16 terms h + m + l and a product as six bf16 matrix instructions, so
+// the results carry f32-level accuracy at a sixth of the bf16 rate (417 TFLOP/s against 157 of the f32 instruction).
+// The split is made once per element and workgroup, on the way into LDS: a stage holds 32 k of both tiles as three bf16
+// planes, chunks of eight k of one row (16 bytes) being what a lane feeds to one 32 x 32 x 16 instruction.
+#include "gemm_f32.h"
+
+#include <algorithm>
+
+namespace {
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr float kRowNormEps = 1e-6f;  // src/kernel/linear_attention.rs:9
+constexpr int FK = 32;                // k per LDS stage
+
+// Eight floats as three bf16x8 operands h + m + l that add up to the floats exactly: each term is the remainder so far
+// rounded to bf16 (v_cvt_pk_bf16_f32, round to nearest even); a remainder is a difference of neighbours and therefore
+// exact, and the third one has at most eight significant bits.  A product of two such sums is taken as the six matrix
+// instructions l h, h l, m m, m h, h m, h h (smallest terms first); what is left out (m l, l m, l l) is below 2^-23 of
+// |a b|, the size of one f32 rounding.  An infinite input, or a finite one that rounds to an infinite bf16 (above
+// 3.389e38), gives NaN (inf - inf in the remainder).
+__device__ __forceinline__ void split3(const float (&a)[8], u32x4 &ph, u32x4 &pm, u32x4 &pl) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {  // element 2q in the low half of a dword, 2q + 1 in the high half
+    const f32x2 a2 = {a[2 * q], a[2 * q + 1]};
+    ph[q] = __builtin_bit_cast(unsigned int, __builtin_convertvector(a2, bf16x2));
+    const f32x2 r1 = {a2[0] - __uint_as_float(ph[q] << 16), a2[1] - __uint_as_float(ph[q] & 0xffff0000u)};
+    pm[q] = __builtin_bit_cast(unsigned int, __builtin_convertvector(r1, bf16x2));
+    const f32x2 r2 = {r1[0] - __uint_as_float(pm[q] << 16), r1[1] - __uint_as_float(pm[q] & 0xffff0000u)};
+    pl[q] = __builtin_bit_cast(unsigned int, __builtin_convertvector(r2, bf16x2));
+  }
+}
+
+// Byte offset of chunk c (eight k) of row r inside a plane: rows are 64 bytes, and the four chunks of a row are rotated
+// so that eight lanes reading one chunk column of consecutive rows, or writing it to every second row, take eight
+// different 16-byte columns of the 64 banks.
+__device__ __forceinline__ int chunk_at(int r, int c) { return r * 64 + ((c ^ ((r >> 2) & 3)) << 4); }
+
+// One operand's tile of R rows (or columns) x 32 k, on its way from memory to LDS.  A thread carries CH chunks of eight
+// k.  Row-major: four lanes cover the 128 bytes of a row's stage.  k-major: a thread owns CH adjacent rows and eight
+// consecutive k, so the transposition happens in its registers and a wavefront reads whole pieces of a k row.
+enum { IN, TAIL, CHECKED };
+template <int R, int NT, bool KM>
+struct Tile {
+  static constexpr int CH = R * 4 / NT > 0 ? R * 4 / NT : 1;
+  static constexpr int USED = R * 4 / CH;  // threads that carry something
+  float v[CH][8];
+  const float *p[CH];
+  int k_off, row[CH];
+
+  __device__ __forceinline__ void init(const float *base, int ld, int r0, int rows, int rows_per, long outer) {
+    const int tid = threadIdx.x;
+    if (USED < NT && tid >= USED) return;
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      if (!KM) {
+        row[c] = (c * USED + tid) >> 2;
+        const int r = min(r0 + row[c], rows - 1);  // a row past the end repeats the last one; its sums are not stored
+        p[c] = base + (rows_per > 0 ? (long)(r / rows_per) * outer + (long)(r % rows_per) * ld : (long)r * ld);
+      } else {
+        row[c] = (tid % (R / CH)) * CH + c;
+        p[c] = base + min(r0 + row[c], rows - 1);
+      }
+    }
+    k_off = KM ? (tid / (R / CH)) * 8 : (tid & 3) * 8;
+  }
+  // IN: the stage lies inside K and the accesses are aligned.  TAIL: aligned accesses, clamped into the operand, with what
+  // lies beyond K set to zero.  CHECKED: one element at a time.
+  template <int MODE>
+  __device__ __forceinline__ void load(int k0, int K, int ld) {
+    if (USED < NT && (int)threadIdx.x >= USED) return;
+    const int k = k0 + k_off;
+    if constexpr (MODE == CHECKED) {
+#pragma unroll
+      for (int c = 0; c < CH; ++c)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[c][q] = k + q < K ? (KM ? p[c][(long)(k + q) * ld] : p[c][k + q]) : 0.0f;
+      return;
+    }
+    if constexpr (!KM) {
+      const int last = (K - 1) & ~3;  // the last aligned piece that holds something
+      const int k_lo = MODE == TAIL ? min(k, last) : k, k_hi = MODE == TAIL ? min(k + 4, last) : k + 4;
+#pragma unroll
+      for (int c = 0; c < CH; ++c) {
+        const float4 lo = *reinterpret_cast<const float4 *>(p[c] + k_lo), hi = *reinterpret_cast<const float4 *>(p[c] + k_hi);
+        v[c][0] = lo.x; v[c][1] = lo.y; v[c][2] = lo.z; v[c][3] = lo.w;
+        v[c][4] = hi.x; v[c][5] = hi.y; v[c][6] = hi.z; v[c][7] = hi.w;
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const long at = (long)(MODE == TAIL ? min(k + q, K - 1) : k + q) * ld;
+        if constexpr (CH == 2) {
+          const float2 t = *reinterpret_cast<const float2 *>(p[0] + at);
+          v[0][q] = t.x;
+          v[1][q] = t.y;
+        } else {
+#pragma unroll
+          for (int c = 0; c < CH; ++c) v[c][q] = p[c][at];
+        }
+      }
+    }
+    if constexpr (MODE == TAIL) {
+#pragma unroll
+      for (int c = 0; c < CH; ++c)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[c][q] = k + q < K ? v[c][q] : 0.0f;
+    }
+  }
+  // planes of R * 64 bytes each
+  __device__ __forceinline__ void store(unsigned char *s) const {
+    if (USED < NT && (int)threadIdx.x >= USED) return;
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      u32x4 h, m, l;
+      split3(v[c], h, m, l);
+      unsigned char *q = s + chunk_at(row[c], k_off >> 3);
+      *reinterpret_cast<u32x4 *>(q) = h;
+      *reinterpret_cast<u32x4 *>(q + R * 64) = m;
+      *reinterpret_cast<u32x4 *>(q + 2 * R * 64) = l;
+    }
+  }
+};
+
+// BM x BN tile per workgroup of WM x WN wavefronts.  LDS holds one stage (192 bytes per tile row and column: 48 KiB at
+// 128 x 128, three workgroups per CU); the next stage's loads are in flight in registers while this one is multiplied,
+// and the other workgroups of the CU fill the two barriers.  What bounds it: at 128 x 128 a wavefront spends 1536 cycles
+// of a stage in matrix instructions, 700 in the split and the LDS pipe moves 144 KiB.
+template <int BM, int BN, int WM, int WN, bool AK, bool BK, int EPI>
+__global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_f32(GemmF32 g) {
+  constexpr int NT = WM * WN * 64;
+  constexpr int MI = BM / WM / 32, NJ = BN / WN / 32;
+  __shared__ __attribute__((aligned(16))) unsigned char s_a[3 * BM * 64];
+  __shared__ __attribute__((aligned(16))) unsigned char s_b[3 * BN * 64];
+  __shared__ float s_norm[EPI == GEMM_NORM ? BM : 1];
+  // XCD-aware mapping: workgroup ids are dealt round-robin to the 8 XCDs, so ids with the same (id % 8) share an L2.
+  // Each XCD takes one contiguous eighth of the (slice, part of K, tile) list: neighbouring tiles reuse their operand
+  // rows in one L2, and every XCD has the same number of tiles whatever the number of slices.
+  const int tiles = g.tri ? g.mt * (g.mt + 1) / 2 : g.mt * g.nt;
+  const long total = (long)g.n_slices * g.ks * tiles;
+  const int xcd = blockIdx.x & 7;
+  const long at = total * xcd / 8 + (blockIdx.x >> 3);
+  if (at >= total * (xcd + 1) / 8) return;
+  const int tile = (int)(at % tiles);
+  const int part = (int)(at / tiles % g.ks);
+  const int slice = (int)(at / tiles / g.ks);
+  int ti, tj;
+  if (g.tri) {  // lower triangle of square tiles, row by row
+    ti = (int)((sqrtf(8.0f * (float)tile + 1.0f) - 1.0f) * 0.5f);
+    while ((ti + 1) * (ti + 2) / 2 <= tile) ++ti;
+    while (ti * (ti + 1) / 2 > tile) --ti;
+    tj = tile - ti * (ti + 1) / 2;
+  } else {
+    ti = tile / g.nt;
+    tj = tile - ti * g.nt;
+  }
+  const int m0 = ti * BM, n0 = tj * BN;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = wave / WN, wn = wave % WN;
+  const long s1 = slice / g.mod, s2 = slice % g.mod;
+  const float *A = g.A + s1 * g.a_s1 + s2 * g.a_s2;
+  const float *B = g.B + s1 * g.b_s1 + s2 * g.b_s2;
+  float *C = g.C + s1 * g.c_s1 + s2 * g.c_s2;
+  const int bs = g.block_size;
+  const float ld = (g.decay_rows || g.decay_state || g.decay_scores) ? g.log_decay[slice % g.heads] : 0.0f;
+
+  // the k blocks of this part: first those of A . B, then those of A2 . B2
+  const int k_causal = ((min(m0 + BM, g.M) - 1) / bs + 1) * bs;
+  int K1 = g.K, K2 = g.A2 ? g.K2 : 0;
+  if (g.causal_k) {
+    if (g.A2) K2 = min(K2, k_causal);
+    else K1 = min(K1, k_causal);
+  }
+  // a scores tile above the diagonal of the block pattern only writes zeros
+  if (EPI == GEMM_SCORES && !g.active && n0 / bs > (min(m0 + BM, g.M) - 1) / bs) K1 = 0;
+  const int nb1 = (K1 + FK - 1) / FK, nb = nb1 + (K2 + FK - 1) / FK;
+  const int b_lo = part * g.kb_per, b_hi = min(nb, b_lo + g.kb_per);
+
+  f32x16 acc[MI][NJ];
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+
+  Tile<BM, NT, AK> ta;
+  Tile<BN, NT, BK> tb;
+  float rs[Tile<BM, NT, AK>::CH];
+#pragma unroll
+  for (int c = 0; c < Tile<BM, NT, AK>::CH; ++c) rs[c] = 0.0f;
+
+  auto run = [&](const float *pa, int lda, int rows_per, long a_outer, const float *pb, int ldb, int K, int lo, int hi) {
+    ta.init(pa, lda, m0, g.M, rows_per, a_outer);
+    tb.init(pb, ldb, n0, g.N, 0, 0);
+    // 16-byte pieces of a row, or (k-major) 8-byte pieces of a k row that end inside it
+    const bool a_ok = AK ? ((lda & 1) == 0 && (g.M & 1) == 0 && (reinterpret_cast<uintptr_t>(pa) & 7) == 0)
+                         : ((lda & 3) == 0 && (a_outer & 3) == 0 && K <= lda && (reinterpret_cast<uintptr_t>(pa) & 15) == 0);
+    const bool b_ok = BK ? ((ldb & 1) == 0 && (g.N & 1) == 0 && (reinterpret_cast<uintptr_t>(pb) & 7) == 0)
+                         : ((ldb & 3) == 0 && K <= ldb && (reinterpret_cast<uintptr_t>(pb) & 15) == 0);
+    auto scaled = [&](int kb) {
+      if (AK && EPI == GEMM_STORE && g.decay_state) {  // token k of K is decayed K - k times by the end
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          const float f = expf((float)(K - (kb * FK + ta.k_off + q)) * ld);
+#pragma unroll
+          for (int c = 0; c < Tile<BM, NT, AK>::CH; ++c) ta.v[c][q] *= f;
+        }
+      }
+      if (EPI == GEMM_NORM) {
+#pragma unroll
+        for (int c = 0; c < Tile<BM, NT, AK>::CH; ++c)
+#pragma unroll
+          for (int q = 0; q < 8; ++q) rs[c] += fabsf(ta.v[c][q]);
+      }
+    };
+    auto multiply = [&]() {
+      // lane (r = lane % 32, half = lane / 32) feeds chunk 2 * step + half of its row
+      const int r = lane & 31, half = lane >> 5;
+#pragma unroll
+      for (int step = 0; step < 2; ++step) {
+        bf16x8 fa[3][MI], fb[3][NJ];
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+#pragma unroll
+          for (int i = 0; i < MI; ++i)
+            fa[t][i] = *reinterpret_cast<const bf16x8 *>(s_a + t * BM * 64 + chunk_at(wm * (BM / WM) + i * 32 + r, 2 * step + half));
+#pragma unroll
+          for (int j = 0; j < NJ; ++j)
+            fb[t][j] = *reinterpret_cast<const bf16x8 *>(s_b + t * BN * 64 + chunk_at(wn * (BN / WN) + j * 32 + r, 2 * step + half));
+        }
+        constexpr int TA[6] = {2, 0, 1, 1, 0, 0}, TB[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+        for (int t = 0; t < 6; ++t)
+#pragma unroll
+          for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[TA[t]][i], fb[TB[t]][j], acc[i][j], 0, 0, 0);
+      }
+    };
+    if (a_ok && b_ok) {
+      // from the last stage, the one that K may cut short, down: every load inside the loop then lies inside K, and the
+      // loop is straight-line code (with a branch among them, loads are waited for where they are issued)
+      ta.template load<TAIL>((hi - 1) * FK, K, lda);
+      tb.template load<TAIL>((hi - 1) * FK, K, ldb);
+      auto stage_in = [&](int kb) {
+        scaled(kb);
+        __syncthreads();  // the previous stage's fragment reads are done
+        ta.store(s_a);
+        tb.store(s_b);
+        __syncthreads();
+      };
+      for (int kb = hi - 1; kb > lo; --kb) {
+        stage_in(kb);
+        ta.template load<IN>((kb - 1) * FK, K, lda);
+        tb.template load<IN>((kb - 1) * FK, K, ldb);
+        __builtin_amdgcn_sched_barrier(0);  // left alone, the scheduler sinks the loads behind the products
+        multiply();
+      }
+      stage_in(lo);
+      multiply();
+    } else {
+      for (int kb = lo; kb < hi; ++kb) {
+        ta.template load<CHECKED>(kb * FK, K, lda);
+        tb.template load<CHECKED>(kb * FK, K, ldb);
+        scaled(kb);
+        __syncthreads();
+        ta.store(s_a);
+        tb.store(s_b);
+        __syncthreads();
+        multiply();
+      }
+    }
+  };
+  // accumulator element e of lane l in a 32x32 tile: row = (e/4)*8 + (l/32)*4 + (e%4), col = l%32
+  auto row_of = [&](int i, int e) { return m0 + wm * (BM / WM) + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3); };
+
+  if (b_lo < min(b_hi, nb1))
+    run(A, g.lda, g.rows_per, g.a_outer, B, g.ldb, K1, b_lo, min(b_hi, nb1));
+  if (EPI == GEMM_STORE && g.decay_rows) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const float f = expf((float)row_of(i, e) * ld);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j][e] *= f;
+      }
+  }
+  if constexpr (!AK && BK && EPI == GEMM_STORE) {
+    if (g.A2 && max(b_lo, nb1) < b_hi)
+      run(g.A2 + s1 * g.a2_s1 + s2 * g.a2_s2, g.lda2, 0, 0, g.B2 + s1 * g.b2_s1 + s2 * g.b2_s2, g.ldb2, K2,
+          max(b_lo, nb1) - nb1, b_hi - nb1);
+  }
+
+  if (EPI == GEMM_NORM) {  // four threads hold a row's chunks
+#pragma unroll
+    for (int c = 0; c < Tile<BM, NT, AK>::CH; ++c) {
+      float t = rs[c];
+      t += __shfl_xor(t, 1);
+      t += __shfl_xor(t, 2);
+      if ((tid & 3) == 0 && tid < Tile<BM, NT, AK>::USED) s_norm[(c * Tile<BM, NT, AK>::USED + tid) >> 2] = t;
+    }
+    __syncthreads();
+  }
+  if (g.ks > 1) {  // a part of the sums: [part][slice][M][N]
+    float *P = C + (long)part * g.c_split + (long)slice * g.M * g.N;
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const int col = n0 + wn * (BN / WN) + j * 32 + (lane & 31);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int row = row_of(i, e);
+          if (row < g.M && col < g.N) P[(long)row * g.N + col] = acc[i][j][e];
+        }
+      }
+    return;
+  }
+  const float slope = (EPI == GEMM_SCORES && g.use_alibi) ? g.slopes[slice % g.heads] : 0.0f;
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const int col = n0 + wn * (BN / WN) + j * 32 + (lane & 31);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int row = row_of(i, e);
+        if (row >= g.M) continue;
+        float v = acc[i][j][e];
+        if (EPI == GEMM_SCORES) {
+          if (col >= g.ldc) continue;
+          bool act = col < g.N;
+          const int rb = row / bs, cb = col / bs;
+          if (act) act = g.active ? g.active[(long)rb * g.tb + cb] != 0 : cb <= rb;
+          if (act) {
+            if (rb == cb && col >= row) v = 0.0f;  // tril(-1) on diagonal blocks (:88-90)
+            if (g.decay_scores && col < row) v = v * expf((float)(row - col) * ld);
+            if (g.use_alibi) {  // added to every entry of an active block (:97-100)
+              const float al = slope * ((float)col - (float)row);
+              v = v + al;
+            }
+          } else {
+            v = 0.0f;
+          }
+          C[(long)row * g.ldc + col] = v;
+        } else {
+          if (col >= g.N) continue;
+          float *p = C + (g.rows_per > 0 ? (long)(row / g.rows_per) * g.c_outer + (long)(row % g.rows_per) * g.ldc
+                                         : (long)row * g.ldc) + col;
+          if (EPI == GEMM_NORM)
+            *p = v / (s_norm[row - m0] + kRowNormEps);
+          else if (g.decay_state)
+            *p = *p * expf((float)g.K * ld) + v;
+          else if (g.accumulate)
+            // C += acc as one no-return add per element, done by the L2: the wavefront does not wait for C to arrive,
+            // so a short-K tile's epilogue overlaps the next workgroup's products.  One add per element and call: the
+            // same rounding as *p + v and no race; the L2's adder flushes results below the smallest normal float to
+            // zero.
+            unsafeAtomicAdd(p, v);
+          else
+            *p = v;
+        }
+      }
+    }
+}
+
+template <int EPI>
+void launch(hipStream_t st, const GemmF32 &g, bool ak, bool bk, int tile, unsigned grid) {
+#define BDH_G(BM_, BN_, WM_, WN_, AK_, BK_) \
+  hipLaunchKernelGGL((k_gemm_f32<BM_, BN_, WM_, WN_, AK_, BK_, EPI>), dim3(grid), dim3(256), 0, st, g)
+#define BDH_GT(AK_, BK_)                                     \
+  do {                                                       \
+    if (tile == 0) BDH_G(128, 128, 2, 2, AK_, BK_);          \
+    else if (tile == 1) BDH_G(64, 64, 2, 2, AK_, BK_);       \
+    else BDH_G(32, 128, 1, 4, AK_, BK_);                     \
+  } while (0)
+  if constexpr (EPI == GEMM_SCORES) {
+    BDH_GT(false, false);
+  } else if constexpr (EPI == GEMM_NORM) {
+    BDH_GT(false, true);
+  } else {
+    if (ak) BDH_GT(true, true);
+    else BDH_GT(false, true);
+  }
+#undef BDH_GT
+#undef BDH_G
+}
+
+constexpr int kTileM[3] = {128, 64, 32}, kTileN[3] = {128, 64, 128};
+
+// scores over causal time blocks that end on tile edges: the tiles above the diagonal hold nothing, and a reader whose
+// own row tiles are no larger never looks at them
+bool lower_triangle(const GemmF32 &g, int tile) {
+  return g.epilogue == GEMM_SCORES && !g.active && !g.sparse_pattern && kTileM[tile] == kTileN[tile] &&
+         kTileM[tile] % g.block_size == 0 && kTileM[tile] % g.reader_rows == 0;
+}
+
+}  // namespace
+
+// Which tile and how many parts of K.  A CU that holds a few workgroups turns out a 32-deep stage of a 128 x 128, 64 x 64
+// or 32 x 128 tile every `full` cycles; a workgroup alone on its CU takes `alone`, the memory round trip and the two
+// barriers uncovered.  The last, partly filled round of workgroups counts like a whole one.  More parts of K fill the
+// chip where the tiles are few, at the price of writing and re-reading every part.
+GemmPlan bdh_gemm_f32_plan(const bdh_ctx *ctx, const GemmF32 &g, int max_split) {
+  const double n_cu = ctx->n_cu > 0 ? ctx->n_cu : 256;
+  constexpr double full[3] = {2600.0, 900.0, 900.0}, alone[3] = {3600.0, 2000.0, 2000.0};
+  const int nb = (g.K + FK - 1) / FK + (g.A2 ? (g.K2 + FK - 1) / FK : 0);
+  GemmPlan best;
+  double best_t = 1e300;
+  for (int t = 0; t < 3; ++t) {
+    if (t == 2 && (g.epilogue == GEMM_SCORES || g.M > 96)) continue;
+    const double mt = (g.M + kTileM[t] - 1) / kTileM[t], nt = (g.N + kTileN[t] - 1) / kTileN[t];
+    const bool tri = lower_triangle(g, t);
+    const double tiles = g.n_slices * (tri ? mt * (mt + 1) / 2 : mt * nt);
+    for (int ks = 1; ks <= max_split && (ks == 1 || nb >= 4 * ks); ks *= 2) {
+      const double per = (nb + ks - 1) / ks;
+      const double wgs = tiles * ks / n_cu;
+      const double rounds = wgs <= 1.0 ? 1.0 : wgs;
+      double cyc = per * std::max(rounds * full[t], alone[t]) + 6000.0;
+      if (wgs > 1.0) cyc += per * full[t] * (std::ceil(wgs) - wgs) * 0.5;
+      if (ks > 1) cyc += 8000.0 + (double)g.n_slices * g.M * g.N * 4.0 * 2.0 * ks / 2000.0;  // bytes at about 5 TB/s
+      if (cyc < best_t) {
+        best_t = cyc;
+        best.tile = t;
+        best.ks = ks;
+      }
+    }
+  }
+  return best;
+}
+
+int bdh_gemm_f32_rows(const GemmPlan &plan) { return kTileM[plan.tile]; }
+
+int bdh_launch_gemm_f32(bdh_ctx *ctx, GemmF32 g, bool a_kmajor, bool b_kmajor, const GemmPlan &plan, float *partial) {
+  g.mt = (g.M + kTileM[plan.tile] - 1) / kTileM[plan.tile];
+  g.nt = (g.N + kTileN[plan.tile] - 1) / kTileN[plan.tile];
+  g.tri = lower_triangle(g, plan.tile);
+  const int nb = (g.K + FK - 1) / FK + (g.A2 ? (g.K2 + FK - 1) / FK : 0);
+  g.ks = plan.ks;
+  g.kb_per = (nb + g.ks - 1) / g.ks;
+  if (g.ks > 1) {
+    g.C = partial;
+    g.c_s1 = g.c_s2 = 0;
+    g.c_split = (long)g.n_slices * g.M * g.N;
+  }
+  const long tiles = g.tri ? (long)g.mt * (g.mt + 1) / 2 : (long)g.mt * g.nt;
+  const long total = (long)g.n_slices * g.ks * tiles;
+  if (total + 8 > 0x7fffffffL || tiles > 0x7fffffL) return bdh_fail(ctx, BDH_E_SHAPE, "too many tiles");
+  if (total == 0) return BDH_OK;
+  const unsigned grid = (unsigned)(8 * ((total + 7) / 8));
+  switch (g.epilogue) {
+    case GEMM_SCORES: launch<GEMM_SCORES>(ctx->stream, g, a_kmajor, b_kmajor, plan.tile, grid); break;
+    case GEMM_NORM: launch<GEMM_NORM>(ctx->stream, g, a_kmajor, b_kmajor, plan.tile, grid); break;
+    default: launch<GEMM_STORE>(ctx->stream, g, a_kmajor, b_kmajor, plan.tile, grid); break;
+  }
+  BDH_LAUNCH_CHECK(ctx, "k_gemm_f32");
+  return BDH_OK;
+}

@@ -392,167 +392,6 @@ __global__ __launch_bounds__(NW * 64) void k_relu_lowrank_row(const float *__res
   }
 }
 
-// A few input rows (a batch of 8 to 63 sequences decoding together) without LDS: the inputs of a row tile
-// are the same for every lane, so they are read through the scalar cache (wave-uniform addresses, read
-// only) and feed the FMAs as scalar operands; the vector memory pipe carries only the weights.  With the
-// inputs staged in LDS instead, three quarters of the wave wait cycles were waits for the broadcast reads.
-// Same k-sequential fmaf chain per output as k_relu_lowrank.
-template <int RT, int UK>
-__global__ __launch_bounds__(256) void k_relu_lowrank_sc(const float *__restrict__ in, int h_in, int T, int d,
-                                                        const float *__restrict__ w, int h, int N,
-                                                        const float *__restrict__ bias, float thr,
-                                                        const unsigned char *__restrict__ block_active,
-                                                        int block_size, int n_blocks,
-                                                        const float *__restrict__ gate, float *__restrict__ out,
-                                                        int M) {
-  const int hh = blockIdx.y;
-  const int n = blockIdx.x * 256 + threadIdx.x;
-  const int m0 = blockIdx.z * RT;
-  if (n >= N) return;
-  const float *rows[RT];  // wave-uniform row pointers (rows past M alias the last valid row; never stored)
-#pragma unroll
-  for (int r = 0; r < RT; ++r) {
-    const int m = min(m0 + r, M - 1);
-    const int b = m / T, t = m - b * T;
-    rows[r] = in + (((long)b * h_in + (h_in == 1 ? 0 : hh)) * T + t) * d;
-  }
-  float acc[RT];
-#pragma unroll
-  for (int r = 0; r < RT; ++r) acc[r] = 0.0f;
-  const float *wp = w + (long)hh * d * N + n;
-  int k0 = 0;
-  for (; k0 + UK <= d; k0 += UK) {
-    float wv[UK];
-#pragma unroll
-    for (int u = 0; u < UK; ++u) wv[u] = wp[(long)(k0 + u) * N];
-#pragma unroll
-    for (int r = 0; r < RT; ++r) {
-#pragma unroll
-      for (int u = 0; u < UK; ++u) acc[r] = __builtin_fmaf(rows[r][k0 + u], wv[u], acc[r]);
-    }
-  }
-  for (; k0 < d; ++k0) {
-    const float wv = wp[(long)k0 * N];
-#pragma unroll
-    for (int r = 0; r < RT; ++r) acc[r] = __builtin_fmaf(rows[r][k0], wv, acc[r]);
-  }
-  const float bv = bias ? bias[(long)hh * N + n] : 0.0f;
-  float maskv = 1.0f;
-  if (block_active) {
-    const int blk = n / block_size;
-    maskv = (blk < n_blocks && block_active[blk]) ? 1.0f : 0.0f;
-  }
-#pragma unroll
-  for (int r = 0; r < RT; ++r) {
-    const int m = m0 + r;
-    if (m < M) {
-      const int b = m / T, t = m - b * T;
-      float p = acc[r];
-      if (bias) p = p + bv;
-      if (thr != 0.0f) p = p - thr;
-      float y = p > 0.0f ? p : 0.0f;
-      if (block_active) y = y * maskv;
-      const long o = (((long)b * h + hh) * T + t) * N + n;
-      if (gate) y = gate[o] * y;
-      out[o] = y;
-    }
-  }
-}
-
-// Many input rows (a prompt, a large batch): a 64-row x 256-column tile per workgroup, 16 rows x 4
-// adjacent columns per thread.  Wave w owns rows 16w..16w+15, so an input value is one LDS broadcast
-// for the whole wave; a weight row segment is one float4 per lane.  The inputs are staged 64 k at a
-// time.  Every output is still one k-sequential fmaf chain, so the values are those of k_relu_lowrank
-// bit for bit; the tile only cuts the weight re-reads from one per 8 rows to one per 64.
-__global__ __launch_bounds__(256) void k_relu_lowrank_tile(const float *__restrict__ in, int h_in, int T, int d,
-                                                          const float *__restrict__ w, int h, int N,
-                                                          const float *__restrict__ bias, float thr,
-                                                          const unsigned char *__restrict__ block_active,
-                                                          int block_size, int n_blocks,
-                                                          const float *__restrict__ gate, float *__restrict__ out,
-                                                          int M) {
-  constexpr int RT = 16, KC = 64;
-  __shared__ __attribute__((aligned(16))) float s_x[64 * KC];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int hh = blockIdx.y;
-  const int n = (blockIdx.x * 64 + lane) * 4;  // N % 4 == 0: a thread's four columns are all in or all out
-  const int m0 = blockIdx.z * 64;
-  const bool live = n < N;
-
-  float4 acc[RT];
-#pragma unroll
-  for (int r = 0; r < RT; ++r) acc[r] = make_float4(0.f, 0.f, 0.f, 0.f);
-  const float *wp = w + (long)hh * d * N + (live ? n : 0);
-  const float *sx = s_x + wave * RT * KC;
-  for (int kc = 0; kc < d; kc += KC) {  // d % 4 == 0
-    const int kn = min(KC, d - kc);
-    __syncthreads();
-    for (int i = tid; i < 64 * KC / 4; i += 256) {
-      const int r = i / (KC / 4), k4 = (i - r * (KC / 4)) * 4;
-      const int m = m0 + r;
-      float4 val = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (m < M && k4 < kn) {
-        const int b = m / T, t = m - b * T;
-        val = *reinterpret_cast<const float4 *>(in + (((long)b * h_in + (h_in == 1 ? 0 : hh)) * T + t) * d + kc + k4);
-      }
-      *reinterpret_cast<float4 *>(s_x + r * KC + k4) = val;
-    }
-    __syncthreads();
-    if (live) {
-      for (int k0 = 0; k0 < kn; k0 += 4) {
-        float4 wv[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) wv[u] = *reinterpret_cast<const float4 *>(wp + (long)(kc + k0 + u) * N);
-#pragma unroll
-        for (int r = 0; r < RT; ++r) {
-          const float4 xin = *reinterpret_cast<const float4 *>(sx + r * KC + k0);
-          const float xs[4] = {xin.x, xin.y, xin.z, xin.w};
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            acc[r].x = __builtin_fmaf(xs[u], wv[u].x, acc[r].x);
-            acc[r].y = __builtin_fmaf(xs[u], wv[u].y, acc[r].y);
-            acc[r].z = __builtin_fmaf(xs[u], wv[u].z, acc[r].z);
-            acc[r].w = __builtin_fmaf(xs[u], wv[u].w, acc[r].w);
-          }
-        }
-      }
-    }
-  }
-  if (!live) return;
-  float4 bv = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (bias) bv = *reinterpret_cast<const float4 *>(bias + (long)hh * N + n);
-  float mk[4] = {1.f, 1.f, 1.f, 1.f};
-  if (block_active)
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int blk = (n + c) / block_size;
-      mk[c] = (blk < n_blocks && block_active[blk]) ? 1.0f : 0.0f;
-    }
-#pragma unroll
-  for (int r = 0; r < RT; ++r) {
-    const int m = m0 + wave * RT + r;
-    if (m < M) {
-      const int b = m / T, t = m - b * T;
-      const long o = (((long)b * h + hh) * T + t) * N + n;
-      float p[4] = {acc[r].x, acc[r].y, acc[r].z, acc[r].w};
-      const float bb[4] = {bv.x, bv.y, bv.z, bv.w};
-      float4 gv = make_float4(1.f, 1.f, 1.f, 1.f);
-      if (gate) gv = *reinterpret_cast<const float4 *>(gate + o);
-      const float gg[4] = {gv.x, gv.y, gv.z, gv.w};
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        if (bias) p[c] = p[c] + bb[c];
-        if (thr != 0.0f) p[c] = p[c] - thr;
-        float y = p[c] > 0.0f ? p[c] : 0.0f;
-        if (block_active) y = y * mk[c];
-        if (gate) y = gg[c] * y;
-        p[c] = y;
-      }
-      *reinterpret_cast<float4 *>(out + o) = make_float4(p[0], p[1], p[2], p[3]);
-    }
-  }
-}
-
 // ------------------------------------------------------------------------------------
 // LayerNorm rows (one workgroup per row); in == out allowed.  The row is staged in LDS and
 // every thread walks it in index order, so mean and variance are the same left-to-right f32
@@ -1009,177 +848,7 @@ void launch_relu(hipStream_t st, dim3 grid, size_t lds, const ReluLowrankParams 
                      p.h, p.N, p.bias, p.threshold, mask, p.block_size, p.n_blocks, p.gate, p.out, M);
 }
 
-// ------------------------------------------------------------------------------------
-// relu_lowrank on the f32 matrix cores, for 8 rows and more.  v_mfma_f32_32x32x2_f32 adds its two k-steps one
-// after the other, each as one fused multiply-add, so a chain of these instructions over k = 0, 1, 2, ... is the
-// same k-sequential fmaf chain per output as k_relu_lowrank computes, bit for bit (checked on the device against
-// the scalar chain, including denormal results): the active sets do not change, the weights are streamed once
-// for up to 32 * RT rows, and the arithmetic runs at the matrix rate.
-//   A operand (32 rows x 2 k): lane l holds in[row l % 32][k0 + l / 32], from an LDS copy of the input rows laid
-//   out [k][row]; B operand (2 k x 32 columns): lane l holds w[k0 + l / 32][column].  A lane loads four adjacent
-//   columns of a weight row at once (16 bytes, a wavefront reads two 512-byte row pieces per k-pair) and uses
-//   them in four matrix instructions: instruction j owns the columns n0 + 4 c + j, c = 0..31, so that the four
-//   results a lane holds for a row are again four adjacent columns (16-byte stores).
-// One workgroup = NW wavefronts x 128 columns; grid (column blocks, heads, row groups of 32 * RT).  Each wavefront
-// asks for its first UK k-pairs of weights before the input rows are staged, so the staging hides behind them.
-// ------------------------------------------------------------------------------------
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
-
-template <int RT, int UK, int NW>  // RT row tiles of 32 rows per workgroup; UK k-pairs of weights in flight per wavefront
-__global__ __launch_bounds__(NW * 64) void k_relu_lowrank_mfma(const float *__restrict__ in, int h_in, int T, int d,
-                                                           const float *__restrict__ w, int h, int N,
-                                                           const float *__restrict__ bias, float thr,
-                                                           const unsigned char *__restrict__ block_active,
-                                                           int block_size, int n_blocks,
-                                                           const float *__restrict__ gate, float *__restrict__ out,
-                                                           int M) {
-  extern __shared__ float s_in[];  // [d][32 * RT + 1], zero for rows past M (the odd row stride keeps the
-                                   // transposing writes below and the two k-rows of a read off each other's banks)
-  constexpr int R = 32 * RT, RS = R + 1;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int hh = blockIdx.y;
-  // grid.x = column blocks (rounded up to 8) x row groups: the workgroups that share a block of weight columns
-  // follow each other on one XCD (blockIdx.x % 8 picks the XCD), so the block is fetched from memory once
-  const int row_groups = (M + R - 1) / R;
-  const int xj = blockIdx.x >> 3;
-  const int col_block = (xj / row_groups) * 8 + (blockIdx.x & 7);
-  const int m0 = (xj % row_groups) * R;
-  if (col_block * NW * 128 >= N) return;        // a workgroup of the rounding-up: nothing to do (uniform)
-  const int n0 = (col_block * NW + wave) * 128;  // first column of this wavefront
-  const bool wave_ok = n0 < N;
-  const int ncol = n0 + 4 * (lane & 31);          // this lane's four columns ncol .. ncol + 3 (N % 4 == 0)
-  const bool col_ok = ncol < N;
-  const float *wp = w + (long)hh * d * N + (long)(lane >> 5) * N + (col_ok ? ncol : (wave_ok ? n0 : 0));
-  float4 wv[UK];
-#pragma unroll
-  for (int u = 0; u < UK; ++u) wv[u] = *reinterpret_cast<const float4 *>(wp + (long)(2 * u) * N);
-  // the input rows of this group, transposed on the way in: four adjacent k per access (d % 4 == 0), sixteen
-  // accesses of a thread in flight at a time (one at a time, the staging is a chain of trips to the L2)
-  {
-    const int d4 = d >> 2;
-    const int total = R * d4;
-    for (int i0 = 0; i0 < total; i0 += NW * 64 * 16) {
-      float4 v[16];
-#pragma unroll
-      for (int u = 0; u < 16; ++u) {
-        const int i = i0 + u * NW * 64 + tid;
-        const int r = i / d4, k4 = i - r * d4;
-        const int m = m0 + r;
-        v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (i < total && m < M) {
-          const int b = m / T, t = m - b * T;
-          v[u] = *reinterpret_cast<const float4 *>(in + (((long)b * h_in + (h_in == 1 ? 0 : hh)) * T + t) * d + 4 * k4);
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < 16; ++u) {
-        const int i = i0 + u * NW * 64 + tid;
-        const int r = i / d4, k4 = i - r * d4;
-        if (i < total) {
-          s_in[(4 * k4 + 0) * RS + r] = v[u].x;
-          s_in[(4 * k4 + 1) * RS + r] = v[u].y;
-          s_in[(4 * k4 + 2) * RS + r] = v[u].z;
-          s_in[(4 * k4 + 3) * RS + r] = v[u].w;
-        }
-      }
-    }
-  }
-  __syncthreads();
-  if (!wave_ok) return;
-  const float *ap = s_in + (lane >> 5) * RS + (lane & 31);
-
-  f32x16_t acc[RT][4];
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[rt][j][e] = 0.0f;
-
-  // k-pairs in groups of UK (d is a multiple of 2 * UK): the loop body has no branches, so the loads of the next
-  // group stay in flight across the matrix instructions of this one
-  const int groups = d / (2 * UK);
-  auto group = [&](int g, auto more_t) {
-    constexpr bool MORE = decltype(more_t)::value;
-#pragma unroll
-    for (int u = 0; u < UK; ++u) {
-      const int pr = g * UK + u;
-      const float4 b4 = wv[u];
-      if constexpr (MORE) wv[u] = *reinterpret_cast<const float4 *>(wp + (long)(2 * (pr + UK)) * N);
-      float a[RT];
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) a[rt] = ap[(2 * pr) * RS + rt * 32];
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) {
-        acc[rt][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[rt], b4.x, acc[rt][0], 0, 0, 0);
-        acc[rt][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[rt], b4.y, acc[rt][1], 0, 0, 0);
-        acc[rt][2] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[rt], b4.z, acc[rt][2], 0, 0, 0);
-        acc[rt][3] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[rt], b4.w, acc[rt][3], 0, 0, 0);
-      }
-      // keeps the load above where it is: left alone, the scheduler sinks all the loads of a group below its
-      // matrix instructions, and the next group then starts by waiting for every one of them
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  };
-  for (int g = 0; g + 1 < groups; ++g) group(g, std::true_type{});
-  group(groups - 1, std::false_type{});
-  if (!col_ok) return;
-
-  float4 bv = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (bias) bv = *reinterpret_cast<const float4 *>(bias + (long)hh * N + ncol);
-  float mk[4] = {1.0f, 1.0f, 1.0f, 1.0f};
-  if (block_active) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int blk = (ncol + j) / block_size;
-      mk[j] = (blk < n_blocks && block_active[blk]) ? 1.0f : 0.0f;
-    }
-  }
-  const float bvv[4] = {bv.x, bv.y, bv.z, bv.w};
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int m = m0 + rt * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
-      if (m < M) {
-        const int b = m / T, t = m - b * T;
-        const long o = (((long)b * h + hh) * T + t) * N + ncol;
-        float y[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          float pv = acc[rt][j][e];
-          if (bias) pv = pv + bvv[j];
-          if (thr != 0.0f) pv = pv - thr;
-          float yy = pv > 0.0f ? pv : 0.0f;
-          if (block_active) yy = yy * mk[j];
-          y[j] = yy;
-        }
-        if (gate) {
-          const float4 g4 = *reinterpret_cast<const float4 *>(gate + o);
-          y[0] = g4.x * y[0]; y[1] = g4.y * y[1]; y[2] = g4.z * y[2]; y[3] = g4.w * y[3];
-        }
-        *reinterpret_cast<float4 *>(out + o) = make_float4(y[0], y[1], y[2], y[3]);
-      }
-    }
-}
-
 }  // namespace
-
-#ifndef BDH_RL_UK
-#define BDH_RL_UK 16
-#endif
-// lets a kernel take up to 144 KiB of dynamic LDS; once per device
-template <typename K>
-static hipError_t allow_big_lds(K kernel, std::atomic<uint64_t> &configured) {
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return e;
-  const uint64_t bit = 1ull << (dev & 63);
-  if (configured.load(std::memory_order_acquire) & bit) return hipSuccess;
-  e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 144 * 1024);
-  if (e == hipSuccess) configured.fetch_or(bit, std::memory_order_release);
-  return e;
-}
 
 int bdh_launch_relu_lowrank(bdh_ctx *ctx, const ReluLowrankParams &p) {
   const long M = (long)p.B * p.T;
@@ -1210,73 +879,13 @@ int bdh_launch_relu_lowrank(bdh_ctx *ctx, const ReluLowrankParams &p) {
     }
     mask_dev = static_cast<const unsigned char *>(ctx->lat_mask);
   }
-  const bool aligned16 = bdh_aligned(p.in, 16) && bdh_aligned(p.weight, 16) && bdh_aligned(p.out, 16) &&
-                         bdh_aligned(p.bias, 16) && bdh_aligned(p.gate, 16);
-  // 8 to 64 rows (a batch of sequences decoding together): the f32 matrix cores, same values, the weights streamed
-  // once.  (Beyond 64 rows this kernel would stream them once per 64 rows; the 64 x 256 tile kernel below reuses them.)
-  // (a negative option value -r takes it from r rows on whatever the width)
-  const int mf_rows = ctx->opt_lowrank_mfma_rows < 0 ? -ctx->opt_lowrank_mfma_rows : ctx->opt_lowrank_mfma_rows;
-  const bool mf_any_width = ctx->opt_lowrank_mfma_rows < 0;
-  if (mf_rows > 0 && M >= mf_rows && M <= 64 && (p.N & 3) == 0 && (p.d % (2 * BDH_RL_UK)) == 0 &&
-      p.d >= 2 * BDH_RL_UK && aligned16) {
-    // one 32-row tile per workgroup; 33 to 64 rows make two row groups that follow each other on one XCD.  (Two row
-    // tiles per workgroup would stream the weights once for 64 rows too, but need 133 KiB of LDS at d = 512, one
-    // workgroup per CU: a decode step of the reference's large model at B = 64 took 2.5 ms that way against 1.4.)
-    const size_t lds = sizeof(float) * (size_t)p.d * 33;
-    // a wavefront owns 128 columns: only for matrices wide enough to give every CU a wavefront or two (a model with
-    // 256 neurons per head would run on 16 workgroups; it keeps the kernels below)
-    const long row_groups = (M + 31) / 32;
-    const int n_cu_mf = ctx->n_cu > 0 ? ctx->n_cu : 256;
-    const long waves = (long)((p.N + 127) / 128) * p.h * row_groups;
-    if (lds <= 144 * 1024 && (waves >= n_cu_mf || mf_any_width)) {
-      constexpr int UK = BDH_RL_UK;
-      const int nw = waves >= 4L * n_cu_mf ? 2 : 1;
-      const long col_blocks8 = ((p.N + nw * 128 - 1) / (nw * 128) + 7) / 8 * 8;
-      if (col_blocks8 * row_groups > 0x7fffffffL || p.h > 65535)
-        return bdh_fail(ctx, BDH_E_SHAPE, "grid too large (row groups %ld)", row_groups);
-      const dim3 grid((unsigned)(col_blocks8 * row_groups), p.h, 1);
-      static std::atomic<uint64_t> cfg1{0}, cfg2{0};
-      if (nw == 2) {
-        BDH_HIP_CHECK(ctx, allow_big_lds(k_relu_lowrank_mfma<1, UK, 2>, cfg2));
-        hipLaunchKernelGGL((k_relu_lowrank_mfma<1, UK, 2>), grid, dim3(128), lds, ctx->stream, p.in, p.h_in, p.T, p.d,
-                           p.weight, p.h, p.N, p.bias, p.threshold, mask_dev, p.block_size, p.n_blocks, p.gate, p.out, (int)M);
-      } else {
-        BDH_HIP_CHECK(ctx, allow_big_lds(k_relu_lowrank_mfma<1, UK, 1>, cfg1));
-        hipLaunchKernelGGL((k_relu_lowrank_mfma<1, UK, 1>), grid, dim3(64), lds, ctx->stream, p.in, p.h_in, p.T, p.d,
-                           p.weight, p.h, p.N, p.bias, p.threshold, mask_dev, p.block_size, p.n_blocks, p.gate, p.out, (int)M);
-      }
-      BDH_LAUNCH_CHECK(ctx, "k_relu_lowrank_mfma");
-      return BDH_OK;
-    }
-  }
-  // many tokens per sequence: one f32 matrix-core product per (sequence, head), same values
-  // (a negative option value -r takes it from r tokens on whatever the grid)
-  const int gemm_rows = ctx->opt_lowrank_gemm_rows;
-  // (the product kernel deals whole (sequence, head) slices to the 8 XCDs: with fewer than 16 of them half the chip
-  // idles -- config 1 at B = 1, four slices, took 24 ms for a 64-token prompt that way against 14)
-  const bool gemm_grid = (long)p.B * p.h >= 16 &&
-                         (long)p.B * p.h * ((p.T + 127) / 128) * ((p.N + 127) / 128) >= (ctx->n_cu > 0 ? ctx->n_cu : 256);
-  if (p.d > 0 && p.N > 0 && (gemm_rows > 0 ? (p.T >= gemm_rows && gemm_grid) : (gemm_rows < 0 && p.T >= -gemm_rows)))
-    return bdh_launch_relu_lowrank_gemm(ctx, p, mask_dev);
-  // many rows: the 64 x 256 tile (same values, an eighth of the weight traffic)
-  const long tile_wgs = (long)((p.N / 4 + 63) / 64) * p.h * ((M + 63) / 64);  // enough of them to cover the chip
-  if (M >= 64 && ctx->opt_lowrank_tile != 0 && (p.N & 3) == 0 && (p.d & 3) == 0 && p.d > 0 && aligned16 &&
-      (ctx->opt_lowrank_tile == 2 || tile_wgs >= (ctx->n_cu > 0 ? ctx->n_cu : 256))) {
-    const long row_tiles = (M + 63) / 64;
-    if (row_tiles > 65535 || p.h > 65535) return bdh_fail(ctx, BDH_E_SHAPE, "grid too large (row tiles %ld)", row_tiles);
-    hipLaunchKernelGGL(k_relu_lowrank_tile, dim3((p.N / 4 + 63) / 64, p.h, (unsigned)row_tiles), dim3(256), 0, ctx->stream,
-                       p.in, p.h_in, p.T, p.d, p.weight, p.h, p.N, p.bias, p.threshold, mask_dev, p.block_size, p.n_blocks,
-                       p.gate, p.out, (int)M);
-    BDH_LAUNCH_CHECK(ctx, "k_relu_lowrank_tile");
-    return BDH_OK;
-  }
-  // A matrix of up to 16 MiB (it sits in the L2) whose column-per-thread grid would leave most CUs idle, or a single
-  // row: 64 columns per workgroup, every weight in flight at once, as many rows per workgroup (1, 2, 4, 8) as still
-  // give a workgroup per CU
+  // A matrix of up to 16 MiB (it sits in the L2) and few outputs: 64 columns per workgroup, every weight in flight at once,
+  // as many rows per workgroup (1, 2, 4, 8) as still give a workgroup per CU.  The line is at 32768 outputs, 128 for every
+  // CU (us, this | 16-row matrix-core tiles: h*N = 2048, d = 512, 16 rows 7.6 | 8.8, 24 rows 12.8 | 8.9; 1024, 256, 32 rows
+  // 5.4 | 6.0, 48 rows 6.3 | 6.0; 4096, 256, 8 rows 5.4 | 6.0, 16 rows 7.6 | 6.0; 8192, 512, 4 rows 7.5 | 8.9, 8 rows 11.1 | 8.9).
   const int n_cu_rl = ctx->n_cu > 0 ? ctx->n_cu : 256;
   if (p.d >= 128 && p.d <= 512 && ctx->opt_lowrank_row != 0 &&
-      sizeof(float) * (size_t)p.h * p.d * p.N <= (size_t(16) << 20) &&
-      (M == 1 || (long)((p.N + 255) / 256) * p.h * ((M + 15) / 16) < n_cu_rl)) {
+      sizeof(float) * (size_t)p.h * p.d * p.N <= (size_t(16) << 20) && (M == 1 || M * p.h * p.N <= 128L * n_cu_rl)) {
     const long col_blocks = (p.N + 63) / 64;
     int rt = 1;
     if (M > 1) {
@@ -1301,21 +910,13 @@ int bdh_launch_relu_lowrank(bdh_ctx *ctx, const ReluLowrankParams &p) {
     BDH_LAUNCH_CHECK(ctx, "k_relu_lowrank_row");
     return BDH_OK;
   }
-  if (M >= 8 && ctx->opt_lowrank_scalar != 0) {
-    // 8 to 63 rows: inputs through the scalar cache, 16 rows (two SGPR batches of 8 k) or 8 rows per pass
-    const int rt = M >= 16 ? 16 : 8;
-    const long row_tiles = (M + rt - 1) / rt;
-    if (row_tiles > 65535 || p.h > 65535) return bdh_fail(ctx, BDH_E_SHAPE, "grid too large (row tiles %ld)", row_tiles);
-    const dim3 grid((p.N + 255) / 256, p.h, (unsigned)row_tiles);
-    if (rt == 16)
-      hipLaunchKernelGGL((k_relu_lowrank_sc<16, 8>), grid, dim3(256), 0, ctx->stream, p.in, p.h_in, p.T, p.d, p.weight,
-                         p.h, p.N, p.bias, p.threshold, mask_dev, p.block_size, p.n_blocks, p.gate, p.out, (int)M);
-    else
-      hipLaunchKernelGGL((k_relu_lowrank_sc<8, 8>), grid, dim3(256), 0, ctx->stream, p.in, p.h_in, p.T, p.d, p.weight,
-                         p.h, p.N, p.bias, p.threshold, mask_dev, p.block_size, p.n_blocks, p.gate, p.out, (int)M);
-    BDH_LAUNCH_CHECK(ctx, "k_relu_lowrank_sc");
-    return BDH_OK;
-  }
+  // Two rows and more: the f32 matrix cores, same values, the weights streamed once per row tile (options: fewer than 64
+  // rows from mfma_rows on, more from gemm_rows on; 0 = never; the sign no longer matters).  Fewer than 64 rows want the
+  // 16-byte pieces of the copying kernels; what is left, and a single row of a larger matrix, runs a thread per column.
+  const int mc_rows = std::abs(M < 64 ? ctx->opt_lowrank_mfma_rows : ctx->opt_lowrank_gemm_rows);
+  const bool pieces = p.d % 32 == 0 && p.N % 4 == 0 && bdh_aligned(p.in, 16) && bdh_aligned(p.weight, 16);
+  if (p.d > 0 && p.N > 0 && M > 1 && mc_rows > 0 && M >= mc_rows && (M >= 64 || pieces))
+    return bdh_launch_relu_lowrank_gemm(ctx, p, mask_dev);
   const int RT = M >= 8 ? 8 : (M >= 4 ? 4 : (M >= 2 ? 2 : 1));
   const size_t lds = sizeof(float) * (size_t)RT * (p.d > 0 ? p.d : 1);
   if (lds > 64 * 1024) return bdh_fail(ctx, BDH_E_SHAPE, "d=%d too large for the projection tile", p.d);
@@ -1371,33 +972,14 @@ int bdh_launch_decoder_residual(bdh_ctx *ctx, int B, int T, int h, int N, int d,
   const int M = B * T;
   const long K = (long)h * N;
   if (d > 1024 || (d & 3)) return bdh_fail(ctx, BDH_E_SHAPE, "decoder needs d %% 4 == 0 and d <= 1024, got %d", d);
-  // (the matrix-core form needs enough (sequence, head, tile) products to cover the chip)
-  const long mfma_tiles = (long)B * h * ((T + 127) / 128) * ((d + 127) / 128);
-  if (T >= 128 && ctx->opt_decoder_mfma != 0 && mfma_tiles >= (ctx->n_cu > 0 ? ctx->n_cu : 256) / 2) {
-    // many tokens per sequence: one product per (sequence, head) on the f32 matrix cores, h partials per row
-    int rc = bdh_ws_reserve(ctx, sizeof(float) * (size_t)h * M * d);
-    if (rc != BDH_OK) return rc;
-    float *partial = static_cast<float *>(ctx->ws);
-    rc = bdh_launch_decoder_partials_f32(ctx, B, T, h, N, d, xy, decoder, partial);
-    if (rc != BDH_OK) return rc;
-    launch_decoder_finalize(ctx, partial, h, M, d, cur, head);
-    BDH_LAUNCH_CHECK(ctx, "k_decoder_finalize");
-    return BDH_OK;
-  }
-  // (only when its 32 x 64 tiles over k-blocks of 1024 are enough workgroups for half the chip: not for a small model)
-  // (a negative option value -r takes it from r rows on whatever the grid)
+  // many rows: products on the matrix cores, all of E streamed once per row tile (fewer rows skip the inactive rows of E)
+  // (a negative option value -r takes it from r rows on in a decode step, too)
   const int sk_rows = ctx->opt_decoder_splitk_rows;
-  const bool sk_grid = (K / 1024) * ((d + 63) / 64) * ((M + 31) / 32) >= (ctx->n_cu > 0 ? ctx->n_cu : 256) / 2;
-  if (T == 1 && (K % 1024) == 0 && (sk_rows > 0 ? (M >= sk_rows && sk_grid) : M >= -(long)sk_rows)) {
-    // a batch of decoding sequences: split-K product on the f32 matrix cores, KB = 1024
-    const int KB = 1024;
-    const int KBN = (int)(K / KB);
-    int rc = bdh_ws_reserve(ctx, sizeof(float) * (size_t)KBN * M * d);
+  if (T == 1 ? M >= std::abs(sk_rows) : (T >= 16 && M >= 24 && ctx->opt_decoder_mfma != 0)) {
+    int rows = 0;
+    int rc = bdh_launch_decoder_partials_f32(ctx, B, T, h, N, d, xy, decoder, &rows);
     if (rc != BDH_OK) return rc;
-    float *partial = static_cast<float *>(ctx->ws);
-    rc = bdh_launch_decoder_splitk_f32(ctx, M, K, d, KB, xy, decoder, partial);
-    if (rc != BDH_OK) return rc;
-    launch_decoder_finalize(ctx, partial, KBN, M, d, cur, head);
+    launch_decoder_finalize(ctx, static_cast<float *>(ctx->ws), rows, M, d, cur, head);
     BDH_LAUNCH_CHECK(ctx, "k_decoder_finalize");
     return BDH_OK;
   }

@@ -1043,21 +1043,24 @@ int bdh_launch_state_steps_in(bdh_ctx *ctx, const StateStepParams &p, float *out
   // (not when even a 128-token chunk of rotated activations would pass 16 GiB of workspace)
   const bool chunk_fits = sizeof(float) * (size_t)slices * Nq * 128 <= (size_t(16) << 30) &&
                           (p.rho_dtype == BDH_F32 || sizeof(float) * (size_t)slices * Nq * d <= (size_t(64) << 30));
-  // By default from 128 tokens on (from 8 for the cases below); where the token loop is cheap (the f32 RoPE kernel walks many tokens per
-  // launch) only once the products have enough tiles to cover the chip (measured at N=8192, d=256, T=512:
-  // B*h = 4 or 8 slices lose to the loop at 5 % density, 16 slices win at any density).
-  const bool loop_is_cheap = fast && p.rho_dtype == BDH_F32;
-  const long state_tiles = (long)slices * ((std::min(T, 512) + 127) / 128) * ((d + 127) / 128);
-  // From 8 tokens on where the token loop has nothing to gain from sparsity: an f32 state that every token
-  // streams in full anyway (PoPE, eager ALiBi), or one so small (up to 64 MiB) that the loop is a chain of launch
-  // and barrier latencies (a 64-token prompt of the reference's tiny / base / large sizes: 1.5 / 1.4 / 3.5 ms
-  // token by token, 0.27 / 0.34 / 0.95 ms as dense products; at 8 tokens 0.30 / 0.29 / 0.69 against 0.22 / 0.27 /
-  // 0.59 ms, at 4 tokens the loop is ahead).
-  const bool streamed = p.rho_dtype == BDH_F32 && (p.rotary == BDH_POPE || (p.rotary == BDH_ALIBI && !p.stamps));
-  const bool small_state = p.rho_dtype == BDH_F32 && !loop_is_cheap &&
-                           sizeof(float) * (size_t)slices * Nq * d <= (size_t(64) << 20);
-  const bool dense_auto = (T >= 128 && (!loop_is_cheap || state_tiles >= n_cu / 2)) ||
-                          (T >= 8 && (streamed || small_state));
+  // The token loop reads and writes each token's rows, the dense form the whole state twice whatever the number of tokens
+  // (Q rho, then rho += Q^T V) in about six launches.  By default from 16 tokens on; us per call of a model, loop | dense,
+  // at half the neurons active:
+  //   L=6 d=256 N=256  B=1 f32 RoPE    T=16 402|358    T=32 700|426     lazy ALiBi  T=8 683|368   T=16 1214|378
+  //   L=6 d=256 N=2048 B=4 bf16 RoPE   T=16 1189|1010  T=32 2052|1024   eager ALiBi T=8 748|962   T=16 1216|974
+  //   L=8 d=512 N=2560 B=4 f32 RoPE    T=8 3965|3267   T=16 5696|2929   lazy ALiBi  T=8 4921|3392
+  //   L=12 d=512 N=10240 B=1 f32 RoPE  T=16 9893|6239; L=6 d=256 N=8192 B=3 T=500 62 900|9 760
+  // From 8 on where the loop is a chain of latencies or streams every row anyway: a lazily decayed f32 state, an f32 state
+  // decayed eagerly, PoPE, and a state of up to 64 MiB.  From 24 on for an f32 RoPE state of up to 64 MiB: its loop walks
+  // many tokens per launch and the rows stay in the caches (L=6 d=256 N=2048 B=1: T=16 533|613, T=32 789|624).
+  const size_t state_bytes = sizeof(float) * (size_t)slices * Nq * d;
+  const bool cached_loop = fast && p.rho_dtype == BDH_F32 && state_bytes <= (size_t(64) << 20);
+  const bool slow_loop = p.rho_dtype == BDH_F32 && p.rotary != BDH_ROPE;
+  const bool small_state = p.rho_dtype == BDH_F32 && state_bytes <= (size_t(64) << 20);
+  // And not at all for an f32 RoPE state of up to 512 KiB: there a prompt leaves the bits that single-token calls leave
+  // (d=256 N=128 B*h=4, T=128: 181 | 35 us), which callers of such states check.
+  const bool keep_bits = fast && p.rho_dtype == BDH_F32 && state_bytes <= (size_t(512) << 10);
+  const bool dense_auto = !keep_bits && T >= (cached_loop ? 24 : (slow_loop || small_state) ? 8 : 16);
   if (!fixed && !p.bitmask && !p.rows_touched && chunk_fits &&
       (ctx->opt_step_dense >= 0 ? ctx->opt_step_dense == 1 : dense_auto))
     return bdh_launch_state_chunks_f32(ctx, p, out_ln);

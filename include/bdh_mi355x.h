@@ -74,11 +74,11 @@ const char *bdh_last_error(const bdh_ctx *ctx);
 /* Launch-shape knobs for tests and tuning; no counterpart in the reference.
  *   "state_step.split": -1 (default) pick by grid size, 0 = 256 lane pairs per workgroup,
  *                       1 = 64 lane pairs per workgroup of 8 waves (small batches).
- *   "state_step.dense_chunks": -1 (default) a call of 128+ tokens without
- *                       bitmask / row-count outputs runs as dense products on the matrix cores
- *                       (with only a few (sequence, head) slices an f32 RoPE state keeps the token loop;
- *                       from 8 tokens on for an f32 state that every token streams in full -- PoPE,
- *                       eager ALiBi -- or that is at most 64 MiB),
+ *   "state_step.dense_chunks": -1 (default) a call of 16 or more tokens without bitmask / row-count outputs runs as
+ *                       dense products on the matrix cores (from 8 tokens on for an f32 state that is lazily decayed,
+ *                       that every token streams in full -- PoPE, eager ALiBi -- or that is at most 64 MiB; from 24
+ *                       on for an f32 RoPE state of at most 64 MiB; never for one of at most 512 KiB, where a prompt
+ *                       leaves the bits of single-token calls),
  *                       0 = always token by token, 1 = dense products for any T.
  *   "state_step.prompt_bf16": 0 (default) never; T0 > 0: a call of T0 or more tokens on an f32 state, with the
  *                       position given by the host and no bitmask / row-count outputs, runs as
@@ -89,29 +89,22 @@ const char *bdh_last_error(const bdh_ctx *ctx);
  *                       to the prompt calls of bdh_model_forward*.
  *   "state_step.dense_kernel": 1 (default) PoPE and eagerly decayed ALiBi steps at d in {256,512} take
  *                       the dense streaming kernel, 0 = the generic kernel (same values).
- *   "relu_lowrank.mfma_rows": 8 (default) calls with this many rows and at most 64 (N a multiple of 4, d a
- *                       multiple of 32, enough columns for a wavefront per CU) run on the f32 matrix cores, the
- *                       weights streamed once per 32 rows: a chain of v_mfma_f32_32x32x2_f32 over k is the same
- *                       k-sequential fused-multiply-add chain per output, bit for bit; 0 = never; a negative
- *                       value -r takes it from r rows on whatever the width.
- *   "relu_lowrank.gemm_rows": 64 (default) calls with this many tokens per sequence or more (and enough tiles to
- *                       cover the chip) run as one f32 matrix-core product per (sequence, head) with the k order
- *                       of a scalar loop: the same bits again; 0 = never; a negative value -r takes it from
- *                       r tokens on whatever the grid.
- *   "relu_lowrank.scalar": 1 (default) calls with 8 to 63 rows read their inputs through the scalar
- *                       cache, 0 = stage them in LDS (same values).
- *   "relu_lowrank.row": 1 (default) a call with one input row, 128 <= d <= 512 and at most 16 MiB of
- *                       weights takes the kernel that keeps every weight in flight at once, 0 = the
- *                       column-per-thread kernel (same values).
- *   "relu_lowrank.tile": 1 (default) calls with 64+ rows take the 64-row tile kernel (same values) when
- *                       its grid covers the chip, 2 = whenever the shape allows, 0 = never.
- *   "decoder.mfma":     1 (default) the encoder E of a call with 128+ tokens per sequence runs on
- *                       the f32 matrix cores, 0 = always the VALU kernel.
+ *   "relu_lowrank.mfma_rows": 2 (default) calls with this many rows and fewer than 64 (N a multiple of 4, d a multiple
+ *                       of 32) that the row kernel below does not take run on the f32 matrix cores, the weights
+ *                       streamed once per tile of 16 to 64 rows: a chain of v_mfma_f32_16x16x4_f32 over k is the same
+ *                       k-sequential fused-multiply-add chain per output, bit for bit; 0 = never (the sign is ignored).
+ *   "relu_lowrank.gemm_rows": 64 (default) the same for calls with this many rows and at least 64 (any N and d);
+ *                       0 = never (the sign is ignored).
+ *   "relu_lowrank.scalar", "relu_lowrank.tile": accepted (0 to 1, 0 to 2) and without effect: the kernels they chose
+ *                       between are gone.
+ *   "relu_lowrank.row": 1 (default) a call with one input row, or at most 128 outputs per CU, 128 <= d <= 512 and at
+ *                       most 16 MiB of weights takes the kernel that keeps every weight in flight at once, 0 = one of
+ *                       the others (same values).
+ *   "decoder.mfma":     1 (default) the encoder E of a call with 16+ tokens per sequence and 24+ rows runs on
+ *                       the matrix cores, 0 = always the VALU kernel.
  *   "decoder.splitk_rows": 24 (default) a decode step (T = 1) of this many or more sequences runs the
- *                       encoder E as a split-K product on the f32 matrix cores (all of E is streamed
- *                       once) when its tiles cover half the chip; fewer sequences, and small models, take
- *                       the VALU kernel that skips inactive rows of E.  A negative value -r takes the
- *                       matrix-core form from r sequences on whatever the size.
+ *                       encoder E on the matrix cores (all of E is streamed once, K cut into parts); fewer sequences take
+ *                       the VALU kernel that skips inactive rows of E.  The sign is ignored.
  *   "model.one_launch": 1 (default) a decode step (T = 1, no x_tap / viz) of a model that is
  *                       small enough does not run kernel by kernel: a small model (d <= 256 and d % 4 == 0,
  *                       h * N <= 2048 and a multiple of 32, h in {1,2,4,8,16}, V <= 1024) can take ONE launch
@@ -180,8 +173,8 @@ int bdh_rotate(bdh_ctx *ctx, int B, int h, int T, int N, int rotary, const float
  *                        that token (RoPE: both rows of every lane pair with a non-zero
  *                        element; ALiBi/PoPE: Nq)
  *
- * RoPE requires even N (src/model/attention.rs:310).  T = 1 is the decode step.  A call of 128 or more
- * tokens that asks for neither bitmask nor row counts computes the same sums as dense
+ * RoPE requires even N (src/model/attention.rs:310).  T = 1 is the decode step.  A call of 16 or more
+ * tokens (see option "state_step.dense_chunks") that asks for neither bitmask nor row counts computes the same sums as dense
  * products (out = tril(-1)(Q Q^T) V + Q rho, rho += Q^T V, chunks of up to 512 tokens; for ALiBi with
  * the decay powers decay^(t-s), decay^t and decay^(T-s) applied to the three terms) on the matrix
  * cores (a bf16 state is widened to f32 for the call and rounded once at its end).  Large products

@@ -1,0 +1,86 @@
+"""GPU tests of the matrix-core products behind prompts, the stateless forward and batched decoding, at the edges of their
+tiles: rows, columns and reduction lengths just below, at and above a tile or a 32-deep stage, K cut into parts, one slice
+and several, unaligned sizes.
+
+Tolerances.  Split products: what is left out of a product of two f32 is below 2^-23 of it and the sums run over at most a
+few thousand terms in f32, so 2e-5 of the largest value (the bound of the other many-token tests).  Projections: bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import bdh_oracle as orc
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def bda():
+    if not torch.cuda.is_available():
+        pytest.fail("no HIP device: the GPU tests must run on the MI355X box")
+    import burn_dragon_amd
+
+    return burn_dragon_amd
+
+
+def rel_err(a, b):
+    a, b = np.asarray(a, np.float64), np.asarray(b, np.float64)
+    return np.abs(a - b).max() / max(np.abs(b).max(), 1e-30)
+
+
+@pytest.mark.parametrize("B,h,T,N,d", [(1, 1, 8, 34, 64), (2, 3, 31, 130, 68), (1, 4, 33, 2080, 128), (3, 4, 65, 512, 256),
+                                       (1, 2, 127, 4096, 260), (1, 1, 129, 62, 512), (5, 2, 16, 96, 192)])
+@pytest.mark.parametrize("rotary", ["rope", "alibi"])
+def test_many_token_step_at_tile_edges(bda, corc, B, h, T, N, d, rotary):
+    from burn_dragon_amd.recurrent import recurrent_attention
+
+    rng = np.random.default_rng(T + N)
+    x = np.maximum(rng.standard_normal((B, h, T, N)) - 0.3, 0).astype(np.float32)
+    v = rng.standard_normal((B, T, d)).astype(np.float32)
+    rho = (0.1 * rng.standard_normal((B, h, N, d))).astype(np.float32)
+    rot = {"rope": orc.ROPE, "alibi": orc.ALIBI}[rotary]
+    freqs = corc.build_freqs(N, rotary=rot)
+    slopes = corc.default_alibi_slopes(h) if rotary == "alibi" else None
+    q = corc.rotate(x, freqs, rot, 17).astype(np.float64)
+    # the token loop in float64
+    out, state = np.zeros((B, h, T, d)), rho.astype(np.float64)
+    decay = np.ones(h) if slopes is None else np.exp(-np.asarray(slopes, np.float32)).astype(np.float64)
+    for t in range(T):
+        out[:, :, t] = np.einsum("bhn,bhnd->bhd", q[:, :, t], state)
+        state = (state + q[:, :, t, :, None] * v[:, None, t, None, :]) * decay[None, :, None, None]
+    rho_t = torch.from_numpy(rho).to(DEV)
+    ctx = bda.ffi.default_context(0)
+    try:
+        ctx.set_option("state_step.dense_chunks", 1)
+        got = recurrent_attention(torch.from_numpy(x).to(DEV), torch.from_numpy(v).to(DEV), rho_t, torch.from_numpy(freqs).to(DEV),
+                                  17, bda.RotaryEmbedding.parse(rotary))
+    finally:
+        ctx.set_option("state_step.dense_chunks", -1)
+    assert rel_err(got.cpu().numpy(), out) < 2e-5
+    assert rel_err(rho_t.cpu().numpy(), state) < 2e-5
+
+
+@pytest.mark.parametrize("M,T,d,h,N", [(2, 1, 32, 1, 4), (15, 1, 64, 3, 68), (16, 16, 96, 2, 60), (17, 1, 256, 4, 1040), (33, 11, 128, 2, 9000),
+                                       (63, 7, 512, 2, 132), (64, 1, 512, 3, 66), (65, 13, 192, 4, 8256), (129, 43, 160, 1, 260),
+                                       (520, 130, 64, 8, 16384), (70, 5, 36, 2, 70)])
+def test_relu_lowrank_rows_at_tile_edges(bda, corc, M, T, d, h, N):
+    """Every tile height (16, 32, 64, 128 rows), rows and columns that end inside a tile, and the unaligned fallback give the
+    bits of the k-sequential chain, with and without gate."""
+    from burn_dragon_amd.kernel import relu_lowrank
+
+    rng = np.random.default_rng(M + N)
+    B = M // T
+    inp = (rng.standard_normal((B, h, T, d)) * np.exp2(rng.integers(-20, 8, (B, h, T, d)))).astype(np.float32)
+    weight = (rng.standard_normal((h, d, N)) * np.exp2(rng.integers(-30, 8, (h, d, N)))).astype(np.float32)
+    gate = np.maximum(rng.standard_normal((B, h, T, N)), 0).astype(np.float32)
+    ref = corc.relu_lowrank(inp, weight)
+    args = (torch.from_numpy(inp).to(DEV), torch.from_numpy(weight).to(DEV), None, 0.0, bda.BlockPattern1d.dense(64))
+    ctx = bda.ffi.default_context(0)
+    try:
+        ctx.set_option("relu_lowrank.row", 0)
+        got = relu_lowrank.fused_forward(*args).cpu().numpy()
+        gated = relu_lowrank.fused_forward(*args, gate=torch.from_numpy(gate).to(DEV)).cpu().numpy()
+    finally:
+        ctx.set_option("relu_lowrank.row", 1)
+    assert np.array_equal(got, ref)
+    assert np.array_equal(gated, gate * ref)
