@@ -502,7 +502,7 @@ int bdh_model_forward_fast_ex(bdh_model *m, const int64_t *tokens, int B, int T,
     rc = bdh_fused_state_aligned(ctx, B, h, T, N, d, x, cur, m->freqs, c.rotary == BDH_ALIBI ? m->slopes : nullptr, block,
                                  time_pairs_host, n_time_pairs, c.rotary, 1, attn);
     if (rc != BDH_OK) return rc;
-    rc = bdh_launch_layer_norm(ctx, (int64_t)M * h, d, attn, attn_ln);  // :132
+    rc = bdh_launch_layer_norm_rows(ctx, (int64_t)M * h, d, attn, attn_ln);  // :132
     if (rc != BDH_OK) return rc;
     ReluLowrankParams py{B, h, T, d, h, N, attn_ln, m->w.encoder_v, nullptr, c.relu_threshold, lat_block, latent_blocks_host,
                          n_latent_blocks, x, xy};

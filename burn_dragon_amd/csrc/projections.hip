@@ -429,15 +429,20 @@ __device__ __forceinline__ void ln_stats_in_order(const float *s_row, int d, flo
   den = sqrtf(sq / (float)d + kLnEps);
 }
 
-__global__ __launch_bounds__(256) void k_layer_norm(const float *__restrict__ in, float *__restrict__ out, int d) {
-  extern __shared__ float s_row[];
-  const float *x = in + (long)blockIdx.x * d;
-  float *y = out + (long)blockIdx.x * d;
-  for (int c = threadIdx.x; c < d; c += 256) s_row[c] = x[c];
+// One wavefront per row, blockDim.x / 64 rows per workgroup: the index-order sums are the same work in every lane, so more
+// wavefronts on a row only repeat it (a workgroup of four per row: 25 against 12 us for the embedding of 4088 tokens).
+__global__ void k_layer_norm(const float *__restrict__ in, float *__restrict__ out, int d, long rows) {
+  extern __shared__ float s_rows[];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const long row = (long)blockIdx.x * (blockDim.x >> 6) + wave;
+  float *s_row = s_rows + (long)wave * ((d + 3) & ~3);
+  if (row < rows)
+    for (int c = lane; c < d; c += 64) s_row[c] = in[row * d + c];
   __syncthreads();
+  if (row >= rows) return;
   float mean, den;
   ln_stats_in_order(s_row, d, mean, den);
-  for (int c = threadIdx.x; c < d; c += 256) y[c] = (s_row[c] - mean) / den;
+  for (int c = lane; c < d; c += 64) out[row * d + c] = (s_row[c] - mean) / den;
 }
 
 // LayerNorm of many rows for internal use (the readout of a many-token state step): one wave per row, the
@@ -472,22 +477,26 @@ __global__ __launch_bounds__(256) void k_layer_norm_wave(const float *__restrict
     if (j * 64 + lane < d) y[j * 64 + lane] = (v[j] - mean) / den;
 }
 
-// embed gather + LayerNorm (src/model/bdh.rs:319-322)
-__global__ __launch_bounds__(256) void k_embed_ln(const int64_t *__restrict__ tokens, int d, int V,
-                                                  const float *__restrict__ embed, float *__restrict__ out) {
-  extern __shared__ float s_row[];
-  const int64_t tok = tokens[blockIdx.x];
-  float *y = out + (long)blockIdx.x * d;
-  if (tok < 0 || tok >= V) {  // the reference's gather would panic; poison the row instead
-    for (int c = threadIdx.x; c < d; c += 256) y[c] = __int_as_float(0x7fc00000);
+// embed gather + LayerNorm (src/model/bdh.rs:319-322), a wavefront per row like k_layer_norm
+__global__ void k_embed_ln(const int64_t *__restrict__ tokens, int d, int V, const float *__restrict__ embed,
+                           float *__restrict__ out, long rows) {
+  extern __shared__ float s_rows[];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const long row = (long)blockIdx.x * (blockDim.x >> 6) + wave;
+  float *s_row = s_rows + (long)wave * ((d + 3) & ~3);
+  const int64_t tok = row < rows ? tokens[row] : -1;
+  const bool known = tok >= 0 && tok < V;
+  if (known)
+    for (int c = lane; c < d; c += 64) s_row[c] = embed[tok * d + c];
+  __syncthreads();
+  if (row >= rows) return;
+  if (!known) {  // the reference's gather would panic; poison the row instead
+    for (int c = lane; c < d; c += 64) out[row * d + c] = __int_as_float(0x7fc00000);
     return;
   }
-  const float *x = embed + (long)tok * d;
-  for (int c = threadIdx.x; c < d; c += 256) s_row[c] = x[c];
-  __syncthreads();
   float mean, den;
   ln_stats_in_order(s_row, d, mean, den);
-  for (int c = threadIdx.x; c < d; c += 256) y[c] = (s_row[c] - mean) / den;
+  for (int c = lane; c < d; c += 64) out[row * d + c] = (s_row[c] - mean) / den;
 }
 
 // ------------------------------------------------------------------------------------
@@ -818,6 +827,172 @@ __global__ __launch_bounds__(1024) void k_decoder_finalize(const float *__restri
   lm_head_row(s_grp[2], s_grp[3], s_best, s_arg, m, head.lm_head, head.T, d, head.V, head.logits, head.next_tokens);
 }
 
+// k_decoder_finalize<false> for many rows: a wavefront per row, the partials of a column added in the same order (sixteen
+// groups, each in index order), then the same wave-wide LayerNorms, so the same bits.  What bounds it: the reads of the
+// partials; a workgroup of sixteen wavefronts per row spends most of its time in its one barrier once the rows alone fill
+// the chip (4088 rows of 256, 4 partials: 56 against 10 us).
+__global__ __launch_bounds__(256) void k_decoder_finalize_rows(const float *__restrict__ partial, int KBN, int M, int d,
+                                                               float *__restrict__ cur) {
+  const int lane = threadIdx.x & 63;
+  const long m = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (m >= M) return;
+  const int per = (KBN + 15) >> 4;
+  float vals[16], res[16];
+  float s = 0.0f;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) res[j] = j * 64 + lane < d ? cur[m * d + j * 64 + lane] : 0.0f;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    vals[j] = 0.0f;
+    const int c = j * 64 + lane;
+    if (c < d) {
+      const float *p = partial + m * d + c;
+      const long step = (long)M * d;
+      float v = 0.0f, t = 0.0f;
+      int in_group = 0;
+      for (int kb = 0; kb < KBN; kb += 8) {  // eight partials in flight
+        float x[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) x[u] = p[min(kb + u, KBN - 1) * step];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+          if (kb + u < KBN) {
+            t = in_group == 0 ? x[u] : t + x[u];
+            if (++in_group == per || kb + u == KBN - 1) {
+              v = kb + u < per ? t : v + t;
+              in_group = 0;
+            }
+          }
+      }
+      vals[j] = v;
+      s += v;
+    }
+  }
+  auto wave_sum = [](float v) {
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    return v;
+  };
+  auto spread = [&](float mean) {  // sqrt(var + eps)
+    float q = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+      if (j * 64 + lane < d) {
+        const float t = vals[j] - mean;
+        q += t * t;
+      }
+    return sqrtf(wave_sum(q) / (float)d + kLnEps);
+  };
+  float mean = wave_sum(s) / (float)d;
+  float den = spread(mean);
+  s = 0.0f;
+#pragma unroll
+  for (int j = 0; j < 16; ++j)
+    if (j * 64 + lane < d) {
+      const float mlp = (vals[j] - mean) / den;
+      vals[j] = res[j] + mlp;
+      s += vals[j];
+    }
+  mean = wave_sum(s) / (float)d;
+  den = spread(mean);
+#pragma unroll
+  for (int j = 0; j < 16; ++j)
+    if (j * 64 + lane < d) cur[m * d + j * 64 + lane] = (vals[j] - mean) / den;
+}
+
+// The output head of many rows: RT rows share every weight that is read, a thread per vocabulary column; each logit is the
+// same four k-sequential chains as in lm_head_row, added in order.  (One row per workgroup reads all of W again for every
+// row: 66 against 24 us for 4088 rows, d = 256, V = 256.)  With next_tokens the greedy token of a sequence's last row.
+template <int RT>
+__global__ __launch_bounds__(256) void k_lm_head_rows(const float *__restrict__ cur, const float *__restrict__ W, int M,
+                                                      int T, int d, int V, float *__restrict__ logits,
+                                                      int64_t *__restrict__ next_tokens) {
+  extern __shared__ float s_x[];  // [d][RT]
+  __shared__ float s_best[4];
+  __shared__ int s_arg[4];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int m0 = blockIdx.x * RT;
+  for (int i = tid; i < RT * d; i += 256) {
+    const int r = i / d, k = i - r * d;
+    s_x[k * RT + r] = cur[(long)min(m0 + r, M - 1) * d + k];
+  }
+  __syncthreads();
+  const int per = (d + 3) >> 2;
+  float best[RT];
+  int arg[RT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r) {
+    best[r] = -INFINITY;
+    arg[r] = 0x7fffffff;
+  }
+  for (int c0 = 0; c0 < V; c0 += 256) {
+    const int c = c0 + tid, cc = min(c, V - 1);
+    float sum[RT];
+    for (int grp = 0; grp < 4; ++grp) {
+      const int k0 = grp * per, k1 = min(d, k0 + per);
+      float acc[RT];
+#pragma unroll
+      for (int r = 0; r < RT; ++r) acc[r] = 0.0f;
+      int k = k0;
+      for (; k + 32 <= k1; k += 32) {  // 32 independent loads in flight, then the chains
+        float w[32];
+#pragma unroll
+        for (int u = 0; u < 32; ++u) w[u] = W[(long)(k + u) * V + cc];
+#pragma unroll
+        for (int u = 0; u < 32; ++u)
+#pragma unroll
+          for (int r = 0; r < RT; ++r) acc[r] = __builtin_fmaf(s_x[(k + u) * RT + r], w[u], acc[r]);
+      }
+      for (; k < k1; ++k) {
+        const float w = W[(long)k * V + cc];
+#pragma unroll
+        for (int r = 0; r < RT; ++r) acc[r] = __builtin_fmaf(s_x[k * RT + r], w, acc[r]);
+      }
+#pragma unroll
+      for (int r = 0; r < RT; ++r) sum[r] = grp == 0 ? acc[r] : sum[r] + acc[r];
+    }
+    if (c < V) {
+#pragma unroll
+      for (int r = 0; r < RT; ++r) {
+        if (m0 + r < M) logits[(long)(m0 + r) * V + c] = sum[r];
+        if (sum[r] > best[r]) {  // increasing c: keeps the lowest index on ties
+          best[r] = sum[r];
+          arg[r] = c;
+        }
+      }
+    }
+  }
+  if (!next_tokens) return;
+#pragma unroll
+  for (int r = 0; r < RT; ++r) {
+    const int m = m0 + r;
+    if (m >= M || m % T != T - 1) continue;  // uniform over the workgroup
+    float bv = best[r];
+    int ba = arg[r];
+    for (int o = 32; o > 0; o >>= 1) {
+      const float ob = __shfl_xor(bv, o);
+      const int oa = __shfl_xor(ba, o);
+      if (ob > bv || (ob == bv && oa < ba)) {
+        bv = ob;
+        ba = oa;
+      }
+    }
+    __syncthreads();  // the previous row's result has been read
+    if (lane == 0) {
+      s_best[wave] = bv;
+      s_arg[wave] = ba;
+    }
+    __syncthreads();
+    if (tid == 0) {
+      for (int w = 1; w < 4; ++w)
+        if (s_best[w] > bv || (s_best[w] == bv && s_arg[w] < ba)) {
+          bv = s_best[w];
+          ba = s_arg[w];
+        }
+      next_tokens[m / T] = ba == 0x7fffffff ? 0 : ba;
+    }
+  }
+}
+
 __global__ __launch_bounds__(1024) void k_lm_head(const float *__restrict__ cur, const float *__restrict__ W,
                                                   int T, int d, int V, float *__restrict__ logits,
                                                   int64_t *__restrict__ next_tokens) {
@@ -933,10 +1108,17 @@ int bdh_launch_relu_lowrank(bdh_ctx *ctx, const ReluLowrankParams &p) {
   return BDH_OK;
 }
 
+// rows of an index-order LayerNorm kernel per workgroup: four, fewer when they would not fit in LDS
+static int ln_rows_per_wg(int d) { return d <= 4096 ? 4 : 1; }
+static size_t ln_lds(int d) { return sizeof(float) * (size_t)((d + 3) & ~3) * ln_rows_per_wg(d); }
+
 int bdh_launch_layer_norm(bdh_ctx *ctx, int64_t rows, int d, const float *in, float *out) {
   if (rows > 0x7fffffffL) return bdh_fail(ctx, BDH_E_SHAPE, "too many rows");
   if (d > 16384) return bdh_fail(ctx, BDH_E_SHAPE, "LayerNorm row of %d floats does not fit in LDS", d);
-  hipLaunchKernelGGL(k_layer_norm, dim3((unsigned)rows), dim3(256), sizeof(float) * (size_t)d, ctx->stream, in, out, d);
+  if (rows == 0) return BDH_OK;
+  const int per = ln_rows_per_wg(d);
+  hipLaunchKernelGGL(k_layer_norm, dim3((unsigned)((rows + per - 1) / per)), dim3(64 * per), ln_lds(d), ctx->stream, in, out,
+                     d, (long)rows);
   BDH_LAUNCH_CHECK(ctx, "k_layer_norm");
   return BDH_OK;
 }
@@ -953,18 +1135,40 @@ int bdh_launch_layer_norm_rows(bdh_ctx *ctx, int64_t rows, int d, const float *i
 
 int bdh_launch_embed_ln(bdh_ctx *ctx, const int64_t *tokens, int64_t rows, int d, int V, const float *embed,
                         float *out) {
-  hipLaunchKernelGGL(k_embed_ln, dim3((unsigned)rows), dim3(256), sizeof(float) * (size_t)d, ctx->stream, tokens, d, V, embed, out);
+  if (rows == 0) return BDH_OK;
+  const int per = ln_rows_per_wg(d);
+  hipLaunchKernelGGL(k_embed_ln, dim3((unsigned)((rows + per - 1) / per)), dim3(64 * per), ln_lds(d), ctx->stream, tokens, d,
+                     V, embed, out, (long)rows);
   BDH_LAUNCH_CHECK(ctx, "k_embed_ln");
   return BDH_OK;
 }
 
+// From this many rows on they fill the chip a wavefront (second stage) or four to a workgroup (head) each; fewer rows want
+// many wavefronts on one row: with 4 to 32 partials to add, one wavefront is a chain of trips to memory.
+constexpr int kManyRows = 256;
+
+static void launch_lm_head(bdh_ctx *ctx, int M, int T, int d, int V, const float *cur, const float *lm_head, float *logits,
+                           int64_t *next_tokens) {
+  constexpr int RT = 4;
+  if (M >= kManyRows && sizeof(float) * RT * (size_t)d <= 64 * 1024)
+    hipLaunchKernelGGL((k_lm_head_rows<RT>), dim3((M + RT - 1) / RT), dim3(256), sizeof(float) * RT * (size_t)d, ctx->stream,
+                       cur, lm_head, M, T, d, V, logits, next_tokens);
+  else
+    hipLaunchKernelGGL(k_lm_head, dim3(M), dim3(1024), sizeof(float) * ((size_t)d + 1024), ctx->stream, cur, lm_head, T, d, V,
+                       logits, next_tokens);
+}
+
 static void launch_decoder_finalize(bdh_ctx *ctx, const float *partial, int KBN, int M, int d, float *cur,
                                     const DecoderHead *head) {
-  if (head)
+  if (M >= kManyRows) {
+    hipLaunchKernelGGL(k_decoder_finalize_rows, dim3((M + 3) / 4), dim3(256), 0, ctx->stream, partial, KBN, M, d, cur);
+    if (head) launch_lm_head(ctx, M, head->T, d, head->V, cur, head->lm_head, head->logits, head->next_tokens);
+  } else if (head) {
     hipLaunchKernelGGL(k_decoder_finalize<true>, dim3(M), dim3(1024), 0, ctx->stream, partial, KBN, M, d, cur, *head);
-  else
+  } else {
     hipLaunchKernelGGL(k_decoder_finalize<false>, dim3(M), dim3(1024), 0, ctx->stream, partial, KBN, M, d, cur,
                        DecoderHead{});
+  }
 }
 
 int bdh_launch_decoder_residual(bdh_ctx *ctx, int B, int T, int h, int N, int d, const float *xy,
@@ -1080,9 +1284,7 @@ int bdh_launch_decoder_finalize(bdh_ctx *ctx, const float *partial, int KBN, int
 
 int bdh_launch_lm_head(bdh_ctx *ctx, int B, int T, int d, int V, const float *cur, const float *lm_head,
                        float *logits, int64_t *next_tokens) {
-  const int M = B * T;
-  hipLaunchKernelGGL(k_lm_head, dim3(M), dim3(1024), sizeof(float) * ((size_t)d + 1024), ctx->stream, cur, lm_head,
-                     T, d, V, logits, next_tokens);
+  launch_lm_head(ctx, B * T, T, d, V, cur, lm_head, logits, next_tokens);
   BDH_LAUNCH_CHECK(ctx, "k_lm_head");
   return BDH_OK;
 }

@@ -84,3 +84,20 @@ def test_relu_lowrank_rows_at_tile_edges(bda, corc, M, T, d, h, N):
         ctx.set_option("relu_lowrank.row", 1)
     assert np.array_equal(got, ref)
     assert np.array_equal(gated, gate * ref)
+
+
+@pytest.mark.parametrize("T,V,d", [(86, 69, 128), (100, 300, 260), (128, 256, 192)])
+def test_many_rows_through_the_second_stage_and_the_head(bda, T, V, d):
+    """256 rows and more take a wavefront per row in the encoder's second stage and share the head's weights: the same rows in
+    three smaller calls give the same logits to the rounding of the products before them (1e-5), the same greedy tokens."""
+    cfg = bda.BDHConfig(n_layer=2, n_embd=d, n_head=2, mlp_internal_dim_multiplier=2, vocab_size=V)
+    cfg.fused_kernels.set_rotary_embedding(bda.RotaryEmbedding.ALIBI)
+    model = bda.BDH(cfg, DEV, seed=5)
+    tokens = torch.randint(0, V, (3, T), generator=torch.Generator().manual_seed(T))
+    logits, nxt = model.forward_with_state(tokens, model.init_state(), want_next=True)
+    fast = model.forward_fast(tokens)
+    for b in range(3):
+        one, n1 = model.forward_with_state(tokens[b:b + 1], model.init_state(), want_next=True)
+        assert rel_err(logits[b].cpu().numpy(), one[0].cpu().numpy()) < 1e-5
+        assert rel_err(fast[b].cpu().numpy(), model.forward_fast(tokens[b:b + 1])[0].cpu().numpy()) < 1e-5
+        assert int(nxt[b]) == int(n1[0]) == int(logits[b, -1].argmax())
