@@ -7,17 +7,16 @@
 // Stages (all stream-ordered on the context's stream):
 //   1. k_rope_bf16      Q = bf16(rope_f32(x)); the sin/cos of a (t, pair) is computed once and
 //                       reused for every (b,h) slice.
-//   2. k_gemm<SCORES>   S = tril(-1)(Q Q^T) as bf16, lower-triangular 256x256 tiles only, K = N.
-//   3. k_gemm<ACC>      out = S V  (K limited to the causal extent of each row tile)
+//   2. scores           S = tril(-1)(Q Q^T) as bf16, lower-triangular tiles only, K = N.
+//   3. out              S V  (K limited to the causal extent of each row tile)
 //                       (+ Q rho0 first when the state is not known to be zero)
-//   4. k_gemm<ACC>      rho += Q^T V
-// One GEMM kernel serves all products: C[m,n] = sum_k A[m,k] B[n,k] with 256x256x64 workgroup
-// tiles, 8 wavefronts (2x4) of 128x64 each, v_mfma_f32_32x32x16_bf16, f32 accumulators.  B is
+//   4. state            rho += Q^T V
+// All are products C[m,n] = sum_k A[m,k] B[n,k] on v_mfma_f32_32x32x16_bf16 with f32 accumulators: k_gemm_tile
+// (64x64 and 128x128 tiles) and, for many slices, k_gemm_direct (256x256).  B is
 // always k-contiguous in memory (V and rho0 are transposed once by a small kernel).  A is either
 // k-contiguous (copied to LDS as is, fragments read with one 16-byte LDS load) or, for Q^T V,
 // k-major (Q [T,N] with the reduction over T): that tile is also copied as is, [k][m], and the
-// fragments are read with the transposing LDS load of gfx950 (ds_read_b64_tr_b16); a 64-byte
-// column swizzle on every other group of eight k rows keeps the two half-waves on different banks.
+// fragments are read with the transposing LDS load of gfx950 (ds_read_b64_tr_b16).
 #include <algorithm>
 #include <atomic>
 #include <cmath>
@@ -35,7 +34,7 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 constexpr float kTwoPi = 6.28318530717958647692f;
 constexpr int BM = 256, BN = 256, BK = 64;
-constexpr int LDS_STRIDE = BK + 8;  // bf16 elements per LDS row: 144 bytes, conflict-free b128 reads
+constexpr long kFullChip = 256;  // workgroups from which a larger tile pays: one per CU
 
 __device__ __forceinline__ unsigned short f32_to_bf16_bits(float f) {
   unsigned int u = __float_as_uint(f);
@@ -186,16 +185,16 @@ __global__ __launch_bounds__(256) void k_pope_bf16(const uint4 *__restrict__ x, 
   }
 }
 
-// denom[slice][row] = sum over the column tiles of norm_part + eps (src/kernel/linear_attention.rs:8,108), in tile
-// order; tri: only the tiles up to the row's own exist
+// denom[slice][row] = sum over the 64-column groups of norm_part + eps (src/kernel/linear_attention.rs:8,108), in
+// order, so that the tile does not show in the bits; tri: only the tiles up to the row's own exist
 __global__ __launch_bounds__(256) void k_norm_reduce(const float *__restrict__ norm_part, float *__restrict__ denom,
-                                                     int M, int nt, int tri, float eps) {
+                                                     int M, int groups, int tile, int tri, float eps) {
   const int row = blockIdx.x * 256 + threadIdx.x;
   const long slice = blockIdx.y;
   if (row >= M) return;
-  const int last = tri ? row / BM : nt - 1;
+  const int end = tri ? min(groups, (row / tile + 1) * (tile / 64)) : groups;
   float sum = 0.0f;
-  for (int tj = 0; tj <= last; ++tj) sum += norm_part[(slice * nt + tj) * M + row];
+  for (int q = 0; q < end; ++q) sum += norm_part[(slice * groups + q) * M + row];
   denom[slice * M + row] = sum + eps;
 }
 
@@ -232,8 +231,13 @@ struct GemmArgs {
   int mode;            // GM_* bits
   int h;               // heads: slice % h selects head_par
   int block_size;      // GM_ADD_ALIBI: tokens per time block of the causal layout
-  float *norm_part;    // GM_ROWNORM: [slice][nt][M] sums of |S| per column tile
+  float *norm_part;    // GM_ROWNORM: [slice][norm_groups][M] sums of |S| per 64 columns, whatever the tile
+  int norm_groups;
   const float *denom;  // GM_DIVNORM: [slice][M]
+  // k_gemm_tile only: a second pair whose products continue the sums, K limited to the causal extent of the row tile
+  const void *A2, *B2;
+  long a2_batch, b2_batch;
+  int lda2, ldb2, K2, b2_div;
   float head_par[64];  // per head: log of the per-token decay factor, or the additive slope
 };
 
@@ -252,7 +256,7 @@ __device__ __forceinline__ void gemm_epilogue_x(const GemmArgs &g, f32x16 (&acc)
       for (int e = 0; e < 16; ++e) {
         const int row = m0 + wm * 128 + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
         const int rblk = (g.mode & GM_ADD_ALIBI) ? row / bs : 0;
-        float rsum = 0.0f;
+        float rsum[2];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
           const int col = n0 + wn * 64 + j * 32 + (lane & 31);
@@ -262,19 +266,24 @@ __device__ __forceinline__ void gemm_epilogue_x(const GemmArgs &g, f32x16 (&acc)
           if (col >= g.N) v = 0.0f;  // padding columns of the score matrix
           const unsigned short bits = f32_to_bf16_bits(v);
           if (row < g.M && col < g.ldc) C[(long)row * g.ldc + col] = bits;
-          rsum += fabsf(bf16_bits_to_f32(bits));  // what the next product multiplies with
+          rsum[j] = fabsf(bf16_bits_to_f32(bits));  // what the next product multiplies with
         }
         if (g.mode & GM_ROWNORM) {
 #pragma unroll
-          for (int off = 16; off >= 1; off >>= 1) rsum += __shfl_xor(rsum, off);  // the 32 columns of a half-wave
-          if ((lane & 31) == 0) s_red[wn * 256 + wm * 128 + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3)] = rsum;
+          for (int j = 0; j < 2; ++j)  // the 32 columns of a half-wave
+#pragma unroll
+            for (int off = 16; off >= 1; off >>= 1) rsum[j] += __shfl_xor(rsum[j], off);
+          if ((lane & 31) == 0)
+            s_red[wn * 256 + wm * 128 + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3)] = rsum[0] + rsum[1];
         }
       }
     if (g.mode & GM_ROWNORM) {
       __syncthreads();
       if (tid < 256 && m0 + tid < g.M) {
-        const float sum = ((s_red[tid] + s_red[256 + tid]) + s_red[512 + tid]) + s_red[768 + tid];
-        g.norm_part[((long)slice * g.nt + tj) * g.M + m0 + tid] = sum;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (n0 + q * 64 < g.N)
+            g.norm_part[((long)slice * g.norm_groups + n0 / 64 + q) * g.M + m0 + tid] = s_red[q * 256 + tid];
       }
     }
   } else {
@@ -303,25 +312,53 @@ __device__ __forceinline__ void gemm_epilogue_x(const GemmArgs &g, f32x16 (&acc)
   }
 }
 
-// bf16 elements per k row of a k-major tile in LDS: 576 bytes = 64 mod 256, so the four k rows of 64 bytes
-// that 32 lanes of a transposing read touch fall on disjoint quarters of the 64 banks
-constexpr int KM_STRIDE = BM + 32;
+// 16 zero bytes: what a lane copies where its piece lies outside the operand (a padding row, or k beyond the end)
+__device__ const uint4 g_zero_piece = {0u, 0u, 0u, 0u};
 
-template <bool A_KMAJOR, int EPI>
-__global__ __launch_bounds__(512) void k_gemm(GemmArgs g) {
-  __shared__ __attribute__((aligned(16))) unsigned short s_a[BM * LDS_STRIDE];
-  __shared__ __attribute__((aligned(16))) unsigned short s_b[BN * LDS_STRIDE];
-  static_assert(BK * KM_STRIDE <= BM * LDS_STRIDE, "k-major tile must fit");
+// Copies 16 bytes per lane from *src to LDS, the 64 lanes' pieces one after the other from dst (uniform over the
+// wavefront).  Written out because the compiler waits for every copy that it knows of before any LDS read that might
+// see it; in k_gemm_tile the counted wait and the barrier at the start of a stage order the two.
+typedef __attribute__((address_space(3))) void *lds_dst_t;
+__device__ __forceinline__ void copy_piece_to_lds(const void *src, unsigned short *dst) {
+  const unsigned int at = __builtin_amdgcn_readfirstlane((unsigned int)(uintptr_t)(lds_dst_t)dst);
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(at), "v"(src) : "memory");
+}
 
-  // XCD-aware mapping: workgroup ids are dealt round-robin to the 8 XCDs, so workgroups with the
-  // same (id % 8) share an L2; all tiles of one slice go to one XCD.
-  const int xcd = blockIdx.x & 7;
-  const int r = blockIdx.x >> 3;
-  const int slice = xcd + 8 * (r / g.n_tiles);
-  if (slice >= g.n_slices) return;
+// Workgroup barrier that orders LDS accesses only: global loads and stores issued before it stay in flight
+// (__syncthreads also waits for every outstanding global access).
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+constexpr int tile_stages(int TS) { return TS == 64 ? 4 : 2; }
+constexpr int tile_lds_bytes(int TS) { return tile_stages(TS) * 2 * TS * BK * 2; }  // 64 KiB either way: two per CU
+
+// One k step (64) of a TS x TS tile is two panels of TS * 128 bytes, copied straight into LDS by 16-byte pieces, zeros
+// for what lies outside the operands, tile_stages - 1 steps ahead of the products.  A row-major panel keeps 8 pieces a
+// row, piece c of row R at c ^ (R/2 % 8); a k-major panel keeps its k rows, whose 64-byte parts are turned so that the
+// four k rows a transposing read touches lie on different banks.
+// A = A2 behind it continues the same sums (Q rho0 and then S V), the rows scaled in between when the state decays.
+// Every sum runs over k in order, so the tile size does not change a bit of the result.
+// What bounds it with few slices is the wait for the next step's operands, hence small tiles, a list dealt evenly to the
+// XCDs and copies several steps ahead.  A call of 12 slices, 777 tokens, N = 4096, d = 256 took 506 us with 256 x 256
+// tiles staged through registers and whole slices dealt to XCDs, 248 us with this; 4 slices of 64 tokens 352 -> 93 us.
+template <int TS, bool A_KMAJOR, bool SCORES>
+__global__ __launch_bounds__(256, 2) void k_gemm_tile(GemmArgs g) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned short s_dyn[];
+  constexpr int NS = tile_stages(TS), PANEL = TS * BK, STAGE = 2 * PANEL;
+  constexpr int MI = TS / 64;          // 32 x 32 accumulators per wave and direction
+  constexpr int NP = TS * BK / 8 / 256;  // pieces per thread and panel
+  // Workgroup ids are dealt round-robin to the XCDs: each XCD takes an equal run of the (slice, tile) list, so that a few
+  // slices still fill the chip and the tiles of a slice mostly meet in one L2.
+  const int total = g.n_slices * g.n_tiles, per = (total + 7) >> 3;
+  const int at = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per || at >= total) return;
+  const int slice = at / g.n_tiles;
   int ti, tj;
   {
-    const int t = r % g.n_tiles;
+    const int t = at - slice * g.n_tiles;
     if (g.tri) {  // t = i(i+1)/2 + j, 0 <= j <= i
       int i = (int)((sqrtf(8.0f * (float)t + 1.0f) - 1.0f) * 0.5f);
       while (i * (i + 1) / 2 > t) --i;
@@ -333,153 +370,220 @@ __global__ __launch_bounds__(512) void k_gemm(GemmArgs g) {
       tj = t % g.nt;
     }
   }
-  const int m0 = ti * BM, n0 = tj * BN;
-
+  const int m0 = ti * TS, n0 = tj * TS;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 2, wn = wave & 3;  // 2 x 4 waves, 128 x 64 each
+  const int wm = wave >> 1, wn = wave & 1;  // 2 x 2 waves, TS/2 x TS/2 each
 
-  const unsigned short *A = static_cast<const unsigned short *>(g.A) + (long)slice * g.a_batch;
-  const unsigned short *Bh = static_cast<const unsigned short *>(g.B) + (long)(slice / g.b_div) * g.b_batch;
-
-  int K = g.K;
-  if (g.causal_k) K = min(K, m0 + BM);
-
-  f32x16 acc[4][2];
+  f32x16 acc[MI][MI];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < MI; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < MI; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
 
-  // staging registers: 4 chunks of 8 elements per operand per thread
-  uint4 ra[4], rb[4];
-
-  auto load_a = [&](int k0) {
+  // the k loop over one pair of operands
+  auto products = [&](const unsigned short *A, int lda, const unsigned short *B, int ldb, int K) {
+    const unsigned short *zero = reinterpret_cast<const unsigned short *>(&g_zero_piece);
+    const int kc = ((tid & 7) ^ ((tid >> 4) & 7)) * 8;  // this thread's k piece of a row-major panel
+    const unsigned short *pa[NP], *pb[NP];
+    bool va[NP], vb[NP];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int chunk = c * 512 + tid;  // 2048 chunks of 8 elements
-      uint4 v = make_uint4(0u, 0u, 0u, 0u);
+    for (int c = 0; c < NP; ++c) {
+      const int piece = c * 256 + tid, row = piece >> 3;
+      vb[c] = n0 + row < g.N;
+      pb[c] = B + (long)(n0 + row) * ldb + kc;
       if (!A_KMAJOR) {
-        const int row = chunk >> 3, kc = (chunk & 7) * 8;  // 8 chunks per row of 64 k
-        if (m0 + row < g.M && k0 + kc < K) v = *reinterpret_cast<const uint4 *>(A + (long)(m0 + row) * g.lda + k0 + kc);
+        va[c] = m0 + row < g.M;
+        pa[c] = A + (long)(m0 + row) * lda + kc;
       } else {
-        const int kr = chunk >> 5, mc = (chunk & 31) * 8;  // 32 chunks per k row of 256 m
-        if (k0 + kr < K && m0 + mc < g.M) v = *reinterpret_cast<const uint4 *>(A + (long)(k0 + kr) * g.lda + m0 + mc);
-      }
-      ra[c] = v;
-    }
-  };
-  auto load_b = [&](int k0) {
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int chunk = c * 512 + tid;
-      const int row = chunk >> 3, kc = (chunk & 7) * 8;
-      uint4 v = make_uint4(0u, 0u, 0u, 0u);
-      if (n0 + row < g.N && k0 + kc < K) v = *reinterpret_cast<const uint4 *>(Bh + (long)(n0 + row) * g.ldb + k0 + kc);
-      rb[c] = v;
-    }
-  };
-  auto store_tiles = [&]() {
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int chunk = c * 512 + tid;
-      const int row = chunk >> 3, kc = (chunk & 7) * 8;
-      *reinterpret_cast<uint4 *>(s_b + row * LDS_STRIDE + kc) = rb[c];
-      if (!A_KMAJOR) {
-        *reinterpret_cast<uint4 *>(s_a + row * LDS_STRIDE + kc) = ra[c];
-      } else {
-        const int kr = chunk >> 5, mc = (chunk & 31) * 8;
-        *reinterpret_cast<uint4 *>(s_a + kr * KM_STRIDE + (mc ^ (((kr >> 3) & 1) << 5))) = ra[c];
+        const int kr = piece / (TS / 8);
+        const int turn = TS == 128 ? (kr & 3) << 2 : ((kr >> 1) & 1) << 2;
+        const int m = ((piece % (TS / 8)) ^ turn) * 8;
+        va[c] = m0 + m < g.M;
+        pa[c] = A + (long)kr * lda + m0 + m;
       }
     }
-  };
-
-  load_a(0);
-  load_b(0);
-  for (int k0 = 0; k0 < K; k0 += BK) {
-    __syncthreads();  // the previous step's fragment reads are done
-    store_tiles();
-    __syncthreads();
-    if (k0 + BK < K) {  // prefetch the next k tile while the matrix cores work on this one
-      load_a(k0 + BK);
-      load_b(k0 + BK);
-    }
+    const int steps = (K + BK - 1) / BK;
+    auto issue = [&](int s) {
+      unsigned short *dst = s_dyn + (s % NS) * STAGE + wave * 512;
+      const int k0 = s * BK;
 #pragma unroll
-    for (int kk = 0; kk < BK; kk += 16) {
-      bf16x8 fa[4], fb[2];
-      const int kof = kk + (lane >> 5) * 8;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int mrow = wm * 128 + i * 32 + (lane & 31);
-        if (!A_KMAJOR) {
-          fa[i] = *reinterpret_cast<const bf16x8 *>(s_a + mrow * LDS_STRIDE + kof);
-        } else {
-          // transposing LDS read (ds_read_b64_tr_b16): a group of 16 lanes reads a 4(k) x 16(m)
-          // block, lane j of the group supplying the address of row j/4, columns (j%4)*4..+3, and
-          // receives column j for the four k rows.  Two reads give the 8 consecutive k of lane
-          // (m = lane%32, k-group = lane/32).  Rows kof..kof+7 share bit 3 = lane>>5: one swizzle.
-          const int j16 = lane & 15;
-          const int mcol = (wm * 128 + i * 32 + ((lane >> 4) & 1) * 16) ^ ((lane >> 5) << 5);
-          const unsigned short *src = s_a + (kof + (j16 >> 2)) * KM_STRIDE + mcol + (j16 & 3) * 4;
-          typedef short s16x4 __attribute__((ext_vector_type(4)));
-          typedef short s16x8 __attribute__((ext_vector_type(8)));
-          typedef __attribute__((address_space(3))) s16x4 *lds_s16x4_t;
-          const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)(src));
-          const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)(src + 4 * KM_STRIDE));
-          const s16x8 pk = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-          fa[i] = __builtin_bit_cast(bf16x8, pk);
-        }
+      for (int c = 0; c < NP; ++c) {
+        bool in = va[c];
+        if (A_KMAJOR) in = in && k0 + (c * 256 + tid) / (TS / 8) < K;
+        else in = in && k0 + kc < K;
+        copy_piece_to_lds(in ? pa[c] + (A_KMAJOR ? (long)k0 * lda : (long)k0) : zero, dst + c * 2048);
       }
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
-        fb[j] = *reinterpret_cast<const bf16x8 *>(s_b + (wn * 64 + j * 32 + (lane & 31)) * LDS_STRIDE + kof);
+      for (int c = 0; c < NP; ++c)
+        copy_piece_to_lds(vb[c] && k0 + kc < K ? pb[c] + k0 : zero, dst + PANEL + c * 2048);
+    };
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+    for (int s = 0; s < NS - 1; ++s)
+      if (s < steps) issue(s);
+    for (int s = 0; s < steps; ++s) {
+      // the copies of step s have landed when at most those of the steps behind it are outstanding
+      if (s + NS - 2 < steps) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * 2 * NP) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      lds_barrier();  // everyone's copies, and everyone is past the reads of step s - 1
+      if (s + NS - 1 < steps) issue(s + NS - 1);
+      const unsigned short *sa = s_dyn + (s % NS) * STAGE, *sb = sa + PANEL;
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
-    }
-  }
-
-  if constexpr (EPI == EPI_SCORES_X || EPI == EPI_ACC_X) {
-    __syncthreads();  // every wave is past its fragment reads: s_a can hold the row sums
-    gemm_epilogue_x<EPI>(g, acc, slice, m0, n0, tj, wm, wn, lane, tid, reinterpret_cast<float *>(s_a));
-    return;
-  }
-  // epilogue.  Accumulator element e of lane l in a 32x32 tile:
-  //   row = (e/4)*8 + (l/32)*4 + (e%4), col = l%32
+      for (int kk = 0; kk < BK; kk += 16) {
+        bf16x8 fa[MI], fb[MI];
+        const int C = (kk >> 3) + (lane >> 5);
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int col = n0 + wn * 64 + j * 32 + (lane & 31);
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int row = m0 + wm * 128 + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
-        if (row < g.M && col < (EPI == EPI_SCORES ? g.ldc : g.N)) {
-          float v = acc[i][j][e];
-          if (EPI == EPI_SCORES) {
-            unsigned short *C = static_cast<unsigned short *>(g.C) + (long)slice * g.c_batch;
-            C[(long)row * g.ldc + col] = col < row ? f32_to_bf16_bits(v) : (unsigned short)0;  // tril(-1)
+        for (int i = 0; i < MI; ++i) {
+          if (!A_KMAJOR) {
+            const int R = wm * (TS / 2) + i * 32 + (lane & 31);
+            fa[i] = *reinterpret_cast<const bf16x8 *>(sa + R * BK + ((C ^ ((R >> 1) & 7)) << 3));
           } else {
-            float *C = static_cast<float *>(g.C) + (long)slice * g.c_batch;
-            float *p = C + (long)row * g.ldc + col;
-            *p = g.beta ? *p + v : v;
+            // transposing LDS read (ds_read_b64_tr_b16): a group of 16 lanes reads a 4(k) x 16(m) block, lane j of the
+            // group supplying the address of row j/4, columns (j%4)*4..+3, and receives column j for the four k rows.
+            // Two reads give the 8 consecutive k of lane (m = lane%32, k-group = lane/32).
+            const int j16 = lane & 15, kr = C * 8 + (j16 >> 2);
+            const int m = wm * (TS / 2) + i * 32 + ((lane >> 4) & 1) * 16 + (j16 & 3) * 4;
+            const int turn = TS == 128 ? (kr & 3) << 2 : ((kr >> 1) & 1) << 2;  // the same for kr + 4
+            const unsigned short *src = sa + kr * TS + (((m >> 3) ^ turn) << 3) + (m & 7);
+            typedef short s16x4 __attribute__((ext_vector_type(4)));
+            typedef short s16x8 __attribute__((ext_vector_type(8)));
+            typedef __attribute__((address_space(3))) s16x4 *lds_s16x4_t;
+            const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)(src));
+            const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)(src + 4 * TS));
+            const s16x8 pk = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+            fa[i] = __builtin_bit_cast(bf16x8, pk);
           }
         }
+#pragma unroll
+        for (int j = 0; j < MI; ++j) {
+          const int R = wn * (TS / 2) + j * 32 + (lane & 31);
+          fb[j] = *reinterpret_cast<const bf16x8 *>(sb + R * BK + ((C ^ ((R >> 1) & 7)) << 3));
+        }
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int j = 0; j < MI; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
       }
     }
+    lds_barrier();  // every wave is past its reads: the stages are free
+  };
+
+  const int K1 = g.causal_k ? min(g.K, m0 + TS) : g.K;
+  products(static_cast<const unsigned short *>(g.A) + (long)slice * g.a_batch, g.lda,
+           static_cast<const unsigned short *>(g.B) + (long)(slice / g.b_div) * g.b_batch, g.ldb, K1);
+  const float par = g.mode ? g.head_par[slice % g.h] : 0.0f;
+  auto row_of = [&](int i, int e) { return m0 + wm * (TS / 2) + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3); };
+  if constexpr (!SCORES && !A_KMAJOR) {
+    if (g.mode & GM_DECAY_ROWS) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const float rscale = expf((float)row_of(i, e) * par);
+#pragma unroll
+          for (int j = 0; j < MI; ++j) acc[i][j][e] *= rscale;
+        }
+    }
+    if (g.A2) {  // summed by themselves and then added, as in two launches
+      f32x16 first[MI][MI];
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < MI; ++j)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            first[i][j][e] = acc[i][j][e];
+            acc[i][j][e] = 0.0f;
+          }
+      products(static_cast<const unsigned short *>(g.A2) + (long)slice * g.a2_batch, g.lda2,
+               static_cast<const unsigned short *>(g.B2) + (long)(slice / g.b2_div) * g.b2_batch, g.ldb2,
+               min(g.K2, m0 + TS));
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < MI; ++j)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc[i][j][e] = first[i][j][e] + acc[i][j][e];
+    }
+  }
+
+  if constexpr (SCORES) {
+    unsigned short *C = static_cast<unsigned short *>(g.C) + (long)slice * g.c_batch;
+    const int bs = g.block_size > 0 ? g.block_size : 1;
+    float *s_red = reinterpret_cast<float *>(s_dyn);
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int row = row_of(i, e);
+        const int rblk = (g.mode & GM_ADD_ALIBI) ? row / bs : 0;
+        float rsum[MI];
+#pragma unroll
+        for (int j = 0; j < MI; ++j) {
+          const int col = n0 + wn * (TS / 2) + j * 32 + (lane & 31);
+          float v = col < row ? acc[i][j][e] : 0.0f;  // tril(-1)
+          if ((g.mode & GM_DECAY_SCORES) && col < row) v *= expf((float)(row - col) * par);
+          if ((g.mode & GM_ADD_ALIBI) && col / bs <= rblk) v += par * (float)(col - row);
+          if (col >= g.N) v = 0.0f;  // padding columns of the score matrix
+          const unsigned short bits = f32_to_bf16_bits(v);
+          if (row < g.M && col < g.ldc) C[(long)row * g.ldc + col] = bits;
+          rsum[j] = fabsf(bf16_bits_to_f32(bits));  // what the next product multiplies with
+        }
+        if (g.mode & GM_ROWNORM) {
+#pragma unroll
+          for (int j = 0; j < MI; ++j)  // the 32 columns of a half-wave
+#pragma unroll
+            for (int off = 16; off >= 1; off >>= 1) rsum[j] += __shfl_xor(rsum[j], off);
+          if ((lane & 31) == 0) s_red[wn * TS + row - m0] = MI == 1 ? rsum[0] : rsum[0] + rsum[MI - 1];
+        }
+      }
+    if (g.mode & GM_ROWNORM) {
+      __syncthreads();
+      if (tid < TS && m0 + tid < g.M) {
+        float *part = g.norm_part + ((long)slice * g.norm_groups + n0 / 64) * g.M + m0 + tid;
+        if (TS == 64) {
+          part[0] = s_red[tid] + s_red[TS + tid];
+        } else {
+          part[0] = s_red[tid];
+          if (n0 + 64 < g.N) part[g.M] = s_red[TS + tid];
+        }
+      }
+    }
+  } else {
+    float *C = static_cast<float *>(g.C) + (long)slice * g.c_batch;
+    const float sdecay = (g.mode & GM_DECAY_STATE) ? expf((float)g.K * par) : 1.0f;
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < MI; ++j) {
+        const int col = n0 + wn * (TS / 2) + j * 32 + (lane & 31);
+        if (col >= g.N) continue;
+        float old[16];
+        if (g.beta) {  // all asked for before the first is used
+#pragma unroll
+          for (int e = 0; e < 16; ++e) old[e] = C[(long)min(row_of(i, e), g.M - 1) * g.ldc + col];
+        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int row = row_of(i, e);
+          float v = acc[i][j][e];
+          if (g.mode & GM_DIVNORM) v = v / g.denom[(long)slice * g.M + min(row, g.M - 1)];
+          if (g.beta) v = ((g.mode & GM_DECAY_STATE) ? old[e] * sdecay : old[e]) + v;
+          if (row < g.M) C[(long)row * g.ldc + col] = v;
+        }
+      }
+  }
 }
 
 // ------------------------------------------------------------------------------------
-// Fast variant for full tiles (M, N multiples of 256, K a multiple of 64, both operands
-// k-contiguous): the tiles go from global memory straight into LDS (global_load_lds_dwordx4, no
+// 256x256 tiles, K a multiple of 64 (or both operands zero-padded to it), both operands k-contiguous: the tiles go from global memory straight into LDS (global_load_lds_dwordx4, no
 // VGPR staging, no ds_write), double buffered.  LDS tile layout: blocks of 8 rows x 128 bytes
 // (1 KiB, one wave-wide load each); inside a block the 16-byte slot of (row R, k-chunk c) is
 // (R%8)*8 + (c ^ ((R/2)%8)): the LDS has 64 banks and serves a 16-byte read 16 lanes at a time, and
 // 16 consecutive rows at one k-chunk then cover all 64 banks once (no conflicts, no padding).
-// Same accumulation order as k_gemm, so both give identical results.
+// Same accumulation order as k_gemm_tile, so both give identical results.
 // ------------------------------------------------------------------------------------
 typedef __attribute__((address_space(1))) const void *gptr_t;
 typedef __attribute__((address_space(3))) void *lptr_t;
@@ -529,8 +633,8 @@ __global__ __launch_bounds__(512) void k_gemm_direct(GemmArgs g) {
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
     const int bi = c * 8 + wave;  // 32 blocks of 8 rows per operand, 4 per wave
-    pa[c] = A + (long)(m0 + bi * 8 + lr) * g.lda + lc * 8;
-    pb[c] = Bh + (long)(n0 + bi * 8 + lr) * g.ldb + lc * 8;
+    pa[c] = A + (long)min(m0 + bi * 8 + lr, g.M - 1) * g.lda + lc * 8;  // the sums of repeated rows are not stored
+    pb[c] = Bh + (long)min(n0 + bi * 8 + lr, g.N - 1) * g.ldb + lc * 8;
   }
   // scores: A and B are the same matrix, so a tile on the diagonal needs its rows only once
   const bool same_ab = (EPI == EPI_SCORES || EPI == EPI_SCORES_X) && ti == tj && g.A == g.B && g.b_div == 1 &&
@@ -587,6 +691,7 @@ __global__ __launch_bounds__(512) void k_gemm_direct(GemmArgs g) {
       for (int e = 0; e < 16; ++e) {
         const int row = m0 + wm * 128 + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
         const float v = acc[i][j][e];
+        if (row >= g.M || col >= (EPI == EPI_SCORES ? g.ldc : g.N)) continue;
         if (EPI == EPI_SCORES) {
           unsigned short *C = static_cast<unsigned short *>(g.C) + (long)slice * g.c_batch;
           C[(long)row * g.ldc + col] = col < row ? f32_to_bf16_bits(v) : (unsigned short)0;  // tril(-1)
@@ -680,14 +785,6 @@ __device__ __forceinline__ void direct_mainloop(f32x16 (&acc)[4][2], const unsig
     cur ^= 1;
   }
 #undef BDH_ISSUE
-}
-
-// Workgroup barrier that orders LDS accesses only: global loads and stores issued before it stay in flight
-// (__syncthreads also waits for every outstanding global access).
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 struct ChunkOutArgs {
@@ -1123,7 +1220,7 @@ __device__ __forceinline__ void state_stream_body(const StateUpdArgs &g, unsigne
       const int kof = kk * 16 + (lane >> 5) * 8;
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        // transposing LDS read: see k_gemm
+        // transposing LDS read: see k_gemm_tile
         const int j16 = lane & 15;
         const int mcol = (i * 32 + ((lane >> 4) & 1) * 16) ^ ((lane >> 5) << 5);
         const unsigned short *src = s_a + (kof + (j16 >> 2)) * ST_ASTRIDE + mcol + (j16 & 3) * 4;
@@ -1220,32 +1317,40 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BDH_ST_WAVE
   else state_stream_body<false>(g, s_dyn);
 }
 
-template <bool AK, int EPI>
-hipError_t launch_gemm(hipStream_t st, const GemmArgs &g) {
-  const int groups = (g.n_slices + 7) / 8;
-  const bool full = !AK && g.M % BM == 0 && g.N % BN == 0 && g.K % BK == 0 && g.lda % 8 == 0 && g.ldb % 8 == 0 &&
-                    ((EPI != EPI_SCORES && EPI != EPI_SCORES_X) || g.ldc == g.N);
-  if constexpr (!AK) {
-    if (full) {
-      constexpr int lds = 4 * 256 * 64 * 2;  // two buffers of two 32 KiB tiles
-      // the attribute belongs to the (kernel, device) pair: remember the devices already configured
-      static std::atomic<uint64_t> configured{0};
-      int dev = 0;
-      hipError_t e = hipGetDevice(&dev);
-      if (e != hipSuccess) return e;
-      const uint64_t bit = 1ull << (dev & 63);
-      if (!(configured.load(std::memory_order_acquire) & bit)) {
-        e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_gemm_direct<EPI>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        if (e != hipSuccess) return e;
-        configured.fetch_or(bit, std::memory_order_release);
-      }
-      hipLaunchKernelGGL((k_gemm_direct<EPI>), dim3(8 * groups * g.n_tiles), dim3(512), lds, st, g);
-      return hipSuccess;
-    }
-  }
-  hipLaunchKernelGGL((k_gemm<AK, EPI>), dim3(8 * groups * g.n_tiles), dim3(512), 0, st, g);
+// dynamic LDS beyond 64 KiB must be allowed per (kernel, device)
+template <typename K>
+hipError_t allow_lds(K kernel, int bytes, std::atomic<uint64_t> &configured) {
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  const uint64_t bit = 1ull << (dev & 63);
+  if (configured.load(std::memory_order_acquire) & bit) return hipSuccess;
+  e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  if (e == hipSuccess) configured.fetch_or(bit, std::memory_order_release);
+  return e;
+}
+
+template <int EPI>
+hipError_t launch_gemm_direct(hipStream_t st, const GemmArgs &g) {
+  constexpr int lds = 4 * 256 * 64 * 2;  // two buffers of two 32 KiB tiles
+  static std::atomic<uint64_t> configured{0};
+  const hipError_t e = allow_lds(k_gemm_direct<EPI>, lds, configured);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((k_gemm_direct<EPI>), dim3(8 * ((g.n_slices + 7) / 8) * g.n_tiles), dim3(512), lds, st, g);
   return hipSuccess;
+}
+
+// g.mt, g.nt and g.n_tiles are filled in here.
+template <bool AK, bool SCORES>
+void launch_gemm_tile(hipStream_t st, GemmArgs g, int tile) {
+  g.mt = (g.M + tile - 1) / tile;
+  g.nt = (g.N + tile - 1) / tile;
+  g.n_tiles = g.tri ? g.mt * (g.mt + 1) / 2 : g.mt * g.nt;
+  const unsigned grid = 8u * (unsigned)(((long)g.n_slices * g.n_tiles + 7) / 8);
+  if (tile == 128)
+    hipLaunchKernelGGL((k_gemm_tile<128, AK, SCORES>), dim3(grid), dim3(256), tile_lds_bytes(128), st, g);
+  else
+    hipLaunchKernelGGL((k_gemm_tile<64, AK, SCORES>), dim3(grid), dim3(256), tile_lds_bytes(64), st, g);
 }
 
 // What a pass of the all-scores form does beyond the RoPE recurrence.
@@ -1269,23 +1374,34 @@ static int prefill_pass_scores(bdh_ctx *ctx, int B, int h, int T, int N, int d, 
   const int Nq = pm.rotary == BDH_POPE ? 2 * N : N;
   const bool ext = pm.extended();
   const bool stateless = pm.row_norm;
-  const int Tp = (T + 7) / 8 * 8;  // leading dimension of the score matrix
-  const int mt = (T + BM - 1) / BM;  // row/col tiles of the score matrix
-  const int nt_rho = (Nq + BM - 1) / BM, nt_d = (d + BN - 1) / BN;
+  const bool has_state = !state_is_zero && !stateless;
+  auto tiles = [](long n, int tile) { return (n + tile - 1) / tile; };
+  // The products over the tokens' rows share one tile, since S V reads the scores by whole tiles: the largest with which
+  // the out products still give every CU a workgroup, 256 only where its padding is below an eighth.  Measured, us a call
+  // (ALiBi, N = 4096, d = 256, carried): 32 slices of 2000 tokens 1148 with 256, 1227 with 128; 16 slices of 2048 tokens
+  // (128 output tiles of 256) 762 with 256, 640 with 128; 8 slices of 2048 tokens 446 with 64, 327 with 128.
+  const bool big = d % 256 == 0 && Nq % BK == 0 && S * tiles(T, 256) * (d / 256) >= kFullChip &&
+                   (tiles(T, 256) * 256 - T) * 8 <= T;
+  const int tile_t = big ? 256 : S * tiles(T, 128) * tiles(d, 128) >= kFullChip ? 128 : 64;
+  const int tile_r = S * tiles(Nq, 128) * tiles(d, 128) >= kFullChip ? 128 : 64;
+  const int mt = (int)tiles(T, tile_t), nt_d = (int)tiles(d, tile_t);
   // a time block that straddles two score tiles has additive terms above the tile diagonal: all tiles then
-  const bool full_grid = pm.row_norm && pm.add_alibi && (BM % pm.block_size) != 0;
+  const bool full_grid = pm.row_norm && pm.add_alibi && (tile_t % pm.block_size) != 0;
   const int n_score_tiles = full_grid ? mt * mt : mt * (mt + 1) / 2;
-  const int n_out_tiles = mt * nt_d, n_rho_tiles = nt_rho * nt_d;
+  const int n_out_tiles = mt * nt_d;
+  const int norm_groups = (T + 63) / 64;
+  // leading dimension of the score matrix and of V^T: zeros to a whole piece, to a whole step for the 256-wide tiles
+  const int Tp = big ? (T + 63) / 64 * 64 : (T + 7) / 8 * 8;
   const bool own_q = pm.rotary != BDH_ALIBI;  // ALiBi does not rotate: the products read x itself
 
   // workspace: Q bf16 [S,T,Nq] | scores bf16 [S,T,Tp] | V^T bf16 [B or S,d,Tp] | rho0^T bf16 [S,d,Nq] |
-  //            norm partials f32 [S,mt,T] | denominators f32 [S,T]
+  //            norm partials f32 [S,T/64,T] | denominators f32 [S,T]
   const size_t q_bytes = own_q ? bdh_align_up((size_t)S * T * Nq * 2, 256) : 0;
   const size_t s_bytes = bdh_align_up((size_t)S * T * Tp * 2, 256);
   const size_t vt_bytes = bdh_align_up((size_t)(pm.decay ? S : B) * d * Tp * 2, 256);
   const size_t vs_bytes = pm.decay ? bdh_align_up((size_t)B * d * Tp * 2, 256) : 0;  // undecayed V^T for S V
-  const size_t rt_bytes = (state_is_zero || stateless) ? 0 : bdh_align_up((size_t)S * d * Nq * 2, 256);
-  const size_t np_bytes = pm.row_norm ? bdh_align_up((size_t)S * mt * T * 4, 256) : 0;
+  const size_t rt_bytes = !has_state ? 0 : bdh_align_up((size_t)S * d * Nq * 2, 256);
+  const size_t np_bytes = pm.row_norm ? bdh_align_up((size_t)S * norm_groups * T * 4, 256) : 0;
   const size_t dn_bytes = pm.row_norm ? bdh_align_up((size_t)S * T * 4, 256) : 0;
   int rc = bdh_ws_reserve(ctx, q_bytes + s_bytes + vt_bytes + vs_bytes + rt_bytes + np_bytes + dn_bytes);
   if (rc != BDH_OK) return rc;
@@ -1301,10 +1417,10 @@ static int prefill_pass_scores(bdh_ctx *ctx, int B, int h, int T, int N, int d, 
   float *denom = reinterpret_cast<float *>(take(dn_bytes));
   const unsigned short *Q = own_q ? Qw : reinterpret_cast<const unsigned short *>(x_bf16);
   const long q_slice = own_q ? (long)T * Nq : x_slice;
-  if ((long)S * n_score_tiles > 0x7fffffffL / 16 || (long)S * n_rho_tiles > 0x7fffffffL / 16)
+  if ((long)S * n_score_tiles > 0x7fffffffL / 16 || S * tiles(Nq, tile_r) * tiles(d, tile_r) > 0x7fffffffL / 16)
     return bdh_fail(ctx, BDH_E_SHAPE, "too many tiles (T=%d N=%d)", T, N);
   auto with_mode = [&](GemmArgs &g, int mode) {
-    g.mode = mode; g.h = h; g.block_size = pm.block_size; g.norm_part = norm_part; g.denom = denom;
+    g.mode = mode; g.h = h; g.block_size = pm.block_size; g.norm_part = norm_part; g.norm_groups = norm_groups; g.denom = denom;
     memcpy(g.head_par, pm.head_par, sizeof(g.head_par));
   };
 
@@ -1319,7 +1435,7 @@ static int prefill_pass_scores(bdh_ctx *ctx, int B, int h, int T, int N, int d, 
                        v_bf16, Vt, T, d, Tp, v_batch, h, hp);
     BDH_LAUNCH_CHECK(ctx, "k_transpose_decay_bf16");
   }
-  if (!state_is_zero && !stateless) {
+  if (has_state) {
     hipLaunchKernelGGL(k_transpose_to_bf16<float>, dim3((d + 63) / 64, (Nq + 63) / 64, S), dim3(256), 0, ctx->stream,
                        rho, Rt, Nq, d, Nq, (long)Nq * d);
     BDH_LAUNCH_CHECK(ctx, "k_transpose_to_bf16<rho0>");
@@ -1345,52 +1461,51 @@ static int prefill_pass_scores(bdh_ctx *ctx, int B, int h, int T, int N, int d, 
     g.lda = Nq; g.ldb = Nq; g.ldc = Tp;
     g.M = T; g.N = T; g.K = Nq; g.b_div = 1; g.beta = 0; g.causal_k = 0;
     g.tri = full_grid ? 0 : 1; g.mt = mt; g.nt = mt; g.n_tiles = n_score_tiles; g.n_slices = S;
-    if (ext) {
+    if (ext)
       with_mode(g, (pm.decay ? GM_DECAY_SCORES : 0) | (pm.add_alibi ? GM_ADD_ALIBI : 0) | (pm.row_norm ? GM_ROWNORM : 0));
-      BDH_HIP_CHECK(ctx, (launch_gemm<false, EPI_SCORES_X>(ctx->stream, g)));
-    } else {
-      BDH_HIP_CHECK(ctx, (launch_gemm<false, EPI_SCORES>(ctx->stream, g)));
-    }
-    BDH_LAUNCH_CHECK(ctx, "k_gemm<scores>");
+    if (!big) launch_gemm_tile<false, true>(ctx->stream, g, tile_t);
+    else if (ext) BDH_HIP_CHECK(ctx, launch_gemm_direct<EPI_SCORES_X>(ctx->stream, g));
+    else BDH_HIP_CHECK(ctx, launch_gemm_direct<EPI_SCORES>(ctx->stream, g));
+    BDH_LAUNCH_CHECK(ctx, "scores");
   }
   if (pm.row_norm) {
-    hipLaunchKernelGGL(k_norm_reduce, dim3((T + 255) / 256, S), dim3(256), 0, ctx->stream, norm_part, denom, T, mt,
-                       full_grid ? 0 : 1, 1e-6f);
+    hipLaunchKernelGGL(k_norm_reduce, dim3((T + 255) / 256, S), dim3(256), 0, ctx->stream, norm_part, denom, T,
+                       norm_groups, tile_t, full_grid ? 0 : 1, 1e-6f);
     BDH_LAUNCH_CHECK(ctx, "k_norm_reduce");
   }
-  // 3a. out = Q rho0 (skipped for a fresh state; a decaying state has lost exp(-slope)^t by row t)
-  if (!state_is_zero && !stateless) {
-    GemmArgs g{};
-    g.A = Q; g.B = Rt; g.C = out;
-    g.a_batch = q_slice; g.b_batch = (long)d * Nq; g.c_batch = out_slice;
-    g.lda = Nq; g.ldb = Nq; g.ldc = d;
-    g.M = T; g.N = d; g.K = Nq; g.b_div = 1; g.beta = 0; g.causal_k = 0;
-    g.tri = 0; g.mt = mt; g.nt = nt_d; g.n_tiles = n_out_tiles; g.n_slices = S;
-    if (pm.decay) {
-      with_mode(g, GM_DECAY_ROWS);
-      BDH_HIP_CHECK(ctx, (launch_gemm<false, EPI_ACC_X>(ctx->stream, g)));
-    } else {
-      BDH_HIP_CHECK(ctx, (launch_gemm<false, EPI_ACC>(ctx->stream, g)));
-    }
-    BDH_LAUNCH_CHECK(ctx, "k_gemm<Q rho0>");
+  // 3. out = Q rho0 (skipped for a fresh state; a decaying state has lost exp(-slope)^t by row t) + scores V
+  //    (row-normalised form: divided by the row's sum of |scores| + eps)
+  GemmArgs sv{};
+  sv.A = Sc; sv.B = Vs; sv.C = out;
+  sv.a_batch = (long)T * Tp; sv.b_batch = (long)d * Tp; sv.c_batch = out_slice;
+  sv.lda = Tp; sv.ldb = Tp; sv.ldc = d;
+  sv.M = T; sv.N = d; sv.K = big ? Tp : T; sv.b_div = h; sv.beta = has_state ? 1 : 0;
+  sv.causal_k = full_grid ? 0 : 1;
+  sv.tri = 0; sv.mt = mt; sv.nt = nt_d; sv.n_tiles = n_out_tiles; sv.n_slices = S;
+  GemmArgs qr{};
+  if (has_state) {
+    qr.A = Q; qr.B = Rt; qr.C = out;
+    qr.a_batch = q_slice; qr.b_batch = (long)d * Nq; qr.c_batch = out_slice;
+    qr.lda = Nq; qr.ldb = Nq; qr.ldc = d;
+    qr.M = T; qr.N = d; qr.K = Nq; qr.b_div = 1; qr.beta = 0; qr.causal_k = 0;
+    qr.tri = 0; qr.mt = mt; qr.nt = nt_d; qr.n_tiles = n_out_tiles; qr.n_slices = S;
+    if (pm.decay) with_mode(qr, GM_DECAY_ROWS);
   }
-  // 3b. out (+)= scores V   (row-normalised form: divided by the row's sum of |scores| + eps)
-  {
-    GemmArgs g{};
-    g.A = Sc; g.B = Vs; g.C = out;
-    g.a_batch = (long)T * Tp; g.b_batch = (long)d * Tp; g.c_batch = out_slice;
-    g.lda = Tp; g.ldb = Tp; g.ldc = d;
-    g.M = T; g.N = d; g.K = T; g.b_div = h; g.beta = (state_is_zero || stateless) ? 0 : 1;
-    g.causal_k = full_grid ? 0 : 1;
-    g.tri = 0; g.mt = mt; g.nt = nt_d; g.n_tiles = n_out_tiles; g.n_slices = S;
-    if (pm.row_norm) {
-      with_mode(g, GM_DIVNORM);
-      BDH_HIP_CHECK(ctx, (launch_gemm<false, EPI_ACC_X>(ctx->stream, g)));
-    } else {
-      BDH_HIP_CHECK(ctx, (launch_gemm<false, EPI_ACC>(ctx->stream, g)));
+  if (pm.row_norm) with_mode(sv, GM_DIVNORM);
+  if (!big) {
+    if (has_state) {  // both products in one pass over the output
+      qr.A2 = sv.A; qr.B2 = sv.B;
+      qr.a2_batch = sv.a_batch; qr.b2_batch = sv.b_batch;
+      qr.lda2 = sv.lda; qr.ldb2 = sv.ldb; qr.K2 = T; qr.b2_div = h;
     }
-    BDH_LAUNCH_CHECK(ctx, "k_gemm<S V>");
+    launch_gemm_tile<false, false>(ctx->stream, has_state ? qr : sv, tile_t);
+  } else {
+    if (has_state && pm.decay) BDH_HIP_CHECK(ctx, launch_gemm_direct<EPI_ACC_X>(ctx->stream, qr));
+    else if (has_state) BDH_HIP_CHECK(ctx, launch_gemm_direct<EPI_ACC>(ctx->stream, qr));
+    if (pm.row_norm) BDH_HIP_CHECK(ctx, launch_gemm_direct<EPI_ACC_X>(ctx->stream, sv));
+    else BDH_HIP_CHECK(ctx, launch_gemm_direct<EPI_ACC>(ctx->stream, sv));
   }
+  BDH_LAUNCH_CHECK(ctx, "Q rho0 + S V");
   // 4. rho (+)= Q^T V   (A = Q read k-major; a decaying state: rho = g^T rho + sum_s g^(T-s) q_s (x) v_s)
   if (!stateless) {
     GemmArgs g{};
@@ -1398,29 +1513,12 @@ static int prefill_pass_scores(bdh_ctx *ctx, int B, int h, int T, int N, int d, 
     g.a_batch = q_slice; g.b_batch = (long)d * Tp; g.c_batch = (long)Nq * d;
     g.lda = Nq; g.ldb = Tp; g.ldc = d;
     g.M = Nq; g.N = d; g.K = T; g.b_div = pm.decay ? 1 : h; g.beta = state_is_zero ? 0 : 1; g.causal_k = 0;
-    g.tri = 0; g.mt = nt_rho; g.nt = nt_d; g.n_tiles = n_rho_tiles; g.n_slices = S;
-    if (pm.decay) {
-      with_mode(g, GM_DECAY_STATE);
-      BDH_HIP_CHECK(ctx, (launch_gemm<true, EPI_ACC_X>(ctx->stream, g)));
-    } else {
-      BDH_HIP_CHECK(ctx, (launch_gemm<true, EPI_ACC>(ctx->stream, g)));
-    }
-    BDH_LAUNCH_CHECK(ctx, "k_gemm<Q^T V>");
+    g.tri = 0; g.n_slices = S;
+    if (pm.decay) with_mode(g, GM_DECAY_STATE);
+    launch_gemm_tile<true, false>(ctx->stream, g, tile_r);
+    BDH_LAUNCH_CHECK(ctx, "Q^T V");
   }
   return BDH_OK;
-}
-
-// dynamic LDS beyond 64 KiB must be allowed per (kernel, device)
-template <typename K>
-static hipError_t allow_lds(K kernel, int bytes, std::atomic<uint64_t> &configured) {
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return e;
-  const uint64_t bit = 1ull << (dev & 63);
-  if (configured.load(std::memory_order_acquire) & bit) return hipSuccess;
-  e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  if (e == hipSuccess) configured.fetch_or(bit, std::memory_order_release);
-  return e;
 }
 
 // One pass of the chunk-recurrent form: Tc tokens (a multiple of 256), N a multiple of 256, d = 256.

@@ -431,3 +431,31 @@ def test_fused_state_aligned_takes_the_bf16_form_when_asked(bda, corc, rotary):
     assert not torch.equal(got, exact)  # the option took
     ref_sparse = corc.fused_state_aligned(query, value, freqs, slopes, bs, rot, pairs=pairs)
     assert rel_err(got_sparse.cpu().numpy(), ref_sparse) < 1e-3
+
+@pytest.mark.parametrize("rotary", ["rope", "pope", "alibi"])
+@pytest.mark.parametrize("T,N,d", [(1, 8, 8), (63, 72, 64), (65, 64, 72), (129, 136, 40), (191, 8, 128), (256, 64, 256)])
+def test_every_tile_of_the_prefill_products_gives_the_same_bits(bda, corc, rotary, T, N, d):
+    """At the edges of the 64-, 128- and 256-wide tiles and of a 64-deep step: one sequence takes the smallest tile, 64
+    sequences of 4 heads (256 output tiles) a larger one, and its results are those of the one, bit for bit, because every
+    sum runs over k in order; the one is checked against the token loop of src/model/bdh.rs:288-302."""
+    from burn_dragon_amd.recurrent import prefill_chunked_ex
+
+    B, h = 64, 4
+    rot, nq = ROT[rotary], 2 * N if rotary == "pope" else N
+    x, v, rho0 = _case(T + N + d, 1, h, T, N, d, nq, 0.05)
+    freqs = corc.build_freqs(N, rotary=rot)
+    slopes = corc.default_alibi_slopes(h) if rotary == "alibi" else None
+    q = corc.rotate(x.float().numpy(), freqs, rot, 5)
+    out_ref, rho_ref = corc.recurrent_attention(q, v.float().numpy(), rho0.numpy(),
+                                                decay=None if slopes is None else corc.alibi_decay(slopes))
+    got = []
+    for n in (1, B):
+        rho = rho0.repeat(n, 1, 1, 1).to(DEV)
+        out = prefill_chunked_ex(x.repeat(n, 1, 1, 1).to(DEV), v.repeat(n, 1, 1).to(DEV), rho, torch.from_numpy(freqs).to(DEV), 5,
+                                 rotary=bda.RotaryEmbedding.parse(rotary), alibi_slopes=slopes)
+        torch.cuda.synchronize()
+        got.append((out.cpu(), rho.cpu()))
+    assert rel_err(got[0][0].numpy(), out_ref) < TOL
+    assert rel_err(got[0][1].numpy(), rho_ref) < TOL
+    for one, many in zip(*got):
+        assert torch.equal(many, one.expand_as(many))
