@@ -677,8 +677,13 @@ __global__ __launch_bounds__(256) void k_step_generic(StepPtrs a, RhoT *__restri
 // dense path, D in {256, 512}: PoPE (2N rows) and ALiBi with the eager decay touch every state row on
 // every token, so the step is a streaming read-modify-write of the whole slice.  Same work split and
 // the same order of operations per element as k_step_generic (a workgroup owns 64 rows, wave w takes
-// rows w, w+4, ...), but a lane owns four adjacent columns (one 16-byte access per row) and U rows are
-// in flight per wave.
+// rows w, w+4, ...).  What bounds it is the state's stream: a lane owns 16 bytes of a row (8 bytes of a
+// 512-byte row), the U rows of a group are asked for at once, and the 64 rotated activations are worked
+// out once per workgroup, by a thread each, behind the first group's loads.
+// Against one row's share of four columns per lane, four rows at a time and every lane rotating every
+// row: 48 x 8 x 256 rows of 512 bf16 47 -> 41 us (PoPE, twice the rows, 84 -> 71), 8 x 8 x 4096 rows of
+// 512 bf16 135 -> 92 (4.0 -> 5.8 TB/s with the cache's help), of 512 f32 222 -> 212.  Sixteen rows in
+// flight take so many registers that bf16 rows of 512 lose 4-13 us of that again.
 // ------------------------------------------------------------------------------------
 __device__ __forceinline__ float4 dense_load4(const float *p) { return *reinterpret_cast<const float4 *>(p); }
 __device__ __forceinline__ float4 dense_load4(const unsigned short *p) {
@@ -694,11 +699,53 @@ __device__ __forceinline__ void dense_store4(unsigned short *p, float4 v) {
   *reinterpret_cast<uint2 *>(p) = o;
 }
 
+template <int VW>
+struct DensePiece {  // VW f32 values
+  float v[VW];
+};
+template <typename RhoT, int VW>
+struct DenseRaw;  // the same VW values as they lie in memory
+template <>
+struct DenseRaw<float, 4> {
+  float4 r;
+  __device__ __forceinline__ void load(const float *p) { r = *reinterpret_cast<const float4 *>(p); }
+  __device__ __forceinline__ DensePiece<4> wide() const { return {{r.x, r.y, r.z, r.w}}; }
+  static __device__ __forceinline__ void store(float *p, const DensePiece<4> &e) {
+    *reinterpret_cast<float4 *>(p) = make_float4(e.v[0], e.v[1], e.v[2], e.v[3]);
+  }
+};
+template <int VW>
+struct DenseRaw<unsigned short, VW> {
+  typedef unsigned int words __attribute__((ext_vector_type(VW / 2)));
+  words r;
+  __device__ __forceinline__ void load(const unsigned short *p) { r = *reinterpret_cast<const words *>(p); }
+  __device__ __forceinline__ DensePiece<VW> wide() const {
+    DensePiece<VW> e;
+#pragma unroll
+    for (int i = 0; i < VW / 2; ++i) {
+      e.v[2 * i] = __uint_as_float(r[i] << 16);
+      e.v[2 * i + 1] = __uint_as_float(r[i] & 0xffff0000u);
+    }
+    return e;
+  }
+  static __device__ __forceinline__ void store(unsigned short *p, const DensePiece<VW> &e) {
+    words o;
+#pragma unroll
+    for (int i = 0; i < VW / 2; ++i)
+      o[i] = (unsigned int)f32_to_bf16(e.v[2 * i]) | ((unsigned int)f32_to_bf16(e.v[2 * i + 1]) << 16);
+    *reinterpret_cast<words *>(p) = o;
+  }
+};
+
 template <typename RhoT, int D, int U>
 __global__ __launch_bounds__(256) void k_step_dense(StepPtrs a, RhoT *__restrict__ rho, int Nq, int rotary,
                                                     HeadScalars decay) {
-  constexpr int VPL = D / 256;  // groups of four columns per lane
-  __shared__ float4 s_red[4][D / 4];
+  constexpr int VW = sizeof(RhoT) == 2 && D == 512 ? 8 : 4;  // columns per access
+  constexpr int VPL = D / (64 * VW);                         // accesses per lane and row
+  static_assert(kGenRows % (4 * U) == 0, "whole groups of rows");
+  typedef DenseRaw<RhoT, VW> Raw;
+  __shared__ __attribute__((aligned(16))) float s_red[4][D];
+  __shared__ float s_q[kGenRows];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int slice = blockIdx.x / a.S;
   const int seg = blockIdx.x - slice * a.S;
@@ -706,91 +753,89 @@ __global__ __launch_bounds__(256) void k_step_dense(StepPtrs a, RhoT *__restrict
   const long clock0 = a.pos_dev ? (long)a.pos_dev[b] + a.pos_add : a.pos_int;
   const bool has_decay = rotary == BDH_ALIBI;
   const float dec = has_decay ? decay.v[hh] : 1.0f;
+  const int rows = min(kGenRows, Nq - seg * kGenRows);
 
   // Tokens of this launch, in order.  A workgroup touches only its own state rows, and the barriers of a
   // token order its row stores before the row loads of the next.
   for (int t = 0; t < a.nt; ++t) {
-  const float pos = (float)(clock0 + t);
-  const float *xs = a.x + (long)t * a.x_t_stride + (long)slice * a.x_slice_stride;
-  float4 acc[VPL], vv[VPL];
-  {
-    const float4 *vrow = reinterpret_cast<const float4 *>(a.v + (long)t * a.v_t_stride + (long)b * a.v_batch_stride);
+  RhoT *base = rho + ((long)slice * Nq + (long)seg * kGenRows) * D + lane * VW;
+  Raw rv[U][VPL];
+  auto load_rows = [&](int r0) {  // rows past the end repeat the last one and are not used
 #pragma unroll
-    for (int j = 0; j < VPL; ++j) {
-      acc[j] = make_float4(0.f, 0.f, 0.f, 0.f);
-      vv[j] = vrow[j * 64 + lane];
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int j = 0; j < VPL; ++j) rv[u][j].load(base + (long)min(r0 + 4 * u, rows - 1) * D + j * 64 * VW);
+  };
+  load_rows(wave);
+  DensePiece<VW> acc[VPL], vv[VPL];
+  const float *vrow = a.v + (long)t * a.v_t_stride + (long)b * a.v_batch_stride + lane * VW;
+#pragma unroll
+  for (int j = 0; j < VPL; ++j)
+#pragma unroll
+    for (int c = 0; c < VW; c += 4) {
+      const float4 v4 = *reinterpret_cast<const float4 *>(vrow + j * 64 * VW + c);
+      acc[j].v[c] = acc[j].v[c + 1] = acc[j].v[c + 2] = acc[j].v[c + 3] = 0.0f;
+      vv[j].v[c] = v4.x; vv[j].v[c + 1] = v4.y; vv[j].v[c + 2] = v4.z; vv[j].v[c + 3] = v4.w;
+    }
+  if (tid < rows) {
+    const float *xs = a.x + (long)t * a.x_t_stride + (long)slice * a.x_slice_stride;
+    const int n = seg * kGenRows + tid;
+    if (rotary == BDH_ALIBI) {
+      s_q[tid] = xs[n];  // ALiBi does not rotate (src/model/attention.rs:333-335)
+    } else {             // PoPE (src/model/attention.rs:323-330): rows N..2N-1 are the imaginary parts
+      const int m = n < a.N ? n : n - a.N;
+      const float mag = softplus1(xs[m]);
+      const float ph = rope_phase((float)(clock0 + t), a.freqs[m]);
+      s_q[tid] = n < a.N ? mag * cosf(ph) : mag * sinf(ph);
     }
   }
-  RhoT *base = rho + ((long)slice * Nq + (long)seg * kGenRows) * D;
-  for (int r0 = wave; r0 < kGenRows; r0 += 4 * U) {
-    float4 rv[U][VPL];
-    float qn[U];
-    bool ok[U];
+  // orders s_q only: the rows on their way stay in flight
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+#pragma unroll 1
+  for (int r0 = wave; r0 < rows; r0 += 4 * U) {
+    if (r0 != wave) load_rows(r0);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int r = r0 + 4 * u;
-      ok[u] = r < kGenRows && seg * kGenRows + r < Nq;
-      if (ok[u]) {
-#pragma unroll
-        for (int j = 0; j < VPL; ++j) rv[u][j] = dense_load4(base + (long)r * D + (j * 64 + lane) * 4);
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      qn[u] = 0.0f;
-      if (ok[u]) {
-        const int n = seg * kGenRows + r0 + 4 * u;
-        if (rotary == BDH_ALIBI) {
-          qn[u] = xs[n];  // ALiBi does not rotate (src/model/attention.rs:333-335)
-        } else {          // PoPE (src/model/attention.rs:323-330): rows N..2N-1 are the imaginary parts
-          const int m = n < a.N ? n : n - a.N;
-          const float mag = softplus1(xs[m]);
-          const float ph = rope_phase(pos, a.freqs[m]);
-          qn[u] = n < a.N ? mag * cosf(ph) : mag * sinf(ph);
-        }
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (ok[u]) {
-        const float q = qn[u];
-        RhoT *row = base + (long)(r0 + 4 * u) * D;
+      if (r < rows) {
+        const float q = s_q[r];
 #pragma unroll
         for (int j = 0; j < VPL; ++j) {
-          float4 e = rv[u][j];
-          // readout with the old state (src/model/bdh.rs:293-295), update with the product rounded
-          // before the add (:298), ALiBi decay after the update (:299-301)
-          acc[j].x = __builtin_fmaf(e.x, q, acc[j].x);
-          acc[j].y = __builtin_fmaf(e.y, q, acc[j].y);
-          acc[j].z = __builtin_fmaf(e.z, q, acc[j].z);
-          acc[j].w = __builtin_fmaf(e.w, q, acc[j].w);
-          float t;
-          t = q * vv[j].x; e.x = e.x + t;
-          t = q * vv[j].y; e.y = e.y + t;
-          t = q * vv[j].z; e.z = e.z + t;
-          t = q * vv[j].w; e.w = e.w + t;
-          if (has_decay) {
-            e.x = e.x * dec; e.y = e.y * dec; e.z = e.z * dec; e.w = e.w * dec;
+          DensePiece<VW> e = rv[u][j].wide();
+#pragma unroll
+          for (int c = 0; c < VW; ++c) {
+            // readout with the old state (src/model/bdh.rs:293-295), update with the product rounded
+            // before the add (:298), ALiBi decay after the update (:299-301)
+            acc[j].v[c] = __builtin_fmaf(e.v[c], q, acc[j].v[c]);
+            const float p = q * vv[j].v[c];
+            e.v[c] = e.v[c] + p;
+            if (has_decay) e.v[c] = e.v[c] * dec;
           }
-          dense_store4(row + (j * 64 + lane) * 4, e);
+          Raw::store(base + (long)r * D + j * 64 * VW, e);
         }
       }
     }
   }
 #pragma unroll
-  for (int j = 0; j < VPL; ++j) s_red[wave][j * 64 + lane] = acc[j];
+  for (int j = 0; j < VPL; ++j)
+#pragma unroll
+    for (int c = 0; c < VW; c += 4)
+      *reinterpret_cast<float4 *>(&s_red[wave][(j * 64 + lane) * VW + c]) =
+          make_float4(acc[j].v[c], acc[j].v[c + 1], acc[j].v[c + 2], acc[j].v[c + 3]);
   __syncthreads();
   float *pout = a.partial + (long)t * a.partial_t_stride + (long)blockIdx.x * D;
   for (int c4 = tid; c4 < D / 4; c4 += 256) {
-    float4 s = s_red[0][c4];
+    float4 s = reinterpret_cast<const float4 *>(s_red[0])[c4];
 #pragma unroll
     for (int w = 1; w < 4; ++w) {
-      const float4 p4 = s_red[w][c4];
+      const float4 p4 = reinterpret_cast<const float4 *>(s_red[w])[c4];
       s.x += p4.x; s.y += p4.y; s.z += p4.z; s.w += p4.w;
     }
     reinterpret_cast<float4 *>(pout)[c4] = s;
   }
-  __syncthreads();  // s_red is written again by the next token
+  __syncthreads();  // s_red and s_q are written again by the next token
   }
 }
 
@@ -1172,12 +1217,12 @@ int bdh_launch_state_steps_in(bdh_ctx *ctx, const StateStepParams &p, float *out
       const dim3 grid(slices * S);
       if (p.rho_dtype == BDH_F32) {
         float *rho = static_cast<float *>(p.rho);
-        if (d == 256) hipLaunchKernelGGL((k_step_dense<float, 256, 4>), grid, dim3(256), 0, ctx->stream, a, rho, Nq, p.rotary, decay);
-        else hipLaunchKernelGGL((k_step_dense<float, 512, 4>), grid, dim3(256), 0, ctx->stream, a, rho, Nq, p.rotary, decay);
+        if (d == 256) hipLaunchKernelGGL((k_step_dense<float, 256, 8>), grid, dim3(256), 0, ctx->stream, a, rho, Nq, p.rotary, decay);
+        else hipLaunchKernelGGL((k_step_dense<float, 512, 8>), grid, dim3(256), 0, ctx->stream, a, rho, Nq, p.rotary, decay);
       } else {
         unsigned short *rho = static_cast<unsigned short *>(p.rho);
-        if (d == 256) hipLaunchKernelGGL((k_step_dense<unsigned short, 256, 4>), grid, dim3(256), 0, ctx->stream, a, rho, Nq, p.rotary, decay);
-        else hipLaunchKernelGGL((k_step_dense<unsigned short, 512, 4>), grid, dim3(256), 0, ctx->stream, a, rho, Nq, p.rotary, decay);
+        if (d == 256) hipLaunchKernelGGL((k_step_dense<unsigned short, 256, 8>), grid, dim3(256), 0, ctx->stream, a, rho, Nq, p.rotary, decay);
+        else hipLaunchKernelGGL((k_step_dense<unsigned short, 512, 8>), grid, dim3(256), 0, ctx->stream, a, rho, Nq, p.rotary, decay);
       }
       BDH_LAUNCH_CHECK(ctx, "k_step_dense");
       launch_finalize(ctx->stream, slices, partial, nullptr, S, d, out_t, (long)T * d, out_ln_t, nullptr, (long)T, 2, nt,
