@@ -343,7 +343,7 @@ constexpr int tile_lds_bytes(int TS) { return tile_stages(TS) * 2 * TS * BK * 2;
 // Every sum runs over k in order, so the tile size does not change a bit of the result.
 // What bounds it with few slices is the wait for the next step's operands, hence small tiles, a list dealt evenly to the
 // XCDs and copies several steps ahead.  A call of 12 slices, 777 tokens, N = 4096, d = 256 took 506 us with 256 x 256
-// tiles staged through registers and whole slices dealt to XCDs, 248 us with this; 4 slices of 64 tokens 352 -> 93 us.
+// tiles staged through registers and whole slices dealt to XCDs, 238 us with this; 4 slices of 64 tokens 352 -> 93 us.
 template <int TS, bool A_KMAJOR, bool SCORES>
 __global__ __launch_bounds__(256, 2) void k_gemm_tile(GemmArgs g) {
   extern __shared__ __attribute__((aligned(1024))) unsigned short s_dyn[];
@@ -1376,18 +1376,22 @@ static int prefill_pass_scores(bdh_ctx *ctx, int B, int h, int T, int N, int d, 
   const bool stateless = pm.row_norm;
   const bool has_state = !state_is_zero && !stateless;
   auto tiles = [](long n, int tile) { return (n + tile - 1) / tile; };
-  // The products over the tokens' rows share one tile, since S V reads the scores by whole tiles: the largest with which
-  // the out products still give every CU a workgroup, 256 only where its padding is below an eighth.  Measured, us a call
+  // S V reads the scores by its own whole tiles, which lie within theirs.  The out products take the largest tile that
+  // still gives every CU a workgroup, 256 only where its padding is below an eighth.  Measured, us a call
   // (ALiBi, N = 4096, d = 256, carried): 32 slices of 2000 tokens 1148 with 256, 1227 with 128; 16 slices of 2048 tokens
   // (128 output tiles of 256) 762 with 256, 640 with 128; 8 slices of 2048 tokens 446 with 64, 327 with 128.
   const bool big = d % 256 == 0 && Nq % BK == 0 && S * tiles(T, 256) * (d / 256) >= kFullChip &&
                    (tiles(T, 256) * 256 - T) * 8 <= T;
   const int tile_t = big ? 256 : S * tiles(T, 128) * tiles(d, 128) >= kFullChip ? 128 : 64;
   const int tile_r = S * tiles(Nq, 128) * tiles(d, 128) >= kFullChip ? 128 : 64;
-  const int mt = (int)tiles(T, tile_t), nt_d = (int)tiles(d, tile_t);
+  // The scores, of which there are more tiles, may have the larger one: 12 slices of 777 tokens, whose 168 output tiles
+  // are 64 wide, 248 us a call with scores of 64, 238 with 128 (336 tiles).
+  auto lower = [&](int tile) { return S * tiles(T, tile) * (tiles(T, tile) + 1) / 2; };
+  const int tile_s = !big && lower(128) >= kFullChip ? 128 : tile_t;
+  const int mt = (int)tiles(T, tile_t), nt_d = (int)tiles(d, tile_t), mt_s = (int)tiles(T, tile_s);
   // a time block that straddles two score tiles has additive terms above the tile diagonal: all tiles then
-  const bool full_grid = pm.row_norm && pm.add_alibi && (tile_t % pm.block_size) != 0;
-  const int n_score_tiles = full_grid ? mt * mt : mt * (mt + 1) / 2;
+  const bool full_grid = pm.row_norm && pm.add_alibi && (tile_s % pm.block_size) != 0;
+  const int n_score_tiles = full_grid ? mt_s * mt_s : mt_s * (mt_s + 1) / 2;
   const int n_out_tiles = mt * nt_d;
   const int norm_groups = (T + 63) / 64;
   // leading dimension of the score matrix and of V^T: zeros to a whole piece, to a whole step for the 256-wide tiles
@@ -1460,17 +1464,17 @@ static int prefill_pass_scores(bdh_ctx *ctx, int B, int h, int T, int N, int d, 
     g.a_batch = q_slice; g.b_batch = q_slice; g.c_batch = (long)T * Tp;
     g.lda = Nq; g.ldb = Nq; g.ldc = Tp;
     g.M = T; g.N = T; g.K = Nq; g.b_div = 1; g.beta = 0; g.causal_k = 0;
-    g.tri = full_grid ? 0 : 1; g.mt = mt; g.nt = mt; g.n_tiles = n_score_tiles; g.n_slices = S;
+    g.tri = full_grid ? 0 : 1; g.mt = mt_s; g.nt = mt_s; g.n_tiles = n_score_tiles; g.n_slices = S;
     if (ext)
       with_mode(g, (pm.decay ? GM_DECAY_SCORES : 0) | (pm.add_alibi ? GM_ADD_ALIBI : 0) | (pm.row_norm ? GM_ROWNORM : 0));
-    if (!big) launch_gemm_tile<false, true>(ctx->stream, g, tile_t);
+    if (!big) launch_gemm_tile<false, true>(ctx->stream, g, tile_s);
     else if (ext) BDH_HIP_CHECK(ctx, launch_gemm_direct<EPI_SCORES_X>(ctx->stream, g));
     else BDH_HIP_CHECK(ctx, launch_gemm_direct<EPI_SCORES>(ctx->stream, g));
     BDH_LAUNCH_CHECK(ctx, "scores");
   }
   if (pm.row_norm) {
     hipLaunchKernelGGL(k_norm_reduce, dim3((T + 255) / 256, S), dim3(256), 0, ctx->stream, norm_part, denom, T,
-                       norm_groups, tile_t, full_grid ? 0 : 1, 1e-6f);
+                       norm_groups, tile_s, full_grid ? 0 : 1, 1e-6f);
     BDH_LAUNCH_CHECK(ctx, "k_norm_reduce");
   }
   // 3. out = Q rho0 (skipped for a fresh state; a decaying state has lost exp(-slope)^t by row t) + scores V
