@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "gemm_f32.h"
+#include "lds_copy.h"
 
 namespace {
 
@@ -365,16 +366,6 @@ struct RlTile {
 // instruction (64 cycles for 32 x 32 x 2: 157 TFLOP/s); [1500 x 256] x [256 x 32768] 412 -> 273 us (92 TFLOP/s, of which
 // about 60 us the 200 MB of output), [8192 x 512] x [512 x 131072] 9.8 -> 9.1 ms (120), [128 x 256] x [256 x 1024] 17 -> 10 us
 // against the same products staged through registers, whose loads were waited for where they were issued.
-//
-// Copies 16 bytes per lane from *src to LDS, the 64 lanes' pieces one after the other from dst (uniform over the
-// wavefront).  Written out because the compiler waits for every copy that it knows of before any LDS read that might see
-// it; here the barrier at the end of a stage, behind s_waitcnt, is what orders the two.
-typedef __attribute__((address_space(3))) void *lptr_t;
-__device__ __forceinline__ void copy_to_lds(const float *src, float *dst) {
-  const unsigned int at = __builtin_amdgcn_readfirstlane((unsigned int)(uintptr_t)(lptr_t)dst);
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(at), "v"(src) : "memory");
-}
-
 template <int BM, int BN>
 __global__ __launch_bounds__(256) void k_relu_lowrank_direct(RlArgs g) {
   using Tl = RlTile<BM, BN, 2, 2>;
@@ -404,12 +395,12 @@ __global__ __launch_bounds__(256) void k_relu_lowrank_direct(RlArgs g) {
   auto issue = [&](int buf) {
 #pragma unroll
     for (int c = 0; c < CA; ++c) {
-      copy_to_lds(pa[c], s_tiles + buf * STAGE + (c * 256 + wave * 64) * 4);
+      bdh_copy_to_lds(pa[c], s_tiles + buf * STAGE + (c * 256 + wave * 64) * 4);
       pa[c] += SK;
     }
 #pragma unroll
     for (int c = 0; c < CB; ++c) {
-      copy_to_lds(pb[c], s_tiles + buf * STAGE + BM * SK + (c * 256 + wave * 64) * 4);
+      bdh_copy_to_lds(pb[c], s_tiles + buf * STAGE + BM * SK + (c * 256 + wave * 64) * 4);
       pb[c] += b_step;
     }
   };
@@ -509,12 +500,12 @@ __global__ __launch_bounds__(256) void k_relu_lowrank_rows(RlArgs g) {
     float *s = s_tiles + buf * STAGE;
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
-      copy_to_lds(pb[c], s + BM * SK + (c * 256 + wave * 64) * 4);
+      bdh_copy_to_lds(pb[c], s + BM * SK + (c * 256 + wave * 64) * 4);
       pb[c] += b_step;
     }
 #pragma unroll
     for (int c = 0; c < CA; ++c) {
-      if (BM * 8 >= 256 || wave * 64 < BM * 8) copy_to_lds(pa[c], s + (c * 256 + wave * 64) * 4);
+      if (BM * 8 >= 256 || wave * 64 < BM * 8) bdh_copy_to_lds(pa[c], s + (c * 256 + wave * 64) * 4);
       pa[c] += SK;
     }
   };

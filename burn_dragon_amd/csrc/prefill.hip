@@ -24,6 +24,7 @@
 #include <type_traits>
 
 #include "bdh_internal.h"
+#include "lds_copy.h"
 
 namespace {
 
@@ -315,15 +316,6 @@ __device__ __forceinline__ void gemm_epilogue_x(const GemmArgs &g, f32x16 (&acc)
 // 16 zero bytes: what a lane copies where its piece lies outside the operand (a padding row, or k beyond the end)
 __device__ const uint4 g_zero_piece = {0u, 0u, 0u, 0u};
 
-// Copies 16 bytes per lane from *src to LDS, the 64 lanes' pieces one after the other from dst (uniform over the
-// wavefront).  Written out because the compiler waits for every copy that it knows of before any LDS read that might
-// see it; in k_gemm_tile the counted wait and the barrier at the start of a stage order the two.
-typedef __attribute__((address_space(3))) void *lds_dst_t;
-__device__ __forceinline__ void copy_piece_to_lds(const void *src, unsigned short *dst) {
-  const unsigned int at = __builtin_amdgcn_readfirstlane((unsigned int)(uintptr_t)(lds_dst_t)dst);
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(at), "v"(src) : "memory");
-}
-
 // Workgroup barrier that orders LDS accesses only: global loads and stores issued before it stay in flight
 // (__syncthreads also waits for every outstanding global access).
 __device__ __forceinline__ void lds_barrier() {
@@ -413,11 +405,11 @@ __global__ __launch_bounds__(256, 2) void k_gemm_tile(GemmArgs g) {
         bool in = va[c];
         if (A_KMAJOR) in = in && k0 + (c * 256 + tid) / (TS / 8) < K;
         else in = in && k0 + kc < K;
-        copy_piece_to_lds(in ? pa[c] + (A_KMAJOR ? (long)k0 * lda : (long)k0) : zero, dst + c * 2048);
+        bdh_copy_to_lds(in ? pa[c] + (A_KMAJOR ? (long)k0 * lda : (long)k0) : zero, dst + c * 2048);
       }
 #pragma unroll
       for (int c = 0; c < NP; ++c)
-        copy_piece_to_lds(vb[c] && k0 + kc < K ? pb[c] + k0 : zero, dst + PANEL + c * 2048);
+        bdh_copy_to_lds(vb[c] && k0 + kc < K ? pb[c] + k0 : zero, dst + PANEL + c * 2048);
     };
 #pragma unroll
     for (int s = 0; s < NS - 1; ++s)
