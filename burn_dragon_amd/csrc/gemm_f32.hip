@@ -6,6 +6,8 @@
 // planes, chunks of eight k of one row (16 bytes) being what a lane feeds to one 32 x 32 x 16 instruction.
 #include "gemm_f32.h"
 
+#include "tile_index.h"
+
 #include <algorithm>
 
 namespace {
@@ -65,7 +67,7 @@ struct Tile {
         p[c] = base + (rows_per > 0 ? (long)(r / rows_per) * outer + (long)(r % rows_per) * ld : (long)r * ld);
       } else {
         row[c] = (tid % (R / CH)) * CH + c;
-        p[c] = base + min(r0 + row[c], rows - 1);
+        p[c] = base + bdh_kmajor_row(r0, row[0], c, CH, rows);
       }
     }
     k_off = KM ? (tid / (R / CH)) * 8 : (tid & 3) * 8;
@@ -199,7 +201,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_f32(GemmF32 g) {
   auto run = [&](const float *pa, int lda, int rows_per, long a_outer, const float *pb, int ldb, int K, int lo, int hi) {
     ta.init(pa, lda, m0, g.M, rows_per, a_outer);
     tb.init(pb, ldb, n0, g.N, 0, 0);
-    // 16-byte pieces of a row, or (k-major) 8-byte pieces of a k row that end inside it
+    // 16-byte pieces of a row, or (k-major) pairs of a k row, which end inside it (bdh_kmajor_row)
     const bool a_ok = AK ? ((lda & 1) == 0 && (g.M & 1) == 0 && (reinterpret_cast<uintptr_t>(pa) & 7) == 0)
                          : ((lda & 3) == 0 && (a_outer & 3) == 0 && K <= lda && (reinterpret_cast<uintptr_t>(pa) & 15) == 0);
     const bool b_ok = BK ? ((ldb & 1) == 0 && (g.N & 1) == 0 && (reinterpret_cast<uintptr_t>(pb) & 7) == 0)

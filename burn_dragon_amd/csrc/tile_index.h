@@ -1,0 +1,20 @@
+// Index rules of the tiled products that can be checked without a GPU (no HIP headers).
+#pragma once
+
+#if defined(__HIPCC__)
+#define BDH_HOST_DEVICE __host__ __device__ __forceinline__
+#else
+#define BDH_HOST_DEVICE inline
+#endif
+
+// A thread of a k-major tile owns `ch` adjacent rows that start at row r0 + lead of the operand (lead a multiple of ch, r0 of
+// the tile) and reads them with one access per k where `rows` is a multiple of ch, and one by one elsewhere.  The row that
+// its c-th value comes from: its own, or, past the end, one of the last whole group -- every access of ch values then starts
+// at a multiple of ch and ends inside the operand.  What a repeated row adds up to is not stored.
+BDH_HOST_DEVICE int bdh_kmajor_row(int r0, int lead, int c, int ch, int rows) {
+  if (rows % ch == 0) {
+    const int first = r0 + lead < rows - ch ? r0 + lead : rows - ch;
+    return first + c;
+  }
+  return r0 + lead + c < rows - 1 ? r0 + lead + c : rows - 1;
+}

@@ -1,0 +1,29 @@
+// The rows that the threads of a k-major tile read (bdh_kmajor_row), for every width up to 640 and every tile: inside the
+// operand, aligned where a group is read at once, and the thread's own row wherever it has one.
+#include <cstdio>
+
+#include "../burn_dragon_amd/csrc/tile_index.h"
+
+int main() {
+  const int tiles[3] = {128, 64, 32}, threads = 256;
+  long checked = 0;
+  for (int rows = 1; rows <= 640; ++rows)
+    for (int R : tiles) {
+      const int ch = R * 4 / threads > 0 ? R * 4 / threads : 1;
+      for (int r0 = 0; r0 < rows; r0 += R)
+        for (int lead = 0; lead < R; lead += ch) {
+          for (int c = 0; c < ch; ++c) {
+            const int at = bdh_kmajor_row(r0, lead, c, ch, rows);
+            if (at < 0 || at >= rows) return std::printf("rows %d tile %d: row %d\n", rows, R, at), 1;
+            if (r0 + lead + c < rows && at != r0 + lead + c) return std::printf("rows %d tile %d: %d for %d\n", rows, R, at, r0 + lead + c), 1;
+            ++checked;
+          }
+          if (rows % ch == 0) {  // read at once, from the first of the group
+            const int first = bdh_kmajor_row(r0, lead, 0, ch, rows);
+            if (first % ch != 0 || first + ch > rows) return std::printf("rows %d tile %d: group at %d\n", rows, R, first), 1;
+          }
+        }
+    }
+  std::printf("ok %ld\n", checked);
+  return 0;
+}
