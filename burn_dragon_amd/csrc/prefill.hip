@@ -224,7 +224,7 @@ struct GemmArgs {
   int M, N, K;
   int b_div;           // B slice index = slice / b_div (V is shared by the h heads of a batch entry)
   int beta;            // EPI_ACC: add to the existing C
-  int causal_k;        // limit K of row tile i to min(K, (i+1)*BM)   (S V product)
+  int causal_k;        // S V product: K of a row tile ends with the tile, rounded up to a multiple of this (0: no limit)
   int tri;             // 1: tiles enumerate the lower triangle (row tile >= col tile) of an mt x mt grid
   int mt, nt;          // tile grid (rows, cols); rows are visited from the last (largest causal K) down
   int n_tiles, n_slices;
@@ -462,7 +462,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_tile(GemmArgs g) {
     lds_barrier();  // every wave is past its reads: the stages are free
   };
 
-  const int K1 = g.causal_k ? min(g.K, m0 + TS) : g.K;
+  const int K1 = g.causal_k ? min(g.K, (m0 + TS + g.causal_k - 1) / g.causal_k * g.causal_k) : g.K;
   products(static_cast<const unsigned short *>(g.A) + (long)slice * g.a_batch, g.lda,
            static_cast<const unsigned short *>(g.B) + (long)(slice / g.b_div) * g.b_batch, g.ldb, K1);
   const float par = g.mode ? g.head_par[slice % g.h] : 0.0f;
@@ -1381,7 +1381,8 @@ static int prefill_pass_scores(bdh_ctx *ctx, int B, int h, int T, int N, int d, 
   auto lower = [&](int tile) { return S * tiles(T, tile) * (tiles(T, tile) + 1) / 2; };
   const int tile_s = !big && lower(128) >= kFullChip ? 128 : tile_t;
   const int mt = (int)tiles(T, tile_t), nt_d = (int)tiles(d, tile_t), mt_s = (int)tiles(T, tile_s);
-  // a time block that straddles two score tiles has additive terms above the tile diagonal: all tiles then
+  // a time block that straddles two score tiles has additive terms above the tile diagonal: all tiles then, and no causal
+  // limit on the K of S V
   const bool full_grid = pm.row_norm && pm.add_alibi && (tile_s % pm.block_size) != 0;
   const int n_score_tiles = full_grid ? mt_s * mt_s : mt_s * (mt_s + 1) / 2;
   const int n_out_tiles = mt * nt_d;
@@ -1476,7 +1477,8 @@ static int prefill_pass_scores(bdh_ctx *ctx, int B, int h, int T, int N, int d, 
   sv.a_batch = (long)T * Tp; sv.b_batch = (long)d * Tp; sv.c_batch = out_slice;
   sv.lda = Tp; sv.ldb = Tp; sv.ldc = d;
   sv.M = T; sv.N = d; sv.K = big ? Tp : T; sv.b_div = h; sv.beta = has_state ? 1 : 0;
-  sv.causal_k = full_grid ? 0 : 1;
+  // (an output tile narrower than a time block needs the scores up to the block's end, which is inside its score tile)
+  sv.causal_k = full_grid ? 0 : pm.row_norm && pm.add_alibi ? tile_s : tile_t;
   sv.tri = 0; sv.mt = mt; sv.nt = nt_d; sv.n_tiles = n_out_tiles; sv.n_slices = S;
   GemmArgs qr{};
   if (has_state) {

@@ -459,3 +459,21 @@ def test_every_tile_of_the_prefill_products_gives_the_same_bits(bda, corc, rotar
     assert rel_err(got[0][1].numpy(), rho_ref) < TOL
     for one, many in zip(*got):
         assert torch.equal(many, one.expand_as(many))
+
+
+@pytest.mark.parametrize("h,T,d,bs", [(4, 1408, 64, 128), (8, 1000, 64, 128), (2, 300, 64, 96), (4, 1408, 64, 64)])
+def test_row_normalised_alibi_with_time_blocks_wider_than_the_output_tiles(bda, corc, h, T, d, bs):
+    """A 128-token time block has additive terms above the diagonal of a 64-wide output tile, also where the scores take
+    128-wide tiles (few output tiles, many score tiles)."""
+    from burn_dragon_amd.recurrent import prefill_chunked_ex
+
+    N = 16
+    rng = np.random.default_rng(T + bs)
+    x = torch.from_numpy(np.maximum(rng.standard_normal((1, h, T, N)) - 0.5, 0).astype(np.float32)).to(torch.bfloat16)
+    v = torch.from_numpy(rng.standard_normal((1, T, d)).astype(np.float32)).to(torch.bfloat16)
+    slopes = corc.default_alibi_slopes(h)
+    freqs = corc.build_freqs(N, rotary=orc.ALIBI)
+    ref = corc.fused_state_aligned(x.float().numpy(), v.float().numpy(), freqs, slopes, bs, orc.ALIBI)
+    out = prefill_chunked_ex(x.to(DEV), v.to(DEV), None, torch.from_numpy(freqs).to(DEV), 0, rotary=bda.RotaryEmbedding.ALIBI,
+                             alibi_slopes=slopes, row_normalize=True, block_size=bs)
+    assert rel_err(out.cpu().numpy(), ref) < TOL
