@@ -210,7 +210,8 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_f32(GemmF32 g) {
       if (AK && EPI == GEMM_STORE && g.decay_state) {  // token k of K is decayed K - k times by the end
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-          const float f = expf((float)(K - (kb * FK + ta.k_off + q)) * ld);
+          // (beyond K, where the operand is zero: 1, for the power of a steep decay would be infinite there)
+          const float f = expf((float)max(K - (kb * FK + ta.k_off + q), 0) * ld);
 #pragma unroll
           for (int c = 0; c < Tile<BM, NT, AK>::CH; ++c) ta.v[c][q] *= f;
         }

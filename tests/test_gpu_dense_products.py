@@ -101,3 +101,28 @@ def test_many_rows_through_the_second_stage_and_the_head(bda, T, V, d):
         assert rel_err(logits[b].cpu().numpy(), one[0].cpu().numpy()) < 1e-5
         assert rel_err(fast[b].cpu().numpy(), model.forward_fast(tokens[b:b + 1])[0].cpu().numpy()) < 1e-5
         assert int(nxt[b]) == int(n1[0]) == int(logits[b, -1].argmax())
+
+
+@pytest.mark.parametrize("T", [9, 31, 33, 65, 520])
+@pytest.mark.parametrize("slope", [4.0, 80.0])
+def test_steep_decay_over_a_ragged_prompt(bda, corc, T, slope):
+    """A prompt that ends inside a 32-deep stage, through the dense form, with a state that loses up to e^-80 per token."""
+    from burn_dragon_amd.recurrent import recurrent_attention
+
+    B, h, N, d = 2, 2, 96, 128
+    rng = np.random.default_rng(T)
+    x = np.maximum(rng.standard_normal((B, h, T, N)) - 0.3, 0).astype(np.float32)
+    v = rng.standard_normal((B, T, d)).astype(np.float32)
+    rho = (0.1 * rng.standard_normal((B, h, N, d))).astype(np.float32)
+    slopes = np.array([slope, 0.5], np.float32)
+    out, state = np.zeros((B, h, T, d)), rho.astype(np.float64)
+    decay = np.exp(-slopes).astype(np.float64)
+    for t in range(T):
+        out[:, :, t] = np.einsum("bhn,bhnd->bhd", x[:, :, t].astype(np.float64), state)
+        state = (state + x[:, :, t, :, None].astype(np.float64) * v[:, None, t, None, :]) * decay[None, :, None, None]
+    rho_t = torch.from_numpy(rho).to(DEV)
+    got = recurrent_attention(torch.from_numpy(x).to(DEV), torch.from_numpy(v).to(DEV), rho_t, torch.zeros(N, device=DEV), 0,
+                              bda.RotaryEmbedding.ALIBI, slopes)
+    for hh in range(h):
+        assert rel_err(got.cpu().numpy()[:, hh], out[:, hh]) < 2e-5
+        assert rel_err(rho_t.cpu().numpy()[:, hh], state[:, hh]) < 2e-5 or np.abs(state[:, hh]).max() < 1e-30
