@@ -767,8 +767,8 @@ int bdh_launch_state_chunks_f32(bdh_ctx *ctx, const StateStepParams &p, float *o
   const bool alibi = p.rotary == BDH_ALIBI;
   if (p.stamps && !alibi) return bdh_fail(ctx, BDH_E_INVAL, "decay stamps only apply to ALiBi");
   float log_decay[64] = {0};
-  if (alibi)  // log of the ROUNDED per-token factor, as in the lazily decayed step (src/model/attention.rs:181-186)
-    for (int i = 0; i < h; ++i) log_decay[i] = (float)log((double)expf(-p.slopes_host[i]));
+  if (alibi)
+    for (int i = 0; i < h; ++i) log_decay[i] = bdh_log_decay(p.slopes_host[i]);
   if (p.stamps) {  // a lazily decayed state: apply what is pending, the products below decay every row themselves
     int rc0 = bdh_launch_alibi_materialize(ctx, B, h, N, d, p.slopes_host, p.position, p.positions_dev, p.rho,
                                            p.rho_dtype, p.stamps);

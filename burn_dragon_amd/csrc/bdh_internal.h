@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
@@ -97,6 +98,13 @@ int bdh_stage_reserve(bdh_ctx *ctx, size_t bytes);
   } while (0)
 
 static inline size_t bdh_align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
+
+// The log of the ROUNDED per-token decay factor expf(-slope) (src/model/attention.rs:181-186), for the forms that need powers
+// of it.  Finite: a factor that rounds to zero (slopes above 103) still has the zeroth power 1, and 0 * -inf would be NaN.
+static inline float bdh_log_decay(float slope) {
+  const double l = log((double)expf(-slope));
+  return l < -1e4 ? -1e4f : (float)l;
+}
 static inline bool bdh_aligned(const void *p, size_t a) {
   return (reinterpret_cast<uintptr_t>(p) % a) == 0;
 }

@@ -1666,7 +1666,7 @@ int bdh_launch_state_prefill_bf16(bdh_ctx *ctx, const StateStepParams &p, float 
   if (p.rotary == BDH_ALIBI) {
     if (h > 64) return bdh_fail(ctx, BDH_E_SHAPE, "at most 64 heads with ALiBi slopes (h=%d)", h);
     pm.decay = true;
-    for (int i = 0; i < h; ++i) pm.head_par[i] = (float)log((double)expf(-p.slopes_host[i]));
+    for (int i = 0; i < h; ++i) pm.head_par[i] = bdh_log_decay(p.slopes_host[i]);
   }
   if (p.stamps) {  // a lazily decayed state: apply what is pending, the products decay every row themselves
     const int rc0 = bdh_launch_alibi_materialize(ctx, B, h, N, d, p.slopes_host, p.position, nullptr, p.rho, p.rho_dtype,
@@ -1762,7 +1762,7 @@ extern "C" int bdh_prefill_chunked_ex(bdh_ctx *ctx, int B, int h, int T, int N, 
     else bdh_default_alibi_slopes(h, slopes);
     pm.decay = true;
     // log of the ROUNDED per-token factor (src/model/attention.rs:181-186), as the lazily decayed step uses it
-    for (int i = 0; i < h; ++i) pm.head_par[i] = (float)log((double)expf(-slopes[i]));
+    for (int i = 0; i < h; ++i) pm.head_par[i] = bdh_log_decay(slopes[i]);
   }
   return prefill_chunked_impl(ctx, B, h, T, N, d, x_bf16, v_bf16, freqs, position, chunk, flags, rho, out, pm);
 }

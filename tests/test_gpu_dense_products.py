@@ -104,9 +104,10 @@ def test_many_rows_through_the_second_stage_and_the_head(bda, T, V, d):
 
 
 @pytest.mark.parametrize("T", [9, 31, 33, 65, 520])
-@pytest.mark.parametrize("slope", [4.0, 80.0])
+@pytest.mark.parametrize("slope", [4.0, 80.0, 120.0])
 def test_steep_decay_over_a_ragged_prompt(bda, corc, T, slope):
-    """A prompt that ends inside a 32-deep stage, through the dense form, with a state that loses up to e^-80 per token."""
+    """A prompt that ends inside a 32-deep stage, through the dense form, with a state that loses up to e^-80 per
+    token or, at a slope of 120 (whose factor rounds to zero), all of it."""
     from burn_dragon_amd.recurrent import recurrent_attention
 
     B, h, N, d = 2, 2, 96, 128
