@@ -1086,14 +1086,16 @@ int bdh_launch_relu_lowrank(bdh_ctx *ctx, const ReluLowrankParams &p) {
     return BDH_OK;
   }
   // Two rows and more: the f32 matrix cores, same values, the weights streamed once per row tile (options: fewer than 64
-  // rows from mfma_rows on, more from gemm_rows on; 0 = never; the sign no longer matters).  Fewer than 64 rows want the
-  // 16-byte pieces of the copying kernels; what is left, and a single row of a larger matrix, runs a thread per column.
+  // rows from mfma_rows on, more from gemm_rows on; 0 = never).  Fewer than 64 rows want the 16-byte pieces of the copying
+  // kernels; what is left, and a single row of a larger matrix, runs a thread per column with its input rows in LDS.  Eight
+  // rows and more that do not fit there (d above 2048) take the matrix cores whatever the options say.
   const int mc_rows = std::abs(M < 64 ? ctx->opt_lowrank_mfma_rows : ctx->opt_lowrank_gemm_rows);
   const bool pieces = p.d % 32 == 0 && p.N % 4 == 0 && bdh_aligned(p.in, 16) && bdh_aligned(p.weight, 16);
-  if (p.d > 0 && p.N > 0 && M > 1 && mc_rows > 0 && M >= mc_rows && (M >= 64 || pieces))
-    return bdh_launch_relu_lowrank_gemm(ctx, p, mask_dev);
   const int RT = M >= 8 ? 8 : (M >= 4 ? 4 : (M >= 2 ? 2 : 1));
   const size_t lds = sizeof(float) * (size_t)RT * (p.d > 0 ? p.d : 1);
+  if (p.d > 0 && p.N > 0 && M > 1 &&
+      ((mc_rows > 0 && M >= mc_rows && (M >= 64 || pieces)) || (RT == 8 && lds > 64 * 1024)))
+    return bdh_launch_relu_lowrank_gemm(ctx, p, mask_dev);
   if (lds > 64 * 1024) return bdh_fail(ctx, BDH_E_SHAPE, "d=%d too large for the projection tile", p.d);
   const long row_tiles = (M + RT - 1) / RT;
   if (row_tiles > 65535 || p.h > 65535) return bdh_fail(ctx, BDH_E_SHAPE, "grid too large (row tiles %ld)", row_tiles);

@@ -127,3 +127,19 @@ def test_steep_decay_over_a_ragged_prompt(bda, corc, T, slope):
     for hh in range(h):
         assert rel_err(got.cpu().numpy()[:, hh], out[:, hh]) < 2e-5
         assert rel_err(rho_t.cpu().numpy()[:, hh], state[:, hh]) < 2e-5 or np.abs(state[:, hh]).max() < 1e-30
+
+
+@pytest.mark.parametrize("M,d,N", [(8, 2050, 10), (63, 2052, 6), (9, 4100, 4), (8, 16388, 3), (40, 2080, 7)])
+def test_relu_lowrank_wide_rows(bda, corc, M, d, N):
+    """Eight rows and more of a width that neither comes in 16-byte pieces nor fits into LDS: the bits of the k-sequential
+    chain."""
+    from burn_dragon_amd.kernel import relu_lowrank
+
+    h = 2
+    rng = np.random.default_rng(M + N)
+    inp = rng.standard_normal((M, h, 1, d)).astype(np.float32)
+    weight = rng.standard_normal((h, d, N)).astype(np.float32)
+    ref = corc.relu_lowrank(inp, weight)
+    got = relu_lowrank.fused_forward(torch.from_numpy(inp).to(DEV), torch.from_numpy(weight).to(DEV), None, 0.0,
+                                     bda.BlockPattern1d.dense(64))
+    assert np.array_equal(got.cpu().numpy(), ref)
