@@ -1026,6 +1026,52 @@ int bdh_step_scratch_resolve(bdh_ctx *ctx) {
   return BDH_OK;
 }
 
+// From how many tokens on a call runs as dense products unless told otherwise.  The token loop reads and writes each token's
+// rows, the dense form the whole state about three times whatever the number of tokens, and a bf16 state as f32 besides.  The
+// host does not know how many neurons fire; the line lies where the two take equally long at 5 % of them (a trained model),
+// so that such a prompt is never slower than its loop; with more of them firing the dense form wins earlier and the call gives
+// that up, with 1 % the line would lie up to twice as far out.  us per call and layer, loop | dense (d = 256 unless given):
+//                                            5 %                                       50 %
+//   f32 RoPE    N=2048  B*h=4      8 MiB     T=24 41|57     T=48 74|59                 T=24 66|57      T=48 125|59
+//               N=8192  B*h=12    96 MiB     T=32 161|186   T=48 228|186               T=32 609|186    T=48 907|186
+//               N=16384 B*h=16 d=512 512 MiB T=32 510|635   T=48 746|657               T=32 4494|639   T=48 6780|671
+//   lazy ALiBi  N=8192  B*h=12    96 MiB     T=16 127|187   T=24 203|189               T=8 240|180
+//   f32         N=16384 B*h=16 d=512 512 MiB T=32 622|731   T=48 916|766               T=8 955|728
+//   bf16 RoPE   N=2048  B*h=16    32 MiB     T=16 94|111    T=24 133|112               T=16 125|110
+//               N=2048  B*h=64   128 MiB     T=32 233|299   T=48 368|327               T=16 305|297
+//               N=16384 B*h=16 d=512 512 MiB T=64 1091|1249 T=96 1621|1347             T=16 1121|1213  T=24 1684|1219
+//   bf16 lazy   N=8192  B*h=12    96 MiB     T=24 217|250   T=32 279|254               T=8 293|243
+//   bf16 eager  N=2048  B*h=16    32 MiB     T=16 88|104    T=24 129|107               (every row, whatever fires)
+// MiB is the state's size in f32.  The estimates below are within about a quarter of what was measured.
+static int dense_form_from(const StateStepParams &p, bool fast) {
+  const int Nq = p.rotary == BDH_POPE ? 2 * p.N : p.N;
+  const double mib = sizeof(float) * (double)p.B * p.h * Nq * p.d / (1 << 20);
+  const bool f32 = p.rho_dtype == BDH_F32, cached = mib <= 64.0;
+  const bool lazy = p.rotary == BDH_ALIBI && p.stamps;
+  // An f32 RoPE state of up to 512 KiB at d in {256, 512} is always walked: there a prompt leaves the bits that single-token
+  // calls leave (181 against 35 us for 128 tokens).
+  if (f32 && fast && mib <= 0.5) return INT32_MAX;
+  // A loop that streams every row, or one that is a chain of latencies: 8 tokens in the loop are as long as the products
+  // (N=256, B*h=4, us at T = 8: lazy ALiBi 53|34, eager 28|29, PoPE 31|33; N=8192, B*h=12: eager 223|162, PoPE 459|303).
+  if (f32 && p.rotary == BDH_ALIBI && !p.stamps) return 8;
+  if (f32 && p.rotary == BDH_POPE) return 8;
+  if (f32 && !fast && cached) return 8;
+  // us: the products, and one token of the loop at 5 %
+  double dense_mib, token;
+  if (p.rotary == BDH_ROPE) {
+    dense_mib = f32 ? 1.15 : 2.25;
+    token = !f32 ? 5.5 + 0.023 * mib : !fast ? 2.4 + 0.075 * mib : cached ? 1.4 + 0.011 * mib : 1.4 + 0.03 * mib;
+  } else if (lazy) {
+    dense_mib = f32 ? 1.35 : 2.35;
+    token = f32 ? 6.5 + 0.026 * mib : 2.8 + 0.065 * mib;
+  } else {  // a bf16 state of which every row is streamed
+    dense_mib = 2.35;
+    token = std::max(4.2 + 0.03 * mib, 0.14 * mib);
+  }
+  const double dense = 30.0 + dense_mib * mib + 0.005 * Nq;
+  return (int)std::min(128.0, std::max(16.0, std::ceil(dense / token)));
+}
+
 void *bdh_step_scratch_ptr(const bdh_ctx *ctx) {
   if (ctx->device < 0 || ctx->device >= kStepScratchDevices) return nullptr;
   std::lock_guard<std::mutex> lock(g_step_scratch_mutex);
@@ -1088,24 +1134,7 @@ int bdh_launch_state_steps_in(bdh_ctx *ctx, const StateStepParams &p, float *out
   // (not when even a 128-token chunk of rotated activations would pass 16 GiB of workspace)
   const bool chunk_fits = sizeof(float) * (size_t)slices * Nq * 128 <= (size_t(16) << 30) &&
                           (p.rho_dtype == BDH_F32 || sizeof(float) * (size_t)slices * Nq * d <= (size_t(64) << 30));
-  // The token loop reads and writes each token's rows, the dense form the whole state twice whatever the number of tokens
-  // (Q rho, then rho += Q^T V) in about six launches.  By default from 16 tokens on; us per call of a model, loop | dense,
-  // at half the neurons active:
-  //   L=6 d=256 N=256  B=1 f32 RoPE    T=16 402|358    T=32 700|426     lazy ALiBi  T=8 683|368   T=16 1214|378
-  //   L=6 d=256 N=2048 B=4 bf16 RoPE   T=16 1189|1010  T=32 2052|1024   eager ALiBi T=8 748|962   T=16 1216|974
-  //   L=8 d=512 N=2560 B=4 f32 RoPE    T=8 3965|3267   T=16 5696|2929   lazy ALiBi  T=8 4921|3392
-  //   L=12 d=512 N=10240 B=1 f32 RoPE  T=16 9893|6239; L=6 d=256 N=8192 B=3 T=500 62 900|9 760
-  // From 8 on where the loop is a chain of latencies or streams every row anyway: a lazily decayed f32 state, an f32 state
-  // decayed eagerly, PoPE, and a state of up to 64 MiB.  From 24 on for an f32 RoPE state of up to 64 MiB: its loop walks
-  // many tokens per launch and the rows stay in the caches (L=6 d=256 N=2048 B=1: T=16 533|613, T=32 789|624).
-  const size_t state_bytes = sizeof(float) * (size_t)slices * Nq * d;
-  const bool cached_loop = fast && p.rho_dtype == BDH_F32 && state_bytes <= (size_t(64) << 20);
-  const bool slow_loop = p.rho_dtype == BDH_F32 && p.rotary != BDH_ROPE;
-  const bool small_state = p.rho_dtype == BDH_F32 && state_bytes <= (size_t(64) << 20);
-  // And not at all for an f32 RoPE state of up to 512 KiB: there a prompt leaves the bits that single-token calls leave
-  // (d=256 N=128 B*h=4, T=128: 181 | 35 us), which callers of such states check.
-  const bool keep_bits = fast && p.rho_dtype == BDH_F32 && state_bytes <= (size_t(512) << 10);
-  const bool dense_auto = !keep_bits && T >= (cached_loop ? 24 : (slow_loop || small_state) ? 8 : 16);
+  const bool dense_auto = T >= dense_form_from(p, fast);
   if (!fixed && !p.bitmask && !p.rows_touched && chunk_fits &&
       (ctx->opt_step_dense >= 0 ? ctx->opt_step_dense == 1 : dense_auto))
     return bdh_launch_state_chunks_f32(ctx, p, out_ln);

@@ -74,11 +74,14 @@ const char *bdh_last_error(const bdh_ctx *ctx);
 /* Launch-shape knobs for tests and tuning; no counterpart in the reference.
  *   "state_step.split": -1 (default) pick by grid size, 0 = 256 lane pairs per workgroup,
  *                       1 = 64 lane pairs per workgroup of 8 waves (small batches).
- *   "state_step.dense_chunks": -1 (default) a call of 16 or more tokens without bitmask / row-count outputs runs as
- *                       dense products on the matrix cores (from 8 tokens on for an f32 state that is lazily decayed,
- *                       that every token streams in full -- PoPE, eager ALiBi -- or that is at most 64 MiB; from 24
- *                       on for an f32 RoPE state of at most 64 MiB; never for one of at most 512 KiB, where a prompt
- *                       leaves the bits of single-token calls),
+ *   "state_step.dense_chunks": -1 (default) a call of many tokens without bitmask / row-count outputs runs as dense
+ *                       products on the matrix cores: from 8 tokens on for an f32 state that every token streams in full
+ *                       (PoPE, eager ALiBi), or of at most 64 MiB with lazily decayed rows or a d other than 256 and
+ *                       512; else from where the products are as fast as the token loop with 5 % of the neurons active
+ *                       (between 16 and 128 tokens, by state size, type and rotary).  Never for an f32 RoPE state of
+ *                       at most 512 KiB (B*h*N*d floats, d 256 or 512): there a call of any number of tokens leaves the
+ *                       bits that single-token calls leave.  Any other call of many tokens agrees with them to f32
+ *                       rounding (a bf16 state is rounded once at its end instead of after every token),
  *                       0 = always token by token, 1 = dense products for any T.
  *   "state_step.prompt_bf16": 0 (default) never; T0 > 0: a call of T0 or more tokens on an f32 state, with the
  *                       position given by the host and no bitmask / row-count outputs, runs as
@@ -173,8 +176,9 @@ int bdh_rotate(bdh_ctx *ctx, int B, int h, int T, int N, int rotary, const float
  *                        that token (RoPE: both rows of every lane pair with a non-zero
  *                        element; ALiBi/PoPE: Nq)
  *
- * RoPE requires even N (src/model/attention.rs:310).  T = 1 is the decode step.  A call of 16 or more
- * tokens (see option "state_step.dense_chunks") that asks for neither bitmask nor row counts computes the same sums as dense
+ * RoPE requires even N (src/model/attention.rs:310).  T = 1 is the decode step.  A call of many tokens (8 to
+ * 128 and more, see option "state_step.dense_chunks") that asks for neither bitmask nor row counts computes the same
+ * sums as dense
  * products (out = tril(-1)(Q Q^T) V + Q rho, rho += Q^T V, chunks of up to 512 tokens; for ALiBi with
  * the decay powers decay^(t-s), decay^t and decay^(T-s) applied to the three terms) on the matrix
  * cores (a bf16 state is widened to f32 for the call and rounded once at its end).  Large products
