@@ -898,22 +898,18 @@ int bdh_launch_state_chunks_f32(bdh_ctx *ctx, const StateStepParams &p, float *o
   return BDH_OK;
 }
 
-// The encoder E over many rows (src/model/bdh.rs:383,436-438): mixed [B*T, h*N] . decoder [h*N, d] as one product per head
-// (T = 1: mixed is contiguous per sequence, one product), K cut into as many parts as the chip wants.
+// The encoder E over the rows of prompts (src/model/bdh.rs:383,436-438): mixed [B*T, h*N] . decoder [h*N, d] as one product
+// per head, K cut into as many parts as the chip wants.
 // partial [*rows_out][B*T][d] receives the terms of every output row; the caller sums them in order.
 int bdh_launch_decoder_partials_f32(bdh_ctx *ctx, int B, int T, int h, int N, int d, const float *xy, const float *decoder,
                                     int *rows_out) {
   GemmF32 g;
   g.A = xy; g.B = decoder;
   g.lda = N; g.ldb = d; g.ldc = d; g.M = B * T; g.N = d;
-  if (T == 1) {
-    g.lda = g.K = h * N;
-  } else {
-    g.K = N; g.n_slices = h; g.mod = h;
-    g.a_s2 = (long)T * N; g.b_s2 = (long)N * d; g.c_s2 = (long)B * T * d;
-    g.rows_per = T; g.a_outer = (long)h * T * N;
-    g.c_outer = (long)T * d;
-  }
+  g.K = N; g.n_slices = h; g.mod = h;
+  g.a_s2 = (long)T * N; g.b_s2 = (long)N * d; g.c_s2 = (long)B * T * d;
+  g.rows_per = T; g.a_outer = (long)h * T * N;
+  g.c_outer = (long)T * d;
   const size_t one = sizeof(float) * (size_t)g.n_slices * g.M * d;
   const GemmPlan plan = bdh_gemm_f32_plan(ctx, g, (int)std::min<size_t>(64, std::max<size_t>(1, (size_t(256) << 20) / one)));
   int rc = bdh_ws_reserve(ctx, one * plan.ks);

@@ -224,8 +224,8 @@ int bdh_launch_decoder_residual(bdh_ctx *ctx, int B, int T, int h, int N, int d,
                                 const float *xy, const float *decoder, float *cur,
                                 const DecoderHead *head = nullptr);
 // logits = cur . lm_head (+ argmax of the last token per sequence) (src/model/bdh.rs:446-449)
-// attention_parallel.hip: the encoder's terms [*rows_out][B*T][d] in the context's workspace, from products on the matrix
-// cores (all of E is streamed, whatever is active)
+// attention_parallel.hip: the encoder's terms [*rows_out][B*T][d] of prompts in the context's workspace, from products on
+// the matrix cores (all of E is streamed, whatever is active)
 int bdh_launch_decoder_partials_f32(bdh_ctx *ctx, int B, int T, int h, int N, int d, const float *xy, const float *decoder,
                                     int *rows_out);
 int bdh_launch_lm_head(bdh_ctx *ctx, int B, int T, int d, int V, const float *cur,

@@ -3,6 +3,7 @@
 // Reference semantics: src/kernel/relu_lowrank.rs:7-37, src/model/bdh.rs:86-89, :319-322,
 // :346-350, :370-384, :436-449.
 #include "bdh_internal.h"
+#include "lds_copy.h"
 
 #include <algorithm>
 #include <atomic>
@@ -499,6 +500,8 @@ __global__ void k_embed_ln(const int64_t *__restrict__ tokens, int d, int V, con
   for (int c = lane; c < d; c += 64) out[row * d + c] = (s_row[c] - mean) / den;
 }
 
+__device__ const float4 g_zero_f4 = {0.0f, 0.0f, 0.0f, 0.0f};  // what a copy reads where its piece lies outside the operand
+
 // ------------------------------------------------------------------------------------
 // decoder: partial[kb][m][:] = sum_{k in block kb} mixed[m,k] * E[k,:]
 // mixed[m = b*T+t, k = hh*N+n] = xy[b,hh,t,n].  Rows of E whose xy is zero for every row
@@ -597,6 +600,122 @@ __global__ __launch_bounds__(256) void k_decoder_partial(const float *__restrict
         partial[((long)kb * M + m) * d + c] = s_red[c] + s_red[d + c] + s_red[2 * d + c] + s_red[3 * d + c];
     __syncthreads();
   }
+}
+
+// The encoder's first stage for a batch of decoding sequences (T = 1, so a row of xy is K contiguous values): the sums of
+// k_decoder_partial -- per k-block of KB rows of E four chains of fused multiply-adds over k = w, w + 4, ..., added as
+// ((c0 + c1) + c2) + c3 -- on the f32 matrix cores, whose v_mfma_f32_16x16x4_f32 adds its four k one after the other.
+// Four accumulators per tile, instruction w of a 16 deep step taking k = w, w + 4, w + 8, w + 12: the same bits, with
+// every row of E read once per 16 * RT sequences instead of once per eight.  (SPLIT: the k-blocks of 1024 of the form for
+// many sequences and a large E, one chain per block that runs 0, 8, 1, 9, ..., 7, 15 through each 16.)
+// A workgroup takes the k-blocks [blk * bpw, +bpw) and adds their sums in order: bpw is a sixteenth of the blocks, as
+// k_decoder_finalize would group them, or one.
+// Tile 16 * RT x 64, copied straight to LDS 32 k at a time into two buffers in turn.  What bounds it: a few workgroups per
+// CU, each a chain of KB / 32 trips to the L2.
+template <int RT, bool SPLIT>
+__global__ __launch_bounds__(256) void k_decoder_rows(const float *__restrict__ xy, const float *__restrict__ E,
+                                                      float *__restrict__ partial, long K, int d, int KB, int bpw, int M) {
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  constexpr int BM = 16 * RT, BN = 64, SK = 32, STAGE = (BM + BN) * SK, NA = SPLIT ? 1 : 4;
+  extern __shared__ __attribute__((aligned(1024))) float s_tiles[];  // two stages of xy [BM][32], E [32][64]
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int n0 = blockIdx.x * BN, m0 = blockIdx.y * BM;
+  const long k_lo = (long)blockIdx.z * bpw * KB, k_hi = min(K, k_lo + (long)bpw * KB);
+  // piece c of 16 bytes of row r of xy sits at place c ^ r / 2; of a row of E at place c ^ 4 x, x = which of the four k of
+  // an instruction the row is: the reads below then cover the 64 banks once
+  auto k_turn = [](int k) { return SPLIT ? ((k >> 3) & 1) | ((k & 1) << 1) : (k >> 2) & 3; };
+  constexpr int CA = (BM * 8 + 255) / 256;
+  const float *pa[CA], *pb[2];
+  int ka[CA], kb[2];  // this thread's k inside a stage
+#pragma unroll
+  for (int c = 0; c < CA; ++c) {
+    const int piece = c * 256 + tid, row = piece >> 3;
+    ka[c] = ((piece & 7) ^ ((row >> 1) & 7)) * 4;
+    pa[c] = xy + (long)min(m0 + row, M - 1) * K + k_lo + ka[c];
+  }
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const int piece = c * 256 + tid;
+    kb[c] = piece >> 4;
+    pb[c] = E + (k_lo + kb[c]) * d + min(n0 + ((piece & 15) ^ (k_turn(kb[c]) << 2)) * 4, d - 4);
+  }
+  const float *zero = reinterpret_cast<const float *>(&g_zero_f4);
+  auto issue = [&](long k0, int buf) {  // rows of E and values of xy beyond K are zero (K % 4 == 0)
+    float *s = s_tiles + buf * STAGE;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      bdh_copy_to_lds(k0 + kb[c] < K ? pb[c] : zero, s + BM * SK + (c * 256 + wave * 64) * 4);
+      pb[c] += (long)SK * d;
+    }
+#pragma unroll
+    for (int c = 0; c < CA; ++c) {
+      if (BM * 8 >= 256 || wave * 64 < BM * 8)
+        bdh_copy_to_lds(k0 + ka[c] < K ? pa[c] : zero, s + (c * 256 + wave * 64) * 4);
+      pa[c] += SK;
+    }
+  };
+  f32x4 total[RT], acc[NA][RT];
+#pragma unroll
+  for (int i = 0; i < RT; ++i) {
+    total[i] = (f32x4)(0.0f);
+#pragma unroll
+    for (int a = 0; a < NA; ++a) acc[a][i] = (f32x4)(0.0f);
+  }
+  const int r = lane & 15, q = lane >> 4;
+  issue(k_lo, 0);
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  int cur = 0;
+  for (long k0 = k_lo; k0 < k_hi; k0 += SK) {
+    if (k0 + SK < k_hi) issue(k0 + SK, cur ^ 1);  // lands while the matrix cores work on this stage
+    const float *sa = s_tiles + cur * STAGE, *sb = sa + BM * SK;
+    float fa[2][4][RT], fb[2][4];
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const int k = 16 * s + (SPLIT ? 2 * w + (q >> 1) + 8 * (q & 1) : 4 * q + w);
+        fb[s][w] = sb[k * BN + ((wave * 16 + r) ^ (q << 4))];
+#pragma unroll
+        for (int i = 0; i < RT; ++i) {
+          const int row = i * 16 + r;
+          fa[s][w][i] = sa[row * SK + ((k >> 2) ^ ((row >> 1) & 7)) * 4 + (k & 3)];
+        }
+      }
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int w = 0; w < 4; ++w)
+#pragma unroll
+        for (int i = 0; i < RT; ++i)
+          acc[SPLIT ? 0 : w][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[s][w][i], fb[s][w], acc[SPLIT ? 0 : w][i], 0, 0, 0);
+    if ((k0 + SK - k_lo) % KB == 0 || k0 + SK >= k_hi) {  // a k-block ends (KB % 32 == 0)
+#pragma unroll
+      for (int i = 0; i < RT; ++i) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float v = acc[0][i][e];
+          if constexpr (!SPLIT) v = ((v + acc[1][i][e]) + acc[2][i][e]) + acc[3][i][e];
+          total[i][e] += v;
+        }
+#pragma unroll
+        for (int a = 0; a < NA; ++a) acc[a][i] = (f32x4)(0.0f);
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    cur ^= 1;
+  }
+  // element e of lane l: row = (l/16)*4 + e, column = l%16
+  const int col = n0 + wave * 16 + r;
+  if (col >= d) return;
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int m = m0 + i * 16 + q * 4 + e;
+      if (m < M) partial[((long)blockIdx.z * M + m) * d + col] = total[i][e];
+    }
 }
 
 // The encoder's first stage for ONE row (a decode step of one sequence): partial[kb][:] = sum over the KB rows of
@@ -1173,15 +1292,45 @@ static void launch_decoder_finalize(bdh_ctx *ctx, const float *partial, int KBN,
   }
 }
 
+// The whole encoder of a batch of decoding sequences by k_decoder_rows.  The second stage adds the k-blocks in sixteen
+// groups; a workgroup adds up a whole group where the groups alone give every CU a workgroup.  The tile: 16 rows while that
+// leaves at most four workgroups for every CU, the chain of one tile being what counts; else 32, or 64 for more rows than
+// that, so that E passes fewer times.
+static int launch_decoder_rows(bdh_ctx *ctx, int M, long K, int d, int KB, bool split, const float *xy, const float *decoder,
+                               float *cur, const DecoderHead *head) {
+  const long n_cu = ctx->n_cu > 0 ? ctx->n_cu : 256;
+  const int KBN = (int)((K + KB - 1) / KB), per = (KBN + 15) / 16;
+  auto tiles = [&](int rows) { return (long)((d + 63) / 64) * ((M + rows - 1) / rows); };
+  const int bpw = tiles(16) * ((KBN + per - 1) / per) >= n_cu ? per : 1;
+  const int parts = (KBN + bpw - 1) / bpw;
+  const int rt = tiles(16) * parts <= 4 * n_cu ? 1 : M <= 32 ? 2 : 4;
+  int rc = bdh_ws_reserve(ctx, sizeof(float) * (size_t)parts * M * d);
+  if (rc != BDH_OK) return rc;
+  float *partial = static_cast<float *>(ctx->ws);
+  const dim3 grid((d + 63) / 64, (M + 16 * rt - 1) / (16 * rt), parts);
+  if (grid.y > 65535 || grid.z > 65535) return bdh_fail(ctx, BDH_E_SHAPE, "grid too large (%d rows, %d parts)", M, parts);
+#define BDH_DR(RT_, SPLIT_)                                                                                            \
+  hipLaunchKernelGGL((k_decoder_rows<RT_, SPLIT_>), grid, dim3(256), 2 * (16 * RT_ + 64) * 32 * sizeof(float), ctx->stream, \
+                     xy, decoder, partial, K, d, KB, bpw, M)
+  if (split) {
+    if (rt == 1) BDH_DR(1, true); else if (rt == 2) BDH_DR(2, true); else BDH_DR(4, true);
+  } else {
+    if (rt == 1) BDH_DR(1, false); else if (rt == 2) BDH_DR(2, false); else BDH_DR(4, false);
+  }
+#undef BDH_DR
+  BDH_LAUNCH_CHECK(ctx, "k_decoder_rows");
+  launch_decoder_finalize(ctx, partial, parts, M, d, cur, head);
+  BDH_LAUNCH_CHECK(ctx, "k_decoder_finalize");
+  return BDH_OK;
+}
+
 int bdh_launch_decoder_residual(bdh_ctx *ctx, int B, int T, int h, int N, int d, const float *xy,
                                 const float *decoder, float *cur, const DecoderHead *head) {
   const int M = B * T;
   const long K = (long)h * N;
   if (d > 1024 || (d & 3)) return bdh_fail(ctx, BDH_E_SHAPE, "decoder needs d %% 4 == 0 and d <= 1024, got %d", d);
-  // many rows: products on the matrix cores, all of E streamed once per row tile (fewer rows skip the inactive rows of E)
-  // (a negative option value -r takes it from r rows on in a decode step, too)
-  const int sk_rows = ctx->opt_decoder_splitk_rows;
-  if (T == 1 ? M >= std::abs(sk_rows) : (T >= 16 && M >= 24 && ctx->opt_decoder_mfma != 0)) {
+  // a prompt: products on the matrix cores, all of E streamed once per row tile (fewer rows skip the inactive rows of E)
+  if (T >= 16 && M >= 24 && ctx->opt_decoder_mfma != 0) {
     int rows = 0;
     int rc = bdh_launch_decoder_partials_f32(ctx, B, T, h, N, d, xy, decoder, &rows);
     if (rc != BDH_OK) return rc;
@@ -1189,14 +1338,23 @@ int bdh_launch_decoder_residual(bdh_ctx *ctx, int B, int T, int h, int N, int d,
     BDH_LAUNCH_CHECK(ctx, "k_decoder_finalize");
     return BDH_OK;
   }
+  const long n_cu = ctx->n_cu > 0 ? ctx->n_cu : 256;
   const int RT = M >= 8 ? 8 : (M >= 4 ? 4 : (M >= 2 ? 2 : 1));
   const int row_tiles = (M + RT - 1) / RT;
   // k-block size: enough workgroups to fill the chip, few enough partials
   // about two workgroups per CU: more k-blocks only add partials for the second stage to read
   int KB = 1024;
-  while (KB > 128 && ((K + KB - 1) / KB) * row_tiles < 2L * (ctx->n_cu > 0 ? ctx->n_cu : 256)) KB >>= 1;
+  while (KB > 128 && ((K + KB - 1) / KB) * row_tiles < 2 * n_cu) KB >>= 1;
   // a small model: down to 32 rows of E per workgroup, until there is a workgroup per CU
-  while (KB > 32 && ((K + KB - 1) / KB) * row_tiles < (ctx->n_cu > 0 ? ctx->n_cu : 256)) KB >>= 1;
+  while (KB > 32 && ((K + KB - 1) / KB) * row_tiles < n_cu) KB >>= 1;
+  // a batch of decoding sequences: the f32 matrix cores, the same bits; k-blocks of 1024 with a chain each once those fill
+  // half the chip in 32 x 64 tiles (a negative option value -r: from r sequences on, whatever the size)
+  const int sk_rows = ctx->opt_decoder_splitk_rows;
+  if (T == 1 && M >= std::abs(sk_rows) && (K & 3) == 0 && bdh_aligned(xy, 16) && bdh_aligned(decoder, 16)) {
+    const bool split = K % 1024 == 0 && (sk_rows < 0 || K / 1024 * ((d + 63) / 64) * ((M + 31) / 32) >= n_cu / 2);
+    if (split) KB = 1024;
+    return launch_decoder_rows(ctx, M, K, d, KB, split, xy, decoder, cur, head);
+  }
   const int KBN = (int)((K + KB - 1) / KB);
   size_t lds = sizeof(float) * (size_t)RT * KB;
   if (lds < sizeof(float) * 4u * d) lds = sizeof(float) * 4u * d;

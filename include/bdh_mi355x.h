@@ -106,8 +106,10 @@ const char *bdh_last_error(const bdh_ctx *ctx);
  *   "decoder.mfma":     1 (default) the encoder E of a call with 16+ tokens per sequence and 24+ rows runs on
  *                       the matrix cores, 0 = always the VALU kernel.
  *   "decoder.splitk_rows": 24 (default) a decode step (T = 1) of this many or more sequences runs the
- *                       encoder E on the matrix cores (all of E is streamed once, K cut into parts); fewer sequences take
- *                       the VALU kernel that skips inactive rows of E.  The sign is ignored.
+ *                       encoder E on the f32 matrix cores (all of E is streamed): the bits of the VALU kernel, which fewer
+ *                       sequences take and which skips the inactive rows of E; where k-blocks of 1024 fill half the chip,
+ *                       one chain per block instead (values agree to 1e-5).  A negative value -r takes that second form
+ *                       from r sequences on whatever the size (h * N a multiple of 1024).
  *   "model.one_launch": 1 (default) a decode step (T = 1, no x_tap / viz) of a model that is
  *                       small enough does not run kernel by kernel: a small model (d <= 256 and d % 4 == 0,
  *                       h * N <= 2048 and a multiple of 32, h in {1,2,4,8,16}, V <= 1024) can take ONE launch

@@ -176,3 +176,36 @@ def test_short_prompts_walk_the_state_where_that_is_faster_at_five_percent(bda, 
         finally:
             ctx.set_option("state_step.dense_chunks", -1)
     assert torch.equal(outs[0], outs[1]) == (not dense)
+
+
+@pytest.mark.parametrize("B,d,h,mult", [(48, 512, 8, 4), (24, 256, 4, 8), (33, 68, 2, 3), (64, 192, 4, 5), (65, 260, 2, 16),
+                                        (300, 64, 2, 2), (26, 256, 4, 128)])
+def test_batched_decode_encoder_on_the_matrix_cores(bda, B, d, h, mult):
+    """The encoder E of a batch of decoding sequences: row tiles of 16, 32 and 64, rows and columns that end inside a tile, a
+    reduction that is no multiple of a 32-deep stage, k-blocks added up in one workgroup and in the second stage.  The bits
+    of the VALU kernel, except in the last case, which is large enough for the form with one chain per block of 1024: there
+    and where that form is forced, 2^-24 per step of a few dozen steps, 1e-5."""
+    cfg = bda.BDHConfig(n_layer=1, n_embd=d, n_head=h, mlp_internal_dim_multiplier=mult, vocab_size=64)
+    cfg.fused_kernels.set_rotary_embedding(bda.RotaryEmbedding.ALIBI)
+    model = bda.BDH(cfg, DEV, seed=3)
+    N = mult * d // h
+    g = torch.Generator(device=DEV).manual_seed(B)
+    rho = 0.1 * torch.randn((1, B, h, N, d), device=DEV, generator=g)
+    tokens = torch.randint(0, 64, (B, 1), device=DEV, generator=g)
+    ctx = bda.ffi.default_context(0)
+    logits = {}
+    ctx.set_option("model.one_launch", 0)
+    try:
+        for rows in (24, -24, 1 << 30):
+            ctx.set_option("decoder.splitk_rows", rows)
+            state = model.init_state()
+            state.position, state.storage = 9, rho.clone()
+            state.layers[0].rho = state.storage[0]
+            logits[rows] = model.forward_with_state(tokens, state).clone()
+    finally:
+        ctx.set_option("decoder.splitk_rows", 24)
+        ctx.set_option("model.one_launch", 1)
+    valu = logits[1 << 30]
+    assert torch.equal(logits[24], valu) == (mult < 128)
+    assert rel_err(logits[24].cpu().numpy(), valu.cpu().numpy()) < 1e-5
+    assert rel_err(logits[-24].cpu().numpy(), valu.cpu().numpy()) < 1e-5
