@@ -1339,7 +1339,7 @@ int bdh_launch_decoder_residual(bdh_ctx *ctx, int B, int T, int h, int N, int d,
     return BDH_OK;
   }
   const long n_cu = ctx->n_cu > 0 ? ctx->n_cu : 256;
-  const int RT = M >= 8 ? 8 : (M >= 4 ? 4 : (M >= 2 ? 2 : 1));
+  const int RT = M >= 8 && d <= 512 ? 8 : (M >= 4 ? 4 : (M >= 2 ? 2 : 1));  // (wider rows: four in registers)
   const int row_tiles = (M + RT - 1) / RT;
   // k-block size: enough workgroups to fill the chip, few enough partials
   // about two workgroups per CU: more k-blocks only add partials for the second stage to read
@@ -1378,7 +1378,7 @@ int bdh_launch_decoder_residual(bdh_ctx *ctx, int B, int T, int h, int N, int d,
       hipLaunchKernelGGL((k_decoder_partial<1, 2, 8>), grid, dim3(256), lds, ctx->stream, xy, decoder, partial, T, h, N, d,
                          KB, M);
   } else {
-    if (RT >= 4) BDH_DEC(4, 4); else if (RT == 2) BDH_DEC(2, 4); else BDH_DEC(1, 4);
+    if (RT == 4) BDH_DEC(4, 4); else if (RT == 2) BDH_DEC(2, 4); else BDH_DEC(1, 4);
   }
 #undef BDH_DEC
   BDH_LAUNCH_CHECK(ctx, "k_decoder_partial");

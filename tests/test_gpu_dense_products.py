@@ -179,7 +179,7 @@ def test_short_prompts_walk_the_state_where_that_is_faster_at_five_percent(bda, 
 
 
 @pytest.mark.parametrize("B,d,h,mult", [(48, 512, 8, 4), (24, 256, 4, 8), (33, 68, 2, 3), (64, 192, 4, 5), (65, 260, 2, 16),
-                                        (300, 64, 2, 2), (26, 256, 4, 128)])
+                                        (300, 64, 2, 2), (40, 640, 2, 2), (26, 256, 4, 128)])
 def test_batched_decode_encoder_on_the_matrix_cores(bda, B, d, h, mult):
     """The encoder E of a batch of decoding sequences: row tiles of 16, 32 and 64, rows and columns that end inside a tile, a
     reduction that is no multiple of a 32-deep stage, k-blocks added up in one workgroup and in the second stage.  The bits
@@ -209,3 +209,22 @@ def test_batched_decode_encoder_on_the_matrix_cores(bda, B, d, h, mult):
     assert torch.equal(logits[24], valu) == (mult < 128)
     assert rel_err(logits[24].cpu().numpy(), valu.cpu().numpy()) < 1e-5
     assert rel_err(logits[-24].cpu().numpy(), valu.cpu().numpy()) < 1e-5
+
+
+@pytest.mark.parametrize("B,T,d", [(8, 1, 516), (13, 1, 768), (3, 5, 640), (23, 1, 1024), (30, 1, 1024)])
+def test_encoder_of_wide_rows_covers_every_row(bda, B, T, d):
+    """Rows wider than 512, eight and more of them: each sequence gets the logits of a call of its own (other orders of the
+    sums over 1024 and fewer terms: 1e-5)."""
+    cfg = bda.BDHConfig(n_layer=2, n_embd=d, n_head=2, mlp_internal_dim_multiplier=1, vocab_size=64)
+    cfg.fused_kernels.set_rotary_embedding(bda.RotaryEmbedding.ALIBI)
+    model = bda.BDH(cfg, DEV, seed=3)
+    tokens = torch.randint(0, 64, (B, T + 1), generator=torch.Generator().manual_seed(d))
+
+    def last(rows):
+        state = model.init_state()
+        model.forward_with_state(tokens[rows, :1], state)  # the first token reads an empty state: nothing to encode
+        return model.forward_with_state(tokens[rows, 1:], state).cpu().numpy()
+
+    whole = last(slice(0, B))
+    for b in range(B):
+        assert rel_err(whole[b], last(slice(b, b + 1))[0]) < 1e-5
