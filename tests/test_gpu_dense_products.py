@@ -228,3 +228,27 @@ def test_encoder_of_wide_rows_covers_every_row(bda, B, T, d):
     whole = last(slice(0, B))
     for b in range(B):
         assert rel_err(whole[b], last(slice(b, b + 1))[0]) < 1e-5
+
+
+@pytest.mark.parametrize("T,N,d", [(128, 256, 256), (200, 256, 256), (2048, 256, 64)])
+def test_split_products_round_the_large_sum_once(bda, T, N, d):
+    """Row-normalised attention against float64.  A sum of K = 256 products is rounded K / 16 times on the way, the relative
+    error of one rounding being at most 2^-24 and 2^-25.8 in the mean square, over sums that grow: sqrt(16 / 3) * 2^-25.8 =
+    0.4e-7 for the scores, their own rounding, and as much again for the second product; 1.8e-7 = 3 * 2^-24 leaves room for a
+    factor of two.  Sums rounded at each of the six instructions of a step are at 2.7e-7."""
+    from burn_dragon_amd.kernel.linear_attention import build_freqs, default_alibi_slopes, fused_state_aligned
+
+    h, block = 2, 64
+    g = torch.Generator(device=DEV).manual_seed(T)
+    q = torch.relu(torch.randn((1, h, T, N), device=DEV, generator=g))
+    v = torch.randn((1, 1, T, d), device=DEV, generator=g)
+    slopes = torch.tensor(default_alibi_slopes(h))
+    out = fused_state_aligned(q, v, build_freqs(N, 65536.0, bda.RotaryEmbedding.ALIBI, device=DEV), slopes,
+                              bda.BlockPattern2d.dense(block), bda.RotaryEmbedding.ALIBI)
+    i = torch.arange(T, device=DEV)
+    S = torch.matmul(q.double(), q.double().transpose(-1, -2).contiguous())
+    S = torch.where(i[None, :] < i[:, None], S, 0.0)
+    bias = slopes.to(DEV).double()[None, :, None, None] * (i[None, :] - i[:, None]).double()
+    S = torch.where(i[None, :] // block <= i[:, None] // block, S + bias, 0.0)
+    ref = torch.matmul(S, v.double().expand(1, h, T, d).contiguous()) / (S.abs().sum(-1, keepdim=True) + 1e-6)
+    assert float((out.double() - ref).norm() / ref.norm()) < 1.8e-7
