@@ -1173,13 +1173,19 @@ int bdh_launch_relu_lowrank(bdh_ctx *ctx, const ReluLowrankParams &p) {
     }
     mask_dev = static_cast<const unsigned char *>(ctx->lat_mask);
   }
+  const bool pieces = p.d % 32 == 0 && p.N % 4 == 0 && bdh_aligned(p.in, 16) && bdh_aligned(p.weight, 16);
   // A matrix of up to 16 MiB (it sits in the L2) and few outputs: 64 columns per workgroup, every weight in flight at once,
   // as many rows per workgroup (1, 2, 4, 8) as still give a workgroup per CU.  The line is at 32768 outputs, 128 for every
   // CU (us, this | 16-row matrix-core tiles: h*N = 2048, d = 512, 16 rows 7.6 | 8.8, 24 rows 12.8 | 8.9; 1024, 256, 32 rows
   // 5.4 | 6.0, 48 rows 6.3 | 6.0; 4096, 256, 8 rows 5.4 | 6.0, 16 rows 7.6 | 6.0; 8192, 512, 4 rows 7.5 | 8.9, 8 rows 11.1 | 8.9).
-  const int n_cu_rl = ctx->n_cu > 0 ? ctx->n_cu : 256;
+  // Fewer than 64 rows that do not come in 16-byte pieces have the thread-per-column kernel for an alternative, a chain of d
+  // LDS reads: four times as many outputs then, eight times up to d = 256 (us, this | that: h*N = 4088, d = 250, 63 rows
+  // 13.0 | 17.6; 16376, 200, 16 rows 12.8 | 15.0, 24 rows 20 | 15; 4104, 500, 24 rows 19 | 29, 32 rows 33 | 29; 8192, 260, 8 rows
+  // 10.5 | 17.2, 24 rows 33 | 17.5).
+  const long n_cu_rl = ctx->n_cu > 0 ? ctx->n_cu : 256;
+  const long row_line = (pieces || M >= 64 ? 128 : p.d <= 256 ? 1024 : 512) * n_cu_rl;
   if (p.d >= 128 && p.d <= 512 && ctx->opt_lowrank_row != 0 &&
-      sizeof(float) * (size_t)p.h * p.d * p.N <= (size_t(16) << 20) && (M == 1 || M * p.h * p.N <= 128L * n_cu_rl)) {
+      sizeof(float) * (size_t)p.h * p.d * p.N <= (size_t(16) << 20) && (M == 1 || M * p.h * p.N <= row_line)) {
     const long col_blocks = (p.N + 63) / 64;
     int rt = 1;
     if (M > 1) {
@@ -1205,15 +1211,16 @@ int bdh_launch_relu_lowrank(bdh_ctx *ctx, const ReluLowrankParams &p) {
     return BDH_OK;
   }
   // Two rows and more: the f32 matrix cores, same values, the weights streamed once per row tile (options: fewer than 64
-  // rows from mfma_rows on, more from gemm_rows on; 0 = never).  Fewer than 64 rows want the 16-byte pieces of the copying
-  // kernels; what is left, and a single row of a larger matrix, runs a thread per column with its input rows in LDS.  Eight
-  // rows and more that do not fit there (d above 2048) take the matrix cores whatever the options say.
+  // rows from mfma_rows on, more from gemm_rows on; 0 = never).  Fewer than 32 rows want the 16-byte pieces of the copying
+  // kernels; what is left, and a single row of a larger matrix, runs a thread per column with its input rows in LDS, which
+  // reads the weights again for every eight rows (without pieces, us, this | the checked 64 x 64 tiles: h*N = 65520, d = 250,
+  // 16 rows 26 | 35, 24 rows 35 | 35, 32 rows 44 | 36, 63 rows 79 | 41; d = 100, 24 rows 16 | 18, 48 rows 26 | 20).  Eight rows
+  // and more that do not fit there (d above 2048) take the matrix cores whatever the options say.
   const int mc_rows = std::abs(M < 64 ? ctx->opt_lowrank_mfma_rows : ctx->opt_lowrank_gemm_rows);
-  const bool pieces = p.d % 32 == 0 && p.N % 4 == 0 && bdh_aligned(p.in, 16) && bdh_aligned(p.weight, 16);
   const int RT = M >= 8 ? 8 : (M >= 4 ? 4 : (M >= 2 ? 2 : 1));
   const size_t lds = sizeof(float) * (size_t)RT * (p.d > 0 ? p.d : 1);
   if (p.d > 0 && p.N > 0 && M > 1 &&
-      ((mc_rows > 0 && M >= mc_rows && (M >= 64 || pieces)) || (RT == 8 && lds > 64 * 1024)))
+      ((mc_rows > 0 && M >= mc_rows && (M >= 32 || pieces)) || (RT == 8 && lds > 64 * 1024)))
     return bdh_launch_relu_lowrank_gemm(ctx, p, mask_dev);
   if (lds > 64 * 1024) return bdh_fail(ctx, BDH_E_SHAPE, "d=%d too large for the projection tile", p.d);
   const long row_tiles = (M + RT - 1) / RT;

@@ -252,3 +252,18 @@ def test_split_products_round_the_large_sum_once(bda, T, N, d):
     S = torch.where(i[None, :] // block <= i[:, None] // block, S + bias, 0.0)
     ref = torch.matmul(S, v.double().expand(1, h, T, d).contiguous()) / (S.abs().sum(-1, keepdim=True) + 1e-6)
     assert float((out.double() - ref).norm() / ref.norm()) < 1.8e-7
+
+
+@pytest.mark.parametrize("M,d,h,N", [(7, 130, 2, 515), (16, 250, 4, 1022), (24, 256, 4, 515), (31, 384, 4, 1030), (31, 200, 3, 67),
+                                     (32, 384, 4, 1030), (33, 100, 2, 9001), (63, 250, 4, 1022), (63, 700, 2, 30)])
+def test_relu_lowrank_without_16_byte_pieces(bda, corc, M, d, h, N):
+    """Widths that no 16-byte access fits, around the lines between the few-outputs kernel, the thread-per-column kernel and
+    the checked matrix-core tiles: the bits of the k-sequential chain."""
+    from burn_dragon_amd.kernel import relu_lowrank
+
+    rng = np.random.default_rng(M + N)
+    inp = rng.standard_normal((M, 1, 1, d)).astype(np.float32)
+    weight = rng.standard_normal((h, d, N)).astype(np.float32)
+    got = relu_lowrank.fused_forward(torch.from_numpy(inp).to(DEV), torch.from_numpy(weight).to(DEV), None, 0.0,
+                                     bda.BlockPattern1d.dense(64))
+    assert np.array_equal(got.cpu().numpy(), corc.relu_lowrank(inp, weight))
