@@ -430,20 +430,20 @@ __device__ __forceinline__ void ln_stats_in_order(const float *s_row, int d, flo
   den = sqrtf(sq / (float)d + kLnEps);
 }
 
-// One wavefront per row, blockDim.x / 64 rows per workgroup: the index-order sums are the same work in every lane, so more
-// wavefronts on a row only repeat it (a workgroup of four per row: 25 against 12 us for the embedding of 4088 tokens).
-__global__ void k_layer_norm(const float *__restrict__ in, float *__restrict__ out, int d, long rows) {
+// `per` rows per workgroup of 256 threads, 256 / per threads each (see ln_rows_per_wg).
+__global__ __launch_bounds__(256) void k_layer_norm(const float *__restrict__ in, float *__restrict__ out, int d, long rows,
+                                                    int per) {
   extern __shared__ float s_rows[];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const long row = (long)blockIdx.x * (blockDim.x >> 6) + wave;
-  float *s_row = s_rows + (long)wave * ((d + 3) & ~3);
+  const int nt = 256 / per, lane = threadIdx.x % nt;
+  const long row = (long)blockIdx.x * per + threadIdx.x / nt;
+  float *s_row = s_rows + (long)(threadIdx.x / nt) * ((d + 3) & ~3);
   if (row < rows)
-    for (int c = lane; c < d; c += 64) s_row[c] = in[row * d + c];
+    for (int c = lane; c < d; c += nt) s_row[c] = in[row * d + c];
   __syncthreads();
   if (row >= rows) return;
   float mean, den;
   ln_stats_in_order(s_row, d, mean, den);
-  for (int c = lane; c < d; c += 64) out[row * d + c] = (s_row[c] - mean) / den;
+  for (int c = lane; c < d; c += nt) out[row * d + c] = (s_row[c] - mean) / den;
 }
 
 // LayerNorm of many rows for internal use (the readout of a many-token state step): one wave per row, the
@@ -478,26 +478,26 @@ __global__ __launch_bounds__(256) void k_layer_norm_wave(const float *__restrict
     if (j * 64 + lane < d) y[j * 64 + lane] = (v[j] - mean) / den;
 }
 
-// embed gather + LayerNorm (src/model/bdh.rs:319-322), a wavefront per row like k_layer_norm
-__global__ void k_embed_ln(const int64_t *__restrict__ tokens, int d, int V, const float *__restrict__ embed,
-                           float *__restrict__ out, long rows) {
+// embed gather + LayerNorm (src/model/bdh.rs:319-322), rows laid out like k_layer_norm's
+__global__ __launch_bounds__(256) void k_embed_ln(const int64_t *__restrict__ tokens, int d, int V,
+                                                  const float *__restrict__ embed, float *__restrict__ out, long rows, int per) {
   extern __shared__ float s_rows[];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const long row = (long)blockIdx.x * (blockDim.x >> 6) + wave;
-  float *s_row = s_rows + (long)wave * ((d + 3) & ~3);
+  const int nt = 256 / per, lane = threadIdx.x % nt;
+  const long row = (long)blockIdx.x * per + threadIdx.x / nt;
+  float *s_row = s_rows + (long)(threadIdx.x / nt) * ((d + 3) & ~3);
   const int64_t tok = row < rows ? tokens[row] : -1;
   const bool known = tok >= 0 && tok < V;
   if (known)
-    for (int c = lane; c < d; c += 64) s_row[c] = embed[tok * d + c];
+    for (int c = lane; c < d; c += nt) s_row[c] = embed[tok * d + c];
   __syncthreads();
   if (row >= rows) return;
   if (!known) {  // the reference's gather would panic; poison the row instead
-    for (int c = lane; c < d; c += 64) out[row * d + c] = __int_as_float(0x7fc00000);
+    for (int c = lane; c < d; c += nt) out[row * d + c] = __int_as_float(0x7fc00000);
     return;
   }
   float mean, den;
   ln_stats_in_order(s_row, d, mean, den);
-  for (int c = lane; c < d; c += 64) out[row * d + c] = (s_row[c] - mean) / den;
+  for (int c = lane; c < d; c += nt) out[row * d + c] = (s_row[c] - mean) / den;
 }
 
 __device__ const float4 g_zero_f4 = {0.0f, 0.0f, 0.0f, 0.0f};  // what a copy reads where its piece lies outside the operand
@@ -1236,17 +1236,20 @@ int bdh_launch_relu_lowrank(bdh_ctx *ctx, const ReluLowrankParams &p) {
   return BDH_OK;
 }
 
-// rows of an index-order LayerNorm kernel per workgroup: four, fewer when they would not fit in LDS
-static int ln_rows_per_wg(int d) { return d <= 4096 ? 4 : 1; }
-static size_t ln_lds(int d) { return sizeof(float) * (size_t)((d + 3) & ~3) * ln_rows_per_wg(d); }
+// Rows of an index-order LayerNorm kernel per workgroup of 256 threads.  The sums are the same work in every wavefront, so four
+// rows to a workgroup once there are more than two workgroups of one for every CU (us, one | four rows: 1536 x 256 10.3 | 6.7,
+// 1024 x 1000 26 | 18, 512 x 1000 16.1 | 17.6, 64 x 4096 55 | 63: with few rows the loads and stores of a row want all four
+// wavefronts); wider rows than 4096 fit into LDS one at a time.
+static int ln_rows_per_wg(const bdh_ctx *ctx, int64_t rows, int d) { return d <= 4096 && rows > 2L * (ctx->n_cu > 0 ? ctx->n_cu : 256) ? 4 : 1; }
+static size_t ln_lds(int d, int per) { return sizeof(float) * (size_t)((d + 3) & ~3) * per; }
 
 int bdh_launch_layer_norm(bdh_ctx *ctx, int64_t rows, int d, const float *in, float *out) {
   if (rows > 0x7fffffffL) return bdh_fail(ctx, BDH_E_SHAPE, "too many rows");
   if (d > 16384) return bdh_fail(ctx, BDH_E_SHAPE, "LayerNorm row of %d floats does not fit in LDS", d);
   if (rows == 0) return BDH_OK;
-  const int per = ln_rows_per_wg(d);
-  hipLaunchKernelGGL(k_layer_norm, dim3((unsigned)((rows + per - 1) / per)), dim3(64 * per), ln_lds(d), ctx->stream, in, out,
-                     d, (long)rows);
+  const int per = ln_rows_per_wg(ctx, rows, d);
+  hipLaunchKernelGGL(k_layer_norm, dim3((unsigned)((rows + per - 1) / per)), dim3(256), ln_lds(d, per), ctx->stream, in, out, d,
+                     (long)rows, per);
   BDH_LAUNCH_CHECK(ctx, "k_layer_norm");
   return BDH_OK;
 }
@@ -1264,9 +1267,9 @@ int bdh_launch_layer_norm_rows(bdh_ctx *ctx, int64_t rows, int d, const float *i
 int bdh_launch_embed_ln(bdh_ctx *ctx, const int64_t *tokens, int64_t rows, int d, int V, const float *embed,
                         float *out) {
   if (rows == 0) return BDH_OK;
-  const int per = ln_rows_per_wg(d);
-  hipLaunchKernelGGL(k_embed_ln, dim3((unsigned)((rows + per - 1) / per)), dim3(64 * per), ln_lds(d), ctx->stream, tokens, d,
-                     V, embed, out, (long)rows);
+  const int per = ln_rows_per_wg(ctx, rows, d);
+  hipLaunchKernelGGL(k_embed_ln, dim3((unsigned)((rows + per - 1) / per)), dim3(256), ln_lds(d, per), ctx->stream, tokens, d, V,
+                     embed, out, (long)rows, per);
   BDH_LAUNCH_CHECK(ctx, "k_embed_ln");
   return BDH_OK;
 }

@@ -267,3 +267,11 @@ def test_relu_lowrank_without_16_byte_pieces(bda, corc, M, d, h, N):
     got = relu_lowrank.fused_forward(torch.from_numpy(inp).to(DEV), torch.from_numpy(weight).to(DEV), None, 0.0,
                                      bda.BlockPattern1d.dense(64))
     assert np.array_equal(got.cpu().numpy(), corc.relu_lowrank(inp, weight))
+
+
+@pytest.mark.parametrize("rows,d", [(3, 4096), (512, 36), (513, 36), (515, 1001), (2, 4100), (600, 4097)])
+def test_layer_norm_one_and_four_rows_per_workgroup(bda, corc, rows, d):
+    from burn_dragon_amd.recurrent import layer_norm
+
+    x = np.random.default_rng(d).standard_normal((rows, d)).astype(np.float32)
+    assert np.array_equal(layer_norm(torch.from_numpy(x).to(DEV)).cpu().numpy(), corc.layer_norm(x))
