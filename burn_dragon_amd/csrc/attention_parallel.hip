@@ -769,11 +769,6 @@ int bdh_launch_state_chunks_f32(bdh_ctx *ctx, const StateStepParams &p, float *o
   float log_decay[64] = {0};
   if (alibi)
     for (int i = 0; i < h; ++i) log_decay[i] = bdh_log_decay(p.slopes_host[i]);
-  if (p.stamps) {  // a lazily decayed state: apply what is pending, the products below decay every row themselves
-    int rc0 = bdh_launch_alibi_materialize(ctx, B, h, N, d, p.slopes_host, p.position, p.positions_dev, p.rho,
-                                           p.rho_dtype, p.stamps);
-    if (rc0 != BDH_OK) return rc0;
-  }
   if (S > 0x7fffffffL / 4096) return bdh_fail(ctx, BDH_E_SHAPE, "B*h too large");
   // chunk length: a multiple of 128 between 128 and 512 whose rotated activations stay under 4 GiB
   const size_t per_token = sizeof(float) * (size_t)S * Nq;
@@ -841,6 +836,11 @@ int bdh_launch_state_chunks_f32(bdh_ctx *ctx, const StateStepParams &p, float *o
   const size_t wide_bytes = bf16_state ? bdh_align_up(sizeof(float) * n_state, 256) : 0;
   int rc = bdh_ws_reserve(ctx, q_bytes + sc_bytes + parts_bytes + wide_bytes);
   if (rc != BDH_OK) return rc;
+  if (p.stamps) {  // a lazily decayed state: apply what is pending, the products below decay every row themselves
+    int rc0 = bdh_launch_alibi_materialize(ctx, B, h, N, d, p.slopes_host, p.position, p.positions_dev, p.rho,
+                                           p.rho_dtype, p.stamps);
+    if (rc0 != BDH_OK) return rc0;
+  }
   char *ws = static_cast<char *>(ctx->ws);
   float *q = reinterpret_cast<float *>(ws);
   float *scores = reinterpret_cast<float *>(ws + q_bytes);

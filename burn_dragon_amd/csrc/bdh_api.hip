@@ -17,6 +17,8 @@ int bdh_fail(bdh_ctx *ctx, int status, const char *fmt, ...) {
 int bdh_ws_reserve(bdh_ctx *ctx, size_t bytes) {
   if (bytes <= ctx->ws_bytes) return BDH_OK;
   bytes = bdh_align_up(bytes, size_t(1) << 20);
+  if (ctx->opt_ws_max_mib > 0 && bytes > (size_t)ctx->opt_ws_max_mib << 20)
+    return bdh_fail(ctx, BDH_E_NOMEM, "workspace of %zu bytes: workspace.max_mib is %d", bytes, ctx->opt_ws_max_mib);
   if (ctx->ws) {
     BDH_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
     BDH_HIP_CHECK(ctx, hipFree(ctx->ws));
@@ -201,6 +203,11 @@ int bdh_ctx_set_option(bdh_ctx *ctx, const char *name, int value) {
   if (strcmp(name, "state_step.prompt_bf16") == 0) {
     if (value < 0) return bdh_fail(ctx, BDH_E_INVAL, "state_step.prompt_bf16 takes 0 (never) or a token count");
     ctx->opt_step_prompt_bf16 = value;
+    return BDH_OK;
+  }
+  if (strcmp(name, "workspace.max_mib") == 0) {
+    if (value < 0) return bdh_fail(ctx, BDH_E_INVAL, "workspace.max_mib takes 0 (no limit) or a size in MiB");
+    ctx->opt_ws_max_mib = value;
     return BDH_OK;
   }
   return bdh_fail(ctx, BDH_E_INVAL, "unknown option '%s'", name);

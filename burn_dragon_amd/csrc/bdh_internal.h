@@ -32,6 +32,7 @@ struct bdh_ctx {
   int opt_lowrank_mfma_rows = 2;  // relu_lowrank of fewer than 64 rows takes the f32 matrix cores from this many on (0: never)
   int opt_step_dense_kernel = 1;  // 0: PoPE / eager ALiBi at d in {256,512} take the generic kernel
   int opt_decoder_splitk_rows = 24;  // decode-step encoder on the matrix cores from this many sequences on
+  int opt_ws_max_mib = 0;   // the workspace never grows beyond this (0: no limit)
   int opt_fsa_path = -1;    // fused_state_aligned: -1 choose by T, 0 row kernel, 1 f32 matrix cores
   int opt_model_fused_rows = 1;  // 0: a one-sequence decode step never folds its reductions into the projections
   int opt_model_fused_kb = 256;  // rows of E per workgroup of the encoder's first stage in that form

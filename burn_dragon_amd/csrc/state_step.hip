@@ -1136,8 +1136,11 @@ int bdh_launch_state_steps_in(bdh_ctx *ctx, const StateStepParams &p, float *out
                           (p.rho_dtype == BDH_F32 || sizeof(float) * (size_t)slices * Nq * d <= (size_t(64) << 30));
   const bool dense_auto = T >= dense_form_from(p, fast);
   if (!fixed && !p.bitmask && !p.rows_touched && chunk_fits &&
-      (ctx->opt_step_dense >= 0 ? ctx->opt_step_dense == 1 : dense_auto))
-    return bdh_launch_state_chunks_f32(ctx, p, out_ln);
+      (ctx->opt_step_dense >= 0 ? ctx->opt_step_dense == 1 : dense_auto)) {
+    // without room for its workspace (a whole f32 copy of a bf16 state) nothing has been launched: the token loop needs less
+    const int rc = bdh_launch_state_chunks_f32(ctx, p, out_ln);
+    if (rc != BDH_E_NOMEM || ctx->opt_step_dense == 1) return rc;
+  }
   // tokens per launch: the f32 RoPE kernel, the generic and the dense streaming kernel walk several, as many as
   // 64 MiB of partials allow
   const size_t partial_one = bdh_align_up(sizeof(float) * (size_t)slices * S * d, 256);

@@ -82,7 +82,10 @@ const char *bdh_last_error(const bdh_ctx *ctx);
  *                       at most 512 KiB (B*h*N*d floats, d 256 or 512): there a call of any number of tokens leaves the
  *                       bits that single-token calls leave.  Any other call of many tokens agrees with them to f32
  *                       rounding (a bf16 state is rounded once at its end instead of after every token),
- *                       0 = always token by token, 1 = dense products for any T.
+ *                       0 = always token by token, 1 = dense products for any T.  A call whose dense form finds no room
+ *                       for its workspace (a bf16 state: an f32 copy of it) is walked token by token, except with 1.
+ *   "workspace.max_mib": 0 (default) the context's workspace grows as calls need it; else a call that needs more fails with
+ *                       BDH_E_NOMEM as if the device had no more memory.
  *   "state_step.prompt_bf16": 0 (default) never; T0 > 0: a call of T0 or more tokens on an f32 state, with the
  *                       position given by the host and no bitmask / row-count outputs, runs as
  *                       bdh_prefill_chunked_ex does: on the bf16 matrix cores, activations, values and scores

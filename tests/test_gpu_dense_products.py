@@ -275,3 +275,36 @@ def test_layer_norm_one_and_four_rows_per_workgroup(bda, corc, rows, d):
 
     x = np.random.default_rng(d).standard_normal((rows, d)).astype(np.float32)
     assert np.array_equal(layer_norm(torch.from_numpy(x).to(DEV)).cpu().numpy(), corc.layer_norm(x))
+
+
+@pytest.mark.parametrize("kind", ["rope", "lazy"])
+def test_prompt_without_room_for_the_dense_form_is_walked(bda, kind):
+    """A bf16 state whose f32 copy does not fit: the token loop's bits, no error; an error where the dense form was asked for."""
+    from burn_dragon_amd.kernel.linear_attention import build_freqs
+    from burn_dragon_amd.recurrent import recurrent_attention, recurrent_attention_lazy_alibi
+
+    B, h, T, N, d = 4, 4, 96, 8192, 256  # 128 MiB of f32 state
+    g = torch.Generator(device=DEV).manual_seed(1)
+    x = torch.relu(torch.randn((B, h, T, N), device=DEV, generator=g) - 1.645)
+    v = torch.randn((B, T, d), device=DEV, generator=g)
+    rho = (0.01 * torch.randn((B, h, N, d), device=DEV, generator=g)).bfloat16()
+    stamps = torch.randint(0, 8, (B, h, N), device=DEV, generator=g, dtype=torch.int32)
+    freqs = build_freqs(N, 65536.0, bda.RotaryEmbedding.ROPE, device=DEV).reshape(-1)
+
+    def call(mib, mode):
+        ctx = bda.ffi.Context(0)
+        ctx.set_option("workspace.max_mib", mib)
+        ctx.set_option("state_step.dense_chunks", mode)
+        state, at = rho.clone(), stamps.clone()
+        if kind == "rope":
+            out = recurrent_attention(x, v, state, freqs, 7, bda.RotaryEmbedding.ROPE, ctx=ctx)
+        else:
+            out = recurrent_attention_lazy_alibi(x, v, state, at, 7, ctx=ctx)
+        torch.cuda.synchronize()
+        return out, state, at
+
+    walked, short, dense = call(0, 0), call(72, -1), call(0, -1)
+    assert all(torch.equal(a, b) for a, b in zip(walked, short))
+    assert not torch.equal(dense[0], walked[0])  # with room the products are taken
+    with pytest.raises(bda.ffi.BdhError):
+        call(72, 1)
