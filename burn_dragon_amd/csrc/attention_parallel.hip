@@ -817,7 +817,6 @@ int bdh_launch_state_chunks_f32(bdh_ctx *ctx, const StateStepParams &p, float *o
     r.decay_state = alibi;
     const size_t most = size_t(256) << 20;
     const size_t one_s = sizeof(float) * (size_t)S * tc * tc, one_o = sizeof(float) * (size_t)S * tc * d;
-    o.A2 = reinterpret_cast<const float *>(1);  // counts K2 in the plan; set below
     c.p_out = bdh_gemm_f32_plan(ctx, o, (int)std::min<size_t>(32, std::max<size_t>(1, most / one_o)));
     g.reader_rows = bdh_gemm_f32_rows(c.p_out);
     c.p_scores = bdh_gemm_f32_plan(ctx, g, (int)std::min<size_t>(32, std::max<size_t>(1, most / one_s)));

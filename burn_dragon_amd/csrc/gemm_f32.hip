@@ -431,7 +431,7 @@ bool lower_triangle(const GemmF32 &g, int tile) {
 GemmPlan bdh_gemm_f32_plan(const bdh_ctx *ctx, const GemmF32 &g, int max_split) {
   const double n_cu = ctx->n_cu > 0 ? ctx->n_cu : 256;
   constexpr double full[3] = {2600.0, 900.0, 900.0}, alone[3] = {3600.0, 2000.0, 2000.0};
-  const int nb = (g.K + FK - 1) / FK + (g.A2 ? (g.K2 + FK - 1) / FK : 0);
+  const int nb = (g.K + FK - 1) / FK + (g.K2 + FK - 1) / FK;
   GemmPlan best;
   double best_t = 1e300;
   for (int t = 0; t < 3; ++t) {
@@ -462,7 +462,7 @@ int bdh_launch_gemm_f32(bdh_ctx *ctx, GemmF32 g, bool a_kmajor, bool b_kmajor, c
   g.mt = (g.M + kTileM[plan.tile] - 1) / kTileM[plan.tile];
   g.nt = (g.N + kTileN[plan.tile] - 1) / kTileN[plan.tile];
   g.tri = lower_triangle(g, plan.tile);
-  const int nb = (g.K + FK - 1) / FK + (g.A2 ? (g.K2 + FK - 1) / FK : 0);
+  const int nb = (g.K + FK - 1) / FK + (g.K2 + FK - 1) / FK;
   g.ks = plan.ks;
   g.kb_per = (nb + g.ks - 1) / g.ks;
   if (g.ks > 1) {

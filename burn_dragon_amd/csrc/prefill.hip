@@ -35,7 +35,6 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 constexpr float kTwoPi = 6.28318530717958647692f;
 constexpr int BM = 256, BN = 256, BK = 64;
-constexpr long kFullChip = 256;  // workgroups from which a larger tile pays: one per CU
 
 __device__ __forceinline__ unsigned short f32_to_bf16_bits(float f) {
   unsigned int u = __float_as_uint(f);
@@ -1367,19 +1366,20 @@ static int prefill_pass_scores(bdh_ctx *ctx, int B, int h, int T, int N, int d, 
   const bool ext = pm.extended();
   const bool stateless = pm.row_norm;
   const bool has_state = !state_is_zero && !stateless;
+  const long full_chip = ctx->n_cu > 0 ? ctx->n_cu : 256;  // workgroups from which a larger tile pays: one per CU
   auto tiles = [](long n, int tile) { return (n + tile - 1) / tile; };
   // S V reads the scores by its own whole tiles, which lie within theirs.  The out products take the largest tile that
   // still gives every CU a workgroup, 256 only where its padding is below an eighth.  Measured, us a call
   // (ALiBi, N = 4096, d = 256, carried): 32 slices of 2000 tokens 1148 with 256, 1227 with 128; 16 slices of 2048 tokens
   // (128 output tiles of 256) 762 with 256, 640 with 128; 8 slices of 2048 tokens 446 with 64, 327 with 128.
-  const bool big = d % 256 == 0 && Nq % BK == 0 && S * tiles(T, 256) * (d / 256) >= kFullChip &&
+  const bool big = d % 256 == 0 && Nq % BK == 0 && S * tiles(T, 256) * (d / 256) >= full_chip &&
                    (tiles(T, 256) * 256 - T) * 8 <= T;
-  const int tile_t = big ? 256 : S * tiles(T, 128) * tiles(d, 128) >= kFullChip ? 128 : 64;
-  const int tile_r = S * tiles(Nq, 128) * tiles(d, 128) >= kFullChip ? 128 : 64;
+  const int tile_t = big ? 256 : S * tiles(T, 128) * tiles(d, 128) >= full_chip ? 128 : 64;
+  const int tile_r = S * tiles(Nq, 128) * tiles(d, 128) >= full_chip ? 128 : 64;
   // The scores, of which there are more tiles, may have the larger one: 12 slices of 777 tokens, whose 168 output tiles
   // are 64 wide, 248 us a call with scores of 64, 238 with 128 (336 tiles).
   auto lower = [&](int tile) { return S * tiles(T, tile) * (tiles(T, tile) + 1) / 2; };
-  const int tile_s = !big && lower(128) >= kFullChip ? 128 : tile_t;
+  const int tile_s = !big && lower(128) >= full_chip ? 128 : tile_t;
   const int mt = (int)tiles(T, tile_t), nt_d = (int)tiles(d, tile_t), mt_s = (int)tiles(T, tile_s);
   // a time block that straddles two score tiles has additive terms above the tile diagonal: all tiles then, and no causal
   // limit on the K of S V
