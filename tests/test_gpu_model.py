@@ -37,6 +37,17 @@ def assert_close(lhs, rhs, atol, rtol):
     assert not (np.abs(lhs - rhs) > atol + rtol * np.abs(rhs)).any(), f"max diff {np.abs(lhs - rhs).max()}"
 
 
+def _with_kernels(call):
+    """The call's result and the names of the kernels it ran, so that a test knows which one it looked at."""
+    from torch.profiler import ProfilerActivity, profile
+
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        result = call()
+        torch.cuda.synchronize()
+    return result, " ".join(e.key for e in prof.key_averages())
+
+
 def test_relu_lowrank_fused_matches_reference(bda):
     """tests/fused_kernel_tests.rs:35-68 on the device path: input [2,1,5,6], weight [1,3,6,8],
     bias [3,1,8], threshold 0.25, BlockPattern1d::from_blocks(3,[0,2]); atol = rtol = 1e-5."""
@@ -86,8 +97,8 @@ def test_relu_lowrank_single_row_small_matrix_bit_exact(bda, corc, d, N, h, h_in
                                       (4, 16, 1), (2, 100, 1), (3, 43, 4)])
 def test_relu_lowrank_bit_exact_against_oracle(bda, corc, B, T, h_in):
     """One k-sequential FMA chain per output on both sides: values, and therefore the active
-    sets, are identical bit for bit whatever the launch tiling -- also on the f32 matrix cores, which calls
-    of 8 to 64 rows take by default (a chain of v_mfma_f32_32x32x2_f32 over k is that same chain)."""
+    sets, are identical bit for bit whatever the launch tiling: the kernel for few outputs, the matrix cores (a chain of
+    v_mfma_f32_16x16x4_f32 or 32x32x2 over k is that same chain) and the thread-per-column kernel."""
     from burn_dragon_amd.kernel import relu_lowrank
 
     h, d, N = 4, 256, 640
@@ -101,19 +112,20 @@ def test_relu_lowrank_bit_exact_against_oracle(bda, corc, B, T, h_in):
     assert np.array_equal(got.cpu().numpy(), ref)
     assert 0.4 < (ref > 0).mean() < 0.6
     ctx = bda.ffi.default_context(0)
-    try:  # the matrix cores (8 to 64 rows; by default only for wide matrices), the scalar-input kernels (8 to 63
-        # rows) and the LDS-staged ones all give the same bits
-        ctx.set_option("relu_lowrank.mfma_rows", -8)
-        mfma = relu_lowrank.fused_forward(*args)
+    M = B * T
+    try:
+        ctx.set_option("relu_lowrank.row", 0)
+        mfma, ran = _with_kernels(lambda: relu_lowrank.fused_forward(*args))
+        assert any(k in ran for k in ("k_relu_lowrank_rows", "k_relu_lowrank_direct")) == (M > 1)
         ctx.set_option("relu_lowrank.mfma_rows", 0)
-        scalar = relu_lowrank.fused_forward(*args)
-        ctx.set_option("relu_lowrank.scalar", 0)
-        lds = relu_lowrank.fused_forward(*args)
+        ctx.set_option("relu_lowrank.gemm_rows", 0)
+        lds, ran = _with_kernels(lambda: relu_lowrank.fused_forward(*args))
+        assert not any(k in ran for k in ("k_relu_lowrank_rows", "k_relu_lowrank_direct", "k_relu_lowrank_row<"))
     finally:
-        ctx.set_option("relu_lowrank.scalar", 1)
-        ctx.set_option("relu_lowrank.mfma_rows", 8)
+        ctx.set_option("relu_lowrank.row", 1)
+        ctx.set_option("relu_lowrank.mfma_rows", 2)
+        ctx.set_option("relu_lowrank.gemm_rows", 64)
     assert np.array_equal(mfma.cpu().numpy(), ref)
-    assert np.array_equal(scalar.cpu().numpy(), ref)
     assert np.array_equal(lds.cpu().numpy(), ref)
     gated = relu_lowrank.fused_forward(*args, gate=torch.from_numpy(gate).to(DEV))
     assert np.array_equal(gated.cpu().numpy(), gate * ref)
@@ -139,13 +151,17 @@ def test_relu_lowrank_on_the_matrix_cores_with_every_option(bda, corc, M, d, N, 
     args = (torch.from_numpy(inp).to(DEV), torch.from_numpy(weight).to(DEV), torch.from_numpy(bias).to(DEV), 0.01, layout)
     ctx = bda.ffi.default_context(0)
     try:
-        ctx.set_option("relu_lowrank.mfma_rows", -8)  # whatever the width
-        got = relu_lowrank.fused_forward(*args).cpu().numpy()
+        ctx.set_option("relu_lowrank.row", 0)
+        got, ran = _with_kernels(lambda: relu_lowrank.fused_forward(*args).cpu().numpy())
+        assert "k_relu_lowrank_rows" in ran or "k_relu_lowrank_direct" in ran
         gated = relu_lowrank.fused_forward(*args, gate=torch.from_numpy(gate).to(DEV)).cpu().numpy()
         ctx.set_option("relu_lowrank.mfma_rows", 0)
+        ctx.set_option("relu_lowrank.gemm_rows", 0)
         valu = relu_lowrank.fused_forward(*args).cpu().numpy()
     finally:
-        ctx.set_option("relu_lowrank.mfma_rows", 8)
+        ctx.set_option("relu_lowrank.row", 1)
+        ctx.set_option("relu_lowrank.mfma_rows", 2)
+        ctx.set_option("relu_lowrank.gemm_rows", 64)
     assert np.array_equal(got, ref)
     assert np.array_equal(valu, ref)
     assert np.array_equal(gated, gate * ref)
@@ -154,12 +170,11 @@ def test_relu_lowrank_on_the_matrix_cores_with_every_option(bda, corc, M, d, N, 
 
 @pytest.mark.parametrize("B,T,h_in,d,N", [(2, 100, 1, 256, 640), (1, 300, 3, 72, 203), (3, 64, 1, 512, 1024),
                                           (4, 130, 1, 64, 8192)])
-def test_relu_lowrank_as_a_matrix_core_product_per_sequence(bda, corc, B, T, h_in, d, N):
-    """Many tokens per sequence: one f32 matrix-core product per (sequence, head) whose k order is that of a scalar
-    loop, so the outputs are again the bits of the oracle's fmaf chain -- with bias, threshold, block mask and gate,
-    ragged tiles in rows, columns and k (K = 72 is not a multiple of the 16-wide stage), wide value ranges.  The last
-    case (N a multiple of 256, 768 tiles of 128 x 256) takes the wide-tile instance that long prompts of a large
-    model run on."""
+def test_relu_lowrank_of_many_rows_as_a_matrix_core_product(bda, corc, B, T, h_in, d, N):
+    """Many rows: one f32 matrix-core product per head whose k order is that of a scalar loop, so the outputs are again
+    the bits of the oracle's fmaf chain -- with bias, threshold, block mask and gate, ragged tiles in rows, columns and
+    k (K = 72 is not a multiple of the 16-wide stage of the checked tiles), wide value ranges; the thread-per-column
+    kernel beside it."""
     from burn_dragon_amd.kernel import relu_lowrank
 
     h = 3
@@ -174,8 +189,8 @@ def test_relu_lowrank_as_a_matrix_core_product_per_sequence(bda, corc, B, T, h_i
     args = (torch.from_numpy(inp).to(DEV), torch.from_numpy(weight).to(DEV), torch.from_numpy(bias).to(DEV), 0.01, layout)
     ctx = bda.ffi.default_context(0)
     try:
-        ctx.set_option("relu_lowrank.gemm_rows", -64)  # whatever the grid
-        got = relu_lowrank.fused_forward(*args).cpu().numpy()
+        got, ran = _with_kernels(lambda: relu_lowrank.fused_forward(*args).cpu().numpy())
+        assert "k_relu_lowrank_direct" in ran or "k_relu_lowrank_rows" in ran or "k_relu_lowrank_gemm" in ran
         gated = relu_lowrank.fused_forward(*args, gate=torch.from_numpy(gate).to(DEV)).cpu().numpy()
         ctx.set_option("relu_lowrank.gemm_rows", 0)
         tile = relu_lowrank.fused_forward(*args).cpu().numpy()
@@ -188,8 +203,8 @@ def test_relu_lowrank_as_a_matrix_core_product_per_sequence(bda, corc, B, T, h_i
 
 
 def test_relu_lowrank_many_rows_with_bias_threshold_and_mask(bda, corc):
-    """The 64-row tile kernel (B*T >= 64) with every optional input, bit-exact against the oracle, and
-    identical to the 8-row kernel."""
+    """The checked matrix-core tiles (B*T >= 64, sizes without 16-byte pieces) with every optional input, bit-exact against
+    the oracle, and identical to the 8-row kernel."""
     from burn_dragon_amd.kernel import relu_lowrank
 
     B, T, h, d, N = 2, 70, 3, 36, 200  # ragged in rows, columns and k
@@ -202,16 +217,17 @@ def test_relu_lowrank_many_rows_with_bias_threshold_and_mask(bda, corc):
     args = (torch.from_numpy(inp).to(DEV), torch.from_numpy(weight).to(DEV), torch.from_numpy(bias).to(DEV), 0.05, layout)
     ctx = bda.ffi.default_context(0)
     try:
-        ctx.set_option("relu_lowrank.tile", 2)  # the default keeps the tile kernel for grids that cover the chip
-        got = relu_lowrank.fused_forward(*args).cpu().numpy()
-        ctx.set_option("relu_lowrank.tile", 0)
-        small = relu_lowrank.fused_forward(*args).cpu().numpy()
+        got, ran = _with_kernels(lambda: relu_lowrank.fused_forward(*args).cpu().numpy())
+        assert "k_relu_lowrank_gemm" in ran
+        ctx.set_option("relu_lowrank.gemm_rows", 0)
+        small, ran = _with_kernels(lambda: relu_lowrank.fused_forward(*args).cpu().numpy())
+        assert "k_relu_lowrank<" in ran
     finally:
-        ctx.set_option("relu_lowrank.tile", 1)
+        ctx.set_option("relu_lowrank.gemm_rows", 64)
     assert np.array_equal(got, ref)
     assert 0.05 < (ref > 0).mean() < 0.2
     assert np.array_equal(got, small)
-    # a shape whose tile grid covers the chip takes the tile kernel by default
+    # a wider one, of 16-byte pieces, by default
     big_w = (0.05 * rng.standard_normal((4, 64, 8192))).astype(np.float32)
     big_in = rng.standard_normal((2, 1, 128, 64)).astype(np.float32)
     big = relu_lowrank.fused_forward(torch.from_numpy(big_in).to(DEV), torch.from_numpy(big_w).to(DEV), None, 0.0,
@@ -281,7 +297,7 @@ def test_inference_paths_run_across_configs(bda, corc, rotary, fused):
 
 @pytest.mark.parametrize("rotary", ["rope", "pope"])
 def test_long_prompt_takes_the_dense_chunk_form(bda, corc, rotary):
-    """A prompt of 128+ tokens runs the state update as dense products on the f32 matrix cores; logits and
+    """A prompt of 150 tokens runs the state update as dense products on the matrix cores; logits and
     state agree with the oracle's token loop, and decoding continues from that state."""
     cfg = bda.BDHConfig(n_layer=2, n_embd=32, n_head=2, mlp_internal_dim_multiplier=8, vocab_size=64, dropout=0.0)
     cfg.fused_kernels.set_block_sizes(4, 4)
@@ -370,8 +386,8 @@ def test_forward_fast_with_sparse_block_patterns(bda, T):
 
 
 def test_batched_decode_step_takes_the_split_k_encoder(bda, corc):
-    """24+ sequences decoding together: the encoder E runs as a split-K product on the f32 matrix cores (the
-    weights are streamed once); logits against the oracle and against the VALU kernel."""
+    """24+ sequences decoding together: the encoder E runs on the f32 matrix cores, here forced into the form with one chain
+    per k-block of 1024; logits against the oracle and against the VALU kernel."""
     cfg = bda.BDHConfig(n_layer=2, n_embd=64, n_head=4, mlp_internal_dim_multiplier=64, vocab_size=64)  # N = 1024
     cfg.fused_kernels.set_rotary_embedding(bda.RotaryEmbedding.parse("rope"))
     shape, w, model = _model_pair(bda, cfg, seed=5)
