@@ -568,6 +568,103 @@ __global__ __launch_bounds__(256, 2) void k_gemm_tile(GemmArgs g) {
   }
 }
 
+// The state product of a fresh state: C[m,n] = sum_k A[k,m] B[n,k] in 256 x 256 tiles, 8 wavefronts (2 x 4) of 128 x 64
+// each.  A (Q, k-major) is staged through registers one step ahead and lies in LDS as in memory, [k][m], the 64-byte parts of
+// every other group of eight k rows swapped; fragments are read with the transposing LDS load.  Same sums as k_gemm_tile.
+// What bounds it: a tile's few steps (T / 64) and its 256 KiB of output, one workgroup per CU; the 128 wide tiles read every
+// piece of Q twice as often (32 slices, N = 9856, d = 512, 753 tokens: 404 against 524 us, 0.60 PFLOP/s).
+constexpr int KM_STRIDE = BM + 32;  // bf16 per k row in LDS: 576 bytes = 64 mod 256, so four k rows fall on different banks
+constexpr int LDS_STRIDE = BK + 8;  // bf16 per row of B in LDS: 144 bytes, conflict-free 16-byte reads
+
+__global__ __launch_bounds__(512) void k_gemm_state(GemmArgs g) {
+  __shared__ __attribute__((aligned(16))) unsigned short s_a[BK * KM_STRIDE];
+  __shared__ __attribute__((aligned(16))) unsigned short s_b[BN * LDS_STRIDE];
+  // each XCD takes an equal run of the (slice, tile) list, as in k_gemm_tile
+  const int total = g.n_slices * g.n_tiles, per = (total + 7) >> 3;
+  const int at = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per || at >= total) return;
+  const int slice = at / g.n_tiles, t = at - slice * g.n_tiles;
+  const int m0 = t / g.nt * BM, n0 = t % g.nt * BN;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = wave >> 2, wn = wave & 3;
+  const unsigned short *A = static_cast<const unsigned short *>(g.A) + (long)slice * g.a_batch;
+  const unsigned short *B = static_cast<const unsigned short *>(g.B) + (long)(slice / g.b_div) * g.b_batch;
+  const int K = g.K;
+
+  f32x16 acc[4][2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+
+  uint4 ra[4], rb[4];  // 4 pieces of 8 values per operand and thread
+  auto load = [&](int k0) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int piece = c * 512 + tid;
+      const int kr = piece >> 5, mc = (piece & 31) * 8;  // 32 pieces per k row of A
+      const int row = piece >> 3, kc = (piece & 7) * 8;  // 8 pieces per row of B
+      ra[c] = rb[c] = make_uint4(0u, 0u, 0u, 0u);
+      if (k0 + kr < K && m0 + mc < g.M) ra[c] = *reinterpret_cast<const uint4 *>(A + (long)(k0 + kr) * g.lda + m0 + mc);
+      if (n0 + row < g.N && k0 + kc < K) rb[c] = *reinterpret_cast<const uint4 *>(B + (long)(n0 + row) * g.ldb + k0 + kc);
+    }
+  };
+  load(0);
+  for (int k0 = 0; k0 < K; k0 += BK) {
+    __syncthreads();  // the previous step's fragment reads are done
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int piece = c * 512 + tid;
+      const int kr = piece >> 5, mc = (piece & 31) * 8;
+      *reinterpret_cast<uint4 *>(s_a + kr * KM_STRIDE + (mc ^ (((kr >> 3) & 1) << 5))) = ra[c];
+      *reinterpret_cast<uint4 *>(s_b + (piece >> 3) * LDS_STRIDE + (piece & 7) * 8) = rb[c];
+    }
+    __syncthreads();
+    if (k0 + BK < K) load(k0 + BK);  // on its way while the matrix cores work on this step
+#pragma unroll
+    for (int kk = 0; kk < BK; kk += 16) {
+      bf16x8 fa[4], fb[2];
+      const int kof = kk + (lane >> 5) * 8;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        // as in k_gemm_tile; rows kof .. kof + 7 share bit 3 = lane / 32: one swap
+        const int j16 = lane & 15;
+        const int m = (wm * 128 + i * 32 + ((lane >> 4) & 1) * 16) ^ ((lane >> 5) << 5);
+        const unsigned short *src = s_a + (kof + (j16 >> 2)) * KM_STRIDE + m + (j16 & 3) * 4;
+        typedef short s16x4 __attribute__((ext_vector_type(4)));
+        typedef short s16x8 __attribute__((ext_vector_type(8)));
+        typedef __attribute__((address_space(3))) s16x4 *lds_s16x4_t;
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)(src));
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)(src + 4 * KM_STRIDE));
+        const s16x8 pk = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        fa[i] = __builtin_bit_cast(bf16x8, pk);
+      }
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        fb[j] = *reinterpret_cast<const bf16x8 *>(s_b + (wn * 64 + j * 32 + (lane & 31)) * LDS_STRIDE + kof);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
+    }
+  }
+  float *C = static_cast<float *>(g.C) + (long)slice * g.c_batch;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int col = n0 + wn * 64 + j * 32 + (lane & 31);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int row = m0 + wm * 128 + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
+        if (row < g.M && col < g.N) C[(long)row * g.ldc + col] = acc[i][j][e];
+      }
+    }
+}
+
 // ------------------------------------------------------------------------------------
 // 256x256 tiles, K a multiple of 64 (or both operands zero-padded to it), both operands k-contiguous: the tiles go from global memory straight into LDS (global_load_lds_dwordx4, no
 // VGPR staging, no ds_write), double buffered.  LDS tile layout: blocks of 8 rows x 128 bytes
@@ -1375,7 +1472,15 @@ static int prefill_pass_scores(bdh_ctx *ctx, int B, int h, int T, int N, int d, 
   const bool big = d % 256 == 0 && Nq % BK == 0 && S * tiles(T, 256) * (d / 256) >= full_chip &&
                    (tiles(T, 256) * 256 - T) * 8 <= T;
   const int tile_t = big ? 256 : S * tiles(T, 128) * tiles(d, 128) >= full_chip ? 128 : 64;
-  const int tile_r = S * tiles(Nq, 128) * tiles(d, 128) >= full_chip ? 128 : 64;
+  // The state product of a fresh state is bound by what a tile reads and by its latency: 256 wide from a workgroup for every CU
+  // on, unless the last round would be mostly empty (us a call, 256 | 128: 32 slices, N = 9856, d = 512, 200 tokens 403 | 474;
+  // 64 slices, N = 9856, d = 384, 200 tokens 663 | 733; 16 slices, N = 4096, d = 256, 753 tokens 184 | 190; 4 slices of 9856
+  // and d = 384, 1.2 rounds, 144 | 104; ALiBi 32 slices, N = 4096, d = 512, 753 tokens 373 | 425).  A carried one is read and
+  // scaled as well: more, smaller workgroups then (32 slices, N = 9856, d = 512, 753 tokens 2130 | 1705).
+  const long tiles_r = S * tiles(Nq, 256) * tiles(d, 256), rounds_r = (tiles_r + full_chip - 1) / full_chip;
+  const bool wide_r = state_is_zero && d > 128 && tiles_r >= full_chip &&
+                      (tiles_r >= 2 * full_chip || 4 * rounds_r * full_chip <= 5 * tiles_r);
+  const int tile_r = wide_r ? 256 : S * tiles(Nq, 128) * tiles(d, 128) >= full_chip ? 128 : 64;
   // The scores, of which there are more tiles, may have the larger one: 12 slices of 777 tokens, whose 168 output tiles
   // are 64 wide, 248 us a call with scores of 64, 238 with 128 (336 tiles).
   auto lower = [&](int tile) { return S * tiles(T, tile) * (tiles(T, tile) + 1) / 2; };
@@ -1513,7 +1618,14 @@ static int prefill_pass_scores(bdh_ctx *ctx, int B, int h, int T, int N, int d, 
     g.M = Nq; g.N = d; g.K = T; g.b_div = pm.decay ? 1 : h; g.beta = state_is_zero ? 0 : 1; g.causal_k = 0;
     g.tri = 0; g.n_slices = S;
     if (pm.decay) with_mode(g, GM_DECAY_STATE);
-    launch_gemm_tile<true, false>(ctx->stream, g, tile_r);
+    if (tile_r == 256) {
+      g.nt = (int)tiles(d, 256);
+      g.n_tiles = (int)tiles(Nq, 256) * g.nt;
+      const dim3 grid(8u * (unsigned)(((long)S * g.n_tiles + 7) / 8));
+      hipLaunchKernelGGL(k_gemm_state, grid, dim3(512), 0, ctx->stream, g);
+    } else {
+      launch_gemm_tile<true, false>(ctx->stream, g, tile_r);
+    }
     BDH_LAUNCH_CHECK(ctx, "Q^T V");
   }
   return BDH_OK;

@@ -477,3 +477,25 @@ def test_row_normalised_alibi_with_time_blocks_wider_than_the_output_tiles(bda, 
     out = prefill_chunked_ex(x.to(DEV), v.to(DEV), None, torch.from_numpy(freqs).to(DEV), 0, rotary=bda.RotaryEmbedding.ALIBI,
                              alibi_slopes=slopes, row_normalize=True, block_size=bs)
     assert rel_err(out.cpu().numpy(), ref) < TOL
+
+
+@pytest.mark.parametrize("B,h,T,N,d", [(16, 8, 70, 264, 136), (16, 8, 129, 200, 264), (32, 8, 9, 256, 256), (16, 8, 64, 512, 256)])
+@pytest.mark.parametrize("rotary", ["rope", "pope", "alibi"])
+def test_wide_state_product_of_a_fresh_state(bda, B, h, T, N, d, rotary):
+    """Fresh states large enough for 256 wide tiles of the state product (edges of tiles, tokens that end inside a step of 64):
+    the state is bit for bit what a carried state of zeros, which takes smaller tiles, becomes."""
+    from burn_dragon_amd.kernel.linear_attention import build_freqs
+    from burn_dragon_amd.recurrent import prefill_chunked_ex
+
+    R = bda.RotaryEmbedding.parse(rotary)
+    g = torch.Generator(device="cuda:0").manual_seed(T)
+    x = torch.relu(torch.randn((B, h, T, N), device="cuda:0", generator=g)).to(torch.bfloat16)
+    v = torch.randn((B, T, d), device="cuda:0", generator=g).to(torch.bfloat16)
+    freqs = build_freqs(N, 65536.0, R, device="cuda:0")
+    rows = 2 * N if rotary == "pope" else N
+    fresh = torch.full((B, h, rows, d), 7.0, device="cuda:0")
+    carried = torch.zeros((B, h, rows, d), device="cuda:0")
+    out_f = prefill_chunked_ex(x, v, fresh, freqs, 3, rotary=R, state_is_zero=True, all_scores=True)
+    out_c = prefill_chunked_ex(x, v, carried, freqs, 3, rotary=R, state_is_zero=False, all_scores=True)
+    assert torch.equal(fresh, carried) and torch.equal(out_f, out_c)
+    assert float(fresh.abs().max()) > 0

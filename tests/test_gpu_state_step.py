@@ -342,7 +342,7 @@ def test_lazy_alibi_decay_matches_the_eager_reference_semantics(gpu, corc, dtype
 
 @pytest.fixture
 def dense_chunks(gpu):
-    """Forces the many-token dense form (f32 matrix cores) for the duration of a test."""
+    """Forces the many-token dense form for the duration of a test."""
     ffi, _ = gpu
     ctx = ffi.default_context(0)
     ctx.set_option("state_step.dense_chunks", 1)
@@ -417,8 +417,8 @@ def test_dense_chunk_form_split_products_keep_f32_accuracy(gpu, corc, dense_chun
 
 def test_dense_chunk_form_equals_step_kernels_and_handles_device_positions(gpu, corc):
     """The same call through the sparse step kernels and through the dense form; per-sequence device
-    positions; T = 128 takes the dense form by default once the products have enough tiles to cover the
-    chip (B*h = 96 slices here; with a handful of slices the multi-token f32 RoPE kernel is kept)."""
+    positions; T = 128 takes the dense form by default (B*h = 96 slices here), but an f32 RoPE state of at most 512 KiB
+    is always walked: there a call of any number of tokens leaves the bits of single-token calls."""
     ffi, recurrent_attention = gpu
     ctx = ffi.default_context(0)
     B, h, T, N, d = 24, 4, 128, 128, 256
@@ -433,7 +433,7 @@ def test_dense_chunk_form_equals_step_kernels_and_handles_device_positions(gpu, 
     out_d, rho_d = _run_plain(recurrent_attention, x, v, rho, freqs, 0, orc.ROPE, positions)
     assert rel_err(out_d, out_s) < 2e-5 and rel_err(rho_d, rho_s) < 2e-5
     assert not np.array_equal(out_d, out_s)  # different summation order: the dense form did run
-    # a handful of slices at the same shape: the default keeps the token loop (identical bits)
+    # 512 KiB of state: the default keeps the token loop (identical bits)
     try:
         ctx.set_option("state_step.dense_chunks", 0)
         out_few_loop, _ = _run_plain(recurrent_attention, x[:1], v[:1], rho[:1], freqs, 5, orc.ROPE)
