@@ -409,7 +409,7 @@ def test_dense_chunk_form_split_products_keep_f32_accuracy(gpu, corc, dense_chun
     def rms_err(a, b):
         return float(np.sqrt(np.mean((a.astype(np.float64) - b) ** 2)) / np.sqrt(np.mean(b ** 2)))
 
-    # measured: 2.35e-7 and 2.42e-7 (the f32 matrix instructions: 2.74e-7 and 2.53e-7)
+    # measured: 1.40e-7 and 1.10e-7 (the f32 matrix instructions: 2.74e-7 and 2.53e-7)
     assert rms_err(out, out_ref) < 6e-7, rms_err(out, out_ref)
     assert rms_err(rho_new, rho_ref) < 6e-7, rms_err(rho_new, rho_ref)
     assert rel_err(out, out_ref) < 2e-6 and rel_err(rho_new, rho_ref) < 2e-6
