@@ -57,13 +57,17 @@ struct bdh_model {
   // activation scratch, grown on demand to the largest (B,T) seen
   void *act = nullptr;
   size_t act_bytes = 0;
+  // scratch of the two-launch layer of a model that fits the one-launch step, at most 4 MiB of projection weights; sized at creation for every batch that
+  // form is taken for: a decode step of such a model never allocates, and a captured one keeps its buffer whatever runs later
+  float *phase_act = nullptr;
 };
 
 int bdh_fail(bdh_ctx *ctx, int status, const char *fmt, ...);
 
 // model_phase.hip: a decode step in two launches per layer (T = 1, f32 state, 128 <= d <= 512, N a multiple of 64)
-bool bdh_model_phase_fits(const bdh_model_config &c);
-size_t bdh_model_phase_scratch_floats(const bdh_model_config &c, int B);
+bool bdh_model_phase_fits(const bdh_model *m);
+int bdh_model_phase_most(const bdh_model *m, int rho_dtype, bool lazy);  // sequences
+size_t bdh_model_phase_scratch_floats(const bdh_model *m, int B);
 int bdh_launch_model_phases(bdh_model *m, const int64_t *tokens, int B, float *scratch, void *rho, int rho_dtype, int32_t *stamps,
                             int64_t position,
                             const int32_t *positions_dev, float **cur_final, float **dec_partial, int *G_out);

@@ -1,5 +1,6 @@
 // The whole cached step, BDH::forward_with_state (src/model/bdh.rs:309-450), as a
 // stream-ordered sequence of the kernels of this library.
+#include <algorithm>
 #include <new>
 #include <vector>
 
@@ -7,6 +8,11 @@
 #include <utility>
 
 namespace {
+
+// a model that fits the one-launch step, with at most 4 MiB of projection weights
+bool has_phase_act(const bdh_model_config &c) {
+  return bdh_model_small_fits(c) && sizeof(float) * (size_t)3 * c.n_head * c.latent * c.n_embd * c.n_layer <= (size_t(4) << 20);
+}
 
 int ensure_act(bdh_model *m, size_t bytes) {
   if (bytes <= m->act_bytes) return BDH_OK;
@@ -102,6 +108,15 @@ int bdh_model_create(bdh_ctx *ctx, const bdh_model_config *c, const bdh_model_we
     delete m;
     return bdh_fail(ctx, BDH_E_HIP, "freqs table upload: %s", hipGetErrorString(e));
   }
+  if (has_phase_act(*c) && bdh_model_phase_fits(m)) {
+    size_t most = 0;
+    for (int B = bdh_model_phase_most(m, BDH_F32, false); B > 0; --B)  // whatever the state's type: at most 1365
+      most = std::max(most, bdh_model_phase_scratch_floats(m, B));
+    if (hipMalloc(reinterpret_cast<void **>(&m->phase_act), sizeof(float) * most) != hipSuccess) {
+      (void)hipGetLastError();
+      m->phase_act = nullptr;  // such a model takes the one-launch step
+    }
+  }
   *out = m;
   return BDH_OK;
 }
@@ -111,6 +126,7 @@ int bdh_model_destroy(bdh_model *m) {
   if (m->ctx) (void)hipStreamSynchronize(m->ctx->stream);
   if (m->freqs) (void)hipFree(m->freqs);
   if (m->act) (void)hipFree(m->act);
+  if (m->phase_act) (void)hipFree(m->phase_act);
   delete m;
   return BDH_OK;
 }
@@ -207,30 +223,28 @@ int model_forward_impl(bdh_model *m, const int64_t *tokens, int B, int T, StateR
   void *rho = st.rho(0);
   int32_t *stamps = st.stamps(0);
 
-  // A decode step (one token per sequence, f32 state, no by-products) need not run kernel by kernel:
-  //  * a small model (d <= 256, h*N <= 2048) can run the whole step in ONE launch, a workgroup per sequence; one CU then
-  //    streams all the projection weights of the step, W bytes;
+  // A decode step (one token per sequence, no by-products) need not run kernel by kernel:
   //  * a mid-size model (128 <= d <= 512, up to 64 blocks of 64 neurons) can run TWO launches per layer, a workgroup
-  //    per block; every workgroup streams its share of the layer's weights once per sequence.
-  // Measured at the sizes of the reference's configurations (W = 3 / 6.75 / 12 / 96 MiB; us per step, one launch | two
-  // per layer | kernel by kernel): tiny 77|77|112 at B=1, 84|100|145 at B=64; small 152|82|130 at B=1, 168|127|195 at
-  // B=64, 323|442|478 at B=256; base 223|83|123 at B=1, 273|210|240 at B=64, 559|-|654 at B=256; large -|210|308 at
-  // B=1, -|519|554 at B=16, -|1092|981 at B=33.
+  //    per block; every workgroup streams its share of the layer's weights once per sequence (bdh_model_phase_most);
+  //  * a small model (d <= 256, h*N <= 2048) can run the whole step in ONE launch, a workgroup per sequence; one CU then
+  //    streams all the projection weights of the step, W bytes.
+  // us per step, one launch | two per layer | kernel by kernel: W = 3 MiB 76|39|112 at B=1, 77|42|- at B=16, 79|57|145 at
+  // B=64, 90|94|- at B=192; 6.75 MiB 129|55|130 at B=1, 143|116|195 at B=64, 165|196|- at B=128; 12 MiB 189|46|123 at B=1,
+  // 205|129|188 at B=64; 96 MiB -|114|308 at B=1, -|309|470 at B=16, -|576|607 at B=32.
   if (T == 1 && !x_tap && !viz && !logs && contiguous && ctx->opt_model_one_launch != 0) {
-    const size_t w_layer = sizeof(float) * (size_t)3 * h * N * d;
-    const size_t w_bytes = w_layer * L;
+    const size_t w_bytes = sizeof(float) * (size_t)3 * h * N * d * L;
     const bool small_fits = bdh_model_small_fits(c);
-    const bool forced = ctx->opt_model_one_launch == 2;
-    const bool one_first = small_fits && (forced || w_bytes <= (size_t(4) << 20));
-    const bool phases = !one_first && bdh_model_phase_fits(c) && B <= ctx->opt_model_phase_batch &&
-                        (size_t)B * w_layer <= (size_t(256) << 20);
-    const int b_min = w_bytes <= (size_t(8) << 20) ? 16 : 128;
-    if (one_first || (!phases && small_fits && B >= b_min))
+    const bool small = has_phase_act(c);
+    const bool forced = ctx->opt_model_one_launch == 2 && small_fits;
+    const bool phases = !forced && bdh_model_phase_fits(m) && B <= ctx->opt_model_phase_batch &&
+                        B <= bdh_model_phase_most(m, rho_dtype, stamps != nullptr) && (!small || m->phase_act);
+    const int b_min = small ? 1 : w_bytes <= (size_t(8) << 20) ? 16 : 128;
+    if (forced || (!phases && small_fits && B >= b_min))
       return bdh_launch_model_small(m, tokens, B, rho, rho_dtype, stamps, position, positions_dev, logits, next_tokens);
     if (phases) {
-      int rc2 = ensure_act(m, sizeof(float) * bdh_model_phase_scratch_floats(c, B));
+      int rc2 = small ? BDH_OK : ensure_act(m, sizeof(float) * bdh_model_phase_scratch_floats(m, B));
       if (rc2 != BDH_OK) return rc2;
-      float *scratch = static_cast<float *>(m->act);
+      float *scratch = small ? m->phase_act : static_cast<float *>(m->act);
       float *cur_final = nullptr, *dpart = nullptr;
       int G = 0;
       rc2 = bdh_launch_model_phases(m, tokens, B, scratch, rho, rho_dtype, stamps, position, positions_dev, &cur_final,

@@ -8,9 +8,17 @@
 //            rows (readout, update, decay), the readout partial of the workgroup;
 //   phase B: LN(sum of the head's readout partials), D_y and the gate for its 64 neurons, the encoder partial of
 //            those 64 rows of E.
-// The sums over partials are redone by every workgroup that needs them (a few KiB from the L2).  Projections
-// keep the k-sequential fmaf chain of k_relu_lowrank; the other sums are taken in a fixed tree of their own
-// (results agree with the kernel-by-kernel step to rounding, not bit for bit).
+// The sums over partials are redone by every workgroup that needs them (a few KiB from the L2).  All sums are taken in a
+// fixed tree of their own (results agree with the kernel-by-kernel step to rounding, not bit for bit).
+//
+// What bounds it: latency.  Both phases ask for everything whose address does not depend on a result -- the partials, the
+// weights, the state rows or the rows of E -- in the order in which it is needed, before they wait for any of it: one trip
+// to memory per launch where one after the other takes three.  Weights come 16 bytes a lane, sixteen lanes per row of k,
+// so a lane's part of a column's sum has d / (4 waves) terms and the parts meet over lanes and in LDS once; a chain over
+// all of k, handed from wave to wave, took 2.0 us of phase A at d = 256 and 3.2 at 512.  Every wave redoes the LayerNorms
+// on its own copy of the row: no barriers between their sums.  First start to last end of a launch, one sequence, d = 256,
+// 1024 neurons: phase A 9.2 -> 4.3 us, phase B 5.7 -> 2.5; d = 512, 2048 neurons: 12.5 -> 6.6, 7.7 -> 3.5.  The 1.5 us from the
+// end of one launch to the start of the next remain.
 #include "bdh_internal.h"
 
 namespace {
@@ -22,9 +30,9 @@ struct PhaseArgs {
   const int64_t *tokens;      // first layer only: [B] tokens, the layer's input is LN(embed[token]) (else null)
   const float *embed;         // [V][d]
   int V;
-  const float *cur_in;        // [B][d] the layer's input (before the pending encoder second stage, if any)
-  float *cur_out;             // [B][d] written by the first workgroup of a sequence when it computed the input itself
-  const float *dec_partial;   // [G][B][d] encoder partials of the previous layer, or null
+  const float *cur_in;        // [B][d] the layer's input before the pending encoder second stage (not the first layer)
+  float *cur_out;             // [B][d] the layer's input, written by the first workgroup of a sequence
+  const float *dec_partial;   // [G][B][d] encoder partials of the previous layer (not the first layer)
   float *x;                   // [B][h*N]
   float *attn_partial;        // [B][h][N/64][d]
   float *dec_partial_out;     // [G][B][d], G = h * N / 64
@@ -38,182 +46,346 @@ struct PhaseArgs {
   float decay[64], log_decay[64];
 };
 
+// The wave of the workgroup, in a scalar register: addresses that only depend on it cost the lanes nothing.
+__device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
+// p[at / 4]: one base for the wave, a 32-bit byte offset per lane
+template <typename V, typename T>
+__device__ __forceinline__ V load_at(const T *p, unsigned int at) {
+  return *reinterpret_cast<const V *>(reinterpret_cast<const char *>(p) + at);
+}
+
+// Orders a wave's own LDS writes and reads of other lanes' values for the compiler (the hardware runs them in order).
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// All lanes get the sum over the lanes l, l ^ 16, l ^ 32, l ^ 48.
+__device__ __forceinline__ float sum_over_rows(float v) {
+  const unsigned int u = __float_as_uint(v);
+  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  const unsigned int w = __float_as_uint(v);
+  const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+// All lanes get the wave's sum: lanes 1 and 2 apart, the mirrored half row and row, then the four rows.
 __device__ __forceinline__ float wave_sum(float v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
+  v += dpp<0xb1>(v);
+  v += dpp<0x4e>(v);
+  v += dpp<0x141>(v);
+  v += dpp<0x140>(v);
+  return sum_over_rows(v);
 }
 
-// LayerNorm statistics of d <= 64 * NW values held one per thread by threads 0..d-1; every thread calls it.
-template <int NW>
-__device__ __forceinline__ void block_ln_stats(float v, bool has, int d, float *s_st, float &mean, float &den) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  __syncthreads();  // s_st may still be read from an earlier use
-  const float s = wave_sum(has ? v : 0.0f);
-  if (lane == 0) s_st[wave] = s;
-  __syncthreads();
-  float t = s_st[0];
-#pragma unroll
-  for (int w = 1; w < NW; ++w) t += s_st[w];
-  mean = t / (float)d;
-  const float c = has ? v - mean : 0.0f;
-  const float q = wave_sum(c * c);
-  if (lane == 0) s_st[NW + wave] = q;
-  __syncthreads();
-  float u = s_st[NW];
-#pragma unroll
-  for (int w = 1; w < NW; ++w) u += s_st[NW + w];
-  den = sqrtf(u / (float)d + kLnEps);
+// v / den for many v and one den, r = 1 / den rounded: one correction of v * r by its remainder gives the rounded quotient
+// (P. Markstein, IBM J. Res. Dev. 34, 1990) in three operations instead of the ten of a division.
+__device__ __forceinline__ float quotient(float v, float den, float r) {
+  const float q = v * r;
+  return __builtin_fmaf(__builtin_fmaf(-q, den, v), r, q);
 }
 
-// The 64 weights of this wave's span of k for column n, asked for at once (rows past d are clamped to the last
-// one and weighted zero: loads under a branch would not be issued back to back).
-__device__ __forceinline__ void load_span(const float *__restrict__ w, int hh, int d, int N, int n, int k_lo, float *wv) {
-  const float *wp = w + (long)hh * d * N + n;
+// LayerNorm of a row held by one wave, column j * 64 + lane in v[j] (src/model/bdh.rs:86-89); zero beyond d.
+template <int CJ>
+__device__ __forceinline__ void wave_layer_norm(float (&v)[CJ], int d) {
+  const int lane = threadIdx.x & 63;
+  const float fd = (float)d, rd = 1.0f / fd;
+  float s = 0.0f;
 #pragma unroll
-  for (int u = 0; u < 64; ++u) {
-    const float t = wp[(long)min(k_lo + u, d - 1) * N];
-    wv[u] = k_lo + u < d ? t : 0.0f;
+  for (int j = 0; j < CJ; ++j) s += j * 64 + lane < d ? v[j] : 0.0f;
+  const float mean = quotient(wave_sum(s), fd, rd);
+  float q = 0.0f;
+#pragma unroll
+  for (int j = 0; j < CJ; ++j) {
+    const float c = j * 64 + lane < d ? v[j] - mean : 0.0f;
+    v[j] = c;
+    q += c * c;
   }
+  const float den = sqrtf(quotient(wave_sum(q), fd, rd) + kLnEps), r = 1.0f / den;
+#pragma unroll
+  for (int j = 0; j < CJ; ++j) v[j] = quotient(v[j], den, r);
 }
 
-// The column's fmaf chain, extended span by span in k order; the accumulator travels through LDS.  s_in holds
-// the input row, zero beyond d.  Returns the full sum in the last wave.
-template <int NW>
-__device__ __forceinline__ float chain_spans(const float *s_in, const float *wv, float *s_acc) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int k_lo = wave * 64;
-  float acc = 0.0f;
+// How the NW waves of a workgroup share rows of d <= DC floats and the NB neurons of its block.
+template <int DC, int NW, int NB>
+struct Shape {
+  static constexpr int NT = NW * 64;
+  static constexpr int CJ = DC / 64;            // columns per lane where every wave holds the whole row
+  static constexpr int RG = NT * 4 / DC;        // rows of partial sums that one 16-byte access of the workgroup covers
+  static constexpr int PG = 64 / RG;            // ... and how many accesses 64 of them take
+  static constexpr int LPW = NB / 4;            // lanes per row of a weight block, 16 bytes each
+  static constexpr int KR = DC / NW / (64 / LPW);  // rows of a weight block per lane
+  static constexpr int LPR = DC < 256 ? 32 : 64;  // lanes per state row (or row of E), 16 or 8 bytes each
+  static constexpr int VPL = DC / (4 * LPR);    // pieces of a row per lane
+  static constexpr int RPI = 64 / LPR;          // rows per access of a wave
+  static constexpr int RU = NB / NW / RPI;      // accesses for a wave's share of NB rows
+};
+
+// The sum of `rows` <= 64 rows of d floats, the next one `stride` floats on: asked for by ask(), column j * 64 + lane of the
+// sum in v[j] of every wave by collect(), which holds a barrier.
+template <int DC, int NW>
+struct RowSum {
+  using S = Shape<DC, NW, 64>;
+  float4 t[S::PG];
+  __device__ __forceinline__ void ask(const float *__restrict__ src, long stride, int rows, int d) {
+    const int rg = threadIdx.x / (DC / 4), c = threadIdx.x % (DC / 4) * 4;
+    const unsigned int at = (c < d ? c : 0) * 4u, step = (unsigned int)stride * 4u;
 #pragma unroll
-  for (int stage = 0; stage < NW; ++stage) {
-    if (wave == stage) {
-      if (stage > 0) acc = s_acc[lane];
-#pragma unroll
-      for (int u = 0; u < 64; ++u) acc = __builtin_fmaf(s_in[k_lo + u], wv[u], acc);
-      if (stage < NW - 1) s_acc[lane] = acc;
+    for (int i = 0; i < S::PG; ++i) {
+      t[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (i == 0 || i * S::RG < rows)  // uniform
+        t[i] = load_at<float4>(src, at + min(i * S::RG + rg, rows - 1) * step);
     }
-    if (stage < NW - 1) __syncthreads();
   }
-  return acc;
+  __device__ __forceinline__ void collect(int rows, float4 *s_part, float (&v)[S::CJ]) {
+    const int rg = threadIdx.x / (DC / 4);
+    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int i = 0; i < S::PG; ++i) {
+      const bool in = i * S::RG + rg < rows;
+      s.x += in ? t[i].x : 0.0f;
+      s.y += in ? t[i].y : 0.0f;
+      s.z += in ? t[i].z : 0.0f;
+      s.w += in ? t[i].w : 0.0f;
+    }
+    s_part[threadIdx.x] = s;  // [RG][DC]
+    __syncthreads();
+    const float *f = reinterpret_cast<const float *>(s_part) + (threadIdx.x & 63);
+#pragma unroll
+    for (int j = 0; j < S::CJ; ++j) {
+      v[j] = f[j * 64];
+#pragma unroll
+      for (int r = 1; r < S::RG; ++r) v[j] += f[r * DC + j * 64];
+    }
+  }
+};
+
+// row . w for NB columns of a weight matrix [d][N] (`weight` points at the first of them): ask() requests this wave's
+// DC / NW rows of k, dot() returns the sum of column lane % NB in every wave (it holds a barrier).  s_row: the wave's own
+// copy of the input row, zero beyond d.
+template <int DC, int NW, int NB>
+struct Project {
+  using S = Shape<DC, NW, NB>;
+  float4 w[S::KR];
+  static __device__ __forceinline__ int first_k() { return wave_id() * (DC / NW) + (int)(threadIdx.x & 63) / S::LPW * S::KR; }
+  __device__ __forceinline__ void ask(const float *__restrict__ weight, int d, int N) {
+    const int k0 = first_k();
+    unsigned int at = (min(k0, d - 1) * N + (threadIdx.x & (S::LPW - 1)) * 4) * 4u;
+#pragma unroll
+    for (int u = 0; u < S::KR; ++u) {
+      w[u] = load_at<float4>(weight, at);
+      at += k0 + u < d - 1 ? N * 4u : 0u;  // not beyond the last row
+    }
+  }
+  __device__ __forceinline__ float dot(const float *s_row, int d, float (*s_acc)[NB]) {
+    const int lane = threadIdx.x & 63, k0 = first_k();
+    if (d < DC) {  // what was asked for beyond the last row of k does not count
+#pragma unroll
+      for (int u = 0; u < S::KR; ++u)
+        if (k0 + u >= d) w[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    float r[S::KR];
+#pragma unroll
+    for (int u = 0; u < S::KR; ++u) r[u] = s_row[k0 + u];
+    float p[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < S::KR; ++u) {
+      p[0] = __builtin_fmaf(r[u], w[u].x, p[0]);
+      p[1] = __builtin_fmaf(r[u], w[u].y, p[1]);
+      p[2] = __builtin_fmaf(r[u], w[u].z, p[2]);
+      p[3] = __builtin_fmaf(r[u], w[u].w, p[3]);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {  // over the lanes with the same columns: LPW apart
+      if (S::LPW <= 4) p[e] += dpp<0x124>(p[e]);  // rotations of a row of sixteen by four and eight
+      if (S::LPW <= 8) p[e] += dpp<0x128>(p[e]);
+      p[e] = sum_over_rows(p[e]);
+    }
+    if (lane < S::LPW) *reinterpret_cast<float4 *>(&s_acc[wave_id()][lane * 4]) = make_float4(p[0], p[1], p[2], p[3]);
+    __syncthreads();
+    const int c = lane & (NB - 1);
+    float s = s_acc[0][c];
+#pragma unroll
+    for (int w2 = 1; w2 < NW; ++w2) s += s_acc[w2][c];
+    return s;
+  }
+};
+
+// out[0..d) = the sum over the workgroup of the lanes' pieces of a row (Shape::VPL each; lanes of one wave that hold the
+// same columns are added first).  Holds a barrier.
+template <int DC, int NW>
+__device__ __forceinline__ void write_row_sum(const float4 (&acc)[Shape<DC, NW, 64>::VPL], float (*s_red)[DC], int d,
+                                              float *__restrict__ out) {
+  using S = Shape<DC, NW, 64>;
+  const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
+#pragma unroll
+  for (int j = 0; j < S::VPL; ++j) {
+    float4 t = acc[j];
+    if (S::RPI == 2) {
+      t.x += __shfl_xor(t.x, 32);
+      t.y += __shfl_xor(t.y, 32);
+      t.z += __shfl_xor(t.z, 32);
+      t.w += __shfl_xor(t.w, 32);
+    }
+    if (S::RPI == 1 || lane < S::LPR) *reinterpret_cast<float4 *>(&s_red[wave][(j * S::LPR + lane) * 4]) = t;
+  }
+  __syncthreads();
+  for (int c = tid; c < d; c += S::NT) {
+    float s = s_red[0][c];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) s += s_red[w][c];
+    out[c] = s;
+  }
+}
+
+// A load through the scalar cache (the address is the same for the whole wave and nothing in this launch writes it).
+template <typename T>
+__device__ __forceinline__ T scalar_load(const T *p) {
+  return *reinterpret_cast<const __attribute__((address_space(4))) T *>(reinterpret_cast<uintptr_t>(p));
+}
+
+// Four state elements as they are stored.
+__device__ __forceinline__ float4 load_raw(const float *p) { return *reinterpret_cast<const float4 *>(p); }
+__device__ __forceinline__ uint2 load_raw(const unsigned short *p) { return *reinterpret_cast<const uint2 *>(p); }
+__device__ __forceinline__ float4 widen(float4 v) { return v; }
+__device__ __forceinline__ float4 widen(uint2 v) {
+  return make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),
+                     __uint_as_float(v.y & 0xffff0000u));
 }
 
 // ---- phase A ---------------------------------------------------------------------------------------------------
-template <int NW, typename RhoT>
-__global__ __launch_bounds__(NW * 64) void k_layer_phase_a(PhaseArgs a) {
-  constexpr int VPL = (NW + 3) / 4;  // float4 per lane per state row: columns (j*64 + lane)*4
-  constexpr int kFlight = 64 / NW < 16 ? 64 / NW : 16;  // state rows in flight per wave: all of its share of a dense block
-  __shared__ __align__(16) float s_cur[NW * 64];
-  __shared__ float s_x[64];
-  __shared__ float s_acc[64];
-  __shared__ float s_st[2 * NW];
-  __shared__ unsigned char s_list[NW][64];
-  __shared__ float4 s_red[NW][VPL * 64];
+// AHEAD: all NB state rows are asked for before it is known which of them are visited (the launcher says when); otherwise
+// the visited ones once they are.
+// FIRST: the first layer, whose input is the LayerNorm of the embedding row.
+template <int DC, int NW, int NB, typename RhoT, bool AHEAD, bool FIRST>
+__global__ __launch_bounds__(NW * 64, AHEAD || DC == 512 ? 2 : 4) void k_layer_phase_a(PhaseArgs a) {
+  using S = Shape<DC, NW, NB>;
+  typedef decltype(load_raw((const RhoT *)nullptr)) Raw;
+  __shared__ float4 s_part[S::NT];
+  __shared__ __align__(16) float s_cur[NW][DC];  // every wave's own copy of the layer's input, zero beyond d
+  __shared__ __align__(16) float s_acc[NW][NB];
+  __shared__ unsigned char s_list[NW][NB];
+  __shared__ __align__(16) float s_red[NW][DC];
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int lane = threadIdx.x & 63, wave = wave_id();
+  const int nblk = blockIdx.x, hh = blockIdx.y, b = blockIdx.z;
   const int d = a.d, h = a.h, N = a.N;
-  const int nblk_n = N >> 6;
-  const int nblk = blockIdx.x % nblk_n;
-  const int hh = (blockIdx.x / nblk_n) % h;
-  const int b = blockIdx.x / (nblk_n * h);
-  const int n = nblk * 64 + lane;  // this lane's neuron of the head
-  const long pos = a.pos_dev ? (long)a.pos_dev[b] : a.pos;
-  const float posf = (float)pos;
-
-  // weights of D_x first: they do not depend on anything computed here
-  float wv[64];
-  load_span(a.enc, hh, d, N, n, wave * 64, wv);
-
-  // the layer's input: cur, after the pending second stage of the previous layer's encoder
-  // (src/model/bdh.rs:383, 436-441: cur = LN(cur + LN(mixed . decoder)))
-  {
-    const bool has = tid < d;
-    float cur = 0.0f;
-    if (a.tokens) {  // embedding row and its LayerNorm (src/model/bdh.rs:319-322); a bad token poisons the row
-      const int64_t tok = a.tokens[b];
-      const bool bad = tok < 0 || tok >= a.V;
-      const float v = has ? (bad ? __int_as_float(0x7fc00000) : a.embed[(long)tok * d + tid]) : 0.0f;
-      float mean, den;
-      block_ln_stats<NW>(v, has, d, s_st, mean, den);
-      cur = has ? (v - mean) / den : 0.0f;
-      if (has && hh == 0 && nblk == 0) a.cur_out[(long)b * d + tid] = cur;
-    } else if (has) {
-      cur = a.cur_in[(long)b * d + tid];
-    }
-    if (a.dec_partial) {
-      const int G = h * nblk_n;
-      float mlp = 0.0f;
-      if (has) {
-        int g = 0;
-        for (; g + 8 <= G; g += 8) {
-          float t[8];
-#pragma unroll
-          for (int u = 0; u < 8; ++u) t[u] = a.dec_partial[((long)(g + u) * a.B + b) * d + tid];
-#pragma unroll
-          for (int u = 0; u < 8; ++u) mlp += t[u];
-        }
-        for (; g < G; ++g) mlp += a.dec_partial[((long)g * a.B + b) * d + tid];
-      }
-      float mean, den;
-      block_ln_stats<NW>(mlp, has, d, s_st, mean, den);
-      const float z = has ? cur + (mlp - mean) / den : 0.0f;
-      block_ln_stats<NW>(z, has, d, s_st, mean, den);
-      cur = has ? (z - mean) / den : 0.0f;
-      if (has && hh == 0 && nblk == 0) a.cur_out[(long)b * d + tid] = cur;
-    }
-    s_cur[tid] = cur;  // zero beyond d
-  }
-  __syncthreads();
-
-  // x = relu(cur . encoder - thr) for the 64 neurons (src/model/bdh.rs:337-351)
-  {
-    const float acc = chain_spans<NW>(s_cur, wv, s_acc);
-    if (wave == NW - 1) {
-      float p = acc;
-      if (a.thr != 0.0f) p = p - a.thr;
-      const float xv = p > 0.0f ? p : 0.0f;
-      s_x[lane] = xv;
-      a.x[((long)b * h + hh) * N + n] = xv;
-    }
-  }
-  __syncthreads();
-
-  // the state rows of these neurons (src/model/bdh.rs:232-306): readout with the old rows, rank-1 update with
-  // value = cur, ALiBi decay; only visited rows are touched.  Every wave prepares the same list (lane = neuron)
-  // and takes every NW-th entry of it.
+  const float dec = a.decay[hh], log_dec = a.log_decay[hh];
+  // the kernel arguments in one go: fetched where each is used, they are eight waits one after the other
+  asm volatile("" ::"s"(a.tokens), "s"(a.embed), "s"(a.cur_in), "s"(a.cur_out), "s"(a.dec_partial), "s"(a.x), "s"(a.attn_partial),
+               "s"(a.enc), "s"(a.freqs), "s"(a.rho), "s"(a.stamps), "s"(a.pos_dev), "s"(a.pos), "s"(a.B), "s"(a.V), "s"(d),
+               "s"(h), "s"(N), "s"(a.rotary), "s"(a.thr), "s"(dec), "s"(log_dec));
+  const int nblk_n = N / NB;
+  const int nl = lane & (NB - 1), n = nblk * NB + nl;  // this lane's neuron of the block and of the head
   const bool alibi = a.rotary == BDH_ALIBI, pope = a.rotary == BDH_POPE;
   const int Nq = pope ? 2 * N : N;
   RhoT *rho = static_cast<RhoT *>(a.rho) + ((long)b * h + hh) * (long)Nq * d;
   int32_t *st = a.stamps ? a.stamps + ((long)b * h + hh) * N : nullptr;
   const bool lazy = alibi && st != nullptr;
-  const float dec = alibi ? a.decay[hh] : 1.0f;
-  float4 acc[VPL], vv[VPL];
+
+  // everything this launch reads, in the order of use
+  float cur[S::CJ];
+  RowSum<DC, NW> partials;
+  bool bad = false;
+  if constexpr (FIRST) {  // embedding row (src/model/bdh.rs:319-322); a bad token poisons the row
+    const int64_t tok = scalar_load(a.tokens + b);
+    bad = tok < 0 || tok >= a.V;
+    const float *e = a.embed + (bad ? 0 : (long)tok * d);
 #pragma unroll
-  for (int j = 0; j < VPL; ++j) {
-    const int c = (j * 64 + lane) * 4;
+    for (int j = 0; j < S::CJ; ++j) cur[j] = e[min(j * 64 + lane, d - 1)];
+  } else {
+    partials.ask(a.dec_partial + (long)b * d, (long)a.B * d, h * nblk_n, d);
+#pragma unroll
+    for (int j = 0; j < S::CJ; ++j) cur[j] = a.cur_in[(long)b * d + min(j * 64 + lane, d - 1)];
+  }
+  Project<DC, NW, NB> dx;
+  dx.ask(a.enc + (long)hh * d * N + nblk * NB, d, N);
+  const long pos = a.pos_dev ? (long)scalar_load(a.pos_dev + b) : a.pos;
+  const float posf = (float)pos;
+  const float freq = a.freqs[n];
+  const int stamp = *(lazy ? st + n : reinterpret_cast<const int32_t *>(a.freqs + n));  // unused unless lazy: no branch
+  const int sub = S::RPI == 2 ? lane >> 5 : 0, cl = lane & (S::LPR - 1);
+  Raw rv[S::RU][S::VPL];
+  // the row of slot u: row `base` of the head (the same for the wave), `more` (0 or, for half a wave, some) rows further on
+  auto load_row = [&](int u, long base, int more) {
+#pragma unroll
+    for (int j = 0; j < S::VPL; ++j) {
+      const int c = (j * S::LPR + cl) * 4;
+      rv[u][j] = load_raw(rho + base * d + (more * d + (c < d ? c : 0)));
+    }
+  };
+  // first row of slot u of this wave's share of the block when all are taken
+  auto own_row = [&](int u) { return (wave * S::RU + u) * S::RPI; };
+  if constexpr (AHEAD) {
+#pragma unroll
+    for (int u = 0; u < S::RU; ++u) load_row(u, nblk * NB + own_row(u), sub);
+  }
+
+  __builtin_amdgcn_sched_barrier(0);  // nothing is waited for before all of it is on its way
+
+  // the layer's input: cur, after the pending second stage of the previous layer's encoder
+  // (src/model/bdh.rs:383, 436-441: cur = LN(cur + LN(mixed . decoder)))
+  if constexpr (FIRST) {
+    if (bad) {
+#pragma unroll
+      for (int j = 0; j < S::CJ; ++j) cur[j] = __int_as_float(0x7fc00000);
+    }
+  } else {
+    float mlp[S::CJ];
+    partials.collect(h * nblk_n, s_part, mlp);
+    wave_layer_norm<S::CJ>(mlp, d);
+#pragma unroll
+    for (int j = 0; j < S::CJ; ++j) cur[j] = cur[j] + mlp[j];
+  }
+  wave_layer_norm<S::CJ>(cur, d);
+#pragma unroll
+  for (int j = 0; j < S::CJ; ++j) s_cur[wave][j * 64 + lane] = j * 64 + lane < d ? cur[j] : 0.0f;
+  if (hh == 0 && nblk == 0 && wave == 0) {
+#pragma unroll
+    for (int j = 0; j < S::CJ; ++j)
+      if (j * 64 + lane < d) a.cur_out[(long)b * d + j * 64 + lane] = cur[j];
+  }
+  wave_lds_order();
+
+  // x = relu(cur . encoder - thr) for the 64 neurons (src/model/bdh.rs:337-351), the same in every wave
+  float xn = dx.dot(s_cur[wave], d, s_acc);
+  if (a.thr != 0.0f) xn = xn - a.thr;
+  xn = xn > 0.0f ? xn : 0.0f;
+  if (wave == 0 && lane < NB) a.x[((long)b * h + hh) * N + n] = xn;
+
+  // the state rows of these neurons (src/model/bdh.rs:232-306): readout with the old rows, rank-1 update with
+  // value = cur, ALiBi decay; only visited rows are touched
+  float4 acc[S::VPL], vv[S::VPL];
+#pragma unroll
+  for (int j = 0; j < S::VPL; ++j) {
     acc[j] = make_float4(0.f, 0.f, 0.f, 0.f);
-    vv[j] = c < d ? *reinterpret_cast<const float4 *>(&s_cur[c]) : make_float4(0.f, 0.f, 0.f, 0.f);
+    vv[j] = *reinterpret_cast<const float4 *>(&s_cur[wave][(j * S::LPR + cl) * 4]);
   }
   for (int part = 0; part < (pope ? 2 : 1); ++part) {  // PoPE: real rows n, then imaginary rows N + n
     float q_l = 0.0f, scale_l = 1.0f;
     bool touch_l = false;
-    const float xn = s_x[lane];
     if (alibi) {  // q = x (src/model/attention.rs:332-349)
       q_l = xn;
       touch_l = lazy ? (q_l != 0.0f) : true;
       if (lazy && touch_l) {
-        const long k = pos - (long)st[n];
-        if (k > 0) scale_l = expf((float)k * a.log_decay[hh]);
+        const long k = pos - (long)stamp;
+        if (k > 0) scale_l = expf((float)k * log_dec);
       }
     } else if (pope) {  // src/model/attention.rs:323-330
       const float mag = logf(expf(xn * 1.0f) + 1.0f) / 1.0f;
-      const float raw = posf * a.freqs[n];
+      const float raw = posf * freq;
       const float ph = (raw - floorf(raw)) * kTwoPi;
       q_l = part == 0 ? mag * cosf(ph) : mag * sinf(ph);
       touch_l = true;
     } else {  // RoPE (src/model/attention.rs:305-321)
-      const float xo = s_x[lane ^ 1];
+      const float xo = dpp<0xb1>(xn);  // the other neuron of the pair
       touch_l = (xn != 0.0f) || (xo != 0.0f);
       if (touch_l) {
-        const float raw = posf * a.freqs[n];
+        const float raw = posf * freq;
         const float ph = (raw - floorf(raw)) * kTwoPi;
         float sn, cs;
         sincosf(ph, &sn, &cs);
@@ -222,216 +394,251 @@ __global__ __launch_bounds__(NW * 64) void k_layer_phase_a(PhaseArgs a) {
         q_l = t0 + t1;
       }
     }
-    const unsigned long long m = __ballot(touch_l);
-    const int count = __popcll(m);
-    if (touch_l) s_list[wave][__popcll(m & ((1ull << lane) - 1ull))] = (unsigned char)lane;
-    // (LDS operations of one wave execute in order: the list is read back below without a barrier)
-    const long row_base = (long)(part * N + nblk * 64);
-    for (int i0 = wave; i0 < count; i0 += NW * kFlight) {
-      int src[kFlight];
-      bool ok[kFlight];
-      float4 rv[kFlight][VPL];
+    const unsigned long long m = __ballot(touch_l && lane < NB);
+    const long row_base = (long)(part * N + nblk * NB);
+    int src[S::RU];  // the row of slot u, and whether it is visited
+    bool ok[S::RU];
+    if constexpr (AHEAD) {
 #pragma unroll
-      for (int u = 0; u < kFlight; ++u) {
-        const int idx = i0 + u * NW;
-        const int listed = s_list[wave][idx & 63];  // read whether or not the slot is used: no branch
+      for (int u = 0; u < S::RU; ++u) {
+        src[u] = own_row(u) + sub;
+        ok[u] = S::RPI == 1 ? (m >> own_row(u)) & 1 : (m >> own_row(u) >> sub) & 1;
+      }
+    } else {  // every wave makes the same list of visited rows and takes every NW-th entry (pair of entries) of it
+      const int count = __popcll(m);
+      if (touch_l && lane < NB) s_list[wave][__popcll(m & ((1ull << lane) - 1ull))] = (unsigned char)lane;
+      wave_lds_order();
+#pragma unroll
+      for (int u = 0; u < S::RU; ++u) {
+        const int idx = (u * NW + wave) * S::RPI + sub;
+        const int listed = s_list[wave][idx & (NB - 1)];  // read whether or not the slot is used: no branch
         ok[u] = idx < count;
         src[u] = ok[u] ? listed : 0;
+        if (S::RPI == 1) src[u] = __builtin_amdgcn_readfirstlane(src[u]);
       }
 #pragma unroll
-      for (int u = 0; u < kFlight; ++u) {
-        const RhoT *row = rho + (row_base + src[u]) * d;
+      for (int u = 0; u < S::RU; ++u)
+        if (u * NW * S::RPI < count)  // uniform
+          load_row(u, row_base + (S::RPI == 1 ? src[u] : 0), S::RPI == 1 ? 0 : src[u]);
+    }
 #pragma unroll
-        for (int j = 0; j < VPL; ++j) {
-          const int c = (j * 64 + lane) * 4;
-          rv[u][j] = bdh_rho_load4(row + (c < d ? c : 0));
-        }
+    for (int u = 0; u < S::RU; ++u) {
+      if (!AHEAD && u * NW * S::RPI >= __popcll(m)) break;
+      float q_src, scale = 1.0f;
+      if (S::RPI == 1) {
+        q_src = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(q_l), src[u]));
+        if (lazy) scale = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(scale_l), src[u]));
+      } else {
+        q_src = __shfl(q_l, src[u], 64);
+        if (lazy) scale = __shfl(scale_l, src[u], 64);
       }
+      if (S::RPI == 1 && !ok[u]) continue;  // uniform
+      const float qn = ok[u] ? q_src : 0.0f;
+      RhoT *row = rho + (row_base + (S::RPI == 1 ? src[u] : 0)) * d + (S::RPI == 1 ? 0 : src[u]) * d;
+      Raw old[S::VPL];
 #pragma unroll
-      for (int u = 0; u < kFlight; ++u) {
-        const int lu = __builtin_amdgcn_readfirstlane(src[u]);
-        const float q_src = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(q_l), lu));
-        const float scale = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(scale_l), lu));
-        const float qn = ok[u] ? q_src : 0.0f;
-        RhoT *row = rho + (row_base + src[u]) * d;
+      for (int j = 0; j < S::VPL; ++j) old[j] = rv[u][j];
+      if (AHEAD && pope && part == 0) load_row(u, (long)N + nblk * NB + own_row(u), sub);  // its imaginary row
 #pragma unroll
-        for (int j = 0; j < VPL; ++j) {
-          const int c = (j * 64 + lane) * 4;
-          float4 e = rv[u][j];
-          if (!ok[u]) e = make_float4(0.f, 0.f, 0.f, 0.f);
-          if (lazy) {
-            e.x *= scale; e.y *= scale; e.z *= scale; e.w *= scale;
-          }
-          acc[j].x = __builtin_fmaf(e.x, qn, acc[j].x);
-          acc[j].y = __builtin_fmaf(e.y, qn, acc[j].y);
-          acc[j].z = __builtin_fmaf(e.z, qn, acc[j].z);
-          acc[j].w = __builtin_fmaf(e.w, qn, acc[j].w);
-          float t;
-          t = qn * vv[j].x; e.x = e.x + t;
-          t = qn * vv[j].y; e.y = e.y + t;
-          t = qn * vv[j].z; e.z = e.z + t;
-          t = qn * vv[j].w; e.w = e.w + t;
-          if (alibi) {  // src/model/bdh.rs:299-301
-            e.x *= dec; e.y *= dec; e.z *= dec; e.w *= dec;
-          }
-          if (ok[u] && c < d) bdh_rho_store4(row + c, e);
+      for (int j = 0; j < S::VPL; ++j) {
+        const int c = (j * S::LPR + cl) * 4;
+        float4 e = widen(old[j]);
+        if (!ok[u]) e = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (lazy) {
+          e.x *= scale; e.y *= scale; e.z *= scale; e.w *= scale;
         }
+        acc[j].x = __builtin_fmaf(e.x, qn, acc[j].x);
+        acc[j].y = __builtin_fmaf(e.y, qn, acc[j].y);
+        acc[j].z = __builtin_fmaf(e.z, qn, acc[j].z);
+        acc[j].w = __builtin_fmaf(e.w, qn, acc[j].w);
+        float t;
+        t = qn * vv[j].x; e.x = e.x + t;
+        t = qn * vv[j].y; e.y = e.y + t;
+        t = qn * vv[j].z; e.z = e.z + t;
+        t = qn * vv[j].w; e.w = e.w + t;
+        if (alibi) {  // src/model/bdh.rs:299-301
+          e.x *= dec; e.y *= dec; e.z *= dec; e.w *= dec;
+        }
+        if (ok[u] && c < d) bdh_rho_store4(row + c, e);
       }
     }
-    __syncthreads();  // every wave has read the stamps before the first one replaces them
-    if (lazy && touch_l && wave == 0) st[n] = (int32_t)min(pos + 1, 0x7fffffffL);
   }
-#pragma unroll
-  for (int j = 0; j < VPL; ++j) s_red[wave][j * 64 + lane] = acc[j];
-  __syncthreads();
-  float *pout = a.attn_partial + (((long)b * h + hh) * nblk_n + nblk) * d;
-  for (int c4 = tid; c4 < d / 4; c4 += NW * 64) {
-    const int j = c4 >> 6, l = c4 & 63;  // column group c4 lives in lane l, piece j
-    float4 s = s_red[0][j * 64 + l];
-#pragma unroll
-    for (int w = 1; w < NW; ++w) {
-      const float4 t = s_red[w][j * 64 + l];
-      s.x += t.x; s.y += t.y; s.z += t.z; s.w += t.w;
-    }
-    reinterpret_cast<float4 *>(pout)[c4] = s;
-  }
+  write_row_sum<DC, NW>(acc, s_red, d, a.attn_partial + (((long)b * h + hh) * nblk_n + nblk) * d);
+  // behind the barrier in there: every wave has its stamps
+  if (lazy && xn != 0.0f && wave == 0 && lane < NB) st[n] = (int32_t)min(pos + 1, 0x7fffffffL);
 }
 
 // ---- phase B ---------------------------------------------------------------------------------------------------
-template <int NW>
-__global__ __launch_bounds__(NW * 64) void k_layer_phase_b(PhaseArgs a) {
-  __shared__ float s_in[NW * 64];
-  __shared__ float s_xy[64];
-  __shared__ float s_acc[64];
-  __shared__ float s_st[2 * NW];
+template <int DC, int NW, int NB>
+__global__ __launch_bounds__(NW * 64, 2) void k_layer_phase_b(PhaseArgs a) {
+  using S = Shape<DC, NW, NB>;
+  __shared__ float4 s_part[S::NT];
+  __shared__ __align__(16) float s_in[NW][DC];
+  __shared__ __align__(16) float s_acc[NW][NB];
+  __shared__ __align__(16) float s_red[NW][DC];
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int lane = threadIdx.x & 63, wave = wave_id();
+  const int nblk = blockIdx.x, hh = blockIdx.y, b = blockIdx.z;
   const int d = a.d, h = a.h, N = a.N;
-  const int nblk_n = N >> 6;
-  const int nblk = blockIdx.x % nblk_n;
-  const int hh = (blockIdx.x / nblk_n) % h;
-  const int b = blockIdx.x / (nblk_n * h);
-  const int n = nblk * 64 + lane;
+  asm volatile("" ::"s"(a.attn_partial), "s"(a.x), "s"(a.enc_v), "s"(a.dec), "s"(a.dec_partial_out), "s"(a.B), "s"(d), "s"(h),
+               "s"(N), "s"(a.thr));  // in one go, as above
+  const int nblk_n = N / NB;
 
-  float wv[64];
-  load_span(a.enc_v, hh, d, N, n, wave * 64, wv);
-  const float xg = wave == NW - 1 ? a.x[((long)b * h + hh) * N + n] : 0.0f;  // the gate, needed last
-
-  // LayerNorm of the head's readout (src/model/bdh.rs:359): the partials of the head's workgroups, in order
-  {
-    const bool has = tid < d;
-    float at = 0.0f;
-    if (has) {
-      const float *pp = a.attn_partial + ((long)b * h + hh) * nblk_n * d + tid;
-      int g = 0;
-      for (; g + 8 <= nblk_n; g += 8) {
-        float t[8];
+  // everything this launch reads, in the order of use: the readout partials of the head, its part of D_y, the gate, and
+  // these NB rows of E
+  RowSum<DC, NW> partials;
+  partials.ask(a.attn_partial + ((long)b * h + hh) * nblk_n * d, d, nblk_n, d);
+  Project<DC, NW, NB> dy;
+  dy.ask(a.enc_v + (long)hh * d * N + nblk * NB, d, N);
+  const float gate = a.x[((long)b * h + hh) * N + nblk * NB + (lane & (NB - 1))];
+  const int sub = S::RPI == 2 ? lane >> 5 : 0, cl = lane & (S::LPR - 1);
+  float4 ev[S::RU][S::VPL];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) t[u] = pp[(long)(g + u) * d];
+  for (int u = 0; u < S::RU; ++u) {
+    const float *e = a.dec + ((long)hh * N + nblk * NB + (wave * S::RU + u) * S::RPI) * d;
 #pragma unroll
-        for (int u = 0; u < 8; ++u) at += t[u];
-      }
-      for (; g < nblk_n; ++g) at += pp[(long)g * d];
-    }
-    float mean, den;
-    block_ln_stats<NW>(at, has, d, s_st, mean, den);
-    s_in[tid] = has ? (at - mean) / den : 0.0f;
-  }
-  __syncthreads();
-
-  // xy = x * relu(LN(attn) . encoder_v - thr) for the 64 neurons (src/model/bdh.rs:361-381)
-  {
-    const float acc = chain_spans<NW>(s_in, wv, s_acc);
-    if (wave == NW - 1) {
-      float p = acc;
-      if (a.thr != 0.0f) p = p - a.thr;
-      const float y = p > 0.0f ? p : 0.0f;
-      s_xy[lane] = xg * y;
+    for (int j = 0; j < S::VPL; ++j) {
+      const int c = (j * S::LPR + cl) * 4;
+      ev[u][j] = load_at<float4>(e, (sub * d + (c < d ? c : 0)) * 4u);
     }
   }
-  __syncthreads();
 
-  // encoder partial of these 64 rows of E (src/model/bdh.rs:383): one column per thread, the 64 rows in flight
-  if (tid < d) {
-    const float *ep = a.dec + ((long)hh * N + nblk * 64) * d + tid;
-    float ev[64];
+  __builtin_amdgcn_sched_barrier(0);
+
+  // LayerNorm of the head's readout (src/model/bdh.rs:359)
+  {
+    float at[S::CJ];
+    partials.collect(nblk_n, s_part, at);
+    wave_layer_norm<S::CJ>(at, d);
 #pragma unroll
-    for (int u = 0; u < 64; ++u) ev[u] = ep[(long)u * d];
-    float acc = 0.0f;
-#pragma unroll
-    for (int u = 0; u < 64; ++u) acc = __builtin_fmaf(s_xy[u], ev[u], acc);
-    const int g = hh * nblk_n + nblk;
-    a.dec_partial_out[((long)g * a.B + b) * d + tid] = acc;
+    for (int j = 0; j < S::CJ; ++j) s_in[wave][j * 64 + lane] = j * 64 + lane < d ? at[j] : 0.0f;
+    wave_lds_order();
   }
+  // xy = x * relu(LN(attn) . encoder_v - thr) for the 64 neurons (src/model/bdh.rs:361-381), the same in every wave
+  float y = dy.dot(s_in[wave], d, s_acc);
+  if (a.thr != 0.0f) y = y - a.thr;
+  const float xy = gate * (y > 0.0f ? y : 0.0f);
+
+  // encoder partial of these rows of E (src/model/bdh.rs:383)
+  float4 acc[S::VPL];
+#pragma unroll
+  for (int j = 0; j < S::VPL; ++j) acc[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+  for (int u = 0; u < S::RU; ++u) {
+    const int r = (wave * S::RU + u) * S::RPI + sub;
+    const float q = S::RPI == 1 ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(xy), r)) : __shfl(xy, r, 64);
+#pragma unroll
+    for (int j = 0; j < S::VPL; ++j) {
+      acc[j].x = __builtin_fmaf(q, ev[u][j].x, acc[j].x);
+      acc[j].y = __builtin_fmaf(q, ev[u][j].y, acc[j].y);
+      acc[j].z = __builtin_fmaf(q, ev[u][j].z, acc[j].z);
+      acc[j].w = __builtin_fmaf(q, ev[u][j].w, acc[j].w);
+    }
+  }
+  write_row_sum<DC, NW>(acc, s_red, d, a.dec_partial_out + ((long)(hh * nblk_n + nblk) * a.B + b) * d);
 }
 
 // ---- head -----------------------------------------------------------------------------------------------------
 // The last layer's pending second stage, then the logits and the greedy token (src/model/bdh.rs:436-449): one
-// workgroup of 16 waves per sequence.  logits[v] = sum_k cur[k] * lm_head[k][v]: 1024 / pad64(V) groups split k,
-// each one fmaf chain over its span with 32 rows in flight; the groups are added in order; the lowest index wins ties.
+// workgroup of 16 waves per sequence.  logits[v] = sum_k cur[k] * lm_head[k][v]: a thread takes NC adjacent columns and one
+// of GK spans of k, in one fmaf chain per column whose first AHEAD rows are asked for before the LayerNorms (wave 0 makes
+// those); the spans are added in order; the lowest index wins ties.  What bounds it: one CU fetches all of lm_head, 64 bytes
+// a cycle.
+template <int NC>
 __global__ __launch_bounds__(1024) void k_phase_head(const float *__restrict__ cur_in, const float *__restrict__ dec_partial,
                                                      int G, int B, int d, const float *__restrict__ lm_head, int V,
                                                      float *__restrict__ logits, int64_t *__restrict__ next) {
+  constexpr int AHEAD = 64 / NC;
+  typedef float Cols __attribute__((ext_vector_type(NC)));
   __shared__ float s_cur[512];
-  __shared__ float s_st[32];
-  __shared__ float s_grp[1024];
+  __shared__ float4 s_part[1024];
+  __shared__ __align__(16) float s_grp[1024 * NC];
   __shared__ float s_best[16];
   __shared__ int s_arg[16];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
   const int b = blockIdx.x;
-  {
-    const bool has = tid < d;
-    float mlp = 0.0f;
-    if (has) {
-      int g = 0;
-      for (; g + 8 <= G; g += 8) {
-        float t[8];
+  // partial rows r0, r0 + 8, ... and four columns per thread (d <= 512)
+  const int r0 = tid >> 7, c4 = (tid & 127) * 4;
+  float4 t[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) t[u] = dec_partial[((long)(g + u) * B + b) * d + tid];
+  for (int i = 0; i < 8; ++i) {
+    t[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (i == 0 || i * 8 < G)  // uniform
+      t[i] = *reinterpret_cast<const float4 *>(dec_partial + ((long)min(r0 + i * 8, G - 1) * B + b) * d + (c4 < d ? c4 : 0));
+  }
+  float cur[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) mlp += t[u];
-      }
-      for (; g < G; ++g) mlp += dec_partial[((long)g * B + b) * d + tid];
+  for (int j = 0; j < 8; ++j) cur[j] = wave == 0 && j * 64 < d ? cur_in[(long)b * d + min(j * 64 + lane, d - 1)] : 0.0f;
+  const int per_row = (V + NC - 1) / NC;  // threads per row of lm_head
+  const int span = (per_row + 63) & ~63, GK = 1024 / span;
+  const int g = tid / span, c = (tid - g * span) * NC;
+  const int per = (d + GK - 1) / GK;
+  const bool busy = g < GK && c < V;
+  const int k0 = min(d, g * per), k1 = busy ? min(d, k0 + per) : k0;
+  const float *wp = lm_head + (busy ? c : 0);
+  Cols wv[AHEAD];
+#pragma unroll
+  for (int u0 = 0; u0 < AHEAD; u0 += 16) {
+    if (u0 < per) {  // uniform
+#pragma unroll
+      for (int u = 0; u < 16; ++u) wv[u0 + u] = *reinterpret_cast<const Cols *>(wp + (long)min(k0 + u0 + u, d - 1) * V);
     }
-    const float base = has ? cur_in[(long)b * d + tid] : 0.0f;
-    float mean, den;
-    block_ln_stats<16>(mlp, has, d, s_st, mean, den);
-    const float z = has ? base + (mlp - mean) / den : 0.0f;
-    block_ln_stats<16>(z, has, d, s_st, mean, den);
-    if (tid < 512) s_cur[tid] = has ? (z - mean) / den : 0.0f;
+  }
+  __builtin_amdgcn_sched_barrier(0);
+
+  float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const bool in = r0 + i * 8 < G;
+    sum.x += in ? t[i].x : 0.0f;
+    sum.y += in ? t[i].y : 0.0f;
+    sum.z += in ? t[i].z : 0.0f;
+    sum.w += in ? t[i].w : 0.0f;
+  }
+  s_part[tid] = sum;  // [8][512]
+  __syncthreads();
+  if (wave == 0) {
+    float mlp[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float *f = reinterpret_cast<const float *>(s_part) + j * 64 + lane;
+      mlp[j] = f[0];
+#pragma unroll
+      for (int r = 1; r < 8; ++r) mlp[j] += f[r * 512];
+    }
+    wave_layer_norm<8>(mlp, d);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) cur[j] = cur[j] + mlp[j];
+    wave_layer_norm<8>(cur, d);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s_cur[j * 64 + lane] = cur[j];
   }
   __syncthreads();
-  const int Vp = (V + 63) & ~63;
-  const int GK = 1024 / Vp;
-  const int g = tid / Vp, c = tid - g * Vp;
-  const int per = (d + GK - 1) / GK;
-  if (g < GK && c < V) {
-    const int k0 = min(d, g * per), k1 = min(d, k0 + per);
-    float acc = 0.0f;
-    int k = k0;
-    for (; k + 32 <= k1; k += 32) {
-      float wv[32];
+  if (busy) {
+    Cols acc = 0.0f;
+    auto add16 = [&](int k, const Cols *w) {  // a row past the span counts as zero
 #pragma unroll
-      for (int u = 0; u < 32; ++u) wv[u] = lm_head[(long)(k + u) * V + c];
+      for (int u = 0; u < 16; ++u) {
+        const bool in = k + u < k1;
+        acc = __builtin_elementwise_fma(Cols(s_cur[in ? k + u : 0]), in ? w[u] : Cols(0.0f), acc);
+      }
+    };
 #pragma unroll
-      for (int u = 0; u < 32; ++u) acc = __builtin_fmaf(s_cur[k + u], wv[u], acc);
+    for (int u0 = 0; u0 < AHEAD; u0 += 16)
+      if (u0 < per) add16(k0 + u0, wv + u0);
+    for (int k = k0 + AHEAD; k < k0 + per; k += 16) {  // narrow vocabularies and long rows only
+#pragma unroll
+      for (int u = 0; u < 16; ++u) wv[u] = *reinterpret_cast<const Cols *>(wp + (long)min(k + u, d - 1) * V);
+      add16(k, wv);
     }
-    for (; k + 8 <= k1; k += 8) {
-      float wv[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) wv[u] = lm_head[(long)(k + u) * V + c];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) acc = __builtin_fmaf(s_cur[k + u], wv[u], acc);
-    }
-    for (; k < k1; ++k) acc = __builtin_fmaf(s_cur[k], lm_head[(long)k * V + c], acc);
-    s_grp[g * Vp + c] = acc;
+    *reinterpret_cast<Cols *>(&s_grp[g * span * NC + c]) = acc;
   }
   __syncthreads();
   float best = -INFINITY;
   int arg = 0x7fffffff;
   if (tid < V) {
     float v = s_grp[tid];
-    for (int gg = 1; gg < GK; ++gg) v += s_grp[gg * Vp + tid];
+    for (int gg = 1; gg < GK; ++gg) v += s_grp[gg * span * NC + tid];
     logits[(long)b * V + tid] = v;
     if (v > best) {
       best = v;
@@ -462,20 +669,69 @@ __global__ __launch_bounds__(1024) void k_phase_head(const float *__restrict__ c
   }
 }
 
+// The two launches of a layer.
+template <int DC, int NW, int NB, typename RhoT, bool AHEAD>
+void launch_phase_a(hipStream_t stream, dim3 grid, bool first, const PhaseArgs &a) {
+  if (first) hipLaunchKernelGGL((k_layer_phase_a<DC, NW, NB, RhoT, AHEAD, true>), grid, dim3(NW * 64), 0, stream, a);
+  else hipLaunchKernelGGL((k_layer_phase_a<DC, NW, NB, RhoT, AHEAD, false>), grid, dim3(NW * 64), 0, stream, a);
+}
+template <int DC, int NW, int NB>
+void launch_layer(hipStream_t stream, dim3 grid, int rho_dtype, bool ahead, bool first, const PhaseArgs &a) {
+  if (rho_dtype == BDH_BF16) {
+    if (ahead) launch_phase_a<DC, NW, NB, unsigned short, true>(stream, grid, first, a);
+    else launch_phase_a<DC, NW, NB, unsigned short, false>(stream, grid, first, a);
+  } else {
+    if (ahead) launch_phase_a<DC, NW, NB, float, true>(stream, grid, first, a);
+    else launch_phase_a<DC, NW, NB, float, false>(stream, grid, first, a);
+  }
+  hipLaunchKernelGGL((k_layer_phase_b<DC, NW, NB>), grid, dim3(NW * 64), 0, stream, a);
+}
+
 }  // namespace
 
-bool bdh_model_phase_fits(const bdh_model_config &c) {
+bool bdh_model_phase_fits(const bdh_model *m) {
+  const bdh_model_config &c = m->cfg;
   if (c.rotary != BDH_ROPE && c.rotary != BDH_ALIBI && c.rotary != BDH_POPE) return false;
   if (c.n_embd < 128 || c.n_embd > 512 || (c.n_embd & 3) != 0) return false;
   if (c.latent < 64 || (c.latent & 63) != 0) return false;  // whole 64-neuron blocks
   if (c.n_head < 1 || c.n_head > 64 || c.n_layer < 1) return false;
   // every workgroup of a sequence sums the partials of all the others: only while those are few
   if ((long)c.n_head * (c.latent / 64) > 64) return false;
-  return true;
+  // 16-byte loads
+  return bdh_aligned(m->w.encoder, 16) && bdh_aligned(m->w.encoder_v, 16) && bdh_aligned(m->w.decoder, 16);
 }
 
-size_t bdh_model_phase_scratch_floats(const bdh_model_config &c, int B) {
-  const size_t d = c.n_embd, cols = (size_t)c.n_head * c.latent, G = cols / 64;
+// Neurons of a workgroup's block.  Fewer share the bytes that a CU has to fetch among more CUs and make more partials, which
+// every workgroup adds up: 32 while those blocks number at most 64 and every workgroup has a CU to itself, 64 otherwise (us a
+// step, 32 | 64: 4 layers of 1024 neurons, d = 256, 1 sequence 46 | 52, 8 sequences (256 workgroups) 52 | 56, 16 sequences
+// 66 | 61; 8 layers of 2048, d = 512, 1 sequence 114 | 131, 4 sequences 134 | 146, 8 sequences 223 | 172).
+static int block_neurons(const bdh_ctx *ctx, const bdh_model_config &c, int B) {
+  const long n_cu = ctx->n_cu > 0 ? ctx->n_cu : 256, blocks = (long)c.n_head * c.latent / 32;
+  return blocks <= 64 && blocks * B <= n_cu ? 32 : 64;
+}
+
+// The most sequences that the two-launch layer is taken for: while batch x weights of a layer (every workgroup streams its
+// share once per sequence) stay below a bound from measurement.  us a step, two launches per layer | the other form:
+//   a model that the one-launch step takes as well, up to 8 MiB of weights: 3 MiB, 128 sequences 72 to 79 | 84 to 88, 192
+//   sequences 94 to 106 | 90 to 98; 6.75 MiB, 64 sequences 116 | 143, 128 sequences 196 | 165: 128 MiB
+//   f32, 12 MiB a layer, 24 sequences 290 to 535 | 367 to 604 kernel by kernel, 32 sequences 377 to 670 | 377 to 672; 3 MiB a
+//   layer, 128 sequences 214 to 288 | 265 to 327, 192 sequences 336 | 299: 384 MiB
+//   bf16, 12 MiB a layer, 24 sequences 281 to 487 | 287 to 504, 32 sequences 352 to 622 | 317 to 574: 288 MiB
+//   bf16 and lazily decayed, 12 MiB a layer, 128 sequences 1126 to 1839 | 1742 to 2520: 1536 MiB
+int bdh_model_phase_most(const bdh_model *m, int rho_dtype, bool lazy) {
+  const bdh_model_config &c = m->cfg;
+  const size_t w_layer = sizeof(float) * (size_t)3 * c.n_head * c.latent * c.n_embd;
+  const size_t mib = bdh_model_small_fits(c) && w_layer * c.n_layer <= (size_t(8) << 20) ? 128
+                     : rho_dtype != BDH_BF16                                              ? 384
+                     : lazy                                                               ? 1536
+                                                                                          : 288;
+  const size_t most = (mib << 20) / w_layer;
+  return most > 65535 ? 65535 : (int)most;
+}
+
+size_t bdh_model_phase_scratch_floats(const bdh_model *m, int B) {
+  const bdh_model_config &c = m->cfg;
+  const size_t d = c.n_embd, cols = (size_t)c.n_head * c.latent, G = cols / block_neurons(m->ctx, c, B);
   // cur ping-pong | x | readout partials | encoder partials
   return 2 * bdh_align_up((size_t)B * d, 64) + bdh_align_up((size_t)B * cols, 64) + bdh_align_up((size_t)B * G * d, 64) +
          bdh_align_up(G * (size_t)B * d, 64);
@@ -488,11 +744,12 @@ int bdh_launch_model_phases(bdh_model *m, const int64_t *tokens, int B, float *s
                             const int32_t *positions_dev, float **cur_final, float **dec_partial, int *G_out) {
   bdh_ctx *ctx = m->ctx;
   const bdh_model_config &c = m->cfg;
-  if (!bdh_model_phase_fits(c)) return bdh_fail(ctx, BDH_E_SHAPE, "model does not fit the two-launch layer");
+  if (!bdh_model_phase_fits(m)) return bdh_fail(ctx, BDH_E_SHAPE, "model does not fit the two-launch layer");
   const int d = c.n_embd, h = c.n_head, N = c.latent, L = c.n_layer;
-  const size_t cols = (size_t)h * N, G = cols / 64;
-  const long grid = (long)B * h * (N / 64);
-  if (grid > 0x7fffffffL) return bdh_fail(ctx, BDH_E_SHAPE, "grid too large");
+  const int nb = block_neurons(ctx, c, B);
+  const size_t cols = (size_t)h * N, G = cols / nb;
+  if (B > 65535) return bdh_fail(ctx, BDH_E_SHAPE, "grid too large");
+  const dim3 grid((unsigned)(N / nb), (unsigned)h, (unsigned)B);
   float *cur[2] = {scratch, scratch + bdh_align_up((size_t)B * d, 64)};
   float *x = cur[1] + bdh_align_up((size_t)B * d, 64);
   float *attn_partial = x + bdh_align_up((size_t)B * cols, 64);
@@ -519,7 +776,11 @@ int bdh_launch_model_phases(bdh_model *m, const int64_t *tokens, int B, float *s
       a.decay[i] = expf(-m->slopes[i]);                 // src/model/attention.rs:181-186
       a.log_decay[i] = (float)log((double)a.decay[i]);  // of the rounded factor, as the lazy state step
     }
-  const int nw = (d + 63) / 64;
+  // Phase A asks for all state rows ahead where every row is visited anyway, and where the rows are bf16 and short: half the
+  // bytes, so the rows that were asked for in vain cost less than the trip (us a step, ahead | visited rows only: d = 256,
+  // 64 blocks, RoPE, 16 sequences bf16 199 | 211, f32 256 | 255; 128 neurons per head, d = 128, f32 44 | 39; PoPE 42 | 43).
+  const bool dense = c.rotary == BDH_POPE || (c.rotary == BDH_ALIBI && !stamps);
+  const bool ahead = dense || (rho_dtype == BDH_BF16 && (nb == 32 || (d > 128 && d <= 256)));
   int in = 0;  // cur[in] is the layer's input; a layer with a pending second stage writes cur[in ^ 1]
   a.embed = m->w.embed;
   a.V = c.vocab;
@@ -530,21 +791,15 @@ int bdh_launch_model_phases(bdh_model *m, const int64_t *tokens, int B, float *s
     a.dec_partial = l > 0 ? dpart : nullptr;
     a.rho = static_cast<char *>(rho) + (size_t)l * B * h * Nq * d * (rho_dtype == BDH_BF16 ? 2 : 4);
     a.stamps = stamps ? stamps + (size_t)l * B * h * N : nullptr;
-#define BDH_PHASE(K_, NW_) hipLaunchKernelGGL((K_<NW_>), dim3((unsigned)grid), dim3(NW_ * 64), 0, ctx->stream, a)
-#define BDH_PHASE_A(NW_)                                                                                           \
-  do {                                                                                                             \
-    if (rho_dtype == BDH_BF16)                                                                                     \
-      hipLaunchKernelGGL((k_layer_phase_a<NW_, unsigned short>), dim3((unsigned)grid), dim3(NW_ * 64), 0, ctx->stream, a); \
-    else                                                                                                           \
-      hipLaunchKernelGGL((k_layer_phase_a<NW_, float>), dim3((unsigned)grid), dim3(NW_ * 64), 0, ctx->stream, a);   \
+#define BDH_PHASE(DC_, NW_)                                                                              \
+  do {                                                                                                   \
+    if (nb == 64) launch_layer<DC_, NW_, 64>(ctx->stream, grid, rho_dtype, ahead, l == 0, a);            \
+    else launch_layer<DC_, NW_, 32>(ctx->stream, grid, rho_dtype, ahead, l == 0, a);                     \
   } while (0)
-    if (nw <= 2) BDH_PHASE_A(2); else if (nw <= 4) BDH_PHASE_A(4); else BDH_PHASE_A(8);
-    BDH_LAUNCH_CHECK(ctx, "k_layer_phase_a");
-    if (l > 0) in ^= 1;  // phase A has applied the pending second stage: the layer's input is now cur[in ^ 1]
-    if (nw <= 2) BDH_PHASE(k_layer_phase_b, 2); else if (nw <= 4) BDH_PHASE(k_layer_phase_b, 4); else BDH_PHASE(k_layer_phase_b, 8);
-    BDH_LAUNCH_CHECK(ctx, "k_layer_phase_b");
+    if (d <= 128) BDH_PHASE(128, 4); else if (d <= 256) BDH_PHASE(256, 8); else BDH_PHASE(512, 8);
 #undef BDH_PHASE
-#undef BDH_PHASE_A
+    BDH_LAUNCH_CHECK(ctx, "k_layer_phase_a/b");
+    if (l > 0) in ^= 1;  // phase A has applied the pending second stage: the layer's input is now cur[in ^ 1]
   }
   *cur_final = cur[in];
   *dec_partial = dpart;
@@ -558,8 +813,11 @@ int bdh_launch_phase_head(bdh_model *m, int B, const float *cur, const float *de
   bdh_ctx *ctx = m->ctx;
   const bdh_model_config &c = m->cfg;
   if (c.vocab > 1024 || c.n_embd > 512) return bdh_fail(ctx, BDH_E_SHAPE, "head kernel needs V <= 1024 and d <= 512");
-  hipLaunchKernelGGL(k_phase_head, dim3((unsigned)B), dim3(1024), 0, ctx->stream, cur, dec_partial, G, B, c.n_embd,
-                     m->w.lm_head, c.vocab, logits, next_tokens);
+#define BDH_HEAD(NC_)                                                                                                      \
+  hipLaunchKernelGGL((k_phase_head<NC_>), dim3((unsigned)B), dim3(1024), 0, ctx->stream, cur, dec_partial, G, B, c.n_embd, \
+                     m->w.lm_head, c.vocab, logits, next_tokens)
+  if (c.vocab % 4 == 0 && bdh_aligned(m->w.lm_head, 16)) BDH_HEAD(4); else BDH_HEAD(1);
+#undef BDH_HEAD
   BDH_LAUNCH_CHECK(ctx, "k_phase_head");
   return BDH_OK;
 }

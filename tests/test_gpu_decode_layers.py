@@ -1,0 +1,76 @@
+"""The two-launch layer of a decode step at the sizes where it can go wrong: row widths at the edges of the three kernel
+widths (128, 256, 512), one and many blocks of neurons, the smallest and largest number of them, blocks of 32 and of 64,
+vocabularies read four columns at a time and one at a time, weights that are not 16-byte aligned."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+def rel_err(a, b):
+    a, b = a.double().cpu(), b.double().cpu()
+    return float((a - b).abs().max() / b.abs().max().clamp_min(1e-30))
+
+
+@pytest.mark.parametrize("state", ["f32", "bf16"])
+@pytest.mark.parametrize("rotary,lazy", [("rope", False), ("pope", False), ("alibi", False), ("alibi", True)])
+@pytest.mark.parametrize("d,h,N,V,B,aligned", [
+    (128, 1, 64, 69, 1, True),      # two blocks of 32
+    (128, 4, 128, 1024, 17, True),  # sixteen blocks of 32 a sequence, more workgroups than a chip of 256 has
+    (132, 3, 64, 1021, 2, True),    # a row that barely leaves the narrowest kernel
+    (252, 3, 192, 40, 3, True),     # rows that do not fill the middle kernel, blocks no multiple of its access
+    (256, 2, 1024, 256, 2, True),   # 64 blocks of 32
+    (256, 4, 1024, 64, 2, True),    # 64 blocks of 64
+    (260, 1, 64, 516, 1, True),
+    (512, 4, 64, 1024, 3, True),
+    (256, 4, 128, 256, 2, False),   # refused by this form: another one gives the same values
+])
+def test_two_launch_layer_edges(state, rotary, lazy, d, h, N, V, B, aligned):
+    import burn_dragon_amd as bda
+    from burn_dragon_amd import ffi
+
+    cfg = bda.BDHConfig(n_layer=2, n_embd=d, n_head=h, mlp_internal_dim_multiplier=1, vocab_size=V, dropout=0.0)
+    # N per head is multiplier * n_embd / n_head: choose the neurons directly
+    cfg.latent_per_head = lambda: N
+    cfg.fused_kernels.set_rotary_embedding(bda.RotaryEmbedding.parse(rotary))
+    g = torch.Generator(device=DEV).manual_seed(d + N)
+    w = {"embed": torch.randn((V, d), device=DEV, generator=g)}
+    for name, shape in (("encoder", (h, d, N)), ("encoder_v", (h, d, N)), ("decoder", (h * N, d)), ("lm_head", (d, V))):
+        w[name] = 0.05 * torch.randn(shape, device=DEV, generator=g)
+    if not aligned:  # four bytes off
+        for name, t in w.items():
+            flat = torch.empty(t.numel() + 1, device=DEV)
+            flat[1:] = t.reshape(-1)
+            w[name] = flat[1:].view(t.shape)
+    models = [bda.BDH(cfg, DEV, weights=w, alibi_lazy=lazy, rho_dtype=ffi.BF16 if state == "bf16" else ffi.F32) for _ in range(2)]
+    assert all((t.data_ptr() % 16 == 0) == aligned for t in models[0].params.values())
+    ctx = bda.ffi.default_context(0)
+    states = [m.init_state() for m in models]
+    start = 0.1 * torch.randn((2, B, h, models[0].latent_q, d), device=DEV, generator=g)
+    for m, s in zip(models, states):
+        m._ensure_state(s, B)
+        s.storage.copy_(start)
+        s.position = 5
+        if lazy:
+            s.stamps.fill_(3)  # two tokens of decay pending
+    tokens = torch.randint(0, V, (3, B, 1), device=DEV, generator=g)
+    for t in range(3):
+        got, nxt = models[0].forward_with_state(tokens[t], states[0], want_next=True)
+        try:
+            ctx.set_option("model.one_launch", 0)
+            ref = models[1].forward_with_state(tokens[t], states[1])
+        finally:
+            ctx.set_option("model.one_launch", 1)
+        torch.cuda.synchronize()
+        # f32: other summation trees over at most 4096 terms.  bf16: the inputs of a rounding differ in their last bits, so a
+        # stored element may land one bf16 step (2^-8 of it) apart; thousands of them average out in a readout
+        assert rel_err(got, ref) < (1e-5 if state == "f32" else 2e-3), t
+        assert torch.equal(nxt.reshape(-1), got[:, 0].argmax(-1))
+    for m, s in zip(models, states):
+        m.materialize_state(s)
+    torch.cuda.synchronize()
+    assert rel_err(states[0].storage.float(), states[1].storage.float()) < (1e-5 if state == "f32" else 3 * 2.0 ** -8)
+    if lazy:
+        assert torch.equal(states[0].stamps, states[1].stamps)
