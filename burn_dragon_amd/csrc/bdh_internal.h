@@ -269,3 +269,53 @@ __device__ __forceinline__ void bdh_rho_store4(unsigned short *p, float4 v) {
   o.y = bdh_bf16_rne(v.z) | (bdh_bf16_rne(v.w) << 16);
   *reinterpret_cast<uint2 *>(p) = o;
 }
+
+// ---- sums over a wavefront ----------------------------------------------------------
+template <int CTRL>
+__device__ __forceinline__ float bdh_dpp(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+// All lanes get the sum over the lanes l, l ^ 32, l ^ 16, l ^ 48: v + (its neighbour 32 away), then 16 away.
+__device__ __forceinline__ float bdh_sum_over_rows(float v) {
+  const unsigned int u = __float_as_uint(v);
+  const auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  const unsigned int w = __float_as_uint(v);
+  const auto b = __builtin_amdgcn_permlane16_swap(w, w, false, false);
+  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+// All lanes get the wave's sum: the bits of `for (o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o)` without its six trips
+// through LDS.  (A rotation of a row of sixteen by four reaches the lane 4 away in either half: those are equal by then.)
+__device__ __forceinline__ float bdh_wave_sum(float v) {
+  v = bdh_sum_over_rows(v);
+  v += bdh_dpp<0x128>(v);  // row rotated by 8
+  v += bdh_dpp<0x124>(v);  // by 4
+  v += bdh_dpp<0x4e>(v);   // lanes 2 apart
+  v += bdh_dpp<0xb1>(v);   // neighbours
+  return v;
+}
+// v / den for many v and one den, r = 1 / den rounded: one correction of v * r by its remainder gives the rounded quotient
+// (P. Markstein, IBM J. Res. Dev. 34, 1990) in three operations instead of the ten of a division.
+__device__ __forceinline__ float bdh_quotient(float v, float den, float r) {
+  const float q = v * r;
+  return __builtin_fmaf(__builtin_fmaf(-q, den, v), r, q);
+}
+// 0 + p[0] + p[step] + ... in index order (n the same for the wave), 16, 8 or 4 of the n values on their way at a time.
+template <int U, typename V>
+__device__ __forceinline__ void bdh_add_in_order(V &s, const V *p, long step) {
+  V t[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) t[u] = p[u * step];
+#pragma unroll
+  for (int u = 0; u < U; ++u) s += t[u];
+}
+template <typename V>
+__device__ __forceinline__ V bdh_sum_in_order(const V *p, long step, int n) {
+  V s = V{};
+  int g = 0;
+  for (; g + 16 <= n; g += 16) bdh_add_in_order<16>(s, p + g * step, step);
+  if (g + 8 <= n) { bdh_add_in_order<8>(s, p + g * step, step); g += 8; }
+  if (g + 4 <= n) { bdh_add_in_order<4>(s, p + g * step, step); g += 4; }
+  for (; g < n; ++g) s += p[g * step];
+  return s;
+}

@@ -60,35 +60,6 @@ __device__ __forceinline__ void wave_lds_order() {
   __builtin_amdgcn_wave_barrier();
 }
 
-// All lanes get the sum over the lanes l, l ^ 16, l ^ 32, l ^ 48.
-__device__ __forceinline__ float sum_over_rows(float v) {
-  const unsigned int u = __float_as_uint(v);
-  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-  const unsigned int w = __float_as_uint(v);
-  const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
-  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
-}
-template <int CTRL>
-__device__ __forceinline__ float dpp(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
-}
-// All lanes get the wave's sum: lanes 1 and 2 apart, the mirrored half row and row, then the four rows.
-__device__ __forceinline__ float wave_sum(float v) {
-  v += dpp<0xb1>(v);
-  v += dpp<0x4e>(v);
-  v += dpp<0x141>(v);
-  v += dpp<0x140>(v);
-  return sum_over_rows(v);
-}
-
-// v / den for many v and one den, r = 1 / den rounded: one correction of v * r by its remainder gives the rounded quotient
-// (P. Markstein, IBM J. Res. Dev. 34, 1990) in three operations instead of the ten of a division.
-__device__ __forceinline__ float quotient(float v, float den, float r) {
-  const float q = v * r;
-  return __builtin_fmaf(__builtin_fmaf(-q, den, v), r, q);
-}
-
 // LayerNorm of a row held by one wave, column j * 64 + lane in v[j] (src/model/bdh.rs:86-89); zero beyond d.
 template <int CJ>
 __device__ __forceinline__ void wave_layer_norm(float (&v)[CJ], int d) {
@@ -97,7 +68,7 @@ __device__ __forceinline__ void wave_layer_norm(float (&v)[CJ], int d) {
   float s = 0.0f;
 #pragma unroll
   for (int j = 0; j < CJ; ++j) s += j * 64 + lane < d ? v[j] : 0.0f;
-  const float mean = quotient(wave_sum(s), fd, rd);
+  const float mean = bdh_quotient(bdh_wave_sum(s), fd, rd);
   float q = 0.0f;
 #pragma unroll
   for (int j = 0; j < CJ; ++j) {
@@ -105,9 +76,9 @@ __device__ __forceinline__ void wave_layer_norm(float (&v)[CJ], int d) {
     v[j] = c;
     q += c * c;
   }
-  const float den = sqrtf(quotient(wave_sum(q), fd, rd) + kLnEps), r = 1.0f / den;
+  const float den = sqrtf(bdh_quotient(bdh_wave_sum(q), fd, rd) + kLnEps), r = 1.0f / den;
 #pragma unroll
-  for (int j = 0; j < CJ; ++j) v[j] = quotient(v[j], den, r);
+  for (int j = 0; j < CJ; ++j) v[j] = bdh_quotient(v[j], den, r);
 }
 
 // How the NW waves of a workgroup share rows of d <= DC floats and the NB neurons of its block.
@@ -201,9 +172,9 @@ struct Project {
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {  // over the lanes with the same columns: LPW apart
-      if (S::LPW <= 4) p[e] += dpp<0x124>(p[e]);  // rotations of a row of sixteen by four and eight
-      if (S::LPW <= 8) p[e] += dpp<0x128>(p[e]);
-      p[e] = sum_over_rows(p[e]);
+      if (S::LPW <= 4) p[e] += bdh_dpp<0x124>(p[e]);  // rotations of a row of sixteen by four and eight
+      if (S::LPW <= 8) p[e] += bdh_dpp<0x128>(p[e]);
+      p[e] = bdh_sum_over_rows(p[e]);
     }
     if (lane < S::LPW) *reinterpret_cast<float4 *>(&s_acc[wave_id()][lane * 4]) = make_float4(p[0], p[1], p[2], p[3]);
     __syncthreads();
@@ -382,7 +353,7 @@ __global__ __launch_bounds__(NW * 64, AHEAD || DC == 512 ? 2 : 4) void k_layer_p
       q_l = part == 0 ? mag * cosf(ph) : mag * sinf(ph);
       touch_l = true;
     } else {  // RoPE (src/model/attention.rs:305-321)
-      const float xo = dpp<0xb1>(xn);  // the other neuron of the pair
+      const float xo = bdh_dpp<0xb1>(xn);  // the other neuron of the pair
       touch_l = (xn != 0.0f) || (xo != 0.0f);
       if (touch_l) {
         const float raw = posf * freq;

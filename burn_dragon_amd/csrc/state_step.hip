@@ -927,8 +927,7 @@ __global__ __launch_bounds__(256) void k_step_finalize(const float *__restrict__
     const int c = j * 256 + tid;
     float s = 0.0f;
     if (c < d) {
-#pragma unroll 16
-      for (int g = 0; g < S; ++g) s += p[(long)g * d + c];
+      s = bdh_sum_in_order(p + c, d, S);
       out[(long)slice * out_slice_stride + c] = s;
       lsum += s;
     }
@@ -942,15 +941,12 @@ __global__ __launch_bounds__(256) void k_step_finalize(const float *__restrict__
   }
   if (!LN) return;
   // LayerNorm over d: mean, biased variance, (x-mean)/sqrt(var+eps)
-  __shared__ float s_part[4];
-  __shared__ float s_stat[2];
+  __shared__ float s_sum[4], s_sq[4];
   const int lane = tid & 63, wave = tid >> 6;
-  for (int o = 32; o > 0; o >>= 1) lsum += __shfl_xor(lsum, o);
-  if (lane == 0) s_part[wave] = lsum;
+  lsum = bdh_wave_sum(lsum);
+  if (lane == 0) s_sum[wave] = lsum;
   __syncthreads();
-  if (tid == 0) s_stat[0] = (s_part[0] + s_part[1] + s_part[2] + s_part[3]) / (float)d;
-  __syncthreads();
-  const float mean = s_stat[0];
+  const float mean = (s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3]) / (float)d;
   float lsq = 0.0f;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
@@ -960,13 +956,10 @@ __global__ __launch_bounds__(256) void k_step_finalize(const float *__restrict__
       lsq += t * t;
     }
   }
-  for (int o = 32; o > 0; o >>= 1) lsq += __shfl_xor(lsq, o);
+  lsq = bdh_wave_sum(lsq);
+  if (lane == 0) s_sq[wave] = lsq;
   __syncthreads();
-  if (lane == 0) s_part[wave] = lsq;
-  __syncthreads();
-  if (tid == 0) s_stat[1] = sqrtf((s_part[0] + s_part[1] + s_part[2] + s_part[3]) / (float)d + 1e-5f);
-  __syncthreads();
-  const float den = s_stat[1];
+  const float den = sqrtf((s_sq[0] + s_sq[1] + s_sq[2] + s_sq[3]) / (float)d + 1e-5f);
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int c = j * 256 + tid;
