@@ -463,39 +463,50 @@ __global__ __launch_bounds__(256) void k_relu_lowrank_direct(RlArgs g) {
 // added one after the other (the bits of the scalar chain again).  A wavefront owns 16 columns, so a chain of d steps takes
 // 8 cycles a step and row tile where the 32 x 32 instruction takes 32, and a few rows give four times the wavefronts: what
 // bounds it is the stream of the weights, every one of them copied to LDS once per 16 * RT rows.
-// Two stages in LDS: a third or fourth changed nothing.  us per call, the VALU and matrix-core kernels it took over from |
-// this: h*N = 1024, d = 256, 63 rows 7.6 | 6.1; 8192, 512, 48 rows 52.5 | 11.5; 32768, 256, 16 rows 29.7 | 8.4;
-// 131072, 512 (268 MB of weights), 16 rows 57.9 | 47.8, 32 rows 65.5 | 58.6.
-template <int RT>
+// Where the workgroups are few, it is the chain of waits: a stage's copies are NS - 1 stages ahead, its operands are read
+// into registers while those of the stage before are multiplied, and the gate is asked for at the start (us, before | now, D_x
+// and D_y of a decode step: 8 heads of 256, d = 512, 48 sequences 10.5 | 8.2; 4 heads of 4096, d = 256, 3 sequences 8.0 | 6.1).
+// us per call, the VALU and matrix-core kernels it took over from | this: 8192, 512, 48 rows 52.5 | 11.5; 32768, 256, 16 rows
+// 29.7 | 8.4; 131072, 512 (268 MB of weights), 16 rows 57.9 | 47.8, 32 rows 65.5 | 58.6.
+template <int RT, int NS>
 __global__ __launch_bounds__(256) void k_relu_lowrank_rows(RlArgs g) {
   typedef float f32x4 __attribute__((ext_vector_type(4)));
   constexpr int BM = 16 * RT, BN = 64, SK = 32;
   constexpr int STAGE = (BM + BN) * SK;
-  extern __shared__ __attribute__((aligned(1024))) float s_tiles[];  // two stages of A [BM][32], W [32][64]
-  const int tiles = g.mt * g.nt;
-  const long total = (long)g.h * tiles;
+  extern __shared__ __attribute__((aligned(1024))) float s_tiles[];  // NS stages of A [BM][32], W [32][64]
+  const int tiles = g.mt * g.nt, total = g.h * tiles;  // the launcher keeps the total within an int
   const int xcd = blockIdx.x & 7;
-  const long at = total * xcd / 8 + (blockIdx.x >> 3);
-  if (at >= total * (xcd + 1) / 8) return;
-  const int hh = (int)(at / tiles), tile = (int)(at % tiles);
-  const int m0 = (tile % g.mt) * BM, n0 = (tile / g.mt) * BN;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int lo = (int)((long)total * xcd / 8), hi = (int)((long)total * (xcd + 1) / 8);
+  const int at = lo + (int)(blockIdx.x >> 3);
+  if (at >= hi) return;
+  const int hh = at / tiles, tile = at - hh * tiles;
+  const int col_tile = tile / g.mt;
+  const int m0 = (tile - col_tile * g.mt) * BM, n0 = col_tile * BN;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const float *W = g.W + (long)hh * g.d * g.N;
+  // row m of A and of C: sequence, token
+  auto place = [&](int m, int &b, int &t) {
+    b = g.T == 1 ? m : m / g.T;
+    t = g.T == 1 ? 0 : m - b * g.T;
+  };
   // A: BM * 8 pieces of 16 bytes, W: 512; a piece of row r of A sits at place (piece ^ r / 2), one of k row k of W at place
   // (piece ^ 4 (k % 4)): the 4-byte reads below then cover the 64 banks once
   constexpr int CA = (BM * 8 + 255) / 256;
   const float *pa[CA], *pb[2];
 #pragma unroll
-  for (int c = 0; c < CA; ++c) {
-    const int piece = c * 256 + tid, row = piece >> 3, m = min(m0 + row, g.M - 1);
-    pa[c] = g.A + (long)(m / g.T) * g.a_outer + (long)hh * g.a_head + (long)(m % g.T) * g.d + ((piece & 7) ^ ((row >> 1) & 7)) * 4;
-  }
-#pragma unroll
   for (int c = 0; c < 2; ++c) {
     const int piece = c * 256 + tid, k = piece >> 4;
     pb[c] = W + (long)k * g.N + min(n0 + ((piece & 15) ^ ((k & 3) << 2)) * 4, g.N - 4);
   }
+#pragma unroll
+  for (int c = 0; c < CA; ++c) {
+    const int piece = c * 256 + tid, row = piece >> 3;
+    int b, t;
+    place(min(m0 + row, g.M - 1), b, t);
+    pa[c] = g.A + (long)b * g.a_outer + (long)hh * g.a_head + (long)t * g.d + ((piece & 7) ^ ((row >> 1) & 7)) * 4;
+  }
   const long b_step = (long)SK * g.N;
+  const bool carries_a = BM * 8 >= 256 || wave * 64 < BM * 8;  // does this wave copy pieces of A
   auto issue = [&](int buf) {
     float *s = s_tiles + buf * STAGE;
 #pragma unroll
@@ -505,41 +516,66 @@ __global__ __launch_bounds__(256) void k_relu_lowrank_rows(RlArgs g) {
     }
 #pragma unroll
     for (int c = 0; c < CA; ++c) {
-      if (BM * 8 >= 256 || wave * 64 < BM * 8) bdh_copy_to_lds(pa[c], s + (c * 256 + wave * 64) * 4);
+      if (carries_a) bdh_copy_to_lds(pa[c], s + (c * 256 + wave * 64) * 4);
       pa[c] += SK;
     }
   };
+  // where element e of row tile i of this lane goes (element e of lane l: row = (l/16)*4 + e, column = l%16), its gate
+  const int r = lane & 15, q = lane >> 4;
+  const int col = n0 + wave * 16 + r;
+  const int stages = g.d / SK;
+  for (int s = 0; s < NS - 1 && s < stages; ++s) issue(s);
+  // behind the first copies: these values are needed last, and their trip to memory is the chain's to hide
+  float gv[RT][4];
+  if (g.gate) {
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        int b, t;
+        place(min(m0 + i * 16 + q * 4 + e, g.M - 1), b, t);
+        gv[i][e] = g.gate[(((long)b * g.h + hh) * g.T + t) * g.N + min(col, g.N - 1)];
+      }
+  }
   f32x4 acc[RT];
 #pragma unroll
   for (int i = 0; i < RT; ++i) acc[i] = (f32x4)(0.0f);
-  const int r = lane & 15, q = lane >> 4;
-  issue(0);
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  int cur = 0;
-  for (int k0 = 0; k0 < g.d; k0 += SK) {
-    if (k0 + SK < g.d) issue(cur ^ 1);  // lands while the matrix cores work on this stage
-    const float *sa = s_tiles + cur * STAGE, *sb = sa + BM * SK;
-    float fa[SK / 4][RT], fb[SK / 4];
+  // The operands of a stage are read into registers while those of the stage before are multiplied.
+  float fa[2][SK / 4][RT], fb[2][SK / 4];
+  auto read = [&](int s, int into) {
+    const float *sa = s_tiles + s % NS * STAGE, *sb = sa + BM * SK;
 #pragma unroll
     for (int c = 0; c < SK / 4; ++c) {
-      fb[c] = sb[(4 * c + q) * BN + ((wave * 16 + r) ^ (q << 4))];
+      fb[into][c] = sb[(4 * c + q) * BN + ((wave * 16 + r) ^ (q << 4))];
 #pragma unroll
       for (int i = 0; i < RT; ++i) {
         const int row = i * 16 + r;
-        fa[c][i] = sa[row * SK + (c ^ ((row >> 1) & 7)) * 4 + q];
+        fa[into][c][i] = sa[row * SK + (c ^ ((row >> 1) & 7)) * 4 + q];
       }
     }
+  };
+  auto multiply = [&](int from) {
 #pragma unroll
     for (int c = 0; c < SK / 4; ++c)
 #pragma unroll
-      for (int i = 0; i < RT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[c][i], fb[c], acc[i], 0, 0, 0);
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    cur ^= 1;
+      for (int i = 0; i < RT; ++i)
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[from][c][i], fb[from][c], acc[i], 0, 0, 0);
+  };
+  auto step = [&](int s, int into) {
+    const int later = min(NS - 2, stages - 1 - s);
+    if (carries_a) bdh_wait_for_stage<2 + CA, NS - 2>(later);
+    else bdh_wait_for_stage<2, NS - 2>(later);
+    __syncthreads();  // stage s is there for every wave, and stage s - 1 has been read: its place takes stage s + NS - 1
+    if (s + NS - 1 < stages) issue((s + NS - 1) % NS);
+    read(s, into);
+    if (s > 0) multiply(into ^ 1);
+  };
+  for (int s = 0; s < stages; s += 2) {  // two at a time: the registers have fixed names
+    step(s, 0);
+    if (s + 1 < stages) step(s + 1, 1);
   }
-  // element e of lane l: row = (l/16)*4 + e, column = l%16
-  const int col = n0 + wave * 16 + r;
+  if (stages & 1) multiply(0);
+  else multiply(1);
   if (col >= g.N) return;
   const float bv = g.bias ? g.bias[(long)hh * g.N + col] : 0.0f;
   float mk = 1.0f;
@@ -548,31 +584,20 @@ __global__ __launch_bounds__(256) void k_relu_lowrank_rows(RlArgs g) {
     mk = (blk < g.n_blocks && g.mask[blk]) ? 1.0f : 0.0f;
   }
 #pragma unroll
-  for (int i = 0; i < RT; ++i) {
-    const int row = m0 + i * 16 + q * 4;
-    int b = row / g.T, t = row - b * g.T;
-    long o[4];
-    float gv[4];
+  for (int i = 0; i < RT; ++i)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      o[e] = row + e < g.M ? (((long)b * g.h + hh) * g.T + t) * g.N + col : -1;
-      if (++t == g.T) { t = 0; ++b; }
-    }
-    if (g.gate) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) gv[e] = g.gate[o[e] >= 0 ? o[e] : 0];
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
+      const int m = m0 + i * 16 + q * 4 + e;
       float pv = acc[i][e];
       if (g.bias) pv = pv + bv;
       if (g.thr != 0.0f) pv = pv - g.thr;
       float y = pv > 0.0f ? pv : 0.0f;
       if (g.mask) y = y * mk;
-      if (g.gate) y = gv[e] * y;
-      if (o[e] >= 0) g.C[o[e]] = y;
+      if (g.gate) y = gv[i][e] * y;
+      int b, t;
+      place(m, b, t);
+      if (m < g.M) g.C[(((long)b * g.h + hh) * g.T + t) * g.N + col] = y;
     }
-  }
 }
 
 // any d and N: 64 x 64 tiles staged through registers, with checks
@@ -983,9 +1008,15 @@ int bdh_launch_relu_lowrank_gemm(bdh_ctx *ctx, const ReluLowrankParams &p, const
   const dim3 grid((unsigned)(8 * ((total + 7) / 8)));
 #define BDH_RLD(KERNEL_, ROWS_, COLS_) \
   hipLaunchKernelGGL((KERNEL_), grid, dim3(256), 2 * (ROWS_ + COLS_) * 32 * sizeof(float), ctx->stream, g)
-  if (rt == 1) BDH_RLD(k_relu_lowrank_rows<1>, 16, 64);
-  else if (rt == 2) BDH_RLD(k_relu_lowrank_rows<2>, 32, 64);
-  else if (rt == 4) BDH_RLD(k_relu_lowrank_rows<4>, 64, 64);
+  // Stages of the ring: more copies in flight where the workgroups are too few to cover each other's trips, fewer where LDS
+  // decides how many of them a CU holds (us, two | four stages: 96 workgroups 9.3 | 8.3, 256 6.8 | 6.1, 1024 13.8 | 15.0).
+#define BDH_RLR(RT_, NS_) \
+  hipLaunchKernelGGL((k_relu_lowrank_rows<RT_, NS_>), grid, dim3(256), NS_ * (16 * RT_ + 64) * 32 * sizeof(float), ctx->stream, g)
+  if (rt == 1 && total <= 2 * n_cu) BDH_RLR(1, 4);
+  else if (rt == 1) BDH_RLR(1, 2);
+  else if (rt == 2) BDH_RLR(2, 3);
+  else if (rt == 4) BDH_RLR(4, 2);
+#undef BDH_RLR
   else if (big) BDH_RLD((k_relu_lowrank_direct<128, 128>), 128, 128);
   else if (direct) BDH_RLD((k_relu_lowrank_direct<64, 64>), 64, 64);
   else hipLaunchKernelGGL(k_relu_lowrank_gemm, grid, dim3(256), 0, ctx->stream, g);

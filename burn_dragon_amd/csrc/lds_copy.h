@@ -16,3 +16,18 @@ __device__ __forceinline__ void bdh_copy_to_lds(const void *src, void *dst) {
   const unsigned int at = __builtin_amdgcn_readfirstlane((unsigned int)(uintptr_t)(bdh_lds_ptr_t)dst);
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"{m0}"(at), "v"(src) : "memory");
 }
+
+// Waits until no more than `later` stages of COPIES copies each, issued by this wavefront after the stage that it needs, are
+// still on their way (at most MOST of them are ever asked about).  Loads come back in the order of their issue.
+template <int COPIES, int MOST>
+__device__ __forceinline__ void bdh_wait_for_stage(int later) {
+  if constexpr (MOST > 0) {
+    if (later >= MOST) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(COPIES * MOST) : "memory");
+      return;
+    }
+    bdh_wait_for_stage<COPIES, MOST - 1>(later);
+  } else {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+}
