@@ -241,7 +241,7 @@ __global__ __launch_bounds__(NTHR) void k_relu_lowrank_row1(RowArgs a, int d, co
           const float tx = vals[j].x - mean, ty = vals[j].y - mean, tz = vals[j].z - mean, tw = vals[j].w - mean;
           q += (tx * tx + ty * ty) + (tz * tz + tw * tw);
         }
-      const float den = sqrtf(wave_sum(q) / (float)d + kLnEps);
+      const float den = sqrtf(bdh_wave_sum(q) / (float)d + kLnEps);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         vals[j].x = (vals[j].x - mean) / den; vals[j].y = (vals[j].y - mean) / den;
@@ -610,16 +610,17 @@ __global__ __launch_bounds__(256) void k_decoder_partial(const float *__restrict
 // many sequences and a large E, one chain per block that runs 0, 8, 1, 9, ..., 7, 15 through each 16.)
 // A workgroup takes the k-blocks [blk * bpw, +bpw) and adds their sums in order: bpw is a sixteenth of the blocks, as
 // k_decoder_finalize would group them, or one.
-// Tile 16 * RT x 64, copied straight to LDS 32 k at a time into two buffers in turn.  What bounds it: a few workgroups per
-// CU, each a chain of KB / 32 trips to the L2 (48 sequences, K = 2048, d = 512: 6.3 us; the same product in parts of K from
-// split bf16 terms took 8.0).
-template <int RT, bool SPLIT>
+// Tile 16 * RT x 64, copied straight to LDS 32 k at a time into a ring of NS stages, the operands of a stage read into registers
+// while those of the stage before are multiplied.  What bounds it: the trips to memory of a few workgroups per CU, which is
+// why the copies run NS - 1 stages ahead (two stages | now, us: 48 sequences, K = 2048, d = 512 6.3 | 5.6; 60, 16384, 256
+// 30 | 19; 60, 32768, 512 65 | 36; 24, 131072, 512 189 | 71).
+template <int RT, bool SPLIT, int NS>
 __global__ __launch_bounds__(256) void k_decoder_rows(const float *__restrict__ xy, const float *__restrict__ E,
                                                       float *__restrict__ partial, long K, int d, int KB, int bpw, int M) {
   typedef float f32x4 __attribute__((ext_vector_type(4)));
   constexpr int BM = 16 * RT, BN = 64, SK = 32, STAGE = (BM + BN) * SK, NA = SPLIT ? 1 : 4;
-  extern __shared__ __attribute__((aligned(1024))) float s_tiles[];  // two stages of xy [BM][32], E [32][64]
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  extern __shared__ __attribute__((aligned(1024))) float s_tiles[];  // NS stages of xy [BM][32], E [32][64]
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n0 = blockIdx.x * BN, m0 = blockIdx.y * BM;
   const long k_lo = (long)blockIdx.z * bpw * KB, k_hi = min(K, k_lo + (long)bpw * KB);
   // piece c of 16 bytes of row r of xy sits at place c ^ r / 2; of a row of E at place c ^ 4 x, x = which of the four k of
@@ -641,6 +642,7 @@ __global__ __launch_bounds__(256) void k_decoder_rows(const float *__restrict__ 
     pb[c] = E + (k_lo + kb[c]) * d + min(n0 + ((piece & 15) ^ (k_turn(kb[c]) << 2)) * 4, d - 4);
   }
   const float *zero = reinterpret_cast<const float *>(&g_zero_f4);
+  const bool carries_xy = BM * 8 >= 256 || wave * 64 < BM * 8;  // does this wave copy pieces of xy
   auto issue = [&](long k0, int buf) {  // rows of E and values of xy beyond K are zero (K % 4 == 0)
     float *s = s_tiles + buf * STAGE;
 #pragma unroll
@@ -650,8 +652,7 @@ __global__ __launch_bounds__(256) void k_decoder_rows(const float *__restrict__ 
     }
 #pragma unroll
     for (int c = 0; c < CA; ++c) {
-      if (BM * 8 >= 256 || wave * 64 < BM * 8)
-        bdh_copy_to_lds(k0 + ka[c] < K ? pa[c] : zero, s + (c * 256 + wave * 64) * 4);
+      if (carries_xy) bdh_copy_to_lds(k0 + ka[c] < K ? pa[c] : zero, s + (c * 256 + wave * 64) * 4);
       pa[c] += SK;
     }
   };
@@ -663,34 +664,36 @@ __global__ __launch_bounds__(256) void k_decoder_rows(const float *__restrict__ 
     for (int a = 0; a < NA; ++a) acc[a][i] = (f32x4)(0.0f);
   }
   const int r = lane & 15, q = lane >> 4;
-  issue(k_lo, 0);
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  int cur = 0;
-  for (long k0 = k_lo; k0 < k_hi; k0 += SK) {
-    if (k0 + SK < k_hi) issue(k0 + SK, cur ^ 1);  // lands while the matrix cores work on this stage
-    const float *sa = s_tiles + cur * STAGE, *sb = sa + BM * SK;
-    float fa[2][4][RT], fb[2][4];
+  // The operands of a stage are read into registers while those of the stage before are multiplied.
+  const int stages = (int)((k_hi - k_lo + SK - 1) / SK), per_block = KB / SK;  // KB % 32 == 0
+  float fa[2][2][4][RT], fb[2][2][4];
+  auto read = [&](int st, int into) {
+    const float *sa = s_tiles + st % NS * STAGE, *sb = sa + BM * SK;
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
       for (int w = 0; w < 4; ++w) {
         const int k = 16 * s + (SPLIT ? 2 * w + (q >> 1) + 8 * (q & 1) : 4 * q + w);
-        fb[s][w] = sb[k * BN + ((wave * 16 + r) ^ (q << 4))];
+        fb[into][s][w] = sb[k * BN + ((wave * 16 + r) ^ (q << 4))];
 #pragma unroll
         for (int i = 0; i < RT; ++i) {
           const int row = i * 16 + r;
-          fa[s][w][i] = sa[row * SK + ((k >> 2) ^ ((row >> 1) & 7)) * 4 + (k & 3)];
+          fa[into][s][w][i] = sa[row * SK + ((k >> 2) ^ ((row >> 1) & 7)) * 4 + (k & 3)];
         }
       }
+  };
+  int in_block = 0;
+  auto multiply = [&](int from, bool last) {
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
       for (int w = 0; w < 4; ++w)
 #pragma unroll
         for (int i = 0; i < RT; ++i)
-          acc[SPLIT ? 0 : w][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[s][w][i], fb[s][w], acc[SPLIT ? 0 : w][i], 0, 0, 0);
-    if ((k0 + SK - k_lo) % KB == 0 || k0 + SK >= k_hi) {  // a k-block ends (KB % 32 == 0)
+          acc[SPLIT ? 0 : w][i] =
+              __builtin_amdgcn_mfma_f32_16x16x4f32(fa[from][s][w][i], fb[from][s][w], acc[SPLIT ? 0 : w][i], 0, 0, 0);
+    if (++in_block == per_block || last) {  // a k-block ends
+      in_block = 0;
 #pragma unroll
       for (int i = 0; i < RT; ++i) {
 #pragma unroll
@@ -703,10 +706,23 @@ __global__ __launch_bounds__(256) void k_decoder_rows(const float *__restrict__ 
         for (int a = 0; a < NA; ++a) acc[a][i] = (f32x4)(0.0f);
       }
     }
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    cur ^= 1;
+  };
+  auto step = [&](int st, int into) {
+    const int later = min(NS - 2, stages - 1 - st);
+    if (carries_xy) bdh_wait_for_stage<2 + CA, NS - 2>(later);
+    else bdh_wait_for_stage<2, NS - 2>(later);
+    __syncthreads();  // stage st is there for every wave, and the one before has been read: its place takes stage st + NS - 1
+    if (st + NS - 1 < stages) issue(k_lo + (long)(st + NS - 1) * SK, (st + NS - 1) % NS);
+    read(st, into);
+    if (st > 0) multiply(into ^ 1, false);
+  };
+  for (int st = 0; st < NS - 1 && st < stages; ++st) issue(k_lo + (long)st * SK, st);
+  for (int st = 0; st < stages; st += 2) {  // two at a time: the registers have fixed names
+    step(st, 0);
+    if (st + 1 < stages) step(st + 1, 1);
   }
+  if (stages & 1) multiply(0, true);
+  else multiply(1, true);
   // element e of lane l: row = (l/16)*4 + e, column = l%16
   const int col = n0 + wave * 16 + r;
   if (col >= d) return;
@@ -850,7 +866,7 @@ __global__ __launch_bounds__(1024) void k_decoder_finalize(const float *__restri
   __shared__ float s_grp[16][1024];
   __shared__ float s_best[4];
   __shared__ int s_arg[4];
-  const int m = blockIdx.x, lane = threadIdx.x & 63, grp = threadIdx.x >> 6;
+  const int m = blockIdx.x, lane = threadIdx.x & 63, grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int per = (KBN + 15) >> 4;
   const int kb0 = min(KBN, grp * per), kb1 = min(KBN, kb0 + per);
   // the residual row is fetched while the partials are summed: it was written by another
@@ -864,22 +880,9 @@ __global__ __launch_bounds__(1024) void k_decoder_finalize(const float *__restri
   for (int j = 0; j < 4; ++j) {
     const int c = (j * 64 + lane) * 4;  // d % 4 == 0
     if (c < d) {
-      float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-      int kb = kb0;
-      for (; kb + 16 <= kb1; kb += 16) {
-        float4 t[16];
-#pragma unroll
-        for (int u = 0; u < 16; ++u) t[u] = *reinterpret_cast<const float4 *>(partial + ((long)(kb + u) * M + m) * d + c);
-#pragma unroll
-        for (int u = 0; u < 16; ++u) {
-          v.x += t[u].x; v.y += t[u].y; v.z += t[u].z; v.w += t[u].w;
-        }
-      }
-      for (; kb < kb1; ++kb) {
-        const float4 t = *reinterpret_cast<const float4 *>(partial + ((long)kb * M + m) * d + c);
-        v.x += t.x; v.y += t.y; v.z += t.z; v.w += t.w;
-      }
-      *reinterpret_cast<float4 *>(&s_grp[grp][c]) = v;
+      typedef float Quad __attribute__((ext_vector_type(4)));
+      const Quad q = bdh_sum_in_order(reinterpret_cast<const Quad *>(partial + ((long)kb0 * M + m) * d + c), (long)M * d / 4, kb1 - kb0);
+      *reinterpret_cast<Quad *>(&s_grp[grp][c]) = q;
     }
   }
   __syncthreads();
@@ -900,11 +903,7 @@ __global__ __launch_bounds__(1024) void k_decoder_finalize(const float *__restri
     }
     vals[j] = v;
   }
-  auto wave_sum = [](float v) {
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
-  };
-  float mean = wave_sum(s) / (float)d;
+  float mean = bdh_wave_sum(s) / (float)d;
   float q = 0.0f;
 #pragma unroll
   for (int j = 0; j < 16; ++j)
@@ -912,7 +911,7 @@ __global__ __launch_bounds__(1024) void k_decoder_finalize(const float *__restri
       const float t = vals[j] - mean;
       q += t * t;
     }
-  float den = sqrtf(wave_sum(q) / (float)d + kLnEps);
+  float den = sqrtf(bdh_wave_sum(q) / (float)d + kLnEps);
   s = 0.0f;
 #pragma unroll
   for (int j = 0; j < 16; ++j) {
@@ -923,7 +922,7 @@ __global__ __launch_bounds__(1024) void k_decoder_finalize(const float *__restri
       s += vals[j];
     }
   }
-  mean = wave_sum(s) / (float)d;
+  mean = bdh_wave_sum(s) / (float)d;
   q = 0.0f;
 #pragma unroll
   for (int j = 0; j < 16; ++j)
@@ -931,7 +930,7 @@ __global__ __launch_bounds__(1024) void k_decoder_finalize(const float *__restri
       const float t = vals[j] - mean;
       q += t * t;
     }
-  den = sqrtf(wave_sum(q) / (float)d + kLnEps);
+  den = sqrtf(bdh_wave_sum(q) / (float)d + kLnEps);
 #pragma unroll
   for (int j = 0; j < 16; ++j) {
     const int c = j * 64 + lane;
@@ -988,10 +987,6 @@ __global__ __launch_bounds__(256) void k_decoder_finalize_rows(const float *__re
       s += v;
     }
   }
-  auto wave_sum = [](float v) {
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
-  };
   auto spread = [&](float mean) {  // sqrt(var + eps)
     float q = 0.0f;
 #pragma unroll
@@ -1000,9 +995,9 @@ __global__ __launch_bounds__(256) void k_decoder_finalize_rows(const float *__re
         const float t = vals[j] - mean;
         q += t * t;
       }
-    return sqrtf(wave_sum(q) / (float)d + kLnEps);
+    return sqrtf(bdh_wave_sum(q) / (float)d + kLnEps);
   };
-  float mean = wave_sum(s) / (float)d;
+  float mean = bdh_wave_sum(s) / (float)d;
   float den = spread(mean);
   s = 0.0f;
 #pragma unroll
@@ -1012,7 +1007,7 @@ __global__ __launch_bounds__(256) void k_decoder_finalize_rows(const float *__re
       vals[j] = res[j] + mlp;
       s += vals[j];
     }
-  mean = wave_sum(s) / (float)d;
+  mean = bdh_wave_sum(s) / (float)d;
   den = spread(mean);
 #pragma unroll
   for (int j = 0; j < 16; ++j)
@@ -1303,30 +1298,40 @@ static void launch_decoder_finalize(bdh_ctx *ctx, const float *partial, int KBN,
   }
 }
 
-// The whole encoder of a batch of decoding sequences by k_decoder_rows.  The second stage adds the k-blocks in sixteen
-// groups; a workgroup adds up a whole group where the groups alone give every CU a workgroup.  The tile: 16 rows while that
-// leaves at most four workgroups for every CU, the chain of one tile being what counts; else 32, or 64 for more rows than
-// that, so that E passes fewer times.
+// The whole encoder of a batch of decoding sequences by k_decoder_rows.  In the form with the VALU kernel's bits the second
+// stage adds the k-blocks in sixteen groups, and a workgroup adds up a whole group where the groups alone give every CU a
+// workgroup; the tile is 16 rows while that leaves at most four workgroups for every CU, the chain of one tile being what
+// counts, else 32, or 64 for more rows than that, so that E passes fewer times.  In the other form (one chain per k-block of
+// 1024) a workgroup takes as many k-blocks as leave four workgroups for every CU, and at most 64 parts for the second stage;
+// 32 rows a tile where those tiles give every CU two (us of both kernels: 24 sequences, K = 131072, d = 512, 32 rows, two
+// k-blocks 71 + 8, one 75 + 11, eight with 16 rows 131 + 6; 60, 32768, 512, one 36 + 7, two with 16 rows 47 + 6; 48, 131072,
+// 512, 32 rows, two 110, 64 rows, two 114).
 static int launch_decoder_rows(bdh_ctx *ctx, int M, long K, int d, int KB, bool split, const float *xy, const float *decoder,
                                float *cur, const DecoderHead *head) {
   const long n_cu = ctx->n_cu > 0 ? ctx->n_cu : 256;
   const int KBN = (int)((K + KB - 1) / KB), per = (KBN + 15) / 16;
   auto tiles = [&](int rows) { return (long)((d + 63) / 64) * ((M + rows - 1) / rows); };
-  const int bpw = tiles(16) * ((KBN + per - 1) / per) >= n_cu ? per : 1;
+  int bpw, rt;
+  if (split) {
+    rt = M > 16 && tiles(32) * KBN >= 2 * n_cu ? 2 : 1;
+    bpw = (int)std::max<long>((KBN + 63) / 64, std::min<long>(per, tiles(16 * rt) * KBN / (4 * n_cu)));
+  } else {
+    bpw = tiles(16) * ((KBN + per - 1) / per) >= n_cu ? per : 1;
+    rt = tiles(16) * ((KBN + bpw - 1) / bpw) <= 4 * n_cu ? 1 : M <= 32 ? 2 : 4;
+  }
   const int parts = (KBN + bpw - 1) / bpw;
-  const int rt = tiles(16) * parts <= 4 * n_cu ? 1 : M <= 32 ? 2 : 4;
   int rc = bdh_ws_reserve(ctx, sizeof(float) * (size_t)parts * M * d);
   if (rc != BDH_OK) return rc;
   float *partial = static_cast<float *>(ctx->ws);
   const dim3 grid((d + 63) / 64, (M + 16 * rt - 1) / (16 * rt), parts);
   if (grid.y > 65535 || grid.z > 65535) return bdh_fail(ctx, BDH_E_SHAPE, "grid too large (%d rows, %d parts)", M, parts);
-#define BDH_DR(RT_, SPLIT_)                                                                                            \
-  hipLaunchKernelGGL((k_decoder_rows<RT_, SPLIT_>), grid, dim3(256), 2 * (16 * RT_ + 64) * 32 * sizeof(float), ctx->stream, \
-                     xy, decoder, partial, K, d, KB, bpw, M)
+#define BDH_DR(RT_, SPLIT_, NS_)                                                                                       \
+  hipLaunchKernelGGL((k_decoder_rows<RT_, SPLIT_, NS_>), grid, dim3(256), NS_ * (16 * RT_ + 64) * 32 * sizeof(float), \
+                     ctx->stream, xy, decoder, partial, K, d, KB, bpw, M)
   if (split) {
-    if (rt == 1) BDH_DR(1, true); else if (rt == 2) BDH_DR(2, true); else BDH_DR(4, true);
+    if (rt == 1) BDH_DR(1, true, 4); else BDH_DR(2, true, 3);
   } else {
-    if (rt == 1) BDH_DR(1, false); else if (rt == 2) BDH_DR(2, false); else BDH_DR(4, false);
+    if (rt == 1) BDH_DR(1, false, 4); else if (rt == 2) BDH_DR(2, false, 3); else BDH_DR(4, false, 3);
   }
 #undef BDH_DR
   BDH_LAUNCH_CHECK(ctx, "k_decoder_rows");

@@ -1,6 +1,7 @@
-"""The two-launch layer of a decode step at the sizes where it can go wrong: row widths at the edges of the three kernel
-widths (128, 256, 512), one and many blocks of neurons, the smallest and largest number of them, blocks of 32 and of 64,
-vocabularies read four columns at a time and one at a time, weights that are not 16-byte aligned."""
+"""The kernels of a decode step at the sizes where they can go wrong.  The two-launch layer: row widths at the edges of the
+three kernel widths (128, 256, 512), one and many blocks of neurons, the smallest and largest number of them, blocks of 32
+and of 64, vocabularies read four columns at a time and one at a time, weights that are not 16-byte aligned.  The projections
+and the encoder of a few rows: rings of copies that are longer than the work, and tiles that end inside."""
 import pytest
 import torch
 
@@ -74,3 +75,59 @@ def test_two_launch_layer_edges(state, rotary, lazy, d, h, N, V, B, aligned):
     assert rel_err(states[0].storage.float(), states[1].storage.float()) < (1e-5 if state == "f32" else 3 * 2.0 ** -8)
     if lazy:
         assert torch.equal(states[0].stamps, states[1].stamps)
+
+
+@pytest.mark.parametrize("d", [32, 64, 96, 160, 512])
+@pytest.mark.parametrize("B,T,h,N", [(2, 1, 3, 4), (5, 3, 2, 60), (17, 1, 3, 68), (33, 1, 1, 260), (63, 1, 2, 64),
+                                     (20, 1, 2, 40960), (40, 1, 1, 66000)])
+def test_projection_rings_keep_the_bits_of_the_scalar_chain(d, B, T, h, N):
+    """1 to 16 stages of 32 k through rings of 2, 3 and 4; row tiles of 16, 32 and 64; bias, mask and gate: the bits of the
+    thread-per-column kernel, which adds the same products in the same order."""
+    import burn_dragon_amd as bda
+    from burn_dragon_amd.kernel import relu_lowrank
+
+    g = torch.Generator(device=DEV).manual_seed(d + N)
+    x = torch.randn((B, h, T, d), device=DEV, generator=g)
+    w = torch.randn((h, d, N), device=DEV, generator=g)
+    bias = torch.randn((h, 1, N), device=DEV, generator=g)
+    gate = torch.randn((B, h, T, N), device=DEV, generator=g)
+    layout = bda.BlockPattern1d.from_blocks(16, list(range(0, (N + 15) // 16, 2)))
+    ctx = bda.ffi.default_context(0)
+    call = lambda: relu_lowrank.fused_forward(x, w, bias, 0.25, layout, gate=gate)
+    try:
+        ctx.set_option("relu_lowrank.row", 0)
+        got = call()
+        ctx.set_option("relu_lowrank.mfma_rows", 0)
+        assert torch.equal(got, call())
+    finally:
+        ctx.set_option("relu_lowrank.mfma_rows", 2)
+        ctx.set_option("relu_lowrank.row", 1)
+
+
+@pytest.mark.parametrize("B,mult", [(17, 130), (33, 64), (16, 64)])
+def test_encoder_of_a_batch_in_parts_of_several_k_blocks(B, mult):
+    """The form with one chain per k-block of 1024, d = 512: 32 rows a tile with two k-blocks (the last part holding one) and
+    with one k-block a workgroup, 16 rows a tile.  Against the VALU kernel: 2^-24 per step of a few dozen steps, 1e-5."""
+    import burn_dragon_amd as bda
+
+    d, V = 512, 64
+    cfg = bda.BDHConfig(n_layer=1, n_embd=d, n_head=1, mlp_internal_dim_multiplier=mult, vocab_size=V)
+    cfg.fused_kernels.set_rotary_embedding(bda.RotaryEmbedding.ALIBI)
+    model = bda.BDH(cfg, DEV, seed=3)
+    g = torch.Generator(device=DEV).manual_seed(B)
+    tokens = torch.randint(0, V, (B, 1), device=DEV, generator=g)
+    rho = torch.empty((1, B, 1, mult * d, d), device=DEV)
+    rho.normal_(0.0, 0.1, generator=g)
+    ctx = bda.ffi.default_context(0)
+    logits = []
+    try:
+        for rows in (-16, 1 << 30):
+            ctx.set_option("decoder.splitk_rows", rows)
+            state = model.init_state()
+            state.position, state.storage = 9, rho.clone()
+            state.layers[0].rho = state.storage[0]
+            logits.append(model.forward_with_state(tokens, state))
+    finally:
+        ctx.set_option("decoder.splitk_rows", 24)
+    assert not torch.equal(logits[0], logits[1])
+    assert rel_err(logits[0], logits[1]) < 1e-5
