@@ -48,7 +48,7 @@ struct GemmF32 {
 };
 constexpr int GEMM_STORE = 0, GEMM_SCORES = 1, GEMM_NORM = 2;
 
-// How a product is cut: tile (0: 128 x 128, 1: 64 x 64, 2: 32 x 128) and the number of parts of K.
+// How a product is cut: tile (0: 128 x 128, 1: 64 x 64, 2: 32 x 128, 3: 128 x 256) and the number of parts of K.
 struct GemmPlan {
   int tile = 0, ks = 1;
 };

@@ -134,16 +134,20 @@ struct Tile {
   }
 };
 
-// BM x BN tile per workgroup of WM x WN wavefronts.  LDS holds one stage (192 bytes per tile row and column: 48 KiB at
+// BM x BN tile per workgroup of WM x WN wavefronts.  With four wavefronts LDS holds one stage (192 bytes per tile row and column: 48 KiB at
 // 128 x 128; the registers allow two workgroups per CU); the next stage's loads are in flight in registers while this one is multiplied,
 // and the other workgroups of the CU fill the two barriers.  What bounds it: at 128 x 128 a wavefront spends 1536 cycles
 // of a stage in matrix instructions, 700 in the split and the LDS pipe moves 144 KiB.
+// Eight wavefronts (TURNS): two stages in LDS, two on every SIMD (wavefronts w and w + 4).  Between two barriers one of the
+// two multiplies the stage that is there and then splits the next one into the other buffer, its partner does the two in the
+// other order: the conversions of one run under the matrix instructions of the other.
 template <int BM, int BN, int WM, int WN, bool AK, bool BK, int EPI>
 __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_f32(GemmF32 g) {
+  constexpr bool TURNS = WM * WN == 8;
   constexpr int NT = WM * WN * 64;
   constexpr int MI = BM / WM / 32, NJ = BN / WN / 32;
-  __shared__ __attribute__((aligned(16))) unsigned char s_a[3 * BM * 64];
-  __shared__ __attribute__((aligned(16))) unsigned char s_b[3 * BN * 64];
+  __shared__ __attribute__((aligned(16))) unsigned char s_a[(TURNS ? 2 : 1) * 3 * BM * 64];
+  __shared__ __attribute__((aligned(16))) unsigned char s_b[(TURNS ? 2 : 1) * 3 * BN * 64];
   __shared__ float s_norm[EPI == GEMM_NORM ? BM : 1];
   // XCD-aware mapping: workgroup ids are dealt round-robin to the 8 XCDs, so ids with the same (id % 8) share an L2.
   // Each XCD takes one contiguous eighth of the (slice, part of K, tile) list: neighbouring tiles reuse their operand
@@ -167,7 +171,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_f32(GemmF32 g) {
     tj = tile - ti * g.nt;
   }
   const int m0 = ti * BM, n0 = tj * BN;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN;
   const long s1 = slice / g.mod, s2 = slice % g.mod;
   const float *A = g.A + s1 * g.a_s1 + s2 * g.a_s2;
@@ -227,20 +231,22 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_f32(GemmF32 g) {
           for (int q = 0; q < 8; ++q) rs[c] += fabsf(ta.v[c][q]);
       }
     };
-    auto multiply = [&]() {
+    auto multiply = [&](int buf) {
+      const unsigned char *sa = s_a + buf * 3 * BM * 64, *sb = s_b + buf * 3 * BN * 64;
       // lane (r = lane % 32, half = lane / 32) feeds chunk 2 * step + half of its row
       const int r = lane & 31, half = lane >> 5;
 #pragma unroll
       for (int step = 0; step < 2; ++step) {
+        if (TURNS) __builtin_amdgcn_sched_barrier(0);  // one step's fragments at a time
         bf16x8 fa[3][MI], fb[3][NJ];
 #pragma unroll
         for (int t = 0; t < 3; ++t) {
 #pragma unroll
           for (int i = 0; i < MI; ++i)
-            fa[t][i] = *reinterpret_cast<const bf16x8 *>(s_a + t * BM * 64 + chunk_at(wm * (BM / WM) + i * 32 + r, 2 * step + half));
+            fa[t][i] = *reinterpret_cast<const bf16x8 *>(sa + t * BM * 64 + chunk_at(wm * (BM / WM) + i * 32 + r, 2 * step + half));
 #pragma unroll
           for (int j = 0; j < NJ; ++j)
-            fb[t][j] = *reinterpret_cast<const bf16x8 *>(s_b + t * BN * 64 + chunk_at(wn * (BN / WN) + j * 32 + r, 2 * step + half));
+            fb[t][j] = *reinterpret_cast<const bf16x8 *>(sb + t * BN * 64 + chunk_at(wn * (BN / WN) + j * 32 + r, 2 * step + half));
         }
         constexpr int TA[6] = {2, 0, 1, 1, 0, 0}, TB[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
@@ -259,22 +265,52 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_f32(GemmF32 g) {
       // loop is straight-line code (with a branch among them, loads are waited for where they are issued)
       ta.template load<TAIL>((hi - 1) * FK, K, lda);
       tb.template load<TAIL>((hi - 1) * FK, K, ldb);
-      auto stage_in = [&](int kb) {
+      auto put = [&](int kb, int buf) {
         scaled(kb);
-        __syncthreads();  // the previous stage's fragment reads are done
-        ta.store(s_a);
-        tb.store(s_b);
-        __syncthreads();
+        ta.store(s_a + buf * 3 * BM * 64);
+        tb.store(s_b + buf * 3 * BN * 64);
       };
-      for (int kb = hi - 1; kb > lo; --kb) {
-        stage_in(kb);
-        ta.template load<IN>((kb - 1) * FK, K, lda);
-        tb.template load<IN>((kb - 1) * FK, K, ldb);
-        __builtin_amdgcn_sched_barrier(0);  // left alone, the scheduler sinks the loads behind the products
-        multiply();
+      auto ask = [&](int kb) {
+        ta.template load<IN>(kb * FK, K, lda);
+        tb.template load<IN>(kb * FK, K, ldb);
+      };
+      if constexpr (TURNS) {
+        __syncthreads();  // the fragment reads of an earlier pair of operands are done
+        put(hi - 1, 0);
+        if (hi - 1 > lo) ask(hi - 2);
+        __syncthreads();
+        int buf = 0;
+        const bool first_half = wave < 4;
+        for (int kb = hi - 1; kb > lo; --kb, buf ^= 1) {  // stage kb is in LDS, stage kb - 1 in registers or on its way there
+          // the last of these asks for stage lo once more: what comes is not used
+          if (!first_half) {
+            put(kb - 1, buf ^ 1);
+            ask(max(kb - 2, lo));
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          multiply(buf);
+          __builtin_amdgcn_sched_barrier(0);
+          if (first_half) {
+            put(kb - 1, buf ^ 1);
+            ask(max(kb - 2, lo));
+          }
+          __syncthreads();
+        }
+        multiply(buf);
+      } else {
+        for (int kb = hi - 1; kb > lo; --kb) {
+          __syncthreads();  // the previous stage's fragment reads are done
+          put(kb, 0);
+          __syncthreads();
+          ask(kb - 1);
+          __builtin_amdgcn_sched_barrier(0);  // left alone, the scheduler sinks the loads behind the products
+          multiply(0);
+        }
+        __syncthreads();
+        put(lo, 0);
+        __syncthreads();
+        multiply(0);
       }
-      stage_in(lo);
-      multiply();
     } else {
       for (int kb = lo; kb < hi; ++kb) {
         ta.template load<CHECKED>(kb * FK, K, lda);
@@ -284,7 +320,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_f32(GemmF32 g) {
         ta.store(s_a);
         tb.store(s_b);
         __syncthreads();
-        multiply();
+        multiply(0);
       }
     }
 #pragma unroll
@@ -343,6 +379,33 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_f32(GemmF32 g) {
       }
     return;
   }
+  if (EPI == GEMM_STORE && (g.accumulate || g.decay_state) && g.rows_per == 0) {
+    // C = C + acc or g^K C + acc: all of this wave's elements are asked for before the first is used.  (The L2's adder, one
+    // no-return add per element, took 215 us where this takes 176: 12 slices of [8192 x 500] x [500 x 256].)
+    float old[MI][NJ][16];
+    auto place = [&](int i, int j, int e) {  // past the edge: the last row or column again
+      return C + (long)min(row_of(i, e), g.M - 1) * g.ldc + min(n0 + wn * (BN / WN) + j * 32 + (lane & 31), g.N - 1);
+    };
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) old[i][j][e] = *place(i, j, e);
+    const float keep = g.decay_state ? expf((float)g.K * ld) : 1.0f;
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const bool in = n0 + wn * (BN / WN) + j * 32 + (lane & 31) < g.N;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const float was = g.decay_state ? old[i][j][e] * keep : old[i][j][e];
+          if (in && row_of(i, e) < g.M) *place(i, j, e) = was + acc[i][j][e];
+        }
+      }
+    return;
+  }
   const float slope = (EPI == GEMM_SCORES && g.use_alibi) ? g.slopes[slice % g.heads] : 0.0f;
 #pragma unroll
   for (int i = 0; i < MI; ++i)
@@ -376,14 +439,6 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_f32(GemmF32 g) {
                                          : (long)row * g.ldc) + col;
           if (EPI == GEMM_NORM)
             *p = v / (s_norm[row - m0] + kRowNormEps);
-          else if (g.decay_state)
-            *p = *p * expf((float)g.K * ld) + v;
-          else if (g.accumulate)
-            // C += acc as one no-return add per element, done by the L2: the wavefront does not wait for C to arrive,
-            // so a short-K tile's epilogue overlaps the next workgroup's products.  One add per element and call: the
-            // same rounding as *p + v and no race; the L2's adder flushes results below the smallest normal float to
-            // zero.
-            unsafeAtomicAdd(p, v);
           else
             *p = v;
         }
@@ -394,12 +449,13 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_f32(GemmF32 g) {
 template <int EPI>
 void launch(hipStream_t st, const GemmF32 &g, bool ak, bool bk, int tile, unsigned grid) {
 #define BDH_G(BM_, BN_, WM_, WN_, AK_, BK_) \
-  hipLaunchKernelGGL((k_gemm_f32<BM_, BN_, WM_, WN_, AK_, BK_, EPI>), dim3(grid), dim3(256), 0, st, g)
+  hipLaunchKernelGGL((k_gemm_f32<BM_, BN_, WM_, WN_, AK_, BK_, EPI>), dim3(grid), dim3(WM_ * WN_ * 64), 0, st, g)
 #define BDH_GT(AK_, BK_)                                     \
   do {                                                       \
     if (tile == 0) BDH_G(128, 128, 2, 2, AK_, BK_);          \
     else if (tile == 1) BDH_G(64, 64, 2, 2, AK_, BK_);       \
-    else BDH_G(32, 128, 1, 4, AK_, BK_);                     \
+    else if (tile == 2) BDH_G(32, 128, 1, 4, AK_, BK_);      \
+    else BDH_G(128, 256, 2, 4, AK_, BK_);                    \
   } while (0)
   if constexpr (EPI == GEMM_SCORES) {
     BDH_GT(false, false);
@@ -413,7 +469,7 @@ void launch(hipStream_t st, const GemmF32 &g, bool ak, bool bk, int tile, unsign
 #undef BDH_G
 }
 
-constexpr int kTileM[3] = {128, 64, 32}, kTileN[3] = {128, 64, 128};
+constexpr int kTileM[4] = {128, 64, 32, 128}, kTileN[4] = {128, 64, 128, 256};
 
 // scores over causal time blocks that end on tile edges: the tiles above the diagonal hold nothing, and a reader whose
 // own row tiles are no larger never looks at them
@@ -426,25 +482,34 @@ bool lower_triangle(const GemmF32 &g, int tile) {
 
 // Which tile and how many parts of K.  A CU that holds a few workgroups turns out a 32-deep stage of a 128 x 128, 64 x 64
 // or 32 x 128 tile every `full` cycles; a workgroup alone on its CU takes `alone`, the memory round trip and the two
-// barriers uncovered.  The last, partly filled round of workgroups counts like a whole one.  More parts of K fill the
+// barriers uncovered.  The last, partly filled round of workgroups counts like a whole one.  A 128 x 256 tile has its CU to
+// itself: a stage takes `turn`, and nothing covers its first loads and its last stores, `turn_end` a tile (12 slices of
+// [500 x 8192] x [8192 x 256] in 5 parts: 161 us, in 128 x 128 tiles and 8 parts 185; with a K of 500, [8192 x 500] x [500 x 256],
+// 181 against 176; 32 slices of [511 x 511] x [511 x 256] 56 against 46).  More parts of K fill the
 // chip where the tiles are few, at the price of writing and re-reading every part.
 GemmPlan bdh_gemm_f32_plan(const bdh_ctx *ctx, const GemmF32 &g, int max_split) {
   const double n_cu = ctx->n_cu > 0 ? ctx->n_cu : 256;
   constexpr double full[3] = {2600.0, 900.0, 900.0}, alone[3] = {3600.0, 2000.0, 2000.0};
+  constexpr double turn = 3620.0, turn_end = 33000.0;
   const int nb = (g.K + FK - 1) / FK + (g.K2 + FK - 1) / FK;
   GemmPlan best;
   double best_t = 1e300;
-  for (int t = 0; t < 3; ++t) {
+  for (int t = 0; t < 4; ++t) {
     if (t == 2 && (g.epilogue == GEMM_SCORES || g.M > 96)) continue;
     const double mt = (g.M + kTileM[t] - 1) / kTileM[t], nt = (g.N + kTileN[t] - 1) / kTileN[t];
     const bool tri = lower_triangle(g, t);
     const double tiles = g.n_slices * (tri ? mt * (mt + 1) / 2 : mt * nt);
-    for (int ks = 1; ks <= max_split && (ks == 1 || nb >= 4 * ks); ks *= 2) {
+    for (int ks = 1; ks <= max_split && (ks == 1 || nb >= 4 * ks); ks = t == 3 ? ks + 1 : ks * 2) {
       const double per = (nb + ks - 1) / ks;
       const double wgs = tiles * ks / n_cu;
       const double rounds = wgs <= 1.0 ? 1.0 : wgs;
-      double cyc = per * std::max(rounds * full[t], alone[t]) + 6000.0;
-      if (wgs > 1.0) cyc += per * full[t] * (std::ceil(wgs) - wgs) * 0.5;
+      double cyc;
+      if (t == 3) {
+        cyc = std::ceil(rounds) * (per * turn + turn_end);
+      } else {
+        cyc = per * std::max(rounds * full[t], alone[t]) + 6000.0;
+        if (wgs > 1.0) cyc += per * full[t] * (std::ceil(wgs) - wgs) * 0.5;
+      }
       if (ks > 1) cyc += 8000.0 + (double)g.n_slices * g.M * g.N * 4.0 * 2.0 * ks / 2000.0;  // bytes at about 5 TB/s
       if (cyc < best_t) {
         best_t = cyc;

@@ -1,0 +1,47 @@
+"""The 128 x 256 tile of the split-bf16 products (two stages in LDS, two wavefronts of a SIMD in turns), which only large calls
+take: row and column edges inside a tile, a reduction that ends inside a stage, operands that do not come in aligned pieces,
+a second pair of operands, parts of K; and the state update's read-modify-write at ragged sizes."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("rotary,T,N,d", [("rope", 490, 4096, 256), ("rope", 491, 4098, 500), ("alibi", 490, 4096, 500),
+                                          ("alibi", 487, 4097, 509), ("alibi", 130, 8192, 256)])
+def test_wide_tile_against_float64(rotary, T, N, d):
+    """out = tril(-1)(Q Q^T) V + Q rho, rho += Q^T V (ALiBi: with powers of the decay), frequencies of zero so that Q = x.
+    Sums of up to 8192 terms rounded once per 16: 2^-24 * sqrt(512) = 1.4e-6 of a sum of equal terms; 4e-6 of the largest."""
+    import burn_dragon_amd as bda
+    from burn_dragon_amd.recurrent import recurrent_attention
+
+    B, h = 3, 4
+    rot = bda.RotaryEmbedding.parse(rotary)
+    g = torch.Generator(device=DEV).manual_seed(T + N)
+    x = torch.relu(torch.randn((B, h, T, N), device=DEV, generator=g))
+    v = torch.randn((B, T, d), device=DEV, generator=g)
+    rho = 0.1 * torch.randn((B, h, N, d), device=DEV, generator=g)
+    before = rho.clone()
+    freqs = torch.zeros(N, device=DEV)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        out = recurrent_attention(x, v, rho, freqs, 0, rot)
+        torch.cuda.synchronize()
+    names = [e.key for e in prof.key_averages()]
+    assert any("k_gemm_f32<128, 256" in n for n in names), names
+    decay = torch.ones(h, dtype=torch.float64, device=DEV)
+    if rotary == "alibi":
+        from burn_dragon_amd.kernel.linear_attention import default_alibi_slopes
+
+        slopes = torch.as_tensor(default_alibi_slopes(h), dtype=torch.float32)
+        decay = torch.exp(-slopes).double().to(DEV)
+    t = torch.arange(T, device=DEV, dtype=torch.float64)
+    for b in range(B):
+        for i in range(h):
+            q, val, r0 = x[b, i].double(), v[b].double(), before[b, i].double()
+            powers = decay[i] ** (t[:, None] - t[None, :]).clamp_min(0)
+            want = ((q @ q.T).tril(-1) * powers) @ val + (decay[i] ** t)[:, None] * (q @ r0)
+            state = decay[i] ** T * r0 + ((decay[i] ** (T - t))[:, None] * q).T @ val
+            assert float((out[b, i].double() - want).abs().max() / want.abs().max()) < 4e-6
+            assert float((rho[b, i].double() - state).abs().max() / state.abs().max()) < 4e-6
