@@ -93,62 +93,95 @@ __global__ __launch_bounds__(256) void k_rope_bf16(const uint4 *__restrict__ x, 
   }
 }
 
-// ------------------------------------------------------------------------------------
-// batched transpose to bf16: in [batch][R][C] (f32 or bf16) -> out [batch][C][ldo], ldo >= R,
-// columns R..ldo-1 of the output are zero-filled.  64x64 tiles through LDS.
-// ------------------------------------------------------------------------------------
-template <typename TIn>
-__global__ __launch_bounds__(256) void k_transpose_to_bf16(const TIn *__restrict__ in, unsigned short *__restrict__ out,
-                                                          int R, int C, int ldo, long in_batch) {
-  __shared__ unsigned short tile[64][66];
-  const long batch = blockIdx.z;
-  const int r0 = blockIdx.y * 64, c0 = blockIdx.x * 64;
-  const TIn *src = in + batch * in_batch;
-  unsigned short *dst = out + batch * (long)C * ldo;
-  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-  for (int rr = ty; rr < 64; rr += 4) {
-    const int r = r0 + rr, c = c0 + tx;
-    unsigned short v = 0;
-    if (r < R && c < C) {
-      if constexpr (sizeof(TIn) == 4) v = f32_to_bf16_bits((float)src[(long)r * C + c]);
-      else v = (unsigned short)src[(long)r * C + c];
-    }
-    tile[rr][tx] = v;
-  }
-  __syncthreads();
-  for (int cc = ty; cc < 64; cc += 4) {
-    const int c = c0 + cc, r = r0 + tx;
-    if (c < C && r < ldo) dst[(long)c * ldo + r] = tile[tx][cc];  // rows >= R were staged as zero
-  }
-}
-
 struct HeadPar {
   float v[64];
 };
 
-// V^T per (b,h) slice for a decaying state (src/model/bdh.rs:299-301): in bf16 [B][R][C] -> out bf16
-// [B*h][C][ldo] with row r (token r of R) scaled by exp((R - r) * log_decay[head]) -- the decay a token's update
-// has seen by the end of the pass.  Columns R..ldo-1 of the output are zero-filled.
-__global__ __launch_bounds__(256) void k_transpose_decay_bf16(const unsigned short *__restrict__ in,
-                                                              unsigned short *__restrict__ out, int R, int C, int ldo,
-                                                              long in_batch, int h, HeadPar log_decay) {
-  __shared__ unsigned short tile[64][66];
-  const long slice = blockIdx.z;
-  const float ld = log_decay.v[slice % h];
-  const int r0 = blockIdx.y * 64, c0 = blockIdx.x * 64;
-  const unsigned short *src = in + (slice / h) * in_batch;
-  unsigned short *dst = out + slice * (long)C * ldo;
-  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-  for (int rr = ty; rr < 64; rr += 4) {
-    const int r = r0 + rr, c = c0 + tx;
-    unsigned short v = 0;
-    if (r < R && c < C) v = f32_to_bf16_bits(bf16_bits_to_f32(src[(long)r * C + c]) * expf((float)(R - r) * ld));
-    tile[rr][tx] = v;
+// ------------------------------------------------------------------------------------
+// The operands of the all-scores form that have to be transposed, in one launch, 64 x 64 tiles through LDS:
+//   vs [B][d][Tp]    V^T, columns T.. zero
+//   vt [B*h][d][Tp]  with a decaying state (src/model/bdh.rs:299-301): V^T per slice, token r scaled by
+//                    exp((T - r) * log_decay[head]), the decay a token's update has seen by the end of the pass
+//   rt [B*h][d][Nq]  the carried state, transposed and rounded
+// What bounds it: the bytes of the state (12 slices of 4096 x 256: 75 MB in 14.9 us with V and its four scaled copies; three
+// launches of 2-byte accesses took 19.2, 9.9 and 7.8 us).
+// ------------------------------------------------------------------------------------
+struct TransposeArgs {
+  const unsigned short *v;
+  const float *rho;
+  unsigned short *vs, *vt, *rt;
+  long v_batch;
+  int B, h, T, d, Tp, Nq;
+  int v_tiles, kinds;  // tiles of one V^T; 1 + the heads of a decaying state
+  HeadPar log_decay;
+};
+__global__ __launch_bounds__(256) void k_transpose_operands(TransposeArgs a) {
+  __shared__ __attribute__((aligned(16))) unsigned short tile[64][66];
+  const int tid = threadIdx.x, ct = (a.d + 63) >> 6;
+  const int v_blocks = a.v_tiles * a.B * a.kinds;
+  int at = blockIdx.x;
+  unsigned short *dst;
+  int r0, c0, ldo;
+  if (at < v_blocks) {
+    const int kind = at / (a.v_tiles * a.B);
+    at -= kind * a.v_tiles * a.B;
+    const int b = at / a.v_tiles, t = at - b * a.v_tiles;
+    r0 = t / ct * 64;
+    c0 = (t - t / ct * ct) * 64;
+    ldo = a.Tp;
+    dst = kind == 0 ? a.vs + (long)b * a.d * ldo : a.vt + ((long)b * a.h + kind - 1) * a.d * ldo;
+    const float ld = kind == 0 ? 0.0f : a.log_decay.v[kind - 1];
+    const unsigned short *src = a.v + b * a.v_batch;
+    auto scaled = [&](unsigned short x, int r) {
+      return kind == 0 ? x : f32_to_bf16_bits(bf16_bits_to_f32(x) * expf((float)(a.T - r) * ld));
+    };
+    if ((a.d & 7) == 0) {  // pieces of 16 bytes are all in or all out
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int rr = (tid >> 3) + 32 * i, cc = (tid & 7) * 8, r = r0 + rr;
+        uint4 w = make_uint4(0u, 0u, 0u, 0u);
+        if (r < a.T && c0 + cc < a.d) w = *reinterpret_cast<const uint4 *>(src + (long)r * a.d + c0 + cc);
+        const unsigned int ww[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          *reinterpret_cast<unsigned int *>(&tile[rr][cc + 2 * q]) =
+              (unsigned int)scaled((unsigned short)(ww[q] & 0xffffu), r) |
+              ((unsigned int)scaled((unsigned short)(ww[q] >> 16), r) << 16);
+      }
+    } else {
+      for (int i = tid; i < 64 * 64; i += 256) {
+        const int rr = i >> 6, cc = i & 63, r = r0 + rr;
+        tile[rr][cc] = r < a.T && c0 + cc < a.d ? scaled(src[(long)r * a.d + c0 + cc], r) : (unsigned short)0;
+      }
+    }
+  } else {
+    at -= v_blocks;
+    const int tiles = ct * ((a.Nq + 63) >> 6), slice = at / tiles, t = at - slice * tiles;
+    r0 = t / ct * 64;
+    c0 = (t - t / ct * ct) * 64;
+    ldo = a.Nq;
+    dst = a.rt + (long)slice * a.d * ldo;
+    const float *src = a.rho + (long)slice * a.Nq * a.d;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {  // d % 8 == 0 where there is a state
+      const int rr = (tid >> 4) + 16 * i, cc = (tid & 15) * 4, r = r0 + rr;
+      float4 w = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (r < a.Nq && c0 + cc < a.d) w = *reinterpret_cast<const float4 *>(src + (long)r * a.d + c0 + cc);
+      unsigned int *to = reinterpret_cast<unsigned int *>(&tile[rr][cc]);
+      to[0] = (unsigned int)f32_to_bf16_bits(w.x) | ((unsigned int)f32_to_bf16_bits(w.y) << 16);
+      to[1] = (unsigned int)f32_to_bf16_bits(w.z) | ((unsigned int)f32_to_bf16_bits(w.w) << 16);
+    }
   }
   __syncthreads();
-  for (int cc = ty; cc < 64; cc += 4) {
-    const int c = c0 + cc, r = r0 + tx;
-    if (c < C && r < ldo) dst[(long)c * ldo + r] = tile[tx][cc];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {  // eight rows of a column, 16 bytes (ldo % 8 == 0)
+    const int cc = (tid >> 3) + 32 * i, rr = (tid & 7) * 8;
+    unsigned int w[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      w[q] = (unsigned int)tile[rr + 2 * q][cc] | ((unsigned int)tile[rr + 2 * q + 1][cc] << 16);
+    if (c0 + cc < a.d && r0 + rr < ldo)
+      *reinterpret_cast<uint4 *>(dst + (long)(c0 + cc) * ldo + r0 + rr) = make_uint4(w[0], w[1], w[2], w[3]);
   }
 }
 
@@ -1527,20 +1560,19 @@ static int prefill_pass_scores(bdh_ctx *ctx, int B, int h, int T, int N, int d, 
   };
 
   // 0. V^T (and rho0^T): make every B operand k-contiguous
-  hipLaunchKernelGGL(k_transpose_to_bf16<unsigned short>, dim3((d + 63) / 64, (Tp + 63) / 64, B), dim3(256), 0,
-                     ctx->stream, v_bf16, Vs, T, d, Tp, v_batch);
-  BDH_LAUNCH_CHECK(ctx, "k_transpose_to_bf16<V>");
-  if (pm.decay) {
-    HeadPar hp;
-    memcpy(hp.v, pm.head_par, sizeof(hp.v));
-    hipLaunchKernelGGL(k_transpose_decay_bf16, dim3((d + 63) / 64, (Tp + 63) / 64, S), dim3(256), 0, ctx->stream,
-                       v_bf16, Vt, T, d, Tp, v_batch, h, hp);
-    BDH_LAUNCH_CHECK(ctx, "k_transpose_decay_bf16");
-  }
-  if (has_state) {
-    hipLaunchKernelGGL(k_transpose_to_bf16<float>, dim3((d + 63) / 64, (Nq + 63) / 64, S), dim3(256), 0, ctx->stream,
-                       rho, Rt, Nq, d, Nq, (long)Nq * d);
-    BDH_LAUNCH_CHECK(ctx, "k_transpose_to_bf16<rho0>");
+  {
+    TransposeArgs t{};
+    t.v = v_bf16; t.rho = rho;
+    t.vs = Vs; t.vt = Vt; t.rt = Rt;
+    t.v_batch = v_batch;
+    t.B = B; t.h = h; t.T = T; t.d = d; t.Tp = Tp; t.Nq = Nq;
+    t.v_tiles = ((d + 63) / 64) * ((Tp + 63) / 64);
+    t.kinds = pm.decay ? 1 + h : 1;
+    memcpy(t.log_decay.v, pm.head_par, sizeof(t.log_decay.v));
+    const long blocks = (long)t.v_tiles * B * t.kinds + (has_state ? (long)((d + 63) / 64) * ((Nq + 63) / 64) * S : 0);
+    if (blocks > 0x7fffffffL) return bdh_fail(ctx, BDH_E_SHAPE, "too many tiles (T=%d N=%d)", T, N);
+    hipLaunchKernelGGL(k_transpose_operands, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, t);
+    BDH_LAUNCH_CHECK(ctx, "k_transpose_operands");
   }
   // 1. rotation
   if (own_q) {
