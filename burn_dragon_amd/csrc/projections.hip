@@ -1319,8 +1319,13 @@ static int launch_decoder_rows(bdh_ctx *ctx, int M, long K, int d, int KB, bool 
     bpw = tiles(16) * ((KBN + per - 1) / per) >= n_cu ? per : 1;
     rt = tiles(16) * ((KBN + bpw - 1) / bpw) <= 4 * n_cu ? 1 : M <= 32 ? 2 : 4;
   }
-  const int parts = (KBN + bpw - 1) / bpw;
+  int parts = (KBN + bpw - 1) / bpw;
   int rc = bdh_ws_reserve(ctx, sizeof(float) * (size_t)parts * M * d);
+  if (rc == BDH_E_NOMEM && split && bpw < per) {  // less room: sixteen parts
+    bpw = per;
+    parts = (KBN + bpw - 1) / bpw;
+    rc = bdh_ws_reserve(ctx, sizeof(float) * (size_t)parts * M * d);
+  }
   if (rc != BDH_OK) return rc;
   float *partial = static_cast<float *>(ctx->ws);
   const dim3 grid((d + 63) / 64, (M + 16 * rt - 1) / (16 * rt), parts);
@@ -1363,11 +1368,18 @@ int bdh_launch_decoder_residual(bdh_ctx *ctx, int B, int T, int h, int N, int d,
   while (KB > 128 && ((K + KB - 1) / KB) * row_tiles < 2 * n_cu) KB >>= 1;
   // a small model: down to 32 rows of E per workgroup, until there is a workgroup per CU
   while (KB > 32 && ((K + KB - 1) / KB) * row_tiles < n_cu) KB >>= 1;
-  // a batch of decoding sequences: the f32 matrix cores, the same bits; k-blocks of 1024 with a chain each once those fill
-  // half the chip in 32 x 64 tiles (a negative option value -r: from r sequences on, whatever the size)
+  // A batch of decoding sequences: the f32 matrix cores, the same bits; k-blocks of 1024 with a chain each once those fill
+  // half the chip in 32 x 64 tiles (a negative option value -r: from r sequences on, whatever the size).  The VALU kernel
+  // skips the rows of E that no sequence needs and reads the others once per eight sequences: it is the better one for fewer
+  // than 24 sequences with long rows (us a step, VALU | this: d = 512, E of 268 MB, 8 sequences 5045 | 5115; of 67 MB, 16
+  // sequences 1941 | 1944), and for fewer than 8 unless E is small (d = 256, E of 34 MB, 3 sequences 458 | 490, 8 sequences
+  // 818 | 753; E of 17 MB, 9 sequences 396 | 331, 2 sequences 238 | 230; d = 192, 6 MB, 7 sequences 179 | 171).
   const int sk_rows = ctx->opt_decoder_splitk_rows;
-  if (T == 1 && M >= std::abs(sk_rows) && (K & 3) == 0 && bdh_aligned(xy, 16) && bdh_aligned(decoder, 16)) {
-    const bool split = K % 1024 == 0 && (sk_rows < 0 || K / 1024 * ((d + 63) / 64) * ((M + 31) / 32) >= n_cu / 2);
+  const long many = std::abs(sk_rows);
+  const long few = many > 24 ? many : std::min<long>(many, K * d <= (4L << 20) ? 2 : d <= 256 ? 8 : 24);
+  if (T == 1 && M >= few && (K & 3) == 0 && bdh_aligned(xy, 16) && bdh_aligned(decoder, 16)) {
+    const bool split = M >= many && K % 1024 == 0 &&
+                       (sk_rows < 0 || K / 1024 * ((d + 63) / 64) * ((M + 31) / 32) >= n_cu / 2);
     if (split) KB = 1024;
     return launch_decoder_rows(ctx, M, K, d, KB, split, xy, decoder, cur, head);
   }

@@ -131,3 +131,35 @@ def test_encoder_of_a_batch_in_parts_of_several_k_blocks(B, mult):
         ctx.set_option("decoder.splitk_rows", 24)
     assert not torch.equal(logits[0], logits[1])
     assert rel_err(logits[0], logits[1]) < 1e-5
+
+
+@pytest.mark.parametrize("B,d,h,mult", [(2, 128, 4, 4), (3, 256, 4, 8), (7, 68, 2, 3), (5, 512, 8, 8), (9, 256, 4, 72), (8, 192, 4, 65)])
+def test_encoder_of_a_few_sequences_keeps_the_bits_of_the_valu_kernel(B, d, h, mult):
+    """Two sequences and more of a small E, eight and more of a large one with d <= 256, on the f32 matrix cores."""
+    import burn_dragon_amd as bda
+
+    V = 64
+    cfg = bda.BDHConfig(n_layer=1, n_embd=d, n_head=h, mlp_internal_dim_multiplier=mult, vocab_size=V)
+    cfg.fused_kernels.set_rotary_embedding(bda.RotaryEmbedding.ALIBI)
+    model = bda.BDH(cfg, DEV, seed=3)
+    g = torch.Generator(device=DEV).manual_seed(B)
+    tokens = torch.randint(0, V, (B, 1), device=DEV, generator=g)
+    rho = 0.1 * torch.randn((1, B, h, mult * d // h, d), device=DEV, generator=g)
+    ctx = bda.ffi.default_context(0)
+    logits, names = [], []
+    ctx.set_option("model.one_launch", 0)
+    try:
+        for rows in (24, 1 << 30):
+            ctx.set_option("decoder.splitk_rows", rows)
+            state = model.init_state()
+            state.position, state.storage = 9, rho.clone()
+            state.layers[0].rho = state.storage[0]
+            with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+                logits.append(model.forward_with_state(tokens, state))
+                torch.cuda.synchronize()
+            names.append(" ".join(e.key for e in prof.key_averages()))
+    finally:
+        ctx.set_option("decoder.splitk_rows", 24)
+        ctx.set_option("model.one_launch", 1)
+    assert "k_decoder_rows" in names[0] and "k_decoder_rows" not in names[1]
+    assert torch.equal(logits[0], logits[1])
