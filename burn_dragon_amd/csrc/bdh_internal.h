@@ -64,7 +64,7 @@ struct bdh_model {
 
 int bdh_fail(bdh_ctx *ctx, int status, const char *fmt, ...);
 
-// model_phase.hip: a decode step in two launches per layer (T = 1, f32 state, 128 <= d <= 512, N a multiple of 64)
+// model_phase.hip: a decode step in two launches per layer (T = 1, f32 state, 128 <= d <= 512, N a multiple of 32)
 bool bdh_model_phase_fits(const bdh_model *m);
 int bdh_model_phase_most(const bdh_model *m, int rho_dtype, bool lazy);  // sequences
 size_t bdh_model_phase_scratch_floats(const bdh_model *m, int B);

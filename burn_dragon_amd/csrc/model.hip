@@ -224,7 +224,7 @@ int model_forward_impl(bdh_model *m, const int64_t *tokens, int B, int T, StateR
   int32_t *stamps = st.stamps(0);
 
   // A decode step (one token per sequence, no by-products) need not run kernel by kernel:
-  //  * a mid-size model (128 <= d <= 512, up to 64 blocks of 64 neurons) can run TWO launches per layer, a workgroup
+  //  * a mid-size model (128 <= d <= 512, up to 64 blocks of 64 or 32 neurons) can run TWO launches per layer, a workgroup
   //    per block; every workgroup streams its share of the layer's weights once per sequence (bdh_model_phase_most);
   //  * a small model (d <= 256, h*N <= 2048) can run the whole step in ONE launch, a workgroup per sequence; one CU then
   //    streams all the projection weights of the step, W bytes.

@@ -664,21 +664,21 @@ bool bdh_model_phase_fits(const bdh_model *m) {
   const bdh_model_config &c = m->cfg;
   if (c.rotary != BDH_ROPE && c.rotary != BDH_ALIBI && c.rotary != BDH_POPE) return false;
   if (c.n_embd < 128 || c.n_embd > 512 || (c.n_embd & 3) != 0) return false;
-  if (c.latent < 64 || (c.latent & 63) != 0) return false;  // whole 64-neuron blocks
+  if (c.latent < 32 || (c.latent & 31) != 0) return false;  // whole blocks of 64 or 32 neurons
   if (c.n_head < 1 || c.n_head > 64 || c.n_layer < 1) return false;
   // every workgroup of a sequence sums the partials of all the others: only while those are few
-  if ((long)c.n_head * (c.latent / 64) > 64) return false;
+  if ((long)c.n_head * (c.latent / ((c.latent & 63) == 0 ? 64 : 32)) > 64) return false;
   // 16-byte loads
   return bdh_aligned(m->w.encoder, 16) && bdh_aligned(m->w.encoder_v, 16) && bdh_aligned(m->w.decoder, 16);
 }
 
-// Neurons of a workgroup's block.  Fewer share the bytes that a CU has to fetch among more CUs and make more partials, which
+// Neurons of a workgroup's block: 64 or, always where a head has an odd number of those, 32.  Fewer share the bytes that a CU has to fetch among more CUs and make more partials, which
 // every workgroup adds up: 32 while those blocks number at most 64 and every workgroup has a CU to itself, 64 otherwise (us a
 // step, 32 | 64: 4 layers of 1024 neurons, d = 256, 1 sequence 46 | 52, 8 sequences (256 workgroups) 52 | 56, 16 sequences
 // 66 | 61; 8 layers of 2048, d = 512, 1 sequence 114 | 131, 4 sequences 134 | 146, 8 sequences 223 | 172).
 static int block_neurons(const bdh_ctx *ctx, const bdh_model_config &c, int B) {
   const long n_cu = ctx->n_cu > 0 ? ctx->n_cu : 256, blocks = (long)c.n_head * c.latent / 32;
-  return blocks <= 64 && blocks * B <= n_cu ? 32 : 64;
+  return (c.latent & 63) != 0 || (blocks <= 64 && blocks * B <= n_cu) ? 32 : 64;
 }
 
 // The most sequences that the two-launch layer is taken for: while batch x weights of a layer (every workgroup streams its
@@ -689,13 +689,18 @@ static int block_neurons(const bdh_ctx *ctx, const bdh_model_config &c, int B) {
 //   layer, 128 sequences 214 to 288 | 265 to 327, 192 sequences 336 | 299: 384 MiB
 //   bf16, 12 MiB a layer, 24 sequences 281 to 487 | 287 to 504, 32 sequences 352 to 622 | 317 to 574: 288 MiB
 //   bf16 and lazily decayed, 12 MiB a layer, 128 sequences 1126 to 1839 | 1742 to 2520: 1536 MiB
+//   an odd number of 32-neuron blocks per head, which are not taken two at a time: 0.9 MiB a layer, 64 sequences 79 to 85 |
+//   100 to 117, 128 sequences 121 to 133 | 103 to 118: 72 MiB; 2.5 MiB a layer, 64 sequences 164 to 181 | 174 to 225, 128
+//   sequences 299 to 321 | 217 to 294: 192 MiB
 int bdh_model_phase_most(const bdh_model *m, int rho_dtype, bool lazy) {
   const bdh_model_config &c = m->cfg;
   const size_t w_layer = sizeof(float) * (size_t)3 * c.n_head * c.latent * c.n_embd;
-  const size_t mib = bdh_model_small_fits(c) && w_layer * c.n_layer <= (size_t(8) << 20) ? 128
-                     : rho_dtype != BDH_BF16                                              ? 384
-                     : lazy                                                               ? 1536
-                                                                                          : 288;
+  const bool one_launch = bdh_model_small_fits(c) && w_layer * c.n_layer <= (size_t(8) << 20);
+  const size_t mib = (c.latent & 63) != 0    ? (one_launch ? 72 : 192)
+                     : one_launch            ? 128
+                     : rho_dtype != BDH_BF16 ? 384
+                     : lazy                  ? 1536
+                                             : 288;
   const size_t most = (mib << 20) / w_layer;
   return most > 65535 ? 65535 : (int)most;
 }

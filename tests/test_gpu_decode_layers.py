@@ -26,6 +26,10 @@ def rel_err(a, b):
     (256, 4, 1024, 64, 2, True),    # 64 blocks of 64
     (260, 1, 64, 516, 1, True),
     (512, 4, 64, 1024, 3, True),
+    (128, 4, 32, 69, 3, True),      # a single block of 32 per head
+    (192, 4, 96, 256, 40, True),    # an odd number of them, more workgroups than a chip of 256 has at once
+    (512, 2, 1024, 64, 1, True),    # 64 blocks of 32
+    (128, 1, 2016, 33, 2, True),    # 63 blocks of 32
     (256, 4, 128, 256, 2, False),   # refused by this form: another one gives the same values
 ])
 def test_two_launch_layer_edges(state, rotary, lazy, d, h, N, V, B, aligned):
