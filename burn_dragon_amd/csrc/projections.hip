@@ -447,7 +447,10 @@ __global__ __launch_bounds__(256) void k_layer_norm(const float *__restrict__ in
 }
 
 // LayerNorm of many rows for internal use (the readout of a many-token state step): one wave per row, the
-// statistics by wave reduction instead of the index-order sums above (d <= 1024)
+// statistics by wave reduction instead of the index-order sums above (d <= 64 * J).  What bounds it: a row's trip to memory
+// and two sums over a wave, so all loads of a row are on their way at once and the sums are made with register moves (16352 rows of 256:
+// 9.5 -> 7.7 us = 4.4 TB/s).
+template <int J>
 __global__ __launch_bounds__(256) void k_layer_norm_wave(const float *__restrict__ in, float *__restrict__ out, int d,
                                                          long rows) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -455,27 +458,22 @@ __global__ __launch_bounds__(256) void k_layer_norm_wave(const float *__restrict
   if (row >= rows) return;
   const float *x = in + row * d;
   float *y = out + row * d;
-  float v[16], s = 0.0f;
+  float v[J], s = 0.0f;
 #pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    const int c = j * 64 + lane;
-    v[j] = c < d ? x[c] : 0.0f;
-    s += v[j];
-  }
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-  const float mean = s / (float)d;
+  for (int j = 0; j < J; ++j) v[j] = x[min(j * 64 + lane, d - 1)];
+#pragma unroll
+  for (int j = 0; j < J; ++j) s += j * 64 + lane < d ? v[j] : 0.0f;
+  const float mean = bdh_wave_sum(s) / (float)d;
   float q = 0.0f;
 #pragma unroll
-  for (int j = 0; j < 16; ++j)
-    if (j * 64 + lane < d) {
-      const float c = v[j] - mean;
-      q += c * c;
-    }
-  for (int o = 32; o > 0; o >>= 1) q += __shfl_xor(q, o);
-  const float den = sqrtf(q / (float)d + kLnEps);
+  for (int j = 0; j < J; ++j) {
+    v[j] -= mean;
+    q += j * 64 + lane < d ? v[j] * v[j] : 0.0f;
+  }
+  const float den = sqrtf(bdh_wave_sum(q) / (float)d + kLnEps);
 #pragma unroll
-  for (int j = 0; j < 16; ++j)
-    if (j * 64 + lane < d) y[j * 64 + lane] = (v[j] - mean) / den;
+  for (int j = 0; j < J; ++j)
+    if (j * 64 + lane < d) y[j * 64 + lane] = v[j] / den;
 }
 
 // embed gather + LayerNorm (src/model/bdh.rs:319-322), rows laid out like k_layer_norm's
@@ -946,71 +944,71 @@ __global__ __launch_bounds__(1024) void k_decoder_finalize(const float *__restri
   lm_head_row(s_grp[2], s_grp[3], s_best, s_arg, m, head.lm_head, head.T, d, head.V, head.logits, head.next_tokens);
 }
 
-// k_decoder_finalize<false> for many rows: a wavefront per row, the partials of a column added in the same order (sixteen
-// groups, each in index order), then the same wave-wide LayerNorms, so the same bits.  What bounds it: the reads of the
-// partials; a workgroup of sixteen wavefronts per row spends most of its time in its one barrier once the rows alone fill
-// the chip (4088 rows of 256, 4 partials: 56 against 10 us).
+// k_decoder_finalize<false> for many rows: a wavefront per row (d <= 64 * J), the partials of a column added in the same order
+// (sixteen groups, each in index order), then the same wave-wide LayerNorms, so the same bits.  What bounds it: the reads of
+// the partials, U of them for all columns on their way at once; a workgroup of sixteen wavefronts per row spends most of its
+// time in its one barrier once the rows alone fill the chip (4088 rows of 256, 4 partials: 56 us against 7).
+// One column after the other, a trip to memory each, it took 9.7; 1500 rows of 256, 16 partials 22 -> 9.
+template <int J, int U>
 __global__ __launch_bounds__(256) void k_decoder_finalize_rows(const float *__restrict__ partial, int KBN, int M, int d,
                                                                float *__restrict__ cur) {
   const int lane = threadIdx.x & 63;
   const long m = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (m >= M) return;
   const int per = (KBN + 15) >> 4;
-  float vals[16], res[16];
+  const long step = (long)M * d;
+  const float *p = partial + m * d;
+  float vals[J], t[J], res[J];
   float s = 0.0f;
+  int col[J];
 #pragma unroll
-  for (int j = 0; j < 16; ++j) res[j] = j * 64 + lane < d ? cur[m * d + j * 64 + lane] : 0.0f;
-#pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    vals[j] = 0.0f;
-    const int c = j * 64 + lane;
-    if (c < d) {
-      const float *p = partial + m * d + c;
-      const long step = (long)M * d;
-      float v = 0.0f, t = 0.0f;
-      int in_group = 0;
-      for (int kb = 0; kb < KBN; kb += 8) {  // eight partials in flight
-        float x[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) x[u] = p[min(kb + u, KBN - 1) * step];
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-          if (kb + u < KBN) {
-            t = in_group == 0 ? x[u] : t + x[u];
-            if (++in_group == per || kb + u == KBN - 1) {
-              v = kb + u < per ? t : v + t;
-              in_group = 0;
-            }
-          }
-      }
-      vals[j] = v;
-      s += v;
-    }
+  for (int j = 0; j < J; ++j) {
+    col[j] = min(j * 64 + lane, d - 1);
+    res[j] = cur[m * d + col[j]];
+    vals[j] = t[j] = 0.0f;
   }
+  int in_group = 0;
+  for (int kb = 0; kb < KBN; kb += U) {
+    float x[U][J];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int j = 0; j < J; ++j) x[u][j] = p[min(kb + u, KBN - 1) * step + col[j]];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (kb + u < KBN) {
+        const bool first = in_group == 0, last = in_group + 1 == per || kb + u == KBN - 1;
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+          t[j] = first ? x[u][j] : t[j] + x[u][j];
+          if (last) vals[j] = kb + u < per ? t[j] : vals[j] + t[j];
+        }
+        in_group = last ? 0 : in_group + 1;
+      }
+  }
+#pragma unroll
+  for (int j = 0; j < J; ++j) s += j * 64 + lane < d ? vals[j] : 0.0f;
   auto spread = [&](float mean) {  // sqrt(var + eps)
     float q = 0.0f;
 #pragma unroll
-    for (int j = 0; j < 16; ++j)
-      if (j * 64 + lane < d) {
-        const float t = vals[j] - mean;
-        q += t * t;
-      }
+    for (int j = 0; j < J; ++j) {
+      const float c = vals[j] - mean;
+      q += j * 64 + lane < d ? c * c : 0.0f;
+    }
     return sqrtf(bdh_wave_sum(q) / (float)d + kLnEps);
   };
   float mean = bdh_wave_sum(s) / (float)d;
   float den = spread(mean);
   s = 0.0f;
 #pragma unroll
-  for (int j = 0; j < 16; ++j)
-    if (j * 64 + lane < d) {
-      const float mlp = (vals[j] - mean) / den;
-      vals[j] = res[j] + mlp;
-      s += vals[j];
-    }
+  for (int j = 0; j < J; ++j) {
+    vals[j] = res[j] + (vals[j] - mean) / den;
+    s += j * 64 + lane < d ? vals[j] : 0.0f;
+  }
   mean = bdh_wave_sum(s) / (float)d;
   den = spread(mean);
 #pragma unroll
-  for (int j = 0; j < 16; ++j)
+  for (int j = 0; j < J; ++j)
     if (j * 64 + lane < d) cur[m * d + j * 64 + lane] = (vals[j] - mean) / den;
 }
 
@@ -1255,7 +1253,8 @@ int bdh_launch_layer_norm_rows(bdh_ctx *ctx, int64_t rows, int d, const float *i
   const int64_t blocks = (rows + 3) / 4;
   if (blocks > 0x7fffffffL) return bdh_fail(ctx, BDH_E_SHAPE, "too many rows");
   if (rows == 0) return BDH_OK;
-  hipLaunchKernelGGL(k_layer_norm_wave, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, in, out, d, (long)rows);
+  auto *kernel = d <= 256 ? k_layer_norm_wave<4> : d <= 512 ? k_layer_norm_wave<8> : k_layer_norm_wave<16>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, in, out, d, (long)rows);
   BDH_LAUNCH_CHECK(ctx, "k_layer_norm_wave");
   return BDH_OK;
 }
@@ -1288,7 +1287,10 @@ static void launch_lm_head(bdh_ctx *ctx, int M, int T, int d, int V, const float
 static void launch_decoder_finalize(bdh_ctx *ctx, const float *partial, int KBN, int M, int d, float *cur,
                                     const DecoderHead *head) {
   if (M >= kManyRows) {
-    hipLaunchKernelGGL(k_decoder_finalize_rows, dim3((M + 3) / 4), dim3(256), 0, ctx->stream, partial, KBN, M, d, cur);
+    auto *kernel = d <= 256   ? k_decoder_finalize_rows<4, 4>
+                   : d <= 512 ? k_decoder_finalize_rows<8, 4>
+                              : k_decoder_finalize_rows<16, 2>;
+    hipLaunchKernelGGL(kernel, dim3((M + 3) / 4), dim3(256), 0, ctx->stream, partial, KBN, M, d, cur);
     if (head) launch_lm_head(ctx, M, head->T, d, head->V, cur, head->lm_head, head->logits, head->next_tokens);
   } else if (head) {
     hipLaunchKernelGGL(k_decoder_finalize<true>, dim3(M), dim3(1024), 0, ctx->stream, partial, KBN, M, d, cur, *head);

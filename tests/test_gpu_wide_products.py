@@ -45,3 +45,20 @@ def test_wide_tile_against_float64(rotary, T, N, d):
             state = decay[i] ** T * r0 + ((decay[i] ** (T - t))[:, None] * q).T @ val
             assert float((out[b, i].double() - want).abs().max() / want.abs().max()) < 4e-6
             assert float((rho[b, i].double() - state).abs().max() / state.abs().max()) < 4e-6
+
+
+@pytest.mark.parametrize("T,d", [(128, 256), (90, 260), (100, 512), (88, 516), (86, 1024)])
+def test_rows_of_every_width_through_layer_norm_and_second_stage(T, d):
+    """A wavefront holds a row in 4, 8 or 16 registers a lane once a call has 256 rows; a step has its own kernels.  Five stages,
+    each a sum of up to 1024 terms: 5 * 2^-24 * sqrt(1024) = 1e-5 of the largest logit, twice that allowed."""
+    import burn_dragon_amd as bda
+
+    cfg = bda.BDHConfig(n_layer=1, n_embd=d, n_head=2, mlp_internal_dim_multiplier=1, vocab_size=40)
+    cfg.fused_kernels.set_rotary_embedding(bda.RotaryEmbedding.ALIBI)
+    model = bda.BDH(cfg, DEV, seed=d)
+    tokens = torch.randint(0, 40, (3, T), generator=torch.Generator().manual_seed(T))
+    logits = model.forward_with_state(tokens, model.init_state())
+    state = model.init_state()
+    for t in range(T):
+        one = model.forward_with_state(tokens[:, t:t + 1], state)[:, 0]
+        assert (logits[:, t] - one).abs().max() <= 2e-5 * one.abs().max()
