@@ -62,3 +62,28 @@ def test_rows_of_every_width_through_layer_norm_and_second_stage(T, d):
     for t in range(T):
         one = model.forward_with_state(tokens[:, t:t + 1], state)[:, 0]
         assert (logits[:, t] - one).abs().max() <= 2e-5 * one.abs().max()
+
+
+@pytest.mark.parametrize("h,T,d,block", [(11, 511, 256, 1), (16, 450, 260, 64), (13, 500, 200, 48), (33, 321, 96, 1)])
+def test_row_normalised_attention_in_small_tiles(h, T, d, block):
+    """Chips full of 64 x 64 tiles: odd and even slices walk their row tiles in opposite orders, a time block crosses tiles or
+    not.  Errors of a sum rounded once per 16 products, K = 64 and then T: sqrt(T / 48) * 2^-25.8 < 0.6e-7 for the second
+    product, 0.4e-7 for the scores and as much for storing them; 3 * 2^-24 = 1.8e-7."""
+    import burn_dragon_amd as bda
+    from burn_dragon_amd.kernel.linear_attention import build_freqs, default_alibi_slopes, fused_state_aligned
+
+    B, N = 3, 64
+    g = torch.Generator(device=DEV).manual_seed(T)
+    q = torch.relu(torch.randn((B, h, T, N), device=DEV, generator=g))
+    v = torch.randn((B, 1, T, d), device=DEV, generator=g)
+    slopes = torch.tensor(default_alibi_slopes(h))
+    out = fused_state_aligned(q, v, build_freqs(N, 65536.0, bda.RotaryEmbedding.ALIBI, device=DEV), slopes,
+                              bda.BlockPattern2d.dense(block), bda.RotaryEmbedding.ALIBI)
+    i = torch.arange(T, device=DEV)
+    S = torch.matmul(q.double(), q.double().transpose(-1, -2).contiguous())
+    S = torch.where(i[None, :] < i[:, None], S, 0.0)
+    bias = slopes.to(DEV).double()[None, :, None, None] * (i[None, :] - i[:, None]).double()
+    S = torch.where(i[None, :] // block <= i[:, None] // block, S + bias, 0.0)
+    ref = torch.matmul(S, v.double().expand(B, h, T, d).contiguous()) / (S.abs().sum(-1, keepdim=True) + 1e-6)
+    for s in range(h):  # every slice: one in the wrong order would be wrong alone
+        assert float((out[:, s].double() - ref[:, s]).norm() / ref[:, s].norm()) < 1.8e-7
