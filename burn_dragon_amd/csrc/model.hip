@@ -110,7 +110,7 @@ int bdh_model_create(bdh_ctx *ctx, const bdh_model_config *c, const bdh_model_we
   }
   if (has_phase_act(*c) && bdh_model_phase_fits(m)) {
     size_t most = 0;
-    for (int B = bdh_model_phase_most(m, BDH_F32, false); B > 0; --B)  // whatever the state's type: at most 1365
+    for (int B = bdh_model_phase_most(m, BDH_F32, false); B > 0; --B)  // whatever the state's type: at most 1536
       most = std::max(most, bdh_model_phase_scratch_floats(m, B));
     if (hipMalloc(reinterpret_cast<void **>(&m->phase_act), sizeof(float) * most) != hipSuccess) {
       (void)hipGetLastError();

@@ -2,12 +2,12 @@
 // Kernel by kernel a layer of BDH::forward_with_state (src/model/bdh.rs:336-441) is D_x, state step, its second
 // stage, D_y, encoder partials, encoder second stage; at a few sequences each of those is a launch latency plus a
 // trip or two to memory.  The only points where a layer needs data from the whole sequence are the LayerNorm of
-// a head's readout and the LayerNorm of the encoder output, so a workgroup that owns 64 neurons of one head of
-// one sequence can run everything between them on its own:
-//   phase A: [previous layer's cur = LN(cur + LN(sum of encoder partials))]  D_x for its 64 neurons, their state
+// a head's readout and the LayerNorm of the encoder output, so a workgroup that owns 64 (or 32) neurons of one head
+// of one sequence can run everything between them on its own:
+//   phase A: [previous layer's cur = LN(cur + LN(sum of encoder partials))]  D_x for its neurons, their state
 //            rows (readout, update, decay), the readout partial of the workgroup;
-//   phase B: LN(sum of the head's readout partials), D_y and the gate for its 64 neurons, the encoder partial of
-//            those 64 rows of E.
+//   phase B: LN(sum of the head's readout partials), D_y and the gate for its neurons, the encoder partial of
+//            those rows of E.
 // The sums over partials are redone by every workgroup that needs them (a few KiB from the L2).  All sums are taken in a
 // fixed tree of their own (results agree with the kernel-by-kernel step to rounding, not bit for bit).
 //
@@ -34,8 +34,8 @@ struct PhaseArgs {
   float *cur_out;             // [B][d] the layer's input, written by the first workgroup of a sequence
   const float *dec_partial;   // [G][B][d] encoder partials of the previous layer (not the first layer)
   float *x;                   // [B][h*N]
-  float *attn_partial;        // [B][h][N/64][d]
-  float *dec_partial_out;     // [G][B][d], G = h * N / 64
+  float *attn_partial;        // [B][h][N / block][d]
+  float *dec_partial_out;     // [G][B][d], G = h * N / block
   const float *enc, *enc_v, *dec, *freqs;
   void *rho;                  // this layer's state [B][h][Nq][d], f32 or bf16
   int32_t *stamps;            // this layer's stamps [B][h][N] or null
@@ -672,10 +672,11 @@ bool bdh_model_phase_fits(const bdh_model *m) {
   return bdh_aligned(m->w.encoder, 16) && bdh_aligned(m->w.encoder_v, 16) && bdh_aligned(m->w.decoder, 16);
 }
 
-// Neurons of a workgroup's block: 64 or, always where a head has an odd number of those, 32.  Fewer share the bytes that a CU has to fetch among more CUs and make more partials, which
-// every workgroup adds up: 32 while those blocks number at most 64 and every workgroup has a CU to itself, 64 otherwise (us a
-// step, 32 | 64: 4 layers of 1024 neurons, d = 256, 1 sequence 46 | 52, 8 sequences (256 workgroups) 52 | 56, 16 sequences
-// 66 | 61; 8 layers of 2048, d = 512, 1 sequence 114 | 131, 4 sequences 134 | 146, 8 sequences 223 | 172).
+// Neurons of a workgroup's block.  A head whose N is no multiple of 64 takes 32.  For the others: fewer neurons share the
+// bytes that a CU has to fetch among more CUs and make more partials, which every workgroup adds up: 32 while those blocks
+// number at most 64 and every workgroup has a CU to itself, 64 otherwise (us a step, 32 | 64: 4 layers of 1024 neurons, d =
+// 256, 1 sequence 46 | 52, 8 sequences (256 workgroups) 52 | 56, 16 sequences 66 | 61; 8 layers of 2048, d = 512, 1 sequence
+// 114 | 131, 4 sequences 134 | 146, 8 sequences 223 | 172).
 static int block_neurons(const bdh_ctx *ctx, const bdh_model_config &c, int B) {
   const long n_cu = ctx->n_cu > 0 ? ctx->n_cu : 256, blocks = (long)c.n_head * c.latent / 32;
   return (c.latent & 63) != 0 || (blocks <= 64 && blocks * B <= n_cu) ? 32 : 64;

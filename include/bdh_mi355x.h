@@ -23,10 +23,9 @@
  *   - Entry points may grow the context's workspace (hipMalloc) the first time a shape is seen: run a
  *     step of each shape once before capturing calls in a HIP graph.
  *   - There is no CPU fallback: without a HIP device every compute entry point fails.
- *   - State (`rho`) and output (`out`) buffers are ordinary device memory (hipMalloc: coarse-grained).  Calls
- *     of many tokens add their products into them with the L2's no-return f32 adder (one add per element and call,
- *     so no ordering question); fine-grained or host-coherent allocations may not perform such an add and would
- *     lose updates silently.  Sums of that path below the smallest normal float are flushed to zero.
+ *   - State (`rho`) and output (`out`) buffers are ordinary device memory (hipMalloc: coarse-grained), the kind
+ *     every kernel here is built and measured for.  Calls of many tokens read each element of the state, add the
+ *     call's product and write it back, one thread per element and call; no atomic add is used.
  *   - bdh_ctx_set_stream only swaps the stream: the context's workspace is shared by all of its calls, so the
  *     caller orders the old stream's queued work before the new stream's (an event), or uses one context per stream.
  */
