@@ -132,8 +132,9 @@ __global__ __launch_bounds__(256) void k_transpose_operands(TransposeArgs a) {
     dst = kind == 0 ? a.vs + (long)b * a.d * ldo : a.vt + ((long)b * a.h + kind - 1) * a.d * ldo;
     const float ld = kind == 0 ? 0.0f : a.log_decay.v[kind - 1];
     const unsigned short *src = a.v + b * a.v_batch;
+    // (behind the last token the factor would grow, without bound under a steep decay, and 0 * inf is not the zero of a pad)
     auto scaled = [&](unsigned short x, int r) {
-      return kind == 0 ? x : f32_to_bf16_bits(bf16_bits_to_f32(x) * expf((float)(a.T - r) * ld));
+      return kind == 0 || r >= a.T ? x : f32_to_bf16_bits(bf16_bits_to_f32(x) * expf((float)(a.T - r) * ld));
     };
     if ((a.d & 7) == 0) {  // pieces of 16 bytes are all in or all out
 #pragma unroll

@@ -96,6 +96,33 @@ def test_alibi_prefill_custom_slopes_then_decode_steps(bda, corc):
     assert rel_err(rho.cpu().numpy(), rho_ref) < TOL
 
 
+@pytest.mark.parametrize("fresh", [False, True])
+@pytest.mark.parametrize("T,N,d", [(33, 40, 72), (34, 40, 72), (35, 40, 72), (36, 40, 72), (37, 40, 72), (38, 40, 72),
+                                   (39, 40, 72), (41, 16384, 256)])  # the last one, fresh: 256 wide tiles of the state
+def test_steep_decay_over_a_ragged_prompt(bda, T, N, d, fresh):
+    """A prompt that ends inside a piece of eight tokens, with heads whose state loses e^-15, e^-80 or, at a slope of 120
+    (whose factor rounds to zero), all of it per token: what pads the last piece adds nothing."""
+    from burn_dragon_amd.recurrent import prefill_chunked_ex
+
+    B, h = 1, 4
+    slopes = np.array([15.0, 80.0, 120.0, 0.5], np.float32)
+    x, v, rho0 = _case(T + N, B, h, T, N, d, N, 0.0 if fresh else 0.05)
+    rho = rho0.clone().to(DEV)
+    out = prefill_chunked_ex(x.to(DEV), v.to(DEV), rho, None, 3, rotary=bda.RotaryEmbedding.ALIBI, alibi_slopes=slopes,
+                             state_is_zero=fresh)
+    # the token loop of src/model/bdh.rs:288-302, in float64
+    xd, vd, state = x.to(DEV).double(), v.to(DEV).double(), rho0.to(DEV).double()
+    decay = torch.from_numpy(np.exp(-slopes)).to(DEV).double()[None, :, None, None]
+    want = torch.zeros((B, h, T, d), device=DEV, dtype=torch.float64)
+    for t in range(T):
+        want[:, :, t] = (xd[:, :, t, :, None] * state).sum(2)
+        state = (state + xd[:, :, t, :, None] * vd[:, None, t, None, :]) * decay
+    assert torch.isfinite(out).all() and torch.isfinite(rho).all()
+    for hh in range(h):
+        assert rel_err(out[:, hh].cpu(), want[:, hh].cpu()) < TOL or not want[:, hh].any()
+        assert rel_err(rho[:, hh].cpu(), state[:, hh].cpu()) < TOL or state[:, hh].abs().max() < 1e-30
+
+
 def test_rope_through_the_extended_entry_point_is_the_plain_call(bda, corc):
     """rotary = RoPE without row normalisation is bdh_prefill_chunked, bit for bit (chunk-recurrent form included)."""
     from burn_dragon_amd.recurrent import prefill_chunked, prefill_chunked_ex
