@@ -25,6 +25,7 @@
 
 #include "bdh_internal.h"
 #include "lds_copy.h"
+#include "tile_index.h"
 
 namespace {
 
@@ -164,10 +165,19 @@ __global__ __launch_bounds__(256) void k_transpose_operands(TransposeArgs a) {
     dst = a.rt + (long)slice * a.d * ldo;
     const float *src = a.rho + (long)slice * a.Nq * a.d;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {  // d % 8 == 0 where there is a state
+    for (int i = 0; i < 4; ++i) {  // PoPE and ALiBi take any d
       const int rr = (tid >> 4) + 16 * i, cc = (tid & 15) * 4, r = r0 + rr;
+      const int n = r < a.Nq ? bdh_columns_of_piece(c0 + cc, 4, a.d) : 0;
+      const float *p = src + (long)r * a.d + c0 + cc;
       float4 w = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (r < a.Nq && c0 + cc < a.d) w = *reinterpret_cast<const float4 *>(src + (long)r * a.d + c0 + cc);
+      if ((a.d & 3) == 0) {
+        if (n == 4) w = *reinterpret_cast<const float4 *>(p);
+      } else {
+        if (n > 0) w.x = p[0];
+        if (n > 1) w.y = p[1];
+        if (n > 2) w.z = p[2];
+        if (n > 3) w.w = p[3];
+      }
       unsigned int *to = reinterpret_cast<unsigned int *>(&tile[rr][cc]);
       to[0] = (unsigned int)f32_to_bf16_bits(w.x) | ((unsigned int)f32_to_bf16_bits(w.y) << 16);
       to[1] = (unsigned int)f32_to_bf16_bits(w.z) | ((unsigned int)f32_to_bf16_bits(w.w) << 16);

@@ -18,3 +18,10 @@ BDH_HOST_DEVICE int bdh_kmajor_row(int r0, int lead, int c, int ch, int rows) {
   }
   return r0 + lead + c < rows - 1 ? r0 + lead + c : rows - 1;
 }
+
+// A thread owns the `piece` columns from c on (a multiple of piece) of rows of `cols` values that lie one behind the other: how
+// many of them exist.  Where cols % piece == 0 that is all or none, and a row's pieces are aligned as the first one is: one
+// access each.  Elsewhere a row starts anywhere and its last piece ends inside the next row, or behind the last one: one by one.
+BDH_HOST_DEVICE int bdh_columns_of_piece(int c, int piece, int cols) {
+  return c >= cols ? 0 : cols - c < piece ? cols - c : piece;
+}

@@ -48,6 +48,9 @@ ROT = {"rope": orc.ROPE, "alibi": orc.ALIBI, "pope": orc.POPE}
     (300, 264, 72, 0.0, 0, 0),       # fresh state, two score tiles
     (512, 256, 256, 0.05, 33, 0),    # full tiles: operands straight from global memory into LDS
     (600, 128, 64, 0.05, 9, 256),    # three passes: the state (and its decay) carried between them
+    (70, 24, 70, 0.05, 5, 0),        # rows of the carried state that do not come in 16-byte pieces
+    (50, 72, 37, 0.05, 0, 24),       # nor in whole words of two rounded values, over three passes
+    (50, 72, 35, 0.0, 0, 24),        # the same of a fresh state that later passes find carried
 ])
 def test_recurrent_prefill_pope_and_alibi(bda, corc, rotary, T, N, d, rho0_scale, position, chunk):
     """Oracle = the sequential loop of src/model/bdh.rs:288-302 (PoPE rotation of attention.rs:323-330; ALiBi decay of

@@ -1,6 +1,9 @@
 // The rows that the threads of a k-major tile read (bdh_kmajor_row), for every width up to 640 and every tile: inside the
-// operand, aligned where a group is read at once, and the thread's own row wherever it has one.
+// operand, aligned where a group is read at once, and the thread's own row wherever it has one.  And the columns that the
+// pieces of a 64 wide tile read (bdh_columns_of_piece): each column of a row once, none behind it, all of an aligned piece or
+// none of it where it is read at once.
 #include <cstdio>
+#include <initializer_list>
 
 #include "../burn_dragon_amd/csrc/tile_index.h"
 
@@ -23,6 +26,19 @@ int main() {
             if (first % ch != 0 || first + ch > rows) return std::printf("rows %d tile %d: group at %d\n", rows, R, first), 1;
           }
         }
+    }
+  for (int cols = 1; cols <= 640; ++cols)
+    for (int piece : {4, 8}) {
+      int read = 0;
+      for (int c0 = 0; c0 < cols; c0 += 64)
+        for (int cc = 0; cc < 64; cc += piece) {
+          const int n = bdh_columns_of_piece(c0 + cc, piece, cols);
+          if (n < 0 || n > piece || (n > 0 && c0 + cc + n > cols)) return std::printf("cols %d piece of %d at %d: %d\n", cols, piece, c0 + cc, n), 1;
+          if (cols % piece == 0 && n != 0 && n != piece) return std::printf("cols %d: a part of an aligned piece of %d\n", cols, piece), 1;
+          read += n;
+        }
+      if (read != cols) return std::printf("cols %d: %d read in pieces of %d\n", cols, read, piece), 1;
+      checked += cols;
     }
   std::printf("ok %ld\n", checked);
   return 0;
