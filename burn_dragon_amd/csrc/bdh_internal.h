@@ -295,7 +295,7 @@ __device__ __forceinline__ float bdh_wave_sum(float v) {
   return v;
 }
 // v / den for many v and one den, r = 1 / den rounded: one correction of v * r by its remainder gives the rounded quotient
-// (P. Markstein, IBM J. Res. Dev. 34, 1990) in three operations instead of the ten of a division.
+// (P. Markstein, IBM J. Res. Dev. 34, 1990) in three operations instead of the ten of a division.  v and den are finite.
 __device__ __forceinline__ float bdh_quotient(float v, float den, float r) {
   const float q = v * r;
   return __builtin_fmaf(__builtin_fmaf(-q, den, v), r, q);

@@ -19,6 +19,8 @@
 // on its own copy of the row: no barriers between their sums.  First start to last end of a launch, one sequence, d = 256,
 // 1024 neurons: phase A 9.2 -> 4.3 us, phase B 5.7 -> 2.5; d = 512, 2048 neurons: 12.5 -> 6.6, 7.7 -> 3.5.  The 1.5 us from the
 // end of one launch to the start of the next remain.
+#include <cfloat>
+
 #include "bdh_internal.h"
 
 namespace {
@@ -76,9 +78,13 @@ __device__ __forceinline__ void wave_layer_norm(float (&v)[CJ], int d) {
     v[j] = c;
     q += c * c;
   }
-  const float den = sqrtf(bdh_quotient(bdh_wave_sum(q), fd, rd) + kLnEps), r = 1.0f / den;
+  // A variance beyond the floats is infinite and the row then zero, as the divisions have it: the remainder inf - inf of
+  // either quotient must not come in.
+  const float sum = bdh_wave_sum(q);
+  const float den = sqrtf((sum <= FLT_MAX ? bdh_quotient(sum, fd, rd) : sum) + kLnEps), r = 1.0f / den;
+  const float finite = fminf(den, FLT_MAX);
 #pragma unroll
-  for (int j = 0; j < CJ; ++j) v[j] = bdh_quotient(v[j], den, r);
+  for (int j = 0; j < CJ; ++j) v[j] = bdh_quotient(v[j], finite, r);
 }
 
 // How the NW waves of a workgroup share rows of d <= DC floats and the NB neurons of its block.

@@ -167,3 +167,44 @@ def test_encoder_of_a_few_sequences_keeps_the_bits_of_the_valu_kernel(B, d, h, m
         ctx.set_option("model.one_launch", 1)
     assert "k_decoder_rows" in names[0] and "k_decoder_rows" not in names[1]
     assert torch.equal(logits[0], logits[1])
+
+
+@pytest.mark.parametrize("huge", ["embed", "decoder", "state"])
+@pytest.mark.parametrize("d,h,N,V", [(128, 2, 64, 64), (260, 1, 64, 33)])
+def test_two_launch_layer_norms_of_rows_whose_variance_is_no_float(huge, d, h, N, V):
+    """A row whose variance is infinite is zero (c / inf), in the embedding, the encoder or the readout: the same values as
+    kernel by kernel, and nothing that is no number."""
+    import burn_dragon_amd as bda
+
+    B = 3
+    cfg = bda.BDHConfig(n_layer=2, n_embd=d, n_head=h, mlp_internal_dim_multiplier=1, vocab_size=V, dropout=0.0)
+    cfg.latent_per_head = lambda: N
+    cfg.fused_kernels.set_rotary_embedding(bda.RotaryEmbedding.ROPE)
+    g = torch.Generator(device=DEV).manual_seed(d)
+    w = {"embed": torch.randn((V, d), device=DEV, generator=g)}
+    for name, shape in (("encoder", (h, d, N)), ("encoder_v", (h, d, N)), ("decoder", (h * N, d)), ("lm_head", (d, V))):
+        w[name] = 0.05 * torch.randn(shape, device=DEV, generator=g)
+    if huge == "embed":
+        w["embed"][1] *= 1e20  # one sequence's row
+    elif huge == "decoder":
+        w["decoder"] *= 1e24
+    model = bda.BDH(cfg, DEV, weights=w)
+    start = torch.randn((2, B, h, N, d), device=DEV, generator=g) * (1e22 if huge == "state" else 0.1)
+    tokens = torch.tensor([[0], [1], [2]], device=DEV)
+    ctx = bda.ffi.default_context(0)
+    logits, after = [], []
+    try:
+        for form in (1, 0):
+            ctx.set_option("model.one_launch", form)
+            state = model.init_state()
+            state.position, state.storage = 5, start.clone()
+            for i, layer in enumerate(state.layers):
+                layer.rho = state.storage[i]
+            logits.append(model.forward_with_state(tokens, state))
+            after.append(state.storage)
+    finally:
+        ctx.set_option("model.one_launch", 1)
+    torch.cuda.synchronize()
+    assert torch.isfinite(logits[1]).all() and torch.isfinite(after[1]).all()
+    assert rel_err(logits[0], logits[1]) < 1e-5
+    assert rel_err(after[0], after[1]) < 1e-5
