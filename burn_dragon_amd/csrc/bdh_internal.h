@@ -57,16 +57,17 @@ struct bdh_model {
   // activation scratch, grown on demand to the largest (B,T) seen
   void *act = nullptr;
   size_t act_bytes = 0;
-  // scratch of the two-launch layer of a model that fits the one-launch step, at most 4 MiB of projection weights; sized at creation for every batch that
-  // form is taken for: a decode step of such a model never allocates, and a captured one keeps its buffer whatever runs later
+  // scratch of the two-launch layer of a model that fits the one-launch step, at most 4 MiB of projection weights; sized at
+  // creation for every batch that form is taken for: a decode step of such a model never allocates, and a captured one keeps
+  // its buffer whatever runs later.  One buffer a model: its steps follow one another, captured ones too.
   float *phase_act = nullptr;
 };
 
 int bdh_fail(bdh_ctx *ctx, int status, const char *fmt, ...);
 
-// model_phase.hip: a decode step in two launches per layer (T = 1, f32 state, 128 <= d <= 512, N a multiple of 32)
+// model_phase.hip: a decode step in two launches per layer (T = 1, 128 <= d <= 512, N a multiple of 32)
 bool bdh_model_phase_fits(const bdh_model *m);
-int bdh_model_phase_most(const bdh_model *m, int rho_dtype, bool lazy);  // sequences
+bool bdh_model_phase_pays(const bdh_model *m, int B, int rho_dtype, bool lazy);
 size_t bdh_model_phase_scratch_floats(const bdh_model *m, int B);
 int bdh_launch_model_phases(bdh_model *m, const int64_t *tokens, int B, float *scratch, void *rho, int rho_dtype, int32_t *stamps,
                             int64_t position,
@@ -78,6 +79,7 @@ int bdh_launch_decoder_finalize(bdh_ctx *ctx, const float *partial, int KBN, int
 
 // model_small.hip: the one-launch decode step of a small model (T = 1, f32 state)
 bool bdh_model_small_fits(const bdh_model_config &c);
+int bdh_model_one_launch_from(const bdh_model_config &c);  // sequences; 0: never
 int bdh_launch_model_small(bdh_model *m, const int64_t *tokens, int B, void *rho, int rho_dtype, int32_t *stamps, int64_t position,
                            const int32_t *positions_dev, float *logits, int64_t *next_tokens);
 

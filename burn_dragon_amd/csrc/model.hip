@@ -10,9 +10,7 @@
 namespace {
 
 // a model that fits the one-launch step, with at most 4 MiB of projection weights
-bool has_phase_act(const bdh_model_config &c) {
-  return bdh_model_small_fits(c) && sizeof(float) * (size_t)3 * c.n_head * c.latent * c.n_embd * c.n_layer <= (size_t(4) << 20);
-}
+bool has_phase_act(const bdh_model_config &c) { return bdh_model_one_launch_from(c) == 1; }
 
 int ensure_act(bdh_model *m, size_t bytes) {
   if (bytes <= m->act_bytes) return BDH_OK;
@@ -109,9 +107,15 @@ int bdh_model_create(bdh_ctx *ctx, const bdh_model_config *c, const bdh_model_we
     return bdh_fail(ctx, BDH_E_HIP, "freqs table upload: %s", hipGetErrorString(e));
   }
   if (has_phase_act(*c) && bdh_model_phase_fits(m)) {
+    // every batch that the two-launch layer is taken for, whatever the state's type
+    auto taken = [&](int B) {
+      return bdh_model_phase_pays(m, B, BDH_F32, false) || bdh_model_phase_pays(m, B, BDH_BF16, false) ||
+             bdh_model_phase_pays(m, B, BDH_BF16, true);
+    };
+    int B = (int)std::min<size_t>(65535, (size_t(480) << 20) / (sizeof(float) * (size_t)3 * c->n_head * c->latent * c->n_embd));
+    while (B > 1 && !taken(B)) --B;
     size_t most = 0;
-    for (int B = bdh_model_phase_most(m, BDH_F32, false); B > 0; --B)  // whatever the state's type: at most 1536
-      most = std::max(most, bdh_model_phase_scratch_floats(m, B));
+    for (; B > 0; --B) most = std::max(most, bdh_model_phase_scratch_floats(m, B));
     if (hipMalloc(reinterpret_cast<void **>(&m->phase_act), sizeof(float) * most) != hipSuccess) {
       (void)hipGetLastError();
       m->phase_act = nullptr;  // such a model takes the one-launch step
@@ -225,21 +229,19 @@ int model_forward_impl(bdh_model *m, const int64_t *tokens, int B, int T, StateR
 
   // A decode step (one token per sequence, no by-products) need not run kernel by kernel:
   //  * a mid-size model (128 <= d <= 512, up to 64 blocks of 64 or 32 neurons) can run TWO launches per layer, a workgroup
-  //    per block; every workgroup streams its share of the layer's weights once per sequence (bdh_model_phase_most);
+  //    per block; every workgroup streams its share of the layer's weights once per sequence (bdh_model_phase_pays);
   //  * a small model (d <= 256, h*N <= 2048) can run the whole step in ONE launch, a workgroup per sequence; one CU then
   //    streams all the projection weights of the step, W bytes.
-  // us per step, one launch | two per layer | kernel by kernel: W = 3 MiB 76|39|112 at B=1, 77|42|- at B=16, 79|57|145 at
-  // B=64, 90|94|- at B=192; 6.75 MiB 129|55|130 at B=1, 143|116|195 at B=64, 165|196|- at B=128; 12 MiB 189|46|123 at B=1,
-  // 205|129|188 at B=64; 96 MiB -|114|308 at B=1, -|309|470 at B=16, -|576|607 at B=32.
+  // us per step, half the neurons firing, one launch | two per layer | kernel by kernel: W = 3 MiB 76|41|103 at B=1, 80|56|121
+  // at B=42, 87|81|137 at B=127; 6.75 MiB 129|55|130 at B=1, 143|116|195 at B=64; 12 MiB 211|47|100 at B=1, 232|149|175 at
+  // B=64; 96 MiB -|114|308 at B=1, -|309|470 at B=16, -|576|607 at B=32.
   if (T == 1 && !x_tap && !viz && !logs && contiguous && ctx->opt_model_one_launch != 0) {
-    const size_t w_bytes = sizeof(float) * (size_t)3 * h * N * d * L;
-    const bool small_fits = bdh_model_small_fits(c);
+    const int one_from = bdh_model_one_launch_from(c);
     const bool small = has_phase_act(c);
-    const bool forced = ctx->opt_model_one_launch == 2 && small_fits;
+    const bool forced = ctx->opt_model_one_launch == 2 && one_from > 0;
     const bool phases = !forced && bdh_model_phase_fits(m) && B <= ctx->opt_model_phase_batch &&
-                        B <= bdh_model_phase_most(m, rho_dtype, stamps != nullptr) && (!small || m->phase_act);
-    const int b_min = small ? 1 : w_bytes <= (size_t(8) << 20) ? 16 : 128;
-    if (forced || (!phases && small_fits && B >= b_min))
+                        bdh_model_phase_pays(m, B, rho_dtype, stamps != nullptr) && (!small || m->phase_act);
+    if (forced || (!phases && one_from > 0 && B >= one_from))
       return bdh_launch_model_small(m, tokens, B, rho, rho_dtype, stamps, position, positions_dev, logits, next_tokens);
     if (phases) {
       int rc2 = small ? BDH_OK : ensure_act(m, sizeof(float) * bdh_model_phase_scratch_floats(m, B));

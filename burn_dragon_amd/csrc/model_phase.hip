@@ -19,6 +19,7 @@
 // on its own copy of the row: no barriers between their sums.  First start to last end of a launch, one sequence, d = 256,
 // 1024 neurons: phase A 9.2 -> 4.3 us, phase B 5.7 -> 2.5; d = 512, 2048 neurons: 12.5 -> 6.6, 7.7 -> 3.5.  The 1.5 us from the
 // end of one launch to the start of the next remain.
+#include <algorithm>
 #include <cfloat>
 
 #include "bdh_internal.h"
@@ -688,28 +689,41 @@ static int block_neurons(const bdh_ctx *ctx, const bdh_model_config &c, int B) {
   return (c.latent & 63) != 0 || (blocks <= 64 && blocks * B <= n_cu) ? 32 : 64;
 }
 
-// The most sequences that the two-launch layer is taken for: while batch x weights of a layer (every workgroup streams its
-// share once per sequence) stay below a bound from measurement.  us a step, two launches per layer | the other form:
-//   a model that the one-launch step takes as well, up to 8 MiB of weights: 3 MiB, 128 sequences 72 to 79 | 84 to 88, 192
-//   sequences 94 to 106 | 90 to 98; 6.75 MiB, 64 sequences 116 | 143, 128 sequences 196 | 165: 128 MiB
-//   f32, 12 MiB a layer, 24 sequences 290 to 535 | 367 to 604 kernel by kernel, 32 sequences 377 to 670 | 377 to 672; 3 MiB a
-//   layer, 128 sequences 214 to 288 | 265 to 327, 192 sequences 336 | 299: 384 MiB
-//   bf16, 12 MiB a layer, 24 sequences 281 to 487 | 287 to 504, 32 sequences 352 to 622 | 317 to 574: 288 MiB
-//   bf16 and lazily decayed, 12 MiB a layer, 128 sequences 1126 to 1839 | 1742 to 2520: 1536 MiB
-//   an odd number of 32-neuron blocks per head, which are not taken two at a time: 0.9 MiB a layer, 64 sequences 79 to 85 |
-//   100 to 117, 128 sequences 121 to 133 | 103 to 118: 72 MiB; 2.5 MiB a layer, 64 sequences 164 to 181 | 174 to 225, 128
-//   sequences 299 to 321 | 217 to 294: 192 MiB
-int bdh_model_phase_most(const bdh_model *m, int rho_dtype, bool lazy) {
+// Whether the two-launch layer is the fastest form of a decode step of B sequences: while batch x weights of a layer (every
+// workgroup streams its share once per sequence) stay below a bound in MiB from measurement.  The other forms leave out more of
+// what inactive neurons do not need, so each line was looked for with half of the neurons firing and with a twentieth (one
+// figure below where every state row is visited whatever fires: PoPE, and ALiBi not lazily decayed).  Time of the other form
+// over that of two launches, half | a twentieth, at so many MiB.  Kernel by kernel:
+//   f32, d = 256 RoPE 288: 1.02 | 0.92, 336: 0.99 | 0.83; ALiBi 384: 1.06; PoPE 384: 0.94 to 1.07.  d = 512 RoPE 288: 1.05 | 1.01, 320: 0.95 | 0.84.
+//     A row between 256 and 512 columns is work for 512: d = 384 RoPE 216: 1.13 | 0.98, 288: 0.98 | 0.82
+//   bf16, d = 256 and 512 (for which the state step has fast kernels) RoPE 192: 1.00 to 1.14 | 0.98 to 1.26, 224: 0.90 to 0.95 | 0.89 to
+//     0.98; ALiBi 224: 0.98 to 1.05, 256: 0.97; lazily decayed 288: 1.28 to 1.81 | 1.07 to 1.34, 381: 1.50 | 0.95, d = 512 576: 1.70 | 1.05.
+//     Other d: d = 192 RoPE 250: 1.44 | 0.93, ALiBi 284: 1.38, PoPE 284: 2.2; d = 384 RoPE 256: 1.23 | 0.97
+//   d = 128, 384: f32 1.11 | 1.02, bf16 1.71 | 1.15; lazily decayed bf16 480: 1.83 | 1.1
+//   an odd number of 32-neuron blocks per head, which are not taken two at a time: f32 RoPE 144: 1.39 | 1.26, 160: 1.01 | 0.85; bf16
+//     162: 1.36 | 0.94; PoPE and ALiBi 192: 1.2 to 1.5
+// One launch for the whole step, where that is the other form: a CU spends it on its sequence's w MiB a layer, and takes the
+// next sequence when it has done one.  w = 0.19 RoPE 48: 1.05 | 1.12, 96 (512 sequences) 1.41 | 1.56; w = 0.38 64: 1.01 | 1.05, 80: 0.99 | 0.98;
+//   w = 0.75 80: 1.15 | 1.09, 96: 1.10 | 1.08, 112: 0.96 | 0.93; w = 1.1 96: 1.12 | 1.04, 112: 1.00 | 0.93; w = 1.7 135: 1.22 | 1.06, 162: 1.01 | 0.90,
+//   PoPE 236: 1.08; w = 3 225: 1.37 | 1.31; odd blocks w = 0.28 45: 1.06 | 1.07, w = 0.84 64: 1.08 | 0.99, 80: 0.96 | 0.86
+bool bdh_model_phase_pays(const bdh_model *m, int B, int rho_dtype, bool lazy) {
   const bdh_model_config &c = m->cfg;
-  const size_t w_layer = sizeof(float) * (size_t)3 * c.n_head * c.latent * c.n_embd;
-  const bool one_launch = bdh_model_small_fits(c) && w_layer * c.n_layer <= (size_t(8) << 20);
-  const size_t mib = (c.latent & 63) != 0    ? (one_launch ? 72 : 192)
-                     : one_launch            ? 128
-                     : rho_dtype != BDH_BF16 ? 384
-                     : lazy                  ? 1536
-                                             : 288;
-  const size_t most = (mib << 20) / w_layer;
-  return most > 65535 ? 65535 : (int)most;
+  const int d = c.n_embd;
+  const double w = sizeof(float) * 3.0 * c.n_head * c.latent * d / (1 << 20), mib = w * B;
+  const bool bf16 = rho_dtype == BDH_BF16, odd = (c.latent & 63) != 0;
+  const bool pope = c.rotary == BDH_POPE, eager = c.rotary == BDH_ALIBI && !lazy;
+  double kernels;
+  if (odd) kernels = bf16 || pope || eager ? 192 : 144;
+  else if (d <= 128) kernels = bf16 && lazy ? 480 : 384;
+  else if (!bf16) kernels = pope ? 384 : d > 256 ? d * 9 / 16 : eager ? 384 : 288;
+  else if (lazy) kernels = d == 256 ? 380 : d == 512 ? 576 : d > 256 ? d * 9 / 16 : 256;
+  else if (d == 256 || d == 512) kernels = eager ? 224 : 192;
+  else kernels = pope || eager ? 288 : 256;
+  if (B > 65535 || mib > kernels) return false;
+  const int from_one = bdh_model_one_launch_from(c), n_cu = m->ctx->n_cu > 0 ? m->ctx->n_cu : 256;
+  if (from_one == 0 || B < from_one) return true;
+  const double one = pope || eager ? 20 + 110 * w : std::max(36 + 60 * w, std::min(44 + 70 * w, 96.0));
+  return mib <= (odd ? 0.71 : 1.0) * one * ((B + n_cu - 1) / n_cu);
 }
 
 size_t bdh_model_phase_scratch_floats(const bdh_model *m, int B) {

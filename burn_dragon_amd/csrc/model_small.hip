@@ -374,6 +374,16 @@ bool bdh_model_small_fits(const bdh_model_config &c) {
   return true;
 }
 
+// From how many sequences on the one-launch step is taken where two launches per layer are not: a CU streams all the weights
+// for its sequence, so the more of them, the more sequences it takes to be worth it (us a step, one launch | kernel by kernel,
+// d = 128 to 256: 3 MiB 1 sequence 76|103; 6.75 MiB 64 sequences 143|195; 12 MiB 128 sequences 247 to 325|181 to 325, 256 457|471).
+// 0: never.
+int bdh_model_one_launch_from(const bdh_model_config &c) {
+  if (!bdh_model_small_fits(c)) return 0;
+  const size_t w_bytes = sizeof(float) * (size_t)3 * c.n_head * c.latent * c.n_embd * c.n_layer;
+  return w_bytes <= (size_t(4) << 20) ? 1 : w_bytes <= (size_t(8) << 20) ? 16 : 128;
+}
+
 int bdh_launch_model_small(bdh_model *m, const int64_t *tokens, int B, void *rho, int rho_dtype, int32_t *stamps,
                            int64_t position,
                            const int32_t *positions_dev, float *logits, int64_t *next_tokens) {

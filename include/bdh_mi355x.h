@@ -118,9 +118,9 @@ const char *bdh_last_error(const bdh_ctx *ctx);
  *                       small enough does not run kernel by kernel: a mid-size model (128 <= d <= 512, N a multiple
  *                       of 64 and at most 64 blocks of 64 neurons, or of 32 and at most 64 blocks of 32, 16-byte
  *                       aligned weights) takes TWO launches per layer, a workgroup per block of neurons, while
- *                       batch x weights of a layer stay under 384 MiB (a bf16 state 288 MiB, lazily decayed 1536 MiB;
- *                       a model of at most 8 MiB of projection weights per step that fits the next form 128 MiB; N no
- *                       multiple of 64: 192 and 72 MiB); a small model (d <= 256 and d % 4 == 0,
+ *                       batch x weights of a layer stay under a bound (by state type, rotary and d between 144 and
+ *                       576 MiB; where the next form is the other one, less) from which on another form is the faster
+ *                       one when few neurons fire; a small model (d <= 256 and d % 4 == 0,
  *                       h * N <= 2048 and a multiple of 32, h in {1,2,4,8,16}, V <= 1024) can take ONE launch
  *                       for the whole step, a workgroup per sequence (where it does not take the other: always for
  *                       up to 4 MiB of projection weights per step, else only for large batches).

@@ -208,3 +208,50 @@ def test_two_launch_layer_norms_of_rows_whose_variance_is_no_float(huge, d, h, N
     assert torch.isfinite(logits[1]).all() and torch.isfinite(after[1]).all()
     assert rel_err(logits[0], logits[1]) < 1e-5
     assert rel_err(after[0], after[1]) < 1e-5
+
+
+def _model_of(d, h, N, layers=1, rotary="rope", dtype="f32", lazy=False, vocab=64):
+    import burn_dragon_amd as bda
+    from burn_dragon_amd import ffi
+
+    cfg = bda.BDHConfig(n_layer=layers, n_embd=d, n_head=h, mlp_internal_dim_multiplier=1, vocab_size=vocab, dropout=0.0)
+    cfg.latent_per_head = lambda: N
+    cfg.fused_kernels.set_rotary_embedding(bda.RotaryEmbedding.parse(rotary))
+    g = torch.Generator(device=DEV).manual_seed(d + N)
+    w = {"embed": torch.randn((vocab, d), device=DEV, generator=g)}
+    for name, shape in (("encoder", (h, d, N)), ("encoder_v", (h, d, N)), ("decoder", (h * N, d)), ("lm_head", (d, vocab))):
+        w[name] = 0.05 * torch.randn(shape, device=DEV, generator=g)
+    return bda.BDH(cfg, DEV, weights=w, alibi_lazy=lazy, rho_dtype=ffi.BF16 if dtype == "bf16" else ffi.F32)
+
+
+def _kernels_of_a_step(model, B):
+    state = model.init_state()
+    model._ensure_state(state, B)
+    state.position = 3
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        model.forward_with_state(torch.zeros((B, 1), device=DEV, dtype=torch.int64), state)
+        torch.cuda.synchronize()
+    return " ".join(e.key for e in prof.key_averages())
+
+
+@pytest.mark.parametrize("d,h,N,layers,kind,most,other", [
+    (128, 4, 128, 4, ("rope", "f32", False), 128, "k_model_step"),     # 3 MiB of weights: a workgroup per sequence behind it
+    (192, 4, 192, 4, ("rope", "f32", False), 81, "k_model_step"),      # 6.75 MiB
+    (192, 4, 192, 4, ("pope", "f32", False), 121, "k_model_step"),     # every row visited whatever fires
+    (256, 4, 256, 4, ("rope", "f32", False), 96, "k_decoder"),         # 3 MiB a layer
+    (256, 4, 256, 4, ("alibi", "f32", False), 127, "k_model_step"),
+    (256, 4, 256, 4, ("rope", "bf16", False), 64, "k_decoder"),
+    (256, 4, 256, 4, ("alibi", "bf16", True), 126, "k_decoder"),
+    (512, 8, 256, 2, ("rope", "bf16", False), 16, "k_decoder"),
+    (384, 4, 384, 2, ("rope", "f32", False), 32, "k_decoder"),         # work for 512 columns
+    (128, 4, 1024, 2, ("rope", "f32", False), 64, "k_decoder"),
+    (192, 4, 96, 4, ("rope", "f32", False), 80, "k_model_step"),       # an odd number of blocks of 32
+    (384, 4, 288, 2, ("rope", "f32", False), 28, "k_decoder"),
+])
+def test_where_the_two_launch_layer_ends(d, h, N, layers, kind, most, other):
+    """The batch from which on another form is faster where few of the neurons fire."""
+    rotary, dtype, lazy = kind
+    model = _model_of(d, h, N, layers, rotary, dtype, lazy)
+    inside, outside = _kernels_of_a_step(model, most), _kernels_of_a_step(model, most + 1)
+    assert "k_layer_phase_a" in inside and "k_layer_phase_b" in inside
+    assert "k_layer_phase" not in outside and other in outside
