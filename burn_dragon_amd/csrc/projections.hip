@@ -1372,13 +1372,17 @@ int bdh_launch_decoder_residual(bdh_ctx *ctx, int B, int T, int h, int N, int d,
   while (KB > 32 && ((K + KB - 1) / KB) * row_tiles < n_cu) KB >>= 1;
   // A batch of decoding sequences: the f32 matrix cores, the same bits; k-blocks of 1024 with a chain each once those fill
   // half the chip in 32 x 64 tiles (a negative option value -r: from r sequences on, whatever the size).  The VALU kernel
-  // skips the rows of E that no sequence needs and reads the others once per eight sequences: it is the better one for fewer
-  // than 24 sequences with long rows (us a step, VALU | this: d = 512, E of 268 MB, 8 sequences 5045 | 5115; of 67 MB, 16
-  // sequences 1941 | 1944), and for fewer than 8 unless E is small (d = 256, E of 34 MB, 3 sequences 458 | 490, 8 sequences
-  // 818 | 753; E of 17 MB, 9 sequences 396 | 331, 2 sequences 238 | 230; d = 192, 6 MB, 7 sequences 179 | 171).
+  // skips the rows of E that no sequence needs and reads the others once per eight sequences: the longer the rows, the larger E
+  // and the fewer neurons fire, the longer it is the better one.  Its time a step over this kernel's, half of the neurons firing |
+  // a twentieth: E of 4 to 8 MiB, 2 sequences 1.02 to 1.06 | 1.00 to 1.02; d = 256, 10 to 16 MiB, 2 sequences 0.95 to 1.03 | 0.90 to
+  // 0.96, 3 sequences 1.04 to 1.09 | 0.98 to 1.02, 32 MiB, 8 sequences 1.09 | 1.05, 48 MiB 1.04 | 0.95; d = 128, 64 MiB, 8 sequences 1.07 |
+  // 1.04; d = 384 to 768, 10 to 16 MiB, 2 sequences 0.92 to 0.97 | 0.88 to 0.95, 8 sequences 0.99 to 1.02 | 0.96 to 1.01, 12 sequences 1.00
+  // to 1.06 | 0.97 to 1.07.
   const int sk_rows = ctx->opt_decoder_splitk_rows;
   const long many = std::abs(sk_rows);
-  const long few = many > 24 ? many : std::min<long>(many, K * d <= (4L << 20) ? 2 : d <= 256 ? 8 : 24);
+  const long mib = (K * d * 4 + (1L << 20) - 1) >> 20;
+  const long few = many > 24 ? many
+                   : std::min<long>(many, mib <= 8 ? 2 : d > 256 ? (mib <= 16 ? 12 : 24) : mib <= 16 ? 3 : d <= 128 || mib <= 32 ? 8 : 24);
   if (T == 1 && M >= few && (K & 3) == 0 && bdh_aligned(xy, 16) && bdh_aligned(decoder, 16)) {
     const bool split = M >= many && K % 1024 == 0 &&
                        (sk_rows < 0 || K / 1024 * ((d + 63) / 64) * ((M + 31) / 32) >= n_cu / 2);

@@ -109,8 +109,9 @@ const char *bdh_last_error(const bdh_ctx *ctx);
  *                       the matrix cores, 0 = always the VALU kernel.
  *   "decoder.splitk_rows": 24 (default) a decode step (T = 1) of this many or more sequences runs the
  *                       encoder E on the f32 matrix cores (all of E is streamed): the bits of the VALU kernel, which fewer
- *                       sequences take and which skips the inactive rows of E.  With a value of at most 24, eight sequences
- *                       and more with d <= 256, and two and more with an E of at most 16 MiB, take it too (the same bits).
+ *                       sequences take and which skips the inactive rows of E.  With a value of at most 24, two sequences
+ *                       and more with an E of at most 8 MiB take it too (the same bits), with an E of up to 16 MiB three and
+ *                       more (d > 256: twelve), with d <= 256 and up to 32 MiB (d <= 128: any) eight and more.
  *                       From this many sequences on, where k-blocks of 1024 fill half the chip,
  *                       one chain per block instead (values agree to 1e-5).  A negative value -r takes that second form
  *                       from r sequences on whatever the size (h * N a multiple of 1024).

@@ -255,3 +255,29 @@ def test_where_the_two_launch_layer_ends(d, h, N, layers, kind, most, other):
     inside, outside = _kernels_of_a_step(model, most), _kernels_of_a_step(model, most + 1)
     assert "k_layer_phase_a" in inside and "k_layer_phase_b" in inside
     assert "k_layer_phase" not in outside and other in outside
+
+
+@pytest.mark.parametrize("d,h,N,first", [
+    (512, 8, 512, 2),     # 8 MiB
+    (512, 8, 576, 12),    # 9 MiB
+    (512, 8, 1088, 24),   # 17 MiB
+    (256, 4, 2052, 3),    # a little over 8 MiB
+    (256, 4, 4096, 3),    # 16 MiB
+    (256, 4, 4100, 8),
+    (256, 4, 8192, 8),    # 32 MiB
+    (256, 4, 8196, 24),
+    (128, 4, 17000, 8),
+])
+def test_where_the_encoder_of_a_batch_takes_the_matrix_cores(d, h, N, first):
+    """Below this batch the kernel that skips the rows of inactive neurons is the faster one where few of them fire."""
+    import burn_dragon_amd as bda
+
+    model = _model_of(d, h, N, rotary="alibi")
+    ctx = bda.ffi.default_context(0)
+    ctx.set_option("model.one_launch", 0)
+    try:
+        below, there = _kernels_of_a_step(model, first - 1), _kernels_of_a_step(model, first)
+    finally:
+        ctx.set_option("model.one_launch", 1)
+    assert "k_decoder_partial" in below and "k_decoder_rows" not in below
+    assert "k_decoder_rows" in there and "k_decoder_partial" not in there
