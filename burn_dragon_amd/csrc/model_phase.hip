@@ -57,6 +57,13 @@ __device__ __forceinline__ V load_at(const T *p, unsigned int at) {
   return *reinterpret_cast<const V *>(reinterpret_cast<const char *>(p) + at);
 }
 
+// Four weights of a caller's array, which floats may begin at any address of theirs: one 16-byte load all the same.
+__device__ __forceinline__ float4 load_weights(const float *p, unsigned int at) {
+  typedef float Quad __attribute__((ext_vector_type(4), aligned(4)));
+  const Quad q = load_at<Quad>(p, at);
+  return make_float4(q.x, q.y, q.z, q.w);
+}
+
 // Orders a wave's own LDS writes and reads of other lanes' values for the compiler (the hardware runs them in order).
 __device__ __forceinline__ void wave_lds_order() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -155,7 +162,7 @@ struct Project {
     unsigned int at = (min(k0, d - 1) * N + (threadIdx.x & (S::LPW - 1)) * 4) * 4u;
 #pragma unroll
     for (int u = 0; u < S::KR; ++u) {
-      w[u] = load_at<float4>(weight, at);
+      w[u] = load_weights(weight, at);
       at += k0 + u < d - 1 ? N * 4u : 0u;  // not beyond the last row
     }
   }
@@ -477,7 +484,7 @@ __global__ __launch_bounds__(NW * 64, 2) void k_layer_phase_b(PhaseArgs a) {
 #pragma unroll
     for (int j = 0; j < S::VPL; ++j) {
       const int c = (j * S::LPR + cl) * 4;
-      ev[u][j] = load_at<float4>(e, (sub * d + (c < d ? c : 0)) * 4u);
+      ev[u][j] = load_weights(e, (sub * d + (c < d ? c : 0)) * 4u);
     }
   }
 
@@ -674,9 +681,7 @@ bool bdh_model_phase_fits(const bdh_model *m) {
   if (c.latent < 32 || (c.latent & 31) != 0) return false;  // whole blocks of 64 or 32 neurons
   if (c.n_head < 1 || c.n_head > 64 || c.n_layer < 1) return false;
   // every workgroup of a sequence sums the partials of all the others: only while those are few
-  if ((long)c.n_head * (c.latent / ((c.latent & 63) == 0 ? 64 : 32)) > 64) return false;
-  // 16-byte loads
-  return bdh_aligned(m->w.encoder, 16) && bdh_aligned(m->w.encoder_v, 16) && bdh_aligned(m->w.decoder, 16);
+  return (long)c.n_head * (c.latent / ((c.latent & 63) == 0 ? 64 : 32)) <= 64;
 }
 
 // Neurons of a workgroup's block.  A head whose N is no multiple of 64 takes 32.  For the others: fewer neurons share the

@@ -117,11 +117,11 @@ const char *bdh_last_error(const bdh_ctx *ctx);
  *                       from r sequences on whatever the size (h * N a multiple of 1024).
  *   "model.one_launch": 1 (default) a decode step (T = 1, no x_tap / viz) of a model that is
  *                       small enough does not run kernel by kernel: a mid-size model (128 <= d <= 512, N a multiple
- *                       of 64 and at most 64 blocks of 64 neurons, or of 32 and at most 64 blocks of 32, 16-byte
- *                       aligned weights) takes TWO launches per layer, a workgroup per block of neurons, while
- *                       batch x weights of a layer stay under a bound (by state type, rotary and d between 144 and
- *                       576 MiB; where the next form is the other one, less) from which on another form is the faster
- *                       one when few neurons fire; a small model (d <= 256 and d % 4 == 0,
+ *                       of 64 and at most 64 blocks of 64 neurons, or of 32 and at most 64 blocks of 32) takes TWO
+ *                       launches per layer, a workgroup per block of neurons, while batch x weights of a layer stay
+ *                       under a bound (by state type, rotary and d between 144 and 576 MiB; where the next form is
+ *                       the other one, less) from which on another form is the faster one when few neurons fire; a
+ *                       small model (d <= 256 and d % 4 == 0,
  *                       h * N <= 2048 and a multiple of 32, h in {1,2,4,8,16}, V <= 1024) can take ONE launch
  *                       for the whole step, a workgroup per sequence (where it does not take the other: always for
  *                       up to 4 MiB of projection weights per step, else only for large batches).
