@@ -23,7 +23,8 @@ struct GemmF32 {
   int lda2 = 0, ldb2 = 0, K2 = 0;
   // What is done with the sums.
   //   GEMM_STORE   C = acc, or C += acc (accumulate); with decay_rows the A . B part of row t is scaled by g^t; with
-  //                decay_state token k of A is scaled by g^(K-k) and C = g^K C + acc
+  //                decay_state token k of A is scaled by g^(K-k) and C = g^K C + acc.  The two that read C take it in one
+  //                piece (rows_per == 0), others are refused.
   //   GEMM_SCORES  square, C zero above the diagonal of the block pattern, see the fields below
   //   GEMM_NORM    C = acc / (sum_k |A[m,k]| + 1e-6)
   int epilogue = 0;

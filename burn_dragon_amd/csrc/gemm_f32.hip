@@ -382,7 +382,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_f32(GemmF32 g) {
       }
     return;
   }
-  if (EPI == GEMM_STORE && (g.accumulate || g.decay_state) && g.rows_per == 0) {
+  if (EPI == GEMM_STORE && (g.accumulate || g.decay_state)) {  // C in one piece: the launcher sees to it
     // C = C + acc or g^K C + acc: all of this wave's elements are asked for before the first is used.  (The L2's adder, one
     // no-return add per element, took 215 us where this takes 176: 12 slices of [8192 x 500] x [500 x 256].)
     float old[MI][NJ][16];
@@ -542,6 +542,8 @@ GemmPlan bdh_gemm_f32_plan(const bdh_ctx *ctx, const GemmF32 &g, int max_split) 
 int bdh_gemm_f32_rows(const GemmPlan &plan) { return kTileM[plan.tile]; }
 
 int bdh_launch_gemm_f32(bdh_ctx *ctx, GemmF32 g, bool a_kmajor, bool b_kmajor, const GemmPlan &plan, float *partial) {
+  if ((g.accumulate || g.decay_state) && g.rows_per > 0)
+    return bdh_fail(ctx, BDH_E_UNSUPPORTED, "a product that is added to what C holds takes C in one piece");
   g.mt = (g.M + kTileM[plan.tile] - 1) / kTileM[plan.tile];
   g.nt = (g.N + kTileN[plan.tile] - 1) / kTileN[plan.tile];
   g.tri = lower_triangle(g, plan.tile);
