@@ -211,10 +211,6 @@ __global__ __launch_bounds__(NTHR) void k_relu_lowrank_row1(RowArgs a, int d, co
   }
   __syncthreads();
   {
-    auto wave_sum = [](float v) {
-      for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-      return v;
-    };
     float4 vals[4];
     float s = 0.0f;
 #pragma unroll
@@ -233,7 +229,7 @@ __global__ __launch_bounds__(NTHR) void k_relu_lowrank_row1(RowArgs a, int d, co
       vals[j] = v;
     }
     auto layer_norm4 = [&](float total) {  // vals <- (vals - mean) / sqrt(var + eps) over the d columns
-      const float mean = wave_sum(total) / (float)d;
+      const float mean = bdh_wave_sum(total) / (float)d;
       float q = 0.0f;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
