@@ -215,7 +215,10 @@ __global__ __launch_bounds__(256) void k_scores_reduce(const float *__restrict__
 }
 
 // out[slice][t0 + t][:] = the sum of the parts [part][slice][tc][d], in order, and, when out_ln is given, its LayerNorm
-// (src/model/bdh.rs:359).  One wavefront per row, d <= 1024.
+// (src/model/bdh.rs:359).  One wavefront per row, d <= 64 * J.  What bounds it: the trips to memory, one for U parts of the whole
+// row (one part and 64 columns at a time, us: 32 parts, 140 rows of 384 25.8 | 6.2; 8 parts, 786 rows of 512 19.2 | 5.2; 2 parts, 5496 rows of
+// 128 5.0 | 4.9).
+template <int J, int U>
 __global__ __launch_bounds__(256) void k_rows_reduce(const float *__restrict__ parts, int ks, long c_split, int tc, int d,
                                                      long rows, float *__restrict__ out, float *__restrict__ out_ln,
                                                      long slice_stride) {
@@ -223,28 +226,42 @@ __global__ __launch_bounds__(256) void k_rows_reduce(const float *__restrict__ p
   const long r = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (r >= rows) return;
   const long o = r / tc * slice_stride + r % tc * d;
-  float v[16], s = 0.0f;
+  const float *p = parts + r * d;
+  float v[J], s = 0.0f;
+  int col[J];
 #pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    const int c = j * 64 + lane;
+  for (int j = 0; j < J; ++j) {
+    col[j] = min(j * 64 + lane, d - 1);
     v[j] = 0.0f;
-    if (c < d) {
-      for (int k = 0; k < ks; ++k) v[j] += parts[k * c_split + r * d + c];
-      out[o + c] = v[j];
+  }
+  for (int k = 0; k < ks; k += U) {
+    float x[U][J];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int j = 0; j < J; ++j) x[u][j] = p[min(k + u, ks - 1) * c_split + col[j]];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (k + u < ks) {
+#pragma unroll
+        for (int j = 0; j < J; ++j) v[j] += x[u][j];
+      }
+  }
+#pragma unroll
+  for (int j = 0; j < J; ++j)
+    if (j * 64 + lane < d) {
+      out[o + j * 64 + lane] = v[j];
       s += v[j];
     }
-  }
   if (!out_ln) return;
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
-  const float mean = s / (float)d;
+  const float mean = bdh_wave_sum(s) / (float)d;
   float q = 0.0f;
 #pragma unroll
-  for (int j = 0; j < 16; ++j)
+  for (int j = 0; j < J; ++j)
     if (j * 64 + lane < d) q += (v[j] - mean) * (v[j] - mean);
-  for (int off = 32; off > 0; off >>= 1) q += __shfl_xor(q, off);
-  const float den = sqrtf(q / (float)d + kLnEps);
+  const float den = sqrtf(bdh_wave_sum(q) / (float)d + kLnEps);
 #pragma unroll
-  for (int j = 0; j < 16; ++j)
+  for (int j = 0; j < J; ++j)
     if (j * 64 + lane < d) out_ln[o + j * 64 + lane] = (v[j] - mean) / den;
 }
 
@@ -898,7 +915,8 @@ int bdh_launch_state_chunks_f32(bdh_ctx *ctx, const StateStepParams &p, float *o
     if (rc != BDH_OK) return rc;
     if (c.p_out.ks > 1) {
       const long rows = S * tc;
-      hipLaunchKernelGGL(k_rows_reduce, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, ctx->stream, parts, c.p_out.ks,
+      auto *kernel = d <= 256 ? k_rows_reduce<4, 8> : d <= 512 ? k_rows_reduce<8, 4> : k_rows_reduce<16, 2>;
+      hipLaunchKernelGGL(kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, ctx->stream, parts, c.p_out.ks,
                          rows * d, tc, d, rows, p.out + (long)t0 * d, out_ln ? out_ln + (long)t0 * d : nullptr, (long)T * d);
       BDH_LAUNCH_CHECK(ctx, "k_rows_reduce");
       normed = tc == T;
