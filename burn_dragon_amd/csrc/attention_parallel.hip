@@ -481,7 +481,7 @@ __global__ __launch_bounds__(256) void k_relu_lowrank_direct(RlArgs g) {
 // 8 cycles a step and row tile where the 32 x 32 instruction takes 32, and a few rows give four times the wavefronts: what
 // bounds it is the stream of the weights, every one of them copied to LDS once per 16 * RT rows.
 // Where the workgroups are few, it is the chain of waits: a stage's copies are NS - 1 stages ahead, its operands are read
-// into registers while those of the stage before are multiplied, and the gate is asked for at the start (us, before | now, D_x
+// into registers while those of the stage before are multiplied, and the gate is asked for with the first copies (us, before | now, D_x
 // and D_y of a decode step: 8 heads of 256, d = 512, 48 sequences 10.5 | 8.2; 4 heads of 4096, d = 256, 3 sequences 8.0 | 6.1).
 // us per call, the VALU and matrix-core kernels it took over from | this: 8192, 512, 48 rows 52.5 | 11.5; 32768, 256, 16 rows
 // 29.7 | 8.4; 131072, 512 (268 MB of weights), 16 rows 57.9 | 47.8, 32 rows 65.5 | 58.6.
@@ -542,7 +542,8 @@ __global__ __launch_bounds__(256) void k_relu_lowrank_rows(RlArgs g) {
   const int col = n0 + wave * 16 + r;
   const int stages = g.d / SK;
   for (int s = 0; s < NS - 1 && s < stages; ++s) issue(s);
-  // behind the first copies: these values are needed last, and their trip to memory is the chain's to hide
+  // Behind the first copies, so that their trip to memory runs beside those of the first stages.  The waits below count them
+  // as well: the first stage is used when these are there too, not only its own copies.
   float gv[RT][4];
   if (g.gate) {
 #pragma unroll

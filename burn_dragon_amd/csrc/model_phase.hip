@@ -336,7 +336,7 @@ __global__ __launch_bounds__(NW * 64, AHEAD || DC == 512 ? 2 : 4) void k_layer_p
   }
   wave_lds_order();
 
-  // x = relu(cur . encoder - thr) for the 64 neurons (src/model/bdh.rs:337-351), the same in every wave
+  // x = relu(cur . encoder - thr) for the block's neurons (src/model/bdh.rs:337-351), the same in every wave
   float xn = dx.dot(s_cur[wave], d, s_acc);
   if (a.thr != 0.0f) xn = xn - a.thr;
   xn = xn > 0.0f ? xn : 0.0f;
@@ -499,7 +499,7 @@ __global__ __launch_bounds__(NW * 64, 2) void k_layer_phase_b(PhaseArgs a) {
     for (int j = 0; j < S::CJ; ++j) s_in[wave][j * 64 + lane] = j * 64 + lane < d ? at[j] : 0.0f;
     wave_lds_order();
   }
-  // xy = x * relu(LN(attn) . encoder_v - thr) for the 64 neurons (src/model/bdh.rs:361-381), the same in every wave
+  // xy = x * relu(LN(attn) . encoder_v - thr) for the block's neurons (src/model/bdh.rs:361-381), the same in every wave
   float y = dy.dot(s_in[wave], d, s_acc);
   if (a.thr != 0.0f) y = y - a.thr;
   const float xy = gate * (y > 0.0f ? y : 0.0f);

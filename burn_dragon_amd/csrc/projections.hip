@@ -603,7 +603,8 @@ __global__ __launch_bounds__(256) void k_decoder_partial(const float *__restrict
 // every row of E read once per 16 * RT sequences instead of once per eight.  (SPLIT: the k-blocks of 1024 of the form for
 // many sequences and a large E, one chain per block that runs 0, 8, 1, 9, ..., 7, 15 through each 16.)
 // A workgroup takes the k-blocks [blk * bpw, +bpw) and adds their sums in order: bpw is a sixteenth of the blocks, as
-// k_decoder_finalize would group them, or one.
+// k_decoder_finalize would group them, or one; with SPLIT as many as leave four workgroups for every CU, and at most 64 parts
+// (launch_decoder_rows).
 // Tile 16 * RT x 64, copied straight to LDS 32 k at a time into a ring of NS stages, the operands of a stage read into registers
 // while those of the stage before are multiplied.  What bounds it: the trips to memory of a few workgroups per CU, which is
 // why the copies run NS - 1 stages ahead (two stages | now, us: 48 sequences, K = 2048, d = 512 6.3 | 5.6; 60, 16384, 256

@@ -28,6 +28,8 @@
  *     call's product and write it back, one thread per element and call; no atomic add is used.
  *   - bdh_ctx_set_stream only swaps the stream: the context's workspace is shared by all of its calls, so the
  *     caller orders the old stream's queued work before the new stream's (an event), or uses one context per stream.
+ *     A model's calls share its scratch in the same way, captured ones too: graphs that hold steps of one model are
+ *     replayed one after another, not side by side on two streams.
  */
 #ifndef BDH_MI355X_H
 #define BDH_MI355X_H
