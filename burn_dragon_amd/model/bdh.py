@@ -174,7 +174,8 @@ class BDH:
         """Captures ONE greedy decode step (forward_with_state on the last sampled token, argmax kept on
         the device, position advanced on the device) in a HIP graph.  Every replay is one token for
         every sequence of the batch; nothing crosses to the host between tokens (the reference syncs
-        and copies the logits every token, src/generation.rs:114-124)."""
+        and copies the logits every token, src/generation.rs:114-124).  Graphs of one model share its scratch:
+        their replays follow one another, on one stream or ordered by events."""
         return DecodeGraph(self, state, tokens)
 
     def forward(self, tokens: torch.Tensor) -> torch.Tensor:

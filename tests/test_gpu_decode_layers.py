@@ -31,6 +31,7 @@ def rel_err(a, b):
     (512, 2, 1024, 64, 1, True),    # 64 blocks of 32
     (128, 1, 2016, 33, 2, True),    # 63 blocks of 32
     (256, 4, 128, 256, 2, False),   # weights four bytes off
+    (128, 1, 128, 64, 400, True),   # more sequences than a chip of 256 takes in one round of the one-launch step
 ])
 def test_two_launch_layer_edges(state, rotary, lazy, d, h, N, V, B, aligned):
     import burn_dragon_amd as bda
