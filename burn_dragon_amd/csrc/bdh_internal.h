@@ -201,7 +201,6 @@ struct ReluLowrankRowParams {
   const int64_t *tokens = nullptr;  // mode 3: device, the one token; partial = the embedding table, rows = V
 };
 int bdh_launch_relu_lowrank_row(bdh_ctx *ctx, const ReluLowrankRowParams &p);
-bool bdh_relu_lowrank_row_fits(int d, int rows);
 // The first stage of the encoder for one row (M = 1): partial[kb][:] = sum over k-block kb of xy[k] E[k,:], KB rows
 // per block; *KBN_out = number of blocks.  partial must hold KBN * d floats.
 int bdh_launch_decoder_partial_row(bdh_ctx *ctx, int h, int N, int d, const float *xy, const float *decoder, int KB,

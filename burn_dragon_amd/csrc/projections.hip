@@ -110,16 +110,21 @@ __global__ __launch_bounds__(NTHR) void k_relu_lowrank(const float *__restrict__
 // One input row per head that the kernel makes itself (a decode step of one sequence).  The reductions of a layer whose
 // inputs come from other CUs -- the sum of the state step's readout partials with its LayerNorm (src/model/bdh.rs:359),
 // the sum of the encoder's partials with the two LayerNorms and the residual (:436-441) -- run in front of the
-// projection that consumes their result, in every workgroup, behind the workgroup's first UK weight loads: as launches
+// projection that consumes their result, in every workgroup, in front of the workgroup's weight loads: as launches
 // of their own each is a launch gap plus a chain of dependent trips to memory.
 //   MODE 1: row(hh) = LN(sum_g partial[hh][g][:])                      rows = S partial rows per head
 //   MODE 2: row     = LN(cur_old + LN(sum_kb partial[kb][:]))          rows = KBN, the same row for every head;
 //           workgroup (0, 0) writes it to cur_new (another buffer than cur_old: other workgroups still read that)
 //   MODE 3: row     = LN(embed[tokens[0]][:])   (src/model/bdh.rs:319-322; a token outside [0, V) gives a NaN row, as
 //           k_embed_ln does)                      partial = the embedding table, rows = V; written to cur_new too
-// The NW waves split the partial rows, a lane owns four adjacent columns of up to four column groups (d <= 1024),
-// every wave then finishes the row on its own with wave shuffles (the same arithmetic in every wave and workgroup, so
-// all of them hold the same bits).  Then k_relu_lowrank's one k-sequential fmaf chain per output.
+// What bounds it: the stream of the weights, in one trip to memory.  A workgroup of 16 wavefronts owns CW columns and every
+// wavefront a sixteenth of k: 16 bytes a lane, all of a workgroup's weights on their way at once, behind the partial rows,
+// which are needed first.  The waves split the partial rows, D threads add up the waves' sums, every wave makes the
+// LayerNorms itself (the same arithmetic in all of them, so they hold the same bits); a column's sum is sixteen chains of
+// D / 16 fused multiply-adds, added in order.  4 heads of 8192 neurons, D = 256 (32 MiB of weights), us, a thread per column
+// and a chain of D terms in four trips | now: MODE 1 9.0 | 8.5, MODE 2 10.6 | 9.5 (3.5 to 3.9 TB/s of weights
+// that the state's stream has driven out of the caches), a token of 6 layers 242 | 230.
+// PIECES: rows of W are whole, aligned 16-byte pieces; else the same lanes read their columns one by one.
 struct RowArgs {
   const float *partial;
   int rows;
@@ -128,164 +133,148 @@ struct RowArgs {
   const int64_t *tokens;  // MODE 3
 };
 
-template <int MODE, int UK, int NTHR>
-__global__ __launch_bounds__(NTHR) void k_relu_lowrank_row1(RowArgs a, int d, const float *__restrict__ w, int h, int N,
-                                                           float thr, const float *__restrict__ gate,
-                                                           float *__restrict__ out) {
-  constexpr int NW = NTHR / 64;
-  extern __shared__ float s_row[];  // [d] the finished row | [NW][d] the waves' partial sums
-  float *s_in = s_row;
-  float *s_grp = s_row + d;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+template <int MODE, int D, int CW, bool PIECES>
+__global__ __launch_bounds__(1024) void k_relu_lowrank_row1(RowArgs a, const float *__restrict__ w, int N, float thr,
+                                                           const float *__restrict__ gate, float *__restrict__ out) {
+  constexpr int NW = 16, SPAN = D / NW;        // waves, k of a wave
+  constexpr int LANES = CW / 4, RPI = 64 / LANES;  // lanes to a row of W, rows to an access
+  constexpr int NL = SPAN / RPI;               // accesses of a lane
+  constexpr int J = D / 256, U = 8 / J;        // column groups of a lane, partial rows on their way at a time
+  __shared__ __attribute__((aligned(16))) float s_grp[NW * D];  // the waves' sums of the partial rows, then of the products
+  __shared__ __attribute__((aligned(16))) float s_in[D];        // the sum of the partial rows, then the finished row
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hh = blockIdx.y;
-  const int n = blockIdx.x * NTHR + tid;
-  const bool col = n < N;
-  const float *wp = w + (long)hh * d * N + (col ? n : 0);
-  float wv[UK];
-  const float *src = a.partial + (MODE == 1 ? (long)hh * a.rows * d : 0);
+  const int n0 = blockIdx.x * CW;
+  const float *src = a.partial + (MODE == 1 ? (long)hh * a.rows * D : 0);
   int n_rows = a.rows;
   bool bad_token = false;
   if (MODE == 3) {
     const long tok = a.tokens[0];
     bad_token = tok < 0 || tok >= a.rows;
-    src = a.partial + (bad_token ? 0 : tok) * d;
+    src = a.partial + (bad_token ? 0 : tok) * D;
     n_rows = 1;
   }
   const int per = (n_rows + NW - 1) / NW;
   const int r0 = min(n_rows, wave * per), r1 = min(n_rows, r0 + per);
-  // Order of the requests (a wavefront has at most 63 memory operations outstanding and they complete in issue order):
-  // the first 32 partial rows of the lane's first column group, then the first UK weight rows, so that the row is
-  // being made while the weights are on their way (d >= UK).
-  const bool head32 = r0 + 32 <= r1;  // uniform over the wave
-  float4 t0[32];
-  if (head32) {
+  // Loads come back in the order of their issue: the first U partial rows of every column group, then the weights, so that
+  // the row is made while the weights are on their way.  (No loads under a branch: rows past the end repeat the last one.)
+  float4 t[U][J];
 #pragma unroll
-    for (int u = 0; u < 32; ++u) t0[u] = *reinterpret_cast<const float4 *>(src + (long)(r0 + u) * d + lane * 4);
-  }
+  for (int u = 0; u < U; ++u)
 #pragma unroll
-  for (int u = 0; u < UK; ++u) wv[u] = wp[(long)u * N];
-  float4 res[4];
+    for (int j = 0; j < J; ++j)
+      t[u][j] = *reinterpret_cast<const float4 *>(src + (long)min(r0 + u, n_rows - 1) * D + (j * 64 + lane) * 4);
+  float4 res[J];
   if (MODE == 2) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int c = (j * 64 + lane) * 4;
-      res[j] = c < d ? *reinterpret_cast<const float4 *>(a.cur_old + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int j = 0; j < J; ++j) res[j] = *reinterpret_cast<const float4 *>(a.cur_old + (j * 64 + lane) * 4);
+  }
+  const int c = n0 + (lane % LANES) * 4, k_lane = wave * SPAN + lane / LANES;
+  float4 wv[NL];
+  {
+    const float *wp = w + ((long)hh * D + k_lane) * N;
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const float *p = wp + (long)i * RPI * N;
+      if (PIECES)
+        wv[i] = *reinterpret_cast<const float4 *>(p + min(c, N - 4));  // four columns are all in or all out
+      else
+        wv[i] = make_float4(p[min(c, N - 1)], p[min(c + 1, N - 1)], p[min(c + 2, N - 1)], p[min(c + 3, N - 1)]);
     }
   }
+  const bool mine = tid < CW && n0 + tid < N;  // this thread finishes a column
+  float gv = 1.0f;
+  if (gate) gv = gate[(long)hh * N + min(n0 + min(tid, CW - 1), N - 1)];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int c = (j * 64 + lane) * 4;
-    if (c < d) {
-      float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-      int r = r0;
-      if (j == 0 && head32) {
+  for (int j = 0; j < J; ++j) {
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-        for (int u = 0; u < 32; ++u) {
-          v.x += t0[u].x; v.y += t0[u].y; v.z += t0[u].z; v.w += t0[u].w;
-        }
-        r += 32;
+    for (int u = 0; u < U; ++u)
+      if (r0 + u < r1) {
+        v.x += t[u][j].x; v.y += t[u][j].y; v.z += t[u][j].z; v.w += t[u][j].w;
       }
-      for (; r + 32 <= r1; r += 32) {  // 32 rows in flight: the sum is a chain of trips to the L2
-        float4 t[32];
-#pragma unroll
-        for (int u = 0; u < 32; ++u) t[u] = *reinterpret_cast<const float4 *>(src + (long)(r + u) * d + c);
-#pragma unroll
-        for (int u = 0; u < 32; ++u) {
-          v.x += t[u].x; v.y += t[u].y; v.z += t[u].z; v.w += t[u].w;
-        }
-      }
-      if (r < r1) {  // up to 31 rows left: all asked for at once
-        float4 t[31];
-#pragma unroll
-        for (int u = 0; u < 31; ++u)
-          t[u] = r + u < r1 ? *reinterpret_cast<const float4 *>(src + (long)(r + u) * d + c) : make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-        for (int u = 0; u < 31; ++u)
-          if (r + u < r1) {
-            v.x += t[u].x; v.y += t[u].y; v.z += t[u].z; v.w += t[u].w;
-          }
-      }
-      if (MODE == 3 && bad_token) v = make_float4(NAN, NAN, NAN, NAN);
-      *reinterpret_cast<float4 *>(s_grp + wave * d + c) = v;
+    for (int r = r0 + U; r < r1; ++r) {  // (more partial rows than 16 * U)
+      const float4 x = *reinterpret_cast<const float4 *>(src + (long)r * D + (j * 64 + lane) * 4);
+      v.x += x.x; v.y += x.y; v.z += x.z; v.w += x.w;
     }
+    if (MODE == 3 && bad_token) v = make_float4(NAN, NAN, NAN, NAN);
+    *reinterpret_cast<float4 *>(s_grp + wave * D + (j * 64 + lane) * 4) = v;
   }
   __syncthreads();
-  {
-    float4 vals[4];
-    float s = 0.0f;
+  if (tid < D) {
+    float v = s_grp[tid];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int c = (j * 64 + lane) * 4;
-      float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (c < d) {
-        v = *reinterpret_cast<const float4 *>(s_grp + c);
+    for (int g = 1; g < NW; ++g) v += s_grp[g * D + tid];
+    s_in[tid] = v;
+  }
+  __syncthreads();
+  float4 vals[J];
+  float s = 0.0f;
 #pragma unroll
-        for (int g = 1; g < NW; ++g) {
-          const float4 t = *reinterpret_cast<const float4 *>(s_grp + g * d + c);
-          v.x += t.x; v.y += t.y; v.z += t.z; v.w += t.w;
-        }
-        s += (v.x + v.y) + (v.z + v.w);
-      }
-      vals[j] = v;
+  for (int j = 0; j < J; ++j) {
+    vals[j] = *reinterpret_cast<const float4 *>(s_in + (j * 64 + lane) * 4);
+    s += (vals[j].x + vals[j].y) + (vals[j].z + vals[j].w);
+  }
+  auto layer_norm4 = [&](float total) {  // vals <- (vals - mean) / sqrt(var + eps) over the D columns
+    const float mean = bdh_wave_sum(total) / (float)D;
+    float q = 0.0f;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      vals[j].x -= mean; vals[j].y -= mean; vals[j].z -= mean; vals[j].w -= mean;
+      q += (vals[j].x * vals[j].x + vals[j].y * vals[j].y) + (vals[j].z * vals[j].z + vals[j].w * vals[j].w);
     }
-    auto layer_norm4 = [&](float total) {  // vals <- (vals - mean) / sqrt(var + eps) over the d columns
-      const float mean = bdh_wave_sum(total) / (float)d;
-      float q = 0.0f;
+    const float den = sqrtf(bdh_wave_sum(q) / (float)D + kLnEps);
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if ((j * 64 + lane) * 4 < d) {
-          const float tx = vals[j].x - mean, ty = vals[j].y - mean, tz = vals[j].z - mean, tw = vals[j].w - mean;
-          q += (tx * tx + ty * ty) + (tz * tz + tw * tw);
-        }
-      const float den = sqrtf(bdh_wave_sum(q) / (float)d + kLnEps);
+    for (int j = 0; j < J; ++j) {
+      vals[j].x /= den; vals[j].y /= den; vals[j].z /= den; vals[j].w /= den;
+    }
+  };
+  layer_norm4(s);
+  if (MODE == 2) {
+    s = 0.0f;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        vals[j].x = (vals[j].x - mean) / den; vals[j].y = (vals[j].y - mean) / den;
-        vals[j].z = (vals[j].z - mean) / den; vals[j].w = (vals[j].w - mean) / den;
-      }
-    };
+    for (int j = 0; j < J; ++j) {
+      vals[j].x += res[j].x; vals[j].y += res[j].y; vals[j].z += res[j].z; vals[j].w += res[j].w;
+      s += (vals[j].x + vals[j].y) + (vals[j].z + vals[j].w);
+    }
     layer_norm4(s);
-    if (MODE == 2) {
-      s = 0.0f;
+  }
+  __syncthreads();  // every wave has read the sums
+  if (wave == 0) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if ((j * 64 + lane) * 4 < d) {
-          vals[j].x += res[j].x; vals[j].y += res[j].y; vals[j].z += res[j].z; vals[j].w += res[j].w;
-          s += (vals[j].x + vals[j].y) + (vals[j].z + vals[j].w);
-        }
-      layer_norm4(s);
-    }
-    if (wave == 0) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int c = (j * 64 + lane) * 4;
-        if (c < d) {
-          *reinterpret_cast<float4 *>(s_in + c) = vals[j];
-          if (MODE != 1 && blockIdx.x == 0 && hh == 0) *reinterpret_cast<float4 *>(a.cur_new + c) = vals[j];
-        }
-      }
+    for (int j = 0; j < J; ++j) {
+      *reinterpret_cast<float4 *>(s_in + (j * 64 + lane) * 4) = vals[j];
+      if (MODE != 1 && blockIdx.x == 0 && hh == 0) *reinterpret_cast<float4 *>(a.cur_new + (j * 64 + lane) * 4) = vals[j];
     }
   }
   __syncthreads();
 
-  float acc = 0.0f;
+  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-  for (int u = 0; u < UK; ++u) acc = __builtin_fmaf(s_in[u], wv[u], acc);
-  int k0 = UK;
-  for (; k0 + UK <= d; k0 += UK) {
-#pragma unroll
-    for (int u = 0; u < UK; ++u) wv[u] = wp[(long)(k0 + u) * N];
-#pragma unroll
-    for (int u = 0; u < UK; ++u) acc = __builtin_fmaf(s_in[k0 + u], wv[u], acc);
+  for (int i = 0; i < NL; ++i) {
+    const float x = s_in[k_lane + i * RPI];
+    acc.x = __builtin_fmaf(x, wv[i].x, acc.x);
+    acc.y = __builtin_fmaf(x, wv[i].y, acc.y);
+    acc.z = __builtin_fmaf(x, wv[i].z, acc.z);
+    acc.w = __builtin_fmaf(x, wv[i].w, acc.w);
   }
-  for (; k0 < d; ++k0) acc = __builtin_fmaf(s_in[k0], wp[(long)k0 * N], acc);
-  if (!col) return;
-  float pv = acc;
+#pragma unroll
+  for (int o = LANES; o < 64; o <<= 1) {  // the rows of an access
+    acc.x += __shfl_xor(acc.x, o);
+    acc.y += __shfl_xor(acc.y, o);
+    acc.z += __shfl_xor(acc.z, o);
+    acc.w += __shfl_xor(acc.w, o);
+  }
+  if (lane < LANES) *reinterpret_cast<float4 *>(s_grp + wave * CW + lane * 4) = acc;
+  __syncthreads();
+  if (!mine) return;
+  float pv = s_grp[tid];
+#pragma unroll
+  for (int g = 1; g < NW; ++g) pv += s_grp[g * CW + tid];
   if (thr != 0.0f) pv = pv - thr;
   float y = pv > 0.0f ? pv : 0.0f;
-  const long o = (long)hh * N + n;
-  if (gate) y = gate[o] * y;
-  out[o] = y;
+  if (gate) y = gv * y;
+  out[(long)hh * N + n0 + tid] = y;
 }
 
 // A few input rows against a SMALL weight matrix (a few MiB: it sits in the L2): with one thread per column there
@@ -1418,23 +1407,32 @@ int bdh_launch_decoder_residual(bdh_ctx *ctx, int B, int T, int h, int N, int d,
   return BDH_OK;
 }
 
-bool bdh_relu_lowrank_row_fits(int d, int rows) { return d >= 64 && d <= 1024 && (d & 3) == 0 && rows >= 1; }
-
 int bdh_launch_relu_lowrank_row(bdh_ctx *ctx, const ReluLowrankRowParams &p) {
-  if (!bdh_relu_lowrank_row_fits(p.d, p.rows)) return bdh_fail(ctx, BDH_E_SHAPE, "fused row projection: d=%d rows=%d", p.d, p.rows);
-  constexpr int NTHR = 128, UK = 64;
-  const dim3 grid((p.N + NTHR - 1) / NTHR, p.h);
-  const size_t lds = sizeof(float) * (size_t)p.d * (1 + NTHR / 64);
+  if ((p.d != 256 && p.d != 512) || p.N < 1 || p.rows < 1)
+    return bdh_fail(ctx, BDH_E_SHAPE, "fused row projection: d=%d N=%d rows=%d", p.d, p.N, p.rows);
   const RowArgs a{p.partial, p.rows, p.cur_old, p.cur_new, p.tokens};
-  if (p.mode == 1)
-    hipLaunchKernelGGL((k_relu_lowrank_row1<1, UK, NTHR>), grid, dim3(NTHR), lds, ctx->stream, a, p.d, p.weight, p.h, p.N,
-                       p.threshold, p.gate, p.out);
-  else if (p.mode == 3)
-    hipLaunchKernelGGL((k_relu_lowrank_row1<3, UK, NTHR>), grid, dim3(NTHR), lds, ctx->stream, a, p.d, p.weight, p.h, p.N,
-                       p.threshold, p.gate, p.out);
-  else
-    hipLaunchKernelGGL((k_relu_lowrank_row1<2, UK, NTHR>), grid, dim3(NTHR), lds, ctx->stream, a, p.d, p.weight, p.h, p.N,
-                       p.threshold, p.gate, p.out);
+  const bool pieces = p.N % 4 == 0 && bdh_aligned(p.weight, 16);
+  // Columns of a workgroup: a workgroup for every CU if narrower ones give that; wider ones add up the partial rows less often.
+  const long n_cu = ctx->n_cu > 0 ? ctx->n_cu : 256;
+  auto groups = [&](int cw) { return (long)((p.N + cw - 1) / cw) * p.h; };
+  const int cw = groups(128) >= n_cu ? 128 : groups(64) >= n_cu ? 64 : 32;
+  const dim3 grid((p.N + cw - 1) / cw, p.h);
+#define BDH_ROW1(MODE_, D_, CW_, PIECES_)                                                                                   \
+  hipLaunchKernelGGL((k_relu_lowrank_row1<MODE_, D_, CW_, PIECES_>), grid, dim3(1024), 0, ctx->stream, a, p.weight, p.N, \
+                     p.threshold, p.gate, p.out)
+#define BDH_ROW1_P(MODE_, D_, CW_) \
+  do { if (pieces) BDH_ROW1(MODE_, D_, CW_, true); else BDH_ROW1(MODE_, D_, CW_, false); } while (0)
+#define BDH_ROW1_C(MODE_, D_) \
+  do { if (cw == 128) BDH_ROW1_P(MODE_, D_, 128); else if (cw == 64) BDH_ROW1_P(MODE_, D_, 64); else BDH_ROW1_P(MODE_, D_, 32); } while (0)
+#define BDH_ROW1_D(MODE_) \
+  do { if (p.d == 256) BDH_ROW1_C(MODE_, 256); else BDH_ROW1_C(MODE_, 512); } while (0)
+  if (p.mode == 1) BDH_ROW1_D(1);
+  else if (p.mode == 2) BDH_ROW1_D(2);
+  else BDH_ROW1_D(3);
+#undef BDH_ROW1_D
+#undef BDH_ROW1_C
+#undef BDH_ROW1_P
+#undef BDH_ROW1
   BDH_LAUNCH_CHECK(ctx, "k_relu_lowrank_row1");
   return BDH_OK;
 }

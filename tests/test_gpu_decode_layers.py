@@ -83,6 +83,57 @@ def test_two_launch_layer_edges(state, rotary, lazy, d, h, N, V, B, aligned):
         assert torch.equal(states[0].stamps, states[1].stamps)
 
 
+@pytest.mark.parametrize("d,h,N,aligned", [
+    (256, 4, 8192, True),   # 128 columns a workgroup, one for every CU of a chip of 256
+    (256, 4, 8190, True),   # ... the last one not full, rows that are no whole 16-byte pieces
+    (256, 4, 4100, True),   # 64 columns a workgroup, the last one with four
+    (256, 4, 8192, False),  # weights four bytes off
+    (512, 1, 70, True),     # 32 columns a workgroup, one partial row
+    (512, 2, 4092, True),
+    (512, 1, 4092, False),
+])
+def test_projections_of_one_row_that_make_their_row(d, h, N, aligned):
+    """The four-launch layer at the edges of its projections' workgroups, against the kernel-by-kernel step: sums of at most
+    512 terms in another order, 1e-5."""
+    import burn_dragon_amd as bda
+
+    V = 64
+    cfg = bda.BDHConfig(n_layer=2, n_embd=d, n_head=h, mlp_internal_dim_multiplier=1, vocab_size=V, dropout=0.0)
+    cfg.latent_per_head = lambda: N
+    cfg.fused_kernels.set_rotary_embedding(bda.RotaryEmbedding.ROPE)
+    g = torch.Generator(device=DEV).manual_seed(d + N)
+    w = {"embed": torch.randn((V, d), device=DEV, generator=g)}
+    for name, shape in (("encoder", (h, d, N)), ("encoder_v", (h, d, N)), ("decoder", (h * N, d)), ("lm_head", (d, V))):
+        w[name] = 0.05 * torch.randn(shape, device=DEV, generator=g)
+    if not aligned:  # four bytes off
+        for name, t in w.items():
+            flat = torch.empty(t.numel() + 1, device=DEV)
+            flat[1:] = t.reshape(-1)
+            w[name] = flat[1:].view(t.shape)
+    models = [bda.BDH(cfg, DEV, weights=w) for _ in range(2)]
+    assert all((t.data_ptr() % 16 == 0) == aligned for t in models[0].params.values())
+    ctx = bda.ffi.default_context(0)
+    states = [m.init_state() for m in models]
+    start = 0.1 * torch.randn((2, 1, h, N, d), device=DEV, generator=g)
+    for m, s in zip(models, states):
+        m._ensure_state(s, 1)
+        s.storage.copy_(start)
+        s.position = 5
+    tokens = torch.randint(0, V, (3, 1, 1), device=DEV, generator=g)
+    assert "k_relu_lowrank_row1" in _kernels_of_a_step(models[0], 1)
+    for t in range(3):
+        got, nxt = models[0].forward_with_state(tokens[t], states[0], want_next=True)
+        try:
+            ctx.set_option("model.fused_rows", 0)
+            ref = models[1].forward_with_state(tokens[t], states[1])
+        finally:
+            ctx.set_option("model.fused_rows", 1)
+        torch.cuda.synchronize()
+        assert rel_err(got, ref) < 1e-5, t
+        assert torch.equal(nxt.reshape(-1), got[:, 0].argmax(-1))
+    assert rel_err(states[0].storage, states[1].storage) < 1e-5
+
+
 @pytest.mark.parametrize("d", [32, 64, 96, 160, 512])
 @pytest.mark.parametrize("B,T,h,N", [(2, 1, 3, 4), (5, 3, 2, 60), (17, 1, 3, 68), (33, 1, 1, 260), (63, 1, 2, 64),
                                      (20, 1, 2, 40960), (40, 1, 1, 66000)])
