@@ -483,14 +483,17 @@ __global__ __launch_bounds__(256) void k_relu_lowrank_direct(RlArgs g) {
 // Where the workgroups are few, it is the chain of waits: a stage's copies are NS - 1 stages ahead, its operands are read
 // into registers while those of the stage before are multiplied, and the gate is asked for with the first copies (us, before | now, D_x
 // and D_y of a decode step: 8 heads of 256, d = 512, 48 sequences 10.5 | 8.2; 4 heads of 4096, d = 256, 3 sequences 8.0 | 6.1).
+// WHOLE: LDS holds all NS stages of d = 32 NS, the whole tile is on its way before the first wait, four stages to a barrier
+// (us, ring of four | whole: d = 512, 32 to 256 workgroups 8.2 | 6.5, d = 256, up to 512 of them 5.6 | 4.5; what is left is the chain
+// of d / 4 instructions, 32 cycles each).
 // us per call, the VALU and matrix-core kernels it took over from | this: 8192, 512, 48 rows 52.5 | 11.5; 32768, 256, 16 rows
 // 29.7 | 8.4; 131072, 512 (268 MB of weights), 16 rows 57.9 | 47.8, 32 rows 65.5 | 58.6.
-template <int RT, int NS>
+template <int RT, int NS, bool WHOLE>
 __global__ __launch_bounds__(256) void k_relu_lowrank_rows(RlArgs g) {
   typedef float f32x4 __attribute__((ext_vector_type(4)));
   constexpr int BM = 16 * RT, BN = 64, SK = 32;
   constexpr int STAGE = (BM + BN) * SK;
-  extern __shared__ __attribute__((aligned(1024))) float s_tiles[];  // NS stages of A [BM][32], W [32][64]
+  __shared__ __attribute__((aligned(1024))) float s_tiles[NS * STAGE];  // NS stages of A [BM][32], W [32][64]
   const int tiles = g.mt * g.nt, total = g.h * tiles;  // the launcher keeps the total within an int
   const int xcd = blockIdx.x & 7;
   const int lo = (int)((long)total * xcd / 8), hi = (int)((long)total * (xcd + 1) / 8);
@@ -540,12 +543,10 @@ __global__ __launch_bounds__(256) void k_relu_lowrank_rows(RlArgs g) {
   // where element e of row tile i of this lane goes (element e of lane l: row = (l/16)*4 + e, column = l%16), its gate
   const int r = lane & 15, q = lane >> 4;
   const int col = n0 + wave * 16 + r;
-  const int stages = g.d / SK;
-  for (int s = 0; s < NS - 1 && s < stages; ++s) issue(s);
-  // Behind the first copies, so that their trip to memory runs beside those of the first stages.  The waits below count them
-  // as well: the first stage is used when these are there too, not only its own copies.
+  const int stages = WHOLE ? NS : g.d / SK;
   float gv[RT][4];
-  if (g.gate) {
+  auto ask_gate = [&]() {
+    if (!g.gate) return;
 #pragma unroll
     for (int i = 0; i < RT; ++i)
 #pragma unroll
@@ -554,6 +555,16 @@ __global__ __launch_bounds__(256) void k_relu_lowrank_rows(RlArgs g) {
         place(min(m0 + i * 16 + q * 4 + e, g.M - 1), b, t);
         gv[i][e] = g.gate[(((long)b * g.h + hh) * g.T + t) * g.N + min(col, g.N - 1)];
       }
+  };
+  if constexpr (WHOLE) {
+    ask_gate();
+#pragma unroll
+    for (int s = 0; s < NS; ++s) issue(s);
+  } else {
+    for (int s = 0; s < NS - 1 && s < stages; ++s) issue(s);
+    // Behind the first copies, so that their trip to memory runs beside those of the first stages.  The waits below count
+    // them as well: the first stage is used when these are there too, not only its own copies.
+    ask_gate();
   }
   f32x4 acc[RT];
 #pragma unroll
@@ -588,12 +599,29 @@ __global__ __launch_bounds__(256) void k_relu_lowrank_rows(RlArgs g) {
     read(s, into);
     if (s > 0) multiply(into ^ 1);
   };
-  for (int s = 0; s < stages; s += 2) {  // two at a time: the registers have fixed names
-    step(s, 0);
-    if (s + 1 < stages) step(s + 1, 1);
+  if constexpr (WHOLE) {
+    constexpr int GRP = 4;  // stages to a wait and a barrier
+    static_assert(NS % GRP == 0, "whole groups, the last stage's operands in the second set");
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      if (s % GRP == 0) {  // the next GRP stages are there for every wave
+        if (carries_a) bdh_wait_for_stage<2 + CA, NS - GRP>(NS - GRP - s);
+        else bdh_wait_for_stage<2, NS - GRP>(NS - GRP - s);
+        __syncthreads();
+      }
+      read(s, s & 1);
+      __builtin_amdgcn_sched_barrier(0);  // left alone, the scheduler sinks these reads to their use
+      if (s > 0) multiply((s & 1) ^ 1);
+    }
+    multiply(1);
+  } else {
+    for (int s = 0; s < stages; s += 2) {  // two at a time: the registers have fixed names
+      step(s, 0);
+      if (s + 1 < stages) step(s + 1, 1);
+    }
+    if (stages & 1) multiply(0);
+    else multiply(1);
   }
-  if (stages & 1) multiply(0);
-  else multiply(1);
   if (col >= g.N) return;
   const float bv = g.bias ? g.bias[(long)hh * g.N + col] : 0.0f;
   float mk = 1.0f;
@@ -1028,13 +1056,15 @@ int bdh_launch_relu_lowrank_gemm(bdh_ctx *ctx, const ReluLowrankParams &p, const
 #define BDH_RLD(KERNEL_, ROWS_, COLS_) \
   hipLaunchKernelGGL((KERNEL_), grid, dim3(256), 2 * (ROWS_ + COLS_) * 32 * sizeof(float), ctx->stream, g)
   // Stages of the ring: more copies in flight where the workgroups are too few to cover each other's trips, fewer where LDS
-  // decides how many of them a CU holds (us, two | four stages: 96 workgroups 9.3 | 8.3, 256 6.8 | 6.1, 1024 13.8 | 15.0).
-#define BDH_RLR(RT_, NS_) \
-  hipLaunchKernelGGL((k_relu_lowrank_rows<RT_, NS_>), grid, dim3(256), NS_ * (16 * RT_ + 64) * 32 * sizeof(float), ctx->stream, g)
-  if (rt == 1 && total <= 2 * n_cu) BDH_RLR(1, 4);
-  else if (rt == 1) BDH_RLR(1, 2);
-  else if (rt == 2) BDH_RLR(2, 3);
-  else if (rt == 4) BDH_RLR(4, 2);
+  // decides how many of them a CU holds (us, two | four stages: 96 workgroups 9.3 | 8.3, 256 6.8 | 6.1, 1024 13.8 | 15.0); all of
+  // them where the 10 KiB a stage leave a CU its share of the workgroups: one with d = 512, two with d = 256.
+#define BDH_RLR(RT_, NS_, WHOLE_) hipLaunchKernelGGL((k_relu_lowrank_rows<RT_, NS_, WHOLE_>), grid, dim3(256), 0, ctx->stream, g)
+  if (rt == 1 && total <= n_cu && g.d == 512) BDH_RLR(1, 16, true);
+  else if (rt == 1 && total <= 2 * n_cu && g.d == 256) BDH_RLR(1, 8, true);
+  else if (rt == 1 && total <= 2 * n_cu) BDH_RLR(1, 4, false);
+  else if (rt == 1) BDH_RLR(1, 2, false);
+  else if (rt == 2) BDH_RLR(2, 3, false);
+  else if (rt == 4) BDH_RLR(4, 2, false);
 #undef BDH_RLR
   else if (big) BDH_RLD((k_relu_lowrank_direct<128, 128>), 128, 128);
   else if (direct) BDH_RLD((k_relu_lowrank_direct<64, 64>), 64, 64);

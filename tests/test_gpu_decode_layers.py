@@ -134,11 +134,11 @@ def test_projections_of_one_row_that_make_their_row(d, h, N, aligned):
     assert rel_err(states[0].storage, states[1].storage) < 1e-5
 
 
-@pytest.mark.parametrize("d", [32, 64, 96, 160, 512])
+@pytest.mark.parametrize("d", [32, 64, 96, 160, 256, 512])
 @pytest.mark.parametrize("B,T,h,N", [(2, 1, 3, 4), (5, 3, 2, 60), (17, 1, 3, 68), (33, 1, 1, 260), (63, 1, 2, 64),
                                      (20, 1, 2, 40960), (40, 1, 1, 66000)])
 def test_projection_rings_keep_the_bits_of_the_scalar_chain(d, B, T, h, N):
-    """1 to 16 stages of 32 k through rings of 2, 3 and 4; row tiles of 16, 32 and 64; bias, mask and gate: the bits of the
+    """1 to 16 stages of 32 k through rings of 2, 3 and 4 and, where there are few workgroups, all of them at once; row tiles of 16, 32 and 64; bias, mask and gate: the bits of the
     thread-per-column kernel, which adds the same products in the same order."""
     import burn_dragon_amd as bda
     from burn_dragon_amd.kernel import relu_lowrank
