@@ -174,6 +174,11 @@ int bdh_ctx_set_option(bdh_ctx *ctx, const char *name, int value) {
     ctx->opt_lowrank_row = value;
     return BDH_OK;
   }
+  if (strcmp(name, "state_step.past_caches") == 0) {
+    if (value < -1 || value > 1) return bdh_fail(ctx, BDH_E_INVAL, "state_step.past_caches takes -1, 0 or 1");
+    ctx->opt_step_past_caches = value;
+    return BDH_OK;
+  }
   if (strcmp(name, "state_step.dense_kernel") == 0) {
     if (value < 0 || value > 1) return bdh_fail(ctx, BDH_E_INVAL, "state_step.dense_kernel takes 0 or 1");
     ctx->opt_step_dense_kernel = value;

@@ -30,6 +30,7 @@ struct bdh_ctx {
   int opt_model_phase_batch = 1 << 30;  // two launches per layer for a decode step of at most this many sequences (0: never)
   int opt_lowrank_gemm_rows = 64;  // relu_lowrank of 64 rows and more takes the f32 matrix cores from this many on (0: never)
   int opt_lowrank_mfma_rows = 2;  // relu_lowrank of fewer than 64 rows takes the f32 matrix cores from this many on (0: never)
+  int opt_step_past_caches = -1;  // -1: by what passes between two visits of a row; 0 / 1: never / always
   int opt_step_dense_kernel = 1;  // 0: PoPE / eager ALiBi at d in {256,512} take the generic kernel
   int opt_decoder_splitk_rows = 24;  // decode-step encoder on the matrix cores from this many sequences on
   int opt_ws_max_mib = 0;   // the workspace never grows beyond this (0: no limit)
@@ -131,6 +132,8 @@ struct StateStepParams {
   // T = 1 on the RoPE kernels (d in {256, 512}) only: leave the readout as the per-workgroup partial sums
   // [B*h][S][d] in the context's workspace (the caller's next kernel adds them up): no second stage, `out` unused
   struct StepPartials *partials_out = nullptr;
+  // bytes of all the states and weights that the caller's step walks before it comes back to this state; 0: not known
+  size_t walked = 0;
 };
 struct StepPartials {
   const float *partial = nullptr;

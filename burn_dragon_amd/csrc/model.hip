@@ -220,6 +220,8 @@ int model_forward_impl(bdh_model *m, const int64_t *tokens, int B, int T, StateR
   const size_t M = (size_t)B * T;
   st.layer_bytes = (size_t)B * h * Nq * d * (rho_dtype == BDH_BF16 ? 2 : 4);
   st.stamps_layer = (size_t)B * h * N;
+  // what passes between two visits of a layer's state: every layer's state and the weights, which all layers share
+  const size_t walked = st.layer_bytes * L + sizeof(float) * 3 * (size_t)h * N * d;
   for (int l = 0; l < L; ++l)
     if (!bdh_aligned(st.rho(l), 16)) return bdh_fail(ctx, BDH_E_ALIGN, "rho needs 16-byte alignment");
   // the fused decode forms below walk one allocation: layers given one by one take them only when they are adjacent
@@ -295,7 +297,7 @@ int model_forward_impl(bdh_model *m, const int64_t *tokens, int B, int T, StateR
       if (rc2 != BDH_OK) return rc2;
       StepPartials sp;
       StateStepParams ps{1, h, 1, N, d, c.rotary, rho_dtype, xr, cur_a, m->freqs, position, positions_dev, nullptr,
-                         st.rho(l), nullptr, nullptr, nullptr, nullptr, &sp};
+                         st.rho(l), nullptr, nullptr, nullptr, nullptr, &sp, walked};
       rc2 = bdh_launch_state_steps(ctx, ps);
       if (rc2 != BDH_OK) return rc2;
       // :359,370-381  xy = x * relu(LN(sum of the readout partials) . encoder_v - thr)
@@ -335,7 +337,8 @@ int model_forward_impl(bdh_model *m, const int64_t *tokens, int B, int T, StateR
                                           attn_ln, nullptr, nullptr);
     } else {
       StateStepParams ps{B, h, T, N, d, c.rotary, rho_dtype, x_l, cur, m->freqs, position, positions_dev,
-                         c.rotary == BDH_ALIBI ? m->slopes : nullptr, st.rho(l), attn, nullptr, nullptr, st.stamps(l)};
+                         c.rotary == BDH_ALIBI ? m->slopes : nullptr, st.rho(l), attn, nullptr, nullptr, st.stamps(l),
+                         nullptr, walked};
       rc = bdh_launch_state_steps_ln(ctx, ps, attn_ln);
     }
     if (rc != BDH_OK) return rc;

@@ -49,13 +49,29 @@ struct StepPtrs {
   long x_t_stride = 0, v_t_stride = 0, partial_t_stride = 0, cnt_t_stride = 0, bm_t_stride = 0;
 };
 
+// One access of a state row.  NT: the row goes past the caches (see stream_past_caches below for when).
+template <bool NT, typename V>
+__device__ __forceinline__ V state_load(const V *p) {
+  typedef unsigned int Quad __attribute__((ext_vector_type(4)));
+  if constexpr (!NT) return *p;
+  else if constexpr (sizeof(V) == 16) return __builtin_bit_cast(V, __builtin_nontemporal_load(reinterpret_cast<const Quad *>(p)));
+  else return __builtin_nontemporal_load(p);
+}
+template <bool NT, typename V>
+__device__ __forceinline__ void state_store(V *p, V v) {
+  typedef unsigned int Quad __attribute__((ext_vector_type(4)));
+  if constexpr (!NT) *p = v;
+  else if constexpr (sizeof(V) == 16) __builtin_nontemporal_store(__builtin_bit_cast(Quad, v), reinterpret_cast<Quad *>(p));
+  else __builtin_nontemporal_store(v, p);
+}
+
 // ------------------------------------------------------------------------------------
 // fast path: RoPE, f32 state, D in {256, 512}
 // ------------------------------------------------------------------------------------
 // SPLIT > 1: the workgroup still has WAVES waves but owns only WAVES*64/SPLIT lane pairs; the
 // first WAVES/SPLIT waves compact them and all waves walk the list.  Used when there are few
 // (b,h) slices, so that a small batch still spreads over every CU with enough loads in flight.
-template <int D, int WAVES, int U, int SPLIT, bool MULTI>
+template <int D, int WAVES, int U, int SPLIT, bool MULTI, bool NT>
 __global__ __launch_bounds__(WAVES * 64) void k_step_rope_f32(StepPtrs a, float *__restrict__ rho) {
   constexpr int VPL = D / 256;             // float4 per lane per row
   constexpr int PPB = WAVES * 64 / SPLIT;  // lane pairs per workgroup
@@ -162,8 +178,8 @@ __global__ __launch_bounds__(WAVES * 64) void k_step_rope_f32(StepPtrs a, float 
         const float4 *rp = reinterpret_cast<const float4 *>(base + (long)s_idx[i] * (2 * D));
 #pragma unroll
         for (int j = 0; j < VPL; ++j) {
-          r0[u][j] = rp[j * 64 + lane];
-          r1[u][j] = rp[D / 4 + j * 64 + lane];
+          r0[u][j] = state_load<NT>(rp + j * 64 + lane);
+          r1[u][j] = state_load<NT>(rp + D / 4 + j * 64 + lane);
         }
       }
     }
@@ -196,8 +212,8 @@ __global__ __launch_bounds__(WAVES * 64) void k_step_rope_f32(StepPtrs a, float 
           t = qq.y * vj.y; o.y = o.y + t;
           t = qq.y * vj.z; o.z = o.z + t;
           t = qq.y * vj.w; o.w = o.w + t;
-          wp[j * 64 + lane] = e;
-          wp[D / 4 + j * 64 + lane] = o;
+          state_store<NT>(wp + j * 64 + lane, e);
+          state_store<NT>(wp + D / 4 + j * 64 + lane, o);
         }
       }
     }
@@ -229,7 +245,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_step_rope_f32(StepPtrs a, float 
 // owns a neuron also reads its stamp, turns it into the catch-up factor decay^(clock - stamp)
 // and writes the new stamp clock + 1.
 // ------------------------------------------------------------------------------------
-template <int D, int WAVES, int U>
+template <int D, int WAVES, int U, bool NT>
 __global__ __launch_bounds__(WAVES * 64) void k_step_alibi_lazy_f32(StepPtrs a, float *__restrict__ rho,
                                                                    int32_t *__restrict__ stamps, HeadScalars decay,
                                                                    HeadScalars log_decay) {
@@ -325,7 +341,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_step_alibi_lazy_f32(StepPtrs a, 
       if (i < total) {
         const float4 *rp = reinterpret_cast<const float4 *>(base + (long)s_idx[i] * D);
 #pragma unroll
-        for (int j = 0; j < VPL; ++j) r[u][j] = rp[j * 64 + lane];
+        for (int j = 0; j < VPL; ++j) r[u][j] = state_load<NT>(rp + j * 64 + lane);
       }
     }
 #pragma unroll
@@ -348,7 +364,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_step_alibi_lazy_f32(StepPtrs a, 
           t = qs.x * vj.y; e.y = (e.y + t) * dec;
           t = qs.x * vj.z; e.z = (e.z + t) * dec;
           t = qs.x * vj.w; e.w = (e.w + t) * dec;
-          wp[j * 64 + lane] = e;
+          state_store<NT>(wp + j * 64 + lane, e);
         }
       }
     }
@@ -373,7 +389,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_step_alibi_lazy_f32(StepPtrs a, 
 // fast path: RoPE, bf16 state (f32 accumulate), D in {256, 512}.  A lane pair's two rows are
 // 4*D contiguous bytes; each lane owns D/256 16-byte pieces (8 bf16) of that chunk.
 // ------------------------------------------------------------------------------------
-template <int D, int WAVES, int U, int SPLIT>
+template <int D, int WAVES, int U, int SPLIT, bool NT>
 __global__ __launch_bounds__(WAVES * 64) void k_step_rope_bf16(StepPtrs a, unsigned short *__restrict__ rho) {
   constexpr int PL = D / 256;      // 16-byte pieces per lane per pair (D=256: 1, D=512: 2)
   constexpr int PPB = WAVES * 64 / SPLIT;
@@ -469,7 +485,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_step_rope_bf16(StepPtrs a, unsig
       if (i < total) {
         const uint4 *rp = reinterpret_cast<const uint4 *>(base + (long)s_idx[i] * (2 * D));
 #pragma unroll
-        for (int j = 0; j < PL; ++j) r[u][j] = rp[j * 64 + lane];
+        for (int j = 0; j < PL; ++j) r[u][j] = state_load<NT>(rp + j * 64 + lane);
       }
     }
 #pragma unroll
@@ -493,7 +509,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_step_rope_bf16(StepPtrs a, unsig
             hi = hi + t1;
             o[k] = pack_bf16_rne(lo, hi);
           }
-          wp[j * 64 + lane] = make_uint4(o[0], o[1], o[2], o[3]);
+          state_store<NT>(wp + j * 64 + lane, make_uint4(o[0], o[1], o[2], o[3]));
         }
       }
     }
@@ -524,14 +540,14 @@ __global__ __launch_bounds__(WAVES * 64) void k_step_rope_bf16(StepPtrs a, unsig
 constexpr int kGenRows = 64;
 constexpr int kGenMaxCols = 16;  // d <= 64 * 16
 
-template <typename RhoT>
-__device__ __forceinline__ float rho_load(const RhoT *p);
-template <>
-__device__ __forceinline__ float rho_load<float>(const float *p) { return *p; }
-template <>
-__device__ __forceinline__ float rho_load<unsigned short>(const unsigned short *p) { return bf16_to_f32(*p); }
-__device__ __forceinline__ void rho_store(float *p, float v) { *p = v; }
-__device__ __forceinline__ void rho_store(unsigned short *p, float v) { *p = f32_to_bf16(v); }
+template <bool NT>
+__device__ __forceinline__ float rho_load(const float *p) { return state_load<NT>(p); }
+template <bool NT>
+__device__ __forceinline__ float rho_load(const unsigned short *p) { return bf16_to_f32(state_load<NT>(p)); }
+template <bool NT>
+__device__ __forceinline__ void rho_store(float *p, float v) { state_store<NT>(p, v); }
+template <bool NT>
+__device__ __forceinline__ void rho_store(unsigned short *p, float v) { state_store<NT>(p, f32_to_bf16(v)); }
 
 // Per state row (all d columns) of the generic path: readout with the old row, rank-1 update, optional
 // decay; a lazily decayed row is brought up to date first.
@@ -540,7 +556,7 @@ __device__ __forceinline__ void rho_store(unsigned short *p, float v) { *p = f32
 // decay^(clock - stamps[n]).  Only rows with a non-zero activation are read, brought up to date,
 // updated, decayed once (src/model/bdh.rs:299-301) and stamped clock+1; all other rows are left
 // alone, so the step stays as sparse as the activations.
-template <typename RhoT, int MAXC, int FL>  // d <= 64 * MAXC; FL state rows in flight per wave
+template <typename RhoT, int MAXC, int FL, bool NT>  // d <= 64 * MAXC; FL state rows in flight per wave
 __global__ __launch_bounds__(256) void k_step_generic(StepPtrs a, RhoT *__restrict__ rho, int d, int Nq,
                                                       int rotary, int has_decay, HeadScalars decay,
                                                       HeadScalars log_decay, int32_t *__restrict__ stamps) {
@@ -626,7 +642,7 @@ __global__ __launch_bounds__(256) void k_step_generic(StepPtrs a, RhoT *__restri
 #pragma unroll
         for (int j = 0; j < MAXC; ++j) {
           const int c = j * 64 + lane;
-          if (j < ncol && c < d) rv[u][j] = rho_load<RhoT>(row + c);
+          if (j < ncol && c < d) rv[u][j] = rho_load<NT>(row + c);
         }
       }
     }
@@ -647,7 +663,7 @@ __global__ __launch_bounds__(256) void k_step_generic(StepPtrs a, RhoT *__restri
             const float outer = qn * vv[j];
             r = r + outer;
             if (has_dec) r = r * dec;
-            rho_store(row + c, r);
+            rho_store<NT>(row + c, r);
           }
         }
       }
@@ -708,17 +724,20 @@ struct DenseRaw;  // the same VW values as they lie in memory
 template <>
 struct DenseRaw<float, 4> {
   float4 r;
-  __device__ __forceinline__ void load(const float *p) { r = *reinterpret_cast<const float4 *>(p); }
+  template <bool NT>
+  __device__ __forceinline__ void load(const float *p) { r = state_load<NT>(reinterpret_cast<const float4 *>(p)); }
   __device__ __forceinline__ DensePiece<4> wide() const { return {{r.x, r.y, r.z, r.w}}; }
+  template <bool NT>
   static __device__ __forceinline__ void store(float *p, const DensePiece<4> &e) {
-    *reinterpret_cast<float4 *>(p) = make_float4(e.v[0], e.v[1], e.v[2], e.v[3]);
+    state_store<NT>(reinterpret_cast<float4 *>(p), make_float4(e.v[0], e.v[1], e.v[2], e.v[3]));
   }
 };
 template <int VW>
 struct DenseRaw<unsigned short, VW> {
   typedef unsigned int words __attribute__((ext_vector_type(VW / 2)));
   words r;
-  __device__ __forceinline__ void load(const unsigned short *p) { r = *reinterpret_cast<const words *>(p); }
+  template <bool NT>
+  __device__ __forceinline__ void load(const unsigned short *p) { r = state_load<NT>(reinterpret_cast<const words *>(p)); }
   __device__ __forceinline__ DensePiece<VW> wide() const {
     DensePiece<VW> e;
 #pragma unroll
@@ -728,16 +747,17 @@ struct DenseRaw<unsigned short, VW> {
     }
     return e;
   }
+  template <bool NT>
   static __device__ __forceinline__ void store(unsigned short *p, const DensePiece<VW> &e) {
     words o;
 #pragma unroll
     for (int i = 0; i < VW / 2; ++i)
       o[i] = (unsigned int)f32_to_bf16(e.v[2 * i]) | ((unsigned int)f32_to_bf16(e.v[2 * i + 1]) << 16);
-    *reinterpret_cast<words *>(p) = o;
+    state_store<NT>(reinterpret_cast<words *>(p), o);
   }
 };
 
-template <typename RhoT, int D, int U>
+template <typename RhoT, int D, int U, bool NT>
 __global__ __launch_bounds__(256) void k_step_dense(StepPtrs a, RhoT *__restrict__ rho, int Nq, int rotary,
                                                     HeadScalars decay) {
   constexpr int VW = sizeof(RhoT) == 2 && D == 512 ? 8 : 4;  // columns per access
@@ -764,7 +784,7 @@ __global__ __launch_bounds__(256) void k_step_dense(StepPtrs a, RhoT *__restrict
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int j = 0; j < VPL; ++j) rv[u][j].load(base + (long)min(r0 + 4 * u, rows - 1) * D + j * 64 * VW);
+      for (int j = 0; j < VPL; ++j) rv[u][j].template load<NT>(base + (long)min(r0 + 4 * u, rows - 1) * D + j * 64 * VW);
   };
   load_rows(wave);
   DensePiece<VW> acc[VPL], vv[VPL];
@@ -813,7 +833,7 @@ __global__ __launch_bounds__(256) void k_step_dense(StepPtrs a, RhoT *__restrict
             e.v[c] = e.v[c] + p;
             if (has_decay) e.v[c] = e.v[c] * dec;
           }
-          Raw::store(base + (long)r * D + j * 64 * VW, e);
+          Raw::template store<NT>(base + (long)r * D + j * 64 * VW, e);
         }
       }
     }
@@ -863,7 +883,7 @@ __global__ __launch_bounds__(256) void k_alibi_materialize(RhoT *__restrict__ rh
         dense_store4(p + c, e);
       }
     } else {
-      for (int c = lane; c < d; c += 64) rho_store(p + c, rho_load<RhoT>(p + c) * scale);
+      for (int c = lane; c < d; c += 64) rho_store<false>(p + c, rho_load<false>(p + c) * scale);
     }
   }
   if (lane == 0) stamps[row] = (int32_t)min(clock, 0x7fffffffL);
@@ -984,11 +1004,21 @@ __global__ __launch_bounds__(256) void k_fill_zero_u32(uint32_t *__restrict__ p,
 }
 
 template <int D, int WAVES, int U, int SPLIT>
-void launch_fast(hipStream_t st, int blocks, const StepPtrs &a, float *rho) {
+void launch_fast(hipStream_t st, int blocks, const StepPtrs &a, float *rho, bool past_caches) {
   if (a.nt > 1)
-    hipLaunchKernelGGL((k_step_rope_f32<D, WAVES, U, SPLIT, true>), dim3(blocks), dim3(WAVES * 64), 0, st, a, rho);
+    hipLaunchKernelGGL((k_step_rope_f32<D, WAVES, U, SPLIT, true, false>), dim3(blocks), dim3(WAVES * 64), 0, st, a, rho);
+  else if (past_caches)
+    hipLaunchKernelGGL((k_step_rope_f32<D, WAVES, U, SPLIT, false, true>), dim3(blocks), dim3(WAVES * 64), 0, st, a, rho);
   else
-    hipLaunchKernelGGL((k_step_rope_f32<D, WAVES, U, SPLIT, false>), dim3(blocks), dim3(WAVES * 64), 0, st, a, rho);
+    hipLaunchKernelGGL((k_step_rope_f32<D, WAVES, U, SPLIT, false, false>), dim3(blocks), dim3(WAVES * 64), 0, st, a, rho);
+}
+
+template <int D, int WAVES, int U, int SPLIT>
+void launch_fast(hipStream_t st, int blocks, const StepPtrs &a, unsigned short *rho, bool past_caches) {
+  if (past_caches)
+    hipLaunchKernelGGL((k_step_rope_bf16<D, WAVES, U, SPLIT, true>), dim3(blocks), dim3(WAVES * 64), 0, st, a, rho);
+  else
+    hipLaunchKernelGGL((k_step_rope_bf16<D, WAVES, U, SPLIT, false>), dim3(blocks), dim3(WAVES * 64), 0, st, a, rho);
 }
 
 }  // namespace
@@ -1063,6 +1093,24 @@ static int dense_form_from(const StateStepParams &p, bool fast) {
   }
   const double dense = 30.0 + dense_mib * mib + 0.005 * Nq;
   return (int)std::min(128.0, std::max(16.0, std::ceil(dense / token)));
+}
+
+// Do the rows of a one-token step go past the caches (loads and stores with the streaming hint)?  The chip's last cache holds
+// 256 MiB.  Where the states and weights that pass between two visits of a row are more than that, a cached row is gone before
+// it is read again and has driven out weights (and, written, waits its turn to be written back while the next kernel reads):
+// decode steps by kernels, cached | past them: 12 layers of 16384 neurons a head, 8 sequences, d = 512, 24 GiB of state 9950 us
+// | 9490; 6 of 8192, d = 256, 2 to 16 sequences, a twentieth to half of the neurons firing 0.959 to 1.002 of the time; eager ALiBi
+// and PoPE, 0.6 to 1.6 GB, d = 192 and 512 0.90 to 0.95; bf16 RoPE 0.94 to 0.99.  Where all of it stays, the hint costs: 4 layers
+// of 3072 neurons, d = 192, 4 sequences (180 MB) 1.01.  A single layer stepped again and again finds a good part of its rows in
+// the cache even where it is larger (1 GiB, a twentieth firing, 45.4 | 47.3 us), unless every step walks all of it.  The dense
+// kernel's bf16 rows gain nothing (8 layers, d = 512, 48 sequences 609 | 614).
+static bool stream_past_caches(const bdh_ctx *ctx, const StateStepParams &p) {
+  if (p.T > 1) return false;  // a launch may walk its rows token after token
+  if (ctx->opt_step_past_caches >= 0) return ctx->opt_step_past_caches == 1;
+  const bool f32 = p.rho_dtype == BDH_F32, every_row = p.rotary == BDH_POPE || (p.rotary == BDH_ALIBI && !p.stamps);
+  if (every_row && !f32 && (p.d == 256 || p.d == 512)) return false;
+  const size_t own = (size_t)p.B * p.h * p.N * p.d * (p.rotary == BDH_POPE ? 2 : 1) * (f32 ? 4 : 2);
+  return std::max(p.walked, every_row ? own : 0) > (size_t(256) << 20);
 }
 
 void *bdh_step_scratch_ptr(const bdh_ctx *ctx) {
@@ -1170,6 +1218,7 @@ int bdh_launch_state_steps_in(bdh_ctx *ctx, const StateStepParams &p, float *out
     }
   if (p.stamps && p.rotary != BDH_ALIBI) return bdh_fail(ctx, BDH_E_INVAL, "decay stamps only apply to ALiBi");
 
+  const bool past_caches = stream_past_caches(ctx, p);
   const int NW = (N + 63) / 64;
   for (int t = 0; t < T; t += group) {
     const int nt = std::min(group, T - t);
@@ -1203,20 +1252,16 @@ int bdh_launch_state_steps_in(bdh_ctx *ctx, const StateStepParams &p, float *out
       const int blocks = slices * S;
       if (p.rho_dtype == BDH_F32) {
         float *rho = static_cast<float *>(p.rho);
-        if (d == 256 && !split) launch_fast<256, 4, 2, 1>(ctx->stream, blocks, a, rho);
-        if (d == 256 && split) launch_fast<256, 8, 8, 8>(ctx->stream, blocks, a, rho);
-        if (d == 512 && !split) launch_fast<512, 4, 2, 1>(ctx->stream, blocks, a, rho);
-        if (d == 512 && split) launch_fast<512, 8, 2, 8>(ctx->stream, blocks, a, rho);
+        if (d == 256 && !split) launch_fast<256, 4, 2, 1>(ctx->stream, blocks, a, rho, past_caches);
+        if (d == 256 && split) launch_fast<256, 8, 8, 8>(ctx->stream, blocks, a, rho, past_caches);
+        if (d == 512 && !split) launch_fast<512, 4, 2, 1>(ctx->stream, blocks, a, rho, past_caches);
+        if (d == 512 && split) launch_fast<512, 8, 2, 8>(ctx->stream, blocks, a, rho, past_caches);
       } else {
         unsigned short *rho = static_cast<unsigned short *>(p.rho);
-        if (d == 256 && !split)
-          hipLaunchKernelGGL((k_step_rope_bf16<256, 4, 8, 1>), dim3(blocks), dim3(256), 0, ctx->stream, a, rho);
-        if (d == 256 && split)
-          hipLaunchKernelGGL((k_step_rope_bf16<256, 8, 4, 8>), dim3(blocks), dim3(512), 0, ctx->stream, a, rho);
-        if (d == 512 && !split)
-          hipLaunchKernelGGL((k_step_rope_bf16<512, 4, 2, 1>), dim3(blocks), dim3(256), 0, ctx->stream, a, rho);
-        if (d == 512 && split)
-          hipLaunchKernelGGL((k_step_rope_bf16<512, 8, 2, 8>), dim3(blocks), dim3(512), 0, ctx->stream, a, rho);
+        if (d == 256 && !split) launch_fast<256, 4, 8, 1>(ctx->stream, blocks, a, rho, past_caches);
+        if (d == 256 && split) launch_fast<256, 8, 4, 8>(ctx->stream, blocks, a, rho, past_caches);
+        if (d == 512 && !split) launch_fast<512, 4, 2, 1>(ctx->stream, blocks, a, rho, past_caches);
+        if (d == 512 && split) launch_fast<512, 8, 2, 8>(ctx->stream, blocks, a, rho, past_caches);
       }
       BDH_LAUNCH_CHECK(ctx, "k_step_rope");
       if (p.partials_out) {  // the caller's next kernel adds the partials up
@@ -1228,26 +1273,22 @@ int bdh_launch_state_steps_in(bdh_ctx *ctx, const StateStepParams &p, float *out
                       a.partial_t_stride, a.cnt_t_stride);
       BDH_LAUNCH_CHECK(ctx, "k_step_finalize");
     } else if (fast_lazy) {
-      float *rho = static_cast<float *>(p.rho);
-      if (d == 256)
-        hipLaunchKernelGGL((k_step_alibi_lazy_f32<256, 4, 4>), dim3(slices * S), dim3(256), 0, ctx->stream, a, rho,
-                           p.stamps, decay, log_decay);
-      else
-        hipLaunchKernelGGL((k_step_alibi_lazy_f32<512, 4, 4>), dim3(slices * S), dim3(256), 0, ctx->stream, a, rho,
-                           p.stamps, decay, log_decay);
+      auto *kernel = d == 256 ? (past_caches ? k_step_alibi_lazy_f32<256, 4, 4, true> : k_step_alibi_lazy_f32<256, 4, 4, false>)
+                              : (past_caches ? k_step_alibi_lazy_f32<512, 4, 4, true> : k_step_alibi_lazy_f32<512, 4, 4, false>);
+      hipLaunchKernelGGL(kernel, dim3(slices * S), dim3(256), 0, ctx->stream, a, static_cast<float *>(p.rho), p.stamps, decay,
+                         log_decay);
       BDH_LAUNCH_CHECK(ctx, "k_step_alibi_lazy_f32");
       launch_finalize(ctx->stream, slices, partial, pair_cnt, S, d, out_t, (long)T * d, out_ln_t, rows_t, (long)T, 1);
       BDH_LAUNCH_CHECK(ctx, "k_step_finalize");
     } else if (fast_dense) {
       const dim3 grid(slices * S);
       if (p.rho_dtype == BDH_F32) {
-        float *rho = static_cast<float *>(p.rho);
-        if (d == 256) hipLaunchKernelGGL((k_step_dense<float, 256, 8>), grid, dim3(256), 0, ctx->stream, a, rho, Nq, p.rotary, decay);
-        else hipLaunchKernelGGL((k_step_dense<float, 512, 8>), grid, dim3(256), 0, ctx->stream, a, rho, Nq, p.rotary, decay);
+        auto *kernel = d == 256 ? (past_caches ? k_step_dense<float, 256, 8, true> : k_step_dense<float, 256, 8, false>)
+                                : (past_caches ? k_step_dense<float, 512, 8, true> : k_step_dense<float, 512, 8, false>);
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, ctx->stream, a, static_cast<float *>(p.rho), Nq, p.rotary, decay);
       } else {
-        unsigned short *rho = static_cast<unsigned short *>(p.rho);
-        if (d == 256) hipLaunchKernelGGL((k_step_dense<unsigned short, 256, 8>), grid, dim3(256), 0, ctx->stream, a, rho, Nq, p.rotary, decay);
-        else hipLaunchKernelGGL((k_step_dense<unsigned short, 512, 8>), grid, dim3(256), 0, ctx->stream, a, rho, Nq, p.rotary, decay);
+        auto *kernel = d == 256 ? k_step_dense<unsigned short, 256, 8, false> : k_step_dense<unsigned short, 512, 8, false>;
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, ctx->stream, a, static_cast<unsigned short *>(p.rho), Nq, p.rotary, decay);
       }
       BDH_LAUNCH_CHECK(ctx, "k_step_dense");
       launch_finalize(ctx->stream, slices, partial, nullptr, S, d, out_t, (long)T * d, out_ln_t, nullptr, (long)T, 2, nt,
@@ -1260,9 +1301,11 @@ int bdh_launch_state_steps_in(bdh_ctx *ctx, const StateStepParams &p, float *out
       }
     } else {
       // registers for the columns a row really has: the narrower the rows, the more of them in flight
-#define BDH_GEN(T_, MAXC_, FL_)                                                                                   \
-  hipLaunchKernelGGL((k_step_generic<T_, MAXC_, FL_>), dim3(slices * S), dim3(256), 0, ctx->stream, a,           \
+#define BDH_GEN_NT(T_, MAXC_, FL_, NT_)                                                                           \
+  hipLaunchKernelGGL((k_step_generic<T_, MAXC_, FL_, NT_>), dim3(slices * S), dim3(256), 0, ctx->stream, a,      \
                      static_cast<T_ *>(p.rho), d, Nq, p.rotary, has_decay, decay, log_decay, p.stamps)
+#define BDH_GEN(T_, MAXC_, FL_) \
+  do { if (past_caches) BDH_GEN_NT(T_, MAXC_, FL_, true); else BDH_GEN_NT(T_, MAXC_, FL_, false); } while (0)
       if (p.rho_dtype == BDH_F32) {
         if (d <= 128) BDH_GEN(float, 2, 16); else if (d <= 256) BDH_GEN(float, 4, 8);
         else if (d <= 512) BDH_GEN(float, 8, 4); else BDH_GEN(float, 16, 4);
@@ -1270,6 +1313,7 @@ int bdh_launch_state_steps_in(bdh_ctx *ctx, const StateStepParams &p, float *out
         if (d <= 128) BDH_GEN(unsigned short, 2, 16); else if (d <= 256) BDH_GEN(unsigned short, 4, 8);
         else if (d <= 512) BDH_GEN(unsigned short, 8, 4); else BDH_GEN(unsigned short, 16, 4);
       }
+#undef BDH_GEN_NT
 #undef BDH_GEN
       BDH_LAUNCH_CHECK(ctx, "k_step_generic");
       launch_finalize(ctx->stream, slices, partial, nullptr, S, d, out_t, (long)T * d, out_ln_t, nullptr, (long)T, 2, nt,

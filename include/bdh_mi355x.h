@@ -96,6 +96,9 @@ const char *bdh_last_error(const bdh_ctx *ctx);
  *                       to the prompt calls of bdh_model_forward*.
  *   "state_step.dense_kernel": 1 (default) PoPE and eagerly decayed ALiBi steps at d in {256,512} take
  *                       the dense streaming kernel, 0 = the generic kernel (same values).
+ *   "state_step.past_caches": -1 (default) the rows of a one-token step are loaded and stored with the streaming hint where
+ *                       the states and weights that pass between two visits of a row exceed the last cache (256 MiB),
+ *                       0 = never, 1 = always (same bits).
  *   "relu_lowrank.mfma_rows": 2 (default) calls with this many rows and fewer than 64 (N a multiple of 4, d a multiple
  *                       of 32) that the row kernel below does not take run on the f32 matrix cores, the weights
  *                       streamed once per tile of 16 to 64 rows: a chain of v_mfma_f32_16x16x4_f32 over k is the same

@@ -642,3 +642,34 @@ def test_dense_streaming_kernel_equals_generic_kernel_and_oracle(gpu, corc, rota
     out_ref, rho_ref = corc.recurrent_attention(q, v, rho0.copy(), None if slopes is None else corc.alibi_decay(slopes))
     tol = 2e-5 if dtype == torch.float32 else 2e-2
     assert rel_err(res[0][0], out_ref) < tol and rel_err(res[0][1], rho_ref) < tol
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rotary,lazy", [(orc.ROPE, False), (orc.ALIBI, True), (orc.ALIBI, False), (orc.POPE, False)])
+@pytest.mark.parametrize("B,h,N,d", [(1, 2, 130, 256), (300, 4, 254, 256), (2, 2, 514, 512), (2, 3, 66, 192), (3, 1, 40, 36)])
+def test_rows_past_the_caches_keep_their_bits(gpu, rotary, lazy, B, h, N, d, dtype):
+    """The streaming hint changes where a row is kept, never what it holds: every kernel of a one-token step with it and
+    without it, two steps one after the other on the same state."""
+    ffi, recurrent_attention = gpu
+    from burn_dragon_amd.positional import RotaryEmbedding
+    from burn_dragon_amd.recurrent import recurrent_attention_lazy_alibi
+
+    dev, ctx = "cuda:0", ffi.default_context(0)
+    g = torch.Generator(device=dev).manual_seed(N + d)
+    x = torch.relu(torch.randn((2, B, h, 1, N), device=dev, generator=g) - 0.5)
+    v = torch.randn((2, B, 1, d), device=dev, generator=g)
+    rho0 = torch.randn((B, h, 2 * N if rotary == orc.POPE else N, d), device=dev, generator=g).to(dtype)
+    freqs = 0.1 * torch.rand(N, device=dev, generator=g)
+    got = []
+    for mode in (0, 1):
+        rho, stamps = rho0.clone(), torch.zeros((B, h, N), dtype=torch.int32, device=dev)
+        ctx.set_option("state_step.past_caches", mode)
+        try:
+            outs = [recurrent_attention_lazy_alibi(x[t], v[t], rho, stamps, 3 + t) if lazy else
+                    recurrent_attention(x[t], v[t], rho, freqs, 3 + t, RotaryEmbedding(rotary)) for t in range(2)]
+            torch.cuda.synchronize()
+        finally:
+            ctx.set_option("state_step.past_caches", -1)
+        got.append((*outs, rho, stamps))
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+    assert not torch.equal(got[0][2], rho0)
