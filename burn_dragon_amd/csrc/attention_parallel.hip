@@ -990,6 +990,20 @@ int bdh_launch_decoder_partials_f32(bdh_ctx *ctx, int B, int T, int h, int N, in
   return bdh_launch_gemm_f32(ctx, g, false, true, plan, g.C);
 }
 
+// D_y of a prompt: gate * relu(in . W - thr) as split-bf16 products, a slice per head.
+int bdh_launch_relu_lowrank_split(bdh_ctx *ctx, const ReluLowrankParams &p) {
+  GemmF32 g;
+  g.epilogue = GEMM_GATE;
+  g.A = p.in; g.B = p.weight; g.C = p.out; g.gate = p.gate;
+  g.threshold = p.threshold;
+  g.M = p.B * p.T; g.N = p.N; g.K = p.d;
+  g.lda = p.d; g.ldb = g.ldc = p.N;
+  g.n_slices = g.mod = p.h;
+  g.a_s2 = p.h_in == 1 ? 0 : (long)p.T * p.d; g.b_s2 = (long)p.d * p.N; g.c_s2 = (long)p.T * p.N;
+  g.rows_per = p.T; g.a_outer = (long)p.h_in * p.T * p.d; g.c_outer = (long)p.h * p.T * p.N;
+  return bdh_launch_gemm_f32(ctx, g, false, true, bdh_gemm_f32_plan(ctx, g, 1), nullptr);
+}
+
 extern "C" int bdh_rotate(bdh_ctx *ctx, int B, int h, int T, int N, int rotary, const float *x, const float *freqs,
                           int64_t position, const int32_t *positions_dev, float *q) {
   if (!ctx) return BDH_E_INVAL;

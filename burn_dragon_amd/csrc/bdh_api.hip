@@ -169,6 +169,11 @@ int bdh_ctx_set_option(bdh_ctx *ctx, const char *name, int value) {
     ctx->opt_model_phase_batch = value;
     return BDH_OK;
   }
+  if (strcmp(name, "relu_lowrank.split") == 0) {
+    if (value < -1 || value > 1) return bdh_fail(ctx, BDH_E_INVAL, "relu_lowrank.split takes -1, 0 or 1");
+    ctx->opt_lowrank_split = value;
+    return BDH_OK;
+  }
   if (strcmp(name, "relu_lowrank.row") == 0) {
     if (value < 0 || value > 1) return bdh_fail(ctx, BDH_E_INVAL, "relu_lowrank.row takes 0 or 1");
     ctx->opt_lowrank_row = value;

@@ -28,6 +28,7 @@ struct bdh_ctx {
   int opt_model_one_launch = 1;  // small model's decode step in one launch: 1 when it pays, 2 whenever it fits, 0 never
   int opt_lowrank_row = 1;     // 0: relu_lowrank with one input row and a small matrix uses the column-per-thread kernel
   int opt_model_phase_batch = 1 << 30;  // two launches per layer for a decode step of at most this many sequences (0: never)
+  int opt_lowrank_split = -1;  // D_y of a prompt on split-bf16 products: -1 by size, 0 / 1 never / always
   int opt_lowrank_gemm_rows = 64;  // relu_lowrank of 64 rows and more takes the f32 matrix cores from this many on (0: never)
   int opt_lowrank_mfma_rows = 2;  // relu_lowrank of fewer than 64 rows takes the f32 matrix cores from this many on (0: never)
   int opt_step_past_caches = -1;  // -1: by what passes between two visits of a row; 0 / 1: never / always
@@ -180,8 +181,10 @@ struct ReluLowrankParams {
   int n_blocks;
   const float *gate;
   float *out;
+  bool any_order = false;  // the caller does not need the bits of the k-sequential chain (gated calls only)
 };
 int bdh_launch_relu_lowrank(bdh_ctx *ctx, const ReluLowrankParams &p);
+int bdh_launch_relu_lowrank_split(bdh_ctx *ctx, const ReluLowrankParams &p);
 // the same on the f32 matrix cores for many rows per (sequence, head); csrc/attention_parallel.hip
 int bdh_launch_relu_lowrank_gemm(bdh_ctx *ctx, const ReluLowrankParams &p, const unsigned char *mask_dev);
 // relu_lowrank for ONE input row per head whose values are made by the kernel itself from the partial sums an earlier

@@ -27,9 +27,12 @@ struct GemmF32 {
   //                piece (rows_per == 0), others are refused.
   //   GEMM_SCORES  square, C zero above the diagonal of the block pattern, see the fields below
   //   GEMM_NORM    C = acc / (sum_k |A[m,k]| + 1e-6)
+  //   GEMM_GATE    C = gate * max(acc - threshold, 0), the gate laid out as C
   int epilogue = 0;
   bool accumulate = false;
   bool decay_rows = false, decay_state = false, decay_scores = false;
+  const float *gate = nullptr;
+  float threshold = 0.0f;
   int heads = 1;              // head of a slice = slice % heads
   float log_decay[64] = {0};  // log g per head
   // scores of causal time blocks of block_size tokens: dense lower triangle of blocks, or the byte mask active[tb*tb];
@@ -47,7 +50,7 @@ struct GemmF32 {
   int mt = 0, nt = 0, ks = 1, kb_per = 0, tri = 0;
   long c_split = 0;
 };
-constexpr int GEMM_STORE = 0, GEMM_SCORES = 1, GEMM_NORM = 2;
+constexpr int GEMM_STORE = 0, GEMM_SCORES = 1, GEMM_NORM = 2, GEMM_GATE = 3;
 
 // How a product is cut: tile (0: 128 x 128, 1: 64 x 64, 2: 32 x 128, 3: 128 x 256) and the number of parts of K.
 struct GemmPlan {

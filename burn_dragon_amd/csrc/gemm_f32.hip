@@ -409,6 +409,34 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_f32(GemmF32 g) {
       }
     return;
   }
+  if constexpr (EPI == GEMM_GATE) {  // the gates of a row of tiles are asked for before the first is used
+    const float *G = g.gate + s1 * g.c_s1 + s2 * g.c_s2;
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      long at[16];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int row = min(row_of(i, e), g.M - 1);
+        at[e] = g.rows_per > 0 ? (long)(row / g.rows_per) * g.c_outer + (long)(row % g.rows_per) * g.ldc : (long)row * g.ldc;
+      }
+      float gate[NJ][16];
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          gate[j][e] = __builtin_nontemporal_load(G + at[e] + min(n0 + wn * (BN / WN) + j * 32 + (lane & 31), g.N - 1));
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const int col = n0 + wn * (BN / WN) + j * 32 + (lane & 31);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const float v = acc[i][j][e] - g.threshold;
+          if (col < g.N && row_of(i, e) < g.M) __builtin_nontemporal_store(gate[j][e] * (v <= 0.0f ? 0.0f : v), C + at[e] + col);
+        }
+      }
+    }
+    return;
+  }
   const float slope = (EPI == GEMM_SCORES && g.use_alibi) ? g.slopes[slice % g.heads] : 0.0f;
 #pragma unroll
   for (int i = 0; i < MI; ++i)
@@ -462,7 +490,7 @@ void launch(hipStream_t st, const GemmF32 &g, bool ak, bool bk, int tile, unsign
   } while (0)
   if constexpr (EPI == GEMM_SCORES) {
     BDH_GT(false, false);
-  } else if constexpr (EPI == GEMM_NORM) {
+  } else if constexpr (EPI == GEMM_NORM || EPI == GEMM_GATE) {
     BDH_GT(false, true);
   } else {
     if (ak) BDH_GT(true, true);
@@ -562,6 +590,7 @@ int bdh_launch_gemm_f32(bdh_ctx *ctx, GemmF32 g, bool a_kmajor, bool b_kmajor, c
   const unsigned grid = (unsigned)(8 * ((total + 7) / 8));
   switch (g.epilogue) {
     case GEMM_SCORES: launch<GEMM_SCORES>(ctx->stream, g, a_kmajor, b_kmajor, plan.tile, grid); break;
+    case GEMM_GATE: launch<GEMM_GATE>(ctx->stream, g, a_kmajor, b_kmajor, plan.tile, grid); break;
     case GEMM_NORM: launch<GEMM_NORM>(ctx->stream, g, a_kmajor, b_kmajor, plan.tile, grid); break;
     default: launch<GEMM_STORE>(ctx->stream, g, a_kmajor, b_kmajor, plan.tile, grid); break;
   }

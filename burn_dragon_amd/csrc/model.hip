@@ -343,7 +343,8 @@ int model_forward_impl(bdh_model *m, const int64_t *tokens, int B, int T, StateR
     }
     if (rc != BDH_OK) return rc;
     // :361-381  xy = x * relu(LN(attn) . encoder_v - thr)
-    ReluLowrankParams py{B, h, T, d, h, N, attn_ln, m->w.encoder_v, nullptr, c.relu_threshold, 1, nullptr, 0, x_l, xy};
+    ReluLowrankParams py{B, h, T, d, h, N, attn_ln, m->w.encoder_v, nullptr, c.relu_threshold, 1, nullptr, 0, x_l, xy,
+                         T > 1 && !x_tap && !viz};
     rc = bdh_launch_relu_lowrank(ctx, py);
     if (rc != BDH_OK) return rc;
     if (viz) {  // :386-434: first sequence, last token; the state is already this call's updated one
@@ -524,7 +525,7 @@ int bdh_model_forward_fast_ex(bdh_model *m, const int64_t *tokens, int B, int T,
     rc = bdh_launch_layer_norm_rows(ctx, (int64_t)M * h, d, attn, attn_ln);  // :132
     if (rc != BDH_OK) return rc;
     ReluLowrankParams py{B, h, T, d, h, N, attn_ln, m->w.encoder_v, nullptr, c.relu_threshold, lat_block, latent_blocks_host,
-                         n_latent_blocks, x, xy};
+                         n_latent_blocks, x, xy, true};
     rc = bdh_launch_relu_lowrank(ctx, py);  // :134-151
     if (rc != BDH_OK) return rc;
     rc = bdh_launch_decoder_residual(ctx, B, T, h, N, d, xy, m->w.decoder, cur);  // :153-162

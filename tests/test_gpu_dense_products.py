@@ -308,3 +308,37 @@ def test_prompt_without_room_for_the_dense_form_is_walked(bda, kind):
     assert not torch.equal(dense[0], walked[0])  # with room the products are taken
     with pytest.raises(bda.ffi.BdhError):
         call(72, 1)
+
+
+@pytest.mark.parametrize("d,h,N,B,T", [
+    (128, 2, 66, 3, 45),    # rows of several sequences in one tile, columns that end inside it
+    (256, 4, 1024, 2, 64),  # whole tiles
+    (36, 1, 131, 1, 100),   # a k that ends inside a stage, odd rows of the weights
+    (512, 2, 96, 1, 130),
+    (256, 4, 8192, 1, 200),  # by size
+])
+def test_gated_projection_of_a_prompt_on_split_products(d, h, N, B, T):
+    """D_y of a prompt and of the stateless form as split-bf16 products against the f32 chain: sums of d terms in another
+    order, 2^-24 a step, through two layers and a few thousand terms of the encoder: 1e-5."""
+    import burn_dragon_amd as bda
+
+    cfg = bda.BDHConfig(n_layer=2, n_embd=d, n_head=h, mlp_internal_dim_multiplier=1, vocab_size=64, dropout=0.0)
+    cfg.latent_per_head = lambda: N
+    cfg.fused_kernels.set_rotary_embedding(bda.RotaryEmbedding.ALIBI)
+    model = bda.BDH(cfg, DEV, seed=3)
+    g = torch.Generator(device=DEV).manual_seed(N)
+    tokens = torch.randint(0, 64, (B, T), device=DEV, generator=g)
+    ctx = bda.ffi.default_context(0)
+    got = []
+    for split in (0, -1 if N == 8192 else 1):
+        ctx.set_option("relu_lowrank.split", split)
+        try:
+            state = model.init_state()
+            logits = model.forward_with_state(tokens, state)
+            got.append((logits, model.forward_fast(tokens), state.storage))
+            torch.cuda.synchronize()
+        finally:
+            ctx.set_option("relu_lowrank.split", -1)
+    for a, b in zip(*got):
+        assert not torch.equal(a, b)
+        assert float((a - b).abs().max() / a.abs().max()) < 1e-5
