@@ -17,6 +17,13 @@ __device__ __forceinline__ void bdh_copy_to_lds(const void *src, void *dst) {
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"{m0}"(at), "v"(src) : "memory");
 }
 
+// The same from base + offset bytes, base uniform over the wavefront: a loop that moves base along has no vector instructions
+// for its addresses.
+__device__ __forceinline__ void bdh_copy_to_lds(const void *base, unsigned int offset, void *dst) {
+  const unsigned int at = __builtin_amdgcn_readfirstlane((unsigned int)(uintptr_t)(bdh_lds_ptr_t)dst);
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"{m0}"(at), "v"(offset), "s"(base) : "memory");
+}
+
 // Waits until no more than `later` stages of COPIES copies each, issued by this wavefront after the stage that it needs, are
 // still on their way (at most MOST of them are ever asked about).  Loads come back in the order of their issue.
 template <int COPIES, int MOST>

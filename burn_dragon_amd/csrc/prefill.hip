@@ -379,6 +379,10 @@ constexpr int tile_lds_bytes(int TS) { return tile_stages(TS) * 2 * TS * BK * 2;
 // What bounds it with few slices is the wait for the next step's operands, hence small tiles, a list dealt evenly to the
 // XCDs and copies several steps ahead.  A call of 12 slices, 777 tokens, N = 4096, d = 256 took 506 us with 256 x 256
 // tiles staged through registers and whole slices dealt to XCDs, 238 us with this; 4 slices of 64 tokens 352 -> 93 us.
+// What a wave then waited for was itself: addresses worked out for every copy, and each group of products behind its own LDS
+// reads.  Now a copy is a lane's fixed offset from a base that scalar instructions move along, the operands of a group are
+// read a group ahead, across the barrier too, and the copies are asked for under products: that call's three products 75 + 65
+// + 47 -> 65 + 56 + 45 us.
 template <int TS, bool A_KMAJOR, bool SCORES>
 __global__ __launch_bounds__(256, 2) void k_gemm_tile(GemmArgs g) {
   extern __shared__ __attribute__((aligned(1024))) unsigned short s_dyn[];
@@ -406,7 +410,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_tile(GemmArgs g) {
     }
   }
   const int m0 = ti * TS, n0 = tj * TS;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;  // 2 x 2 waves, TS/2 x TS/2 each
 
   f32x16 acc[MI][MI];
@@ -419,88 +423,122 @@ __global__ __launch_bounds__(256, 2) void k_gemm_tile(GemmArgs g) {
 
   // the k loop over one pair of operands
   auto products = [&](const unsigned short *A, int lda, const unsigned short *B, int ldb, int K) {
-    const unsigned short *zero = reinterpret_cast<const unsigned short *>(&g_zero_piece);
+    // Byte offsets of this thread's pieces from the first row (k row) of the tile; rows past the end repeat the last one, and
+    // their sums are not stored.  Only the last step of a K that is no multiple of 64 looks at k: zeros beyond.
     const int kc = ((tid & 7) ^ ((tid >> 4) & 7)) * 8;  // this thread's k piece of a row-major panel
-    const unsigned short *pa[NP], *pb[NP];
-    bool va[NP], vb[NP];
+    unsigned int pa[NP], pb[NP];
 #pragma unroll
     for (int c = 0; c < NP; ++c) {
       const int piece = c * 256 + tid, row = piece >> 3;
-      vb[c] = n0 + row < g.N;
-      pb[c] = B + (long)(n0 + row) * ldb + kc;
+      pb[c] = (unsigned int)(min(row, g.N - 1 - n0) * ldb + kc) * 2u;
       if (!A_KMAJOR) {
-        va[c] = m0 + row < g.M;
-        pa[c] = A + (long)(m0 + row) * lda + kc;
+        pa[c] = (unsigned int)(min(row, g.M - 1 - m0) * lda + kc) * 2u;
       } else {
         const int kr = piece / (TS / 8);
         const int turn = TS == 128 ? (kr & 3) << 2 : ((kr >> 1) & 1) << 2;
         const int m = ((piece % (TS / 8)) ^ turn) * 8;
-        va[c] = m0 + m < g.M;
-        pa[c] = A + (long)kr * lda + m0 + m;
+        pa[c] = (unsigned int)(kr * lda + min(m, g.M - 8 - m0)) * 2u;  // M % 8 == 0
       }
     }
+    const unsigned short *a0 = A + (A_KMAJOR ? (long)m0 : (long)m0 * lda), *b0 = B + (long)n0 * ldb;
     const int steps = (K + BK - 1) / BK;
     auto issue = [&](int s) {
       unsigned short *dst = s_dyn + (s % NS) * STAGE + wave * 512;
       const int k0 = s * BK;
+      const unsigned short *as = a0 + (A_KMAJOR ? (long)k0 * lda : (long)k0), *bs = b0 + k0;
+      if (k0 + BK <= K) {
 #pragma unroll
-      for (int c = 0; c < NP; ++c) {
-        bool in = va[c];
-        if (A_KMAJOR) in = in && k0 + (c * 256 + tid) / (TS / 8) < K;
-        else in = in && k0 + kc < K;
-        bdh_copy_to_lds(in ? pa[c] + (A_KMAJOR ? (long)k0 * lda : (long)k0) : zero, dst + c * 2048);
+        for (int c = 0; c < NP; ++c) bdh_copy_to_lds(as, pa[c], dst + c * 2048);
+#pragma unroll
+        for (int c = 0; c < NP; ++c) bdh_copy_to_lds(bs, pb[c], dst + PANEL + c * 2048);
+      } else {
+        const char *zero = reinterpret_cast<const char *>(&g_zero_piece);
+#pragma unroll
+        for (int c = 0; c < NP; ++c) {
+          const int k = A_KMAJOR ? k0 + (c * 256 + tid) / (TS / 8) : k0 + kc;
+          bdh_copy_to_lds(k < K ? reinterpret_cast<const char *>(as) + pa[c] : zero, dst + c * 2048);
+        }
+#pragma unroll
+        for (int c = 0; c < NP; ++c)
+          bdh_copy_to_lds(k0 + kc < K ? reinterpret_cast<const char *>(bs) + pb[c] : zero, dst + PANEL + c * 2048);
+      }
+    };
+    // The operands of the next 16 k are read into a second set of registers while these are multiplied, also across a step:
+    // a wave may have its SIMD to itself, and nothing else covers the LDS's answer then.
+    bf16x8 fa[2][MI], fb[2][MI];
+    auto read = [&](int s, int kk, int into) {
+      const unsigned short *sa = s_dyn + (s % NS) * STAGE, *sb = sa + PANEL;
+      const int C = (kk >> 3) + (lane >> 5);
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        if (!A_KMAJOR) {
+          const int R = wm * (TS / 2) + i * 32 + (lane & 31);
+          fa[into][i] = *reinterpret_cast<const bf16x8 *>(sa + R * BK + ((C ^ ((R >> 1) & 7)) << 3));
+        } else {
+          // transposing LDS read (ds_read_b64_tr_b16): a group of 16 lanes reads a 4(k) x 16(m) block, lane j of the
+          // group supplying the address of row j/4, columns (j%4)*4..+3, and receives column j for the four k rows.
+          // Two reads give the 8 consecutive k of lane (m = lane%32, k-group = lane/32).
+          const int j16 = lane & 15, kr = C * 8 + (j16 >> 2);
+          const int m = wm * (TS / 2) + i * 32 + ((lane >> 4) & 1) * 16 + (j16 & 3) * 4;
+          const int turn = TS == 128 ? (kr & 3) << 2 : ((kr >> 1) & 1) << 2;  // the same for kr + 4
+          const unsigned short *src = sa + kr * TS + (((m >> 3) ^ turn) << 3) + (m & 7);
+          typedef short s16x4 __attribute__((ext_vector_type(4)));
+          typedef short s16x8 __attribute__((ext_vector_type(8)));
+          typedef __attribute__((address_space(3))) s16x4 *lds_s16x4_t;
+          const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)(src));
+          const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)(src + 4 * TS));
+          const s16x8 pk = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+          fa[into][i] = __builtin_bit_cast(bf16x8, pk);
+        }
       }
 #pragma unroll
-      for (int c = 0; c < NP; ++c)
-        bdh_copy_to_lds(vb[c] && k0 + kc < K ? pb[c] + k0 : zero, dst + PANEL + c * 2048);
+      for (int j = 0; j < MI; ++j) {
+        const int R = wn * (TS / 2) + j * 32 + (lane & 31);
+        fb[into][j] = *reinterpret_cast<const bf16x8 *>(sb + R * BK + ((C ^ ((R >> 1) & 7)) << 3));
+      }
+    };
+    auto multiply = [&](int from) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < MI; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[from][i], fb[from][j], acc[i][j], 0, 0, 0);
+    };
+    // Stage s is there for every wave, and every wave has the last operands of stage s - 1 in registers: its place is free.
+    auto arrive = [&](int s) {
+      // the copies of step s have landed when at most those of the steps behind it are outstanding
+      if (s + NS - 2 < steps) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * 2 * NP) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      lds_barrier();
     };
 #pragma unroll
     for (int s = 0; s < NS - 1; ++s)
       if (s < steps) issue(s);
-    for (int s = 0; s < steps; ++s) {
-      // the copies of step s have landed when at most those of the steps behind it are outstanding
-      if (s + NS - 2 < steps) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * 2 * NP) : "memory");
-      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      lds_barrier();  // everyone's copies, and everyone is past the reads of step s - 1
-      if (s + NS - 1 < steps) issue(s + NS - 1);
-      const unsigned short *sa = s_dyn + (s % NS) * STAGE, *sb = sa + PANEL;
+    if (steps > 0) {
+      arrive(0);
+      read(0, 0, 0);
+      if (NS - 1 < steps) issue(NS - 1);
+    }
+    auto inside = [&](int s) {  // all of a step but its last products
 #pragma unroll
-      for (int kk = 0; kk < BK; kk += 16) {
-        bf16x8 fa[MI], fb[MI];
-        const int C = (kk >> 3) + (lane >> 5);
-#pragma unroll
-        for (int i = 0; i < MI; ++i) {
-          if (!A_KMAJOR) {
-            const int R = wm * (TS / 2) + i * 32 + (lane & 31);
-            fa[i] = *reinterpret_cast<const bf16x8 *>(sa + R * BK + ((C ^ ((R >> 1) & 7)) << 3));
-          } else {
-            // transposing LDS read (ds_read_b64_tr_b16): a group of 16 lanes reads a 4(k) x 16(m) block, lane j of the
-            // group supplying the address of row j/4, columns (j%4)*4..+3, and receives column j for the four k rows.
-            // Two reads give the 8 consecutive k of lane (m = lane%32, k-group = lane/32).
-            const int j16 = lane & 15, kr = C * 8 + (j16 >> 2);
-            const int m = wm * (TS / 2) + i * 32 + ((lane >> 4) & 1) * 16 + (j16 & 3) * 4;
-            const int turn = TS == 128 ? (kr & 3) << 2 : ((kr >> 1) & 1) << 2;  // the same for kr + 4
-            const unsigned short *src = sa + kr * TS + (((m >> 3) ^ turn) << 3) + (m & 7);
-            typedef short s16x4 __attribute__((ext_vector_type(4)));
-            typedef short s16x8 __attribute__((ext_vector_type(8)));
-            typedef __attribute__((address_space(3))) s16x4 *lds_s16x4_t;
-            const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)(src));
-            const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)(src + 4 * TS));
-            const s16x8 pk = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-            fa[i] = __builtin_bit_cast(bf16x8, pk);
-          }
-        }
-#pragma unroll
-        for (int j = 0; j < MI; ++j) {
-          const int R = wn * (TS / 2) + j * 32 + (lane & 31);
-          fb[j] = *reinterpret_cast<const bf16x8 *>(sb + R * BK + ((C ^ ((R >> 1) & 7)) << 3));
-        }
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-#pragma unroll
-          for (int j = 0; j < MI; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
+      for (int q = 0; q < BK / 16 - 1; ++q) {
+        read(s, 16 * (q + 1), (q + 1) & 1);
+        __builtin_amdgcn_sched_barrier(0);  // left alone, the scheduler sinks the reads to their use
+        multiply(q & 1);
       }
+    };
+    // (the last step by itself: behind a branch the compiler would wait for the operands just asked for)
+    for (int s = 0; s + 1 < steps; ++s) {
+      inside(s);
+      arrive(s + 1);
+      read(s + 1, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(1);
+      if (s + NS < steps) issue(s + NS);  // under the products just started
+    }
+    if (steps > 0) {
+      inside(steps - 1);
+      multiply(1);
     }
     lds_barrier();  // every wave is past its reads: the stages are free
   };
