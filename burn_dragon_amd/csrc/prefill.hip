@@ -114,13 +114,12 @@ struct TransposeArgs {
   long v_batch;
   int B, h, T, d, Tp, Nq;
   int v_tiles, kinds;  // tiles of one V^T; 1 + the heads of a decaying state
+  int blocks;          // workgroups of all of it
   HeadPar log_decay;
 };
-__global__ __launch_bounds__(256) void k_transpose_operands(TransposeArgs a) {
-  __shared__ __attribute__((aligned(16))) unsigned short tile[64][66];
+__device__ __forceinline__ void transpose_tile(const TransposeArgs &a, int at, unsigned short (*tile)[66]) {
   const int tid = threadIdx.x, ct = (a.d + 63) >> 6;
   const int v_blocks = a.v_tiles * a.B * a.kinds;
-  int at = blockIdx.x;
   unsigned short *dst;
   int r0, c0, ldo;
   if (at < v_blocks) {
@@ -194,6 +193,10 @@ __global__ __launch_bounds__(256) void k_transpose_operands(TransposeArgs a) {
     if (c0 + cc < a.d && r0 + rr < ldo)
       *reinterpret_cast<uint4 *>(dst + (long)(c0 + cc) * ldo + r0 + rr) = make_uint4(w[0], w[1], w[2], w[3]);
   }
+}
+__global__ __launch_bounds__(256) void k_transpose_operands(TransposeArgs a) {
+  __shared__ __attribute__((aligned(16))) unsigned short tile[64][66];
+  transpose_tile(a, blockIdx.x, tile);
 }
 
 // PoPE (src/model/attention.rs:323-330): x bf16 [S, T, N] -> q bf16 [S, T, 2N] = cat(softplus(x) cos, softplus(x) sin).
@@ -383,9 +386,18 @@ constexpr int tile_lds_bytes(int TS) { return tile_stages(TS) * 2 * TS * BK * 2;
 // reads.  Now a copy is a lane's fixed offset from a base that scalar instructions move along, the operands of a group are
 // read a group ahead, across the barrier too, and the copies are asked for under products: that call's three products 75 + 65
 // + 47 -> 65 + 56 + 45 us.
+// The workgroups behind the tiles (scores only: tr.blocks > 0) transpose what the later products read: they depend on nothing
+// here, and the scores seldom fill the chip to the end (the call above 174 -> 164).
 template <int TS, bool A_KMAJOR, bool SCORES>
-__global__ __launch_bounds__(256, 2) void k_gemm_tile(GemmArgs g) {
+__global__ __launch_bounds__(256, 2) void k_gemm_tile(GemmArgs g, TransposeArgs tr) {
   extern __shared__ __attribute__((aligned(1024))) unsigned short s_dyn[];
+  if constexpr (SCORES) {
+    const int gemm_blocks = 8 * ((g.n_slices * g.n_tiles + 7) >> 3);
+    if ((int)blockIdx.x >= gemm_blocks) {
+      transpose_tile(tr, blockIdx.x - gemm_blocks, reinterpret_cast<unsigned short (*)[66]>(s_dyn));
+      return;
+    }
+  }
   constexpr int NS = tile_stages(TS), PANEL = TS * BK, STAGE = 2 * PANEL;
   constexpr int MI = TS / 64;          // 32 x 32 accumulators per wave and direction
   constexpr int NP = TS * BK / 8 / 256;  // pieces per thread and panel
@@ -1512,15 +1524,15 @@ hipError_t launch_gemm_direct(hipStream_t st, const GemmArgs &g) {
 
 // g.mt, g.nt and g.n_tiles are filled in here.
 template <bool AK, bool SCORES>
-void launch_gemm_tile(hipStream_t st, GemmArgs g, int tile) {
+void launch_gemm_tile(hipStream_t st, GemmArgs g, int tile, const TransposeArgs &tr = TransposeArgs{}) {
   g.mt = (g.M + tile - 1) / tile;
   g.nt = (g.N + tile - 1) / tile;
   g.n_tiles = g.tri ? g.mt * (g.mt + 1) / 2 : g.mt * g.nt;
-  const unsigned grid = 8u * (unsigned)(((long)g.n_slices * g.n_tiles + 7) / 8);
+  const unsigned grid = 8u * (unsigned)(((long)g.n_slices * g.n_tiles + 7) / 8) + (unsigned)tr.blocks;
   if (tile == 128)
-    hipLaunchKernelGGL((k_gemm_tile<128, AK, SCORES>), dim3(grid), dim3(256), tile_lds_bytes(128), st, g);
+    hipLaunchKernelGGL((k_gemm_tile<128, AK, SCORES>), dim3(grid), dim3(256), tile_lds_bytes(128), st, g, tr);
   else
-    hipLaunchKernelGGL((k_gemm_tile<64, AK, SCORES>), dim3(grid), dim3(256), tile_lds_bytes(64), st, g);
+    hipLaunchKernelGGL((k_gemm_tile<64, AK, SCORES>), dim3(grid), dim3(256), tile_lds_bytes(64), st, g, tr);
 }
 
 // What a pass of the all-scores form does beyond the RoPE recurrence.
@@ -1608,18 +1620,23 @@ static int prefill_pass_scores(bdh_ctx *ctx, int B, int h, int T, int N, int d, 
     memcpy(g.head_par, pm.head_par, sizeof(g.head_par));
   };
 
-  // 0. V^T (and rho0^T): make every B operand k-contiguous
-  {
-    TransposeArgs t{};
-    t.v = v_bf16; t.rho = rho;
-    t.vs = Vs; t.vt = Vt; t.rt = Rt;
-    t.v_batch = v_batch;
-    t.B = B; t.h = h; t.T = T; t.d = d; t.Tp = Tp; t.Nq = Nq;
-    t.v_tiles = ((d + 63) / 64) * ((Tp + 63) / 64);
-    t.kinds = pm.decay ? 1 + h : 1;
-    memcpy(t.log_decay.v, pm.head_par, sizeof(t.log_decay.v));
-    const long blocks = (long)t.v_tiles * B * t.kinds + (has_state ? (long)((d + 63) / 64) * ((Nq + 63) / 64) * S : 0);
-    if (blocks > 0x7fffffffL) return bdh_fail(ctx, BDH_E_SHAPE, "too many tiles (T=%d N=%d)", T, N);
+  // 0. V^T (and rho0^T): make every B operand k-contiguous; behind the score tiles where those are in k_gemm_tile and there are at
+  // most 17 such tiles for every CU: the LDS of a score tile leaves each CU two workgroups, too few for more than that (us a
+  // call, its own launch | behind the scores: 272 tiles (T = 64) 32.8 | 27.7, 3852 174 | 164, 4112 210 | 196, 4800 322 | 326,
+  // 8352 195 | 201, 16416 304 | 345).
+  TransposeArgs t{};
+  t.v = v_bf16; t.rho = rho;
+  t.vs = Vs; t.vt = Vt; t.rt = Rt;
+  t.v_batch = v_batch;
+  t.B = B; t.h = h; t.T = T; t.d = d; t.Tp = Tp; t.Nq = Nq;
+  t.v_tiles = ((d + 63) / 64) * ((Tp + 63) / 64);
+  t.kinds = pm.decay ? 1 + h : 1;
+  memcpy(t.log_decay.v, pm.head_par, sizeof(t.log_decay.v));
+  const long blocks = (long)t.v_tiles * B * t.kinds + (has_state ? (long)((d + 63) / 64) * ((Nq + 63) / 64) * S : 0);
+  if (blocks > 0x7fffffffL / 2) return bdh_fail(ctx, BDH_E_SHAPE, "too many tiles (T=%d N=%d)", T, N);
+  const bool behind_scores = !big && blocks <= 17 * full_chip;
+  t.blocks = behind_scores ? (int)blocks : 0;
+  if (!behind_scores) {
     hipLaunchKernelGGL(k_transpose_operands, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, t);
     BDH_LAUNCH_CHECK(ctx, "k_transpose_operands");
   }
@@ -1646,7 +1663,7 @@ static int prefill_pass_scores(bdh_ctx *ctx, int B, int h, int T, int N, int d, 
     g.tri = full_grid ? 0 : 1; g.mt = mt_s; g.nt = mt_s; g.n_tiles = n_score_tiles; g.n_slices = S;
     if (ext)
       with_mode(g, (pm.decay ? GM_DECAY_SCORES : 0) | (pm.add_alibi ? GM_ADD_ALIBI : 0) | (pm.row_norm ? GM_ROWNORM : 0));
-    if (!big) launch_gemm_tile<false, true>(ctx->stream, g, tile_s);
+    if (!big) launch_gemm_tile<false, true>(ctx->stream, g, tile_s, t);
     else if (ext) BDH_HIP_CHECK(ctx, launch_gemm_direct<EPI_SCORES_X>(ctx->stream, g));
     else BDH_HIP_CHECK(ctx, launch_gemm_direct<EPI_SCORES>(ctx->stream, g));
     BDH_LAUNCH_CHECK(ctx, "scores");
