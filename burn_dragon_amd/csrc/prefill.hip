@@ -454,25 +454,24 @@ __global__ __launch_bounds__(256, 2) void k_gemm_tile(GemmArgs g, TransposeArgs 
     }
     const unsigned short *a0 = A + (A_KMAJOR ? (long)m0 : (long)m0 * lda), *b0 = B + (long)n0 * ldb;
     const int steps = (K + BK - 1) / BK;
-    auto issue = [&](int s) {
+    // pieces [c0, c1) of both panels of step s
+    auto issue = [&](int s, int c0, int c1) {
       unsigned short *dst = s_dyn + (s % NS) * STAGE + wave * 512;
       const int k0 = s * BK;
       const unsigned short *as = a0 + (A_KMAJOR ? (long)k0 * lda : (long)k0), *bs = b0 + k0;
       if (k0 + BK <= K) {
 #pragma unroll
-        for (int c = 0; c < NP; ++c) bdh_copy_to_lds(as, pa[c], dst + c * 2048);
+        for (int c = c0; c < c1; ++c) bdh_copy_to_lds(as, pa[c], dst + c * 2048);
 #pragma unroll
-        for (int c = 0; c < NP; ++c) bdh_copy_to_lds(bs, pb[c], dst + PANEL + c * 2048);
+        for (int c = c0; c < c1; ++c) bdh_copy_to_lds(bs, pb[c], dst + PANEL + c * 2048);
       } else {
         const char *zero = reinterpret_cast<const char *>(&g_zero_piece);
 #pragma unroll
-        for (int c = 0; c < NP; ++c) {
+        for (int c = c0; c < c1; ++c) {
           const int k = A_KMAJOR ? k0 + (c * 256 + tid) / (TS / 8) : k0 + kc;
           bdh_copy_to_lds(k < K ? reinterpret_cast<const char *>(as) + pa[c] : zero, dst + c * 2048);
-        }
-#pragma unroll
-        for (int c = 0; c < NP; ++c)
           bdh_copy_to_lds(k0 + kc < K ? reinterpret_cast<const char *>(bs) + pb[c] : zero, dst + PANEL + c * 2048);
+        }
       }
     };
     // The operands of the next 16 k are read into a second set of registers while these are multiplied, also across a step:
@@ -525,31 +524,49 @@ __global__ __launch_bounds__(256, 2) void k_gemm_tile(GemmArgs g, TransposeArgs 
     };
 #pragma unroll
     for (int s = 0; s < NS - 1; ++s)
-      if (s < steps) issue(s);
+      if (s < steps) issue(s, 0, NP);
     if (steps > 0) {
       arrive(0);
       read(0, 0, 0);
-      if (NS - 1 < steps) issue(NS - 1);
     }
-    auto inside = [&](int s) {  // all of a step but its last products
+    // A wave that asks for many copies at once is held up by them (about 100 cycles each).  With three steps on their way they
+    // go out a few at a time, under products; with one (128 wide) the time that it has to arrive counts for more, and all of
+    // them follow the barrier at once (us, at once | spread: readout of the call above in 64 wide tiles 56 | 50, its scores in
+    // 128 wide ones 62 | 71).
+    constexpr bool SPREAD = NS > 2;
+    auto inside = [&](int s, bool more) {  // all of a step but its last products
 #pragma unroll
       for (int q = 0; q < BK / 16 - 1; ++q) {
         read(s, 16 * (q + 1), (q + 1) & 1);
         __builtin_amdgcn_sched_barrier(0);  // left alone, the scheduler sinks the reads to their use
         multiply(q & 1);
+        if (SPREAD && more && q < NP) {
+          issue(s + NS - 1, q, q + 1);
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
     };
+    static_assert(!SPREAD || NP <= BK / 16 - 1, "a piece per group of products");
     // (the last step by itself: behind a branch the compiler would wait for the operands just asked for)
-    for (int s = 0; s + 1 < steps; ++s) {
-      inside(s);
+    if (!SPREAD && NS - 1 < steps) issue(NS - 1, 0, NP);
+    int s = 0;
+    auto next = [&](int s) {
       arrive(s + 1);
       read(s + 1, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
       multiply(1);
-      if (s + NS < steps) issue(s + NS);  // under the products just started
+    };
+    for (; s + NS - 1 < steps; ++s) {
+      inside(s, true);
+      next(s);
+      if (!SPREAD && s + NS < steps) issue(s + NS, 0, NP);  // under the products just started
+    }
+    for (; s + 1 < steps; ++s) {
+      inside(s, false);
+      next(s);
     }
     if (steps > 0) {
-      inside(steps - 1);
+      inside(steps - 1, false);
       multiply(1);
     }
     lds_barrier();  // every wave is past its reads: the stages are free
