@@ -52,7 +52,8 @@ struct GemmF32 {
 };
 constexpr int GEMM_STORE = 0, GEMM_SCORES = 1, GEMM_NORM = 2, GEMM_GATE = 3;
 
-// How a product is cut: tile (0: 128 x 128, 1: 64 x 64, 2: 32 x 128, 3: 128 x 256) and the number of parts of K.
+// How a product is cut: tile (0: 128 x 128, 1: 64 x 64, 2: 32 x 128, 3: 128 x 256, 4: 32 x 32 with K dealt to the wavefronts)
+// and the number of parts of K.
 struct GemmPlan {
   int tile = 0, ks = 1;
 };

@@ -134,6 +134,62 @@ struct Tile {
   }
 };
 
+// What a scores product stores for the sum v of (row, col), col < g.N.
+__device__ __forceinline__ float score_value(const GemmF32 &g, float v, int row, int col, float ld, float slope) {
+  const int rb = row / g.block_size, cb = col / g.block_size;
+  if (!(g.active ? g.active[(long)rb * g.tb + cb] != 0 : cb <= rb)) return 0.0f;
+  if (rb == cb && col >= row) v = 0.0f;  // tril(-1) on diagonal blocks (:88-90)
+  if (g.decay_scores && col < row) v = v * expf((float)(row - col) * ld);
+  if (g.use_alibi) {  // added to every entry of an active block (:97-100)
+    const float al = slope * ((float)col - (float)row);
+    v = v + al;
+  }
+  return v;
+}
+
+// The tile of this workgroup.  XCD-aware mapping: workgroup ids are dealt round-robin to the 8 XCDs, so ids with the same
+// (id % 8) share an L2.  Each XCD takes one contiguous eighth of the (slice, part of K, tile) list: neighbouring tiles reuse
+// their operand rows in one L2, and every XCD has the same number of tiles whatever the number of slices.
+struct TileAt {
+  int part, slice, ti, tj;
+  __device__ __forceinline__ bool find(const GemmF32 &g) {
+    const int tiles = g.tri ? g.mt * (g.mt + 1) / 2 : g.mt * g.nt;
+    const long total = (long)g.n_slices * g.ks * tiles;
+    const int xcd = blockIdx.x & 7;
+    const long at = total * xcd / 8 + (blockIdx.x >> 3);
+    if (at >= total * (xcd + 1) / 8) return false;
+    part = (int)(at / tiles % g.ks);
+    slice = (int)(at / tiles / g.ks);
+    int tile = (int)(at % tiles);
+    // A CU often gets the same tile of several slices: after a long row tile a short one (32 slices of [511 x 511] x [511 x
+    // 256], row tiles of 2 to 16 stages: 38 -> 30 us).
+    if (g.causal_k && (slice & 1)) tile = tiles - 1 - tile;
+    if (g.tri) {  // lower triangle of square tiles, row by row
+      ti = (int)((sqrtf(8.0f * (float)tile + 1.0f) - 1.0f) * 0.5f);
+      while ((ti + 1) * (ti + 2) / 2 <= tile) ++ti;
+      while (ti * (ti + 1) / 2 > tile) --ti;
+      tj = tile - ti * (ti + 1) / 2;
+    } else {
+      ti = tile / g.nt;
+      tj = tile - ti * g.nt;
+    }
+    return true;
+  }
+};
+
+// The ends of K for a tile of rows [m0, m0 + bm) and columns from n0 on: of A . B and of A2 . B2.
+__device__ __forceinline__ void ends_of_k(const GemmF32 &g, bool scores, int m0, int bm, int n0, int &K1, int &K2) {
+  const int bs = g.block_size, last = min(m0 + bm, g.M) - 1, k_causal = (last / bs + 1) * bs;
+  K1 = g.K;
+  K2 = g.A2 ? g.K2 : 0;
+  if (g.causal_k) {
+    if (g.A2) K2 = min(K2, k_causal);
+    else K1 = min(K1, k_causal);
+  }
+  // a scores tile above the diagonal of the block pattern only writes zeros
+  if (scores && !g.active && n0 / bs > last / bs) K1 = 0;
+}
+
 // BM x BN tile per workgroup of WM x WN wavefronts.  With four wavefronts LDS holds one stage (192 bytes per tile row and column: 48 KiB at
 // 128 x 128; the registers allow two workgroups per CU); the next stage's loads are in flight in registers while this one is multiplied,
 // and the other workgroups of the CU fill the two barriers.  What bounds it: at 128 x 128 a wavefront spends 1536 cycles
@@ -149,49 +205,21 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_f32(GemmF32 g) {
   __shared__ __attribute__((aligned(16))) unsigned char s_a[(TURNS ? 2 : 1) * 3 * BM * 64];
   __shared__ __attribute__((aligned(16))) unsigned char s_b[(TURNS ? 2 : 1) * 3 * BN * 64];
   __shared__ float s_norm[EPI == GEMM_NORM ? BM : 1];
-  // XCD-aware mapping: workgroup ids are dealt round-robin to the 8 XCDs, so ids with the same (id % 8) share an L2.
-  // Each XCD takes one contiguous eighth of the (slice, part of K, tile) list: neighbouring tiles reuse their operand
-  // rows in one L2, and every XCD has the same number of tiles whatever the number of slices.
-  const int tiles = g.tri ? g.mt * (g.mt + 1) / 2 : g.mt * g.nt;
-  const long total = (long)g.n_slices * g.ks * tiles;
-  const int xcd = blockIdx.x & 7;
-  const long at = total * xcd / 8 + (blockIdx.x >> 3);
-  if (at >= total * (xcd + 1) / 8) return;
-  const int part = (int)(at / tiles % g.ks);
-  const int slice = (int)(at / tiles / g.ks);
-  int tile = (int)(at % tiles);
-  // A CU often gets the same tile of several slices: after a long row tile a short one (32 slices of [511 x 511] x [511 x
-  // 256], row tiles of 2 to 16 stages: 38 -> 30 us).
-  if (g.causal_k && (slice & 1)) tile = tiles - 1 - tile;
-  int ti, tj;
-  if (g.tri) {  // lower triangle of square tiles, row by row
-    ti = (int)((sqrtf(8.0f * (float)tile + 1.0f) - 1.0f) * 0.5f);
-    while ((ti + 1) * (ti + 2) / 2 <= tile) ++ti;
-    while (ti * (ti + 1) / 2 > tile) --ti;
-    tj = tile - ti * (ti + 1) / 2;
-  } else {
-    ti = tile / g.nt;
-    tj = tile - ti * g.nt;
-  }
-  const int m0 = ti * BM, n0 = tj * BN;
+  TileAt here;
+  if (!here.find(g)) return;
+  const int part = here.part, slice = here.slice;
+  const int m0 = here.ti * BM, n0 = here.tj * BN;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN;
   const long s1 = slice / g.mod, s2 = slice % g.mod;
   const float *A = g.A + s1 * g.a_s1 + s2 * g.a_s2;
   const float *B = g.B + s1 * g.b_s1 + s2 * g.b_s2;
   float *C = g.C + s1 * g.c_s1 + s2 * g.c_s2;
-  const int bs = g.block_size;
   const float ld = (g.decay_rows || g.decay_state || g.decay_scores) ? g.log_decay[slice % g.heads] : 0.0f;
 
   // the k blocks of this part: first those of A . B, then those of A2 . B2
-  const int k_causal = ((min(m0 + BM, g.M) - 1) / bs + 1) * bs;
-  int K1 = g.K, K2 = g.A2 ? g.K2 : 0;
-  if (g.causal_k) {
-    if (g.A2) K2 = min(K2, k_causal);
-    else K1 = min(K1, k_causal);
-  }
-  // a scores tile above the diagonal of the block pattern only writes zeros
-  if (EPI == GEMM_SCORES && !g.active && n0 / bs > (min(m0 + BM, g.M) - 1) / bs) K1 = 0;
+  int K1, K2;
+  ends_of_k(g, EPI == GEMM_SCORES, m0, BM, n0, K1, K2);
   const int nb1 = (K1 + FK - 1) / FK, nb = nb1 + (K2 + FK - 1) / FK;
   const int b_lo = part * g.kb_per, b_hi = min(nb, b_lo + g.kb_per);
 
@@ -450,19 +478,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_f32(GemmF32 g) {
         float v = acc[i][j][e];
         if (EPI == GEMM_SCORES) {
           if (col >= g.ldc) continue;
-          bool act = col < g.N;
-          const int rb = row / bs, cb = col / bs;
-          if (act) act = g.active ? g.active[(long)rb * g.tb + cb] != 0 : cb <= rb;
-          if (act) {
-            if (rb == cb && col >= row) v = 0.0f;  // tril(-1) on diagonal blocks (:88-90)
-            if (g.decay_scores && col < row) v = v * expf((float)(row - col) * ld);
-            if (g.use_alibi) {  // added to every entry of an active block (:97-100)
-              const float al = slope * ((float)col - (float)row);
-              v = v + al;
-            }
-          } else {
-            v = 0.0f;
-          }
+          v = col < g.N ? score_value(g, v, row, col, ld, slope) : 0.0f;
           C[(long)row * g.ldc + col] = v;
         } else {
           if (col >= g.N) continue;
@@ -477,6 +493,137 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_f32(GemmF32 g) {
     }
 }
 
+// 32 x 32 tile per workgroup, for products of few tiles and a short K: the four wavefronts share K, sixteen at a time in turn.
+// An element then belongs to one lane, which loads it where it is fed to the matrix instruction, so nothing passes through LDS
+// but the wavefronts' sums at the end, and four steps are on their way at a time.  What bounds it: a trip to memory or two and the
+// launch; in the tiles above a stage is a chain of loads, conversions, two barriers and dependent products, about 1.2 us long
+// when nothing else is on the CU (us, 64 x 64 | this, 4 slices of a prompt of 128 tokens, N = 256, d = 256: scores 14.8 | 7.8,
+// readout 13.4 | 7.2, state 10.9 | 6.4, encoder 10.7 | 7.2).
+template <bool AK, bool BK, int EPI>
+__global__ __launch_bounds__(256, 2) void k_gemm_f32_small(GemmF32 g) {
+  constexpr int TS = 32, U = 4;
+  __shared__ float s_sum[4][16][64];
+  __shared__ float s_norm[EPI == GEMM_NORM ? 4 : 1][TS];
+  TileAt here;
+  if (!here.find(g)) return;
+  const int slice = here.slice, m0 = here.ti * TS, n0 = here.tj * TS;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 31, half = lane >> 5;
+  const long s1 = slice / g.mod, s2 = slice % g.mod;
+  float *C = g.C + s1 * g.c_s1 + s2 * g.c_s2;
+  const float ld = (g.decay_rows || g.decay_state || g.decay_scores) ? g.log_decay[slice % g.heads] : 0.0f;
+  int K1, K2;
+  ends_of_k(g, EPI == GEMM_SCORES, m0, TS, n0, K1, K2);
+
+  f32x16 acc = (f32x16)(0.0f), low = (f32x16)(0.0f);  // the sums of h h, and of the five smaller terms
+  float rs = 0.0f;
+  auto run = [&](const float *A, int lda, int rows_per, long a_outer, const float *B, int ldb, int K) {
+    const int ar = min(m0 + r, g.M - 1), bc = min(n0 + r, g.N - 1);  // past the end: the last one again, not stored
+    const float *pa = A + (AK ? (long)ar : rows_per > 0 ? (long)(ar / rows_per) * a_outer + (long)(ar % rows_per) * lda : (long)ar * lda);
+    const float *pb = B + (BK ? (long)bc : (long)bc * ldb);
+    const bool a_ok = (lda & 3) == 0 && (a_outer & 3) == 0 && (reinterpret_cast<uintptr_t>(A) & 15) == 0;
+    const bool b_ok = (ldb & 3) == 0 && (reinterpret_cast<uintptr_t>(B) & 15) == 0;
+    float a[U][8], b[U][8];
+    auto eight = [&](float(&v)[8], const float *p, bool kmajor, int ld_, bool whole_pieces, int k) {
+      if (kmajor) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = p[(long)(k + q) * ld_];
+      } else if (whole_pieces) {
+        const float4 lo = *reinterpret_cast<const float4 *>(p + k), hi = *reinterpret_cast<const float4 *>(p + k + 4);
+        v[0] = lo.x; v[1] = lo.y; v[2] = lo.z; v[3] = lo.w;
+        v[4] = hi.x; v[5] = hi.y; v[6] = hi.z; v[7] = hi.w;
+      } else {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = p[k + q];
+      }
+    };
+    auto consume = [&](float(&va)[8], float(&vb)[8], int k) {
+      if (AK && EPI == GEMM_STORE && g.decay_state) {  // token k of K is decayed K - k times by the end (beyond K: by 1)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) va[q] *= expf((float)max(K - (k + q), 0) * ld);
+      }
+      if (EPI == GEMM_NORM) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) rs += fabsf(va[q]);
+      }
+      u32x4 fa[3], fb[3];
+      split3(va, fa[0], fa[1], fa[2]);
+      split3(vb, fb[0], fb[1], fb[2]);
+      constexpr int TA[6] = {2, 0, 1, 1, 0, 0}, TB[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+      for (int t = 0; t < 6; ++t) {
+        f32x16 &sum = t == 5 ? acc : low;
+        sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fa[TA[t]]), __builtin_bit_cast(bf16x8, fb[TB[t]]), sum, 0, 0, 0);
+      }
+    };
+    const int full = K >> 4;  // whole steps of 16
+    for (int s = wave; s < full; s += 4 * U) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k = min(s + 4 * u, full - 1) * 16 + half * 8;  // (past the end: what comes is not used)
+        eight(a[u], pa, AK, lda, a_ok, k);
+        eight(b[u], pb, BK, ldb, b_ok, k);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (s + 4 * u < full) consume(a[u], b[u], (s + 4 * u) * 16 + half * 8);
+    }
+    if ((K & 15) && wave == (full & 3)) {  // what K leaves over, zeros beyond
+      const int k = full * 16 + half * 8;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const bool in = k + q < K;
+        a[0][q] = in ? (AK ? pa[(long)(k + q) * lda] : pa[k + q]) : 0.0f;
+        b[0][q] = in ? (BK ? pb[(long)(k + q) * ldb] : pb[k + q]) : 0.0f;
+      }
+      consume(a[0], b[0], k);
+    }
+    acc += low;
+    low = (f32x16)(0.0f);
+  };
+  run(g.A + s1 * g.a_s1 + s2 * g.a_s2, g.lda, g.rows_per, g.a_outer, g.B + s1 * g.b_s1 + s2 * g.b_s2, g.ldb, K1);
+  if (EPI == GEMM_STORE && g.decay_rows) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[e] *= expf((float)(m0 + (e >> 2) * 8 + half * 4 + (e & 3)) * ld);
+  }
+  if constexpr (!AK && BK && EPI == GEMM_STORE) {
+    if (K2 > 0)
+      run(g.A2 + s1 * g.a2_s1 + s2 * g.a2_s2, g.lda2, 0, 0, g.B2 + s1 * g.b2_s1 + s2 * g.b2_s2, g.ldb2, K2);
+  }
+#pragma unroll
+  for (int e = 0; e < 16; ++e) s_sum[wave][e][lane] = acc[e];
+  if (EPI == GEMM_NORM) {
+    rs += __shfl_xor(rs, 32);
+    if (half == 0) s_norm[wave][r] = rs;
+  }
+  __syncthreads();
+  // wavefront w finishes rows 8 w .. 8 w + 7 of the tile: elements 4 w .. 4 w + 3 of the accumulators, summed in order
+  const int col = n0 + r, row0 = m0 + wave * 8 + half * 4;
+  const float slope = (EPI == GEMM_SCORES && g.use_alibi) ? g.slopes[slice % g.heads] : 0.0f;
+  const bool reads_c = EPI == GEMM_STORE && (g.accumulate || g.decay_state);  // C in one piece: the launcher sees to it
+  const float keep = g.decay_state ? expf((float)g.K * ld) : 1.0f;
+  const float *G = EPI == GEMM_GATE ? g.gate + s1 * g.c_s1 + s2 * g.c_s2 : nullptr;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int row = row0 + e, from = 4 * wave + e;
+    if (row >= g.M || col >= (EPI == GEMM_SCORES ? g.ldc : g.N)) continue;
+    float v = ((s_sum[0][from][lane] + s_sum[1][from][lane]) + s_sum[2][from][lane]) + s_sum[3][from][lane];
+    const long at = (g.rows_per > 0 ? (long)(row / g.rows_per) * g.c_outer + (long)(row % g.rows_per) * g.ldc : (long)row * g.ldc) + col;
+    if (EPI == GEMM_SCORES) v = col < g.N ? score_value(g, v, row, col, ld, slope) : 0.0f;
+    if (EPI == GEMM_NORM) {
+      const int rr = row - m0;
+      v = v / ((((s_norm[0][rr] + s_norm[1][rr]) + s_norm[2][rr]) + s_norm[3][rr]) + kRowNormEps);
+    }
+    if (EPI == GEMM_GATE) {
+      v -= g.threshold;
+      v = G[at] * (v <= 0.0f ? 0.0f : v);
+    }
+    if (reads_c) v = (g.decay_state ? C[at] * keep : C[at]) + v;
+    C[at] = v;
+  }
+}
+
 template <int EPI>
 void launch(hipStream_t st, const GemmF32 &g, bool ak, bool bk, int tile, unsigned grid) {
 #define BDH_G(BM_, BN_, WM_, WN_, AK_, BK_) \
@@ -486,7 +633,8 @@ void launch(hipStream_t st, const GemmF32 &g, bool ak, bool bk, int tile, unsign
     if (tile == 0) BDH_G(128, 128, 2, 2, AK_, BK_);          \
     else if (tile == 1) BDH_G(64, 64, 2, 2, AK_, BK_);       \
     else if (tile == 2) BDH_G(32, 128, 1, 4, AK_, BK_);      \
-    else BDH_G(128, 256, 2, 4, AK_, BK_);                    \
+    else if (tile == 3) BDH_G(128, 256, 2, 4, AK_, BK_);     \
+    else hipLaunchKernelGGL((k_gemm_f32_small<AK_, BK_, EPI>), dim3(grid), dim3(256), 0, st, g); \
   } while (0)
   if constexpr (EPI == GEMM_SCORES) {
     BDH_GT(false, false);
@@ -500,7 +648,7 @@ void launch(hipStream_t st, const GemmF32 &g, bool ak, bool bk, int tile, unsign
 #undef BDH_G
 }
 
-constexpr int kTileM[4] = {128, 64, 32, 128}, kTileN[4] = {128, 64, 128, 256};
+constexpr int kTileM[5] = {128, 64, 32, 128, 32}, kTileN[5] = {128, 64, 128, 256, 32};
 
 // scores over causal time blocks that end on tile edges: the tiles above the diagonal hold nothing, and a reader whose
 // own row tiles are no larger never looks at them
@@ -531,7 +679,11 @@ double causal_share(const GemmF32 &g, int tile_rows) {
 // itself: a stage takes `turn`, and nothing covers its first loads and its last stores, `turn_end` a tile (12 slices of
 // [500 x 8192] x [8192 x 256] in 5 parts: 161 us, in 128 x 128 tiles and 8 parts 185; with a K of 500, [8192 x 500] x [500 x 256],
 // 181 against 176; 32 slices of [511 x 511] x [511 x 256] 56 against 46).  More parts of K fill the
-// chip where the tiles are few, at the price of writing and re-reading every part.
+// chip where the tiles are few, at the price of writing and re-reading every part.  A 32 x 32 tile (k_gemm_f32_small) has no
+// barriers: 750 a stage by itself, 500 where a CU has several.  Whole calls with it over calls without: prompts of 16 to 256
+// tokens through 4 heads of 128 to 256 neurons 0.69 to 0.87, 8 heads of 256, d = 512, 0.76 to 0.92, 4 heads of 1024, 256 tokens
+// 0.91; scoring 128 to 300 tokens 0.67 to 0.96; of 144 calls of 16 to 4088 tokens, up to 8192 neurons a head, four are 2 to 3 %
+// slower.
 GemmPlan bdh_gemm_f32_plan(const bdh_ctx *ctx, const GemmF32 &g, int max_split) {
   const double n_cu = ctx->n_cu > 0 ? ctx->n_cu : 256;
   constexpr double full[3] = {2600.0, 900.0, 900.0}, alone[3] = {3600.0, 2000.0, 2000.0};
@@ -539,18 +691,20 @@ GemmPlan bdh_gemm_f32_plan(const bdh_ctx *ctx, const GemmF32 &g, int max_split) 
   const int nb = (g.K + FK - 1) / FK + (g.K2 + FK - 1) / FK;
   GemmPlan best;
   double best_t = 1e300;
-  for (int t = 0; t < 4; ++t) {
+  for (int t = 0; t < 5; ++t) {
     if (t == 2 && (g.epilogue == GEMM_SCORES || g.M > 96)) continue;
     const double mt = (g.M + kTileM[t] - 1) / kTileM[t], nt = (g.N + kTileN[t] - 1) / kTileN[t];
     const bool tri = lower_triangle(g, t);
     const double tiles = g.n_slices * (tri ? mt * (mt + 1) / 2 : mt * nt);
     const double share = causal_share(g, kTileM[t]);
-    for (int ks = 1; ks <= max_split && (ks == 1 || nb >= 4 * ks); ks = t == 3 ? ks + 1 : ks * 2) {
+    for (int ks = 1; ks <= (t == 4 ? 1 : max_split) && (ks == 1 || nb >= 4 * ks); ks = t == 3 ? ks + 1 : ks * 2) {
       const double per = (nb + ks - 1) / ks, mean = per * share;
       const double wgs = tiles * ks / n_cu;
       const double rounds = wgs <= 1.0 ? 1.0 : wgs;
       double cyc;
-      if (t == 3) {
+      if (t == 4) {
+        cyc = std::max(mean * rounds * 500.0, per * 750.0) + 3000.0;
+      } else if (t == 3) {
         cyc = std::ceil(rounds) * (per * turn + turn_end);
       } else {
         cyc = std::max(mean * rounds * full[t], per * alone[t]) + 6000.0;

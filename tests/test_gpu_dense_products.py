@@ -342,3 +342,71 @@ def test_gated_projection_of_a_prompt_on_split_products(d, h, N, B, T):
     for a, b in zip(*got):
         assert not torch.equal(a, b)
         assert float((a - b).abs().max() / a.abs().max()) < 1e-5
+
+
+def _launched(call):
+    from torch.profiler import ProfilerActivity, profile
+
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        out = call()
+        torch.cuda.synchronize()
+    return out, " ".join(e.key for e in prof.key_averages())
+
+
+@pytest.mark.parametrize("rotary", ["rope", "alibi", "pope"])
+@pytest.mark.parametrize("B,h,T,N,d", [
+    (1, 2, 8, 16, 32),     # one step of k for one of the four wavefronts, tiles that end inside
+    (1, 3, 33, 62, 36),    # a k that ends inside a step, in every product; a second row tile of one row
+    (2, 2, 65, 34, 100),   # rows that are no whole 16-byte pieces
+    (1, 4, 128, 256, 256),
+    (1, 1, 200, 250, 64),
+])
+def test_products_of_few_tiles(bda, rotary, B, h, T, N, d):
+    """32 x 32 tiles whose wavefronts share K: scores, readout and state of a short prompt against the loop over its tokens, the
+    same sums reassociated (a few hundred terms, 2^-24 each): 2e-5 as for the other tiles; the stateless form (time blocks,
+    additive ALiBi terms, row norms) against itself in float64."""
+    from burn_dragon_amd.recurrent import recurrent_attention
+
+    g = torch.Generator(device=DEV).manual_seed(T + N)
+    rot = bda.RotaryEmbedding.parse(rotary)
+    x = torch.relu(torch.randn((B, h, T, N), device=DEV, generator=g))
+    v = torch.randn((B, T, d), device=DEV, generator=g)
+    rho = 0.1 * torch.randn((B, h, 2 * N if rotary == "pope" else N, d), device=DEV, generator=g)
+    freqs = torch.rand(N, device=DEV, generator=g).repeat_interleave(2)[:N].contiguous()
+    ctx = bda.ffi.default_context(0)
+    got = []
+    for mode in (0, 1):
+        state = rho.clone()
+        ctx.set_option("state_step.dense_chunks", mode)
+        try:
+            out, ran = _launched(lambda: recurrent_attention(x, v, state, freqs, 5, rot))
+        finally:
+            ctx.set_option("state_step.dense_chunks", -1)
+        assert ("k_gemm_f32_small" in ran) == (mode == 1)
+        got.append((out, state))
+    for a, b in zip(*got):
+        assert float((a - b).abs().max() / a.abs().max()) < 2e-5
+
+
+@pytest.mark.parametrize("T,N,d,block", [(130, 48, 36, 1), (129, 20, 32, 64), (160, 64, 64, 32)])
+def test_row_norms_of_few_tiles(bda, T, N, d, block):
+    """The stateless form on 32 x 32 tiles against its formula in float64: sums of up to 160 terms over their norm, 1e-5."""
+    from burn_dragon_amd.kernel.block_sparse import BlockPattern2d
+    from burn_dragon_amd.kernel.linear_attention import fused_state_aligned
+
+    B, h = 2, 2
+    g = torch.Generator(device=DEV).manual_seed(T)
+    q = torch.relu(torch.randn((B, h, T, N), device=DEV, generator=g))
+    v = torch.randn((B, 1, T, d), device=DEV, generator=g)
+    slopes = torch.tensor([0.5, 0.25])
+    freqs = torch.zeros((1, 1, 1, N), device=DEV)
+    (out, ran) = _launched(lambda: fused_state_aligned(q, v, freqs, slopes, BlockPattern2d.dense(block), bda.RotaryEmbedding.ALIBI))
+    assert "k_gemm_f32_small" in ran
+    t = torch.arange(T, device=DEV)
+    s = torch.matmul(q.double(), q.double().transpose(-1, -2).contiguous())
+    same = t[:, None] // block == t[None] // block
+    s = torch.where(same & (t[None] >= t[:, None]), torch.zeros_like(s), s)
+    s = s + slopes.to(DEV).double()[:, None, None] * (t[None] - t[:, None]).double()
+    s = torch.where(t[None] // block <= t[:, None] // block, s, torch.zeros_like(s))
+    ref = torch.matmul(s, v.double()) / (s.abs().sum(-1, keepdim=True) + 1e-6)
+    assert float((out.double() - ref).abs().max() / ref.abs().max()) < 1e-5
