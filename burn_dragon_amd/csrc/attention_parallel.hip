@@ -195,15 +195,24 @@ __global__ __launch_bounds__(256) void k_scores_reduce(const float *__restrict__
   const int end = g.active ? g.N : min(g.N, ((min((row | 127) + 1, g.M) - 1) / bs + 1) * bs);
   const float *p = parts + ((long)slice * g.M + row) * g.N;
   float *C = g.C + (long)(slice / g.mod) * g.c_s1 + (long)(slice % g.mod) * g.c_s2 + (long)row * g.ldc;
-  const int rb = row / bs;
+  const int rb = bdh_time_block(g, row);
   const float ld = g.log_decay[slice % g.heads], slope = g.slopes[slice % g.heads];
   for (int col = threadIdx.x; col < end; col += 256) {
-    const int cb = col / bs;
+    const int cb = bdh_time_block(g, col);
     const bool act = g.active ? g.active[(long)rb * g.tb + cb] != 0 : cb <= rb;
     float v = 0.0f;
     if (act) {
-      if (!(rb == cb && col >= row))
-        for (int k = 0; k < g.ks; ++k) v += p[k * c_split + col];
+      if (!(rb == cb && col >= row)) {
+        int k = 0;
+        for (; k + 4 <= g.ks; k += 4) {  // four parts on their way at a time
+          float t[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) t[u] = p[(k + u) * c_split + col];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) v += t[u];
+        }
+        for (; k < g.ks; ++k) v += p[k * c_split + col];
+      }
       if (g.decay_scores && col < row) v = v * expf((float)(row - col) * ld);
       if (g.use_alibi) {
         const float al = slope * ((float)col - (float)row);
@@ -697,6 +706,7 @@ int launch_scores(bdh_ctx *ctx, const GemmF32 &g, const GemmPlan &plan, float *p
   if (rc != BDH_OK || plan.ks == 1) return rc;
   GemmF32 r = g;
   r.ks = plan.ks;
+  r.block_shift = g.block_size > 0 && (g.block_size & (g.block_size - 1)) == 0 ? __builtin_ctz(g.block_size) : -1;
   hipLaunchKernelGGL(k_scores_reduce, dim3((unsigned)((long)g.n_slices * g.M)), dim3(256), 0, ctx->stream, parts,
                      (long)g.n_slices * g.M * g.N, r);
   BDH_LAUNCH_CHECK(ctx, "k_scores_reduce");

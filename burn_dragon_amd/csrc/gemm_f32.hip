@@ -136,7 +136,7 @@ struct Tile {
 
 // What a scores product stores for the sum v of (row, col), col < g.N.
 __device__ __forceinline__ float score_value(const GemmF32 &g, float v, int row, int col, float ld, float slope) {
-  const int rb = row / g.block_size, cb = col / g.block_size;
+  const int rb = bdh_time_block(g, row), cb = bdh_time_block(g, col);
   if (!(g.active ? g.active[(long)rb * g.tb + cb] != 0 : cb <= rb)) return 0.0f;
   if (rb == cb && col >= row) v = 0.0f;  // tril(-1) on diagonal blocks (:88-90)
   if (g.decay_scores && col < row) v = v * expf((float)(row - col) * ld);
@@ -174,6 +174,25 @@ struct TileAt {
       tj = tile - ti * g.nt;
     }
     return true;
+  }
+};
+
+// Where row m of C begins.  The place of the first of 32 neighbouring rows is worked out once, the others follow from it: a
+// division only where they run into the next sequence.
+struct RowPlaces {
+  int first, b0, t0;
+  __device__ __forceinline__ RowPlaces(const GemmF32 &g, int first_row) : first(first_row) {
+    b0 = g.rows_per > 0 ? first_row / g.rows_per : 0;
+    t0 = g.rows_per > 0 ? first_row - b0 * g.rows_per : 0;
+  }
+  __device__ __forceinline__ long at(const GemmF32 &g, int off) const {
+    if (g.rows_per <= 0) return (long)(first + off) * g.ldc;
+    int b = b0, t = t0 + off;
+    if (t >= g.rows_per) {
+      b += t / g.rows_per;
+      t %= g.rows_per;
+    }
+    return (long)b * g.c_outer + (long)t * g.ldc;
   }
 };
 
@@ -442,11 +461,10 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_f32(GemmF32 g) {
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
       long at[16];
+      const int first = min(row_of(i, 0), g.M - 1);
+      const RowPlaces places(g, first);
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int row = min(row_of(i, e), g.M - 1);
-        at[e] = g.rows_per > 0 ? (long)(row / g.rows_per) * g.c_outer + (long)(row % g.rows_per) * g.ldc : (long)row * g.ldc;
-      }
+      for (int e = 0; e < 16; ++e) at[e] = places.at(g, min(row_of(i, e), g.M - 1) - first);
       float gate[NJ][16];
 #pragma unroll
       for (int j = 0; j < NJ; ++j)
@@ -467,7 +485,8 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_f32(GemmF32 g) {
   }
   const float slope = (EPI == GEMM_SCORES && g.use_alibi) ? g.slopes[slice % g.heads] : 0.0f;
 #pragma unroll
-  for (int i = 0; i < MI; ++i)
+  for (int i = 0; i < MI; ++i) {
+    const RowPlaces places(g, row_of(i, 0));
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
       const int col = n0 + wn * (BN / WN) + j * 32 + (lane & 31);
@@ -482,15 +501,12 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_f32(GemmF32 g) {
           C[(long)row * g.ldc + col] = v;
         } else {
           if (col >= g.N) continue;
-          float *p = C + (g.rows_per > 0 ? (long)(row / g.rows_per) * g.c_outer + (long)(row % g.rows_per) * g.ldc
-                                         : (long)row * g.ldc) + col;
-          if (EPI == GEMM_NORM)
-            *p = v / (s_norm[row - m0] + kRowNormEps);
-          else
-            *p = v;
+          if (EPI == GEMM_NORM) v = v / (s_norm[row - m0] + kRowNormEps);
+          C[places.at(g, (e >> 2) * 8 + (e & 3)) + col] = v;
         }
       }
     }
+  }
 }
 
 // 32 x 32 tile per workgroup, for products of few tiles and a short K: the four wavefronts share K, sixteen at a time in turn.
@@ -604,12 +620,13 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f32_small(GemmF32 g) {
   const bool reads_c = EPI == GEMM_STORE && (g.accumulate || g.decay_state);  // C in one piece: the launcher sees to it
   const float keep = g.decay_state ? expf((float)g.K * ld) : 1.0f;
   const float *G = EPI == GEMM_GATE ? g.gate + s1 * g.c_s1 + s2 * g.c_s2 : nullptr;
+  const RowPlaces places(g, row0);
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const int row = row0 + e, from = 4 * wave + e;
     if (row >= g.M || col >= (EPI == GEMM_SCORES ? g.ldc : g.N)) continue;
     float v = ((s_sum[0][from][lane] + s_sum[1][from][lane]) + s_sum[2][from][lane]) + s_sum[3][from][lane];
-    const long at = (g.rows_per > 0 ? (long)(row / g.rows_per) * g.c_outer + (long)(row % g.rows_per) * g.ldc : (long)row * g.ldc) + col;
+    const long at = places.at(g, e) + col;
     if (EPI == GEMM_SCORES) v = col < g.N ? score_value(g, v, row, col, ld, slope) : 0.0f;
     if (EPI == GEMM_NORM) {
       const int rr = row - m0;
@@ -726,6 +743,7 @@ int bdh_gemm_f32_rows(const GemmPlan &plan) { return kTileM[plan.tile]; }
 int bdh_launch_gemm_f32(bdh_ctx *ctx, GemmF32 g, bool a_kmajor, bool b_kmajor, const GemmPlan &plan, float *partial) {
   if ((g.accumulate || g.decay_state) && g.rows_per > 0)
     return bdh_fail(ctx, BDH_E_UNSUPPORTED, "a product that is added to what C holds takes C in one piece");
+  g.block_shift = g.block_size > 0 && (g.block_size & (g.block_size - 1)) == 0 ? __builtin_ctz(g.block_size) : -1;
   g.mt = (g.M + kTileM[plan.tile] - 1) / kTileM[plan.tile];
   g.nt = (g.N + kTileN[plan.tile] - 1) / kTileN[plan.tile];
   g.tri = lower_triangle(g, plan.tile);
