@@ -153,17 +153,18 @@ __device__ __forceinline__ float score_value(const GemmF32 &g, float v, int row,
 struct TileAt {
   int part, slice, ti, tj;
   __device__ __forceinline__ bool find(const GemmF32 &g) {
-    const int tiles = g.tri ? g.mt * (g.mt + 1) / 2 : g.mt * g.nt;
-    const long total = (long)g.n_slices * g.ks * tiles;
-    const int xcd = blockIdx.x & 7;
-    const long at = total * xcd / 8 + (blockIdx.x >> 3);
-    if (at >= total * (xcd + 1) / 8) return false;
-    part = (int)(at / tiles % g.ks);
-    slice = (int)(at / tiles / g.ks);
-    int tile = (int)(at % tiles);
+    // (the launcher keeps the total within an int; 64-bit divisions are a hundred instructions each)
+    const unsigned int tiles = g.tri ? g.mt * (g.mt + 1) / 2 : g.mt * g.nt, total = (unsigned int)g.n_slices * g.ks * tiles;
+    const unsigned int xcd = blockIdx.x & 7, lo = (total >> 3) * xcd + ((total & 7) * xcd >> 3);
+    const unsigned int hi = (total >> 3) * (xcd + 1) + ((total & 7) * (xcd + 1) >> 3), at = lo + (blockIdx.x >> 3);
+    if (at >= hi) return false;
+    const unsigned int whole = at / tiles;
+    int tile = (int)(at - whole * tiles);
+    slice = g.ks == 1 ? (int)whole : (int)(whole / (unsigned int)g.ks);
+    part = (int)whole - slice * g.ks;
     // A CU often gets the same tile of several slices: after a long row tile a short one (32 slices of [511 x 511] x [511 x
     // 256], row tiles of 2 to 16 stages: 38 -> 30 us).
-    if (g.causal_k && (slice & 1)) tile = tiles - 1 - tile;
+    if (g.causal_k && (slice & 1)) tile = (int)tiles - 1 - tile;
     if (g.tri) {  // lower triangle of square tiles, row by row
       ti = (int)((sqrtf(8.0f * (float)tile + 1.0f) - 1.0f) * 0.5f);
       while ((ti + 1) * (ti + 2) / 2 <= tile) ++ti;
