@@ -10,9 +10,9 @@ constexpr int SAMPLE_MAX_V = 8192;
 constexpr int SAMPLE_WAVE_V = 1024;  // up to here one wavefront keeps the whole row in its registers
 
 // Monotone map float -> uint32 (larger float = larger key), so the k-th largest value can be found
-// by a bitwise search over keys.
+// by a bitwise search over keys.  The two zeros are one value, as the comparison of :41-45 has them.
 __device__ __forceinline__ uint32_t order_key(float f) {
-  const uint32_t u = __float_as_uint(f);
+  const uint32_t u = __float_as_uint(f + 0.0f);
   return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 

@@ -150,6 +150,19 @@ def test_greedy_generation_from_the_checkpoint_follows_the_oracle(trained, corc)
     print(repr(text))
 
 
+@pytest.mark.parametrize("V", [256, 2000])
+def test_device_sampler_takes_both_zeros_as_one_value(trained, corc, V):
+    """The k-th largest value is +0.0: the entries with -0.0 are not below it and can be drawn."""
+    from burn_dragon_amd.generation import sample_from_logits
+
+    logits = np.full((4, V), -1.0, np.float32)
+    logits[:, 10:14] = 0.0
+    logits[:, 20:24] = -0.0
+    us = np.array([0.1, 0.4, 0.6, 0.9], np.float32)  # eight equal weights: 0.1 * 8, ... lie between two of them
+    got = sample_from_logits(trained[0], torch.from_numpy(logits).to(DEV), 1.0, 4, torch.from_numpy(us).to(DEV)).tolist()
+    assert got == [corc.sample_from_logits(row, 1.0, 4, float(u))[0] for row, u in zip(logits, us)] == [10, 13, 20, 23]
+
+
 def test_sampled_generation_streams_and_is_reproducible(trained):
     from burn_dragon_amd.generation import (ContextStrategy, GenerationConfig, GenerationSettings, generate_text,
                                             generate_tokens)
