@@ -23,12 +23,17 @@ __device__ __forceinline__ uint32_t order_key(float f) {
 template <typename I>
 __device__ __forceinline__ int weighted_index(float *w, const I *at, int n, int V, float u) {
   const int lane = threadIdx.x & 63;
-  // a chain over the list: 64 entries sit in the lanes' registers and are handed on by readlane, so the chain waits
-  // for one addition per entry and for no memory
+  // a chain over the list: 64 entries sit in the lanes' registers (zeros past the end, which change no sum) and are handed
+  // on by readlane, eight per turn from lanes that the instruction names, so the chain waits for one addition per entry,
+  // not for a lane's number, a branch or memory
   auto chain = [&](float start, float v, int lo) {
-    const int m = min(64, n - lo);
     float s = start;
-    for (int j = 0; j < m; ++j) s += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), j));
+#pragma unroll
+    for (int j = 0; j < 64; j += 8) {
+      if (lo + j >= n) break;  // uniform
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), j + e));
+    }
     return s;
   };
   float sum = 0.f;
@@ -61,10 +66,16 @@ __device__ __forceinline__ int weighted_index(float *w, const I *at, int n, int 
   float cum = 0.f;
   for (int lo = 0; lo < n; lo += 64) {
     const float p = lo + lane < n ? w[lo + lane] : 0.f;
-    const int m = min(64, n - lo);
-    for (int j = 0; j < m; ++j) {
-      cum += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(p), j));
-      if (cum > chosen) return min((int)at[lo + j], V - 1);
+#pragma unroll
+    for (int j = 0; j < 64; j += 8) {
+      if (lo + j >= n) break;  // uniform
+      int below = 0;  // the cumulative weights never fall, so those up to the variate come first
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        cum += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(p), j + e));
+        below += cum > chosen ? 0 : 1;
+      }
+      if (below < 8) return lo + j + below < n ? min((int)at[lo + j + below], V - 1) : V - 1;
     }
   }
   return V - 1;
@@ -73,7 +84,8 @@ __device__ __forceinline__ int weighted_index(float *w, const I *at, int n, int 
 // V <= R * 64: one wavefront per sequence, R values per lane, no barrier.  The k-th largest key is found a bit at a time
 // from ballots of register compares, the survivors are listed with ballot prefix counts, and the index-order sums run
 // over that list only.  Bound by the length of these chains, not by memory (V = 256, k = 40: 43 us for a workgroup
-// with the row in LDS, which paid two barriers per bit and three V-long chains of LDS reads in one lane; 7 us here).
+// with the row in LDS, which paid two barriers per bit and three V-long chains of LDS reads in one lane; 6.9 us with all 32
+// bits looked at and a turn of the chains per entry, 4.5 here).
 template <int R>
 __global__ __launch_bounds__(64) void k_sample_wave(const float *__restrict__ logits, long ld, int V, float temperature,
                                                     int top_k, const float *__restrict__ uniforms,
@@ -100,6 +112,7 @@ __global__ __launch_bounds__(64) void k_sample_wave(const float *__restrict__ lo
 #pragma unroll
       for (int r = 0; r < R; ++r) c += __popcll(__ballot(key[r] >= cand));
       if (c >= top_k) thr = cand;
+      if (c == top_k) break;  // no key between cand and the k-th largest: the same entries survive
     }
 #pragma unroll
     for (int r = 0; r < R; ++r)
