@@ -645,13 +645,50 @@ __global__ __launch_bounds__(1024) void k_phase_head(const float *__restrict__ c
   }
   __syncthreads();
   if (tid == 0) {
-    for (int w = 1; w < 16; ++w)
+    for (int w = 1; w * 64 < V; ++w)  // the waves that hold columns
       if (s_best[w] > best || (s_best[w] == best && s_arg[w] < arg)) {
         best = s_best[w];
         arg = s_arg[w];
       }
     next[b] = arg == 0x7fffffff ? 0 : arg;
   }
+}
+
+// The same without the greedy token, which is all that needs a sequence's logits in one place: a workgroup per 64 columns,
+// which redoes the second stage as phase A does.  Bound by its launch and one trip to memory (d = 256, V = 256, one sequence:
+// 3.5 us, 6.3 where one CU fetched all 256 KiB of lm_head).
+template <int DC, int NW>
+__global__ __launch_bounds__(NW * 64, 2) void k_phase_logits(const float *__restrict__ cur_in,
+                                                             const float *__restrict__ dec_partial, int G, int B, int d,
+                                                             const float *__restrict__ lm_head, int V,
+                                                             float *__restrict__ logits) {
+  using S = Shape<DC, NW, 64>;
+  __shared__ float4 s_part[S::NT];
+  __shared__ __align__(16) float s_cur[NW][DC];
+  __shared__ __align__(16) float s_acc[NW][64];
+  const int lane = threadIdx.x & 63, wave = wave_id(), b = blockIdx.y;
+  const int base = min((int)blockIdx.x * 64, V - 64);  // the last block may make some of its neighbour's columns again, alike
+
+  RowSum<DC, NW> partials;
+  partials.ask(dec_partial + (long)b * d, (long)B * d, G, d);
+  float cur[S::CJ];
+#pragma unroll
+  for (int j = 0; j < S::CJ; ++j) cur[j] = cur_in[(long)b * d + min(j * 64 + lane, d - 1)];
+  Project<DC, NW, 64> head;
+  head.ask(lm_head + base, d, V);
+  __builtin_amdgcn_sched_barrier(0);
+
+  float mlp[S::CJ];
+  partials.collect(G, s_part, mlp);
+  wave_layer_norm<S::CJ>(mlp, d);
+#pragma unroll
+  for (int j = 0; j < S::CJ; ++j) cur[j] = cur[j] + mlp[j];
+  wave_layer_norm<S::CJ>(cur, d);
+#pragma unroll
+  for (int j = 0; j < S::CJ; ++j) s_cur[wave][j * 64 + lane] = j * 64 + lane < d ? cur[j] : 0.0f;
+  wave_lds_order();
+  const float v = head.dot(s_cur[wave], d, s_acc);
+  if (wave == 0) logits[(long)b * V + base + lane] = v;
 }
 
 // The two launches of a layer.
@@ -815,6 +852,18 @@ int bdh_launch_phase_head(bdh_model *m, int B, const float *cur, const float *de
   bdh_ctx *ctx = m->ctx;
   const bdh_model_config &c = m->cfg;
   if (c.vocab > 1024 || c.n_embd > 512) return bdh_fail(ctx, BDH_E_SHAPE, "head kernel needs V <= 1024 and d <= 512");
+  // Without a greedy token 64 columns a workgroup: one CU need not fetch all of lm_head (3.5 us where one workgroup takes
+  // 6.3, V = 256).  Fewer columns than that leave a block's accesses beyond the row.
+  if (!next_tokens && c.vocab >= 64 && G <= 64 && B <= 65535) {
+    const dim3 grid((unsigned)((c.vocab + 63) / 64), (unsigned)B);
+#define BDH_LOGITS(DC_, NW_)                                                                                               \
+  hipLaunchKernelGGL((k_phase_logits<DC_, NW_>), grid, dim3(NW_ * 64), 0, ctx->stream, cur, dec_partial, G, B, c.n_embd,   \
+                     m->w.lm_head, c.vocab, logits)
+    if (c.n_embd <= 128) BDH_LOGITS(128, 4); else if (c.n_embd <= 256) BDH_LOGITS(256, 8); else BDH_LOGITS(512, 8);
+#undef BDH_LOGITS
+    BDH_LAUNCH_CHECK(ctx, "k_phase_logits");
+    return BDH_OK;
+  }
 #define BDH_HEAD(NC_)                                                                                                      \
   hipLaunchKernelGGL((k_phase_head<NC_>), dim3((unsigned)B), dim3(1024), 0, ctx->stream, cur, dec_partial, G, B, c.n_embd, \
                      m->w.lm_head, c.vocab, logits, next_tokens)

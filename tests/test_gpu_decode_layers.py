@@ -83,6 +83,41 @@ def test_two_launch_layer_edges(state, rotary, lazy, d, h, N, V, B, aligned):
         assert torch.equal(states[0].stamps, states[1].stamps)
 
 
+@pytest.mark.parametrize("d,h,N,V,B,aligned", [
+    (128, 4, 128, 64, 1, True),    # one block of 64 columns
+    (128, 4, 128, 69, 3, True),    # ... and one that starts within it
+    (132, 4, 64, 127, 2, True),
+    (256, 4, 128, 128, 2, True),
+    (256, 2, 1024, 1021, 2, False),  # 64 partial rows, weights four bytes off
+    (512, 4, 64, 1024, 3, True),
+    (256, 4, 128, 63, 1, True),    # too few columns: one workgroup
+])
+def test_logits_without_a_greedy_token(d, h, N, V, B, aligned):
+    """The logits of a step that wants no token, 64 columns a workgroup, against those of one that does: sums of at most 512
+    terms in another order, 1e-5."""
+    import burn_dragon_amd as bda
+
+    cfg = bda.BDHConfig(n_layer=2, n_embd=d, n_head=h, mlp_internal_dim_multiplier=1, vocab_size=V, dropout=0.0)
+    cfg.latent_per_head = lambda: N
+    g = torch.Generator(device=DEV).manual_seed(d + V)
+    w = {"embed": torch.randn((V, d), device=DEV, generator=g)}
+    for name, shape in (("encoder", (h, d, N)), ("encoder_v", (h, d, N)), ("decoder", (h * N, d)), ("lm_head", (d, V))):
+        w[name] = 0.05 * torch.randn(shape, device=DEV, generator=g)
+    if not aligned:
+        flat = torch.empty(d * V + 1, device=DEV)
+        flat[1:] = w["lm_head"].reshape(-1)
+        w["lm_head"] = flat[1:].view(d, V)
+    models = [bda.BDH(cfg, DEV, weights=w) for _ in range(2)]
+    states = [m.init_state() for m in models]
+    assert ("k_phase_logits" in _kernels_of_a_step(models[0], B)) == (V >= 64)
+    tokens = torch.randint(0, V, (2, B, 1), device=DEV, generator=g)
+    for t in range(2):
+        got = models[0].forward_with_state(tokens[t], states[0])
+        ref, _ = models[1].forward_with_state(tokens[t], states[1], want_next=True)
+        torch.cuda.synchronize()
+        assert rel_err(got, ref) < 1e-5, t
+
+
 @pytest.mark.parametrize("d,h,N,aligned", [
     (256, 4, 8192, True),   # 128 columns a workgroup, one for every CU of a chip of 256
     (256, 4, 8190, True),   # ... the last one not full, rows that are no whole 16-byte pieces
