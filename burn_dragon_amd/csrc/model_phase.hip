@@ -126,7 +126,7 @@ struct RowSum {
         t[i] = load_at<float4>(src, at + min(i * S::RG + rg, rows - 1) * step);
     }
   }
-  __device__ __forceinline__ void collect(int rows, float4 *s_part, float (&v)[S::CJ]) {
+  __device__ __forceinline__ void add(int rows, float4 *s_part) {  // this thread's part, [RG][DC]
     const int rg = threadIdx.x / (DC / 4);
     float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
@@ -137,7 +137,10 @@ struct RowSum {
       s.z += in ? t[i].z : 0.0f;
       s.w += in ? t[i].w : 0.0f;
     }
-    s_part[threadIdx.x] = s;  // [RG][DC]
+    s_part[threadIdx.x] = s;
+  }
+  __device__ __forceinline__ void collect(int rows, float4 *s_part, float (&v)[S::CJ]) {
+    add(rows, s_part);
     __syncthreads();
     const float *f = reinterpret_cast<const float *>(s_part) + (threadIdx.x & 63);
 #pragma unroll
@@ -525,105 +528,106 @@ __global__ __launch_bounds__(NW * 64, 2) void k_layer_phase_b(PhaseArgs a) {
 
 // ---- head -----------------------------------------------------------------------------------------------------
 // The last layer's pending second stage, then the logits and the greedy token (src/model/bdh.rs:436-449): one
-// workgroup of 16 waves per sequence.  logits[v] = sum_k cur[k] * lm_head[k][v]: a thread takes NC adjacent columns and one
-// of GK spans of k, in one fmaf chain per column whose first AHEAD rows are asked for before the LayerNorms (wave 0 makes
-// those); the spans are added in order; the lowest index wins ties.  What bounds it: one CU fetches all of lm_head, 64 bytes
-// a cycle.
-template <int NC>
+// workgroup of 16 waves per sequence.  logits[v] = sum_k cur[k] * lm_head[k][v]: a thread takes NC adjacent columns (the last
+// thread of a row may take some of its neighbour's again, alike) and one of GK spans of k, in one fmaf chain per column whose
+// first AHEAD rows are asked for before the LayerNorms (wave 0 makes those); the spans of a wave are added in its registers,
+// the others in order; the lowest index wins ties.  What bounds it: the launch, one trip to memory, and for the larger
+// vocabularies that one CU fetches all of lm_head, 64 bytes a cycle.  d = 128, V = 69, one sequence: 7.2 us with a column a
+// thread, half of the threads idle, rows worked on as 512 wide whatever d, and spans of k in whole waves; 5.1 here.
+template <int DC, int NC>
 __global__ __launch_bounds__(1024) void k_phase_head(const float *__restrict__ cur_in, const float *__restrict__ dec_partial,
                                                      int G, int B, int d, const float *__restrict__ lm_head, int V,
                                                      float *__restrict__ logits, int64_t *__restrict__ next) {
-  constexpr int AHEAD = 64 / NC;
-  typedef float Cols __attribute__((ext_vector_type(NC)));
-  __shared__ float s_cur[512];
+  using S = Shape<DC, 16, 64>;
+  constexpr int AHEAD = 16;
+  typedef float Cols __attribute__((ext_vector_type(NC), aligned(4)));
+  __shared__ float s_cur[DC];
   __shared__ float4 s_part[1024];
-  __shared__ __align__(16) float s_grp[1024 * NC];
+  __shared__ float s_grp[1024 * NC];
   __shared__ float s_best[16];
   __shared__ int s_arg[16];
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
   const int b = blockIdx.x;
-  // partial rows r0, r0 + 8, ... and four columns per thread (d <= 512)
-  const int r0 = tid >> 7, c4 = (tid & 127) * 4;
-  float4 t[8];
+  RowSum<DC, 16> partials;
+  partials.ask(dec_partial + (long)b * d, (long)B * d, G, d);
+  float cur[S::CJ];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    t[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (i == 0 || i * 8 < G)  // uniform
-      t[i] = *reinterpret_cast<const float4 *>(dec_partial + ((long)min(r0 + i * 8, G - 1) * B + b) * d + (c4 < d ? c4 : 0));
-  }
-  float cur[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) cur[j] = wave == 0 && j * 64 < d ? cur_in[(long)b * d + min(j * 64 + lane, d - 1)] : 0.0f;
+  for (int j = 0; j < S::CJ; ++j) cur[j] = wave == 0 ? cur_in[(long)b * d + min(j * 64 + lane, d - 1)] : 0.0f;
   const int per_row = (V + NC - 1) / NC;  // threads per row of lm_head
-  const int span = (per_row + 63) & ~63, GK = 1024 / span;
-  const int g = tid / span, c = (tid - g * span) * NC;
+  const int span = per_row <= 16 ? 16 : per_row <= 32 ? 32 : (per_row + 63) & ~63, GK = 1024 / span;
+  const int g = tid / span, c = min((tid - g * span) * NC, V - NC);
   const int per = (d + GK - 1) / GK;
-  const bool busy = g < GK && c < V;
+  const bool busy = g < GK && tid - g * span < per_row;
   const int k0 = min(d, g * per), k1 = busy ? min(d, k0 + per) : k0;
   const float *wp = lm_head + (busy ? c : 0);
   Cols wv[AHEAD];
 #pragma unroll
-  for (int u0 = 0; u0 < AHEAD; u0 += 16) {
+  for (int u0 = 0; u0 < AHEAD; u0 += 4) {
     if (u0 < per) {  // uniform
 #pragma unroll
-      for (int u = 0; u < 16; ++u) wv[u0 + u] = *reinterpret_cast<const Cols *>(wp + (long)min(k0 + u0 + u, d - 1) * V);
+      for (int u = 0; u < 4; ++u) wv[u0 + u] = *reinterpret_cast<const Cols *>(wp + (long)min(k0 + u0 + u, d - 1) * V);
     }
   }
   __builtin_amdgcn_sched_barrier(0);
 
-  float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+  partials.add(G, s_part);
+  __syncthreads();
+  if (tid < DC) {
+    const float *f = reinterpret_cast<const float *>(s_part) + tid;
+    float v = f[0];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const bool in = r0 + i * 8 < G;
-    sum.x += in ? t[i].x : 0.0f;
-    sum.y += in ? t[i].y : 0.0f;
-    sum.z += in ? t[i].z : 0.0f;
-    sum.w += in ? t[i].w : 0.0f;
+    for (int r = 1; r < S::RG; ++r) v += f[r * DC];
+    s_cur[tid] = v;
   }
-  s_part[tid] = sum;  // [8][512]
   __syncthreads();
   if (wave == 0) {
-    float mlp[8];
+    float mlp[S::CJ];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float *f = reinterpret_cast<const float *>(s_part) + j * 64 + lane;
-      mlp[j] = f[0];
+    for (int j = 0; j < S::CJ; ++j) mlp[j] = s_cur[j * 64 + lane];
+    wave_layer_norm<S::CJ>(mlp, d);
 #pragma unroll
-      for (int r = 1; r < 8; ++r) mlp[j] += f[r * 512];
-    }
-    wave_layer_norm<8>(mlp, d);
+    for (int j = 0; j < S::CJ; ++j) cur[j] = cur[j] + mlp[j];
+    wave_layer_norm<S::CJ>(cur, d);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) cur[j] = cur[j] + mlp[j];
-    wave_layer_norm<8>(cur, d);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) s_cur[j * 64 + lane] = cur[j];
+    for (int j = 0; j < S::CJ; ++j) s_cur[j * 64 + lane] = cur[j];
   }
   __syncthreads();
+  Cols acc = 0.0f;
   if (busy) {
-    Cols acc = 0.0f;
-    auto add16 = [&](int k, const Cols *w) {  // a row past the span counts as zero
+    auto add4 = [&](int k, const Cols *w) {  // a row past the span counts as zero
 #pragma unroll
-      for (int u = 0; u < 16; ++u) {
+      for (int u = 0; u < 4; ++u) {
         const bool in = k + u < k1;
         acc = __builtin_elementwise_fma(Cols(s_cur[in ? k + u : 0]), in ? w[u] : Cols(0.0f), acc);
       }
     };
 #pragma unroll
-    for (int u0 = 0; u0 < AHEAD; u0 += 16)
-      if (u0 < per) add16(k0 + u0, wv + u0);
+    for (int u0 = 0; u0 < AHEAD; u0 += 4)
+      if (u0 < per) add4(k0 + u0, wv + u0);
     for (int k = k0 + AHEAD; k < k0 + per; k += 16) {  // narrow vocabularies and long rows only
 #pragma unroll
       for (int u = 0; u < 16; ++u) wv[u] = *reinterpret_cast<const Cols *>(wp + (long)min(k + u, d - 1) * V);
-      add16(k, wv);
+#pragma unroll
+      for (int u = 0; u < 16; u += 4) add4(k + u, wv + u);
     }
-    *reinterpret_cast<Cols *>(&s_grp[g * span * NC + c]) = acc;
+  }
+  // the spans of one wave
+#pragma unroll
+  for (int e = 0; e < NC; ++e) {
+    if (span == 16) acc[e] = bdh_sum_over_rows(acc[e]);
+    else if (span == 32) acc[e] += __shfl_xor(acc[e], 32);
+  }
+  const int rows = min(GK, 16);
+  if (busy && (span >= 64 || lane < span)) {
+#pragma unroll
+    for (int e = 0; e < NC; ++e) s_grp[(span >= 64 ? g : wave) * span * NC + c + e] = acc[e];
   }
   __syncthreads();
   float best = -INFINITY;
   int arg = 0x7fffffff;
   if (tid < V) {
     float v = s_grp[tid];
-    for (int gg = 1; gg < GK; ++gg) v += s_grp[gg * span * NC + tid];
+    for (int r = 1; r < rows; ++r) v += s_grp[r * span * NC + tid];
     logits[(long)b * V + tid] = v;
     if (v > best) {
       best = v;
@@ -864,10 +868,15 @@ int bdh_launch_phase_head(bdh_model *m, int B, const float *cur, const float *de
     BDH_LAUNCH_CHECK(ctx, "k_phase_logits");
     return BDH_OK;
   }
-#define BDH_HEAD(NC_)                                                                                                      \
-  hipLaunchKernelGGL((k_phase_head<NC_>), dim3((unsigned)B), dim3(1024), 0, ctx->stream, cur, dec_partial, G, B, c.n_embd, \
-                     m->w.lm_head, c.vocab, logits, next_tokens)
-  if (c.vocab % 4 == 0 && bdh_aligned(m->w.lm_head, 16)) BDH_HEAD(4); else BDH_HEAD(1);
+#define BDH_HEAD(DC_, NC_)                                                                                                 \
+  hipLaunchKernelGGL((k_phase_head<DC_, NC_>), dim3((unsigned)B), dim3(1024), 0, ctx->stream, cur, dec_partial, G, B,      \
+                     c.n_embd, m->w.lm_head, c.vocab, logits, next_tokens)
+#define BDH_HEAD_OF(NC_)                                                                                                   \
+  do {                                                                                                                     \
+    if (c.n_embd <= 128) BDH_HEAD(128, NC_); else if (c.n_embd <= 256) BDH_HEAD(256, NC_); else BDH_HEAD(512, NC_);        \
+  } while (0)
+  if (c.vocab >= 4) BDH_HEAD_OF(4); else BDH_HEAD_OF(1);
+#undef BDH_HEAD_OF
 #undef BDH_HEAD
   BDH_LAUNCH_CHECK(ctx, "k_phase_head");
   return BDH_OK;

@@ -118,6 +118,35 @@ def test_logits_without_a_greedy_token(d, h, N, V, B, aligned):
         assert rel_err(got, ref) < 1e-5, t
 
 
+@pytest.mark.parametrize("d", [128, 200, 512])
+@pytest.mark.parametrize("V", [2, 3, 4, 61, 64, 65, 128, 129, 257])
+def test_greedy_head_of_few_and_ragged_columns(d, V):
+    """One column and four at a time, the last four of a row overlapping; spans of k added within a wave (up to 64 and 128
+    columns) and across waves: against the kernel-by-kernel step, sums of at most 512 terms in another order, 1e-5."""
+    import burn_dragon_amd as bda
+
+    cfg = bda.BDHConfig(n_layer=1, n_embd=d, n_head=2, mlp_internal_dim_multiplier=1, vocab_size=V, dropout=0.0)
+    cfg.latent_per_head = lambda: 64
+    g = torch.Generator(device=DEV).manual_seed(d + V)
+    w = {"embed": torch.randn((V, d), device=DEV, generator=g)}
+    for name, shape in (("encoder", (2, d, 64)), ("encoder_v", (2, d, 64)), ("decoder", (128, d)), ("lm_head", (d, V))):
+        w[name] = 0.05 * torch.randn(shape, device=DEV, generator=g)
+    models = [bda.BDH(cfg, DEV, weights=w) for _ in range(2)]
+    states = [m.init_state() for m in models]
+    ctx = bda.ffi.default_context(0)
+    tokens = torch.randint(0, V, (2, 3, 1), device=DEV, generator=g)
+    for t in range(2):
+        got, nxt = models[0].forward_with_state(tokens[t], states[0], want_next=True)
+        try:
+            ctx.set_option("model.one_launch", 0)
+            ref = models[1].forward_with_state(tokens[t], states[1])
+        finally:
+            ctx.set_option("model.one_launch", 1)
+        torch.cuda.synchronize()
+        assert rel_err(got, ref) < 1e-5, t
+        assert torch.equal(nxt.reshape(-1), got[:, 0].argmax(-1))
+
+
 @pytest.mark.parametrize("d,h,N,aligned", [
     (256, 4, 8192, True),   # 128 columns a workgroup, one for every CU of a chip of 256
     (256, 4, 8190, True),   # ... the last one not full, rows that are no whole 16-byte pieces
