@@ -13,6 +13,7 @@
 #include "tile_index.h"
 
 #include <algorithm>
+#include <cfloat>
 
 namespace {
 
@@ -196,6 +197,33 @@ struct RowPlaces {
     return (long)b * g.c_outer + (long)t * g.ldc;
   }
 };
+
+// What a gated projection stores for the sum v: a NaN counts as not above the threshold, as in every other projection.
+__device__ __forceinline__ float gated(const GemmF32 &g, float v, float gate) {
+  v -= g.threshold;
+  return gate * (v > 0.0f ? v : 0.0f);
+}
+
+// ROWS x COLS sums of A . B as one k-sequential fused multiply-add chain each, as the projections that have no split compute
+// them.  Where an operand is infinite, a NaN or rounds to an infinite bf16, or a sum leaves the floats, the terms' sum is no
+// number (inf - inf in a remainder, split3) and never a wrong finite one: a projection is then made again in this way.
+template <int ROWS, int COLS>
+__device__ __forceinline__ void chains(const float *const (&a)[ROWS], const float *const (&b)[COLS], int ldb, int K,
+                                       float (&s)[ROWS][COLS]) {
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+    for (int c = 0; c < COLS; ++c) s[r][c] = 0.0f;
+#pragma unroll 4
+  for (int k = 0; k < K; ++k)
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+      for (int c = 0; c < COLS; ++c) s[r][c] = __builtin_fmaf(a[r][k], b[c][(long)k * ldb], s[r][c]);
+}
+__device__ __forceinline__ const float *row_of_a(const GemmF32 &g, const float *A, int row) {
+  return A + (g.rows_per > 0 ? (long)(row / g.rows_per) * g.a_outer + (long)(row % g.rows_per) * g.lda : (long)row * g.lda);
+}
 
 // The ends of K for a tile of rows [m0, m0 + bm) and columns from n0 on: of A . B and of A2 . B2.
 __device__ __forceinline__ void ends_of_k(const GemmF32 &g, bool scores, int m0, int bm, int n0, int &K1, int &K2) {
@@ -457,8 +485,40 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_f32(GemmF32 g) {
       }
     return;
   }
-  if constexpr (EPI == GEMM_GATE) {  // the gates of a row of tiles are asked for before the first is used
+  if constexpr (EPI == GEMM_GATE) {
     const float *G = g.gate + s1 * g.c_s1 + s2 * g.c_s2;
+    auto col_of = [&](int j) { return n0 + wn * (BN / WN) + j * 32 + (lane & 31); };
+    float zero = 0.0f;  // ... while every sum of this lane is finite
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) zero = __builtin_fmaf(acc[i][j][e], 0.0f, zero);
+    if (__any(zero != 0.0f)) {  // rare: all of the wavefront's elements again, four rows at a time
+#pragma unroll 1
+      for (int q = 0; q < MI * 4; ++q) {
+        const int row0 = row_of(q >> 2, (q & 3) * 4);
+        const float *a[4], *b[NJ];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) a[r] = row_of_a(g, A, min(row0 + r, g.M - 1));
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) b[j] = B + min(col_of(j), g.N - 1);
+        float v[4][NJ];
+        chains<4, NJ>(a, b, g.ldb, g.K, v);
+        const int first = min(row0, g.M - 1);
+        const RowPlaces places(g, first);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) {
+            const long at = places.at(g, min(row0 + r, g.M - 1) - first) + col_of(j);
+            if (row0 + r < g.M && col_of(j) < g.N) C[at] = gated(g, v[r][j], G[at]);
+          }
+      }
+      return;
+    }
+    // the gates of a row of tiles are asked for before the first is used
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
       long at[16];
@@ -471,15 +531,13 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_f32(GemmF32 g) {
       for (int j = 0; j < NJ; ++j)
 #pragma unroll
         for (int e = 0; e < 16; ++e)
-          gate[j][e] = __builtin_nontemporal_load(G + at[e] + min(n0 + wn * (BN / WN) + j * 32 + (lane & 31), g.N - 1));
+          gate[j][e] = __builtin_nontemporal_load(G + at[e] + min(col_of(j), g.N - 1));
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
-        const int col = n0 + wn * (BN / WN) + j * 32 + (lane & 31);
+        const int col = col_of(j);
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const float v = acc[i][j][e] - g.threshold;
-          if (col < g.N && row_of(i, e) < g.M) __builtin_nontemporal_store(gate[j][e] * (v <= 0.0f ? 0.0f : v), C + at[e] + col);
-        }
+        for (int e = 0; e < 16; ++e)
+          if (col < g.N && row_of(i, e) < g.M) __builtin_nontemporal_store(gated(g, acc[i][j][e], gate[j][e]), C + at[e] + col);
       }
     }
     return;
@@ -527,6 +585,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f32_small(GemmF32 g) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 31, half = lane >> 5;
   const long s1 = slice / g.mod, s2 = slice % g.mod;
+  const float *A = g.A + s1 * g.a_s1 + s2 * g.a_s2;
+  const float *B = g.B + s1 * g.b_s1 + s2 * g.b_s2;
   float *C = g.C + s1 * g.c_s1 + s2 * g.c_s2;
   const float ld = (g.decay_rows || g.decay_state || g.decay_scores) ? g.log_decay[slice % g.heads] : 0.0f;
   int K1, K2;
@@ -534,12 +594,12 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f32_small(GemmF32 g) {
 
   f32x16 acc = (f32x16)(0.0f), low = (f32x16)(0.0f);  // the sums of h h, and of the five smaller terms
   float rs = 0.0f;
-  auto run = [&](const float *A, int lda, int rows_per, long a_outer, const float *B, int ldb, int K) {
+  auto run = [&](const float *src_a, int lda, int rows_per, long a_outer, const float *src_b, int ldb, int K) {
     const int ar = min(m0 + r, g.M - 1), bc = min(n0 + r, g.N - 1);  // past the end: the last one again, not stored
-    const float *pa = A + (AK ? (long)ar : rows_per > 0 ? (long)(ar / rows_per) * a_outer + (long)(ar % rows_per) * lda : (long)ar * lda);
-    const float *pb = B + (BK ? (long)bc : (long)bc * ldb);
-    const bool a_ok = (lda & 3) == 0 && (a_outer & 3) == 0 && (reinterpret_cast<uintptr_t>(A) & 15) == 0;
-    const bool b_ok = (ldb & 3) == 0 && (reinterpret_cast<uintptr_t>(B) & 15) == 0;
+    const float *pa = src_a + (AK ? (long)ar : rows_per > 0 ? (long)(ar / rows_per) * a_outer + (long)(ar % rows_per) * lda : (long)ar * lda);
+    const float *pb = src_b + (BK ? (long)bc : (long)bc * ldb);
+    const bool a_ok = (lda & 3) == 0 && (a_outer & 3) == 0 && (reinterpret_cast<uintptr_t>(src_a) & 15) == 0;
+    const bool b_ok = (ldb & 3) == 0 && (reinterpret_cast<uintptr_t>(src_b) & 15) == 0;
     float a[U][8], b[U][8];
     auto eight = [&](float(&v)[8], const float *p, bool kmajor, int ld_, bool whole_pieces, int k) {
       if (kmajor) {
@@ -599,7 +659,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f32_small(GemmF32 g) {
     acc += low;
     low = (f32x16)(0.0f);
   };
-  run(g.A + s1 * g.a_s1 + s2 * g.a_s2, g.lda, g.rows_per, g.a_outer, g.B + s1 * g.b_s1 + s2 * g.b_s2, g.ldb, K1);
+  run(A, g.lda, g.rows_per, g.a_outer, B, g.ldb, K1);
   if (EPI == GEMM_STORE && g.decay_rows) {
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[e] *= expf((float)(m0 + (e >> 2) * 8 + half * 4 + (e & 3)) * ld);
@@ -633,9 +693,14 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f32_small(GemmF32 g) {
       const int rr = row - m0;
       v = v / ((((s_norm[0][rr] + s_norm[1][rr]) + s_norm[2][rr]) + s_norm[3][rr]) + kRowNormEps);
     }
-    if (EPI == GEMM_GATE) {
-      v -= g.threshold;
-      v = G[at] * (v <= 0.0f ? 0.0f : v);
+    if constexpr (EPI == GEMM_GATE) {
+      if (!(fabsf(v) <= FLT_MAX)) {
+        const float *a[1] = {row_of_a(g, A, row)}, *b[1] = {B + col};
+        float again[1][1];
+        chains<1, 1>(a, b, g.ldb, g.K, again);
+        v = again[0][0];
+      }
+      v = gated(g, v, G[at]);
     }
     if (reads_c) v = (g.decay_state ? C[at] * keep : C[at]) + v;
     C[at] = v;

@@ -4,6 +4,8 @@ and several, unaligned sizes.
 
 Tolerances.  Split products: what is left out of a product of two f32 is below 2^-23 of it and the sums run over at most a
 few thousand terms in f32, so 2e-5 of the largest value (the bound of the other many-token tests).  Projections: bit for bit."""
+import re
+
 import numpy as np
 import pytest
 import torch
@@ -342,6 +344,52 @@ def test_gated_projection_of_a_prompt_on_split_products(d, h, N, B, T):
     for a, b in zip(*got):
         assert not torch.equal(a, b)
         assert float((a - b).abs().max() / a.abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize("d,h,N,B,T,tile", [
+    (36, 1, 131, 1, 100, "k_gemm_f32_small<"), (128, 2, 66, 3, 45, "k_gemm_f32_small<"),
+    (128, 2, 8192, 1, 100, "k_gemm_f32<64, 64"), (256, 4, 8192, 1, 200, "k_gemm_f32<128, 128"),
+    (768, 4, 8192, 1, 200, "k_gemm_f32<128, 256"),
+])
+@pytest.mark.parametrize("where,value", [("weight", float("nan")), ("weight", float("inf")), ("weight", -float("inf")),
+                                         ("weight", 3.4e38), ("weight", -3.4e38), ("weights", float("nan")),
+                                         ("embedding", float("nan")), ("embedding", float("inf"))])
+def test_gated_projection_of_numbers_that_no_split_holds(bda, d, h, N, B, T, tile, where, value):
+    """D_y of a prompt and of the stateless form with weights and inputs that are infinite, NaN or beyond the largest bf16: on
+    split products as in the f32 chain, where a NaN is not above the threshold and a finite weight keeps its value (what is a
+    number to the bound of the test above, in the same places)."""
+    cfg = bda.BDHConfig(n_layer=1, n_embd=d, n_head=h, mlp_internal_dim_multiplier=1, vocab_size=64, dropout=0.0)
+    cfg.latent_per_head = lambda: N
+    cfg.fused_kernels.set_rotary_embedding(bda.RotaryEmbedding.ROPE if N % 2 == 0 else bda.RotaryEmbedding.ALIBI)
+    g = torch.Generator(device=DEV).manual_seed(N)
+    normal = lambda *shape: 0.02 * torch.randn(shape, device=DEV, generator=g)
+    weights = {"embed": 50 * normal(64, d), "encoder": normal(h, d, N), "encoder_v": normal(h, d, N), "decoder": normal(h * N, d),
+               "lm_head": normal(d, 64)}
+    if where == "embedding":
+        weights["embed"][7, 3] = value
+    else:
+        weights["encoder_v"][0, 5, N - 2] = value
+        if where == "weights":
+            weights["encoder_v"][:, :, ::3] = value
+    model = bda.BDH(cfg, DEV, weights=weights)
+    tokens = torch.randint(8, 64, (B, T), device=DEV, generator=g)
+    tokens[0, T // 2] = 7
+    ctx = bda.ffi.default_context(0)
+    got = []
+    for split in (0, 1):
+        ctx.set_option("relu_lowrank.split", split)
+        try:
+            state = model.init_state()
+            logits, ran = _launched(lambda: model.forward_with_state(tokens, state))
+            got.append((logits, model.forward_fast(tokens), state.storage))
+        finally:
+            ctx.set_option("relu_lowrank.split", -1)
+        assert (re.search(tile + r"[^>]*\b3>", ran) is not None) == (split == 1), ran  # 3: the gated epilogue
+    for a, b in zip(*got):
+        assert torch.equal(torch.isfinite(a), torch.isfinite(b))
+        a, b = (torch.where(torch.isfinite(t), t, 0.0) for t in (a, b))
+        assert float((a - b).abs().max()) <= 1e-5 * float(a.abs().max())
+    assert bool(torch.isfinite(got[0][0][:, : T // 2]).all(-1).any())
 
 
 def _launched(call):
