@@ -388,7 +388,8 @@ constexpr int tile_lds_bytes(int TS) { return tile_stages(TS) * 2 * TS * BK * 2;
 // + 47 -> 65 + 56 + 45 us.
 // The workgroups behind the tiles (scores only: tr.blocks > 0) transpose what the later products read: they depend on nothing
 // here, and the scores seldom fill the chip to the end (the call above 174 -> 164).
-template <int TS, bool A_KMAJOR, bool SCORES>
+// WIDE: rows so wide that the offsets inside a tile take 64 bits (bdh_tile_offsets_fit).
+template <int TS, bool A_KMAJOR, bool SCORES, bool WIDE>
 __global__ __launch_bounds__(256, 2) void k_gemm_tile(GemmArgs g, TransposeArgs tr) {
   extern __shared__ __attribute__((aligned(1024))) unsigned short s_dyn[];
   if constexpr (SCORES) {
@@ -438,18 +439,27 @@ __global__ __launch_bounds__(256, 2) void k_gemm_tile(GemmArgs g, TransposeArgs 
     // Byte offsets of this thread's pieces from the first row (k row) of the tile; rows past the end repeat the last one, and
     // their sums are not stored.  Only the last step of a K that is no multiple of 64 looks at k: zeros beyond.
     const int kc = ((tid & 7) ^ ((tid >> 4) & 7)) * 8;  // this thread's k piece of a row-major panel
-    unsigned int pa[NP], pb[NP];
+    typedef std::conditional_t<WIDE, unsigned long, unsigned int> Offset;
+    auto offset = [](int row, int ld, int col) {
+      if constexpr (WIDE) return ((unsigned long)row * ld + col) * 2u;
+      else return bdh_tile_offset(row, ld, col);
+    };
+    auto copy = [](const unsigned short *base, Offset at, unsigned short *dst) {
+      if constexpr (WIDE) bdh_copy_to_lds(reinterpret_cast<const char *>(base) + at, dst);
+      else bdh_copy_to_lds(base, at, dst);
+    };
+    Offset pa[NP], pb[NP];
 #pragma unroll
     for (int c = 0; c < NP; ++c) {
       const int piece = c * 256 + tid, row = piece >> 3;
-      pb[c] = (unsigned int)(min(row, g.N - 1 - n0) * ldb + kc) * 2u;
+      pb[c] = offset(min(row, g.N - 1 - n0), ldb, kc);
       if (!A_KMAJOR) {
-        pa[c] = (unsigned int)(min(row, g.M - 1 - m0) * lda + kc) * 2u;
+        pa[c] = offset(min(row, g.M - 1 - m0), lda, kc);
       } else {
         const int kr = piece / (TS / 8);
         const int turn = TS == 128 ? (kr & 3) << 2 : ((kr >> 1) & 1) << 2;
         const int m = ((piece % (TS / 8)) ^ turn) * 8;
-        pa[c] = (unsigned int)(kr * lda + min(m, g.M - 8 - m0)) * 2u;  // M % 8 == 0
+        pa[c] = offset(kr, lda, min(m, g.M - 8 - m0));  // M % 8 == 0
       }
     }
     const unsigned short *a0 = A + (A_KMAJOR ? (long)m0 : (long)m0 * lda), *b0 = B + (long)n0 * ldb;
@@ -461,9 +471,9 @@ __global__ __launch_bounds__(256, 2) void k_gemm_tile(GemmArgs g, TransposeArgs 
       const unsigned short *as = a0 + (A_KMAJOR ? (long)k0 * lda : (long)k0), *bs = b0 + k0;
       if (k0 + BK <= K) {
 #pragma unroll
-        for (int c = c0; c < c1; ++c) bdh_copy_to_lds(as, pa[c], dst + c * 2048);
+        for (int c = c0; c < c1; ++c) copy(as, pa[c], dst + c * 2048);
 #pragma unroll
-        for (int c = c0; c < c1; ++c) bdh_copy_to_lds(bs, pb[c], dst + PANEL + c * 2048);
+        for (int c = c0; c < c1; ++c) copy(bs, pb[c], dst + PANEL + c * 2048);
       } else {
         const char *zero = reinterpret_cast<const char *>(&g_zero_piece);
 #pragma unroll
@@ -1539,17 +1549,19 @@ hipError_t launch_gemm_direct(hipStream_t st, const GemmArgs &g) {
   return hipSuccess;
 }
 
-// g.mt, g.nt and g.n_tiles are filled in here.
+// g.mt, g.nt and g.n_tiles are filled in here.  wide: with 64 wide tiles only.
 template <bool AK, bool SCORES>
-void launch_gemm_tile(hipStream_t st, GemmArgs g, int tile, const TransposeArgs &tr = TransposeArgs{}) {
+void launch_gemm_tile(hipStream_t st, GemmArgs g, int tile, bool wide, const TransposeArgs &tr = TransposeArgs{}) {
   g.mt = (g.M + tile - 1) / tile;
   g.nt = (g.N + tile - 1) / tile;
   g.n_tiles = g.tri ? g.mt * (g.mt + 1) / 2 : g.mt * g.nt;
   const unsigned grid = 8u * (unsigned)(((long)g.n_slices * g.n_tiles + 7) / 8) + (unsigned)tr.blocks;
-  if (tile == 128)
-    hipLaunchKernelGGL((k_gemm_tile<128, AK, SCORES>), dim3(grid), dim3(256), tile_lds_bytes(128), st, g, tr);
+  if (wide)
+    hipLaunchKernelGGL((k_gemm_tile<64, AK, SCORES, true>), dim3(grid), dim3(256), tile_lds_bytes(64), st, g, tr);
+  else if (tile == 128)
+    hipLaunchKernelGGL((k_gemm_tile<128, AK, SCORES, false>), dim3(grid), dim3(256), tile_lds_bytes(128), st, g, tr);
   else
-    hipLaunchKernelGGL((k_gemm_tile<64, AK, SCORES>), dim3(grid), dim3(256), tile_lds_bytes(64), st, g, tr);
+    hipLaunchKernelGGL((k_gemm_tile<64, AK, SCORES, false>), dim3(grid), dim3(256), tile_lds_bytes(64), st, g, tr);
 }
 
 // What a pass of the all-scores form does beyond the RoPE recurrence.
@@ -1582,7 +1594,8 @@ static int prefill_pass_scores(bdh_ctx *ctx, int B, int h, int T, int N, int d, 
   // (128 output tiles of 256) 762 with 256, 640 with 128; 8 slices of 2048 tokens 446 with 64, 327 with 128.
   const bool big = d % 256 == 0 && Nq % BK == 0 && S * tiles(T, 256) * (d / 256) >= full_chip &&
                    (tiles(T, 256) * 256 - T) * 8 <= T;
-  const int tile_t = big ? 256 : S * tiles(T, 128) * tiles(d, 128) >= full_chip ? 128 : 64;
+  const bool wide = !bdh_tile_offsets_fit(128, Nq);  // 16.9 M neurons: 64-bit offsets, in 64 wide tiles
+  const int tile_t = big ? 256 : !wide && S * tiles(T, 128) * tiles(d, 128) >= full_chip ? 128 : 64;
   // The state product of a fresh state is bound by what a tile reads and by its latency: 256 wide from a workgroup for every CU
   // on, unless the last round would be mostly empty (us a call, 256 | 128: 32 slices, N = 9856, d = 512, 200 tokens 403 | 474;
   // 64 slices, N = 9856, d = 384, 200 tokens 663 | 733; 16 slices, N = 4096, d = 256, 753 tokens 184 | 190; 4 slices of 9856
@@ -1591,11 +1604,11 @@ static int prefill_pass_scores(bdh_ctx *ctx, int B, int h, int T, int N, int d, 
   const long tiles_r = S * tiles(Nq, 256) * tiles(d, 256), rounds_r = (tiles_r + full_chip - 1) / full_chip;
   const bool wide_r = state_is_zero && d > 128 && tiles_r >= full_chip &&
                       (tiles_r >= 2 * full_chip || 4 * rounds_r * full_chip <= 5 * tiles_r);
-  const int tile_r = wide_r ? 256 : S * tiles(Nq, 128) * tiles(d, 128) >= full_chip ? 128 : 64;
+  const int tile_r = wide_r ? 256 : !wide && S * tiles(Nq, 128) * tiles(d, 128) >= full_chip ? 128 : 64;
   // The scores, of which there are more tiles, may have the larger one: 12 slices of 777 tokens, whose 168 output tiles
   // are 64 wide, 248 us a call with scores of 64, 238 with 128 (336 tiles).
   auto lower = [&](int tile) { return S * tiles(T, tile) * (tiles(T, tile) + 1) / 2; };
-  const int tile_s = !big && lower(128) >= full_chip ? 128 : tile_t;
+  const int tile_s = !big && !wide && lower(128) >= full_chip ? 128 : tile_t;
   const int mt = (int)tiles(T, tile_t), nt_d = (int)tiles(d, tile_t), mt_s = (int)tiles(T, tile_s);
   // a time block that straddles two score tiles has additive terms above the tile diagonal: all tiles then, and no causal
   // limit on the K of S V
@@ -1680,7 +1693,7 @@ static int prefill_pass_scores(bdh_ctx *ctx, int B, int h, int T, int N, int d, 
     g.tri = full_grid ? 0 : 1; g.mt = mt_s; g.nt = mt_s; g.n_tiles = n_score_tiles; g.n_slices = S;
     if (ext)
       with_mode(g, (pm.decay ? GM_DECAY_SCORES : 0) | (pm.add_alibi ? GM_ADD_ALIBI : 0) | (pm.row_norm ? GM_ROWNORM : 0));
-    if (!big) launch_gemm_tile<false, true>(ctx->stream, g, tile_s, t);
+    if (!big) launch_gemm_tile<false, true>(ctx->stream, g, tile_s, wide, t);
     else if (ext) BDH_HIP_CHECK(ctx, launch_gemm_direct<EPI_SCORES_X>(ctx->stream, g));
     else BDH_HIP_CHECK(ctx, launch_gemm_direct<EPI_SCORES>(ctx->stream, g));
     BDH_LAUNCH_CHECK(ctx, "scores");
@@ -1716,7 +1729,7 @@ static int prefill_pass_scores(bdh_ctx *ctx, int B, int h, int T, int N, int d, 
       qr.a2_batch = sv.a_batch; qr.b2_batch = sv.b_batch;
       qr.lda2 = sv.lda; qr.ldb2 = sv.ldb; qr.K2 = T; qr.b2_div = h;
     }
-    launch_gemm_tile<false, false>(ctx->stream, has_state ? qr : sv, tile_t);
+    launch_gemm_tile<false, false>(ctx->stream, has_state ? qr : sv, tile_t, wide);
   } else {
     if (has_state && pm.decay) BDH_HIP_CHECK(ctx, launch_gemm_direct<EPI_ACC_X>(ctx->stream, qr));
     else if (has_state) BDH_HIP_CHECK(ctx, launch_gemm_direct<EPI_ACC>(ctx->stream, qr));
@@ -1739,7 +1752,7 @@ static int prefill_pass_scores(bdh_ctx *ctx, int B, int h, int T, int N, int d, 
       const dim3 grid(8u * (unsigned)(((long)S * g.n_tiles + 7) / 8));
       hipLaunchKernelGGL(k_gemm_state, grid, dim3(512), 0, ctx->stream, g);
     } else {
-      launch_gemm_tile<true, false>(ctx->stream, g, tile_r);
+      launch_gemm_tile<true, false>(ctx->stream, g, tile_r, wide);
     }
     BDH_LAUNCH_CHECK(ctx, "Q^T V");
   }

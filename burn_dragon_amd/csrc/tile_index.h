@@ -25,3 +25,9 @@ BDH_HOST_DEVICE int bdh_kmajor_row(int r0, int lead, int c, int ch, int rows) {
 BDH_HOST_DEVICE int bdh_columns_of_piece(int c, int piece, int cols) {
   return c >= cols ? 0 : cols - c < piece ? cols - c : piece;
 }
+
+// Byte offset of the value at (row, col) of a tile from the tile's first value, in 32 bits: what a copy adds to a base that is
+// the same for a whole wavefront.  It holds while the last row of the tile lies less than 4 GiB behind the first one.
+BDH_HOST_DEVICE unsigned int bdh_tile_offset(int row, int ld, int col) { return ((unsigned int)row * (unsigned int)ld + (unsigned int)col) * 2u; }
+// ... which it does for bf16 rows of ld values in tiles of up to `tile` rows of `tile` columns.
+BDH_HOST_DEVICE bool bdh_tile_offsets_fit(int tile, int ld) { return ((long long)(tile - 1) * ld + tile) * 2 <= 0xffffffffLL; }

@@ -87,3 +87,29 @@ def test_row_normalised_attention_in_small_tiles(h, T, d, block):
     ref = torch.matmul(S, v.double().expand(B, h, T, d).contiguous()) / (S.abs().sum(-1, keepdim=True) + 1e-6)
     for s in range(h):  # every slice: one in the wrong order would be wrong alone
         assert float((out[:, s].double() - ref[:, s]).norm() / ref[:, s].norm()) < 1.8e-7
+
+
+@pytest.mark.parametrize("fresh", [False, True])
+def test_prefill_of_rows_of_more_than_four_gib_a_tile(fresh):
+    """34 M neurons, of which only the first and last few have activations: the bits of the call over those alone (every sum
+    runs over k in order, and a zero adds nothing), the other rows of the state as they were."""
+    from burn_dragon_amd.recurrent import prefill_chunked
+
+    T, N, d, few = 64, 34_209_792, 8, 1024
+    g = torch.Generator(device=DEV).manual_seed(3)
+    x = torch.zeros((1, 1, T, N), device=DEV, dtype=torch.bfloat16)
+    for part in (slice(0, few), slice(N - few, N)):
+        x[..., part] = torch.relu(torch.randn((1, 1, T, few), device=DEV, generator=g)).bfloat16()
+    v = torch.randn((1, T, d), device=DEV, generator=g).bfloat16()
+    rho = torch.zeros((1, 1, N, d), device=DEV) if fresh else 0.1 * torch.randn((1, 1, N, d), device=DEV, generator=g)
+    freqs = torch.rand(N, device=DEV, generator=g)
+
+    def ends(t, dim):
+        return torch.cat([t.narrow(dim, 0, few), t.narrow(dim, N - few, few)], dim).contiguous()
+
+    x_few, rho_few, freqs_few, between = ends(x, 3), ends(rho, 2), ends(freqs, 0), rho[:, :, few:N - few].clone()
+    out = prefill_chunked(x, v, rho, freqs, 5, state_is_zero=fresh)
+    out_few = prefill_chunked(x_few, v, rho_few, freqs_few, 5, state_is_zero=fresh)
+    assert torch.equal(out, out_few) and bool((out != 0).any())
+    assert torch.equal(ends(rho, 2), rho_few)
+    assert torch.equal(rho[:, :, few:N - few], between)

@@ -1,7 +1,8 @@
 // The rows that the threads of a k-major tile read (bdh_kmajor_row), for every width up to 640 and every tile: inside the
 // operand, aligned where a group is read at once, and the thread's own row wherever it has one.  And the columns that the
 // pieces of a 64 wide tile read (bdh_columns_of_piece): each column of a row once, none behind it, all of an aligned piece or
-// none of it where it is read at once.
+// none of it where it is read at once.  And the 32-bit offsets inside a bf16 tile (bdh_tile_offset): those of 64 bits wherever
+// bdh_tile_offsets_fit says so, which is up to the widest rows for which all of them are.
 #include <cstdio>
 #include <initializer_list>
 
@@ -39,6 +40,15 @@ int main() {
         }
       if (read != cols) return std::printf("cols %d: %d read in pieces of %d\n", cols, read, piece), 1;
       checked += cols;
+    }
+  for (int tile : {64, 128})
+    for (long long ld = 8; ld <= 0x7fffffff; ld += ld < 16000000 || (ld > 17000000 && ld < 33000000) || ld > 35000000 ? 999992 : 8) {
+      bool same = true;
+      for (int row : {0, 1, tile / 2 - 1, tile - 2, tile - 1})
+        for (int col : {0, 56, tile - 8})
+          same = same && bdh_tile_offset(row, (int)ld, col) == (unsigned long long)(row * ld + col) * 2;
+      if (bdh_tile_offsets_fit(tile, (int)ld) != same) return std::printf("tile %d rows of %lld: %d\n", tile, ld, same), 1;
+      ++checked;
     }
   std::printf("ok %ld\n", checked);
   return 0;
