@@ -763,10 +763,12 @@ double causal_share(const GemmF32 &g, int tile_rows) {
 // [500 x 8192] x [8192 x 256] in 5 parts: 161 us, in 128 x 128 tiles and 8 parts 185; with a K of 500, [8192 x 500] x [500 x 256],
 // 181 against 176; 32 slices of [511 x 511] x [511 x 256] 56 against 46).  More parts of K fill the
 // chip where the tiles are few, at the price of writing and re-reading every part.  A 32 x 32 tile (k_gemm_f32_small) has no
-// barriers: 750 a stage by itself, 500 where a CU has several.  Whole calls with it over calls without: prompts of 16 to 256
-// tokens through 4 heads of 128 to 256 neurons 0.69 to 0.87, 8 heads of 256, d = 512, 0.76 to 0.92, 4 heads of 1024, 256 tokens
-// 0.91; scoring 128 to 300 tokens 0.67 to 0.96; of 144 calls of 16 to 4088 tokens, up to 8192 neurons a head, four are 2 to 3 %
-// slower.
+// barriers: 750 a stage by itself, 500 where a CU has several, and half of what its last round leaves idle.  Whole calls with it
+// over calls without: prompts of 16 to 256 tokens through 4 heads of 128 to 256 neurons 0.69 to 0.87, 8 heads of 256, d = 512,
+// 0.76 to 0.92, 4 heads of 1024, 256 tokens 0.91; scoring 128 to 300 tokens 0.67 to 0.96; of 144 calls of 16 to 4088 tokens, up
+// to 8192 neurons a head, none is slower by more than its runs differ, up to 2 %.  (With the last round counted as it is filled, 4 slices of [800 x
+// 1024] x [1024 x 256], 3.1 rounds, took 28.0 us in 32 x 32 tiles where 64 x 64 tiles in two parts take 21.0 and 2.4 for their
+// sum; counted as a whole one, 16 slices of a prompt's readout, 2.6 rounds, left them, and the call went from 446 to 473.)
 GemmPlan bdh_gemm_f32_plan(const bdh_ctx *ctx, const GemmF32 &g, int max_split) {
   const double n_cu = ctx->n_cu > 0 ? ctx->n_cu : 256;
   constexpr double full[3] = {2600.0, 900.0, 900.0}, alone[3] = {3600.0, 2000.0, 2000.0};
@@ -786,7 +788,7 @@ GemmPlan bdh_gemm_f32_plan(const bdh_ctx *ctx, const GemmF32 &g, int max_split) 
       const double rounds = wgs <= 1.0 ? 1.0 : wgs;
       double cyc;
       if (t == 4) {
-        cyc = std::max(mean * rounds * 500.0, per * 750.0) + 3000.0;
+        cyc = std::max(mean * (rounds + std::ceil(rounds)) * 250.0, per * 750.0) + 3000.0;
       } else if (t == 3) {
         cyc = std::ceil(rounds) * (per * turn + turn_end);
       } else {

@@ -436,6 +436,20 @@ def test_products_of_few_tiles(bda, rotary, B, h, T, N, d):
         assert float((a - b).abs().max() / a.abs().max()) < 2e-5
 
 
+@pytest.mark.parametrize("B,T,small", [(4, 200, False), (1, 256, True)])
+def test_encoder_tiles_of_a_prompt_count_their_last_round(bda, B, T, small):
+    """The encoder of 800 rows and 4 heads of 1024 neurons: 32 x 32 tiles would be 3.1 rounds of workgroups, and slower than 64 x
+    64 tiles in parts; of 256 rows, one round, they are the faster ones."""
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("rounds of 256 CUs")
+    cfg = bda.BDHConfig(n_layer=1, n_embd=256, n_head=4, mlp_internal_dim_multiplier=16, vocab_size=64)
+    cfg.fused_kernels.set_rotary_embedding(bda.RotaryEmbedding.ROPE)
+    model = bda.BDH(cfg, DEV, seed=3)
+    tokens = torch.randint(0, 64, (B, T), generator=torch.Generator().manual_seed(T))
+    _, ran = _launched(lambda: model.forward_with_state(tokens, model.init_state()))
+    assert ("k_gemm_f32_small" in ran) == small
+
+
 @pytest.mark.parametrize("T,N,d,block", [(130, 48, 36, 1), (129, 20, 32, 64), (160, 64, 64, 32)])
 def test_row_norms_of_few_tiles(bda, T, N, d, block):
     """The stateless form on 32 x 32 tiles against its formula in float64: sums of up to 160 terms over their norm, 1e-5."""
