@@ -189,7 +189,7 @@ int bdh_launch_relu_lowrank_split(bdh_ctx *ctx, const ReluLowrankParams &p);
 int bdh_launch_relu_lowrank_gemm(bdh_ctx *ctx, const ReluLowrankParams &p, const unsigned char *mask_dev);
 // relu_lowrank for ONE input row per head whose values are made by the kernel itself from the partial sums an earlier
 // kernel left (a decode step of one sequence: the two reductions of a layer whose inputs come from other CUs ride in
-// front of the projection that consumes them, behind its first weight loads):
+// front of the projection that consumes them, while its weights are on their way):
 //   mode 1 (D_y, src/model/bdh.rs:359,370-381): row of head hh = LN(sum_g partial[hh][g][:]), g < S
 //   mode 2 (D_x of the next layer, :436-441 then :346-350): row = LN(cur_old + LN(sum_kb dpart[kb][:])), kb < KBN,
 //           shared by the heads; the workgroup (0, 0) also writes it to cur_new

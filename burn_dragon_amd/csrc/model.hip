@@ -265,7 +265,7 @@ int model_forward_impl(bdh_model *m, const int64_t *tokens, int B, int T, StateR
   // A decode step of ONE sequence through a RoPE model too large for the fused forms above: four
   // launches per layer instead of six.  The two reductions whose inputs come from other CUs -- the readout partials with
   // their LayerNorm, the encoder partials with the two LayerNorms and the residual -- are redone by every workgroup of the
-  // projection that consumes the result (D_y, the next layer's D_x), behind its first weight loads.
+  // projection that consumes the result (D_y, the next layer's D_x), while its weights are on their way.
   // Taken while what every workgroup adds up stays small against the weights it streams: at most 64 KiB of readout
   // partials per head (N/128 rows of d floats) and 128 KiB of encoder partials (h*N/KB rows); beyond that the redundant
   // sums cost more than the two launches they replace (measured at d=512, h=8, N=16384: 2.97 against 2.87 ms per token).

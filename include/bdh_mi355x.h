@@ -98,7 +98,8 @@ const char *bdh_last_error(const bdh_ctx *ctx);
  *                       the dense streaming kernel, 0 = the generic kernel (same values).
  *   "state_step.past_caches": -1 (default) the rows of a one-token step are loaded and stored with the streaming hint where
  *                       the states and weights that pass between two visits of a row exceed the last cache (256 MiB),
- *                       0 = never, 1 = always (same bits).
+ *                       0 = never, 1 = always (same bits).  Not the rows of a bf16 PoPE or eagerly decayed ALiBi state
+ *                       in the dense kernel, which gain nothing by it.
  *   "relu_lowrank.split": -1 (default) D_y of a prompt and of bdh_model_forward_fast (no by-products, no latent block mask)
  *                       runs as split-bf16 products (f32 accuracy, another order of the sums than the chain of the other
  *                       projections; sums that are infinite or NaN are made again as that chain) where 128 x 128 tiles
@@ -140,10 +141,12 @@ const char *bdh_last_error(const bdh_ctx *ctx);
  *                       model with n_embd in {256, 512} that is too large for the forms above takes four launches
  *                       per layer instead of six: D_y sums the state step's readout partials and applies their
  *                       LayerNorm itself, the next layer's D_x sums the encoder's partials and applies the two
- *                       LayerNorms and the residual (the first layer's D_x makes its row from the embedding), each
- *                       behind its first weight loads; taken while those sums stay small against the weights
+ *                       LayerNorms and the residual (the first layer's D_x makes its row from the embedding), while
+ *                       the weights are on their way; taken while those sums stay small against the weights
  *                       (N * n_embd <= 2 Mi and n_head * N * n_embd <= 32 Ki * fused_kb: BASELINE config 1 is the
- *                       largest such shape).  0 = kernel by kernel (values agree to 1e-5).
+ *                       largest such shape).  0 = kernel by kernel (values agree to 1e-5; in this form and those
+ *                       of model.one_launch D_x or the row that goes into it is added in another order, so a neuron
+ *                       whose pre-activation is within rounding of the threshold may fire in one form only).
  *   "model.fused_kb":   rows of E per workgroup of the encoder's first stage in that form (128 .. 2048, default 256).
  *   "model.phase_batch": the two-launch layer only for at most this many sequences (default: no limit
  *                       beyond the one above; 0 = never).

@@ -327,6 +327,51 @@ def test_two_launch_layer_norms_of_rows_whose_variance_is_no_float(huge, d, h, N
     assert rel_err(after[0], after[1]) < 1e-5
 
 
+@pytest.mark.parametrize("form", ["model.one_launch", "model.fused_rows"])
+@pytest.mark.parametrize("d,h,N", [(256, 4, 2048), (512, 4, 4096)])
+def test_neurons_that_fire_in_one_form_of_a_decode_step_only_are_at_the_threshold(form, d, h, N):
+    """The fused forms add D_x, and the sums behind its input row, in other orders than the kernels one by one.  Whether a neuron
+    fires may differ only where its pre-activation p, here in float64, is within what rounding does to it: (d + 64) 2^-24
+    sum |row w| for the chain of d terms and the LayerNorm of its row, and 1e-5 |row| |w|, by which the rows of two forms may
+    differ, behind a layer.  Seen from the state: at position 0 a row of it that was zero is x v."""
+    import burn_dragon_amd as bda
+
+    N = 64 * 64 // h if form == "model.one_launch" else N  # ... which takes the two-launch layer up to 64 blocks of 64 neurons
+    model = _model_of(d, h, N, layers=2)
+    w = {k: t.double() for k, t in model.params.items()}
+    g = torch.Generator(device=DEV).manual_seed(N)
+    start = torch.zeros((2, 1, h, N, d), device=DEV)
+    start[0, ..., : d // 2] = 0.1 * torch.randn((h, N, d // 2), device=DEV, generator=g)  # the other half shows what fired
+    ctx, fired, ran = bda.ffi.default_context(0), [], []
+    norm = lambda r: torch.nn.functional.layer_norm(r, (d,), eps=1e-5)
+    for on in (1, 0):
+        ctx.set_option(form, on)
+        try:
+            state = model.init_state()
+            state.position, state.storage = 0, start.clone()
+            for i, layer in enumerate(state.layers):
+                layer.rho = state.storage[i]
+            model.forward_with_state(torch.tensor([[5]], device=DEV), state)
+            ran.append(_kernels_of_a_step(model, 1))
+        finally:
+            ctx.set_option(form, 1)
+        fired.append((state.storage[:, 0, ..., d // 2:] != 0).any(-1))
+    assert ran[0] != ran[1]
+    row = norm(w["embed"][5])
+    for l in range(2):
+        p = torch.einsum("k,hkn->hn", row, w["encoder"])
+        bound = (d + 64) * 2.0 ** -24 * torch.einsum("k,hkn->hn", row.abs(), w["encoder"].abs())
+        if l:
+            bound += 1e-5 * row.norm() * w["encoder"].norm(dim=1)
+        for f in fired:
+            assert bool(((f[l] == (p > 0)) | (p.abs() <= bound)).all()), l
+        assert float((p.abs() <= bound).double().mean()) < 0.01 and 0.3 < float(fired[0][l].double().mean()) < 0.7
+        x = p.clamp_min(0)
+        attn = torch.einsum("hn,hnd->hd", x, start[l, 0].double())
+        y = torch.einsum("hk,hkn->hn", norm(attn), w["encoder_v"]).clamp_min(0)
+        row = norm(row + norm(torch.einsum("n,nd->d", (x * y).reshape(-1), w["decoder"])))
+
+
 def _model_of(d, h, N, layers=1, rotary="rope", dtype="f32", lazy=False, vocab=64):
     import burn_dragon_amd as bda
     from burn_dragon_amd import ffi
