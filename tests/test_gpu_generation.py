@@ -166,24 +166,31 @@ def test_device_sampler_takes_both_zeros_as_one_value(trained, corc, V):
 @pytest.mark.parametrize("top_k", [1, 7, 8, 9, 63, 64, 65, 128, None])
 def test_device_sampler_in_turns_of_eight(trained, corc, top_k):
     """Lists of survivors that end in and at the end of a turn of eight and of 64, with and without ties at the k-th largest
-    value (the search for it ends early only without); variates at both ends.  The index is exact for every draw that is no
-    closer than 1e-5 (some tens of roundings of expf and of the running sums) to a boundary of the cumulative weights."""
+    value (the search for it ends early only without); variates at both ends, and a last survivor that has most of the weight.
+    The index is exact for every draw that is no closer than 1e-5 (some tens of roundings of expf and of the running sums) to
+    the boundary between two survivors; that is every one of these."""
     from burn_dragon_amd.generation import sample_from_logits
 
     model = trained[0]
     rng = np.random.default_rng(top_k or 0)
     V = 256
-    logits = rng.standard_normal((12, V)).astype(np.float32)
-    logits[6:] = np.round(logits[6:] * 2) / 2  # ties
-    us = np.concatenate([rng.random(10), [0.0, 0.99999994]]).astype(np.float32)
+    logits = rng.standard_normal((16, V)).astype(np.float32)
+    logits[6:12] = np.round(logits[6:12] * 2) / 2  # ties
+    logits[12:, 250] = 9.0  # nearly all of the weight, behind every other survivor
+    logits[12:, 251:] = -200.0
+    us = np.concatenate([rng.random(10), [0.0, 0.99999994, 0.0, 0.5, 0.9, 0.99999994]]).astype(np.float32)
     us[5] = 0.99999994
     got = sample_from_logits(model, torch.from_numpy(logits).to(DEV), 0.8, top_k, torch.from_numpy(us).to(DEV)).cpu().numpy()
-    for b in range(12):
+    for b in range(16):
         want, p = corc.sample_from_logits(logits[b], 0.8, top_k, float(us[b]))
-        cum = np.cumsum(p.astype(np.float64))
-        if np.abs(cum - us[b] * cum[-1]).min() < 1e-5:
-            assert p[got[b]] > 0
-            continue
+        survivors = np.flatnonzero(p)
+        cum = np.cumsum(p[survivors].astype(np.float64))
+        boundaries = cum[:-1]  # none before the first survivor, none behind the last
+        assert us[b] == 0.0 or np.abs(boundaries - us[b] * cum[-1]).min(initial=1.0) > 1e-5, b
+        if us[b] == 0.0:
+            assert want == survivors[0]
+        if b == 15:
+            assert want == survivors[-1] == 250
         assert got[b] == want, b
 
 

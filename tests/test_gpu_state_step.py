@@ -6,6 +6,8 @@ the f32 checks here are much tighter (the only differences are the device sincos
 the summation order of the readout).  Index artefacts (active bitmask, touched-row counts) are
 bit-exact.  Untouched state rows must be bit-identical.
 """
+import re
+
 import numpy as np
 import pytest
 import torch
@@ -649,7 +651,7 @@ def test_dense_streaming_kernel_equals_generic_kernel_and_oracle(gpu, corc, rota
 @pytest.mark.parametrize("B,h,N,d", [(1, 2, 130, 256), (300, 4, 254, 256), (2, 2, 514, 512), (2, 3, 66, 192), (3, 1, 40, 36)])
 def test_rows_past_the_caches_keep_their_bits(gpu, rotary, lazy, B, h, N, d, dtype):
     """The streaming hint changes where a row is kept, never what it holds: every kernel of a one-token step with it and
-    without it, two steps one after the other on the same state."""
+    without it, two steps one after the other on the same state.  The dense kernel has no such form for bf16 rows."""
     ffi, recurrent_attention = gpu
     from burn_dragon_amd.positional import RotaryEmbedding
     from burn_dragon_amd.recurrent import recurrent_attention_lazy_alibi
@@ -660,16 +662,25 @@ def test_rows_past_the_caches_keep_their_bits(gpu, rotary, lazy, B, h, N, d, dty
     v = torch.randn((2, B, 1, d), device=dev, generator=g)
     rho0 = torch.randn((B, h, 2 * N if rotary == orc.POPE else N, d), device=dev, generator=g).to(dtype)
     freqs = 0.1 * torch.rand(N, device=dev, generator=g)
-    got = []
+    got, ran = [], []
     for mode in (0, 1):
         rho, stamps = rho0.clone(), torch.zeros((B, h, N), dtype=torch.int32, device=dev)
         ctx.set_option("state_step.past_caches", mode)
         try:
-            outs = [recurrent_attention_lazy_alibi(x[t], v[t], rho, stamps, 3 + t) if lazy else
-                    recurrent_attention(x[t], v[t], rho, freqs, 3 + t, RotaryEmbedding(rotary)) for t in range(2)]
-            torch.cuda.synchronize()
+            with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+                outs = [recurrent_attention_lazy_alibi(x[t], v[t], rho, stamps, 3 + t) if lazy else
+                        recurrent_attention(x[t], v[t], rho, freqs, 3 + t, RotaryEmbedding(rotary)) for t in range(2)]
+                torch.cuda.synchronize()
         finally:
             ctx.set_option("state_step.past_caches", -1)
         got.append((*outs, rho, stamps))
+        names = [e.key for e in prof.key_averages()]
+        steps = [n[n.index("k_step_"):] for n in names if "k_step_" in n and "k_step_finalize" not in n]
+        assert len(steps) == 1, names
+        ran.append(steps[0])
+    dense_bf16 = dtype == torch.bfloat16 and d in (256, 512) and rotary != orc.ROPE and not lazy
+    assert ("k_step_dense" in ran[0]) == (d in (256, 512) and rotary != orc.ROPE and not lazy)
+    assert re.search(r"\bfalse>", ran[0]) and bool(re.search(r"\btrue>", ran[1])) == (not dense_bf16), ran  # NT, the last argument
+    assert (ran[0] == ran[1]) == dense_bf16
     assert all(torch.equal(a, b) for a, b in zip(*got))
     assert not torch.equal(got[0][2], rho0)
