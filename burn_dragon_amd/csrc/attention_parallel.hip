@@ -1001,7 +1001,7 @@ int bdh_launch_decoder_partials_f32(bdh_ctx *ctx, int B, int T, int h, int N, in
 }
 
 // D_y of a prompt: gate * relu(in . W - thr) as split-bf16 products, a slice per head.
-int bdh_launch_relu_lowrank_split(bdh_ctx *ctx, const ReluLowrankParams &p) {
+static GemmF32 gated_product(const ReluLowrankParams &p) {
   GemmF32 g;
   g.epilogue = GEMM_GATE;
   g.A = p.in; g.B = p.weight; g.C = p.out; g.gate = p.gate;
@@ -1011,6 +1011,37 @@ int bdh_launch_relu_lowrank_split(bdh_ctx *ctx, const ReluLowrankParams &p) {
   g.n_slices = g.mod = p.h;
   g.a_s2 = p.h_in == 1 ? 0 : (long)p.T * p.d; g.b_s2 = (long)p.d * p.N; g.c_s2 = (long)p.T * p.N;
   g.rows_per = p.T; g.a_outer = (long)p.h_in * p.T * p.d; g.c_outer = (long)p.h * p.T * p.N;
+  return g;
+}
+
+// Whether they are faster than the f32 chain.  From three 128 x 128 tiles for every two CUs on (us a prompt, 4 layers, chain | split:
+// 4 x 8192 neurons, d = 256, 200 rows 1083 | 1042, 1500 rows 4969 | 4739; 8 x 256, d = 512, 1500 rows (192 tiles) 1041 | 1030,
+// 4088 rows 2281 | 2184; 4 x 256, d = 256, 4088 rows (256 tiles) 843 | 850; 4 x 2048, d = 128, 4088 rows 2620 | 2540), but
+//  - few rows are bound by the weights, which the 16 and 32 row tiles of the chain stream (us, chain | split: 4 x 12288, d = 128, 1
+//    row 5.8 | 11.3, 16 rows 7.8 | 11.8, 32 rows 11.7 | 12.3, 33 rows 17.3 | 13.4; d = 384, 16 rows 14.2 | 21.9, 32 rows 20.2 | 22.2,
+//    33 rows 31.9 | 25.9; 4 x 16384, d = 256, 16 rows 14.2 | 17.8, 17 rows 19.1 | 17.7, 32 rows 20.5 | 18.3; 4 x 12288, d = 64,
+//    32 rows 9.1 | 14.8; without 16-byte pieces, d = 260, 4 x 12289, 8 rows 24.3 | 25.5, 16 rows 29.5 | 25.7);
+//  - rows that end in the first half of a 128 row tile have less padding in the chain's 64 x 64 tiles.  Those take 1.3 us and 0.73
+//    for every 32 of K, a CU one after the other; two 128 x 128 tiles on a CU 12.4 and 2.95, one by itself 8.8 and 2.2 (us, 129 | 193
+//    rows: 4 x 12288, d = 128 chain 38 | 51, split 42 | 43; 4 x 8192, d = 128 27 | 34, 25 | 26; 257 rows: 4 x 6144, d = 192 44.2, 46.6).
+bool bdh_relu_lowrank_split_pays(const bdh_ctx *ctx, const ReluLowrankParams &p) {
+  const long n_cu = ctx->n_cu > 0 ? ctx->n_cu : 256, M = (long)p.B * p.T;
+  auto tiles = [&](int side) { return p.h * ((M + side - 1) / side) * ((p.N + side - 1) / side); };
+  const long big = tiles(128);
+  if (2 * big < 3 * n_cu) return false;
+  const bool pieces = p.d % 32 == 0 && p.N % 4 == 0 && bdh_aligned(p.in, 16) && bdh_aligned(p.weight, 16);
+  if (M <= (pieces ? 16 : 8)) return false;
+  if (!pieces) return true;
+  if (M <= 32) return p.d >= 128 && big >= 2 * n_cu;
+  if (big >= 4 * n_cu || bdh_gemm_f32_rows(bdh_gemm_f32_plan(ctx, gated_product(p), 1)) != 128) return true;
+  const double stages = p.d / 32, per_cu = (double)tiles(64) / n_cu;
+  const long rest = big % (2 * n_cu);
+  const double two = 12.4 + 2.95 * stages, one = 8.8 + 2.2 * stages;
+  return big / (2 * n_cu) * two + (rest > n_cu ? two : rest > 0 ? one : 0.0) <= per_cu * (1.3 + 0.73 * stages);
+}
+
+int bdh_launch_relu_lowrank_split(bdh_ctx *ctx, const ReluLowrankParams &p) {
+  const GemmF32 g = gated_product(p);
   return bdh_launch_gemm_f32(ctx, g, false, true, bdh_gemm_f32_plan(ctx, g, 1), nullptr);
 }
 

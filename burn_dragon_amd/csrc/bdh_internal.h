@@ -184,7 +184,9 @@ struct ReluLowrankParams {
   bool any_order = false;  // the caller does not need the bits of the k-sequential chain (gated calls only)
 };
 int bdh_launch_relu_lowrank(bdh_ctx *ctx, const ReluLowrankParams &p);
+// a gated call in any order as split-bf16 products, and whether that is the faster form; csrc/attention_parallel.hip
 int bdh_launch_relu_lowrank_split(bdh_ctx *ctx, const ReluLowrankParams &p);
+bool bdh_relu_lowrank_split_pays(const bdh_ctx *ctx, const ReluLowrankParams &p);
 // the same on the f32 matrix cores for many rows per (sequence, head); csrc/attention_parallel.hip
 int bdh_launch_relu_lowrank_gemm(bdh_ctx *ctx, const ReluLowrankParams &p, const unsigned char *mask_dev);
 // relu_lowrank for ONE input row per head whose values are made by the kernel itself from the partial sums an earlier

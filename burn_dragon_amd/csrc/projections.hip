@@ -1153,15 +1153,10 @@ int bdh_launch_relu_lowrank(bdh_ctx *ctx, const ReluLowrankParams &p) {
     }
     mask_dev = static_cast<const unsigned char *>(ctx->lat_mask);
   }
-  // D_y of a prompt has no order to keep (it decides no active set): split-bf16 products where their 128 x 128 tiles are three
-  // for every two CUs.  (us a prompt, 4 layers, chain | split: 4 x 8192 neurons, d = 256, 200 rows 1083 | 1042, 1500 rows 4969 | 4739;
-  // 8 x 256, d = 512, 1500 rows (192 tiles) 1041 | 1030, 4088 rows 2281 | 2184; 4 x 256, d = 256, 4088 rows (256 tiles) 843 | 850;
-  // 4 x 2048, d = 128, 4088 rows 2620 | 2540.  One such product, 1500 rows, 4 x 8192 neurons, d = 256: 274 | 217.)
-  if (p.any_order && p.gate && !p.bias && !mask_dev && p.d > 0 && p.N > 0 && ctx->opt_lowrank_split != 0) {
-    const long n_cu_split = ctx->n_cu > 0 ? ctx->n_cu : 256;
-    if (ctx->opt_lowrank_split == 1 || 2 * p.h * ((M + 127) / 128) * ((p.N + 127) / 128) >= 3 * n_cu_split)
-      return bdh_launch_relu_lowrank_split(ctx, p);
-  }
+  // D_y of a prompt has no order to keep (it decides no active set): split-bf16 products where those are faster
+  if (p.any_order && p.gate && !p.bias && !mask_dev && p.d > 0 && p.N > 0 && ctx->opt_lowrank_split != 0 &&
+      (ctx->opt_lowrank_split == 1 || bdh_relu_lowrank_split_pays(ctx, p)))
+    return bdh_launch_relu_lowrank_split(ctx, p);
   const bool pieces = p.d % 32 == 0 && p.N % 4 == 0 && bdh_aligned(p.in, 16) && bdh_aligned(p.weight, 16);
   // A matrix of up to 16 MiB (it sits in the L2) and few outputs: 64 columns per workgroup, every weight in flight at once,
   // as many rows per workgroup (1, 2, 4, 8) as still give a workgroup per CU.  The line is at 32768 outputs, 128 for every

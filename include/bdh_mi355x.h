@@ -102,8 +102,8 @@ const char *bdh_last_error(const bdh_ctx *ctx);
  *                       in the dense kernel, which gain nothing by it.
  *   "relu_lowrank.split": -1 (default) D_y of a prompt and of bdh_model_forward_fast (no by-products, no latent block mask)
  *                       runs as split-bf16 products (f32 accuracy, another order of the sums than the chain of the other
- *                       projections; sums that are infinite or NaN are made again as that chain) where 128 x 128 tiles
- *                       fill the chip, 0 = never, 1 = always.
+ *                       projections; sums that are infinite or NaN are made again as that chain) where those are faster:
+ *                       more than 16 or 32 rows and enough tiles for the chip, 0 = never, 1 = always.
  *   "relu_lowrank.mfma_rows": 2 (default) calls with this many rows and fewer than 64 (N a multiple of 4, d a multiple
  *                       of 32) that the row kernel below does not take run on the f32 matrix cores, the weights
  *                       streamed once per tile of 16 to 64 rows: a chain of v_mfma_f32_16x16x4_f32 over k is the same

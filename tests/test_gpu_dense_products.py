@@ -401,6 +401,24 @@ def _launched(call):
     return out, " ".join(e.key for e in prof.key_averages())
 
 
+@pytest.mark.parametrize("d,h,N,T,split", [
+    (128, 4, 12288, 1, False), (128, 4, 12288, 32, False), (128, 4, 12288, 33, True),    # few rows: the weights bound them
+    (256, 4, 16384, 16, False), (256, 4, 16384, 17, True), (260, 4, 12289, 8, False), (260, 4, 12289, 9, True),
+    (128, 4, 12288, 129, False), (128, 4, 12288, 193, True), (128, 4, 8192, 129, True),  # padding to whole tiles
+    (192, 4, 6144, 257, False), (192, 4, 6144, 385, True), (192, 4, 12288, 257, True),
+])
+def test_where_the_gated_projection_takes_split_products(bda, d, h, N, T, split):
+    """The rows from which on split products are faster than the f32 chain."""
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("rounds of 256 CUs")
+    cfg = bda.BDHConfig(n_layer=1, n_embd=d, n_head=h, mlp_internal_dim_multiplier=1, vocab_size=64)
+    cfg.latent_per_head = lambda: N
+    cfg.fused_kernels.set_rotary_embedding(bda.RotaryEmbedding.ALIBI)
+    model = bda.BDH(cfg, DEV, seed=3)
+    _, ran = _launched(lambda: model.forward_fast(torch.zeros((1, T), device=DEV, dtype=torch.int64)))
+    assert (re.search(r"k_gemm_f32(_small)?<[^>]*\b3>", ran) is not None) == split, ran
+
+
 @pytest.mark.parametrize("rotary", ["rope", "alibi", "pope"])
 @pytest.mark.parametrize("B,h,T,N,d", [
     (1, 2, 8, 16, 32),     # one step of k for one of the four wavefronts, tiles that end inside
