@@ -495,7 +495,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_f32(GemmF32 g) {
       for (int j = 0; j < NJ; ++j)
 #pragma unroll
         for (int e = 0; e < 16; ++e) zero = __builtin_fmaf(acc[i][j][e], 0.0f, zero);
-    if (__any(zero != 0.0f)) {  // rare: all of the wavefront's elements again, four rows at a time
+    if (__any(zero != 0.0f)) {  // rare: all of the wavefront's elements again, eight rows at a time
 #pragma unroll 1
       for (int q = 0; q < MI * 4; ++q) {
         const int row0 = row_of(q >> 2, (q & 3) * 4);
@@ -504,8 +504,25 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_f32(GemmF32 g) {
         for (int r = 0; r < 4; ++r) a[r] = row_of_a(g, A, min(row0 + r, g.M - 1));
 #pragma unroll
         for (int j = 0; j < NJ; ++j) b[j] = B + min(col_of(j), g.N - 1);
+        // A row that holds a NaN has sums that are NaN, whatever the weights.  Lanes 0 to 31 have rows row0 + r, the others rows
+        // four further on: each half looks through its own.
+        bool chain = false;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          bool nan = false;
+          for (int k = lane & 31; k < g.K; k += 32) nan |= a[r][k] != a[r][k];
+          const unsigned long long found = __ballot(nan);
+          chain |= (found & 0xffffffffull) == 0 || (found >> 32) == 0;
+        }
         float v[4][NJ];
-        chains<4, NJ>(a, b, g.ldb, g.K, v);
+        if (chain) {
+          chains<4, NJ>(a, b, g.ldb, g.K, v);
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) v[r][j] = NAN;
+        }
         const int first = min(row0, g.M - 1);
         const RowPlaces places(g, first);
 #pragma unroll
