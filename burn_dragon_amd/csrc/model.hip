@@ -262,7 +262,7 @@ int model_forward_impl(bdh_model *m, const int64_t *tokens, int B, int T, StateR
     }
   }
 
-  // A decode step of ONE sequence through a RoPE model too large for the fused forms above: four
+  // A decode step of ONE sequence through a RoPE model too large for the fused forms above (4 heads of 8192, d = 256): four
   // launches per layer instead of six.  The two reductions whose inputs come from other CUs -- the readout partials with
   // their LayerNorm, the encoder partials with the two LayerNorms and the residual -- are redone by every workgroup of the
   // projection that consumes the result (D_y, the next layer's D_x), while its weights are on their way.

@@ -1100,7 +1100,9 @@ static int dense_form_from(const StateStepParams &p, bool fast) {
 // it is read again and has driven out weights (and, written, waits its turn to be written back while the next kernel reads):
 // decode steps by kernels, cached | past them: 12 layers of 16384 neurons a head, 8 sequences, d = 512, 24 GiB of state 9950 us
 // | 9490; 6 of 8192, d = 256, 2 to 16 sequences, a twentieth to half of the neurons firing 0.959 to 1.002 of the time; eager ALiBi
-// and PoPE, 0.6 to 1.6 GB, d = 192 and 512 0.90 to 0.95; bf16 RoPE 0.94 to 0.99.  Where all of it stays, the hint costs: 4 layers
+// and PoPE, 0.6 to 1.6 GB, d = 192 and 512 0.90 to 0.95; bf16 RoPE 0.94 to 0.99.  (Not where the very same neurons fire at every
+// token and what they touch would stay: 4 to 8 sequences, a twentieth firing, 1.02 to 1.03, a sixth 0.98 to 1.00, half 0.92 to
+// 0.97; with tokens that differ the same models 0.96 to 0.98, 0.94 to 0.98 and 0.92 to 0.96.)  Where all of it stays, the hint costs: 4 layers
 // of 3072 neurons, d = 192, 4 sequences (180 MB) 1.01.  A single layer stepped again and again finds a good part of its rows in
 // the cache even where it is larger (1 GiB, a twentieth firing, 45.4 | 47.3 us), unless every step walks all of it.  The dense
 // kernel's bf16 rows gain nothing (8 layers, d = 512, 48 sequences 609 | 614).

@@ -143,8 +143,8 @@ const char *bdh_last_error(const bdh_ctx *ctx);
  *                       LayerNorm itself, the next layer's D_x sums the encoder's partials and applies the two
  *                       LayerNorms and the residual (the first layer's D_x makes its row from the embedding), while
  *                       the weights are on their way; taken while those sums stay small against the weights
- *                       (N * n_embd <= 2 Mi and n_head * N * n_embd <= 32 Ki * fused_kb: BASELINE config 1 is the
- *                       largest such shape).  0 = kernel by kernel (values agree to 1e-5; in this form and those
+ *                       (N * n_embd <= 2 Mi and n_head * N * n_embd <= 32 Ki * fused_kb: 4 heads of 8192 neurons
+ *                       at n_embd 256 are the largest such shape).  0 = kernel by kernel (values agree to 1e-5; in this form and those
  *                       of model.one_launch D_x or the row that goes into it is added in another order, so a neuron
  *                       whose pre-activation is within rounding of the threshold may fire in one form only).
  *   "model.fused_kb":   rows of E per workgroup of the encoder's first stage in that form (128 .. 2048, default 256).
@@ -229,8 +229,8 @@ int bdh_state_step(bdh_ctx *ctx, int B, int h, int N, int d, int rotary, const f
  * no hipMalloc / hipFree.  A shape whose partials do not fit returns BDH_E_SHAPE and bdh_last_error
  * names the bytes needed: about 4*B*h*S*(d+1) with S workgroups per (sequence, head) slice (S = N/512
  * for RoPE at d in {256,512}, N/128 when that grid would leave CUs idle, N/64 for the other kernels).
- * BASELINE configs 2 and 4 need 2 and 16 MiB.  All calls on one device share the array: calls that overlap on one device (two streams, two
- * contexts) race; calls ordered on one stream do not.  Nothing in the array has to start at zero: every
+ * 32 sequences of 4 heads of 8192 neurons (d = 256) and of 8 heads of 16384 (d = 512) need 2 and 16 MiB.  All calls on one
+ * device share the array: calls that overlap on one device (two streams, two contexts) race; calls ordered on one stream do not.  Nothing in the array has to start at zero: every
  * element that is read was written by the same call.  The array's address is kept for device ids 0..63; a context
  * on a device beyond that returns BDH_E_UNSUPPORTED here. */
 int bdh_state_step_noalloc(bdh_ctx *ctx, int B, int h, int N, int d, int rotary, const float *x,
